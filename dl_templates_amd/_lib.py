@@ -1,9 +1,9 @@
-"""ctypes binding of ``libdlt_hip.so`` (declared in ``include/dlt.h``).
+"""Loads ``libdlt_hip.so`` (declared in ``include/dlt.h``) and its torch binding ``_dlt_torch.so``.
 
-The shared object is built in-tree by ``dl_templates_amd/csrc/Makefile`` (see
-``__graft_entry__.build``).  It is loaded after ``import torch`` so that it binds to the
-HIP runtime PyTorch already holds: one runtime per process, shared streams and pointers.
-There is no CPU fallback: a missing library or a failing call raises.
+Both are built in-tree by ``dl_templates_amd/csrc/Makefile`` (see ``__graft_entry__.build``).  They are loaded after
+``import torch`` so that they bind to the HIP runtime PyTorch already holds: one runtime per process, shared streams
+and pointers.  The operators call the compiled binding (``native``); the ctypes declarations here serve callers of the
+C ABI itself.  There is no CPU fallback: a missing library or a failing call raises.
 """
 from __future__ import annotations
 
@@ -17,6 +17,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdlt_hip.so")
+BINDING_PATH = os.path.join(_HERE, "_dlt_torch.so")
 CSRC_DIR = os.path.join(_HERE, "csrc")
 
 DLT_BF16, DLT_FP16, DLT_FP32 = 0, 1, 2
@@ -152,6 +153,23 @@ def load():
                 _declare(lib)
                 _lib = lib
     return _lib
+
+
+class _Native:
+    """``_dlt_torch``, imported at the first use of one of its functions (the package imports without being built)."""
+
+    def __getattr__(self, name):
+        load()
+        if not os.path.exists(BINDING_PATH):
+            raise RuntimeError(f"{BINDING_PATH} is missing: build it with `make -C {CSRC_DIR}`. There is no CPU fallback.")
+        from . import _dlt_torch
+        for key, fn in vars(_dlt_torch).items():
+            if not key.startswith("_"):
+                setattr(self, key, fn)
+        return getattr(_dlt_torch, name)
+
+
+native = _Native()
 
 
 def check(rc: int) -> None:
