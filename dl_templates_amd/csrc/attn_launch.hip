@@ -7,6 +7,7 @@
 #include "flash_kernel.hpp"
 #include "swam_bwd_kernel.hpp"
 #include "swa2_bwd_kernel.hpp"
+#include "swat_kernel.hpp"
 
 int dlt_launch_fwd_32_32(const FwdArgs&, int, int, hipStream_t);
 int dlt_launch_fwd_64_64(const FwdArgs&, int, int, hipStream_t);
@@ -28,6 +29,8 @@ int dlt_flash_launch_bwd_32_32(const FlashBwdArgs&, int, int, int, hipStream_t);
 int dlt_flash_launch_bwd_64_64(const FlashBwdArgs&, int, int, int, hipStream_t);
 int dlt_flash_launch_bwd_128_128(const FlashBwdArgs&, int, int, int, hipStream_t);
 int dlt_flash_launch_bwd_64_128(const FlashBwdArgs&, int, int, int, hipStream_t);
+int dlt_swat_launch_32(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
+int dlt_swat_launch_64(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_launch_delta_32_32(const BwdArgs&, hipStream_t);
 int dlt_launch_delta_64_64(const BwdArgs&, hipStream_t);
 int dlt_launch_delta_128_128(const BwdArgs&, hipStream_t);
@@ -437,6 +440,57 @@ bool flash_eligible(const AttnProblem& p, const AttnTensors& t, bool with_do) {
   return true;
 }
 
+// ---- marching tile-window kernels: tiles of 16 or 32 tokens, head dim 32 or 64 exactly ------------------------------
+// What they take beyond flash_eligible: windows whose rows fit the LDS ring (3 x 3 tiles; with 16-token tiles also 5 tile
+// columns, and 5 tile rows at head dim 32), and 16-byte rows with 32-bit offsets for every tensor.  Larger tiles stay on the
+// chunked kernels: a window row of 64-token tiles gives a 64-token chunk work for every wave, and its rows do not fit the ring.
+bool swat_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
+  return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && st[4] >= 0 && slab_span(p, st, (int64_t)p.g.TR * p.g.XLq) * 2 <= ((int64_t)1 << 31) - 1;
+}
+bool swat_eligible(const AttnProblem& p, const AttnTensors& t, bool bwd) {
+  if (p.g.mode != DLT_GEOM_SWA || (p.g.S != 16 && p.g.S != 32)) return false;
+  if (p.dk != p.dv || (p.dk != 32 && p.dk != 64)) return false;
+  if (p.g.WR < 1 || p.g.WC < 1 || p.g.WR > 2 || p.g.WC > 2) return false;
+  if (p.g.S == 32 && (p.g.WR != 1 || p.g.WC != 1)) return false;
+  if (p.g.WR == 2 && p.dk != 32) return false;
+  if (!swat_rows_ok(p, t.q, t.qs) || !swat_rows_ok(p, t.k, t.ks) || !swat_rows_ok(p, t.v, t.vs)) return false;
+  if (!bwd) return swat_rows_ok(p, t.out_o, t.os);
+  return swat_rows_ok(p, t.o, t.os) && swat_rows_ok(p, t.d_o, t.dos) && swat_rows_ok(p, t.dq, t.dqs) && swat_rows_ok(p, t.dk, t.dks) &&
+         swat_rows_ok(p, t.dv, t.dvs);
+}
+
+int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t stream) {
+  if (dlt_route_note(DLT_FAMILY_FLASH)) return DLT_OK;
+  SwatArgs a;
+  a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.o; a.d_o = t.d_o; a.out_o = t.out_o; a.dq = t.dq; a.dk = t.dk; a.dv = t.dv;
+  a.lse = t.lse; a.delta = t.delta;
+  for (int i = 0; i < 5; i++) {
+    a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; a.dos[i] = t.dos[i];
+    a.dqs[i] = t.dqs[i]; a.dks[i] = t.dks[i]; a.dvs[i] = t.dvs[i];
+  }
+  for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];
+  a.tm = p.tm; a.g = p.g; a.B = p.B; a.H = p.H;
+  a.scale_log2 = p.sm_scale * 1.4426950408889634f;
+  a.sm_scale = p.sm_scale;
+  a.nstrips = (p.g.XLq + 127) / 128;
+  // Rows per workgroup.  A band costs its rows plus the prologue that fills the ring (the latency of its loads, about two
+  // steps) and re-reads 2 WR rows; workgroups beyond what the chip holds at once (one or two per CU) wait for a whole band.
+  const int halo = 8 + 2 * p.g.WC * (p.g.S / 16), ring = (2 * p.g.WR + 1) * halo * 64 * p.dk;
+  const int64_t slots = (int64_t)dlt_device_cus() * (ring + (2 * p.g.WR + 1) * halo * 128 <= 80 * 1024 ? 2 : 1);
+  const int64_t cols = (int64_t)p.B * p.H * a.nstrips;
+  int64_t best = -1;
+  a.band = p.g.TR; a.nbands = 1;
+  for (int nb = 1; nb <= p.g.TR; nb++) {
+    const int band = (p.g.TR + nb - 1) / nb;
+    if ((p.g.TR + band - 1) / band != nb) continue;
+    const int64_t cost = (cols * nb + slots - 1) / slots * (band + 2);
+    if (best < 0 || cost < best) { best = cost; a.band = band; a.nbands = nb; }
+  }
+  const int64_t grid = cols * a.nbands;
+  if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
+  return p.dk == 32 ? dlt_swat_launch_32(a, p.dtype, bwd, (int)grid, stream) : dlt_swat_launch_64(a, p.dtype, bwd, (int)grid, stream);
+}
+
 int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {
   if (dlt_route_note(DLT_FAMILY_FLASH)) return DLT_OK;
   FlashArgs a;
@@ -570,6 +624,7 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
     for (int i = 0; i < 5; i++) { t2.qs[i] = t.qrs[i]; t2.ks[i] = t.krs[i]; }
     return dlt_attn_forward(p2, t2, stream);
   }
+  if (flash_eligible(p, t, false) && swat_eligible(p, t, false)) return swat_run(p, t, false, stream);
   if (flash_eligible(p, t, false)) return flash_forward(p, t, dc, stream);
   if (swa2_tiles_eligible(p, t, false)) return swa2_forward(p, t, stream);
   if (dlt_route_note(DLT_FAMILY_GENERIC)) return DLT_OK;
@@ -646,6 +701,7 @@ int dlt_attn_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t st
     if (rc != DLT_OK) return rc;
     return dlt_rope_inplace_4d(t.dk, t.dks, p.B, p.H, (int64_t)p.g.TR * p.g.XLk, p.dk, &r, 1, p.dtype, stream);
   }
+  if (flash_eligible(p, t, true) && swat_eligible(p, t, true)) return swat_run(p, t, true, stream);
   if (flash_eligible(p, t, true)) return flash_backward(p, t, dc, stream);
   if (swa2_tiles_eligible(p, t, true)) return swa2_backward(p, t, stream);
   if (dlt_route_note(DLT_FAMILY_GENERIC)) return DLT_OK;

@@ -184,6 +184,19 @@ DLT_DEV void flash_block(int lin, int nblk, int TR, int own, int& bh, int& r, in
   x0 = xb * own;
 }
 
+// Image layout: the heads of a pixel lie side by side (64 bytes each at head dim 32), so the workgroups of all heads of
+// one stretch of tiles are neighbours in launch order: they run at the same time on one XCD, whose L2 then serves the
+// 128-byte lines that two heads share and the whole pages that all of them touch.
+DLT_DEV void flash_block_image(int lin, int nblk, int TR, int H, int own, int& bh, int& r, int& x0) {
+  const int blk = lin / H, h = lin - blk * H;
+  const int per = nblk * TR;
+  const int b = blk / per;
+  const int rem = blk - b * per;
+  bh = b * H + h;
+  r = rem / nblk;
+  x0 = (rem - r * nblk) * own;
+}
+
 // Causal mask: the work of a block grows with its position, and blocks are handed to free CUs in launch order.  Taken
 // (batch, head) by (batch, head), the heavy blocks of the last heads start late and finish alone; here `G` heads at a
 // time are interleaved, heaviest blocks of all of them first.  The host sizes G so that the streamed tensors of a group
@@ -244,6 +257,7 @@ __global__ __launch_bounds__(256, flash_occ_fwd(DK, DV)) void flash_fwd_kernel(c
   int bh, r_own, x0;
   // causal: the blocks with the most keys to visit are launched first
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
+  else if constexpr (IMG) flash_block_image(lin, a.nblk, a.g.TR, a.H, OWN, bh, r_own, x0);
   else flash_block(lin, a.nblk, TILE ? a.g.TR : 1, OWN, bh, r_own, x0);
   const int wq0 = x0 + wave * 16 * NP;                            // first query of this wave
   const int b = bh / a.H, h = bh - b * a.H;
@@ -603,6 +617,7 @@ __global__ __launch_bounds__(256, flash_occ_q(DK, DV)) void flash_bwd_q_kernel(c
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_q, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
+  else if constexpr (IMG) flash_block_image(lin, a.nblk_q, a.g.TR, a.H, OWN, bh, r_own, x0);
   else flash_block(lin, a.nblk_q, TILE ? a.g.TR : 1, OWN, bh, r_own, x0);
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
@@ -790,6 +805,7 @@ __global__ __launch_bounds__(256, flash_occ_kv(DK, DV, MODE)) void flash_bwd_kv_
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_k, a.B * a.H, a.causal_group, OWN, false, bh, r_own, x0);
+  else if constexpr (IMG) flash_block_image(lin, a.nblk_k, a.g.TR, a.H, OWN, bh, r_own, x0);
   else flash_block(lin, a.nblk_k, TILE ? a.g.TR : 1, OWN, bh, r_own, x0);
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* kb_ = reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1];

@@ -102,3 +102,25 @@ def test_small_tiles_forward_backward(B, H, th, tw, S, WR, WC, d, dtype):
     assert (o.float().cpu() - o_w).abs().max().item() <= FWD_TOL
     errs = (_rel(qg.grad, dq_w), _rel(kg.grad, dk_w), _rel(vg.grad, dv_w))
     assert max(errs) <= GRAD_TOL, errs
+
+
+# the marching tile-window kernels (tiles of 16 or 32 tokens, head dim 32 / 64): every instantiated window, single rows and
+# columns, strips of 8 blocks with a remainder, grids smaller than the window, bands of one and of many rows
+MARCH = [(1, 1, 1, 16, 1, 1, 32), (1, 1, 9, 16, 1, 1, 64), (9, 1, 1, 16, 1, 1, 32), (7, 8, 1, 16, 1, 1, 64), (5, 9, 2, 16, 1, 2, 32), (6, 17, 1, 16, 1, 2, 64),
+         (7, 10, 1, 16, 2, 1, 32), (9, 11, 1, 16, 2, 2, 32), (2, 2, 2, 16, 2, 2, 32), (5, 5, 1, 32, 1, 1, 32), (4, 9, 2, 32, 1, 1, 64), (11, 3, 40, 16, 1, 1, 32)]
+
+
+@pytest.mark.parametrize("th,tw,B,S,WR,WC,d", MARCH)
+@pytest.mark.parametrize("image", [False, True])
+def test_marching_tile_windows(th, tw, B, S, WR, WC, d, image):
+    sw = _swa()
+    H, N, dt = 3, th * tw * S, torch.bfloat16 if tw % 2 else torch.float16
+    q, k, v, do = orc.make_qkv(N + S + d, B, H, N, N, d, d, dt)
+    o_w, dq_w, dk_w, dv_w = orc.tiled_swa_grads(q.float(), k.float(), v.float(), do.float(), S, th, tw, WR, WC, 0.2)
+    lay = (lambda t: orc.tokens_to_image(t, th, tw, 4, S // 4).contiguous()) if image else (lambda t: t)
+    qg, kg, vg = (lay(t).cuda().requires_grad_(True) for t in (q, k, v))
+    o = sw.TiledSwaImage.apply(qg, kg, vg, 4, S // 4, WR, WC, 0.2) if image else sw.TiledSwa.apply(qg, kg, vg, S, th, tw, WR, WC, 0.2)
+    o.backward(lay(do).cuda())
+    assert (o.float().cpu() - lay(o_w)).abs().max().item() <= FWD_TOL
+    errs = (_rel(qg.grad, lay(dq_w)), _rel(kg.grad, lay(dk_w)), _rel(vg.grad, lay(dv_w)))
+    assert max(errs) <= GRAD_TOL, errs
