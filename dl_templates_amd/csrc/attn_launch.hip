@@ -25,10 +25,26 @@ int dlt_flash_launch_fwd_32_32(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_fwd_64_64(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_fwd_128_128(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_fwd_64_128(const FlashArgs&, int, int, hipStream_t);
-int dlt_flash_launch_bwd_32_32(const FlashBwdArgs&, int, int, int, hipStream_t);
-int dlt_flash_launch_bwd_64_64(const FlashBwdArgs&, int, int, int, hipStream_t);
-int dlt_flash_launch_bwd_128_128(const FlashBwdArgs&, int, int, int, hipStream_t);
-int dlt_flash_launch_bwd_64_128(const FlashBwdArgs&, int, int, int, hipStream_t);
+int dlt_flash_launch_bwd_q_32_32(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_kv_32_32(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_q_64_64(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_kv_64_64(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_q_128_128(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_kv_128_128(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_q_64_128(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flash_launch_bwd_kv_64_128(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
+int dlt_flashs_fwd_32_32(const FlashArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_q_32_32(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_kv_32_32(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_fwd_64_64(const FlashArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_q_64_64(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_kv_64_64(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_fwd_64_128(const FlashArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_q_64_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_kv_64_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_fwd_128_128(const FlashArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_q_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flashs_bwd_kv_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
 int dlt_swat_launch_32(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_swat_launch_64(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_launch_delta_32_32(const BwdArgs&, hipStream_t);
@@ -491,6 +507,50 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   return p.dk == 32 ? dlt_swat_launch_32(a, p.dtype, bwd, (int)grid, stream) : dlt_swat_launch_64(a, p.dtype, bwd, (int)grid, stream);
 }
 
+// Which kernels a dense / causal pass runs on: 0 = the streamed side passes through LDS chunk by chunk (64 ... 256 own
+// tokens per workgroup), 1 / 2 = it is split over the waves of workgroups that own one or two blocks of 16 tokens
+// (csrc/flash_split_kernel.hpp).  Chunked workgroups win once they fill the chip; below that their time is a start and the
+// chunks of 64 streamed tokens one after the other, however few the workgroups.  The split ones take
+//     fixed + rounds over the CUs * (start and final sum of a workgroup + its 32-token blocks * time of a block on a CU).
+// The constants (us) are least-squares fits to launches of 32 ... 8192 tokens on either side and 4 ... 128 heads, dense and
+// causal; on those the rule picks the fastest of the three but for 0.4 % of the total time.
+//   77 queries x 1500 keys, 16 heads, 64/64: forward 22 -> 10 us, dQ 24 -> 11; 482 keys x 5450 queries, 4 heads: dK/dV 86 -> 26
+struct FlashSplitCost { int own; float start, chunk, fixed1, wg1, block1, fixed2, wg2, block2; };   // own: tokens of a chunked workgroup
+int flash_split(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
+  constexpr float NONE = 1e9f;
+  static const FlashSplitCost COST[3][4] = {   // by pass (forward, dQ, dK/dV) and DimClass::id
+      {{128, 3.50f, .822f, 2.31f, 1.36f, .137f, 1.09f, 3.79f, .141f},    // 64/64
+       {256, 6.78f, 1.493f, .59f, 3.70f, .272f, 0.f, 5.81f, .322f},      // 128/128
+       {256, 6.06f, 1.272f, 1.53f, 2.57f, .174f, 0.f, 5.73f, .185f},     // 64/128
+       {128, 2.94f, .698f, 2.84f, .52f, .055f, 2.41f, 1.13f, .094f}},    // 32/32
+      {{128, 4.84f, .850f, 2.07f, 2.19f, .138f, .43f, 5.72f, .144f},
+       {128, 6.58f, 1.404f, .67f, 4.25f, .289f, NONE, NONE, NONE},
+       {128, 5.43f, 1.073f, .99f, 4.27f, .244f, NONE, NONE, NONE},
+       {128, 4.04f, .750f, 2.73f, .68f, .057f, 2.36f, 1.44f, .090f}},
+      {{128, 4.94f, 1.083f, 1.85f, 2.73f, .134f, 1.36f, 4.59f, .171f},
+       {64, 5.62f, 1.226f, 1.31f, 4.42f, .283f, NONE, NONE, NONE},
+       {128, 5.79f, 1.627f, 1.32f, 4.15f, .185f, NONE, NONE, NONE},
+       {128, 4.28f, 1.038f, 2.51f, 1.14f, .072f, 2.79f, 1.38f, .114f}}};
+  // From 1536 tokens on a causal slab gives the same bits whatever the number of slabs of the call (documented and tested):
+  // the choice must not depend on it there.
+  if (causal && own >= 1536) return 0;
+  const FlashSplitCost& c = COST[pass][dc.id];
+  const float cus = (float)dlt_device_cus();
+  if (bh * ((own + c.own - 1) / c.own) > (int64_t)cus) return 0;
+  float least = c.start + c.chunk * (float)((other + 63) / 64);
+  // the pieces of a row that a head dim below its class does not have are not read
+  const float blocks = (float)((other + 31) / 32) * ((float)dims / (float)(dc.DK + dc.DV));
+  int best = 0;
+  for (int np = 1; np <= 2; np++) {
+    const float rounds = (float)(bh * ((own + 16 * np - 1) / (16 * np))) / cus;
+    // under a causal mask the workgroups of several rounds see about half of the other side
+    const float seen = causal && rounds > 1.f ? 0.55f * blocks : blocks;
+    const float t = (np == 1 ? c.fixed1 : c.fixed2) + (rounds > 1.f ? rounds : 1.f) * (np == 1 ? c.wg1 + c.block1 * seen : c.wg2 + c.block2 * seen);
+    if (t < least) { least = t; best = np; }
+  }
+  return best;
+}
+
 int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {
   if (dlt_route_note(DLT_FAMILY_FLASH)) return DLT_OK;
   FlashArgs a;
@@ -511,6 +571,15 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   const int64_t grid = (int64_t)p.B * p.H * p.g.TR * a.nblk;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "flash forward: grid too large");
+  if (p.g.mode != DLT_GEOM_SWA) {
+    const int np = flash_split(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0);
+    if (np != 0) switch (dc.id) {
+      case 0: return dlt_flashs_fwd_64_64(a, p.dtype, np, stream);
+      case 1: return dlt_flashs_fwd_128_128(a, p.dtype, np, stream);
+      case 3: return dlt_flashs_fwd_32_32(a, p.dtype, np, stream);
+      default: return dlt_flashs_fwd_64_128(a, p.dtype, np, stream);
+    }
+  }
   switch (dc.id) {
     case 0: return dlt_flash_launch_fwd_64_64(a, p.dtype, (int)grid, stream);
     case 1: return dlt_flash_launch_fwd_128_128(a, p.dtype, (int)grid, stream);
@@ -571,12 +640,23 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
   a.sm_scale = p.sm_scale;
   const int64_t grid_q = (int64_t)p.B * p.H * p.g.TR * a.nblk_q, grid_kv = (int64_t)p.B * p.H * p.g.TR * a.nblk_k;
   if (grid_q > 0x7fffffff || grid_kv > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "flash backward: grid too large");
+  // each pass streams its other side through LDS or splits it over the waves, whichever suits its own shape
+  const int64_t nbh = (int64_t)p.B * p.H;
+  const bool seq = p.g.mode != DLT_GEOM_SWA;
+  const int np_q = seq ? flash_split(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0) : 0;
+  const int np_kv = seq ? flash_split(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0) : 0;
+  int rc;
+#define DLT_FLASH_PASS(C)                                                                                                  \
+  rc = np_q != 0 ? dlt_flashs_bwd_q_##C(a, p.dtype, np_q, stream) : dlt_flash_launch_bwd_q_##C(a, p.dtype, (int)grid_q, stream); \
+  if (rc != DLT_OK) return rc;                                                                                             \
+  return np_kv != 0 ? dlt_flashs_bwd_kv_##C(a, p.dtype, np_kv, stream) : dlt_flash_launch_bwd_kv_##C(a, p.dtype, (int)grid_kv, stream)
   switch (dc.id) {
-    case 0: return dlt_flash_launch_bwd_64_64(a, p.dtype, (int)grid_kv, (int)grid_q, stream);
-    case 1: return dlt_flash_launch_bwd_128_128(a, p.dtype, (int)grid_kv, (int)grid_q, stream);
-    case 3: return dlt_flash_launch_bwd_32_32(a, p.dtype, (int)grid_kv, (int)grid_q, stream);
-    default: return dlt_flash_launch_bwd_64_128(a, p.dtype, (int)grid_kv, (int)grid_q, stream);
+    case 0: DLT_FLASH_PASS(64_64);
+    case 1: DLT_FLASH_PASS(128_128);
+    case 3: DLT_FLASH_PASS(32_32);
+    default: DLT_FLASH_PASS(64_128);
   }
+#undef DLT_FLASH_PASS
 }
 
 }  // namespace

@@ -83,9 +83,7 @@ int flash_launch_fwd_t(const FlashArgs& a, int grid, hipStream_t stream) {
 }
 
 template <typename TIO, int MODE>
-int flash_launch_bwd_c(const FlashBwdArgs& a, int grid_kv, int grid_q, hipStream_t stream) {
-  // dQ first: with fuse_delta it produces the delta vector the dK/dV kernel consumes
-  bool dq_done = false;
+int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && flash_async_staging()) {
       constexpr int NP = FLASHD_DQ_NP(DLT_DK, DLT_DV), CK = 64, NW = FLASHD_BWD_NW;
@@ -103,18 +101,21 @@ int flash_launch_bwd_c(const FlashBwdArgs& a, int grid_kv, int grid_q, hipStream
       hipLaunchKernelGGL(kern, dim3(a.B * a.H * ad.nblk_q), dim3(64 * NW), lds, stream, ad);
       dlt_timing_after(stream);
       DLT_CHECK_LAUNCH("flash dQ launch");
-      dq_done = true;
+      return DLT_OK;
     }
   }
-  if (!dq_done) {
-    auto kern = flash_bwd_q_kernel<TIO, DLT_DK, DLT_DV, flash_np_q(DLT_DK, DLT_DV), flash_ck_q(DLT_DK, DLT_DV), MODE>;
-    int rc = flash_set_lds(kern, a.lds_q);
-    if (rc != DLT_OK) return rc;
-    dlt_timing_before(DLT_K_BWD_Q, stream);
-    hipLaunchKernelGGL(kern, dim3(grid_q), dim3(256), a.lds_q, stream, a);
-    dlt_timing_after(stream);
-    DLT_CHECK_LAUNCH("flash dQ launch");
-  }
+  auto kern = flash_bwd_q_kernel<TIO, DLT_DK, DLT_DV, flash_np_q(DLT_DK, DLT_DV), flash_ck_q(DLT_DK, DLT_DV), MODE>;
+  int rc = flash_set_lds(kern, a.lds_q);
+  if (rc != DLT_OK) return rc;
+  dlt_timing_before(DLT_K_BWD_Q, stream);
+  hipLaunchKernelGGL(kern, dim3(grid_q), dim3(256), a.lds_q, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("flash dQ launch");
+  return DLT_OK;
+}
+
+template <typename TIO, int MODE>
+int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     // dense / causal, head dims that are multiples of 8: chunks are copied HBM -> LDS asynchronously (in tile mode,
     // where whole blocks are skipped, the register-staged kernel measured 1.5 % faster)
@@ -150,15 +151,25 @@ int flash_launch_bwd_c(const FlashBwdArgs& a, int grid_kv, int grid_q, hipStream
   return DLT_OK;
 }
 
+// dQ is launched first: with fuse_delta it produces the delta vector the dK/dV kernel consumes
 template <typename TIO>
-int flash_launch_bwd_t(const FlashBwdArgs& a, int grid_kv, int grid_q, hipStream_t stream) {
-  if (a.tile) return a.tm.img ? flash_launch_bwd_c<TIO, 3>(a, grid_kv, grid_q, stream) : flash_launch_bwd_c<TIO, 2>(a, grid_kv, grid_q, stream);
-  return a.causal ? flash_launch_bwd_c<TIO, 1>(a, grid_kv, grid_q, stream) : flash_launch_bwd_c<TIO, 0>(a, grid_kv, grid_q, stream);
+int flash_launch_bwd_q_t(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
+  if (a.tile) return a.tm.img ? flash_launch_bwd_q_c<TIO, 3>(a, grid_q, stream) : flash_launch_bwd_q_c<TIO, 2>(a, grid_q, stream);
+  return a.causal ? flash_launch_bwd_q_c<TIO, 1>(a, grid_q, stream) : flash_launch_bwd_q_c<TIO, 0>(a, grid_q, stream);
+}
+template <typename TIO>
+int flash_launch_bwd_kv_t(const FlashBwdArgs& a, int grid_kv, hipStream_t stream) {
+  if (a.tile) return a.tm.img ? flash_launch_bwd_kv_c<TIO, 3>(a, grid_kv, stream) : flash_launch_bwd_kv_c<TIO, 2>(a, grid_kv, stream);
+  return a.causal ? flash_launch_bwd_kv_c<TIO, 1>(a, grid_kv, stream) : flash_launch_bwd_kv_c<TIO, 0>(a, grid_kv, stream);
 }
 }  // namespace
 
-int DLT_FCAT3(dlt_flash_launch_bwd_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, int dtype, int grid_kv, int grid_q, hipStream_t stream) {
-  return dtype == DLT_BF16 ? flash_launch_bwd_t<bf16_t>(a, grid_kv, grid_q, stream) : flash_launch_bwd_t<f16_t>(a, grid_kv, grid_q, stream);
+int DLT_FCAT3(dlt_flash_launch_bwd_q_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, int dtype, int grid_q, hipStream_t stream) {
+  return dtype == DLT_BF16 ? flash_launch_bwd_q_t<bf16_t>(a, grid_q, stream) : flash_launch_bwd_q_t<f16_t>(a, grid_q, stream);
+}
+
+int DLT_FCAT3(dlt_flash_launch_bwd_kv_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, int dtype, int grid_kv, hipStream_t stream) {
+  return dtype == DLT_BF16 ? flash_launch_bwd_kv_t<bf16_t>(a, grid_kv, stream) : flash_launch_bwd_kv_t<f16_t>(a, grid_kv, stream);
 }
 
 int DLT_FCAT3(dlt_flash_launch_fwd_, DLT_DK, DLT_DV)(const FlashArgs& a, int dtype, int grid, hipStream_t stream) {

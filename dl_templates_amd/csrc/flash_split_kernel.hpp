@@ -1,0 +1,505 @@
+// Dense / causal flash attention for calls with too few own blocks to fill the chip: few queries against many keys (and
+// the transpose), short sequences, few heads.
+//
+// What bounded those calls: the kernels that stream chunks through LDS give one wave 32 own tokens and walk the other side
+// one 64-token chunk after the other, so 77 queries x 1500 keys x 16 heads were 16 workgroups of 24 dependent rounds
+// (22.5 us on 6 % of the CUs).  Here a workgroup owns 16 NP tokens and its NW waves split the OTHER side: wave w takes the
+// 32-token blocks w, w + NW, ...  The waves share nothing while they stream, so there is no barrier in the loop: row operands
+// come straight from HBM / L2 one block ahead, the tensors that are also needed transposed pass through a wave-private LDS
+// tile.  At the end the partial results meet in LDS: (m, l, o) of the forward pass by the usual rescaling, gradients by
+// plain fp32 sums, in a fixed order (results do not depend on timing).
+#pragma once
+#include "flash_kernel.hpp"
+
+template <int D> DLT_DEV int flashs_swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : (t & 7) * (D / 64); }
+
+// wave-private [32 tokens][D] tile, rows of 2 D bytes, 16-byte piece p of token t at p ^ swz(t)
+template <int D>
+struct FlashsTile {
+  static constexpr int BYTES = 64 * D, NV = D / 16;   // 16-byte vectors per lane of one block
+  // rows of block `b` (tokens clamped to the last one), pieces past `dact` are zero
+  static DLT_DEV void load(u32x4 (&r)[NV], const char* base, int sn2, int b, int len, int dact, int lane) {
+#pragma unroll
+    for (int it = 0; it < NV; it++) {
+      const int v = lane + 64 * it, t = v / (D / 8), p = v % (D / 8);
+      r[it] = u32x4{0u, 0u, 0u, 0u};
+      if (8 * p < dact) r[it] = *reinterpret_cast<const u32x4*>(base + (uint32_t)(dlt_imin(32 * b + t, len - 1) * sn2 + 16 * p));
+    }
+  }
+  static DLT_DEV void write(char* s, const u32x4 (&r)[NV], int lane) {
+#pragma unroll
+    for (int it = 0; it < NV; it++) {
+      const int v = lane + 64 * it, t = v / (D / 8), p = v % (D / 8);
+      lds_write16(s + t * 2 * D + 16 * (p ^ flashs_swz<D>(t)), r[it]);
+    }
+  }
+  // A operand, 16 tokens (half mb) x dims 32 c ..
+  static DLT_DEV u32x4 rows(const char* s, int mb, int c, int n, int g) {
+    return lds_read16(s + (16 * mb + n) * 2 * D + 16 * ((4 * c + g) ^ flashs_swz<D>(n)));
+  }
+  // A operand, dims 16 d .. as rows, the 32 tokens along k
+  static DLT_DEV u32x4 trans(const char* s, int d, int n, int g) {
+    const int t = 4 * g + (n >> 2);
+    const char* p = s + t * 2 * D + 16 * ((2 * d + ((n >> 1) & 1)) ^ flashs_swz<D>(t)) + 8 * (n & 1);
+    const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 32 * D);   // token t + 16: same swizzle
+    return u32x4{lo.x, lo.y, hi.x, hi.y};
+  }
+};
+
+// A operand rows straight from HBM: 32 tokens of block b
+template <int D>
+DLT_DEV void flashs_load_rows(u32x4 (&f)[2][D / 32], const char* base, int sn2, int b, int len, int dact, int n, int g) {
+#pragma unroll
+  for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+    for (int c = 0; c < D / 32; c++) {
+      f[mb][c] = u32x4{0u, 0u, 0u, 0u};
+      if (8 * (4 * c + g) < dact)
+        f[mb][c] = *reinterpret_cast<const u32x4*>(base + (uint32_t)(dlt_imin(32 * b + 16 * mb + n, len - 1) * sn2 + 64 * c + 16 * g));
+    }
+}
+
+// Partial [16 NP][D] results of NW waves (C layout: lane n = own token, dims 16 d + 4 g + i) -> their sum, 8 dims per thread and
+// turn: out(row, first dim, 8 values).
+template <int D, int NP, int NW>
+struct FlashsSum {
+  static constexpr int P = D + 4;                      // fp32 row pitch
+  static constexpr int BYTES = NW * 16 * NP * P * 4;
+  static DLT_DEV void put(float* s, const f32x4 (&acc)[NP][D / 16], int wave, int n, int g) {
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int d = 0; d < D / 16; d++) *reinterpret_cast<f32x4*>(s + ((wave * NP + p) * 16 + n) * P + 16 * d + 4 * g) = acc[p][d];
+  }
+  template <typename Out>
+  static DLT_DEV void reduce(const float* s, int tid, Out out) {
+    for (int id = tid; id < 16 * NP * (D / 8); id += 64 * NW) {
+      const int row = id / (D / 8), c = id % (D / 8);
+      f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll
+      for (int w = 0; w < NW; w++) {
+        const float* q = s + (w * 16 * NP + row) * P + 8 * c;
+        a += *reinterpret_cast<const f32x4*>(q);
+        b += *reinterpret_cast<const f32x4*>(q + 4);
+      }
+      float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      out(row, 8 * c, v);
+    }
+  }
+};
+
+// workgroup -> (batch * head, first own token)
+DLT_DEV void flashs_block(int nblk, int own, int& bh, int& x0) {
+  const int lin = xcd_remap(blockIdx.x, gridDim.x);
+  bh = lin / nblk;
+  x0 = (lin - bh * nblk) * own;
+}
+
+template <int DK, int DV, int NP, int NW>
+constexpr int flashs_lds_fwd() {
+  const int tiles = NW * FlashsTile<DV>::BYTES, sum = FlashsSum<DV, NP, NW>::BYTES + 2 * NW * 16 * NP * 4;
+  return tiles > sum ? tiles : sum;
+}
+
+template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
+__global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const FlashArgs a) {
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  constexpr int KC = DK / 32, VB = DV / 16;
+  typedef FlashsTile<DV> VT;
+  typedef FlashsSum<DV, NP, NW> Sum;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bh, x0;
+  flashs_block(a.nblk, 16 * NP, bh, x0);
+  const int b = bh / a.H, h = bh - b * a.H;
+  const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
+  const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
+  const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
+  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
+  const int len = CAUSAL ? dlt_imin(a.Lk, x0 + 16 * NP) : a.Lk;   // causal: keys up to the last own query
+  const int nkb = (len + 31) / 32;
+  char* sV = smem + wave * VT::BYTES;
+
+  u32x4 kf[2][KC], vr[VT::NV];
+  if (wave < nkb) {
+    flashs_load_rows<DK>(kf, kb_, ksn, wave, a.Lk, a.dk, n, g);
+    VT::load(vr, vb_, vsn, wave, a.Lk, a.dv, lane);
+  }
+  RopeDev no_rope = RopeDev{};
+  u32x4 qf[NP][KC];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const int x = x0 + 16 * p + n;
+    swa1_load_own<TIO, CT, DK>(qf[p], qb, 1, a.dk, x < a.Lq ? x * a.qs[2] : (int64_t)-1, g, no_rope, false);
+  }
+  float m_run[NP], l_run[NP];
+  f32x4 acc[NP][VB];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    m_run[p] = -INFINITY;
+    l_run[p] = 0.f;
+#pragma unroll
+    for (int d = 0; d < VB; d++) acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float scale = a.scale_log2;
+  for (int kb = wave; kb < nkb; kb += NW) {
+    VT::write(sV, vr, lane);
+    u32x4 ka[2][KC];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+      for (int c = 0; c < KC; c++) ka[mb][c] = kf[mb][c];
+    if (kb + NW < nkb) {
+      flashs_load_rows<DK>(kf, kb_, ksn, kb + NW, a.Lk, a.dk, n, g);
+      VT::load(vr, vb_, vsn, kb + NW, a.Lk, a.dv, lane);
+    }
+    const bool tail = 32 * kb + 32 > a.Lk || (CAUSAL && 32 * kb + 31 > x0);
+    u32x4 pb[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+      for (int c = 0; c < KC; c++) {
+        s0 = Mma<CT>::mfma(ka[0][c], qf[p][c], s0);
+        s1 = Mma<CT>::mfma(ka[1][c], qf[p][c], s1);
+      }
+      float t[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+      if (tail) {
+        const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, a.Lk - 1) : a.Lk - 1;
+#pragma unroll
+        for (int i = 0; i < 8; i++) t[i] = 32 * kb + 16 * (i >> 2) + 4 * g + (i & 3) <= klim ? t[i] : -INFINITY;
+      }
+      const float mloc = wave_max4(fmaxf(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])), fmaxf(fmaxf(t[4], t[5]), fmaxf(t[6], t[7]))));
+      if (__builtin_amdgcn_ballot_w64((mloc - m_run[p]) * scale > 8.f)) {   // the reference maximum moves (see flash_fwd_kernel)
+        keep_branch();
+        const float m_new = fmaxf(m_run[p], mloc);
+        const float alpha = m_run[p] == m_new ? 1.f : fast_exp2((m_run[p] - m_new) * scale);
+        m_run[p] = m_new;
+#pragma unroll
+        for (int d = 0; d < VB; d++) acc[p][d] *= alpha;
+        l_run[p] *= alpha;
+      }
+      const float neg_m2 = m_run[p] == -INFINITY ? 0.f : -m_run[p] * scale;
+#pragma unroll
+      for (int i = 0; i < 8; i++) t[i] = fast_exp2(fmaf(t[i], scale, neg_m2));
+      pb[p] = pack8<CT>(t);
+      const unsigned one2 = pack2<CT>(1.f, 1.f);   // row sums of the rounded probabilities, per lane group
+      l_run[p] = dot2_acc<CT>(pb[p].w, one2, dot2_acc<CT>(pb[p].z, one2, dot2_acc<CT>(pb[p].y, one2, dot2_acc<CT>(pb[p].x, one2, l_run[p]))));
+    }
+#pragma unroll
+    for (int d = 0; d < VB; d++) {
+      const u32x4 vt = VT::trans(sV, d, n, g);
+#pragma unroll
+      for (int p = 0; p < NP; p++) acc[p][d] = Mma<CT>::mfma(vt, pb[p], acc[p][d]);
+    }
+  }
+  // ---- the waves' partial results meet
+  float* sums = reinterpret_cast<float*>(smem);
+  float* sm = reinterpret_cast<float*>(smem + Sum::BYTES);   // [wave][own] maxima, then row sums
+  float* sl = sm + NW * 16 * NP;
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const float l = wave_sum4(l_run[p]);
+    if (g == 0) {
+      sm[wave * 16 * NP + 16 * p + n] = m_run[p];
+      sl[wave * 16 * NP + 16 * p + n] = l;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    float m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; w++) m = fmaxf(m, sm[w * 16 * NP + 16 * p + n]);
+    const float f = m_run[p] == -INFINITY ? 0.f : fast_exp2((m_run[p] - m) * scale);
+#pragma unroll
+    for (int d = 0; d < VB; d++) acc[p][d] *= f;
+  }
+  Sum::put(sums, acc, wave, n, g);
+  __syncthreads();
+  auto total = [&](int row, float& m, float& l) {
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) m = fmaxf(m, sm[w * 16 * NP + row]);
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float mw = sm[w * 16 * NP + row];
+      l += mw == -INFINITY ? 0.f : sl[w * 16 * NP + row] * fast_exp2((mw - m) * scale);
+    }
+  };
+  TIO* ob = reinterpret_cast<TIO*>(a.o) + b * a.os[0] + h * a.os[1];
+  Sum::reduce(sums, tid, [&](int row, int d0, float* v) {
+    if (x0 + row >= a.Lq || d0 >= a.dv) return;
+    float m, l;
+    total(row, m, l);
+    const float inv = l > 0.f ? fast_rcp(l) : 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] *= inv;
+    Io<TIO, CT>::store8(ob + (x0 + row) * a.os[2] + d0 * a.os[3], v, a.o_vec != 0, a.os[3], dlt_imin(8, a.dv - d0));
+    if (d0 == 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + (x0 + row) * a.ls[2]), m * scale + fast_log2(l));
+  });
+}
+
+template <int DK, int DV, int NP, int NW>
+constexpr int flashs_lds_q() {
+  const int tiles = NW * FlashsTile<DK>::BYTES, sum = FlashsSum<DK, NP, NW>::BYTES;
+  return tiles > sum ? tiles : sum;
+}
+
+// dQ: own = queries, the waves split the keys; delta of the own queries is formed (fuse_delta) and stored on the way
+template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
+__global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const FlashBwdArgs a) {
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16;
+  typedef FlashsTile<DK> KT;
+  typedef FlashsSum<DK, NP, NW> Sum;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bh, x0;
+  flashs_block(a.nblk_q, 16 * NP, bh, x0);
+  const int b = bh / a.H, h = bh - b * a.H;
+  const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
+  const TIO* dob = reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1];
+  const TIO* ob = reinterpret_cast<const TIO*>(a.o) + b * a.os[0] + h * a.os[1];
+  const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
+  const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
+  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
+  const int len = CAUSAL ? dlt_imin(a.Lk, x0 + 16 * NP) : a.Lk;
+  const int nkb = (len + 31) / 32;
+  char* sK = smem + wave * KT::BYTES;
+
+  u32x4 kr[KT::NV], vf[2][VC];
+  if (wave < nkb) {
+    KT::load(kr, kb_, ksn, wave, a.Lk, a.dk_, lane);
+    flashs_load_rows<DV>(vf, vb_, vsn, wave, a.Lk, a.dv_, n, g);
+  }
+  RopeDev no_rope = RopeDev{};
+  u32x4 qf[NP][KC], dof[NP][VC];
+  float nlse[NP];
+  f32x4 dinit[NP], acc[NP][KB];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const int x = x0 + 16 * p + n;
+    const bool in = x < a.Lq;
+    swa1_load_own<TIO, CT, DK>(qf[p], qb, 1, a.dk_, in ? x * a.qs[2] : (int64_t)-1, g, no_rope, false);
+    swa1_load_own<TIO, CT, DV>(dof[p], dob, 1, a.dv_, in ? x * a.dos[2] : (int64_t)-1, g, no_rope, false);
+    const int64_t off = b * a.ls[0] + h * a.ls[1] + (in ? x : 0) * a.ls[2];
+    nlse[p] = in ? -a.lse[off] : 0.f;
+    float del;
+    if (a.fuse_delta != 0) {
+      u32x4 of[VC];
+      swa1_load_own<TIO, CT, DV>(of, ob, 1, a.dv_, in ? x * a.os[2] : (int64_t)-1, g, no_rope, false);
+      float part = 0.f;
+#pragma unroll
+      for (int c = 0; c < VC; c++) {
+        float fo[8], fd[8];
+        unpack8<CT>(of[c], fo);
+        unpack8<CT>(dof[p][c], fd);
+#pragma unroll
+        for (int j = 0; j < 8; j++) part += fo[j] * fd[j];
+      }
+      del = wave_sum4(part);
+      if (wave == 0 && g == 0 && in) store_stream4(a.delta_out + off, del);
+    } else {
+      del = in ? a.delta[off] : 0.f;
+    }
+    dinit[p] = f32x4{-del, -del, -del, -del};
+#pragma unroll
+    for (int d = 0; d < KB; d++) acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float scale = a.scale_log2;
+  for (int kb = wave; kb < nkb; kb += NW) {
+    KT::write(sK, kr, lane);
+    u32x4 va[2][VC];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+      for (int c = 0; c < VC; c++) va[mb][c] = vf[mb][c];
+    if (kb + NW < nkb) {
+      KT::load(kr, kb_, ksn, kb + NW, a.Lk, a.dk_, lane);
+      flashs_load_rows<DV>(vf, vb_, vsn, kb + NW, a.Lk, a.dv_, n, g);
+    }
+    const bool tail = 32 * kb + 32 > a.Lk || (CAUSAL && 32 * kb + 31 > x0);
+    u32x4 dsb[NP];
+    float ds[NP][8];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++) {
+      u32x4 ka[KC];
+#pragma unroll
+      for (int c = 0; c < KC; c++) ka[c] = KT::rows(sK, mb, c, n, g);
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = dinit[p];
+#pragma unroll
+        for (int c = 0; c < KC; c++) s = Mma<CT>::mfma(ka[c], qf[p][c], s);
+#pragma unroll
+        for (int c = 0; c < VC; c++) dp = Mma<CT>::mfma(va[mb][c], dof[p][c], dp);
+        const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, a.Lk - 1) : a.Lk - 1;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float pv = fast_exp2(fmaf(s[i], scale, nlse[p]));
+          if (tail) pv = 32 * kb + 16 * mb + 4 * g + i <= klim ? pv : 0.f;
+          ds[p][4 * mb + i] = pv * dp[i];
+        }
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < NP; p++) dsb[p] = pack8<CT>(ds[p]);
+#pragma unroll
+    for (int d = 0; d < KB; d++) {
+      const u32x4 kt = KT::trans(sK, d, n, g);
+#pragma unroll
+      for (int p = 0; p < NP; p++) acc[p][d] = Mma<CT>::mfma(kt, dsb[p], acc[p][d]);
+    }
+  }
+  float* sums = reinterpret_cast<float*>(smem);
+  __syncthreads();
+  Sum::put(sums, acc, wave, n, g);
+  __syncthreads();
+  TIO* dqb = reinterpret_cast<TIO*>(a.dq) + b * a.dqs[0] + h * a.dqs[1];
+  Sum::reduce(sums, tid, [&](int row, int d0, float* v) {
+    if (x0 + row >= a.Lq || d0 >= a.dk_) return;
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] *= a.sm_scale;
+    Io<TIO, CT>::store8(dqb + (x0 + row) * a.dqs[2] + d0 * a.dqs[3], v, a.dq_vec != 0, a.dqs[3], dlt_imin(8, a.dk_ - d0));
+  });
+}
+
+template <int DK, int DV, int NP, int NW>
+constexpr int flashs_lds_kv() {
+  const int tiles = NW * (FlashsTile<DK>::BYTES + FlashsTile<DV>::BYTES + 256);
+  const int sk = FlashsSum<DK, NP, NW>::BYTES, sv = FlashsSum<DV, NP, NW>::BYTES;
+  return tiles > sk ? (tiles > sv ? tiles : sv) : (sk > sv ? sk : sv);
+}
+
+// dK / dV: own = keys, the waves split the queries
+template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
+__global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const FlashBwdArgs a) {
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16, VB = DV / 16;
+  typedef FlashsTile<DK> QT;
+  typedef FlashsTile<DV> DT;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bh, x0;
+  flashs_block(a.nblk_k, 16 * NP, bh, x0);
+  const int b = bh / a.H, h = bh - b * a.H;
+  const TIO* kb_ = reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1];
+  const TIO* vb_ = reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1];
+  const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1]);
+  const char* dob = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1]);
+  // lanes 0 ... 31 fetch lse2, lanes 32 ... 63 delta of a block's queries
+  const float* scb = (lane < 32 ? a.lse : a.delta) + b * a.ls[0] + h * a.ls[1];
+  const int qsn = (int)a.qs[2] * 2, dosn = (int)a.dos[2] * 2;
+  const int nqb = (a.Lq + 31) / 32;
+  char* sQ = smem + wave * (QT::BYTES + DT::BYTES + 256);
+  char* sD = sQ + QT::BYTES;
+  float* sc = reinterpret_cast<float*>(sD + DT::BYTES);
+
+  u32x4 qr[QT::NV], dr[DT::NV];
+  float scr = 0.f;
+  const int first = (CAUSAL ? x0 / 32 : 0) + wave;   // causal: queries below the first own key see none of the own keys
+  auto fetch = [&](int blk) {
+    QT::load(qr, qb, qsn, blk, a.Lq, a.dk_, lane);
+    DT::load(dr, dob, dosn, blk, a.Lq, a.dv_, lane);
+    scr = scb[dlt_imin(32 * blk + (lane & 31), a.Lq - 1) * a.ls[2]];
+  };
+  if (first < nqb) fetch(first);
+  RopeDev no_rope = RopeDev{};
+  u32x4 kf[NP][KC], vf[NP][VC];
+  f32x4 acc_k[NP][KB], acc_v[NP][VB];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const int x = x0 + 16 * p + n;
+    swa1_load_own<TIO, CT, DK>(kf[p], kb_, 1, a.dk_, x < a.Lk ? x * a.ks[2] : (int64_t)-1, g, no_rope, false);
+    swa1_load_own<TIO, CT, DV>(vf[p], vb_, 1, a.dv_, x < a.Lk ? x * a.vs[2] : (int64_t)-1, g, no_rope, false);
+    // negated: with the products started from delta the matrix pipe delivers -(dP - delta)
+#pragma unroll
+    for (int c = 0; c < VC; c++) {
+      vf[p][c].x ^= 0x80008000u; vf[p][c].y ^= 0x80008000u; vf[p][c].z ^= 0x80008000u; vf[p][c].w ^= 0x80008000u;
+    }
+#pragma unroll
+    for (int d = 0; d < KB; d++) acc_k[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < VB; d++) acc_v[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float scale = a.scale_log2;
+  for (int qbk = first; qbk < nqb; qbk += NW) {
+    QT::write(sQ, qr, lane);
+    DT::write(sD, dr, lane);
+    sc[lane] = scr;
+    if (qbk + NW < nqb) fetch(qbk + NW);
+    const bool tail = 32 * qbk + 32 > a.Lq || (CAUSAL && 32 * qbk < x0 + 16 * NP - 1);
+    float pr[NP][8], ds[NP][8];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++) {
+      u32x4 qa[KC], da[VC];
+#pragma unroll
+      for (int c = 0; c < KC; c++) qa[c] = QT::rows(sQ, mb, c, n, g);
+#pragma unroll
+      for (int c = 0; c < VC; c++) da[c] = DT::rows(sD, mb, c, n, g);
+      const f32x4 lq = *reinterpret_cast<const f32x4*>(sc + 16 * mb + 4 * g), dl = *reinterpret_cast<const f32x4*>(sc + 32 + 16 * mb + 4 * g);
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = dl;
+#pragma unroll
+        for (int c = 0; c < KC; c++) s = Mma<CT>::mfma(qa[c], kf[p][c], s);
+#pragma unroll
+        for (int c = 0; c < VC; c++) dp = Mma<CT>::mfma(da[c], vf[p][c], dp);
+        const int qmin = CAUSAL ? x0 + 16 * p + n : 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float pv = fast_exp2(fmaf(s[i], scale, -lq[i]));
+          if (tail) {
+            const int qi = 32 * qbk + 16 * mb + 4 * g + i;
+            pv = (qi >= qmin && qi < a.Lq) ? pv : 0.f;
+          }
+          pr[p][4 * mb + i] = pv;
+          ds[p][4 * mb + i] = -pv * dp[i];
+        }
+      }
+    }
+    u32x4 pb[NP], dsb[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      pb[p] = pack8<CT>(pr[p]);
+      dsb[p] = pack8<CT>(ds[p]);
+    }
+#pragma unroll
+    for (int d = 0; d < VB; d++) {
+      const u32x4 dt = DT::trans(sD, d, n, g);
+#pragma unroll
+      for (int p = 0; p < NP; p++) acc_v[p][d] = Mma<CT>::mfma(dt, pb[p], acc_v[p][d]);
+    }
+#pragma unroll
+    for (int d = 0; d < KB; d++) {
+      const u32x4 qt = QT::trans(sQ, d, n, g);
+#pragma unroll
+      for (int p = 0; p < NP; p++) acc_k[p][d] = Mma<CT>::mfma(qt, dsb[p], acc_k[p][d]);
+    }
+  }
+  float* sums = reinterpret_cast<float*>(smem);
+  __syncthreads();
+  FlashsSum<DK, NP, NW>::put(sums, acc_k, wave, n, g);
+  __syncthreads();
+  TIO* dkb = reinterpret_cast<TIO*>(a.dk) + b * a.dks[0] + h * a.dks[1];
+  FlashsSum<DK, NP, NW>::reduce(sums, tid, [&](int row, int d0, float* v) {
+    if (x0 + row >= a.Lk || d0 >= a.dk_) return;
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] *= a.sm_scale;
+    Io<TIO, CT>::store8(dkb + (x0 + row) * a.dks[2] + d0 * a.dks[3], v, a.dk_vec != 0, a.dks[3], dlt_imin(8, a.dk_ - d0));
+  });
+  __syncthreads();
+  FlashsSum<DV, NP, NW>::put(sums, acc_v, wave, n, g);
+  __syncthreads();
+  TIO* dvb = reinterpret_cast<TIO*>(a.dv) + b * a.dvs[0] + h * a.dvs[1];
+  FlashsSum<DV, NP, NW>::reduce(sums, tid, [&](int row, int d0, float* v) {
+    if (x0 + row >= a.Lk || d0 >= a.dv_) return;
+    Io<TIO, CT>::store8(dvb + (x0 + row) * a.dvs[2] + d0 * a.dvs[3], v, a.dv_vec != 0, a.dvs[3], dlt_imin(8, a.dv_ - d0));
+  });
+}

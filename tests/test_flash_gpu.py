@@ -310,3 +310,29 @@ def test_gradients_that_cancel_stay_zero_with_fp32_inputs():
     assert qg.grad.abs().max().item() <= 1e-4 and kg.grad.abs().max().item() <= 1e-3
     want = do.bfloat16().float().sum(dim=2, keepdim=True)        # dv = sum over the queries of the rounded dO
     assert (vg.grad.cpu() - want).abs().max().item() <= 1e-3 * want.abs().max().item()
+
+
+# calls whose own blocks do not fill the chip run on the kernels that split the streamed side over the waves of a workgroup:
+# fewer blocks than waves, remainders of 16 and of 32 tokens, one and two own blocks, every head-dim class, dims below a class
+@pytest.mark.parametrize("causal,Lq,Lk,dk,dv,B,H", [
+    (False, 1, 900, 64, 64, 1, 2), (False, 77, 1500, 64, 64, 1, 3), (False, 33, 255, 64, 128, 2, 2), (False, 16, 257, 128, 128, 1, 2), (False, 40, 31, 32, 32, 1, 2),
+    (False, 900, 17, 64, 64, 1, 2), (False, 1100, 40, 128, 128, 1, 2), (False, 130, 600, 80, 80, 1, 3), (False, 600, 100, 24, 16, 2, 2), (False, 1000, 1000, 64, 64, 1, 8),
+    (True, 1, 1, 64, 64, 1, 2), (True, 221, 221, 64, 64, 1, 4), (True, 255, 255, 128, 128, 1, 2), (True, 513, 513, 64, 128, 1, 2), (True, 97, 97, 40, 32, 1, 2),
+    (True, 1030, 1030, 32, 32, 1, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_streamed_side_split_over_waves(causal, Lq, Lk, dk, dv, B, H, dtype):
+    q, k, v, do = orc.make_qkv(Lq + 2 * Lk + dk, B, H, Lq, Lk, dk, dv, dtype)
+    scale = 1 / math.sqrt(dk)
+    o_w, dq_w, dk_w, dv_w = orc.flash_grads(q.float(), k.float(), v.float(), do.float(), causal, scale)
+    outs = []
+    for _ in range(2):
+        qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+        o = _fa().attention(qg, kg, vg, causal, scale)
+        o.backward(do.cuda())
+        outs.append((o.detach(), qg.grad, kg.grad, vg.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    assert (outs[0][0].float().cpu() - o_w).abs().max().item() <= 2e-2
+    errs = [_rel(g, w) for g, w in zip(outs[0][1:], (dq_w, dk_w, dv_w))]
+    assert max(errs) <= 5e-2, errs
+    _, M = _fa()._forward(q.cuda(), k.cuda(), v.cuda(), causal, scale)
+    assert (M.cpu() - orc.flash_lse2(q, k, scale, causal)).abs().max().item() <= 2e-2
