@@ -24,7 +24,7 @@ DLT_BF16, DLT_FP16, DLT_FP32 = 0, 1, 2
 _DTYPES = {torch.bfloat16: DLT_BF16, torch.float16: DLT_FP16, torch.float32: DLT_FP32}
 
 EXPORTS = (
-    "dlt_last_error", "dlt_version", "dlt_rope2d", "dlt_rope2d_pair", "dlt_rope_pe_mask",
+    "dlt_last_error", "dlt_version", "dlt_rope2d", "dlt_rope2d_copy", "dlt_rope2d_pair", "dlt_rope_pe_mask",
     "dlt_swa_fwd", "dlt_swa_bwd", "dlt_swa_neighbors", "dlt_flash_fwd", "dlt_flash_bwd",
     "dlt_timing_enable", "dlt_timing_collect", "dlt_debug_copy",
     "dlt_swa_fwd_image", "dlt_swa_bwd_image", "dlt_swa_image_offsets", "dlt_swa_fwd_rot", "dlt_swa_bwd_rot",
@@ -97,6 +97,8 @@ def _declare(lib) -> None:
     lib.dlt_version.restype = c_int
     lib.dlt_rope2d.restype = c_int
     lib.dlt_rope2d.argtypes = [c_void_p, P64, c_int64, c_int64, c_int64, POINTER(RopeDesc), c_int, c_int, c_void_p]
+    lib.dlt_rope2d_copy.restype = c_int
+    lib.dlt_rope2d_copy.argtypes = [c_void_p, P64, c_void_p, P64, c_int64, c_int64, c_int64, POINTER(RopeDesc), c_int, c_int, c_void_p]
     lib.dlt_rope2d_pair.restype = c_int
     lib.dlt_rope2d_pair.argtypes = [c_void_p, P64, c_int64, c_void_p, P64, c_int64, c_int64, c_int64,
                                     POINTER(RopeDesc), c_int, c_int, c_void_p]

@@ -397,13 +397,17 @@ variable_list RopeBackward::apply(variable_list&& grads) {
   at::AutoDispatchBelowADInplaceOrView below;
   const Rope rope = make_rope(idx.unpack(), row.unpack(), col.unpack());
   require_gpu(grads[0], rope.idx, rope.row, rope.col);
-  Tensor dx = grads[0].clone();
-  Rows r;
-  if (!rows_of(dx, r)) {
-    dx = dx.contiguous();
-    rows_of(dx, r);
+  Tensor dy = grads[0];
+  Rows rs, rd;
+  if (!rows_of(dy, rs)) {
+    dy = dy.contiguous();
+    rows_of(dy, rs);
   }
-  rotate_inplace(dx, r, rope, true);
+  c10::DeviceGuard guard(dy.device());
+  Tensor dx = empty(dy.sizes(), dy.scalar_type(), dy);
+  rows_of(dx, rd);
+  check_rc(dlt_rope2d_copy(dy.const_data_ptr(), rs.s, dx.mutable_data_ptr(), rd.s, rd.nb, dy.size(-2), dy.size(-1), &rope.d, 1, dtype_code(dy),
+                           stream_of(dy)));
   return {dx};
 }
 

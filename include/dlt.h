@@ -62,6 +62,11 @@ typedef struct {
 int dlt_rope2d(void* x, const int64_t x_strides[3], int64_t n_batch, int64_t n_tokens, int64_t n_dim,
                const dlt_rope_t* rope, int inverse, int dtype, void* stream);
 
+/* The same rotation out of place: dst[b, n, :] = rotate(src[b, n, :]), every element written (what the backward pass of
+ * RotaryPE2D computes from a clone of its gradient, src/fused_rope2d.py:150-168).  src and dst must not overlap. */
+int dlt_rope2d_copy(const void* src, const int64_t src_strides[3], void* dst, const int64_t dst_strides[3], int64_t n_batch,
+                    int64_t n_tokens, int64_t n_dim, const dlt_rope_t* rope, int inverse, int dtype, void* stream);
+
 /* The same rotation applied to two tensors (q and k of one attention call) in ONE launch;
  * both share idx/tables, N and C.  Replaces two back-to-back RotaryPE2D launches
  * (README.md:11 composition; src/fused_rope2d.py:197-201 called once per tensor). */

@@ -218,3 +218,29 @@ def test_bad_arguments_raise():
         fr._launch(x, idx, cs, cs, False)
     with pytest.raises(RuntimeError):
         fr._launch(x.cpu(), idx, cs, cs, False)
+
+
+@pytest.mark.parametrize("C,R", [(32, 8), (64, 8), (64, 16), (128, 16), (128, 32), (96, 8), (48, 8), (64, 4), (96, 24)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_module_backward_rotates_out_of_place(C, R, dtype):
+    """The backward pass writes a rotated copy of the gradient: chunk distances 1, 2 and 4, rows with and without dims behind
+    the rotated ones, and the layouts that take the element-wise kernel; B and H as one run of rows and apart."""
+    fr = _mods()
+    B, H, th, tw = 2, 3, 5, 7
+    N = th * tw
+    torch.manual_seed(C + R)
+    m = fr.FusedInplaceRotaryPositionEncoding2D(4 * R, th, tw).cuda()
+    idx = orc.make_rope_idx(4, th, tw, 0.2)
+    x, dy = torch.randn(B, H, N, C).to(dtype), torch.randn(B, H, N, C).to(dtype)
+    for apart in (False, True):
+        leaf = x.cuda().requires_grad_(True)
+        y_in = leaf.clone() if not apart else leaf.transpose(1, 2).contiguous().transpose(1, 2)
+        g = dy.cuda() if not apart else dy.cuda().transpose(1, 2).contiguous().transpose(1, 2)
+        y = m(y_in, idx.cuda())
+        (dx,) = torch.autograd.grad(y, (leaf,), g)
+        tabs = (m.row_buffer.cs_components.cpu(), m.col_buffer.cs_components.cpu())
+        want = orc.rope2d_ref(x.float(), idx, *tabs).to(dtype)
+        xg = x.float().requires_grad_(True)
+        (dx_w,) = torch.autograd.grad(orc.rope2d_ref(xg, idx, *tabs), (xg,), dy.float())
+        assert torch.equal(y.detach().cpu(), want)
+        assert torch.equal(dx.cpu(), dx_w.to(dtype))
