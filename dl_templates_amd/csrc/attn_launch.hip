@@ -507,42 +507,58 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   return p.dk == 32 ? dlt_swat_launch_32(a, p.dtype, bwd, (int)grid, stream) : dlt_swat_launch_64(a, p.dtype, bwd, (int)grid, stream);
 }
 
-// Which kernels a dense / causal pass runs on: 0 = the streamed side passes through LDS chunk by chunk (64 ... 256 own
-// tokens per workgroup), 1 / 2 = it is split over the waves of workgroups that own one or two blocks of 16 tokens
-// (csrc/flash_split_kernel.hpp).  Chunked workgroups win once they fill the chip; below that their time is a start and the
-// chunks of 64 streamed tokens one after the other, however few the workgroups.  The split ones take
+// Which kernels a dense / causal pass runs on:
+//   CHUNKED: the streamed side passes through LDS chunk by chunk, 32 own tokens per wave (64 ... 256 per workgroup);
+//   SLIM:    the same with 8 waves of 16 own tokens: half the work per wave and chunk, twice the workgroups;
+//   SPLIT1, SPLIT2: the streamed side is split over the waves of workgroups that own one or two blocks of 16 tokens
+//            (csrc/flash_split_kernel.hpp).
+// CHUNKED wins once its workgroups fill the chip.  Below that the time of a chunked pass is a start and the chunks of 64 streamed
+// tokens one after the other, however few the workgroups; the split ones take
 //     fixed + rounds over the CUs * (start and final sum of a workgroup + its 32-token blocks * time of a block on a CU).
 // The constants (us) are least-squares fits to launches of 32 ... 8192 tokens on either side and 4 ... 128 heads, dense and
-// causal; on those the rule picks the fastest of the three but for 0.4 % of the total time.
+// causal; on those the rule picks the fastest kernel but for 0.4 % of the total time.
 //   77 queries x 1500 keys, 16 heads, 64/64: forward 22 -> 10 us, dQ 24 -> 11; 482 keys x 5450 queries, 4 heads: dK/dV 86 -> 26
-struct FlashSplitCost { int own; float start, chunk, fixed1, wg1, block1, fixed2, wg2, block2; };   // own: tokens of a chunked workgroup
-int flash_split(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
+//   16 heads, 2048 x 2048: forward 64/128 46 -> 34 us, 128/128 55 -> 41 (SLIM)
+enum { FLASH_CHUNKED = 0, FLASH_SPLIT1 = 1, FLASH_SPLIT2 = 2, FLASH_SLIM = 3 };
+struct FlashCost { int own; float start, chunk, slim_start, slim_chunk, fixed1, wg1, block1, fixed2, wg2, block2; };   // own: tokens of a chunked workgroup
+int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
   constexpr float NONE = 1e9f;
-  static const FlashSplitCost COST[3][4] = {   // by pass (forward, dQ, dK/dV) and DimClass::id
-      {{128, 3.50f, .822f, 2.31f, 1.36f, .137f, 1.09f, 3.79f, .141f},    // 64/64
-       {256, 6.78f, 1.493f, .59f, 3.70f, .272f, 0.f, 5.81f, .322f},      // 128/128
-       {256, 6.06f, 1.272f, 1.53f, 2.57f, .174f, 0.f, 5.73f, .185f},     // 64/128
-       {128, 2.94f, .698f, 2.84f, .52f, .055f, 2.41f, 1.13f, .094f}},    // 32/32
-      {{128, 4.84f, .850f, 2.07f, 2.19f, .138f, .43f, 5.72f, .144f},
-       {128, 6.58f, 1.404f, .67f, 4.25f, .289f, NONE, NONE, NONE},
-       {128, 5.43f, 1.073f, .99f, 4.27f, .244f, NONE, NONE, NONE},
-       {128, 4.04f, .750f, 2.73f, .68f, .057f, 2.36f, 1.44f, .090f}},
-      {{128, 4.94f, 1.083f, 1.85f, 2.73f, .134f, 1.36f, 4.59f, .171f},
-       {64, 5.62f, 1.226f, 1.31f, 4.42f, .283f, NONE, NONE, NONE},
-       {128, 5.79f, 1.627f, 1.32f, 4.15f, .185f, NONE, NONE, NONE},
-       {128, 4.28f, 1.038f, 2.51f, 1.14f, .072f, 2.79f, 1.38f, .114f}}};
-  // From 1536 tokens on a causal slab gives the same bits whatever the number of slabs of the call (documented and tested):
-  // the choice must not depend on it there.
-  if (causal && own >= 1536) return 0;
-  const FlashSplitCost& c = COST[pass][dc.id];
+  static const FlashCost COST[3][4] = {   // by pass (forward, dQ, dK/dV) and DimClass::id
+      {{128, 3.50f, .822f, 2.60f, .730f, 2.31f, 1.36f, .137f, 1.09f, 3.79f, .141f},    // 64/64
+       {256, 6.78f, 1.493f, 2.40f, 1.125f, .59f, 3.70f, .272f, 0.f, 5.81f, .322f},     // 128/128
+       {256, 6.06f, 1.272f, 2.40f, .960f, 1.53f, 2.57f, .174f, 0.f, 5.73f, .185f},     // 64/128
+       {128, 2.94f, .698f, NONE, NONE, 2.84f, .52f, .055f, 2.41f, 1.13f, .094f}},      // 32/32
+      {{128, 4.84f, .850f, NONE, NONE, 2.07f, 2.19f, .138f, .43f, 5.72f, .144f},
+       {128, 6.58f, 1.404f, NONE, NONE, .67f, 4.25f, .289f, NONE, NONE, NONE},
+       {128, 5.43f, 1.073f, NONE, NONE, .99f, 4.27f, .244f, NONE, NONE, NONE},
+       {128, 4.04f, .750f, NONE, NONE, 2.73f, .68f, .057f, 2.36f, 1.44f, .090f}},
+      {{128, 4.94f, 1.083f, NONE, NONE, 1.85f, 2.73f, .134f, 1.36f, 4.59f, .171f},
+       {64, 5.62f, 1.226f, NONE, NONE, 1.31f, 4.42f, .283f, NONE, NONE, NONE},
+       {128, 5.79f, 1.627f, NONE, NONE, 1.32f, 4.15f, .185f, NONE, NONE, NONE},
+       {128, 4.28f, 1.038f, NONE, NONE, 2.51f, 1.14f, .072f, 2.79f, 1.38f, .114f}}};
+  const FlashCost& c = COST[pass][dc.id];
   const float cus = (float)dlt_device_cus();
-  if (bh * ((own + c.own - 1) / c.own) > (int64_t)cus) return 0;
-  float least = c.start + c.chunk * (float)((other + 63) / 64);
+  const auto wgs = [&](int n) { return (float)(bh * ((own + n - 1) / n)); };
+  // From 1536 tokens on a causal slab keeps to the kernels whose tests hold single slabs and whole calls to the same bits.
+  const bool free_order = !(causal && own >= 1536);
+  const float chunks = (float)((other + 63) / 64);
+  const bool spills = pass == 2 && causal && dc.id == 2;   // two own blocks per wave: dK/dV at 64/128 under a mask
+  int best = FLASH_CHUNKED;
+  float least = c.start + c.chunk * chunks;
+  if (wgs(128) > cus) {
+    // A CU has more than one slim workgroup.  Up to two of them run side by side, which still beats the chunked workgroups
+    // at 64/64 and where a mask makes the work uneven (32 heads, 2048 x 2048, causal: 64/128 52 -> 46 us, 128/128 60 -> 49)
+    if ((pass == 0 && c.slim_chunk < NONE && (causal || dc.id == 0)) || spills) return wgs(128) <= 2.f * cus ? FLASH_SLIM : FLASH_CHUNKED;
+    if (wgs(c.own) > cus) return FLASH_CHUNKED;
+  } else {
+    const float t = spills ? c.start + 0.65f * c.chunk * chunks : c.slim_start + c.slim_chunk * chunks;
+    if (t < least) { least = t; best = FLASH_SLIM; }
+  }
   // the pieces of a row that a head dim below its class does not have are not read
   const float blocks = (float)((other + 31) / 32) * ((float)dims / (float)(dc.DK + dc.DV));
-  int best = 0;
-  for (int np = 1; np <= 2; np++) {
-    const float rounds = (float)(bh * ((own + 16 * np - 1) / (16 * np))) / cus;
+  for (int np = 1; free_order && np <= 2; np++) {
+    float rounds = wgs(16 * np) / cus;
+    if (dc.DK + dc.DV > 128) rounds = 0.5f * (rounds + ceilf(rounds));   // one workgroup per CU: a started round is half a round
     // under a causal mask the workgroups of several rounds see about half of the other side
     const float seen = causal && rounds > 1.f ? 0.55f * blocks : blocks;
     const float t = (np == 1 ? c.fixed1 : c.fixed2) + (rounds > 1.f ? rounds : 1.f) * (np == 1 ? c.wg1 + c.block1 * seen : c.wg2 + c.block2 * seen);
@@ -563,6 +579,7 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   a.nblk = (a.Lq + own - 1) / own;
   a.causal = p.g.mode == DLT_GEOM_CAUSAL;
   a.causal_group = flash_causal_group(a.Lk, p.dk, p.dv);
+  a.slim = 0;
   a.tile = p.g.mode == DLT_GEOM_SWA;
   a.g = p.g;
   a.o_vec = tvec_ok(t.out_o, t.os, p.dv, 2);
@@ -572,8 +589,9 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   const int64_t grid = (int64_t)p.B * p.H * p.g.TR * a.nblk;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "flash forward: grid too large");
   if (p.g.mode != DLT_GEOM_SWA) {
-    const int np = flash_split(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0);
-    if (np != 0) switch (dc.id) {
+    const int np = flash_pick(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0);
+    a.slim = np == FLASH_SLIM;
+    if (np == FLASH_SPLIT1 || np == FLASH_SPLIT2) switch (dc.id) {
       case 0: return dlt_flashs_fwd_64_64(a, p.dtype, np, stream);
       case 1: return dlt_flashs_fwd_128_128(a, p.dtype, np, stream);
       case 3: return dlt_flashs_fwd_32_32(a, p.dtype, np, stream);
@@ -643,13 +661,14 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
   // each pass streams its other side through LDS or splits it over the waves, whichever suits its own shape
   const int64_t nbh = (int64_t)p.B * p.H;
   const bool seq = p.g.mode != DLT_GEOM_SWA;
-  const int np_q = seq ? flash_split(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0) : 0;
-  const int np_kv = seq ? flash_split(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0) : 0;
+  const int np_q = seq ? flash_pick(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0) : 0;
+  const int np_kv = seq ? flash_pick(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0) : 0;
+  a.slim = np_kv == FLASH_SLIM;
   int rc;
 #define DLT_FLASH_PASS(C)                                                                                                  \
-  rc = np_q != 0 ? dlt_flashs_bwd_q_##C(a, p.dtype, np_q, stream) : dlt_flash_launch_bwd_q_##C(a, p.dtype, (int)grid_q, stream); \
+  rc = np_q == FLASH_SPLIT1 || np_q == FLASH_SPLIT2 ? dlt_flashs_bwd_q_##C(a, p.dtype, np_q, stream) : dlt_flash_launch_bwd_q_##C(a, p.dtype, (int)grid_q, stream); \
   if (rc != DLT_OK) return rc;                                                                                             \
-  return np_kv != 0 ? dlt_flashs_bwd_kv_##C(a, p.dtype, np_kv, stream) : dlt_flash_launch_bwd_kv_##C(a, p.dtype, (int)grid_kv, stream)
+  return np_kv == FLASH_SPLIT1 || np_kv == FLASH_SPLIT2 ? dlt_flashs_bwd_kv_##C(a, p.dtype, np_kv, stream) : dlt_flash_launch_bwd_kv_##C(a, p.dtype, (int)grid_kv, stream)
   switch (dc.id) {
     case 0: DLT_FLASH_PASS(64_64);
     case 1: DLT_FLASH_PASS(128_128);

@@ -135,11 +135,12 @@ DLT_DEV void flashd_wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) 
 #define FLASHD_NBUF(dk, dv) ((dk) + (dv) > 192 ? 2 : 3)
 #endif
 constexpr int flashd_nbuf(int dk, int dv) { return FLASHD_NBUF(dk, dv); }
-// the same for 8-wave workgroups of the backward kernels (one per CU, 64-token chunks; measured slower than 4-wave
-// workgroups and not instantiated by default: FLASHD_BWD_NW in flash_inst.hpp)
-#ifndef FLASHD_NBUF8
-#define FLASHD_NBUF8 3
-#endif
+// the same for 8-wave workgroups: two in the forward kernel with two query blocks per wave (128-key chunks); with one own
+// block per wave (64-token chunks) as many as leave room for two workgroups per CU
+constexpr int flashd_bufs(int dk, int dv, int np, int nw) {
+  return nw == 4 ? flashd_nbuf(dk, dv) : np == 2 || dk + dv > 192 ? 2 : dk + dv > 128 ? 3 : 4;
+}
+constexpr int flashd_occ(int nw) { return nw == 4 ? 2 : 1; }   // waves per SIMD the register allocation aims for
 
 template <int DK, int DV, int CK>
 struct FlashDBuf {
@@ -152,7 +153,7 @@ struct FlashDBuf {
 
 // ---- dK / dV: own = keys; Q, dO, lse2 and delta stream.  Replaces _attn_bwd_dkdv (src/flash_attn.py:204-307).
 template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_bwd_kv_kernel(const FlashBwdArgs a) {
+__global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_bwd_kv_kernel
     std_.template issue<PAD>(dob, ad, c, buf + B::REG_A, wave);
     if (wave < 2) flashd_issue_scalars<CK>(scal_base, (int)a.ls[2], c, buf + B::REG_A + B::REG_B + wave * (CK * 4), lane);
   };
-  constexpr int NBUF = NW == 4 ? flashd_nbuf(DK, DV) : FLASHD_NBUF8, AHEAD = NBUF - 1;
+  constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;   // copies per wave and chunk (waves 0, 1: more)
   // head dims below the padded ones: the slots of the missing pieces are zeroed once, no copy writes them
 #pragma unroll
@@ -403,7 +404,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_bwd_kv_kernel
 // update per query block, then O^T += V^T P^T (NKB VB transposed operands) with the row sums from a ones-row product.
 // The reads of the second stream are already in flight while the softmax runs.
 template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_fwd_kernel(const FlashArgs a) {
+__global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(const FlashArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef typename TileOf<TIO>::type TL;
   typedef FlashDBuf<DK, DV, CK> B;
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_fwd_kernel(co
   constexpr int PO = DV * (int)sizeof(TL) + 16;
   constexpr int KC = DK / 32, VB = DV / 16, NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
-  constexpr int NBUF = NW == 4 ? flashd_nbuf(DK, DV) : 2, AHEAD = NBUF - 1;   // forward: 128-key chunks
+  constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;
 
   const int tid = threadIdx.x;
@@ -637,7 +638,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_fwd_kernel(co
 // delta pre-pass (:186-202).  Per 32-key block: per 16-key half KC pieces of K (S = K Q^T) and VC pieces of V
 // (dP = V dO^T), then KB transposed pieces of K (dQ^T += K^T dS).
 template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
+__global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
@@ -645,7 +646,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flashd_bwd_q_kernel(
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
   constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16, NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
-  constexpr int NBUF = NW == 4 ? flashd_nbuf(DK, DV) : FLASHD_NBUF8, AHEAD = NBUF - 1;
+  constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;
 
   const int tid = threadIdx.x;

@@ -38,6 +38,25 @@ inline bool flash_async_staging() {
 template <typename KernT>
 int flash_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
+template <typename TIO, int MODE, int NP, int CK, int NW>
+int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
+  // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
+  auto kern = (a.dk != DLT_DK || a.dv != DLT_DV) ? flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
+                                                 : flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
+  constexpr int own = 16 * NP * NW;
+  constexpr int tile = own * (DLT_DV * 2 + 16);
+  constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
+  constexpr int lds = bufs > tile ? bufs : tile;
+  const int rc = flash_set_lds(kern, lds);
+  if (rc != DLT_OK) return rc;
+  a.nblk = (a.Lq + own - 1) / own;
+  dlt_timing_before(DLT_K_FWD, stream);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk), dim3(64 * NW), lds, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("flash forward launch");
+  return DLT_OK;
+}
+
 template <typename TIO, int MODE>
 int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
@@ -45,23 +64,8 @@ int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
     // class and mode against the register-staged kernel: dense -2 % (64/64), -4 % (64/128), -7 % (128/128); causal -4 %
     // (64/64), -18 % (128/128); head dims below the class (80/80, 96/96): -18 % on the step.
     if (a.dk % 8 == 0 && a.dv % 8 == 0 && flash_async_staging()) {
-      constexpr int NP = FLASHD_FWD_NP, CK = FLASHD_FWD_CK(DLT_DK, DLT_DV), NW = FLASHD_FWD_NW(DLT_DK, DLT_DV);
-      // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
-      auto kern = (a.dk != DLT_DK || a.dv != DLT_DV) ? flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
-                                                     : flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
-      constexpr int own = 16 * NP * NW;
-      constexpr int tile = own * (DLT_DV * 2 + 16);
-      constexpr int bufs = (NW == 4 ? flashd_nbuf(DLT_DK, DLT_DV) : 2) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
-      constexpr int lds = bufs > tile ? bufs : tile;
-      const int rc = flash_set_lds(kern, lds);
-      if (rc != DLT_OK) return rc;
-      FlashArgs ad = a;
-      ad.nblk = (a.Lq + own - 1) / own;
-      dlt_timing_before(DLT_K_FWD, stream);
-      hipLaunchKernelGGL(kern, dim3(a.B * a.H * ad.nblk), dim3(64 * NW), lds, stream, ad);
-      dlt_timing_after(stream);
-      DLT_CHECK_LAUNCH("flash forward launch");
-      return DLT_OK;
+      if (a.slim) return flashd_launch_fwd<TIO, MODE, 1, 64, 8>(a, stream);
+      return flashd_launch_fwd<TIO, MODE, FLASHD_FWD_NP, FLASHD_FWD_CK(DLT_DK, DLT_DV), FLASHD_FWD_NW(DLT_DK, DLT_DV)>(a, stream);
     }
   }
   auto kern = flash_fwd_kernel<TIO, DLT_DK, DLT_DV, FLASH_NP, flash_ck_fwd(DLT_DK, DLT_DV), MODE>;
@@ -82,26 +86,49 @@ int flash_launch_fwd_t(const FlashArgs& a, int grid, hipStream_t stream) {
   return a.causal ? flash_launch_fwd_c<TIO, 1>(a, grid, stream) : flash_launch_fwd_c<TIO, 0>(a, grid, stream);
 }
 
+template <typename TIO, int MODE, int NP, int NW>
+int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
+  constexpr int CK = 64;
+  auto kern = (a.dk_ != DLT_DK || a.dv_ != DLT_DV) ? flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
+                                                   : flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
+  constexpr int own = 16 * NP * NW;
+  constexpr int tile = own * (DLT_DK * 2 + 16);
+  constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
+  constexpr int lds = bufs > tile ? bufs : tile;
+  const int rc = flash_set_lds(kern, lds);
+  if (rc != DLT_OK) return rc;
+  a.nblk_q = (a.Lq + own - 1) / own;
+  dlt_timing_before(DLT_K_BWD_Q, stream);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q), dim3(64 * NW), lds, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("flash dQ launch");
+  return DLT_OK;
+}
+
+template <typename TIO, int MODE, int NP, int NW>
+int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
+  constexpr int CK = 64;
+  auto kern = (a.dk_ != DLT_DK || a.dv_ != DLT_DV) ? flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
+                                                   : flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
+  constexpr int own = 16 * NP * NW;
+  constexpr int tile_k = own * (DLT_DK * 2 + 16), tile_v = own * (DLT_DV * 2 + 16);
+  constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF_KV;
+  constexpr int lds = bufs > tile_v ? (bufs > tile_k ? bufs : tile_k) : (tile_v > tile_k ? tile_v : tile_k);
+  const int rc = flash_set_lds(kern, lds);
+  if (rc != DLT_OK) return rc;
+  a.nblk_k = (a.Lk + own - 1) / own;
+  dlt_timing_before(DLT_K_BWD_KV, stream);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k), dim3(64 * NW), lds, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("flash dK/dV launch");
+  return DLT_OK;
+}
+
 template <typename TIO, int MODE>
 int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && flash_async_staging()) {
-      constexpr int NP = FLASHD_DQ_NP(DLT_DK, DLT_DV), CK = 64, NW = FLASHD_BWD_NW;
-      auto kern = (a.dk_ != DLT_DK || a.dv_ != DLT_DV) ? flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
-                                                       : flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
-      constexpr int own = 16 * NP * NW;
-      constexpr int tile = own * (DLT_DK * 2 + 16);
-      constexpr int bufs = (NW == 4 ? flashd_nbuf(DLT_DK, DLT_DV) : FLASHD_NBUF8) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
-      constexpr int lds = bufs > tile ? bufs : tile;
-      int rc = flash_set_lds(kern, lds);
-      if (rc != DLT_OK) return rc;
-      FlashBwdArgs ad = a;
-      ad.nblk_q = (a.Lq + own - 1) / own;
-      dlt_timing_before(DLT_K_BWD_Q, stream);
-      hipLaunchKernelGGL(kern, dim3(a.B * a.H * ad.nblk_q), dim3(64 * NW), lds, stream, ad);
-      dlt_timing_after(stream);
-      DLT_CHECK_LAUNCH("flash dQ launch");
-      return DLT_OK;
+      return flashd_launch_bwd_q<TIO, MODE, FLASHD_DQ_NP(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }
   auto kern = flash_bwd_q_kernel<TIO, DLT_DK, DLT_DV, flash_np_q(DLT_DK, DLT_DV), flash_ck_q(DLT_DK, DLT_DV), MODE>;
@@ -121,22 +148,10 @@ int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream
     // where whole blocks are skipped, the register-staged kernel measured 1.5 % faster)
     const bool scalars_fit = a.ls[2] >= 0 && ((int64_t)a.Lq - 1) * a.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1);   // 32-bit offsets of the lse2 / delta copies
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && scalars_fit && flash_async_staging()) {
-      constexpr int NP = flash_np_kv(DLT_DK, DLT_DV), CK = 64, NW = FLASHD_BWD_NW;
-      auto kern = (a.dk_ != DLT_DK || a.dv_ != DLT_DV) ? flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
-                                                       : flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
-      constexpr int own = 16 * NP * NW;
-      constexpr int tile_k = own * (DLT_DK * 2 + 16), tile_v = own * (DLT_DV * 2 + 16);
-      constexpr int bufs = (NW == 4 ? flashd_nbuf(DLT_DK, DLT_DV) : FLASHD_NBUF8) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF_KV;
-      constexpr int lds = bufs > tile_v ? (bufs > tile_k ? bufs : tile_k) : (tile_v > tile_k ? tile_v : tile_k);
-      int rc = flash_set_lds(kern, lds);
-      if (rc != DLT_OK) return rc;
-      FlashBwdArgs ad = a;
-      ad.nblk_k = (a.Lk + own - 1) / own;
-      dlt_timing_before(DLT_K_BWD_KV, stream);
-      hipLaunchKernelGGL(kern, dim3(a.B * a.H * ad.nblk_k), dim3(64 * NW), lds, stream, ad);
-      dlt_timing_after(stream);
-      DLT_CHECK_LAUNCH("flash dK/dV launch");
-      return DLT_OK;
+      // under a causal mask two own blocks per wave spill at 64/128
+      if constexpr (MODE == 1 && DLT_DK == 64 && DLT_DV == 128)
+        if (a.slim) return flashd_launch_bwd_kv<TIO, MODE, 1, 8>(a, stream);
+      return flashd_launch_bwd_kv<TIO, MODE, flash_np_kv(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }
   {

@@ -227,6 +227,7 @@ struct FlashArgs {
   int32_t B, H, Lq, Lk, dk, dv;
   int32_t nblk;       // workgroups per (batch, head) and grid row
   int32_t causal, causal_group;   // causal_group: see flash_block_causal
+  int32_t slim;       // host only: 8 waves of one own block each (flash_launch_fwd_c)
   int32_t tile;       // MODE 2: Lq = Lk = tokens per grid row, geometry in g
   DltGeom g;
   int32_t o_vec;
@@ -521,6 +522,7 @@ struct FlashBwdArgs {
   int32_t B, H, Lq, Lk, dk_, dv_;
   int32_t nblk_q, nblk_k;
   int32_t causal, causal_group;   // causal_group: see flash_block_causal
+  int32_t slim;                   // host only: dK/dV on 8 waves of one own block each
   int32_t tile;
   DltGeom g;
   int32_t dq_vec, dk_vec, dv_vec;

@@ -318,7 +318,10 @@ def test_gradients_that_cancel_stay_zero_with_fp32_inputs():
     (False, 1, 900, 64, 64, 1, 2), (False, 77, 1500, 64, 64, 1, 3), (False, 33, 255, 64, 128, 2, 2), (False, 16, 257, 128, 128, 1, 2), (False, 40, 31, 32, 32, 1, 2),
     (False, 900, 17, 64, 64, 1, 2), (False, 1100, 40, 128, 128, 1, 2), (False, 130, 600, 80, 80, 1, 3), (False, 600, 100, 24, 16, 2, 2), (False, 1000, 1000, 64, 64, 1, 8),
     (True, 1, 1, 64, 64, 1, 2), (True, 221, 221, 64, 64, 1, 4), (True, 255, 255, 128, 128, 1, 2), (True, 513, 513, 64, 128, 1, 2), (True, 97, 97, 40, 32, 1, 2),
-    (True, 1030, 1030, 32, 32, 1, 8)])
+    (True, 1030, 1030, 32, 32, 1, 8),
+    # 8 waves of one own block (slim) and, with slabs that fill the chip, two own blocks per wave: chunk and block remainders
+    (False, 300, 193, 64, 128, 2, 40), (True, 270, 270, 128, 128, 2, 40), (True, 257, 257, 64, 128, 2, 50), (False, 129, 65, 64, 128, 4, 70),
+    (False, 257, 63, 128, 128, 3, 90), (True, 130, 130, 64, 64, 5, 110), (False, 40, 127, 80, 80, 4, 70), (True, 150, 150, 128, 128, 6, 90)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_streamed_side_split_over_waves(causal, Lq, Lk, dk, dv, B, H, dtype):
     q, k, v, do = orc.make_qkv(Lq + 2 * Lk + dk, B, H, Lq, Lk, dk, dv, dtype)
