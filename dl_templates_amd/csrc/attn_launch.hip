@@ -5,9 +5,9 @@
 #include "swa1_fwd_kernel.hpp"
 #include "swa1_bwd_kernel.hpp"
 #include "flash_kernel.hpp"
-#include "swam_bwd_kernel.hpp"
 #include "swa2_bwd_kernel.hpp"
 #include "swat_kernel.hpp"
+#include "swag_kernel.hpp"
 
 int dlt_launch_fwd_32_32(const FwdArgs&, int, int, hipStream_t);
 int dlt_launch_fwd_64_64(const FwdArgs&, int, int, hipStream_t);
@@ -45,6 +45,12 @@ int dlt_flashs_bwd_kv_64_128(const FlashBwdArgs&, int dtype, int np, hipStream_t
 int dlt_flashs_fwd_128_128(const FlashArgs&, int dtype, int np, hipStream_t);
 int dlt_flashs_bwd_q_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
 int dlt_flashs_bwd_kv_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_swag_launch_32_2(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_32_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_32_4(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_64_2(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_64_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_64_4(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swat_launch_32(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_swat_launch_64(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_launch_delta_32_32(const BwdArgs&, hipStream_t);
@@ -56,8 +62,6 @@ int dlt_swa1_launch_bwd_64(const Swa1BwdArgs&, int, int, int, int, hipStream_t);
 int dlt_swa1_launch_bwd_128(const Swa1BwdArgs&, int, int, int, int, hipStream_t);
 int dlt_swa1_launch_fwd_64(const Swa1FwdArgs&, int, int, hipStream_t);
 int dlt_swa1_launch_fwd_128(const Swa1FwdArgs&, int, int, hipStream_t);
-int dlt_swam_launch_fwd(const SwamFwdArgs&, int, int, hipStream_t);
-int dlt_swam_launch_bwd(const SwamBwdArgs&, int, int, hipStream_t);
 int dlt_swa2_launch_fwd_64(const Swa2FwdArgs&, int, int, hipStream_t);
 int dlt_swa2_launch_bwd_64(const Swa2BwdArgs&, int, int, hipStream_t);
 int dlt_swa2_launch_fwd_128(const Swa2FwdArgs&, int, int, hipStream_t);
@@ -273,47 +277,6 @@ int swa1_forward(const AttnProblem& p, const AttnTensors& t, const Swa1Class& c,
                    : dlt_swa1_launch_fwd_128(a, c.wclass, (int)grid, stream);
 }
 
-// ---- marching token-grid kernels: head dim 64 exactly, windows up to 13 x 13, no rotation or R = 8 ----------
-bool swam_eligible(const AttnProblem& p, const Swa1Class& c) {
-  if (c.D != 64 || p.dk != 64 || p.dv != 64) return false;
-  if (p.g.WR > 6 || p.g.WC > 6) return false;
-  if (c.rope_mode != 0 && !(c.rope_mode == 2 && p.rope.R == 8)) return false;
-  return true;
-}
-
-// rows per workgroup: the longest band (fewest re-fetched halo rows) that still gives every CU a workgroup
-void swam_make_plan(const AttnProblem& p, SwamPlan& plan) {
-  plan.nstrips = (p.g.TC + 15) / 16;
-  const int steps = (p.g.TR + 7) / 8;
-  const int64_t cols = (int64_t)p.B * p.H * plan.nstrips;
-  const int gpu_cus = dlt_device_cus();
-  int ns = 1;
-  for (int cand = 2; cand <= 8 && cand <= steps; cand++)
-    if (cols * ((steps + cand - 1) / cand) >= gpu_cus) ns = cand;
-  plan.band = 8 * ns;
-  plan.nbands = (steps + ns - 1) / ns;
-  dlt_fastdiv_make((uint32_t)(plan.nbands * plan.nstrips), plan.m_bh, plan.s_bh);
-  dlt_fastdiv_make((uint32_t)plan.nstrips, plan.m_st, plan.s_st);
-  dlt_fastdiv_make((uint32_t)p.H, plan.m_h, plan.s_h);
-}
-
-int swam_forward(const AttnProblem& p, const AttnTensors& t, const Swa1Class& c, hipStream_t stream) {
-  if (dlt_route_note(DLT_FAMILY_MARCHING)) return DLT_OK;
-  SwamFwdArgs a;
-  a.p = p;
-  swam_make_plan(p, a.plan);
-  a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.out_o; a.lse = t.lse;
-  for (int i = 0; i < 4; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; }
-  for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];
-  a.q_rot = c.rope_mode != 0 ? t.q_rot : nullptr;
-  a.k_rot = c.rope_mode != 0 ? t.k_rot : nullptr;
-  for (int i = 0; i < 4; i++) { a.qrs[i] = t.qrs[i]; a.krs[i] = t.krs[i]; }
-  a.scale_log2 = p.sm_scale * 1.4426950408889634f;
-  const int64_t grid = (int64_t)p.B * p.H * a.plan.nbands * a.plan.nstrips;
-  if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention forward: grid too large");
-  return dlt_swam_launch_fwd(a, c.rope_mode != 0, (int)grid, stream);
-}
-
 // ---- streaming kernels: head dim 64 or 128 exactly, no rotation, windows up to 21 columns ---------------------------
 bool swa2_eligible(const AttnProblem& p, const Swa1Class& c) {
   return (c.D == 64 || c.D == 128) && p.dk == c.D && p.dv == c.D && c.rope_mode == 0;
@@ -410,28 +373,69 @@ int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream
   return p.dk == 64 ? dlt_swa2_launch_bwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_bwd_128(a, swa2_ncg(p), (int)grid, stream);
 }
 
-// backward on the marching kernels: plain inputs, or rotated inputs with the gradients rotated back on store
-int swam_backward(const AttnProblem& p, const AttnTensors& t, bool rot, hipStream_t stream) {
+// ---- marching token-grid kernels: head dim 32 or 64 exactly, windows up to 13 x 13, by window class ----------------------
+int swag_class(int w) { return w <= 2 ? 2 : (4 + 2 * w + 3) / 4; }   // 4-wide blocks a patch's window spans
+bool swag_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
+  return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && ((int64_t)p.g.TR * p.g.TC - 1) * st[2] * 2 + 2 * p.dk <= (((int64_t)1 << 31) - 1);
+}
+bool swag_eligible(const AttnProblem& p, const AttnTensors& t, const Swa1Class& c, bool bwd) {
+  // rotation: 8 pairs per axis at head dim 64 in the forward pass, gradients turned back where q and k arrive rotated
+  if (c.rope_mode != 0 && !(p.dk == 64 && p.rope.R == 8 && (!bwd || p.rope_prerot))) return false;
+  if (p.dk != p.dv || (p.dk != 32 && p.dk != 64) || p.g.WR > 6 || p.g.WC > 6) return false;
+  if (!swag_rows_ok(p, t.q, t.qs) || !swag_rows_ok(p, t.k, t.ks) || !swag_rows_ok(p, t.v, t.vs)) return false;
+  if (!bwd)
+    return swag_rows_ok(p, t.out_o, t.os) && (t.q_rot == nullptr || (swag_rows_ok(p, t.q_rot, t.qrs) && swag_rows_ok(p, t.k_rot, t.krs)));
+  return swag_rows_ok(p, t.o, t.os) && swag_rows_ok(p, t.d_o, t.dos) && swag_rows_ok(p, t.dq, t.dqs) && swag_rows_ok(p, t.dk, t.dks) &&
+         swag_rows_ok(p, t.dv, t.dvs);
+}
+
+int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t stream) {
   if (dlt_route_note(DLT_FAMILY_MARCHING)) return DLT_OK;
-  SwamBwdArgs a;
-  a.p = p;
-  swam_make_plan(p, a.plan);
-  a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.o; a.d_o = t.d_o; a.lse = t.lse; a.delta = t.delta;
-  a.dq = t.dq; a.dk = t.dk; a.dv = t.dv;
+  SwagArgs a;
+  a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.o; a.d_o = t.d_o; a.out_o = t.out_o; a.dq = t.dq; a.dk = t.dk; a.dv = t.dv;
+  a.lse = t.lse; a.delta = t.delta;
   for (int i = 0; i < 4; i++) {
     a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; a.dos[i] = t.dos[i];
     a.dqs[i] = t.dqs[i]; a.dks[i] = t.dks[i]; a.dvs[i] = t.dvs[i];
   }
   for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];
+  a.g = p.g; a.B = p.B; a.H = p.H;
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
-  const int64_t grid = (int64_t)p.B * p.H * a.plan.nbands * a.plan.nstrips;
-  if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention backward: grid too large");
-  return dlt_swam_launch_bwd(a, rot, (int)grid, stream);
-}
-
-// 16-byte row pieces and 32-bit byte offsets inside a (batch, head) slab of head dim 64
-bool swam_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
-  return tvec_ok(ptr, st, 64, 2) && st[2] >= 0 && ((int64_t)p.g.TR * p.g.TC - 1) * st[2] * 2 + 128 <= (((int64_t)1 << 31) - 1);
+  a.sm_scale = p.sm_scale;
+  a.rope = p.rope;
+  a.rope.enabled = p.rope.enabled && p.rope.R > 0;
+  a.q_rot = t.q_rot; a.k_rot = t.k_rot;
+  for (int i = 0; i < 4; i++) { a.qrs[i] = t.qrs[i]; a.krs[i] = t.krs[i]; }
+  const int nch = swag_class(p.g.WR), ncg = swag_class(p.g.WC);
+  constexpr int pc = SWAG_PC, step = 4 * (8 / pc);
+  a.nstrips = (p.g.TC + 4 * pc - 1) / (4 * pc);
+  // Rows per workgroup: a band costs its steps plus a prologue that fills the ring (about two steps); workgroups beyond what the
+  // chip holds at once (one or two per CU) wait for a whole band.
+  const int nres = nch + 8 / pc - 1, tok = 4 * (4 * pc + 4 * (ncg - 1)), lds = nres * tok * (4 * p.dk + 8);
+  const int64_t slots = (int64_t)dlt_device_cus() * (lds <= 80 * 1024 ? 2 : 1);
+  const int64_t cols = (int64_t)p.B * p.H * a.nstrips;
+  const int steps = (p.g.TR + step - 1) / step;
+  int64_t best = -1;
+  for (int nb = 1; nb <= steps; nb++) {
+    const int per = (steps + nb - 1) / nb;
+    if ((steps + per - 1) / per != nb) continue;
+    const int64_t cost = (cols * nb + slots - 1) / slots * (per + 2);
+    if (best < 0 || cost < best) { best = cost; a.band = per * step; a.nbands = nb; }
+  }
+  const int64_t grid = cols * a.nbands;
+  if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
+  if (p.dk == 32) {
+    switch (nch) {
+      case 2: return dlt_swag_launch_32_2(a, p.dtype, ncg, bwd, (int)grid, stream);
+      case 3: return dlt_swag_launch_32_3(a, p.dtype, ncg, bwd, (int)grid, stream);
+      default: return dlt_swag_launch_32_4(a, p.dtype, ncg, bwd, (int)grid, stream);
+    }
+  }
+  switch (nch) {
+    case 2: return dlt_swag_launch_64_2(a, p.dtype, ncg, bwd, (int)grid, stream);
+    case 3: return dlt_swag_launch_64_3(a, p.dtype, ncg, bwd, (int)grid, stream);
+    default: return dlt_swag_launch_64_4(a, p.dtype, ncg, bwd, (int)grid, stream);
+  }
 }
 
 // ---- flash fast path: dense, causal, and sliding windows over tiles of 16 k tokens -----------
@@ -695,10 +699,7 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
       const bool side_ok = t.q_rot == nullptr || (c.rope_mode != 0 && tvec_ok(t.q_rot, t.qrs, p.dk, es) &&
                                                   tvec_ok(t.k_rot, t.krs, p.dk, es));
       if (side_ok) {
-        // the marching kernels store o in 16-byte pieces and address every tensor with 32-bit offsets
-        const bool rows_fit = swam_rows_ok(p, t.out_o, t.os) &&
-                              (t.q_rot == nullptr || (swam_rows_ok(p, t.q_rot, t.qrs) && swam_rows_ok(p, t.k_rot, t.krs)));
-        if (swam_eligible(p, c) && rows_fit) return swam_forward(p, t, c, stream);
+        if (swag_eligible(p, t, c, false)) return swag_run(p, t, false, stream);
         if (swa2_eligible(p, c) && t.q_rot == nullptr && swa2_rows_ok(p, t.out_o, t.os)) return swa2_forward(p, t, stream);
         // Rotation the marching kernels do not take, with the rotated q / k wanted by the caller: rotating both out of place
         // first (below) and running the streaming kernels on the result is faster than the tile kernels, which rotate every
@@ -767,12 +768,7 @@ int dlt_attn_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t st
                               tvec_ok(t.v, t.vs, p.dv, es), tvec_ok(t.d_o, t.dos, p.dv, es)};
     Swa1Class c;
     if (swa1_eligible(p, streamed, 4, c) && swa1_strides_fit(p, t)) {
-      Swa1Class cm = c;
-      if (p.rope_prerot && cm.rope_mode != 0) cm.rope_mode = 2;   // the marching kernels rotate dq / dk back on store
-      const bool plain_or_prerot = c.rope_mode == 0 || p.rope_prerot;
-      if (plain_or_prerot && swam_eligible(p, cm) && swam_rows_ok(p, t.o, t.os) && swam_rows_ok(p, t.dq, t.dqs) &&
-          swam_rows_ok(p, t.dk, t.dks) && swam_rows_ok(p, t.dv, t.dvs))
-        return swam_backward(p, t, c.rope_mode != 0, stream);
+      if (swag_eligible(p, t, c, true)) return swag_run(p, t, true, stream);
       // lse2 / delta rows are copied with 32-bit byte offsets inside a (batch, head) slab
       if (swa2_eligible(p, c) && swa2_rows_ok(p, t.o, t.os) && swa2_rows_ok(p, t.dq, t.dqs) && swa2_rows_ok(p, t.dk, t.dks) &&
           swa2_rows_ok(p, t.dv, t.dvs) && swa2_scalars_ok(p, t))

@@ -1,0 +1,805 @@
+// Marching kernels for token grids (b_size == 1) at head dims 32 and 64 and windows up to 13 x 13, with or without the fused
+// rotation (head dim 64, 8 rotary pairs per axis, rotated q / k kept): the shape of the benchmark's headline configuration.
+//
+// The window is a compile-time class: NCH x NCG blocks of 4 x 4 keys.  (An earlier version always computed 16 x 16 keys at head
+// dim 64, and head dim 32 ran zero-padded on the tile kernels, which stage every halo row once per band of 4 own rows: 32 slabs
+// of 84 x 82 tokens, d = 64, 11 x 7 window: forward 62 -> 35 us, dQ 79 -> 51, dK/dV 88 -> 53; 64 slabs of the same at d = 32:
+// 89 -> 42, 95 -> 50, 120 -> 56.)  A workgroup owns a strip of 4 PC columns and marches down the grid in steps of 4 PR rows
+// (PR = 8 / PC); wave w owns the 4 x 4 patch of column w % PC and row group w / PC.  The halo rows a step sees
+// (NCH + PR - 1 chunks of 4 rows, both streamed tensors) live in an LDS ring; the chunks of the next step travel HBM ->
+// registers while the current one computes.  The whole window is resident: the softmax is one-shot.
+//
+// In the C layout of a block lane group g holds key row g and element i key column i, lane n is own token (n >> 2, n & 3): the
+// row test enters as the C operand of the score products (0 or -inf), the column tests are lane masks that stay in scalar
+// registers for the whole march.
+//
+// LDS: token rows of 2 D bytes, 16-byte piece p of the token at halo row r, column c at p ^ swz(r, c), where the swizzle only
+// takes c & 3 and r & 1: operand reads and transposing reads are free of bank conflicts and their lane offsets are the same
+// for every block of the window.
+#pragma once
+#include "swat_kernel.hpp"
+
+struct SwagArgs {
+  const void *q, *k, *v, *o, *d_o;
+  void *out_o, *dq, *dk, *dv;
+  float* lse;
+  float* delta;
+  int64_t qs[4], ks[4], vs[4], os[4], dos[4], dqs[4], dks[4], dvs[4], ls[3];
+  DltGeom g;
+  int32_t B, H;
+  int32_t nstrips, band, nbands;   // band: grid rows per workgroup, a multiple of 4 PR
+  float scale_log2, sm_scale;
+  RopeDev rope;              // ROPE kernels: 8 rotary pairs per axis
+  void *q_rot, *k_rot;       // forward: where the rotated q and k go (NULL: nowhere)
+  int64_t qrs[4], krs[4];
+};
+
+// ---- fused rotation (D = 64, 8 rotary pairs per axis: the 16-byte pieces 0, 1 of a row turn by the row angle, 2, 3 by the
+// column angle) --------------------------------------------------------------------------------------------------------
+// Both tables (64 bytes per position) are copied into LDS once per workgroup when they fit: a table row is then four LDS reads
+// behind the arrival of the token's index instead of a dependent global load.
+constexpr int SWAG_TAB_BYTES = 8192;
+struct SwagTab {
+  swat_lds lds;
+  bool in_lds;
+  f32x4 part;   // the 16 bytes this thread copies
+  DLT_DEV void fetch(swat_lds at, const RopeDev& rope, int tid) {
+    lds = at;
+    in_lds = (rope.row_len + rope.col_len) * 64 <= SWAG_TAB_BYTES;
+    const int row = dlt_imin(tid >> 2, rope.row_len + rope.col_len - 1);   // 128 rows of four 16-byte parts
+    const float* p = (row < rope.row_len ? rope.row_cs + (int64_t)row * rope.rs0 : rope.col_cs + (int64_t)(row - rope.row_len) * rope.cs0) + 4 * (tid & 3);
+    part = f32x4{p[0], p[1], p[2], p[3]};
+  }
+  DLT_DEV void store(int tid) const { if (in_lds) *reinterpret_cast<DLT_LDS f32x4*>(lds + 16 * tid) = part; }
+  // NF pairs of (cos, sin) from pair `first` on; false: the axis is not rotated
+  template <int NV4>
+  DLT_DEV bool get(f32x4 (&t)[NV4], int32_t id, int axis, int first, const RopeDev& rope) const {
+    int pos = axis == 0 ? dlt_rope_row(id) : dlt_rope_col(id);
+    const bool rotated = pos >= 0;
+    pos = dlt_imax(0, dlt_imin(pos, (axis == 0 ? rope.row_len : rope.col_len) - 1));
+    if (in_lds) {
+      swat_lds p = lds + ((axis == 0 ? 0 : rope.row_len) + pos) * 64 + 8 * first;
+#pragma unroll
+      for (int j = 0; j < NV4; j++) t[j] = *reinterpret_cast<DLT_LDS f32x4*>(p + 16 * j);
+    } else {
+      const float* p = (axis == 0 ? rope.row_cs + (int64_t)pos * rope.rs0 : rope.col_cs + (int64_t)pos * rope.cs0) + 2 * first;
+#pragma unroll
+      for (int j = 0; j < NV4; j++) t[j] = f32x4{p[4 * j], p[4 * j + 1], p[4 * j + 2], p[4 * j + 3]};
+    }
+    return rotated;
+  }
+};
+
+// one 16-byte piece turned with its partner piece: the arithmetic of the standalone rotation (every product rounded)
+template <typename CT>
+DLT_DEV u32x4 swag_turn(u32x4 self, u32x4 partner, const f32x4 (&t)[4], bool is_x0) {
+  float x[8], y[8];
+  unpack8<CT>(self, x);
+  unpack8<CT>(partner, y);
+  const unsigned sm = rope_sign_mask(is_x0, false);
+#pragma unroll
+  for (int j = 0; j < 8; j++) x[j] = rope_mix_signed(x[j], y[j], t[j >> 1][2 * (j & 1)], t[j >> 1][2 * (j & 1) + 1], sm);
+  return pack8<CT>(x);
+}
+DLT_DEV unsigned swag_lane_xor16(unsigned v, int g) {
+  typedef unsigned pair_t __attribute__((ext_vector_type(2)));
+  const pair_t r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return (g & 1) ? r.x : r.y;
+}
+DLT_DEV float swag_lane_xor32(float v, int g) {
+  typedef unsigned pair_t __attribute__((ext_vector_type(2)));
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const pair_t r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)(g < 2 ? r.y : r.x));
+}
+// Gradient rows (C layout) of rotated q or k -> of the caller's: rounded to the element type first (as the composition of the
+// plain operator and the rotation does), then blocks 0 (row axis) and 1 (column axis) turned back.  Lane group g holds dims
+// 4 g .. 4 g + 3 of a block, its rotary partners sit 32 lanes away; t[axis]: the pairs 4 (g & 1) .. + 3.
+template <typename CT>
+DLT_DEV void swag_turn_back(f32x4 (&acc)[4], float mul, const f32x4 (&t)[2][2], const bool (&rot)[2], int g) {
+#pragma unroll
+  for (int ax = 0; ax < 2; ax++) {
+    const unsigned sm = rope_sign_mask(g < 2, true);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float x = (float)(CT)(acc[ax][i] * mul), y = swag_lane_xor32(x, g);
+      const float z = rope_mix_signed(x, y, t[ax][i >> 1][2 * (i & 1)], t[ax][i >> 1][2 * (i & 1) + 1], sm);
+      acc[ax][i] = rot[ax] ? z : x;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[2 + ax][i] *= mul;
+  }
+}
+
+template <int D, int NCH, int NCG, int PC>
+struct Swag {
+  static constexpr int STRIP = 4 * PC;                                 // own columns of a workgroup
+  static constexpr int PR = 8 / PC, NRES = NCH + PR - 1;               // row groups, resident chunks
+  static constexpr int NB = NCH * NCG, NP = (NB + 1) / 2;              // 4 x 4 key blocks of a window, pairs of them
+  static constexpr int HCW = 4 * PC + 4 * (NCG - 1), TOK = 4 * HCW;    // staged columns, tokens of a chunk
+  static constexpr int ROWB = 2 * D, TB = TOK * ROWB, SLOT = 2 * TB;
+  static constexpr int PIECES = D / 8, NV = 2 * TOK * PIECES, NIT = (NV + 511) / 512;
+  static constexpr int KC = D / 32, DB = D / 16;
+  static constexpr int RING = NRES * SLOT, SCAL = NRES * 2 * TOK * 4;
+  // waves per SIMD: two workgroups per CU where two rings and the registers fit
+  static constexpr int OCC = RING + SCAL <= 80 * 1024 ? 4 : 2, OCC_BWD = D == 32 ? OCC : 2;
+  static_assert((TOK * PIECES) % 64 == 0, "a wave stages one tensor per vector");
+  static_assert(RING + SCAL <= 160 * 1024, "the ring exceeds the LDS");
+};
+
+// patch columns per workgroup: strips of 16 columns (strips of 32 with one row group per step stage fewer halo columns, but
+// measured within 3 % on large grids and up to 18 % slower where the grid's width is no multiple of 32)
+constexpr int SWAG_PC = 4;
+
+template <int D> DLT_DEV int swag_swz(int row, int col) { return D == 32 ? (row & 1) << 1 : (col & 3) | ((row & 1) << 2); }
+
+struct SwagWho { int b, h, r0, r1, c0; };
+DLT_DEV SwagWho swag_who(const SwagArgs& a, int strip) {
+  int lin = xcd_remap(blockIdx.x, gridDim.x);
+  SwagWho w;
+  const int s = lin % a.nstrips; lin /= a.nstrips;
+  const int bd = lin % a.nbands; lin /= a.nbands;
+  w.h = lin % a.H;
+  w.b = lin / a.H;
+  w.c0 = s * strip;
+  w.r0 = bd * a.band;
+  w.r1 = dlt_imin(w.r0 + a.band, a.g.TR);
+  return w;
+}
+
+template <typename C>
+struct SwagRing {
+  swat_lds lds;
+  const char *base0, *base1;
+  uint32_t rs0, rs1;                  // bytes between grid rows
+  uint32_t goff[C::NIT];              // offset inside a grid row
+  int hrow[C::NIT], loff[C::NIT];     // halo row inside a chunk; LDS offset inside a slot
+  bool second[C::NIT];                // wave-uniform
+  int tid, TR;
+
+  DLT_DEV void init(swat_lds lds_, const char* b0, int sn0, const char* b1, int sn1, const SwagArgs& a, int c0, int tid_, int wave) {
+    lds = lds_; base0 = b0; base1 = b1; tid = tid_; TR = a.g.TR;
+    const int TC = a.g.TC;
+    rs0 = (uint32_t)(TC * sn0 * 2);
+    rs1 = (uint32_t)(TC * sn1 * 2);
+#pragma unroll
+    for (int it = 0; it < C::NIT; it++) {
+      const int id = tid + 512 * it;
+      second[it] = 64 * wave + 512 * it >= C::NV / 2;
+      const int v = second[it] ? id - C::NV / 2 : id;
+      const int tok = v / C::PIECES, piece = v % C::PIECES;
+      hrow[it] = tok / C::HCW;
+      const int hc = tok - hrow[it] * C::HCW;
+      // columns outside the grid are clamped onto it: the window tests drop them
+      const int col = dlt_imax(0, dlt_imin(c0 - a.g.WC + hc, TC - 1));
+      goff[it] = (uint32_t)(col * (second[it] ? sn1 : sn0) * 2) + 16 * piece;
+      loff[it] = (second[it] ? C::TB : 0) + tok * C::ROWB + 16 * (piece ^ swag_swz<C::ROWB / 2>(hrow[it], hc));
+    }
+  }
+  DLT_DEV bool has(int it) const { return C::NV % 512 == 0 || it + 1 < C::NIT || tid + 512 * it < C::NV; }
+  // first: grid row of the chunk's first halo row (rows outside the grid are clamped onto it)
+  DLT_DEV void issue(u32x4 (&r)[C::NIT], int first) const {
+#pragma unroll
+    for (int it = 0; it < C::NIT; it++)
+      if (has(it)) {
+        const uint32_t rc = (uint32_t)dlt_imax(0, dlt_imin(first + hrow[it], TR - 1));
+        r[it] = *reinterpret_cast<const u32x4*>((second[it] ? base1 : base0) + (goff[it] + rc * (second[it] ? rs1 : rs0)));
+      }
+  }
+  DLT_DEV void commit(const u32x4 (&r)[C::NIT], int slot) const {
+#pragma unroll
+    for (int it = 0; it < C::NIT; it++)
+      if (has(it)) swat_write16(lds + slot * C::SLOT + loff[it], r[it]);
+  }
+  // chunks of the first step: all requested before the first is written
+  DLT_DEV void fill(int first) const {
+    u32x4 pre[C::NRES][C::NIT];
+#pragma unroll
+    for (int i = 0; i < C::NRES; i++) issue(pre[i], first + 4 * i);
+#pragma unroll
+    for (int i = 0; i < C::NRES; i++) commit(pre[i], i);
+  }
+};
+
+// The ring of the rotating forward kernel: G chunks at a time.  A K item is half of a token row, pieces (2 h, 2 h + 1) = the
+// rotary pair of axis h and (4 + 2 h, 5 + 2 h): a thread turns both partners of its pair with one read of the table row, and the
+// K items of the two chunks a step brings in fill 320 ... 448 of the 512 threads.
+template <typename C, int G>
+struct SwagTurnStage {
+  static constexpr int NK = (G * C::TOK * 2 + 511) / 512, NVV = (G * C::TOK * 8 + 511) / 512;
+  u32x4 k[NK][4], v[NVV];
+  int32_t id[NK];
+  struct At { bool on; int chunk, hr, hc; };
+  static DLT_DEV At at(int i, int per_tok, int tid) {
+    const int x = tid + 512 * i;
+    At p;
+    p.on = x < G * C::TOK * per_tok;
+    p.chunk = x / (C::TOK * per_tok);
+    const int tok = (x - p.chunk * (C::TOK * per_tok)) / per_tok;
+    p.hr = tok / C::HCW;
+    p.hc = tok - p.hr * C::HCW;
+    return p;
+  }
+  // first: grid row of the first chunk's first halo row; chunk c starts 4 c rows further down
+  DLT_DEV void issue(const char* kb, int ksn, const char* vb, int vsn, const SwagArgs& a, int first, int c0, int tid) {
+    const int TC = a.g.TC;
+    auto tok_of = [&](const At& p) {
+      return dlt_imax(0, dlt_imin(first + 4 * p.chunk + p.hr, a.g.TR - 1)) * TC + dlt_imax(0, dlt_imin(c0 - a.g.WC + p.hc, TC - 1));
+    };
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+      const At p = at(i, 2, tid);
+      if (p.on) {
+        const int tok = tok_of(p);
+        id[i] = a.rope.idx[tok];
+        const char* q = kb + (uint32_t)(tok * ksn) + 32 * (tid & 1);
+        k[i][0] = *reinterpret_cast<const u32x4*>(q);
+        k[i][1] = *reinterpret_cast<const u32x4*>(q + 16);
+        k[i][2] = *reinterpret_cast<const u32x4*>(q + 64);
+        k[i][3] = *reinterpret_cast<const u32x4*>(q + 80);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NVV; i++) {
+      const At p = at(i, 8, tid);
+      if (p.on) v[i] = *reinterpret_cast<const u32x4*>(vb + (uint32_t)(tok_of(p) * vsn) + 16 * (tid & 7));
+    }
+  }
+  // the K pairs turned in registers; the workgroup's own tokens are also stored to `out` (NULL: nowhere)
+  template <typename CT>
+  DLT_DEV void turn(const SwagTab& tab, const SwagArgs& a, char* out, int sn2, int first, int r0, int r1, int c0, int tid) {
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+      const At p = at(i, 2, tid);
+      if (!p.on) continue;
+      f32x4 t[4];
+      if (tab.get(t, id[i], tid & 1, 0, a.rope)) {
+        const u32x4 x0 = k[i][0];
+        k[i][0] = swag_turn<CT>(x0, k[i][1], t, true);
+        k[i][1] = swag_turn<CT>(k[i][1], x0, t, false);
+      }
+      const int row = first + 4 * p.chunk + p.hr, col = c0 - a.g.WC + p.hc;
+      if (out != nullptr && row >= r0 && row < r1 && col >= c0 && col < c0 + C::STRIP && col < a.g.TC) {
+        char* q = out + (uint32_t)((row * a.g.TC + col) * sn2) + 32 * (tid & 1);
+        store_stream16(q, k[i][0]);
+        store_stream16(q + 16, k[i][1]);
+        store_stream16(q + 64, k[i][2]);
+        store_stream16(q + 80, k[i][3]);
+      }
+    }
+  }
+  DLT_DEV void commit(swat_lds lds, int slot0, int tid) const {
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+      const At p = at(i, 2, tid);
+      if (!p.on) continue;
+      const int s = slot0 + p.chunk, h = tid & 1, z = swag_swz<64>(p.hr, p.hc);
+      swat_lds d = lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + (p.hr * C::HCW + p.hc) * C::ROWB;
+      swat_write16(d + 16 * ((2 * h) ^ z), k[i][0]);
+      swat_write16(d + 16 * ((2 * h + 1) ^ z), k[i][1]);
+      swat_write16(d + 16 * ((4 + 2 * h) ^ z), k[i][2]);
+      swat_write16(d + 16 * ((5 + 2 * h) ^ z), k[i][3]);
+    }
+#pragma unroll
+    for (int i = 0; i < NVV; i++) {
+      const At p = at(i, 8, tid);
+      if (!p.on) continue;
+      const int s = slot0 + p.chunk;
+      swat_write16(lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + C::TB + (p.hr * C::HCW + p.hc) * C::ROWB + 16 * ((tid & 7) ^ swag_swz<64>(p.hr, p.hc)),
+                   v[i]);
+    }
+  }
+};
+
+// lane parts of the operand addresses of a 4 x 4 block
+template <typename C>
+struct SwagLane {
+  int row[C::KC], tr[C::DB];
+  DLT_DEV void init(int n, int g) {
+    constexpr int D = C::ROWB / 2;
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) row[c] = ((n >> 2) * C::HCW + (n & 3)) * C::ROWB + 16 * ((4 * c + g) ^ swag_swz<D>(n >> 2, n));
+#pragma unroll
+    for (int d = 0; d < C::DB; d++)
+      tr[d] = (g * C::HCW + (n >> 2)) * C::ROWB + 16 * ((2 * d + ((n >> 1) & 1)) ^ swag_swz<D>(g, n >> 2)) + 8 * (n & 1);
+  }
+};
+
+// Common frame of the three kernels: who the wave is and what its lanes own.
+template <typename C, int PC>
+struct SwagFrame {
+  int lane, n, g, wave, pc, rg;
+  SwagWho w;
+  int TR, TC, WR, WC;
+  int col;          // own column (unclamped)
+  int clo, chi;     // visible window columns of the own token
+  DLT_DEV void init(const SwagArgs& a, int tid) {
+    lane = tid & 63; n = lane & 15; g = lane >> 4;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    pc = wave % PC; rg = wave / PC;
+    w = swag_who(a, 4 * PC);
+    TR = a.g.TR; TC = a.g.TC; WR = a.g.WR; WC = a.g.WC;
+    const int cp = w.c0 + 4 * pc;
+    col = cp + (n & 3);
+    clo = dlt_imax(n & 3, WC - cp);
+    chi = dlt_imin((n & 3) + 2 * WC, TC - 1 - cp + WC);
+    if (col >= TC) chi = -1;
+  }
+  DLT_DEV bool sees_col(int j) const { return j >= clo && j <= chi; }
+  // C operand of the score products of key rows 4 i + g: 0 where the row is in the own token's window, else -inf
+  DLT_DEV float row_bias(int i, int rp) const {
+    const int hr = 4 * i + g, qr = n >> 2;
+    const int lo = dlt_imax(qr, WR - rp), hi = dlt_imin(qr + 2 * WR, TR - 1 - rp + WR);
+    return hr >= lo && hr <= hi ? 0.f : -INFINITY;
+  }
+  DLT_DEV int own_row(int rp) const { return rp + (n >> 2); }
+  DLT_DEV bool own_ok(int rp) const { return own_row(rp) < TR && col < TC; }
+  // clamped token index of the own token
+  DLT_DEV int own_tok(int rp) const { return dlt_imin(own_row(rp), TR - 1) * TC + dlt_imin(col, TC - 1); }
+};
+
+// scores of block (i, j): row tests through the C operand, column tests on the result
+template <typename C, typename CT>
+DLT_DEV f32x4 swag_scores(swat_lds blk, const SwagLane<C>& L, const u32x4 (&own)[C::KC], float bias) {
+  f32x4 s = {bias, bias, bias, bias};
+#pragma unroll
+  for (int c = 0; c < C::KC; c++) s = Mma<CT>::mfma(swat_read16(blk + L.row[c]), own[c], s);
+  return s;
+}
+
+// ROPE: K is turned in registers between HBM and LDS, the own queries in theirs
+template <typename TIO, int D, int NCH, int NCG, int PC, bool ROPE>
+__global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_kernel(const SwagArgs a) {
+  typedef Swag<D, NCH, NCG, PC> C;
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  swat_lds lds = (swat_lds)smem;
+  const int tid = threadIdx.x;
+  SwagFrame<C, PC> F;
+  F.init(a, tid);
+  const int b = F.w.b, h = F.w.h, n = F.n, g = F.g;
+  const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
+  const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
+  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
+  SwagRing<C> ring;
+  if constexpr (!ROPE) ring.init(lds, kb_, (int)a.ks[2], vb_, (int)a.vs[2], a, F.w.c0, tid, F.wave);
+  const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1]) + 16 * g;
+  char* ob = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.out_o) + b * a.os[0] + h * a.os[1]);
+  float* lseb = a.lse + b * a.ls[0] + h * a.ls[1];
+  const int qsn = (int)a.qs[2] * 2, osn = (int)a.os[2] * 2;
+  SwagLane<C> L;
+  L.init(n, g);
+  const float scale = a.scale_log2;
+  const unsigned one2 = pack2<CT>(1.f, 1.f);
+  const u32x4 ones = {one2, one2, one2, one2};
+
+  SwagTab tab;
+  char *krb = nullptr, *qrb = nullptr;
+  if constexpr (ROPE) {
+    tab.fetch(lds + C::RING, a.rope, tid);   // requested first: it does not depend on any index
+    if (a.k_rot != nullptr) {
+      krb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.k_rot) + b * a.krs[0] + h * a.krs[1]);
+      qrb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.q_rot) + b * a.qrs[0] + h * a.qrs[1]) + 16 * g;
+    }
+  }
+  const int krsn = ROPE ? (int)a.krs[2] * 2 : 0, qrsn = ROPE ? (int)a.qrs[2] * 2 : 0;
+  u32x4 qn[C::KC];
+  int32_t qid = -1;
+  auto load_q = [&](int rp) {
+    const int tok = F.own_tok(rp);
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) qn[c] = *reinterpret_cast<const u32x4*>(qb + (uint32_t)(tok * qsn) + 64 * c);
+    if constexpr (ROPE) qid = a.rope.idx[tok];
+  };
+  load_q(F.w.r0 + 4 * F.rg);
+  if constexpr (ROPE) {
+    SwagTurnStage<C, C::NRES> pre;
+    pre.issue(kb_, ksn, vb_, vsn, a, F.w.r0 - F.WR, F.w.c0, tid);
+    tab.store(tid);
+    __syncthreads();
+    pre.template turn<CT>(tab, a, krb, krsn, F.w.r0 - F.WR, F.w.r0, F.w.r1, F.w.c0, tid);
+    pre.commit(lds, 0, tid);
+  } else {
+    ring.fill(F.w.r0 - F.WR);
+  }
+  __syncthreads();
+
+  int slot0 = 0;   // slot of the step's first chunk
+  for (int r = F.w.r0; r < F.w.r1; r += 4 * C::PR) {
+    const int rp = r + 4 * F.rg;
+    u32x4 q[C::KC];
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) q[c] = qn[c];
+    pin_loaded(q);
+    if constexpr (ROPE) {
+      f32x4 t[4];
+      const bool rot = tab.get(t, qid, g >> 1, 0, a.rope);
+      const u32x4 partner = {swag_lane_xor16(q[0].x, g), swag_lane_xor16(q[0].y, g), swag_lane_xor16(q[0].z, g), swag_lane_xor16(q[0].w, g)};
+      if (rot) q[0] = swag_turn<CT>(q[0], partner, t, (g & 1) == 0);
+      if (qrb != nullptr && F.own_ok(rp)) {
+#pragma unroll
+        for (int c = 0; c < C::KC; c++) store_stream16(qrb + (uint32_t)(F.own_tok(rp) * qrsn) + 64 * c, q[c]);
+      }
+    }
+    const bool more = r + 4 * C::PR < F.w.r1;
+    u32x4 nx[C::PR][C::NIT];
+    SwagTurnStage<C, C::PR> nt;
+    const int next = r - F.WR + 4 * C::NRES;   // first halo row of the chunks to come
+    if (more) {
+      if constexpr (ROPE) {
+        nt.issue(kb_, ksn, vb_, vsn, a, next, F.w.c0, tid);
+      } else {
+#pragma unroll
+        for (int i = 0; i < C::PR; i++) ring.issue(nx[i], next + 4 * i);
+      }
+      load_q(rp + 4 * C::PR);
+    }
+    if (rp < F.TR && F.w.c0 + 4 * F.pc < F.TC) {
+      swat_lds rowp[NCH];
+#pragma unroll
+      for (int i = 0; i < NCH; i++) {
+        const int s = slot0 + F.rg + i;
+        rowp[i] = lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + 4 * F.pc * C::ROWB;
+      }
+      f32x4 s[C::NB + 1];
+      float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+      for (int i = 0; i < NCH; i++) {
+        const float bias = F.row_bias(i, rp);
+#pragma unroll
+        for (int j = 0; j < NCG; j++) {
+          f32x4 t = swag_scores<C, CT>(rowp[i] + 4 * j * C::ROWB, L, q, bias);
+#pragma unroll
+          for (int e = 0; e < 4; e++) t[e] = F.sees_col(4 * j + e) ? t[e] : -INFINITY;
+          s[i * NCG + j] = t;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < C::NB; k += 2)
+#pragma unroll
+        for (int e = 0; e < 4; e++) mx[e] = fmaxf(fmaxf(mx[e], s[k][e]), s[k + 1 < C::NB ? k + 1 : k][e]);
+      const float m = wave_max4(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
+      const float m_use = m == -INFINITY ? 0.f : m;   // own positions outside the grid see nothing
+      const float neg_m2 = -m_use * scale;
+      f32x4 acc[C::DB], acc_l = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < C::DB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < C::NP; t++) {
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          p[e] = fast_exp2(fmaf(s[b0][e], scale, neg_m2));
+          p[4 + e] = 2 * t + 1 < C::NB ? fast_exp2(fmaf(s[b1][e], scale, neg_m2)) : 0.f;
+        }
+        const u32x4 pb = pack8<CT>(p);
+        swat_lds v0 = rowp[b0 / NCG] + C::TB + 4 * (b0 % NCG) * C::ROWB, v1 = rowp[b1 / NCG] + C::TB + 4 * (b1 % NCG) * C::ROWB;
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(v0 + L.tr[d]), hi = swat_read_tr(v1 + L.tr[d]);
+          acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc[d]);
+        }
+        acc_l = Mma<CT>::mfma(ones, pb, acc_l);
+      }
+      const float l = acc_l[0];
+      if (F.own_ok(rp)) {
+        const int tok = F.own_tok(rp);
+        swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+        if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
+      }
+    }
+    if (more) {
+      if constexpr (ROPE) nt.template turn<CT>(tab, a, krb, krsn, next, F.w.r0, F.w.r1, F.w.c0, tid);
+      __syncthreads();
+      if constexpr (ROPE) {
+        nt.commit(lds, slot0, tid);
+      } else {
+#pragma unroll
+        for (int i = 0; i < C::PR; i++) ring.commit(nx[i], slot0 + i >= C::NRES ? slot0 + i - C::NRES : slot0 + i);
+      }
+      __syncthreads();
+      slot0 = slot0 + C::PR >= C::NRES ? slot0 + C::PR - C::NRES : slot0 + C::PR;
+    }
+  }
+}
+
+// dQ: own = queries, K and V in the ring; delta = rowsum(o dO) of the own queries is formed and stored on the way.
+// ROPE (both backward kernels): q and k arrive rotated, the gradients are turned back on their way out.
+template <typename TIO, int D, int NCH, int NCG, int PC, bool ROPE>
+__global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC_BWD)) void swag_bwd_q_kernel(const SwagArgs a) {
+  typedef Swag<D, NCH, NCG, PC> C;
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  swat_lds lds = (swat_lds)smem;
+  const int tid = threadIdx.x;
+  SwagFrame<C, PC> F;
+  F.init(a, tid);
+  const int b = F.w.b, h = F.w.h, n = F.n, g = F.g;
+  SwagRing<C> ring;
+  ring.init(lds, reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]), (int)a.ks[2],
+            reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]), (int)a.vs[2], a, F.w.c0, tid, F.wave);
+  const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1]) + 16 * g;
+  const char* dob = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1]) + 16 * g;
+  const char* ob = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.o) + b * a.os[0] + h * a.os[1]) + 16 * g;
+  char* dqb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.dq) + b * a.dqs[0] + h * a.dqs[1]);
+  const float* lseb = a.lse + b * a.ls[0] + h * a.ls[1];
+  float* delb = a.delta + b * a.ls[0] + h * a.ls[1];
+  const int qsn = (int)a.qs[2] * 2, dosn = (int)a.dos[2] * 2, osn = (int)a.os[2] * 2, dqsn = (int)a.dqs[2] * 2;
+  SwagLane<C> L;
+  L.init(n, g);
+  const float scale = a.scale_log2;
+
+  SwagTab tab;
+  tab.in_lds = false;
+  int32_t idn = -1;
+  u32x4 qn[C::KC], don[C::KC], on[C::KC];
+  float lsen;
+  auto load_own = [&](int rp) {
+    const int tok = F.own_tok(rp);
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) {
+      qn[c] = *reinterpret_cast<const u32x4*>(qb + (uint32_t)(tok * qsn) + 64 * c);
+      don[c] = *reinterpret_cast<const u32x4*>(dob + (uint32_t)(tok * dosn) + 64 * c);
+      on[c] = *reinterpret_cast<const u32x4*>(ob + (uint32_t)(tok * osn) + 64 * c);
+    }
+    lsen = lseb[tok * a.ls[2]];
+    if constexpr (ROPE) idn = a.rope.idx[tok];
+  };
+  load_own(F.w.r0 + 4 * F.rg);
+  ring.fill(F.w.r0 - F.WR);
+  __syncthreads();
+
+  int slot0 = 0;
+  for (int r = F.w.r0; r < F.w.r1; r += 4 * C::PR) {
+    const int rp = r + 4 * F.rg;
+    u32x4 q[C::KC], d_o[C::KC];
+    float part = 0.f;
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) {
+      q[c] = qn[c];
+      d_o[c] = don[c];
+      float fo[8], fd[8];
+      unpack8<CT>(on[c], fo);
+      unpack8<CT>(d_o[c], fd);
+#pragma unroll
+      for (int j = 0; j < 8; j++) part += fo[j] * fd[j];
+    }
+    pin_loaded(q);
+    const float nlse = -lsen;
+    const float del = wave_sum4(part);
+    const bool ok = F.own_ok(rp);
+    f32x4 tr[2][2];
+    bool rot[2];
+    if constexpr (ROPE) {
+#pragma unroll
+      for (int ax = 0; ax < 2; ax++) rot[ax] = tab.get(tr[ax], idn, ax, 4 * (g & 1), a.rope);
+    }
+    if (g == 0 && ok) store_stream4(delb + F.own_tok(rp) * a.ls[2], del);
+    const bool more = r + 4 * C::PR < F.w.r1;
+    u32x4 nx[C::PR][C::NIT];
+    if (more) {
+#pragma unroll
+      for (int i = 0; i < C::PR; i++) ring.issue(nx[i], r - F.WR + 4 * (C::NRES + i));
+      load_own(rp + 4 * C::PR);
+    }
+    if (rp < F.TR && F.w.c0 + 4 * F.pc < F.TC) {
+      swat_lds rowp[NCH];
+#pragma unroll
+      for (int i = 0; i < NCH; i++) {
+        const int s = slot0 + F.rg + i;
+        rowp[i] = lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + 4 * F.pc * C::ROWB;
+      }
+      f32x4 acc[C::DB];
+#pragma unroll
+      for (int d = 0; d < C::DB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < C::NP; t++) {
+        float ds[8];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const int k = 2 * t + u;
+          if (k >= C::NB) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) ds[4 * u + e] = 0.f;
+            continue;
+          }
+          swat_lds kp = rowp[k / NCG] + 4 * (k % NCG) * C::ROWB;
+          const f32x4 s = swag_scores<C, CT>(kp, L, q, F.row_bias(k / NCG, rp));
+          // the dP products start from -delta: the matrix pipe delivers dP - delta
+          f32x4 dp = {-del, -del, -del, -del};
+#pragma unroll
+          for (int c = 0; c < C::KC; c++) dp = Mma<CT>::mfma(swat_read16(kp + C::TB + L.row[c]), d_o[c], dp);
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float pv = fast_exp2(fmaf(s[e], scale, nlse));
+            ds[4 * u + e] = (F.sees_col(4 * (k % NCG) + e) ? pv : 0.f) * dp[e];
+          }
+        }
+        const u32x4 dsb = pack8<CT>(ds);
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        swat_lds k0 = rowp[b0 / NCG] + 4 * (b0 % NCG) * C::ROWB, k1 = rowp[b1 / NCG] + 4 * (b1 % NCG) * C::ROWB;
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(k0 + L.tr[d]), hi = swat_read_tr(k1 + L.tr[d]);
+          acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
+        }
+      }
+      if constexpr (ROPE) swag_turn_back<CT>(acc, a.sm_scale, tr, rot, g);
+      if (ok) swat_store_row<CT, C::DB>(dqb + (uint32_t)(F.own_tok(rp) * dqsn), acc, ROPE ? 1.f : a.sm_scale, g);
+    }
+    if (more) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < C::PR; i++) ring.commit(nx[i], slot0 + i >= C::NRES ? slot0 + i - C::NRES : slot0 + i);
+      __syncthreads();
+      slot0 = slot0 + C::PR >= C::NRES ? slot0 + C::PR - C::NRES : slot0 + C::PR;
+    }
+  }
+}
+
+// dK / dV: own = keys, Q and dO in the ring with -lse2 and delta of their tokens behind it (the window is symmetric).
+template <typename TIO, int D, int NCH, int NCG, int PC, bool ROPE>
+__global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC_BWD)) void swag_bwd_kv_kernel(const SwagArgs a) {
+  typedef Swag<D, NCH, NCG, PC> C;
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  swat_lds lds = (swat_lds)smem;
+  const int tid = threadIdx.x;
+  SwagFrame<C, PC> F;
+  F.init(a, tid);
+  const int b = F.w.b, h = F.w.h, n = F.n, g = F.g;
+  SwagRing<C> ring;
+  ring.init(lds, reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1]), (int)a.qs[2],
+            reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1]), (int)a.dos[2], a, F.w.c0, tid, F.wave);
+  const float* lseb = a.lse + b * a.ls[0] + h * a.ls[1];
+  const float* delb = a.delta + b * a.ls[0] + h * a.ls[1];
+  DLT_LDS float* scal = reinterpret_cast<DLT_LDS float*>(lds + C::RING);   // [slot][-lse2 | delta][token]
+  const int shr = tid / C::HCW, shc = tid - shr * C::HCW;
+  const int scol = dlt_imax(0, dlt_imin(F.w.c0 - F.WC + shc, F.TC - 1));
+  auto issue_scal = [&](float& x, float& y, int first) {
+    if (tid < C::TOK) {
+      const int tok = dlt_imax(0, dlt_imin(first + shr, F.TR - 1)) * F.TC + scol;
+      x = lseb[tok * a.ls[2]];
+      y = delb[tok * a.ls[2]];
+    }
+  };
+  auto commit_scal = [&](float x, float y, int slot) {
+    if (tid < C::TOK) {
+      scal[slot * 2 * C::TOK + tid] = -x;
+      scal[slot * 2 * C::TOK + C::TOK + tid] = y;
+    }
+  };
+  const char* kb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]) + 16 * g;
+  const char* vb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]) + 16 * g;
+  char* dkb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.dk) + b * a.dks[0] + h * a.dks[1]);
+  char* dvb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.dv) + b * a.dvs[0] + h * a.dvs[1]);
+  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2, dksn = (int)a.dks[2] * 2, dvsn = (int)a.dvs[2] * 2;
+  SwagLane<C> L;
+  L.init(n, g);
+  const float scale = a.scale_log2;
+
+  SwagTab tab;
+  tab.in_lds = false;
+  int32_t idn = -1;
+  u32x4 kn[C::KC], vn[C::KC];
+  auto load_own = [&](int rp) {
+    const int tok = F.own_tok(rp);
+    if constexpr (ROPE) idn = a.rope.idx[tok];
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) {
+      kn[c] = *reinterpret_cast<const u32x4*>(kb + (uint32_t)(tok * ksn) + 64 * c);
+      vn[c] = *reinterpret_cast<const u32x4*>(vb + (uint32_t)(tok * vsn) + 64 * c);
+    }
+  };
+  load_own(F.w.r0 + 4 * F.rg);
+  ring.fill(F.w.r0 - F.WR);
+  {
+    float x[C::NRES], y[C::NRES];
+#pragma unroll
+    for (int i = 0; i < C::NRES; i++) issue_scal(x[i], y[i], F.w.r0 - F.WR + 4 * i);
+#pragma unroll
+    for (int i = 0; i < C::NRES; i++) commit_scal(x[i], y[i], i);
+  }
+  __syncthreads();
+
+  int slot0 = 0;
+  for (int r = F.w.r0; r < F.w.r1; r += 4 * C::PR) {
+    const int rp = r + 4 * F.rg;
+    // the own values are negated and the dP products start from the staged delta: the matrix pipe delivers -(dP - delta)
+    u32x4 k_[C::KC], v_[C::KC];
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) {
+      k_[c] = kn[c];
+      v_[c] = u32x4{vn[c].x ^ 0x80008000u, vn[c].y ^ 0x80008000u, vn[c].z ^ 0x80008000u, vn[c].w ^ 0x80008000u};
+    }
+    pin_loaded(k_);
+    pin_loaded(v_);
+    f32x4 tr[2][2];
+    bool rot[2];
+    if constexpr (ROPE) {
+#pragma unroll
+      for (int ax = 0; ax < 2; ax++) rot[ax] = tab.get(tr[ax], idn, ax, 4 * (g & 1), a.rope);
+    }
+    const bool more = r + 4 * C::PR < F.w.r1;
+    u32x4 nx[C::PR][C::NIT];
+    float sx[C::PR], sy[C::PR];
+    if (more) {
+#pragma unroll
+      for (int i = 0; i < C::PR; i++) {
+        ring.issue(nx[i], r - F.WR + 4 * (C::NRES + i));
+        issue_scal(sx[i], sy[i], r - F.WR + 4 * (C::NRES + i));
+      }
+      load_own(rp + 4 * C::PR);
+    }
+    if (rp < F.TR && F.w.c0 + 4 * F.pc < F.TC) {
+      swat_lds rowp[NCH];
+      DLT_LDS float* scp[NCH];
+#pragma unroll
+      for (int i = 0; i < NCH; i++) {
+        const int s0 = slot0 + F.rg + i, s = s0 >= C::NRES ? s0 - C::NRES : s0;
+        rowp[i] = lds + s * C::SLOT + 4 * F.pc * C::ROWB;
+        scp[i] = scal + s * 2 * C::TOK + g * C::HCW + 4 * F.pc;
+      }
+      f32x4 acc_k[C::DB], acc_v[C::DB];
+#pragma unroll
+      for (int d = 0; d < C::DB; d++) acc_k[d] = acc_v[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < C::NP; t++) {
+        float p[8], ds[8];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const int k = 2 * t + u;
+          if (k >= C::NB) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) p[4 * u + e] = ds[4 * u + e] = 0.f;
+            continue;
+          }
+          swat_lds qp = rowp[k / NCG] + 4 * (k % NCG) * C::ROWB;
+          DLT_LDS float* sp = scp[k / NCG] + 4 * (k % NCG);
+          const f32x4 nl = *reinterpret_cast<DLT_LDS f32x4*>(sp);
+          const f32x4 s = swag_scores<C, CT>(qp, L, k_, F.row_bias(k / NCG, rp));
+          f32x4 dp = *reinterpret_cast<DLT_LDS f32x4*>(sp + C::TOK);
+#pragma unroll
+          for (int c = 0; c < C::KC; c++) dp = Mma<CT>::mfma(swat_read16(qp + C::TB + L.row[c]), v_[c], dp);
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float x = fast_exp2(fmaf(s[e], scale, nl[e])), pv = F.sees_col(4 * (k % NCG) + e) ? x : 0.f;
+            p[4 * u + e] = pv;
+            ds[4 * u + e] = -pv * dp[e];
+          }
+        }
+        const u32x4 pb = pack8<CT>(p), dsb = pack8<CT>(ds);
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        swat_lds q0 = rowp[b0 / NCG] + 4 * (b0 % NCG) * C::ROWB, q1 = rowp[b1 / NCG] + 4 * (b1 % NCG) * C::ROWB;
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(q0 + C::TB + L.tr[d]), hi = swat_read_tr(q1 + C::TB + L.tr[d]);
+          acc_v[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc_v[d]);
+        }
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(q0 + L.tr[d]), hi = swat_read_tr(q1 + L.tr[d]);
+          acc_k[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc_k[d]);
+        }
+      }
+      if constexpr (ROPE) swag_turn_back<CT>(acc_k, a.sm_scale, tr, rot, g);
+      if (F.own_ok(rp)) {
+        const int tok = F.own_tok(rp);
+        swat_store_row<CT, C::DB>(dvb + (uint32_t)(tok * dvsn), acc_v, 1.f, g);
+        swat_store_row<CT, C::DB>(dkb + (uint32_t)(tok * dksn), acc_k, ROPE ? 1.f : a.sm_scale, g);
+      }
+    }
+    if (more) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < C::PR; i++) {
+        const int slot = slot0 + i >= C::NRES ? slot0 + i - C::NRES : slot0 + i;
+        ring.commit(nx[i], slot);
+        commit_scal(sx[i], sy[i], slot);
+      }
+      __syncthreads();
+      slot0 = slot0 + C::PR >= C::NRES ? slot0 + C::PR - C::NRES : slot0 + C::PR;
+    }
+  }
+}

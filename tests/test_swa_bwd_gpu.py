@@ -304,3 +304,33 @@ def test_fused_rope_with_head_dims_below_the_padded_class(d, dv, R, th, tw, W, s
     assert (o.float().cpu() - o_w).abs().max().item() <= FWD_TOL
     errs = (_rel(qg.grad, dq_w), _rel(kg.grad, dk_w), _rel(vg.grad, dv_w))
     assert max(errs) <= GRAD_TOL, errs
+
+
+# the marching kernels by window class: every class of rows and columns at both head dims, one-row and one-column grids, widths
+# and heights around the 16-column strips and 8-row steps, grids smaller than the window, bands of one and of several steps
+MARCH = [(1, 1, 0, 1), (1, 19, 1, 2), (23, 1, 2, 0), (16, 16, 2, 2), (17, 15, 2, 4), (8, 33, 2, 6), (9, 31, 4, 1), (24, 17, 3, 3), (25, 48, 4, 5), (7, 5, 6, 2),
+         (31, 34, 6, 4), (40, 20, 5, 6), (4, 3, 6, 6), (65, 18, 1, 1)]
+
+
+@pytest.mark.parametrize("th,tw,WR,WC", MARCH)
+@pytest.mark.parametrize("d,rope", [(32, False), (64, False), (64, True)])
+def test_marching_window_classes(th, tw, WR, WC, d, rope):
+    sw = _swa()
+    from dl_templates_amd import _lib
+    B, H, N, dt = (3, 30, th * tw, torch.float16) if th == 16 else (1, 3, th * tw, torch.bfloat16)   # 16 x 16: more workgroups than fit at once
+    q, k, v, do = orc.make_qkv(N + d + WR, B, H, N, N, d, d, dt)
+    scale = 0.2
+    qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    if rope:
+        idx = orc.make_rope_idx(3, th, tw, 0.1)
+        rcs, ccs = orc.rope_tables(8, max(th, 120 if th == 9 else 1)), orc.rope_tables(8, tw)   # 9 x 31: tables beyond the copy in LDS
+        want = orc.rope_swa_grads(q.float(), k.float(), v.float(), do.float(), idx, rcs, ccs, 1, th, tw, WR, WC, scale)
+        o = sw.TiledSwaRope.apply(qg, kg, vg, idx.cuda(), rcs.cuda(), ccs.cuda(), 1, th, tw, WR, WC, scale)
+    else:
+        want = orc.tiled_swa_grads(q.float(), k.float(), v.float(), do.float(), 1, th, tw, WR, WC, scale)
+        o = sw.TiledSwa.apply(qg, kg, vg, 1, th, tw, WR, WC, scale)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "marching"
+    o.backward(do.cuda())
+    assert (o.float().cpu() - want[0]).abs().max().item() <= 2e-2
+    errs = (_rel(qg.grad, want[1]), _rel(kg.grad, want[2]), _rel(vg.grad, want[3]))
+    assert max(errs) <= GRAD_TOL, errs
