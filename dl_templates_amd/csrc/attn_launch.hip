@@ -45,6 +45,7 @@ int dlt_flashs_bwd_kv_64_128(const FlashBwdArgs&, int dtype, int np, hipStream_t
 int dlt_flashs_fwd_128_128(const FlashArgs&, int dtype, int np, hipStream_t);
 int dlt_flashs_bwd_q_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
 int dlt_flashs_bwd_kv_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_swag_launch_f32(const SwagArgs&, int nch, int ncg, int grid, hipStream_t);
 int dlt_swag_launch_32_2(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_32_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_32_4(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
@@ -389,6 +390,19 @@ bool swag_eligible(const AttnProblem& p, const AttnTensors& t, const Swa1Class& 
          swag_rows_ok(p, t.dv, t.dvs);
 }
 
+// fp32 tensors of head dim 32, forward pass: the marching kernel on hi + lo pairs.  Head dim 64 in fp32 belongs to the generic
+// family in the routing table that callers of the C ABI rely on, and stays there.
+bool swag_f32_eligible(const AttnProblem& p, const AttnTensors& t) {
+  if (p.g.mode != DLT_GEOM_SWA || p.g.S != 1 || p.tm.img || p.dtype != DLT_FP32 || !(p.sm_scale > 0.f) || t.q_rot != nullptr) return false;
+  if ((p.rope.enabled && p.rope.R > 0) || p.dk != p.dv || p.dk != 32) return false;
+  if (p.g.WR > 6 || p.g.WC > 6) return false;
+  const void* const ptrs[4] = {t.q, t.k, t.v, t.out_o};
+  const int64_t* const st[4] = {t.qs, t.ks, t.vs, t.os};
+  for (int i = 0; i < 4; i++)
+    if (!tvec_ok(ptrs[i], st[i], p.dk, 4) || st[i][2] < 0 || ((int64_t)p.g.TR * p.g.TC - 1) * st[i][2] * 4 + 4 * p.dk > ((int64_t)1 << 31) - 1) return false;
+  return true;
+}
+
 int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t stream) {
   if (dlt_route_note(DLT_FAMILY_MARCHING)) return DLT_OK;
   SwagArgs a;
@@ -411,7 +425,7 @@ int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   a.nstrips = (p.g.TC + 4 * pc - 1) / (4 * pc);
   // Rows per workgroup: a band costs its steps plus a prologue that fills the ring (about two steps); workgroups beyond what the
   // chip holds at once (one or two per CU) wait for a whole band.
-  const int nres = nch + 8 / pc - 1, tok = 4 * (4 * pc + 4 * (ncg - 1)), lds = nres * tok * (4 * p.dk + 8);
+  const int nres = nch + 8 / pc - 1, tok = 4 * (4 * pc + 4 * (ncg - 1)), lds = nres * tok * (p.dtype == DLT_FP32 ? 6 * p.dk : 4 * p.dk + 8);
   const int64_t slots = (int64_t)dlt_device_cus() * (lds <= 80 * 1024 ? 2 : 1);
   const int64_t cols = (int64_t)p.B * p.H * a.nstrips;
   const int steps = (p.g.TR + step - 1) / step;
@@ -424,6 +438,7 @@ int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   }
   const int64_t grid = cols * a.nbands;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
+  if (p.dtype == DLT_FP32) return dlt_swag_launch_f32(a, nch, ncg, (int)grid, stream);
   if (p.dk == 32) {
     switch (nch) {
       case 2: return dlt_swag_launch_32_2(a, p.dtype, ncg, bwd, (int)grid, stream);
@@ -724,6 +739,7 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
     for (int i = 0; i < 5; i++) { t2.qs[i] = t.qrs[i]; t2.ks[i] = t.krs[i]; }
     return dlt_attn_forward(p2, t2, stream);
   }
+  if (swag_f32_eligible(p, t)) return swag_run(p, t, false, stream);
   if (flash_eligible(p, t, false) && swat_eligible(p, t, false)) return swat_run(p, t, false, stream);
   if (flash_eligible(p, t, false)) return flash_forward(p, t, dc, stream);
   if (swa2_tiles_eligible(p, t, false)) return swa2_forward(p, t, stream);

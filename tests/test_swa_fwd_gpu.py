@@ -247,3 +247,19 @@ def test_token_grid_offsets_beyond_32_bits_take_the_generic_kernels():
     kview.copy_(k.cuda())
     got = sw.tiled_swa_fwd(q.cuda(), kview, v.cuda(), 1, th, tw, W, W, 0.125)
     assert (got.float().cpu() - want).abs().max().item() <= FWD_TOL
+
+
+# fp32 tensors at head dim 32: the marching kernel on hi + lo pairs, every window class, edges of the 16-column strips and 8-row steps
+@pytest.mark.parametrize("th,tw,WR,WC", [(1, 1, 0, 0), (8, 16, 2, 2), (9, 17, 3, 1), (16, 16, 3, 3), (7, 33, 2, 6), (31, 15, 6, 2), (32, 32, 4, 4), (25, 20, 5, 6)])
+def test_marching_fp32(th, tw, WR, WC):
+    sw = _swa()
+    from dl_templates_amd import _lib
+    B, H, N, d, scale = 2, 3, th * tw, 32, 1.0
+    q, k, v, _ = orc.make_qkv(N + WR, B, H, N, N, d, d, torch.float32)
+    want, lse_w = orc.tiled_swa_explicit(q, k, v, 1, th, tw, WR, WC, scale, return_lse2=True)
+    flat = [t.permute(0, 2, 1, 3).contiguous().cuda().permute(0, 2, 1, 3) for t in (q, k, v)]   # heads inside the token rows
+    for args in ([t.cuda() for t in (q, k, v)], flat):
+        o, lse = sw._forward(*args, sw._shape(*args, 1, th, tw, WR, WC, scale), None)
+        assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "marching"
+        assert (o.cpu() - want).abs().max().item() <= FWD_TOL
+        assert (lse.cpu() - lse_w).abs().max().item() <= LSE_TOL
