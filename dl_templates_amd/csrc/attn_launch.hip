@@ -303,7 +303,9 @@ bool swa2_compose_ok(const AttnProblem& p, const Swa1Class& c) {
   return (c.D == 64 || c.D == 128) && p.dk == c.D && p.dv == c.D && (int64_t)p.B * p.H * p.g.TR * p.g.TC >= 131072;
 }
 
-void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan, int band = 8) {
+void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan) {
+  constexpr int band = 8;
+  plan.pairs = 0;
   { int c; swa2_split(p, c, plan.npass); }
   plan.S = p.g.S; plan.WCt = p.g.WC;
   dlt_fastdiv_make((uint32_t)p.g.S, plan.m_S, plan.s_S);
@@ -343,10 +345,13 @@ int swa2_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream)
   if (dlt_route_note(DLT_FAMILY_STREAMING)) return DLT_OK;
   Swa2FwdArgs a;
   a.p = p;
-  // head dim 128, more than one band of 8 rows: the forward kernel with two stacked patches per wave (bands of 16 rows);
-  // DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the one-patch kernel for A/B timing and for its tests
+  // Two stacked patches per wave (4 waves per workgroup, two workgroups per CU) from more than one workgroup per CU on; below, a
+  // CU has one workgroup either way and 8 waves of one patch each finish it sooner (64 workgroups 12.8 against 14.2 us, 224
+  // 11.2 / 12.2, 352 26.8 / 25.8).  Its copies need K and V at the same token stride.
+  // DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the one-patch kernel for A/B timing and for its tests.
   static const bool single_patch = [] { const char* e = getenv("DLT_SWA2_SINGLE_PATCH"); return e != nullptr && e[0] == '1'; }();
-  swa2_make_plan(p, a.plan, p.dk == 128 && p.g.TR > 8 && !single_patch ? 16 : 8);
+  swa2_make_plan(p, a.plan);
+  a.plan.pairs = !single_patch && t.ks[2] == t.vs[2] && (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c > dlt_device_cus();
   a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.out_o; a.lse = t.lse;
   for (int i = 0; i < 4; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; }
   for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];

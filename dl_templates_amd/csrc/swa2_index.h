@@ -4,8 +4,8 @@
 //
 // A workgroup of 8 waves owns a band of 8 grid rows x 16 grid columns; wave w owns the 4x4 patch at rows
 // 4 (w >> 2), columns 4 (w & 3).  The halo of the band (8 + 2 WR rows x HCW columns, first halo column = c0 - WC)
-// streams through LDS in chunks of 4 halo rows.  Stacked variant (Swa2Plan::band = 16): a band of 16 grid rows, wave w
-// owns the two 4x4 patches at rows 8 (w >> 2) and 8 (w >> 2) + 4, columns 4 (w & 3): "row group" rg below is then 0 .. 3.
+// streams through LDS in chunks of 4 halo rows.  Forward kernel with two stacked patches per wave
+// (Swa2Plan::pairs): 4 waves, wave w owns the patches at columns 4 w, rows 0 and 4.
 //
 // Tiles of S tokens (1 < S < 16): a grid row then holds TC = tiles * S token slots ("columns" below are slots), a token
 // in tile t sees the slots of tiles t - WCt .. t + WCt, i.e. S WCt + (x mod S) slots to its left and S WCt + S - 1 - (x mod S)
@@ -53,7 +53,8 @@ struct Swa2Plan {
   int32_t npass;   // column passes: a window of more than NCG column groups is walked in npass slices of NCG groups
   int32_t S, WCt;  // tokens per tile, window half-width in tiles
   uint32_t m_S, s_S;   // division by S
-  int32_t band;    // grid rows of a workgroup's band: 8 (one patch per wave) or 16 (two stacked patches per wave)
+  int32_t band;    // grid rows of a workgroup's band: 8
+  int32_t pairs;   // forward pass: 4 waves of two stacked patches instead of 8 waves of one
 };
 
 struct Swa2Geom {

@@ -13,16 +13,13 @@ int swa2_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast
 template <typename TIO, int NCG>
 int swa2_launch_fwd_t(const Swa2FwdArgs& a, int grid, hipStream_t stream) {
   typedef Swa2Cfg<DLT_SWA2_D, NCG> C;
-  auto kern = swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG>;
-  if constexpr (DLT_SWA2_D == 128) {
-    if (a.plan.band == 16) kern = swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG>;   // two stacked patches per wave
-  } else if (a.plan.band != 8) {
-    return dlt_set_error(DLT_ERR_UNSUPPORTED, "streaming token-grid kernels: no instantiation for bands of %d rows", a.plan.band);
-  }
-  int rc = swa2_set_lds(kern, C::LDS);
+  const bool pairs = a.plan.pairs != 0;
+  auto kern = pairs ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG> : swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG>;
+  const int lds = pairs ? C::BUF : C::LDS;
+  int rc = swa2_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;
   dlt_timing_before(DLT_K_FWD, stream);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(SWA2_THREADS), C::LDS, stream, a);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(pairs ? SWA2S_THREADS : SWA2_THREADS), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("token-grid forward launch (streaming kernels)");
   return DLT_OK;

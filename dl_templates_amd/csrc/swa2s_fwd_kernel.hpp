@@ -1,27 +1,41 @@
-// Forward kernel for token grids at head dim 128 (b_size == 1, no rotation), two stacked patches per wave: the work of
-// tiled_swa_fwd_kernel (src/tiled_swa.py:15-133) on the streaming structure of swa2_common.hpp with a band of 16 grid
-// rows per workgroup.  Wave w owns the 4x4 patches at rows 8 (w >> 2) and 8 (w >> 2) + 4, columns 4 (w & 3): both see the
-// same window columns, so every K fragment read from LDS feeds the score products of both patches and every V^T
-// fragment both output products (two matrix instructions per operand read instead of one), and the two independent
-// product chains fill each other's latencies.  A halo row is staged once per 16 own rows.  Scores, maxima and output
-// products are those of swa2_fwd_kernel in the same order; the row sums are taken with two-element dot products on the
-// vector pipe (fp32 accumulation of the rounded probabilities, summed in another order than the matrix instruction of
-// swa2_fwd_kernel does), which frees the registers of that instruction's operands and accumulators: 253 registers at
-// 6 column groups, none spilled.
+// Forward kernel for token grids at head dims 64 and 128 (b_size == 1 and tiles of 2 ... 15 tokens, no rotation), two stacked
+// patches per wave: the work of tiled_swa_fwd_kernel (src/tiled_swa.py:15-133) on the streaming structure of swa2_common.hpp.
+// A workgroup of 4 waves owns a band of 8 rows x 16 columns, wave w the two 4x4 patches at column 4 w: both see the same
+// window columns, so every K fragment read from LDS feeds the score products of both patches and every V^T fragment both
+// output products.
+//
+// K and V of a chunk have ONE buffer each: V of a chunk is copied while its scores are formed, K of the next chunk during
+// the output products, a barrier between the two.  A workgroup then fits into half the LDS of a CU (74 KB at head dim 128,
+// 6 column groups), and the two (head dim 64: up to four) workgroups of a CU are in different phases: one fills the waits of the
+// other.  An earlier version ran 8 waves over bands of 16 rows with both chunk buffers doubled, one workgroup per CU: the waves
+// stood together at every barrier, and half of them had no row of the first two and last two chunks.  Back-to-back calls, 16
+// slabs at d = 128, 21 x 21 window: 128 x 128 tokens 99.4 -> 95.6 us, 97 x 161 107.5 -> 98.0; 32 slabs of 103 x 36, 21 x 7: 54.6
+// -> 46.0; d = 64, 32 slabs of 89 x 98, 15 x 21: 73 -> 66.7 (there against one patch per wave).  Of 106 us in a short burst the
+// matrix and vector instructions account for 71 (the issue port), LDS operand reads and the copies for the rest: without
+// either of the two it runs in 91 ... 94.  Leaving out the column test where a whole group is inside every window, a longer
+// read-ahead of K and copies issued earlier in their phase measured the same within 1 %.
+//
+// The row sums are two-element dot products on the vector pipe (fp32 accumulation of the rounded probabilities): the matrix
+// instruction of swa2_fwd_kernel would take registers that are not there (256 at 6 column groups).
 #pragma once
 #include "swa2_fwd_kernel.hpp"
 
+constexpr int SWA2S_THREADS = 256;
+// waves per SIMD the register budget is sized for (head dim 64 at 6 column groups spills at 3)
+constexpr int swa2s_occ(int D, int NCG) { return D == 64 && NCG == 4 ? 3 : 2; }
+
 template <typename TIO, int D, int NCG>
-__global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2FwdArgs a) {
+__global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_kernel(const Swa2FwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef Swa2Cfg<D, NCG> C;
   constexpr int KC = C::KC, VB = C::VB, NKB = C::NKB;
   constexpr int NG = VB / 4;   // groups of four 16-dim blocks of the output
+  static_assert(C::NI <= 2 * NCG && C::NI <= 2 * NKB * NG && 4 * C::TILE <= C::BUF, "copy slots of a phase; the store epilogue");
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pc = wave & 3, rp = wave >> 2;
+  const int pc = wave;
   const Swa2Geom G0 = swa2_geom(a.p, a.plan);
 
   const char* qb = reinterpret_cast<const char*>(a.q) + 2 * (G0.b * a.qs[0] + G0.h * a.qs[1]);
@@ -32,15 +46,13 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
   const int64_t os2 = a.os[2], ls2 = a.ls[2];
   const float scale = a.scale_log2;
 
-  // staging: waves 0-3 copy the four halo rows of K, waves 4-7 those of V
-  const bool stage_k = wave < 4;
-  const char* sbase = stage_k ? kb_ : vb_;
-  const int ssn2 = (int)(stage_k ? a.ks[2] : a.vs[2]) * 2;
-  const uint32_t srow = (uint32_t)(G0.TC * ssn2);
+  // staging: wave w copies halo row w of every chunk, of K and of V
+  const int sn2 = (int)a.ks[2] * 2;
+  const uint32_t srow = (uint32_t)(G0.TC * sn2);
   Swa2Geom G = G0;   // column pass 0
-  Swa2Stage<C> st;
-  swa2_stage_init(st, G, wave, lane, ssn2);
-  swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
+  Swa2Stage<C> st;   // K and V have the same token stride (dispatch rule)
+  swa2_stage_init(st, G, wave, lane, sn2);
+  swa2_issue(st, G, G.ch_first, kb_, srow, smem, wave);
 
   // own queries of both patches straight into B-operand fragments
   const int c_p = G.c0 + 4 * pc;
@@ -49,10 +61,10 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
   Swa2Win W0[2], W[2];
 #pragma unroll
   for (int p = 0; p < 2; p++) {
-    r_p[p] = G.r0 + 4 * (2 * rp + p);
+    r_p[p] = G.r0 + 4 * p;
     tq[p] = (r_p[p] + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p[p] + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
     swa2_own_frags<KC>(qf[p], qb, (int)a.qs[2] * 2, tq[p], g);
-    W0[p] = swa2_window(G0, 2 * rp + p, pc, n);
+    W0[p] = swa2_window(G0, p, pc, n);
     W[p] = W0[p];
   }
   Swa2Lane<C> L;
@@ -67,7 +79,6 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
     for (int d = 0; d < VB; d++) acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const unsigned one2 = pack2<CT>(1.f, 1.f);
-  int ncg = swa2_pass_ncg(G0.WC, NCG, 0);
 
   swa2_wait_copies();   // also: the own fragments have arrived
   pin_loaded(qf);
@@ -76,18 +87,18 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
   // PM: the patches that see rows of the chunk (bit 0: the upper patch, bit 1: the lower one).  The chunks of a wave come
   // in the order "upper only" (at most one), "both", "lower only" (at most one); the one-patch bodies issue no product,
   // mask, exponential or reduction for the other patch.
-  auto consume = [&](const int ch, Swa2Lds __restrict__ cur, char* __restrict__ nxt, auto more_tag, auto pm_tag) {
-    constexpr bool more = decltype(more_tag)::value;   // a later chunk exists: its copies are issued between the products
+  auto consume = [&](const int ch, auto more_tag, auto pm_tag) {
+    constexpr bool more = decltype(more_tag)::value;   // a later chunk exists: its K is copied between the output products
     constexpr int PM = decltype(pm_tag)::value;
     constexpr bool P0 = (PM & 1) != 0, P1 = (PM & 2) != 0;
-    Swa2Lds sK = cur;
+    Swa2Lds sK = (Swa2Lds)smem;
     Swa2Lds sV = sK + C::REGION;
-    const char* nrow = swa2_issue_row(G, ch + 1, sbase, srow, wave);
-    char* ndst = swa2_issue_dst<C>(nxt, wave);
+    const char* nrow = swa2_issue_row(G, ch, vb_, srow, wave);
+    char* ndst = swa2_issue_dst<C>(smem + C::REGION, wave);
     const int hrow = 4 * ch + g;
-    // both patches see the same window columns (the test of patch 0 serves both: its rows lie above those of patch 1, so
-    // wherever the own token of patch 1 is inside the grid that of patch 0 is too); a patch row outside the grid is
-    // folded into the row test
+    // a lane's keys of a chunk are columns of ONE halo row: the row test drops the lane's maximum and sends its exponents to
+    // -inf, nothing per score; the column test is the same for both patches (the own token of patch 1 lies below that of
+    // patch 0: inside the grid only where that one is)
     const bool row_vis[2] = {(hrow >= W[0].rlo) && (hrow <= W[0].rhi), (hrow >= W[1].rlo) && (hrow <= W[1].rhi) && W[1].cspan >= 0};
     // ---- scores of the chunk, one column group (16 keys) at a time
     float t[2][NKB][8];
@@ -101,7 +112,7 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
     auto mask_max = [&](const int p, const int cg, const f32x4& sv) {
       const int kb = cg >> 1, h4 = 4 * (cg & 1);
 #pragma unroll
-      for (int i = 0; i < 4; i++) t[p][kb][h4 + i] = swa2_visible(W[0], row_vis[p], cg, i, ncg) ? sv[i] : -INFINITY;
+      for (int i = 0; i < 4; i++) t[p][kb][h4 + i] = (unsigned)(4 * cg + i - W[0].clo) <= (unsigned)W[0].cspan ? sv[i] : -INFINITY;
       mx[p][cg & 3] = fmaxf(fmaxf(mx[p][cg & 3], t[p][kb][h4]), t[p][kb][h4 + 1]);
       mx[p][(cg + 2) & 3] = fmaxf(fmaxf(mx[p][(cg + 2) & 3], t[p][kb][h4 + 2]), t[p][kb][h4 + 3]);
     };
@@ -111,11 +122,12 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
     swa2_read_a<C, 0>(sK, L, ka);
     swa2_for<0, NCG>([&](auto cgc) {
       constexpr int cg = decltype(cgc)::value;
-      if constexpr (more) swa2_issue_one<C, cg>(st, nrow, ndst);
-      __builtin_amdgcn_sched_barrier(0);
       f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < KC; c++) {
+      swa2_for<0, KC>([&](auto cc) {
+        constexpr int c = decltype(cc)::value;
+        if constexpr (c == 0) swa2_issue_one<C, 2 * cg>(st, nrow, ndst);
+        if constexpr (c == KC / 2) swa2_issue_one<C, 2 * cg + 1>(st, nrow, ndst);
+        __builtin_amdgcn_sched_barrier(0);
         if constexpr (P0) s0 = Mma<CT>::mfma(ka[c], qf[0][c], s0);
         if constexpr (P1) s1 = Mma<CT>::mfma(ka[c], qf[1][c], s1);
         if constexpr (cg > 0) {
@@ -125,7 +137,7 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (cg + 1 < NCG) ka[c] = swa2_lds16(sK + swa2_read_a_off<C, cg + 1>(L, c));
         __builtin_amdgcn_sched_barrier(0);
-      }
+      });
       if constexpr (P0) sc[0][cg & 1] = s0;
       if constexpr (P1) sc[1][cg & 1] = s1;
     });
@@ -133,8 +145,8 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
     if constexpr (P1) mask_max(1, NCG - 1, sc[1][(NCG - 1) & 1]);
     // reference maxima move only when some score exceeds them by more than 2^8 after scaling (see swa2_fwd_kernel)
     float mloc[2] = {-INFINITY, -INFINITY};
-    if constexpr (P0) mloc[0] = wave_max4(fmaxf(fmaxf(mx[0][0], mx[0][1]), fmaxf(mx[0][2], mx[0][3])));
-    if constexpr (P1) mloc[1] = wave_max4(fmaxf(fmaxf(mx[1][0], mx[1][1]), fmaxf(mx[1][2], mx[1][3])));
+    if constexpr (P0) mloc[0] = wave_max4(row_vis[0] ? fmaxf(fmaxf(mx[0][0], mx[0][1]), fmaxf(mx[0][2], mx[0][3])) : -INFINITY);
+    if constexpr (P1) mloc[1] = wave_max4(row_vis[1] ? fmaxf(fmaxf(mx[1][0], mx[1][1]), fmaxf(mx[1][2], mx[1][3])) : -INFINITY);
     swa2_for<0, 2>([&](auto pc_) {
       constexpr int p = decltype(pc_)::value;
       if constexpr ((PM >> p) & 1) {
@@ -150,7 +162,9 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
         }
       }
     });
-    const float neg_m2[2] = {m_run[0] == -INFINITY ? 0.f : -m_run[0] * scale, m_run[1] == -INFINITY ? 0.f : -m_run[1] * scale};
+    float neg_m2[2];
+#pragma unroll
+    for (int p = 0; p < 2; p++) neg_m2[p] = row_vis[p] ? (m_run[p] == -INFINITY ? 0.f : -m_run[p] * scale) : -INFINITY;
     // ---- O^T += V^T P^T, 32 keys at a time: with two patches every V^T fragment feeds two products
     u32x4 va[4];
     u32x4 pb[2][2];
@@ -172,16 +186,21 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
         }
     };
 #pragma unroll
-    for (int d = 0; d < 4; d++) read_v(std::integral_constant<int, 0>{}, d);
-#pragma unroll
     for (int e = 0; e < 8; e++) prob(0, e);
+    swa2_wait_copies();
+    __syncthreads();   // V of the chunk has landed, every wave is done with its K
+    nrow = swa2_issue_row(G, ch + 1, kb_, srow, wave);
+    ndst = swa2_issue_dst<C>(smem, wave);
+#pragma unroll
+    for (int d = 0; d < 4; d++) read_v(std::integral_constant<int, 0>{}, d);
     swa2_for<0, NKB * NG>([&](auto ic) {
       constexpr int i = decltype(ic)::value, kb = i / NG, grp = i % NG;
-      if constexpr (more) swa2_issue_one<C, NCG + i>(st, nrow, ndst);
-      __builtin_amdgcn_sched_barrier(0);
       const u32x4 pk0 = pb[0][kb & 1], pk1 = pb[1][kb & 1];
-#pragma unroll
-      for (int d = 0; d < 4; d++) {
+      swa2_for<0, 4>([&](auto dc) {
+        constexpr int d = decltype(dc)::value;
+        if constexpr (more && d == 0) swa2_issue_one<C, 2 * i>(st, nrow, ndst);
+        if constexpr (more && d == 2) swa2_issue_one<C, 2 * i + 1>(st, nrow, ndst);
+        __builtin_amdgcn_sched_barrier(0);
         if constexpr (P0) acc[0][4 * grp + d] = Mma<CT>::mfma(va[d], pk0, acc[0][4 * grp + d]);
         if constexpr (P1) acc[1][4 * grp + d] = Mma<CT>::mfma(va[d], pk1, acc[1][4 * grp + d]);
         if constexpr (kb + 1 < NKB) {
@@ -193,7 +212,7 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (i + 1 < NKB * NG) read_v(std::integral_constant<int, i + 1>{}, d);
         __builtin_amdgcn_sched_barrier(0);
-      }
+      });
       if constexpr (grp == NG - 1) {
         // row sums of the rounded probabilities (the values the products above use)
 #pragma unroll
@@ -214,13 +233,16 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
   const int b_lo = ok1 ? W[1].ch_lo : a_hi + 1, b_hi = ok1 ? W[1].ch_hi : a_hi;
   const int w_lo = a_lo;
   const int both_lo = dlt_imax(a_lo, b_lo), both_hi = dlt_imin(a_hi, b_hi);
-  auto copy_only = [&](int ch) {
-    swa2_issue(st, G, ch + 1, sbase, srow, smem + ((ch + 1) & 1) * C::BUF, wave);
+  auto copy_only = [&](int ch, bool more) {
+    swa2_issue(st, G, ch, vb_, srow, smem + C::REGION, wave);
+    swa2_wait_copies();
+    __syncthreads();
+    if (more) swa2_issue(st, G, ch + 1, kb_, srow, smem, wave);
     swa2_wait_copies();
     __syncthreads();
   };
   auto round = [&](int ch, auto pm_tag) {
-    consume(ch, (Swa2Lds)smem + (ch & 1) * C::BUF, smem + ((ch + 1) & 1) * C::BUF, std::true_type{}, pm_tag);
+    consume(ch, std::true_type{}, pm_tag);
     swa2_wait_copies();
     __syncthreads();
   };
@@ -229,28 +251,26 @@ __global__ __launch_bounds__(SWA2_THREADS, 2) void swa2s_fwd_kernel(const Swa2Fw
   typedef std::integral_constant<int, 3> PmBoth;
   for (int pass = 0;;) {
     int ch = G.ch_first;
-    for (; ch < G.ch_last && ch < w_lo; ch++) copy_only(ch);
+    for (; ch < G.ch_last && ch < w_lo; ch++) copy_only(ch, true);
     for (; ch < G.ch_last && ch <= a_hi && ch < both_lo; ch++) round(ch, PmUpper{});
     for (; ch < G.ch_last && ch <= both_hi; ch++) round(ch, PmBoth{});
     for (; ch < G.ch_last && ch <= b_hi; ch++) round(ch, PmLower{});
-    for (; ch < G.ch_last; ch++) copy_only(ch);
+    for (; ch < G.ch_last; ch++) copy_only(ch, true);
     {
       const int cl = G.ch_last;
       const bool in0 = cl >= a_lo && cl <= a_hi, in1 = ok1 && cl >= b_lo && cl <= b_hi;
-      Swa2Lds cur = (Swa2Lds)smem + (cl & 1) * C::BUF;
-      char* nxt = smem + ((cl + 1) & 1) * C::BUF;
-      if (in0 && in1) consume(cl, cur, nxt, std::false_type{}, PmBoth{});
-      else if (in0) consume(cl, cur, nxt, std::false_type{}, PmUpper{});
-      else if (in1) consume(cl, cur, nxt, std::false_type{}, PmLower{});
+      if (in0 && in1) consume(cl, std::false_type{}, PmBoth{});
+      else if (in0) consume(cl, std::false_type{}, PmUpper{});
+      else if (in1) consume(cl, std::false_type{}, PmLower{});
+      else copy_only(cl, false);
     }
-    __syncthreads();   // every wave is done with both chunk buffers
+    __syncthreads();   // every wave is done with the chunk
     if (++pass >= a.plan.npass) break;
     G = swa2_pass_geom(G0, NCG, pass);
     W[0] = swa2_pass_window(W0[0], NCG, pass);
     W[1] = swa2_pass_window(W0[1], NCG, pass);
-    ncg = swa2_pass_ncg(G0.WC, NCG, pass);
-    swa2_stage_init(st, G, wave, lane, ssn2);
-    swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
+    swa2_stage_init(st, G, wave, lane, sn2);
+    swa2_issue(st, G, G.ch_first, kb_, srow, smem, wave);
     swa2_wait_copies();
     __syncthreads();
   }

@@ -263,3 +263,22 @@ def test_marching_fp32(th, tw, WR, WC):
         assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "marching"
         assert (o.cpu() - want).abs().max().item() <= FWD_TOL
         assert (lse.cpu() - lse_w).abs().max().item() <= LSE_TOL
+
+
+# two stacked patches per wave (streaming kernels, more workgroups than CUs): bands without a lower patch, one band and a bit, ragged
+# columns, both window classes, windows in column passes, tiles of 4 tokens, and K / V strides that keep the one-patch kernel
+@pytest.mark.parametrize("B,H,S,th,tw,WR,WC,d", [(1, 300, 1, 3, 5, 7, 7, 128), (1, 300, 1, 4, 16, 2, 3, 128), (1, 150, 1, 9, 15, 10, 10, 128), (2, 40, 1, 17, 18, 3, 8, 128),
+                                                 (1, 70, 1, 13, 33, 2, 12, 128), (1, 150, 1, 8, 17, 7, 9, 64), (1, 70, 1, 16, 31, 7, 2, 64), (1, 130, 4, 9, 7, 1, 1, 64),
+                                                 (1, 130, 4, 8, 5, 2, 2, 128)])
+def test_two_patches_per_wave(B, H, S, th, tw, WR, WC, d):
+    from dl_templates_amd import _lib
+    sw, N, scale = _swa(), S * th * tw, 0.15
+    q, k, v, _ = orc.make_qkv(N + d + WC, B, H, N, N, d, d, torch.bfloat16 if th % 2 else torch.float16)
+    want, lse_w = orc.tiled_swa_explicit(q.float(), k.float(), v.float(), S, th, tw, WR, WC, scale, return_lse2=True)
+    qg, kg, vg = (t.cuda() for t in (q, k, v))
+    wide = torch.zeros(B, H, N, d + 8, dtype=v.dtype, device="cuda")[..., :d]
+    for vx in (vg, wide.copy_(vg)):
+        o, lse = sw._forward(qg, kg, vx, sw._shape(qg, kg, vx, S, th, tw, WR, WC, scale), None)
+        assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
+        assert (o.float().cpu() - want).abs().max().item() <= FWD_TOL
+        assert (lse.cpu() - lse_w).abs().max().item() <= LSE_TOL
