@@ -49,6 +49,8 @@ int dlt_swag_launch_f32(const SwagArgs&, int nch, int ncg, int grid, hipStream_t
 int dlt_swag_launch_32_2(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_32_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_32_4(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_32_5(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
+int dlt_swag_launch_32_6(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_64_2(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_64_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_64_4(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
@@ -379,7 +381,7 @@ int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream
   return p.dk == 64 ? dlt_swa2_launch_bwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_bwd_128(a, swa2_ncg(p), (int)grid, stream);
 }
 
-// ---- marching token-grid kernels: head dim 32 or 64 exactly, windows up to 13 x 13, by window class ----------------------
+// ---- marching token-grid kernels: head dim 32 (windows up to 21 x 21) or 64 (13 x 13) exactly, by window class ----------------------
 int swag_class(int w) { return w <= 2 ? 2 : (4 + 2 * w + 3) / 4; }   // 4-wide blocks a patch's window spans
 bool swag_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
   return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && ((int64_t)p.g.TR * p.g.TC - 1) * st[2] * 2 + 2 * p.dk <= (((int64_t)1 << 31) - 1);
@@ -387,7 +389,9 @@ bool swag_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
 bool swag_eligible(const AttnProblem& p, const AttnTensors& t, const Swa1Class& c, bool bwd) {
   // rotation: 8 pairs per axis at head dim 64 in the forward pass, gradients turned back where q and k arrive rotated
   if (c.rope_mode != 0 && !(p.dk == 64 && p.rope.R == 8 && (!bwd || p.rope_prerot))) return false;
-  if (p.dk != p.dv || (p.dk != 32 && p.dk != 64) || p.g.WR > 6 || p.g.WC > 6) return false;
+  if (p.dk != p.dv || (p.dk != 32 && p.dk != 64)) return false;
+  const int wmax = p.dk == 32 ? 10 : 6;
+  if (p.g.WR > wmax || p.g.WC > wmax) return false;
   if (!swag_rows_ok(p, t.q, t.qs) || !swag_rows_ok(p, t.k, t.ks) || !swag_rows_ok(p, t.v, t.vs)) return false;
   if (!bwd)
     return swag_rows_ok(p, t.out_o, t.os) && (t.q_rot == nullptr || (swag_rows_ok(p, t.q_rot, t.qrs) && swag_rows_ok(p, t.k_rot, t.krs)));
@@ -448,7 +452,9 @@ int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
     switch (nch) {
       case 2: return dlt_swag_launch_32_2(a, p.dtype, ncg, bwd, (int)grid, stream);
       case 3: return dlt_swag_launch_32_3(a, p.dtype, ncg, bwd, (int)grid, stream);
-      default: return dlt_swag_launch_32_4(a, p.dtype, ncg, bwd, (int)grid, stream);
+      case 4: return dlt_swag_launch_32_4(a, p.dtype, ncg, bwd, (int)grid, stream);
+      case 5: return dlt_swag_launch_32_5(a, p.dtype, ncg, bwd, (int)grid, stream);
+      default: return dlt_swag_launch_32_6(a, p.dtype, ncg, bwd, (int)grid, stream);
     }
   }
   switch (nch) {

@@ -51,6 +51,10 @@ int swag_pick(const SwagArgs& a, int ncg, bool bwd, int grid, hipStream_t stream
     case 4: return bwd ? swag_bwd<TIO, 4, ROPE>(a, grid, stream) : swag_fwd<TIO, 4, ROPE>(a, grid, stream);
     default: break;
   }
+  if constexpr (DLT_D == 32) {   // head dim 32: the ring of a 24-column window fits as well
+    if (ncg == 5) return bwd ? swag_bwd<TIO, 5, ROPE>(a, grid, stream) : swag_fwd<TIO, 5, ROPE>(a, grid, stream);
+    if (ncg == 6) return bwd ? swag_bwd<TIO, 6, ROPE>(a, grid, stream) : swag_fwd<TIO, 6, ROPE>(a, grid, stream);
+  }
   return dlt_set_error(DLT_ERR_UNSUPPORTED, "marching token-grid kernels: no instantiation for %d column groups", ncg);
 }
 template <typename TIO>

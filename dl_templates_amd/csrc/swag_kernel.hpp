@@ -1,10 +1,12 @@
-// Marching kernels for token grids (b_size == 1) at head dims 32 and 64 and windows up to 13 x 13, with or without the fused
+// Marching kernels for token grids (b_size == 1) at head dim 64 and windows up to 13 x 13, and at head dim 32 and windows up to 21
+// x 21 (the ring of K and V of the widest class: 129 KB; at head dim 64 it would be twice that), with or without the fused
 // rotation (head dim 64, 8 rotary pairs per axis, rotated q / k kept): the shape of the benchmark's headline configuration.
 //
 // The window is a compile-time class: NCH x NCG blocks of 4 x 4 keys.  (An earlier version always computed 16 x 16 keys at head
 // dim 64, and head dim 32 ran zero-padded on the tile kernels, which stage every halo row once per band of 4 own rows: 32 slabs
 // of 84 x 82 tokens, d = 64, 11 x 7 window: forward 62 -> 35 us, dQ 79 -> 51, dK/dV 88 -> 53; 64 slabs of the same at d = 32:
-// 89 -> 42, 95 -> 50, 120 -> 56.)  A workgroup owns a strip of 4 PC columns and marches down the grid in steps of 4 PR rows
+// 89 -> 42, 95 -> 50, 120 -> 56; 32 slabs of 89 x 98, d = 32, 15 x 21: 94 -> 54, 98 -> 67, 123 -> 78; 16 of 13 x 74, 17 x 17: 14.0 ->
+// 9.6, 14.3 -> 10.3, 17.4 -> 11.4.)  A workgroup owns a strip of 4 PC columns and marches down the grid in steps of 4 PR rows
 // (PR = 8 / PC); wave w owns the 4 x 4 patch of column w % PC and row group w / PC.  The halo rows a step sees
 // (NCH + PR - 1 chunks of 4 rows, both streamed tensors) live in an LDS ring; the chunks of the next step travel HBM ->
 // registers while the current one computes.  The whole window is resident: the softmax is one-shot.

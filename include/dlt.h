@@ -263,7 +263,7 @@ int dlt_debug_copy(void* dst, const void* src, int64_t bytes, void* stream);
  * thread's latest forward / backward call (dlt_swa_*, dlt_flash_*) was routed to.  With dlt_dry_run(1) (per thread) those
  * calls validate their arguments and route, but launch nothing and touch no memory: pointers only need the alignment
  * of the real ones, so the query also works in a process without a GPU.
- *   MARCHING  token grids (b_size 1), head dims 32 and 64, windows up to 13 x 13 (rotation: head dim 64, 8 rotary pairs, in
+ *   MARCHING  token grids (b_size 1), head dim 32, windows up to 21 x 21, and 64, up to 13 x 13 (rotation: head dim 64, 8 rotary pairs, in
  *             the backward pass rotated q / k kept), also the forward pass of fp32 tensors at head dim 32; tiles of 16 or 32
  *             tokens at those head dims report FLASH
  *   STREAMING token grids, head dim 64 / 128, windows up to 93 columns (beyond 21 columns in column passes), no rotation;

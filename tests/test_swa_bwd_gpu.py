@@ -334,3 +334,21 @@ def test_marching_window_classes(th, tw, WR, WC, d, rope):
     assert (o.float().cpu() - want[0]).abs().max().item() <= 2e-2
     errs = (_rel(qg.grad, want[1]), _rel(kg.grad, want[2]), _rel(vg.grad, want[3]))
     assert max(errs) <= GRAD_TOL, errs
+
+
+# the marching kernels of head dim 32 beyond 13 x 13: classes of 5 and 6 blocks per direction, alone and with the smaller ones, grids
+# smaller than the window, around the strips and steps, more workgroups than CUs
+@pytest.mark.parametrize("B,H,th,tw,WR,WC", [(1, 3, 33, 35, 7, 8), (1, 2, 40, 31, 9, 10), (2, 3, 24, 48, 10, 10), (1, 3, 7, 5, 10, 9), (1, 2, 25, 17, 1, 7), (1, 2, 17, 33, 8, 2),
+                                             (1, 3, 31, 16, 4, 9), (1, 2, 16, 40, 10, 4), (1, 2, 9, 15, 6, 8), (1, 2, 41, 20, 8, 6), (2, 70, 16, 17, 9, 7), (1, 1, 1, 30, 7, 10)])
+def test_marching_large_windows(B, H, th, tw, WR, WC):
+    sw, N, d, scale = _swa(), th * tw, 32, 0.2
+    from dl_templates_amd import _lib
+    q, k, v, do = orc.make_qkv(N + d + WR, B, H, N, N, d, d, torch.float16 if th % 2 else torch.bfloat16)
+    want = orc.tiled_swa_grads(q.float(), k.float(), v.float(), do.float(), 1, th, tw, WR, WC, scale)
+    qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    o = sw.TiledSwa.apply(qg, kg, vg, 1, th, tw, WR, WC, scale)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "marching"
+    o.backward(do.cuda())
+    assert (o.float().cpu() - want[0]).abs().max().item() <= 2e-2
+    errs = (_rel(qg.grad, want[1]), _rel(kg.grad, want[2]), _rel(vg.grad, want[3]))
+    assert max(errs) <= GRAD_TOL, errs
