@@ -298,11 +298,14 @@ void swa2_split(const AttnProblem& p, int& ncg_class, int& npass) {
   else { ncg_class = 6; npass = n6; }
 }
 int swa2_ncg(const AttnProblem& p) { int c, n; swa2_split(p, c, n); return c; }
-// the problem without its rotation would run on the streaming kernels
-// and is large enough that the four extra launches (two out-of-place rotations, two in-place inverse rotations) do not
-// cost more than the tile kernels' repeated rotation (measured: a gain from about 10^5 tokens per call on)
+// The problem without its rotation would run on the streaming kernels, and the two extra launches (q and k rotated out of place,
+// dq and dk rotated back in place) cost less than the tile kernels' repeated rotation.  Measured step, tile kernels -> composed:
+// d = 64, 8 slabs of 134 x 66, 19 x 19 window 153 -> 117 us, 2 of 20 x 20, 17 x 17 43 -> 39; d = 128, 8 of 60 x 66, 19 x 19 149 -> 109, 4
+// of 33 x 40, 17 x 17 73 -> 58.  Narrow windows, of which the streaming kernels compute 16 columns, gain little or lose on small
+// grids (d = 128, 2 of 20 x 20, 7 x 7 40 -> 37; 4 of 13 x 17, 5 x 5 29.7 -> 32.2; d = 64, 32 of 24 x 30, 21 x 5 40.9 -> 43.4): up to 7 columns,
+// the tile kernels' place in the routing table, they are composed from 10^5 tokens on.
 bool swa2_compose_ok(const AttnProblem& p, const Swa1Class& c) {
-  return (c.D == 64 || c.D == 128) && p.dk == c.D && p.dv == c.D && (int64_t)p.B * p.H * p.g.TR * p.g.TC >= 131072;
+  return (c.D == 64 || c.D == 128) && p.dk == c.D && p.dv == c.D && (p.g.WC > 3 || (int64_t)p.B * p.H * p.g.TR * p.g.TC >= 131072);
 }
 
 void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan) {
@@ -739,9 +742,10 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
   }
   if (t.q_rot != nullptr) {
     // rotate q and k out of place, then run the plain operator on the rotated tensors (any kernel family)
-    rc = dlt_rope_rotate_copy(t.q, t.qs, t.q_rot, t.qrs, p.B, p.H, (int64_t)p.g.TR * p.g.XLq, p.dk, p.rope, p.dtype, stream);
-    if (rc == DLT_OK)
-      rc = dlt_rope_rotate_copy(t.k, t.ks, t.k_rot, t.krs, p.B, p.H, (int64_t)p.g.TR * p.g.XLk, p.dk, p.rope, p.dtype, stream);
+    const void* const src[2] = {t.q, t.k};
+    void* const dst[2] = {t.q_rot, t.k_rot};
+    const int64_t *const ss[2] = {t.qs, t.ks}, *const ds[2] = {t.qrs, t.krs};
+    rc = dlt_rope_rotate_copy(src, ss, dst, ds, 2, p.B, p.H, (int64_t)p.g.TR * p.g.XLq, p.dk, p.rope, p.dtype, stream);
     if (rc != DLT_OK) return rc;
     AttnProblem p2 = p;
     p2.rope = dlt_make_rope_dev(nullptr, 0);
@@ -819,9 +823,9 @@ int dlt_attn_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t st
     r.idx = p.rope.idx; r.row_cs = p.rope.row_cs; r.col_cs = p.rope.col_cs;
     r.row_cs_stride0 = p.rope.rs0; r.col_cs_stride0 = p.rope.cs0;
     r.n_rdim = p.rope.R; r.row_len = p.rope.row_len; r.col_len = p.rope.col_len;
-    rc = dlt_rope_inplace_4d(t.dq, t.dqs, p.B, p.H, (int64_t)p.g.TR * p.g.XLq, p.dk, &r, 1, p.dtype, stream);
-    if (rc != DLT_OK) return rc;
-    return dlt_rope_inplace_4d(t.dk, t.dks, p.B, p.H, (int64_t)p.g.TR * p.g.XLk, p.dk, &r, 1, p.dtype, stream);
+    void* const x[2] = {t.dq, t.dk};
+    const int64_t* const st[2] = {t.dqs, t.dks};
+    return dlt_rope_inplace_4d(x, st, 2, p.B, p.H, (int64_t)p.g.TR * p.g.XLq, p.dk, &r, 1, p.dtype, stream);
   }
   if (flash_eligible(p, t, true) && swat_eligible(p, t, true)) return swat_run(p, t, true, stream);
   if (flash_eligible(p, t, true)) return flash_backward(p, t, dc, stream);

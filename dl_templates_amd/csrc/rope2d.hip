@@ -150,15 +150,16 @@ __global__ __launch_bounds__(256) void rope2d_generic_kernel(RopeKArgs a) {
 // layout-agnostic companion of the in-place kernels, used when a caller wants the rotated tensor
 // next to the original and the attention kernels cannot produce it themselves.
 struct RopeCopyArgs {
-  const void* src;
-  void* dst;
-  int64_t ss[4], ds[4];
+  const void* src[2];   // blockIdx.z: which tensor
+  void* dst[2];
+  int64_t ss[2][4], ds[2][4];
   int32_t B, H, N, C;
   RopeDev r;
 };
 
 template <typename T>
 __global__ __launch_bounds__(256) void rope2d_copy_kernel(RopeCopyArgs a) {
+  const int64_t *const ss = a.ss[blockIdx.z], *const ds = a.ds[blockIdx.z];
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t per_bh = (int64_t)a.N * a.C;
   const int64_t bh = gid / per_bh;
@@ -166,9 +167,9 @@ __global__ __launch_bounds__(256) void rope2d_copy_kernel(RopeCopyArgs a) {
   const int64_t rem = gid - bh * per_bh;
   const int n = (int)(rem / a.C), d = (int)(rem - (int64_t)n * a.C);
   const int b = (int)(bh / a.H), h = (int)(bh - (int64_t)b * a.H);
-  const T* ps = reinterpret_cast<const T*>(a.src) + b * a.ss[0] + h * a.ss[1] + n * a.ss[2];
-  T* pd = reinterpret_cast<T*>(a.dst) + b * a.ds[0] + h * a.ds[1] + n * a.ds[2];
-  const T self = ps[d * a.ss[3]];
+  const T* ps = reinterpret_cast<const T*>(a.src[blockIdx.z]) + b * ss[0] + h * ss[1] + n * ss[2];
+  T* pd = reinterpret_cast<T*>(a.dst[blockIdx.z]) + b * ds[0] + h * ds[1] + n * ds[2];
+  const T self = ps[d * ss[3]];
   T out = self;
   if (d < 4 * a.r.R) {
     const int region = d / a.r.R, i = d - region * a.r.R, ax = region >> 1;
@@ -180,13 +181,13 @@ __global__ __launch_bounds__(256) void rope2d_copy_kernel(RopeCopyArgs a) {
       const float c = tab[0];
       const float s = a.r.inverse ? -tab[1] : tab[1];
       const bool is_x0 = (region & 1) == 0;
-      const float other = to_f(ps[(is_x0 ? d + a.r.R : d - a.r.R) * a.ss[3]]);
+      const float other = to_f(ps[(is_x0 ? d + a.r.R : d - a.r.R) * ss[3]]);
       float y0, y1;
       rotate(is_x0 ? to_f(self) : other, is_x0 ? other : to_f(self), c, s, y0, y1);
       out = from_f<T>(is_x0 ? y0 : y1);
     }
   }
-  pd[d * a.ds[3]] = out;
+  pd[d * ds[3]] = out;
 }
 
 // value of the lane whose index differs in bit log2(X)
@@ -205,14 +206,15 @@ template <int X> __device__ inline unsigned lane_xor(unsigned v) {
 // thread (32-byte runs per access) 15.7.
 template <typename T, int R8>
 __global__ __launch_bounds__(256) void rope2d_copy_vec_kernel(RopeCopyArgs a, int rows) {
+  const int64_t *const ss = a.ss[blockIdx.z], *const ds = a.ds[blockIdx.z];
   const int nch = a.C >> 3;
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t n = gid / nch;
   if (n >= a.N) return;                                   // partners share the token: they leave together
   const int c = (int)(gid - n * nch);
   const int total = a.B * a.H, b0 = blockIdx.y * rows, b1 = dlt_imin(b0 + rows, total);
-  const T* src = reinterpret_cast<const T*>(a.src) + n * a.ss[2] + 8 * c;
-  T* dst = reinterpret_cast<T*>(a.dst) + n * a.ds[2] + 8 * c;
+  const T* src = reinterpret_cast<const T*>(a.src[blockIdx.z]) + n * ss[2] + 8 * c;
+  T* dst = reinterpret_cast<T*>(a.dst[blockIdx.z]) + n * ds[2] + 8 * c;
   const int ax = c >= 2 * R8 ? 1 : 0;
   const bool is_x0 = (c & R8) == 0;
   const int32_t id = a.r.idx[n];
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(256) void rope2d_copy_vec_kernel(RopeCopyArgs a, in
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
       const int bh = dlt_imin(u0 + u, b1 - 1);
-      v[u] = *reinterpret_cast<const Vec8<T>*>(src + (bh / a.H) * a.ss[0] + (bh % a.H) * a.ss[1]);
+      v[u] = *reinterpret_cast<const Vec8<T>*>(src + (bh / a.H) * ss[0] + (bh % a.H) * ss[1]);
     }
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
@@ -255,7 +257,7 @@ __global__ __launch_bounds__(256) void rope2d_copy_vec_kernel(RopeCopyArgs a, in
             v[u].v[j] = from_f<T>(x + y);
           }
         }
-        *reinterpret_cast<Vec8<T>*>(dst + ((u0 + u) / a.H) * a.ds[0] + ((u0 + u) % a.H) * a.ds[1]) = v[u];
+        *reinterpret_cast<Vec8<T>*>(dst + ((u0 + u) / a.H) * ds[0] + ((u0 + u) % a.H) * ds[1]) = v[u];
       }
     }
   }
@@ -335,19 +337,24 @@ int rope_impl(void* const x[2], const int64_t* const st[2], const int64_t nb[2],
 
 }  // namespace
 
-int dlt_rope_rotate_copy(const void* src, const int64_t* ss, void* dst, const int64_t* ds, int B, int H, int64_t N, int C,
-                         const RopeDev& rope, int dtype, hipStream_t stream) {
+// out-of-place rotation of one or two [B, H, N, C] tensors in one launch
+int dlt_rope_rotate_copy(const void* const src[2], const int64_t* const ss[2], void* const dst[2], const int64_t* const ds[2], int ntens, int B, int H,
+                         int64_t N, int C, const RopeDev& rope, int dtype, hipStream_t stream) {
   if (dlt_route_dry()) return DLT_OK;
   RopeCopyArgs a;
-  a.src = src; a.dst = dst;
-  for (int i = 0; i < 4; i++) { a.ss[i] = ss[i]; a.ds[i] = ds[i]; }
   a.B = B; a.H = H; a.N = (int32_t)N; a.C = C;
   a.r = rope;
   const int es = dlt_elem_size(dtype), vb = 8 * es;
   const int r8 = rope.R / 8;
-  bool vec = rope.R % 8 == 0 && (r8 == 1 || r8 == 2 || r8 == 4) && C % (16 * r8) == 0 && ss[3] == 1 && ds[3] == 1 && (uintptr_t)src % vb == 0 && (uintptr_t)dst % vb == 0 &&
-             (uintptr_t)rope.row_cs % 16 == 0 && (uintptr_t)rope.col_cs % 16 == 0 && rope.rs0 % 4 == 0 && rope.cs0 % 4 == 0;
-  for (int i = 0; i < 3; i++) vec = vec && (ss[i] * es) % vb == 0 && (ds[i] * es) % vb == 0;
+  bool vec = rope.R % 8 == 0 && (r8 == 1 || r8 == 2 || r8 == 4) && C % (16 * r8) == 0 && (uintptr_t)rope.row_cs % 16 == 0 && (uintptr_t)rope.col_cs % 16 == 0 &&
+             rope.rs0 % 4 == 0 && rope.cs0 % 4 == 0;
+  for (int z = 0; z < 2; z++) {
+    const int x = z < ntens ? z : 0;
+    a.src[z] = src[x]; a.dst[z] = dst[x];
+    for (int i = 0; i < 4; i++) { a.ss[z][i] = ss[x][i]; a.ds[z][i] = ds[x][i]; }
+    vec = vec && ss[x][3] == 1 && ds[x][3] == 1 && (uintptr_t)src[x] % vb == 0 && (uintptr_t)dst[x] % vb == 0;
+    for (int i = 0; i < 3; i++) vec = vec && (ss[x][i] * es) % vb == 0 && (ds[x][i] * es) % vb == 0;
+  }
   const int64_t total = (int64_t)B * H * N * C;
   if (total == 0) return DLT_OK;
   const int64_t gx = ((vec ? N * (C / 8) : total) + 255) / 256;
@@ -355,10 +362,10 @@ int dlt_rope_rotate_copy(const void* src, const int64_t* ss, void* dst, const in
   dlt_timing_before(DLT_K_ROPE, stream);
   // rows per workgroup: as many as leave the chip ROPE_COPY_BLOCKS workgroups
   int rows = B * H;
-  while (rows > 1 && gx * ((B * H + rows - 1) / rows) < ROPE_COPY_BLOCKS) rows = (rows + 1) / 2;
+  while (rows > 1 && ntens * gx * ((B * H + rows - 1) / rows) < ROPE_COPY_BLOCKS) rows = (rows + 1) / 2;
   const int64_t gy = ((int64_t)B * H + rows - 1) / rows;
   if (vec && gy > 65535) vec = false;
-  const dim3 grid((unsigned)(vec ? gx : (total + 255) / 256), vec ? (unsigned)gy : 1u), block(256);
+  const dim3 grid((unsigned)(vec ? gx : (total + 255) / 256), vec ? (unsigned)gy : 1u, (unsigned)ntens), block(256);
   if (vec) {
     switch (dtype) {
       case DLT_BF16: launch_copy_vec<bf16_t>(a, r8, rows, grid, stream); break;
@@ -377,19 +384,27 @@ int dlt_rope_rotate_copy(const void* src, const int64_t* ss, void* dst, const in
   return DLT_OK;
 }
 
-// In-place rotation of a [B, H, N, C] tensor with any strides through the standalone kernels: one launch
-// when (B, H) collapses into one batch stride, else one per b.
-int dlt_rope_inplace_4d(void* x, const int64_t* st, int B, int H, int64_t N, int C, const dlt_rope_t* rope, int inverse,
+// In-place rotation of one or two [B, H, N, C] tensors with any strides through the standalone kernels: one launch
+// when (B, H) collapses into one batch stride for each, else one per b.
+int dlt_rope_inplace_4d(void* const x[2], const int64_t* const st[2], int ntens, int B, int H, int64_t N, int C, const dlt_rope_t* rope, int inverse,
                         int dtype, hipStream_t stream) {
   if (dlt_route_dry()) return DLT_OK;
-  const bool flat = B == 1 || st[0] == (int64_t)H * st[1];
-  const int64_t s3[3] = {st[1], st[2], st[3]};
+  bool flat = true;
+  int64_t s3[2][3];
+  for (int z = 0; z < ntens; z++) {
+    flat = flat && (B == 1 || st[z][0] == (int64_t)H * st[z][1]);
+    for (int i = 0; i < 3; i++) s3[z][i] = st[z][i + 1];
+  }
   const int es = dlt_elem_size(dtype);
+  const int64_t* const sts[2] = {s3[0], s3[1]};
   for (int b = 0; b < (flat ? 1 : B); b++) {
-    void* const xs[2] = {static_cast<char*>(x) + (int64_t)b * st[0] * es, nullptr};
-    const int64_t* const sts[2] = {s3, nullptr};
-    const int64_t nb[2] = {flat ? (int64_t)B * H : H, 0};
-    int rc = rope_impl(xs, sts, nb, 1, N, C, rope, inverse, dtype, stream);
+    void* xs[2] = {nullptr, nullptr};
+    int64_t nb[2] = {0, 0};
+    for (int z = 0; z < ntens; z++) {
+      xs[z] = static_cast<char*>(x[z]) + (int64_t)b * st[z][0] * es;
+      nb[z] = flat ? (int64_t)B * H : H;
+    }
+    int rc = rope_impl(xs, sts, nb, ntens, N, C, rope, inverse, dtype, stream);
     if (rc != DLT_OK) return rc;
   }
   return DLT_OK;
@@ -441,7 +456,10 @@ extern "C" int dlt_rope2d_copy(const void* src, const int64_t src_strides[3], vo
   if (rc != DLT_OK || n_batch * n_tokens == 0) return rc;
   DLT_REQUIRE(src != nullptr && dst != nullptr && src != dst, "rope2d_copy: src and dst must be two buffers");
   const int64_t ss[4] = {0, src_strides[0], src_strides[1], src_strides[2]}, ds[4] = {0, dst_strides[0], dst_strides[1], dst_strides[2]};
-  return dlt_rope_rotate_copy(src, ss, dst, ds, 1, (int)n_batch, n_tokens, (int)n_dim, dlt_make_rope_dev(rope, inverse), dtype, (hipStream_t)stream);
+  const void* const srcs[2] = {src, nullptr};
+  void* const dsts[2] = {dst, nullptr};
+  const int64_t *const sss[2] = {ss, nullptr}, *const dss[2] = {ds, nullptr};
+  return dlt_rope_rotate_copy(srcs, sss, dsts, dss, 1, 1, (int)n_batch, n_tokens, (int)n_dim, dlt_make_rope_dev(rope, inverse), dtype, (hipStream_t)stream);
 }
 
 extern "C" int dlt_rope2d_pair(void* x0, const int64_t x0_strides[3], int64_t n_batch0,

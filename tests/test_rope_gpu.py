@@ -244,3 +244,22 @@ def test_module_backward_rotates_out_of_place(C, R, dtype):
         (dx_w,) = torch.autograd.grad(orc.rope2d_ref(xg, idx, *tabs), (xg,), dy.float())
         assert torch.equal(y.detach().cpu(), want)
         assert torch.equal(dx.cpu(), dx_w.to(dtype))
+
+
+@pytest.mark.parametrize("d,R,th,tw,WR,WC,layout", [(64, 8, 9, 17, 8, 4, "bhnd"), (64, 8, 20, 13, 2, 9, "bnhd"), (128, 16, 7, 18, 3, 4, "bhnd"), (128, 32, 12, 12, 10, 5, "bnhd")])
+def test_rotation_composed_with_the_streaming_kernels(d, R, th, tw, WR, WC, layout):
+    """Small grids, windows of more than 7 columns: q and k rotated in one launch, dq and dk turned back in one (one per batch entry
+    where batch and head do not collapse)."""
+    from dl_templates_amd import _lib, tiled_swa as sw
+    B, H, N, scale = 2, 3, th * tw, 0.2
+    q, k, v, do = orc.make_qkv(d + R, B, H, N, N, d, d, torch.bfloat16)
+    idx, rcs, ccs = orc.make_rope_idx(2, th, tw, 0.1), orc.rope_tables(R, th), orc.rope_tables(R, tw)
+    want = orc.rope_swa_grads(q.float(), k.float(), v.float(), do.float(), idx, rcs, ccs, 1, th, tw, WR, WC, scale)
+    place = (lambda t: t.cuda()) if layout == "bhnd" else (lambda t: t.cuda().transpose(1, 2).contiguous().transpose(1, 2))
+    qg, kg, vg = (place(t).requires_grad_(True) for t in (q, k, v))
+    o = sw.TiledSwaRope.apply(qg, kg, vg, idx.cuda(), rcs.cuda(), ccs.cuda(), 1, th, tw, WR, WC, scale)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
+    got = (o,) + torch.autograd.grad(o, (qg, kg, vg), do.cuda())
+    assert (o.float().cpu() - want[0]).abs().max().item() <= 2e-2
+    for a, b in zip(got[1:], want[1:]):
+        assert ((a.float().cpu() - b).abs().max() / b.abs().max()).item() <= 5e-2
