@@ -286,11 +286,18 @@ struct AttnBackward : public Node {
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     if (!grads[0].defined()) return variable_list(3);
+    // Unpacked with autograd as it is: an unpack hook may run the forward pass again (activation checkpointing), and what it runs
+    // has to be recorded.
+    const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack();
+    Tensor idx_, row_, col_;
+    if (has_rope) {
+      idx_ = idx.unpack();
+      row_ = row.unpack();
+      col_ = col.unpack();
+    }
     at::AutoDispatchBelowADInplaceOrView below;
-    auto self = shared_from_this();
-    const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(self), lse_ = lse.unpack();
     Rope rope;
-    if (has_rope) rope = make_rope_for(idx.unpack(), row.unpack(), col.unpack(), q_, q_.size(2));
+    if (has_rope) rope = make_rope_for(idx_, row_, col_, q_, q_.size(2));
     auto g = run_backward(spec, q_, k_, v_, o_, lse_, pad_last(grads[0], v_.size(-1)), has_rope ? &rope : nullptr, rotated);
     return {cut_last(g[0], dk), cut_last(g[1], dk), cut_last(g[2], dv)};
   }
@@ -320,21 +327,21 @@ Tensor attention(Op op, const Tensor& q, const Tensor& k, const Tensor& v, const
     node = make_node<AttnBackward>();
     node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
   }
-  Tensor out;
+  pybind11::gil_scoped_release nogil;
+  Tensor out, pq = q, pk = k, pv = v;
+  Forward f;
+  Spec spec;
+  check_assert(q.dim() >= 2 && k.dim() == q.dim() && v.dim() == q.dim(), "q, k and v must have the same number of dims");
+  const int64_t dk = q.size(-1), dv = v.size(-1);
   {
-    pybind11::gil_scoped_release nogil;
     at::AutoDispatchBelowADInplaceOrView below;
-    Tensor pq = q, pk = k, pv = v;
-    check_assert(q.dim() >= 2 && k.dim() == q.dim() && v.dim() == q.dim(), "q, k and v must have the same number of dims");
-    const int64_t dk = q.size(-1), dv = v.size(-1);
     const Pad pad = op == Op::Flash ? flash_pad(dk, dv, q.scalar_type()) : op == Op::Swa ? swa_pad(dk, dv, q.scalar_type(), dims[0]) : Pad{dk, dv};
     if (C10_UNLIKELY(pad.dk != dk || pad.dv != dv)) {
       pq = pad_last(q, pad.dk);
       pk = pad_last(k, pad.dk);
       pv = pad_last(v, pad.dv);
     }
-    const Spec spec = op == Op::Flash ? flash_spec(pq, pk, pv, causal, scale) : op == Op::Image ? image_spec(pq, pk, pv, dims, scale)
-                                                                                                   : swa_spec(pq, pk, pv, dims, scale);
+    spec = op == Op::Flash ? flash_spec(pq, pk, pv, causal, scale) : op == Op::Image ? image_spec(pq, pk, pv, dims, scale) : swa_spec(pq, pk, pv, dims, scale);
     Rope rope;
     if (rope_t != nullptr) {
       check_assert(rope_t[1].dim() == 3 && rope_t[2].dim() == 3 && rope_t[1].size(1) == rope_t[2].size(1), "row and column table must have one R");
@@ -342,28 +349,29 @@ Tensor attention(Op op, const Tensor& q, const Tensor& k, const Tensor& v, const
       require_gpu(pq, pk, pv);
       rope = make_rope_for(rope_t[0], rope_t[1], rope_t[2], pq, pq.size(2));
     }
-    Forward f = run_forward(spec, pq, pk, pv, rope_t ? &rope : nullptr, keep_rot);
+    f = run_forward(spec, pq, pk, pv, rope_t ? &rope : nullptr, keep_rot);
     out = cut_last(f.o, dv);
-    if (grad) {
-      node->spec = spec;
-      node->dk = dk;
-      node->dv = dv;
-      node->q = SavedVariable(keep_rot ? f.q_rot : pq, false);
-      node->k = SavedVariable(keep_rot ? f.k_rot : pk, false);
-      node->v = SavedVariable(pv, false);
-      node->lse = SavedVariable(f.lse, false);
-      if (rope_t != nullptr) {
-        node->has_rope = true;
-        node->rotated = keep_rot;
-        node->idx = SavedVariable(rope_t[0], false);
-        node->row = SavedVariable(rope_t[1], false);
-        node->col = SavedVariable(rope_t[2], false);
-      }
-      const bool whole = out.is_same(f.o);
-      if (!whole) node->o = SavedVariable(f.o, false);
-      torch::autograd::set_history(out, node);
-      if (whole) node->o = SavedVariable(out, true);
+  }
+  // saved with autograd as it is: pack hooks are the caller's code
+  if (grad) {
+    node->spec = spec;
+    node->dk = dk;
+    node->dv = dv;
+    node->q = SavedVariable(keep_rot ? f.q_rot : pq, false);
+    node->k = SavedVariable(keep_rot ? f.k_rot : pk, false);
+    node->v = SavedVariable(pv, false);
+    node->lse = SavedVariable(f.lse, false);
+    if (rope_t != nullptr) {
+      node->has_rope = true;
+      node->rotated = keep_rot;
+      node->idx = SavedVariable(rope_t[0], false);
+      node->row = SavedVariable(rope_t[1], false);
+      node->col = SavedVariable(rope_t[2], false);
     }
+    const bool whole = out.is_same(f.o);
+    if (!whole) node->o = SavedVariable(f.o, false);
+    torch::autograd::set_history(out, node);
+    if (whole) node->o = SavedVariable(out, true);
   }
   return out;
 }
@@ -394,8 +402,9 @@ void rotate_inplace(const Tensor& x, const Rows& r, const Rope& rope, bool inver
 variable_list RopeBackward::apply(variable_list&& grads) {
   std::lock_guard<std::mutex> lock(mutex_);
   if (!grads[0].defined()) return variable_list(1);
+  const Tensor idx_ = idx.unpack(), row_ = row.unpack(), col_ = col.unpack();   // before the guard: see AttnBackward
   at::AutoDispatchBelowADInplaceOrView below;
-  const Rope rope = make_rope(idx.unpack(), row.unpack(), col.unpack());
+  const Rope rope = make_rope(idx_, row_, col_);
   require_gpu(grads[0], rope.idx, rope.row, rope.col);
   Tensor dy = grads[0];
   Rows rs, rd;

@@ -1,0 +1,87 @@
+"""The operators inside autograd as a program uses it: activation checkpointing and saved-tensor hooks."""
+import math
+
+import pytest
+import torch
+from torch.utils.checkpoint import checkpoint
+
+from oracle import attn_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+TH, TW, D = 6, 10, 64
+SCALE = 1 / math.sqrt(D)
+
+
+def _rope_args():
+    return (orc.make_rope_idx(1, TH, TW, 0.1).cuda(), orc.rope_tables(8, TH).cuda(), orc.rope_tables(8, TW).cuda())
+
+
+def _rotation_module(x):
+    from dl_templates_amd.fused_rope2d import FusedInplaceRotaryPositionEncoding2D as Module
+    return Module(32, TH, TW).cuda()(x, _rope_args()[0])
+
+
+def _ops():
+    """name -> (operator on three tensors, shape of the tensors); every operator with an autograd node."""
+    from dl_templates_amd.flash_attn import attention
+    from dl_templates_amd.fused_rope2d import RotaryPE2D
+    from dl_templates_amd.tiled_swa import TiledSwa, TiledSwaImage, TiledSwaRope
+    tokens, dims = (1, 2, TH * TW, D), (1, TH, TW, 3, 3, SCALE)
+    return {
+        "flash": (lambda q, k, v: attention(q, k, v, False, SCALE), tokens),
+        "flash_padded": (lambda q, k, v: attention(q, k, v, False, SCALE), (1, 2, 50, 36)),
+        "swa": (lambda q, k, v: TiledSwa.apply(q, k, v, *dims), tokens),
+        "swa_rope": (lambda q, k, v: TiledSwaRope.apply(q, k, v, *_rope_args(), *dims), tokens),
+        "swa_rope_again": (lambda q, k, v: TiledSwaRope.apply(q, k, v, *_rope_args(), *dims, False), tokens),
+        "image": (lambda q, k, v: TiledSwaImage.apply(q, k, v, 2, 2, 1, 1, SCALE), (1, TH, TW, 2, D)),
+        "rotation": (lambda q, k, v: RotaryPE2D.apply((q * k * v)[0], *_rope_args()), tokens),
+        "rotation_module": (lambda q, k, v: _rotation_module(q * k * v), tokens),
+    }
+
+
+OPS = ["flash", "flash_padded", "swa", "swa_rope", "swa_rope_again", "image", "rotation", "rotation_module"]
+
+
+def _inputs(name, dtype=torch.bfloat16):
+    op, shape = _ops()[name]
+    gen = torch.Generator().manual_seed(len(name))
+    return op, [torch.randn(shape, generator=gen).to(dtype).cuda().requires_grad_(True) for _ in range(3)]
+
+
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("name", OPS)
+def test_checkpointed_region(name, first):
+    """Non-reentrant checkpointing runs the region again inside an unpack hook of its nodes.  Bit-equal to the plain step, with the
+    operator as the last of the region (its node is the first one unpacked) and as the first."""
+    op, x = _inputs(name)
+    block = (lambda q, k, v: op(q * 2, k * 2, v * 2) * 3) if first else (lambda q, k, v: op(q * 2, k * 2, v * 2))
+    o = block(*x)
+    do = torch.randn_like(o)
+    want = torch.autograd.grad(o, x, do)
+    got_o = checkpoint(block, *x, use_reentrant=False)
+    assert torch.equal(got_o, o)
+    for g, w in zip(torch.autograd.grad(got_o, x, do), want):
+        assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("name", OPS)
+def test_saved_tensor_hooks_run_with_autograd_on(name):
+    op, x = _inputs(name)
+    o = op(*x)
+    do = torch.randn_like(o)
+    want = torch.autograd.grad(o, x, do)
+    leaf, seen = torch.ones(1, device="cuda", requires_grad=True), []
+
+    def hook(where):
+        def run(t):
+            with torch.enable_grad():   # hooks run with gradients off
+                seen.append((where, (leaf * 2).requires_grad))
+            return t.cpu() if where == "pack" else t.cuda()
+        return run
+
+    with torch.autograd.graph.saved_tensors_hooks(hook("pack"), hook("unpack")):
+        o2 = op(*x)
+    got = torch.autograd.grad(o2, x, do)
+    assert {w for w, _ in seen} == {"pack", "unpack"} and all(on for _, on in seen), seen
+    assert torch.equal(o2, o) and all(torch.equal(a, b) for a, b in zip(got, want))
