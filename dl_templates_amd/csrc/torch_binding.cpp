@@ -17,6 +17,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -403,20 +404,28 @@ variable_list RopeBackward::apply(variable_list&& grads) {
   std::lock_guard<std::mutex> lock(mutex_);
   if (!grads[0].defined()) return variable_list(1);
   const Tensor idx_ = idx.unpack(), row_ = row.unpack(), col_ = col.unpack();   // before the guard: see AttnBackward
-  at::AutoDispatchBelowADInplaceOrView below;
-  const Rope rope = make_rope(idx_, row_, col_);
-  require_gpu(grads[0], rope.idx, rope.row, rope.col);
-  Tensor dy = grads[0];
-  Rows rs, rd;
-  if (!rows_of(dy, rs)) {
-    dy = dy.contiguous();
-    rows_of(dy, rs);
+  Tensor dy = grads[0], dx;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Rope rope = make_rope(idx_, row_, col_);
+    require_gpu(dy, rope.idx, rope.row, rope.col);
+    Rows rs, rd;
+    if (!rows_of(dy, rs)) {
+      dy = dy.contiguous();
+      rows_of(dy, rs);
+    }
+    c10::DeviceGuard guard(dy.device());
+    dx = empty(dy.sizes(), dy.scalar_type(), dy);
+    rows_of(dx, rd);
+    check_rc(dlt_rope2d_copy(dy.const_data_ptr(), rs.s, dx.mutable_data_ptr(), rd.s, rd.nb, dy.size(-2), dy.size(-1), &rope.d, 1, dtype_code(dy),
+                             stream_of(dy)));
   }
-  c10::DeviceGuard guard(dy.device());
-  Tensor dx = empty(dy.sizes(), dy.scalar_type(), dy);
-  rows_of(dx, rd);
-  check_rc(dlt_rope2d_copy(dy.const_data_ptr(), rs.s, dx.mutable_data_ptr(), rd.s, rd.nb, dy.size(-2), dy.size(-1), &rope.d, 1, dtype_code(dy),
-                           stream_of(dy)));
+  // differentiable once: a second derivative raises where it is asked for (without a graph it would be dropped in silence)
+  if (C10_UNLIKELY(at::GradMode::is_enabled() && grads[0].requires_grad())) {
+    std::shared_ptr<torch::autograd::DelayedError> once(
+        new torch::autograd::DelayedError("trying to differentiate twice a function that was marked with @once_differentiable", 1), torch::autograd::deleteNode);
+    return (*once)({dx.detach().requires_grad_(true)});
+  }
   return {dx};
 }
 

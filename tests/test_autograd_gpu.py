@@ -1,4 +1,4 @@
-"""The operators inside autograd as a program uses it: activation checkpointing and saved-tensor hooks."""
+"""The operators inside autograd as a program uses it: activation checkpointing, saved-tensor hooks, second derivatives."""
 import math
 
 import pytest
@@ -85,3 +85,16 @@ def test_saved_tensor_hooks_run_with_autograd_on(name):
     got = torch.autograd.grad(o2, x, do)
     assert {w for w, _ in seen} == {"pack", "unpack"} and all(on for _, on in seen), seen
     assert torch.equal(o2, o) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("name", ["rotation", "rotation_module"])
+def test_rotation_refuses_a_second_derivative(name):
+    """A gradient penalty through the rotation raises; ``create_graph`` alone, for first derivatives, is fine."""
+    op, x = _inputs(name, torch.float32)
+    o = op(*x)
+    want = torch.autograd.grad((o ** 2).sum(), x, retain_graph=True)
+    got = torch.autograd.grad((o ** 2).sum(), x, create_graph=True)
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    with pytest.raises(RuntimeError, match="differentiate twice"):
+        ((o ** 2).sum() + 10 * sum((g ** 2).sum() for g in got)).backward()
