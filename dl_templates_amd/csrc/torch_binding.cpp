@@ -6,7 +6,9 @@
 // descriptor and stride arrays built object by object, a device guard object, three to seven torch.empty calls from
 // Python), so every such step waited for the host.  Here the same work is done on the tensor structs themselves.
 //
-// Nothing is kept from one call for the next and nothing is launched that the Python version did not launch.
+// Nothing is kept from one call for the next and nothing is launched that the Python version did not launch.  The Python
+// classes (torch.autograd.Function) stay the general path: a compiled entry point answers NotImplemented to every call that is
+// not a plain eager one (see plain() below), and apply() of its class then goes on through the class.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -14,6 +16,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/function.h>
@@ -101,6 +104,22 @@ Tensor empty(at::IntArrayRef size, at::ScalarType st, const Tensor& like) {
 Tensor grad_like(const Tensor& t) { return t.is_contiguous() ? empty(t.sizes(), t.scalar_type(), t) : at::empty_like(t); }
 
 const int64_t* st(const Tensor& t) { return t.strides().data(); }
+
+// ---- which calls the compiled nodes take -----------------------------------------------------------
+// Plain eager calls: no trace, transform (torch.func) or dispatch mode is active, the tensors are ordinary strided ones and
+// none carries a forward-mode tangent.  Everything else (and its errors) belongs to the autograd.Function classes: a node made
+// here would drop the tangent, be missing from the trace, or hide from the mode.
+bool plain_keys(c10::DispatchKeySet ks, c10::DispatchKeySet allowed) {
+  return (ks.raw_repr() & ~allowed.raw_repr() & ~c10::full_backend_mask) == 0;
+}
+template <typename... T>
+bool plain(const T&... ts) {
+  using K = c10::DispatchKey;
+  constexpr c10::DispatchKeySet MODES = c10::DispatchKeySet({K::BackendSelect, K::ADInplaceOrView}) | c10::autocast_dispatch_keyset;
+  constexpr c10::DispatchKeySet TENSOR = c10::DispatchKeySet({K::Dense, K::ADInplaceOrView, K::AutogradFunctionality}) | c10::autocast_dispatch_keyset;
+  auto one = [&](const Tensor& t) { return plain_keys(t.key_set(), TENSOR) && !t._fw_grad(/*level=*/0).defined(); };
+  return plain_keys(c10::impl::tls_local_dispatch_key_set().included_, MODES) && (one(ts) && ...);
+}
 
 // ---- rotary operands --------------------------------------------------------------------------
 struct Rope {
@@ -286,7 +305,7 @@ struct AttnBackward : public Node {
   }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
-    if (!grads[0].defined()) return variable_list(3);
+    if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();   // as torch.autograd.Function does
     // Unpacked with autograd as it is: an unpack hook may run the forward pass again (activation checkpointing), and what it runs
     // has to be recorded.
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack();
@@ -402,7 +421,7 @@ void rotate_inplace(const Tensor& x, const Rows& r, const Rope& rope, bool inver
 
 variable_list RopeBackward::apply(variable_list&& grads) {
   std::lock_guard<std::mutex> lock(mutex_);
-  if (!grads[0].defined()) return variable_list(1);
+  if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
   const Tensor idx_ = idx.unpack(), row_ = row.unpack(), col_ = col.unpack();   // before the guard: see AttnBackward
   Tensor dy = grads[0], dx;
   {
@@ -493,6 +512,7 @@ PyObject* py_tiled_swa(PyObject*, PyObject* const* a, Py_ssize_t n) {
   count(n, 9, 9);
   int64_t dims[5];
   for (int i = 0; i < 5; i++) dims[i] = int_arg(a[3 + i]);
+  if (!plain(tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]))) Py_RETURN_NOTIMPLEMENTED;
   return THPVariable_Wrap(attention(Op::Swa, tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]), nullptr, dims, false, float_arg(a[8]), false, true));
   END_HANDLE_TH_ERRORS
 }
@@ -512,6 +532,7 @@ PyObject* py_tiled_swa_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t dims[5];
   for (int i = 0; i < 5; i++) dims[i] = int_arg(a[6 + i]);
   const Tensor rope[3] = {tensor_arg(a[3]), tensor_arg(a[4]), tensor_arg(a[5])};
+  if (!plain(tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]), rope[0], rope[1], rope[2])) Py_RETURN_NOTIMPLEMENTED;
   const bool keep = n < 13 || a[12] == Py_None || bool_arg(a[12]);
   return THPVariable_Wrap(attention(Op::Swa, tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]), rope, dims, false, float_arg(a[11]), keep, true));
   END_HANDLE_TH_ERRORS
@@ -522,6 +543,7 @@ PyObject* py_tiled_swa_image(PyObject*, PyObject* const* a, Py_ssize_t n) {
   count(n, 8, 8);
   int64_t dims[4];
   for (int i = 0; i < 4; i++) dims[i] = int_arg(a[3 + i]);
+  if (!plain(tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]))) Py_RETURN_NOTIMPLEMENTED;
   return THPVariable_Wrap(attention(Op::Image, tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]), nullptr, dims, false, float_arg(a[7]), false, true));
   END_HANDLE_TH_ERRORS
 }
@@ -529,6 +551,7 @@ PyObject* py_tiled_swa_image(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   count(n, 5, 5);
+  if (!plain(tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]))) Py_RETURN_NOTIMPLEMENTED;
   return THPVariable_Wrap(attention(Op::Flash, tensor_arg(a[0]), tensor_arg(a[1]), tensor_arg(a[2]), nullptr, nullptr, bool_arg(a[3]), float_arg(a[4]),
                                     false, true));
   END_HANDLE_TH_ERRORS
@@ -577,6 +600,40 @@ PyObject* py_swa_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// (q, k, v, bh, bw, row, col, scale) -> (o, lse2) and (q, k, v, o, lse2, do, the same 5 numbers) -> (dq, dk, dv): no graph
+PyObject* py_image_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  count(n, 8, 8);
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor &q = tensor_arg(a[0]), &k = tensor_arg(a[1]), &v = tensor_arg(a[2]);
+  const int64_t dims[4] = {int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), int_arg(a[6])};
+  const Forward f = run_forward(image_spec(q, k, v, dims, float_arg(a[7])), q, k, v, nullptr, false);
+  return Py_BuildValue("(NN)", THPVariable_Wrap(f.o), THPVariable_Wrap(f.lse));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_image_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  count(n, 11, 11);
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor &q = tensor_arg(a[0]), &k = tensor_arg(a[1]), &v = tensor_arg(a[2]), &o = tensor_arg(a[3]), &lse = tensor_arg(a[4]), &d_o = tensor_arg(a[5]);
+  const int64_t dims[4] = {int_arg(a[6]), int_arg(a[7]), int_arg(a[8]), int_arg(a[9])};
+  auto g = run_backward(image_spec(q, k, v, dims, float_arg(a[10])), q, k, v, o, lse, d_o, nullptr, false);
+  return Py_BuildValue("(NNN)", THPVariable_Wrap(g[0]), THPVariable_Wrap(g[1]), THPVariable_Wrap(g[2]));
+  END_HANDLE_TH_ERRORS
+}
+
+// (q, k, v, o, M, do, causal, scale) -> (dq, dk, dv) without a graph and without padding
+PyObject* py_flash_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  count(n, 8, 8);
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor &q = tensor_arg(a[0]), &k = tensor_arg(a[1]), &v = tensor_arg(a[2]), &o = tensor_arg(a[3]), &lse = tensor_arg(a[4]), &d_o = tensor_arg(a[5]);
+  auto g = run_backward(flash_spec(q, k, v, bool_arg(a[6]), float_arg(a[7])), q, k, v, o, lse, d_o, nullptr, false);
+  return Py_BuildValue("(NNN)", THPVariable_Wrap(g[0]), THPVariable_Wrap(g[1]), THPVariable_Wrap(g[2]));
+  END_HANDLE_TH_ERRORS
+}
+
 // (q, k, v, causal, scale) -> (o, M) without a graph and without padding
 PyObject* py_flash_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -593,6 +650,7 @@ PyObject* py_rope_apply(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   count(n, 4, 4);
   const Tensor& x = tensor_arg(a[0]);
+  if (!plain(x, tensor_arg(a[1]), tensor_arg(a[2]), tensor_arg(a[3]))) Py_RETURN_NOTIMPLEMENTED;
   if (x.dim() != 3) raise_py(PyExc_ValueError, "x must have shape [B', N, C]");
   Rows r;
   rows_of(x, r);
@@ -607,6 +665,7 @@ PyObject* py_rope_heads(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   count(n, 4, 4);
   const Tensor& x = tensor_arg(a[0]);
+  if (!plain(x, tensor_arg(a[1]), tensor_arg(a[2]), tensor_arg(a[3]))) Py_RETURN_NOTIMPLEMENTED;
   if (x.dim() != 4) raise_py(PyExc_ValueError, "x must have shape [B, H, N, C]");
   Rows r;
   if (C10_LIKELY(rows_of(x, r))) {
@@ -670,7 +729,7 @@ PyObject* py_pad_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define DLT_FN(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
 PyMethodDef METHODS[] = {DLT_FN(tiled_swa), DLT_FN(tiled_swa_fwd), DLT_FN(tiled_swa_rope), DLT_FN(tiled_swa_image), DLT_FN(flash), DLT_FN(swa_forward),
-                         DLT_FN(swa_backward), DLT_FN(flash_forward), DLT_FN(rope_apply), DLT_FN(rope_heads), DLT_FN(rope_inplace), DLT_FN(rope_pair),
+                         DLT_FN(swa_backward), DLT_FN(image_forward), DLT_FN(image_backward), DLT_FN(flash_forward), DLT_FN(flash_backward), DLT_FN(rope_apply), DLT_FN(rope_heads), DLT_FN(rope_inplace), DLT_FN(rope_pair),
                          DLT_FN(pad_plan), {nullptr, nullptr, 0, nullptr}};
 #undef DLT_FN
 

@@ -1,6 +1,6 @@
 """Fused in-place 2D rotary position encoding (drop-in for src/fused_rope2d.py).
 
-Same names and call signatures as the reference: ``RotaryPE2D`` (``apply`` with gradients,
+Same names and call signatures as the reference: ``RotaryPE2D`` (autograd.Function,
 src/fused_rope2d.py:124-168), ``FusedInplaceRotaryPositionEncoding2D`` (:171-201).  The
 Triton kernels are replaced by the gfx950 HIP kernel behind ``dlt_rope2d``.
 """
@@ -16,13 +16,31 @@ def _launch(x: torch.Tensor, idx, row_cs, col_cs, inverse: bool) -> None:
     _lib.native.rope_inplace(x, idx, row_cs, col_cs, inverse)
 
 
-class RotaryPE2D:
+class RotaryPE2D(torch.autograd.Function):
     """``apply(x[B', N, C], idx, row_cs_buffer, col_cs_buffer)``: x is rotated IN PLACE and returned
-    (src/fused_rope2d.py:126-145); the backward pass rotates the gradient back (:148-168)."""
+    (src/fused_rope2d.py:126-145); the backward pass rotates the gradient back (:148-168).  Plain eager calls run as one compiled
+    node (csrc/torch_binding.cpp), any other (trace, transform, dispatch mode, forward-mode tangent) through this class."""
+
+    @classmethod
+    def apply(cls, *args):
+        y = _lib.native.rope_apply(*args) if cls is RotaryPE2D else NotImplemented
+        return super().apply(*args) if y is NotImplemented else y
 
     @staticmethod
-    def apply(*args):
-        return _lib.native.rope_apply(*args)
+    def forward(ctx, x, idx, row_cs_buffer, col_cs_buffer):
+        assert row_cs_buffer.shape[1] == col_cs_buffer.shape[1], "row and column table must have one R"
+        assert idx.shape[0] == x.shape[1], "idx must have one entry per token"
+        _launch(x, idx, row_cs_buffer, col_cs_buffer, False)
+        ctx.mark_dirty(x)
+        ctx.save_for_backward(idx, row_cs_buffer, col_cs_buffer)
+        return x
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, do):
+        dx = do.clone()
+        _launch(dx, *ctx.saved_tensors, True)
+        return dx, None, None, None
 
 
 def rope2d_qk_(q: torch.Tensor, k: torch.Tensor, idx: torch.Tensor, row_cs_buffer: torch.Tensor,
@@ -64,4 +82,9 @@ class FusedInplaceRotaryPositionEncoding2D(torch.nn.Module):
 
     def forward(self, x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
         # x: [B, Head, N, C] idx: [N, ]
-        return _lib.native.rope_heads(x, idx, self.row_buffer.cs_components, self.col_buffer.cs_components)
+        rope = (idx, self.row_buffer.cs_components, self.col_buffer.cs_components)
+        y = _lib.native.rope_heads(x, *rope)
+        if y is NotImplemented:
+            B, H, N, C = x.shape
+            y = RotaryPE2D.apply(x.reshape((-1, N, C)), *rope).reshape(x.shape)
+        return y

@@ -1,9 +1,10 @@
 """Tiled 2D sliding-window flash attention (drop-in for src/tiled_swa.py).
 
-``TiledSwa.apply`` keeps the reference's autograd contract (src/tiled_swa.py:602-689): positional
-arguments ``(q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale)``, gradients for q, k and v.  The graph
-nodes and the argument checks are compiled (csrc/torch_binding.cpp).  ``tiled_swa_fwd`` (:564-600) is the no-grad
-forward.  Deliberate differences from the reference, all documented in the C header:
+``TiledSwa`` keeps the reference's autograd contract (src/tiled_swa.py:602-689): an ``autograd.Function`` with positional
+arguments ``(q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale)`` and a backward that returns
+``(dq, dk, dv, None * 6)``.  ``apply`` runs plain eager calls as one compiled node (csrc/torch_binding.cpp); under a trace, a
+``torch.func`` transform or a dispatch mode, and with forward-mode tangents, the class itself runs.  ``tiled_swa_fwd``
+(:564-600) is the no-grad forward.  Deliberate differences from the reference, all documented in the C header:
 outputs have the dtype and device of ``q`` (the reference hard-codes fp16 and the default
 device, :608-609), the saved log-sum-exp is fp32, and tiles smaller than 16 tokens have a
 backward (the reference raises, :660-661).
@@ -76,15 +77,40 @@ def tiled_swa_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b_size: int
     return _lib.native.tiled_swa_fwd(q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale)
 
 
-class TiledSwa:
+def _pad_last(x, d):
+    return x if x.shape[-1] == d else torch.nn.functional.pad(x, (0, d - x.shape[-1]))
+
+
+def _cut_last(x, d):
+    return x if x.shape[-1] == d else x[..., :d].contiguous()
+
+
+class TiledSwa(torch.autograd.Function):
     """``apply(q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale)`` -> o; gradients for q, k, v."""
 
+    @classmethod
+    def apply(cls, *args):
+        o = _lib.native.tiled_swa(*args) if cls is TiledSwa else NotImplemented
+        return super().apply(*args) if o is NotImplemented else o
+
     @staticmethod
-    def apply(*args):
-        return _lib.native.tiled_swa(*args)
+    def forward(ctx, q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale):
+        ctx.dims, plan = (q.shape[-1], v.shape[-1]), _pad_plan(q, v, b_size)
+        if plan is not None:
+            q, k, v = _pad_last(q, plan[0]), _pad_last(k, plan[0]), _pad_last(v, plan[1])
+        ctx.shape = _shape(q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale)
+        o, m = _forward(q, k, v, ctx.shape, None)
+        ctx.save_for_backward(q, k, v, m, o)
+        return _cut_last(o, ctx.dims[1])
+
+    @staticmethod
+    def backward(ctx, do):
+        q, k, v, m, o = ctx.saved_tensors
+        dq, dk, dv = _backward(q, k, v, o, m, _pad_last(do, v.shape[-1]), ctx.shape, None)
+        return (_cut_last(dq, ctx.dims[0]), _cut_last(dk, ctx.dims[0]), _cut_last(dv, ctx.dims[1])) + (None,) * 6
 
 
-class TiledSwaRope:
+class TiledSwaRope(torch.autograd.Function):
     """o = TiledSwa(rope(q), rope(k), v) with the rotation fused into the q / k tile loads.
 
     ``apply(q, k, v, idx, row_cs_buffer, col_cs_buffer, b_size, t_height, t_width, row_size, col_size, sm_scale,
@@ -95,12 +121,39 @@ class TiledSwaRope:
     per-call argument, kept in the call's own graph node: nothing is shared between calls or threads.
     """
 
+    @classmethod
+    def apply(cls, *args):
+        o = _lib.native.tiled_swa_rope(*args) if cls is TiledSwaRope else NotImplemented
+        return super().apply(*args) if o is NotImplemented else o
+
     @staticmethod
-    def apply(*args):
-        return _lib.native.tiled_swa_rope(*args)
+    def forward(ctx, q, k, v, idx, row_cs_buffer, col_cs_buffer, b_size, t_height, t_width, row_size, col_size,
+                sm_scale, save_rotated=None):
+        ctx.n_inputs = 12 if save_rotated is None else 13   # backward returns one entry per argument of apply
+        ctx.dims, plan = (q.shape[-1], v.shape[-1]), _pad_plan(q, v, b_size)
+        if plan is not None:   # zero columns behind the rotated ones
+            q, k, v = _pad_last(q, plan[0]), _pad_last(k, plan[0]), _pad_last(v, plan[1])
+        ctx.shape = _shape(q, k, v, b_size, t_height, t_width, row_size, col_size, sm_scale)
+        assert row_cs_buffer.shape[1] == col_cs_buffer.shape[1], "row and column table must have one R"
+        assert idx.shape[0] == q.shape[2], "idx must have one entry per token"
+        rope = (idx, row_cs_buffer, col_cs_buffer)
+        ctx.rotated = True if save_rotated is None else bool(save_rotated)
+        if ctx.rotated:
+            o, m, q, k = _forward_rot(q, k, v, ctx.shape, rope)
+        else:
+            o, m = _forward(q, k, v, ctx.shape, rope)
+        ctx.save_for_backward(q, k, v, m, o, *rope)
+        return _cut_last(o, ctx.dims[1])
+
+    @staticmethod
+    def backward(ctx, do):
+        q, k, v, m, o, *rope = ctx.saved_tensors
+        run = _backward_rot if ctx.rotated else _backward
+        dq, dk, dv = run(q, k, v, o, m, _pad_last(do, v.shape[-1]), ctx.shape, tuple(rope))
+        return (_cut_last(dq, ctx.dims[0]), _cut_last(dk, ctx.dims[0]), _cut_last(dv, ctx.dims[1])) + (None,) * (ctx.n_inputs - 3)
 
 
-class TiledSwaImage:
+class TiledSwaImage(torch.autograd.Function):
     """``TiledSwa`` on image-layout tensors: q, k ``[B, IH, IW, heads, dk]``, v and o ``[B, IH, IW, heads, dv]``.
 
     ``apply(q, k, v, bh, bw, row_size, col_size, sm_scale)``.  A tile is a block of ``bh x bw`` pixels
@@ -109,9 +162,21 @@ class TiledSwaImage:
     conversion back, without the copies.
     """
 
+    @classmethod
+    def apply(cls, *args):
+        o = _lib.native.tiled_swa_image(*args) if cls is TiledSwaImage else NotImplemented
+        return super().apply(*args) if o is NotImplemented else o
+
     @staticmethod
-    def apply(*args):
-        return _lib.native.tiled_swa_image(*args)
+    def forward(ctx, q, k, v, bh, bw, row_size, col_size, sm_scale):
+        ctx.scalars = (bh, bw, row_size, col_size, sm_scale)
+        o, lse = _lib.native.image_forward(q, k, v, *ctx.scalars)
+        ctx.save_for_backward(q, k, v, o, lse)
+        return o
+
+    @staticmethod
+    def backward(ctx, do):
+        return _lib.native.image_backward(*ctx.saved_tensors, do, *ctx.scalars) + (None,) * 5
 
 
 def swa_image_offsets(t_height: int, t_width: int, bh: int, bw: int, stride_y: int, stride_x: int,

@@ -103,3 +103,14 @@ def test_rope_operands_on_the_host_raise_before_any_launch():
         _lib.rope_desc(idx, tab, tab, n_tokens=17)
     with pytest.raises(TypeError):
         _lib.rope_desc(idx.long(), tab, tab)
+
+
+def test_operators_are_autograd_functions():
+    """Drop-in contract: the operators are autograd.Function classes with forward and backward of their own."""
+    import torch
+    from dl_templates_amd.flash_attn import _attention
+    from dl_templates_amd.fused_rope2d import RotaryPE2D
+    from dl_templates_amd.tiled_swa import TiledSwa, TiledSwaImage, TiledSwaRope
+    for op in (TiledSwa, TiledSwaRope, TiledSwaImage, RotaryPE2D, _attention):
+        assert issubclass(op, torch.autograd.Function)
+        assert "forward" in vars(op) and "backward" in vars(op)
