@@ -233,11 +233,15 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   const int b_lo = ok1 ? W[1].ch_lo : a_hi + 1, b_hi = ok1 ? W[1].ch_hi : a_hi;
   const int w_lo = a_lo;
   const int both_lo = dlt_imax(a_lo, b_lo), both_hi = dlt_imin(a_hi, b_hi);
-  auto copy_only = [&](int ch, bool more) {
+  // a wave without rows in a chunk copies its halo row of V, then of the next chunk's K, at the barriers of consume() and round()
+  auto copy_v = [&](int ch) {
     swa2_issue(st, G, ch, vb_, srow, smem + C::REGION, wave);
     swa2_wait_copies();
     __syncthreads();
-    if (more) swa2_issue(st, G, ch + 1, kb_, srow, smem, wave);
+  };
+  auto copy_only = [&](int ch) {
+    copy_v(ch);
+    swa2_issue(st, G, ch + 1, kb_, srow, smem, wave);
     swa2_wait_copies();
     __syncthreads();
   };
@@ -251,18 +255,18 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   typedef std::integral_constant<int, 3> PmBoth;
   for (int pass = 0;;) {
     int ch = G.ch_first;
-    for (; ch < G.ch_last && ch < w_lo; ch++) copy_only(ch, true);
+    for (; ch < G.ch_last && ch < w_lo; ch++) copy_only(ch);
     for (; ch < G.ch_last && ch <= a_hi && ch < both_lo; ch++) round(ch, PmUpper{});
     for (; ch < G.ch_last && ch <= both_hi; ch++) round(ch, PmBoth{});
     for (; ch < G.ch_last && ch <= b_hi; ch++) round(ch, PmLower{});
-    for (; ch < G.ch_last; ch++) copy_only(ch, true);
+    for (; ch < G.ch_last; ch++) copy_only(ch);
     {
       const int cl = G.ch_last;
       const bool in0 = cl >= a_lo && cl <= a_hi, in1 = ok1 && cl >= b_lo && cl <= b_hi;
       if (in0 && in1) consume(cl, std::false_type{}, PmBoth{});
       else if (in0) consume(cl, std::false_type{}, PmUpper{});
       else if (in1) consume(cl, std::false_type{}, PmLower{});
-      else copy_only(cl, false);
+      else copy_v(cl);   // one barrier, as in consume(): the waves of a workgroup stay in step for the next column pass
     }
     __syncthreads();   // every wave is done with the chunk
     if (++pass >= a.plan.npass) break;

@@ -282,3 +282,22 @@ def test_two_patches_per_wave(B, H, S, th, tw, WR, WC, d):
         assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
         assert (o.float().cpu() - want).abs().max().item() <= FWD_TOL
         assert (lse.cpu() - lse_w).abs().max().item() <= LSE_TOL
+
+
+# two stacked patches per wave in column passes, grids whose last 16-column block has waves outside the grid next to waves with keys in a
+# later pass (60 = 48 + 12 columns, 9 tiles of 4 tokens, ...): all waves of a workgroup pass the same barriers
+@pytest.mark.parametrize("H,S,th,tw,WR,WC,d", [(40, 1, 17, 60, 3, 12, 128), (60, 1, 9, 52, 2, 16, 128), (40, 1, 20, 44, 9, 23, 64), (60, 1, 8, 40, 3, 13, 64),
+                                               (30, 1, 25, 72, 2, 40, 128), (80, 4, 20, 9, 2, 4, 64), (60, 5, 12, 11, 1, 5, 128)])
+def test_two_patches_per_wave_column_passes(H, S, th, tw, WR, WC, d):
+    from dl_templates_amd import _lib
+    sw, N, scale = _swa(), S * th * tw, 0.15
+    q, k, v, _ = orc.make_qkv(N + d + WC, 1, H, N, N, d, d, torch.bfloat16 if H == 40 else torch.float16)
+    one = [t[:, :2].float() for t in (q, k, v)]
+    want, lse_w = orc.tiled_swa_explicit(*one, S, th, tw, WR, WC, scale, return_lse2=True)
+    qg, kg, vg = (t.cuda() for t in (q, k, v))
+    o, lse = sw._forward(qg, kg, vg, sw._shape(qg, kg, vg, S, th, tw, WR, WC, scale), None)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
+    assert (o[:, :2].float().cpu() - want).abs().max().item() <= FWD_TOL
+    assert (lse[:, :2].cpu() - lse_w).abs().max().item() <= LSE_TOL
+    few = sw.tiled_swa_fwd(*(t[:, -2:].contiguous() for t in (qg, kg, vg)), S, th, tw, WR, WC, scale)   # the one-patch kernel
+    assert (o[:, -2:].float() - few.float()).abs().max().item() <= FWD_TOL
