@@ -96,9 +96,9 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     const char* nrow = swa2_issue_row(G, ch, vb_, srow, wave);
     char* ndst = swa2_issue_dst<C>(smem + C::REGION, wave);
     const int hrow = 4 * ch + g;
-    // a lane's keys of a chunk are columns of ONE halo row: the row test drops the lane's maximum and sends its exponents to
-    // -inf, nothing per score; the column test is the same for both patches (the own token of patch 1 lies below that of
-    // patch 0: inside the grid only where that one is)
+    // a lane's keys of a chunk are columns of ONE halo row; the column test is the same for both patches (the own token of patch 1
+    // lies below that of patch 0: inside the grid only where that one is).  The two tests are joined as lane masks (scalar pipe)
+    // and a score outside the window is replaced, whatever it is: an infinite or NaN key row reaches only the queries that see it.
     const bool row_vis[2] = {(hrow >= W[0].rlo) && (hrow <= W[0].rhi), (hrow >= W[1].rlo) && (hrow <= W[1].rhi) && W[1].cspan >= 0};
     // ---- scores of the chunk, one column group (16 keys) at a time
     float t[2][NKB][8];
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     auto mask_max = [&](const int p, const int cg, const f32x4& sv) {
       const int kb = cg >> 1, h4 = 4 * (cg & 1);
 #pragma unroll
-      for (int i = 0; i < 4; i++) t[p][kb][h4 + i] = (unsigned)(4 * cg + i - W[0].clo) <= (unsigned)W[0].cspan ? sv[i] : -INFINITY;
+      for (int i = 0; i < 4; i++) t[p][kb][h4 + i] = (row_vis[p] & ((unsigned)(4 * cg + i - W[0].clo) <= (unsigned)W[0].cspan)) ? sv[i] : -INFINITY;
       mx[p][cg & 3] = fmaxf(fmaxf(mx[p][cg & 3], t[p][kb][h4]), t[p][kb][h4 + 1]);
       mx[p][(cg + 2) & 3] = fmaxf(fmaxf(mx[p][(cg + 2) & 3], t[p][kb][h4 + 2]), t[p][kb][h4 + 3]);
     };
@@ -145,8 +145,8 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     if constexpr (P1) mask_max(1, NCG - 1, sc[1][(NCG - 1) & 1]);
     // reference maxima move only when some score exceeds them by more than 2^8 after scaling (see swa2_fwd_kernel)
     float mloc[2] = {-INFINITY, -INFINITY};
-    if constexpr (P0) mloc[0] = wave_max4(row_vis[0] ? fmaxf(fmaxf(mx[0][0], mx[0][1]), fmaxf(mx[0][2], mx[0][3])) : -INFINITY);
-    if constexpr (P1) mloc[1] = wave_max4(row_vis[1] ? fmaxf(fmaxf(mx[1][0], mx[1][1]), fmaxf(mx[1][2], mx[1][3])) : -INFINITY);
+    if constexpr (P0) mloc[0] = wave_max4(fmaxf(fmaxf(mx[0][0], mx[0][1]), fmaxf(mx[0][2], mx[0][3])));
+    if constexpr (P1) mloc[1] = wave_max4(fmaxf(fmaxf(mx[1][0], mx[1][1]), fmaxf(mx[1][2], mx[1][3])));
     swa2_for<0, 2>([&](auto pc_) {
       constexpr int p = decltype(pc_)::value;
       if constexpr ((PM >> p) & 1) {
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     });
     float neg_m2[2];
 #pragma unroll
-    for (int p = 0; p < 2; p++) neg_m2[p] = row_vis[p] ? (m_run[p] == -INFINITY ? 0.f : -m_run[p] * scale) : -INFINITY;
+    for (int p = 0; p < 2; p++) neg_m2[p] = m_run[p] == -INFINITY ? 0.f : -m_run[p] * scale;
     // ---- O^T += V^T P^T, 32 keys at a time: with two patches every V^T fragment feeds two products
     u32x4 va[4];
     u32x4 pb[2][2];

@@ -142,11 +142,11 @@ __global__ __launch_bounds__(512, (SwagF<D, NCH, NCG>::OCC)) void swag_fwd_f32_k
       float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
       for (int i = 0; i < NCH; i++) {
-        const float bias = F.row_bias(i, rp);
+        const bool row = F.sees_row(i, rp);
 #pragma unroll
         for (int j = 0; j < NCG; j++) {
           swat_lds blk = rowp[i] + 4 * j * C::ROWB;
-          f32x4 t = {bias, bias, bias, bias};
+          f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int c = 0; c < C::KC; c++) {
             const u32x4 kh = swat_read16(blk + L.row[c]), kl = swat_read16(blk + C::TB + L.row[c]);
@@ -156,11 +156,12 @@ __global__ __launch_bounds__(512, (SwagF<D, NCH, NCG>::OCC)) void swag_fwd_f32_k
           }
 #pragma unroll
           for (int e = 0; e < 4; e++) {
-            t[e] = F.sees_col(4 * j + e) ? t[e] : -INFINITY;
+            t[e] = (row & F.sees_col(4 * j + e)) ? t[e] : -INFINITY;
             mx[e] = fmaxf(mx[e], t[e]);
           }
           s[i * NCG + j] = t;
         }
+        __builtin_amdgcn_sched_barrier(0);   // the scores of one row of blocks at a time: read further ahead, the operands spill
       }
       const float m = wave_max4(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
       const float m_use = m == -INFINITY ? 0.f : m;

@@ -12,8 +12,10 @@
 // registers while the current one computes.  The whole window is resident: the softmax is one-shot.
 //
 // In the C layout of a block lane group g holds key row g and element i key column i, lane n is own token (n >> 2, n & 3): the
-// row test enters as the C operand of the score products (0 or -inf), the column tests are lane masks that stay in scalar
-// registers for the whole march.
+// column tests are lane masks that stay in scalar registers for the whole march.  The row test of the forward kernels is a lane
+// mask too, joined to the column's on the scalar pipe: a score outside the window is replaced, whatever it is (an infinite or NaN
+// key row must not reach the queries that do not see it; as an addend of -inf it did).  In the backward kernels it enters as the
+// C operand of the score products (0 or -inf).
 //
 // LDS: token rows of 2 D bytes, 16-byte piece p of the token at halo row r, column c at p ^ swz(r, c), where the swizzle only
 // takes c & 3 and r & 1: operand reads and transposing reads are free of bank conflicts and their lane offsets are the same
@@ -328,19 +330,21 @@ struct SwagFrame {
     if (col >= TC) chi = -1;
   }
   DLT_DEV bool sees_col(int j) const { return j >= clo && j <= chi; }
-  // C operand of the score products of key rows 4 i + g: 0 where the row is in the own token's window, else -inf
-  DLT_DEV float row_bias(int i, int rp) const {
+  // key rows 4 i + g are in the own token's window
+  DLT_DEV bool sees_row(int i, int rp) const {
     const int hr = 4 * i + g, qr = n >> 2;
     const int lo = dlt_imax(qr, WR - rp), hi = dlt_imin(qr + 2 * WR, TR - 1 - rp + WR);
-    return hr >= lo && hr <= hi ? 0.f : -INFINITY;
+    return hr >= lo && hr <= hi;
   }
+  // the same as the C operand of the score products: 0 or -inf
+  DLT_DEV float row_bias(int i, int rp) const { return sees_row(i, rp) ? 0.f : -INFINITY; }
   DLT_DEV int own_row(int rp) const { return rp + (n >> 2); }
   DLT_DEV bool own_ok(int rp) const { return own_row(rp) < TR && col < TC; }
   // clamped token index of the own token
   DLT_DEV int own_tok(int rp) const { return dlt_imin(own_row(rp), TR - 1) * TC + dlt_imin(col, TC - 1); }
 };
 
-// scores of block (i, j): row tests through the C operand, column tests on the result
+// scores of block (i, j) on top of `bias`
 template <typename C, typename CT>
 DLT_DEV f32x4 swag_scores(swat_lds blk, const SwagLane<C>& L, const u32x4 (&own)[C::KC], float bias) {
   f32x4 s = {bias, bias, bias, bias};
@@ -447,12 +451,12 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ke
       float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
       for (int i = 0; i < NCH; i++) {
-        const float bias = F.row_bias(i, rp);
+        const bool row = F.sees_row(i, rp);
 #pragma unroll
         for (int j = 0; j < NCG; j++) {
-          f32x4 t = swag_scores<C, CT>(rowp[i] + 4 * j * C::ROWB, L, q, bias);
+          f32x4 t = swag_scores<C, CT>(rowp[i] + 4 * j * C::ROWB, L, q, 0.f);
 #pragma unroll
-          for (int e = 0; e < 4; e++) t[e] = F.sees_col(4 * j + e) ? t[e] : -INFINITY;
+          for (int e = 0; e < 4; e++) t[e] = (row & F.sees_col(4 * j + e)) ? t[e] : -INFINITY;
           s[i * NCG + j] = t;
         }
       }

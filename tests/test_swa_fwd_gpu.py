@@ -301,3 +301,41 @@ def test_two_patches_per_wave_column_passes(H, S, th, tw, WR, WC, d):
     assert (lse[:, :2].cpu() - lse_w).abs().max().item() <= LSE_TOL
     few = sw.tiled_swa_fwd(*(t[:, -2:].contiguous() for t in (qg, kg, vg)), S, th, tw, WR, WC, scale)   # the one-patch kernel
     assert (o[:, -2:].float() - few.float()).abs().max().item() <= FWD_TOL
+
+
+# a key row with an infinity or NaN in it: the queries whose window does not hold it (up to three rows and columns away they share its
+# 4 x 4 blocks) get what they get without it.  Marching kernels at both head dims, with the rotation, on fp32 tensors; streaming kernels
+# with one and (more workgroups than CUs) two patches per wave, in column passes, on tiles of 4 tokens
+@pytest.mark.parametrize("bad", ["inf", "-inf", "nan row"])
+@pytest.mark.parametrize("H,S,th,tw,WR,WC,d,dtype,rope,family", [
+    (2, 1, 13, 21, 2, 2, 64, torch.bfloat16, False, "marching"), (2, 1, 30, 22, 6, 5, 64, torch.float16, False, "marching"),
+    (2, 1, 13, 21, 1, 3, 32, torch.bfloat16, False, "marching"), (2, 1, 41, 40, 9, 10, 32, torch.bfloat16, False, "marching"),
+    (2, 1, 13, 21, 2, 3, 32, torch.float32, False, "marching"), (2, 1, 30, 22, 6, 6, 32, torch.float32, False, "marching"),
+    (2, 1, 13, 21, 3, 2, 64, torch.bfloat16, True, "marching"), (2, 1, 25, 20, 7, 3, 64, torch.bfloat16, False, "streaming"),
+    (50, 1, 25, 20, 7, 3, 64, torch.bfloat16, False, "streaming"), (2, 1, 25, 20, 2, 3, 128, torch.float16, False, "streaming"),
+    (50, 1, 25, 20, 2, 3, 128, torch.float16, False, "streaming"), (50, 1, 26, 40, 9, 10, 128, torch.bfloat16, False, "streaming"),
+    (40, 1, 17, 60, 3, 12, 128, torch.bfloat16, False, "streaming"), (80, 4, 20, 9, 1, 1, 64, torch.bfloat16, False, "streaming")])
+def test_infinite_and_nan_keys_stay_inside_their_window(H, S, th, tw, WR, WC, d, dtype, rope, family, bad):
+    sw = _swa()
+    from dl_templates_amd import _lib
+    N, r0, c0 = th * tw * S, th // 2, tw // 2
+    q, k, v, _ = (t.cuda() for t in orc.make_qkv(N + WR, 1, H, N, N, d, d, dtype))
+    at = (r0 * tw + c0) * S + S // 2
+    poisoned = k.clone()
+    if bad == "nan row":
+        poisoned[0, :, at] = float("nan")
+    else:
+        poisoned[0, :, at, d - 3] = float(bad)
+    if rope:
+        tabs = (orc.make_rope_idx(1, th, tw, 0.1).cuda(), orc.rope_tables(8, th).cuda(), orc.rope_tables(8, tw).cuda())
+        run = lambda kk: sw.TiledSwaRope.apply(q, kk, v, *tabs, S, th, tw, WR, WC, 0.15)
+    else:
+        run = lambda kk: sw.tiled_swa_fwd(q, kk, v, S, th, tw, WR, WC, 0.15)
+    want = run(k)
+    got = run(poisoned)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == family
+    rows, cols = torch.arange(N, device="cuda") // S // tw, torch.arange(N, device="cuda") // S % tw
+    blind = ((rows - r0).abs() > WR) | ((cols - c0).abs() > WC)
+    assert blind.any() and not blind.all()
+    # the reference maximum of a lane may move with its neighbours': same values up to the rounding of the probabilities
+    assert (got[:, :, blind] - want[:, :, blind]).abs().max().item() <= FWD_TOL
