@@ -1,6 +1,7 @@
 // Marching forward kernel for fp32 token grids (b_size == 1, head dim 32, no rotation): the frame of swag_kernel.hpp with
 // the arithmetic of the generic kernels (q and k as hi + lo bf16 pairs, three products per score; v and the probabilities
-// rounded to bf16 once).
+// rounded to bf16 once).  o is normalised by the sum of the rounded probabilities its product uses; lse2, from which the
+// backward kernels rebuild unrounded ones, comes from the sum of the probabilities as they are.
 //
 // These calls ran on the generic kernels, whose workgroups own 64 consecutive tokens of ONE grid row: on a 16 x 16 map three
 // quarters of a workgroup had no token, and every row staged its whole halo for itself.  Back-to-back calls, before -> after:
@@ -167,6 +168,7 @@ __global__ __launch_bounds__(512, (SwagF<D, NCH, NCG>::OCC)) void swag_fwd_f32_k
       const float m_use = m == -INFINITY ? 0.f : m;
       const float neg_m2 = -m_use * scale;
       f32x4 acc[C::DB], acc_l = {0.f, 0.f, 0.f, 0.f};
+      float psum = 0.f;   // of the probabilities as they are, for lse2
 #pragma unroll
       for (int d = 0; d < C::DB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -178,6 +180,8 @@ __global__ __launch_bounds__(512, (SwagF<D, NCH, NCG>::OCC)) void swag_fwd_f32_k
           p[e] = fast_exp2(fmaf(s[b0][e], scale, neg_m2));
           p[4 + e] = 2 * t + 1 < C::NB ? fast_exp2(fmaf(s[b1][e], scale, neg_m2)) : 0.f;
         }
+#pragma unroll
+        for (int e = 0; e < 8; e++) psum += p[e];
         const u32x4 pb = pack8<CT>(p);
         swat_lds v0 = rowp[b0 / NCG] + 2 * C::TB + 4 * (b0 % NCG) * C::ROWB, v1 = rowp[b1 / NCG] + 2 * C::TB + 4 * (b1 % NCG) * C::ROWB;
 #pragma unroll
@@ -187,13 +191,13 @@ __global__ __launch_bounds__(512, (SwagF<D, NCH, NCG>::OCC)) void swag_fwd_f32_k
         }
         acc_l = Mma<CT>::mfma(ones, pb, acc_l);
       }
-      const float l = acc_l[0];
+      const float l = acc_l[0], lsum = wave_sum4(psum);
       if (F.own_ok(rp)) {
         const int tok = F.own_tok(rp);
         const float inv = fast_rcp(l);
 #pragma unroll
         for (int d = 0; d < C::DB; d++) __builtin_nontemporal_store(acc[d] * inv, reinterpret_cast<f32x4*>(ob + tok * a.os[2] + 16 * d));
-        if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
+        if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(lsum));
       }
     }
     if (more) {

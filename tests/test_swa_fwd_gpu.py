@@ -339,3 +339,20 @@ def test_infinite_and_nan_keys_stay_inside_their_window(H, S, th, tw, WR, WC, d,
     assert blind.any() and not blind.all()
     # the reference maximum of a lane may move with its neighbours': same values up to the rounding of the probabilities
     assert (got[:, :, blind] - want[:, :, blind]).abs().max().item() <= FWD_TOL
+
+
+# fp32 tensors at head dim 32: lse2 is the log of the unrounded probabilities' sum.  What is left are the scores' errors: q and k as
+# hi + lo bf16 pairs drop lo * lo and round lo (2^-18 of |q_i k_i| each, three terms), fp32 sums and exp2 / log2 add a few 2^-23.
+# (A sum of bf16-rounded probabilities is off by up to 2.8e-3 = 2^-9 log2(e).)
+@pytest.mark.parametrize("th,tw,WR,WC", [(8, 16, 0, 1), (9, 17, 1, 1), (16, 16, 3, 3), (31, 15, 6, 2), (25, 20, 5, 6)])
+def test_fp32_lse_keeps_its_bits(th, tw, WR, WC):
+    sw, N, d = _swa(), th * tw, 32
+    from dl_templates_amd import _lib
+    scale = 1 / math.sqrt(d)
+    q, k, v, _ = orc.make_qkv(N + WC, 2, 3, N, N, d, d, torch.float32)
+    _, want = orc.tiled_swa_explicit(q.double(), k.double(), v.double(), 1, th, tw, WR, WC, scale, return_lse2=True)
+    _, lse = sw._forward(q.cuda(), k.cuda(), v.cuda(), sw._shape(q, k, v, 1, th, tw, WR, WC, scale), None)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "marching"
+    products = (q.double().abs() @ k.double().abs().transpose(2, 3)).amax(-1)
+    bound = 4 * 2.0 ** -18 * products * scale / math.log(2) + 1e-6 * (1 + want.abs())
+    assert ((lse.cpu() - want).abs() <= bound).all(), ((lse.cpu() - want).abs() - bound).max()
