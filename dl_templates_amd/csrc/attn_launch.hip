@@ -435,19 +435,12 @@ int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   const int nch = swag_class(p.g.WR), ncg = swag_class(p.g.WC);
   constexpr int pc = SWAG_PC, step = 4 * (8 / pc);
   a.nstrips = (p.g.TC + 4 * pc - 1) / (4 * pc);
-  // Rows per workgroup: a band costs its steps plus a prologue that fills the ring (about two steps); workgroups beyond what the
-  // chip holds at once (one or two per CU) wait for a whole band.
+  // Rows per workgroup: a band's prologue fills the ring; one or two workgroups per CU are on the chip at once.
   const int nres = nch + 8 / pc - 1, tok = 4 * (4 * pc + 4 * (ncg - 1)), lds = nres * tok * (p.dtype == DLT_FP32 ? 6 * p.dk : 4 * p.dk + 8);
   const int64_t slots = (int64_t)dlt_device_cus() * (lds <= 80 * 1024 ? 2 : 1);
   const int64_t cols = (int64_t)p.B * p.H * a.nstrips;
-  const int steps = (p.g.TR + step - 1) / step;
-  int64_t best = -1;
-  for (int nb = 1; nb <= steps; nb++) {
-    const int per = (steps + nb - 1) / nb;
-    if ((steps + per - 1) / per != nb) continue;
-    const int64_t cost = (cols * nb + slots - 1) / slots * (per + 2);
-    if (best < 0 || cost < best) { best = cost; a.band = per * step; a.nbands = nb; }
-  }
+  dlt_band_plan((p.g.TR + step - 1) / step, cols, slots, a.band, a.nbands);
+  a.band *= step;
   const int64_t grid = cols * a.nbands;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
   if (p.dtype == DLT_FP32) return dlt_swag_launch_f32(a, nch, ncg, (int)grid, stream);
@@ -522,19 +515,11 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   a.sm_scale = p.sm_scale;
   a.nstrips = (p.g.XLq + 127) / 128;
-  // Rows per workgroup.  A band costs its rows plus the prologue that fills the ring (the latency of its loads, about two
-  // steps) and re-reads 2 WR rows; workgroups beyond what the chip holds at once (one or two per CU) wait for a whole band.
+  // Rows per workgroup: a band's prologue fills the ring (the latency of its loads) and re-reads 2 WR rows.
   const int halo = 8 + 2 * p.g.WC * (p.g.S / 16), ring = (2 * p.g.WR + 1) * halo * 64 * p.dk;
   const int64_t slots = (int64_t)dlt_device_cus() * (ring + (2 * p.g.WR + 1) * halo * 128 <= 80 * 1024 ? 2 : 1);
   const int64_t cols = (int64_t)p.B * p.H * a.nstrips;
-  int64_t best = -1;
-  a.band = p.g.TR; a.nbands = 1;
-  for (int nb = 1; nb <= p.g.TR; nb++) {
-    const int band = (p.g.TR + nb - 1) / nb;
-    if ((p.g.TR + band - 1) / band != nb) continue;
-    const int64_t cost = (cols * nb + slots - 1) / slots * (band + 2);
-    if (best < 0 || cost < best) { best = cost; a.band = band; a.nbands = nb; }
-  }
+  dlt_band_plan(p.g.TR, cols, slots, a.band, a.nbands);
   const int64_t grid = cols * a.nbands;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
   return p.dk == 32 ? dlt_swat_launch_32(a, p.dtype, bwd, (int)grid, stream) : dlt_swat_launch_64(a, p.dtype, bwd, (int)grid, stream);

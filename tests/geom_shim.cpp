@@ -23,6 +23,7 @@ void shim_slot_pixel(unsigned bh, unsigned bw, unsigned TC, unsigned xs, unsigne
   const DltTokMap tm = dlt_tokmap_image(bh, bw, TC);
   dlt_slot_pixel(tm, xs, *i, *x);
 }
+int shim_band_plan(int units, long long cols, long long slots, int* per, int* nb) { return dlt_band_plan(units, cols, slots, *per, *nb); }
 int shim_rope_row(int idx) { return dlt_rope_row(idx); }
 int shim_rope_col(int idx) { return dlt_rope_col(idx); }
 }

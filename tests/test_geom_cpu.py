@@ -1,7 +1,7 @@
 """CPU checks of the geometry header the host code, the debug exports and every kernel share
 (dl_templates_amd/csrc/dlt_geom.h): window ranges against the oracle's neighbour masks
 (src/tiled_swa.py:701-713), the idx decode (src/fused_rope2d.py:40-45), the token -> pixel map of the
-image layout (src/tiled_swa.py:753-755) and the exact multiply-shift division it uses.  The header is
+image layout (src/tiled_swa.py:753-755), the exact multiply-shift division it uses, and the split of a grid into bands.  The header is
 compiled with the host compiler through tests/geom_shim.cpp; no GPU is involved."""
 import ctypes
 import os
@@ -88,3 +88,29 @@ def test_idx_decode_matches_the_oracle(shim):
     rows, cols = orc.decode_idx(np.array(vals, dtype=np.int32))
     for v, r, c in zip(vals, rows, cols):
         assert shim.shim_rope_row(v) == r and shim.shim_rope_col(v) == c
+
+
+def test_band_plan_is_the_best_split_and_cheap_to_find(shim):
+    """Same split as a search over every band count, in at most 2 sqrt(n) + 2 steps, and few where the grid is long and thin: the plan
+    is made in front of every launch."""
+    def search(units, cols, slots):
+        best = None
+        for nb in range(1, units + 1):
+            per = -(-units // nb)
+            if -(-units // per) == nb:
+                cost = -(-cols * nb // slots) * (per + 2)
+                if best is None or cost < best[0]:
+                    best = (cost, per, nb)
+        return best[1:]
+
+    per, nb = ctypes.c_int(), ctypes.c_int()
+    plan = lambda units, cols, slots: shim.shim_band_plan(units, ctypes.c_longlong(cols), ctypes.c_longlong(slots), ctypes.byref(per), ctypes.byref(nb))
+    rng = random.Random(2)
+    for _ in range(3000):
+        units, cols, slots = rng.choice([rng.randint(1, 40), rng.randint(1, 2000)]), int(2 ** rng.uniform(0, 12)), rng.choice([1, 7, 256, 512])
+        tried = plan(units, cols, slots)
+        assert (per.value, nb.value) == search(units, cols, slots), (units, cols, slots)
+        assert tried <= 2 * units ** 0.5 + 2
+    for units in (65536, 262144, 2 ** 28):
+        for cols in (1, 8, 64, 4096):
+            assert plan(units, cols, 512) <= 1100, (units, cols)
