@@ -534,12 +534,20 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
 // tokens one after the other, however few the workgroups; the split ones take
 //     fixed + rounds over the CUs * (start and final sum of a workgroup + its 32-token blocks * time of a block on a CU).
 // The constants (us) are least-squares fits to launches of 32 ... 8192 tokens on either side and 4 ... 128 heads, dense and
-// causal; on those the rule picks the fastest kernel but for 0.4 % of the total time.
+// causal; on those flash_fastest over all kinds picks the fastest kernel but for 2 % of the total time.
 //   77 queries x 1500 keys, 16 heads, 64/64: forward 22 -> 10 us, dQ 24 -> 11; 482 keys x 5450 queries, 4 heads: dK/dV 86 -> 26
 //   16 heads, 2048 x 2048: forward 64/128 46 -> 34 us, 128/128 55 -> 41 (SLIM)
+//
+// A slab's results do not depend on how many slabs its call holds: the order of summation is chosen for the shape of a slab, as
+// if the call held FLASH_SLABS of them, and only among kernels that give the same bits by the slabs it really holds.  Measured
+// over 1364 shapes of 4 ... 128 slabs against a free choice (time of a pass, geometric mean): 16 slabs + 2 %, 32 the same, 64 + 3 %,
+// 128 + 10 %, 8 + 9 %, 4 + 16 % (1024 queries x 4096 keys, 4 heads, 64/128: dK/dV 35 -> 91 us, the chunked kernel).  FLASH_SLABS = 16 or
+// 24 costs less with few slabs, but 128 slabs then pay 27 or 15 %: at 32 the fewest passes are slower than on chunked kernels alone.
 enum { FLASH_CHUNKED = 0, FLASH_SPLIT1 = 1, FLASH_SPLIT2 = 2, FLASH_SLIM = 3 };
+constexpr int FLASH_SLABS = 32;
+constexpr unsigned FLASH_ALL = 15u;   // bit per kind
 struct FlashCost { int own; float start, chunk, slim_start, slim_chunk, fixed1, wg1, block1, fixed2, wg2, block2; };   // own: tokens of a chunked workgroup
-int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
+int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal, unsigned kinds) {
   constexpr float NONE = 1e9f;
   static const FlashCost COST[3][4] = {   // by pass (forward, dQ, dK/dV) and DimClass::id
       {{128, 3.50f, .822f, 2.60f, .730f, 2.31f, 1.36f, .137f, 1.09f, 3.79f, .141f},    // 64/64
@@ -557,32 +565,48 @@ int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int 
   const FlashCost& c = COST[pass][dc.id];
   const float cus = (float)dlt_device_cus();
   const auto wgs = [&](int n) { return (float)(bh * ((own + n - 1) / n)); };
-  // From 1536 tokens on a causal slab keeps to the kernels whose tests hold single slabs and whole calls to the same bits.
-  const bool free_order = !(causal && own >= 1536);
+  const auto may = [&](int kind) { return (kinds >> kind & 1u) != 0; };
   const float chunks = (float)((other + 63) / 64);
   const bool spills = pass == 2 && causal && dc.id == 2;   // two own blocks per wave: dK/dV at 64/128 under a mask
-  int best = FLASH_CHUNKED;
-  float least = c.start + c.chunk * chunks;
+  int best = -1;
+  float least = 0.f;
+  const auto consider = [&](int kind, float t) {
+    if (may(kind) && (best < 0 || t < least)) { least = t; best = kind; }
+  };
+  consider(FLASH_CHUNKED, c.start + c.chunk * chunks);
   if (wgs(128) > cus) {
     // A CU has more than one slim workgroup.  Up to two of them run side by side, which still beats the chunked workgroups
     // at 64/64 and where a mask makes the work uneven (32 heads, 2048 x 2048, causal: 64/128 52 -> 46 us, 128/128 60 -> 49)
-    if ((pass == 0 && c.slim_chunk < NONE && (causal || dc.id == 0)) || spills) return wgs(128) <= 2.f * cus ? FLASH_SLIM : FLASH_CHUNKED;
-    if (wgs(c.own) > cus) return FLASH_CHUNKED;
+    if ((pass == 0 && c.slim_chunk < NONE && (causal || dc.id == 0)) || spills) {
+      const int kind = wgs(128) <= 2.f * cus ? FLASH_SLIM : FLASH_CHUNKED;
+      if (may(kind)) return kind;
+    }
+    if (wgs(c.own) > cus && may(FLASH_CHUNKED)) return FLASH_CHUNKED;
   } else {
-    const float t = spills ? c.start + 0.65f * c.chunk * chunks : c.slim_start + c.slim_chunk * chunks;
-    if (t < least) { least = t; best = FLASH_SLIM; }
+    consider(FLASH_SLIM, spills ? c.start + 0.65f * c.chunk * chunks : c.slim_start + c.slim_chunk * chunks);
   }
   // the pieces of a row that a head dim below its class does not have are not read
   const float blocks = (float)((other + 31) / 32) * ((float)dims / (float)(dc.DK + dc.DV));
-  for (int np = 1; free_order && np <= 2; np++) {
+  for (int np = 1; np <= 2; np++) {
     float rounds = wgs(16 * np) / cus;
     if (dc.DK + dc.DV > 128) rounds = 0.5f * (rounds + ceilf(rounds));   // one workgroup per CU: a started round is half a round
     // under a causal mask the workgroups of several rounds see about half of the other side
     const float seen = causal && rounds > 1.f ? 0.55f * blocks : blocks;
-    const float t = (np == 1 ? c.fixed1 : c.fixed2) + (rounds > 1.f ? rounds : 1.f) * (np == 1 ? c.wg1 + c.block1 * seen : c.wg2 + c.block2 * seen);
-    if (t < least) { least = t; best = np; }
+    consider(np == 1 ? FLASH_SPLIT1 : FLASH_SPLIT2,
+             (np == 1 ? c.fixed1 : c.fixed2) + (rounds > 1.f ? rounds : 1.f) * (np == 1 ? c.wg1 + c.block1 * seen : c.wg2 + c.block2 * seen));
   }
-  return best;
+  return best < 0 ? FLASH_SLIM : best;   // SLIM alone, beyond one workgroup per CU
+}
+// Kinds that give a slab the same bits as `kind`: one and two own blocks per split workgroup; slim and chunked workgroups where both
+// pass 64 tokens at a time (the chunked forward kernels at 64/128 and 128/128 pass 128: other reference maxima of the softmax).
+unsigned flash_same_bits(int pass, const DimClass& dc, int kind) {
+  if (kind == FLASH_SPLIT1 || kind == FLASH_SPLIT2) return 1u << FLASH_SPLIT1 | 1u << FLASH_SPLIT2;
+  if (pass == 0 && (dc.id == 1 || dc.id == 2)) return 1u << kind;
+  return 1u << FLASH_CHUNKED | 1u << FLASH_SLIM;
+}
+int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
+  const int order = flash_fastest(pass, dc, dims, FLASH_SLABS, own, other, causal, FLASH_ALL);
+  return flash_fastest(pass, dc, dims, bh, own, other, causal, flash_same_bits(pass, dc, order));
 }
 
 int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {

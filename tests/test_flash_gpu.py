@@ -339,3 +339,28 @@ def test_streamed_side_split_over_waves(causal, Lq, Lk, dk, dv, B, H, dtype):
     assert max(errs) <= 5e-2, errs
     _, M = _fa()._forward(q.cuda(), k.cuda(), v.cuda(), causal, scale)
     assert (M.cpu() - orc.flash_lse2(q, k, scale, causal)).abs().max().item() <= 2e-2
+
+
+# one rule picks the order of summation from the shape of a slab: shapes on both sides of it in every head-dim class, the slab counts on both
+# sides of the choices that are left (one or two own blocks per split workgroup, slim or chunked workgroups)
+@pytest.mark.parametrize("causal,Lq,Lk,dk,dv,counts", [
+    (False, 77, 1500, 64, 64, (1, 16, 130)), (False, 40, 700, 128, 128, (1, 100)), (False, 500, 60, 64, 128, (1, 40)), (False, 33, 300, 32, 32, (1, 300)),
+    (False, 1000, 1000, 64, 64, (1, 8, 70)), (False, 600, 2500, 64, 128, (1, 12, 60)), (False, 700, 700, 80, 80, (1, 50)), (False, 1200, 300, 128, 128, (1, 30)),
+    (True, 90, 90, 64, 64, (1, 200)), (True, 255, 255, 128, 128, (1, 70)), (True, 513, 513, 64, 128, (1, 8, 70)), (True, 1030, 1030, 64, 64, (1, 9, 40)),
+    (True, 1100, 1100, 128, 128, (1, 16, 40)), (True, 300, 300, 40, 24, (1, 150)), (True, 2000, 2000, 64, 64, (1, 40)), (True, 1800, 1800, 64, 128, (1, 20, 40))])
+def test_a_slab_has_the_same_bits_in_any_call(causal, Lq, Lk, dk, dv, counts):
+    scale = 1 / math.sqrt(dk)
+    gen = torch.Generator(device="cuda").manual_seed(Lq + Lk)
+    full = [torch.randn(1, max(counts), n, d, generator=gen, device="cuda").to(torch.bfloat16) for n, d in ((Lq, dk), (Lk, dk), (Lk, dv), (Lq, dv))]
+    runs = []
+    for n in counts:
+        q, k, v = (t[:, -n:].contiguous().requires_grad_(True) for t in full[:3])
+        o = _fa().attention(q, k, v, causal, scale)
+        _, M = _fa()._forward(q.detach(), k.detach(), v.detach(), causal, scale)
+        runs.append((o.detach(), M) + torch.autograd.grad(o, (q, k, v), full[3][:, -n:].contiguous()))
+    for run in runs[1:]:
+        m = min(counts)
+        assert [torch.equal(a[:, -m:], b[:, -m:]) for a, b in zip(runs[0], run)] == [True] * 5
+    for a, b in zip(runs[-2], runs[-1]):
+        n = counts[-2]
+        assert torch.equal(a[:, -n:], b[:, -n:])
