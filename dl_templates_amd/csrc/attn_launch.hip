@@ -540,11 +540,13 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
 //
 // A slab's results do not depend on how many slabs its call holds: the order of summation is chosen for the shape of a slab, as
 // if the call held FLASH_SLABS of them, and only among kernels that give the same bits by the slabs it really holds.  Measured
-// over 1364 shapes of 4 ... 128 slabs against a free choice (time of a pass, geometric mean): 16 slabs + 2 %, 32 the same, 64 + 3 %,
-// 128 + 10 %, 8 + 9 %, 4 + 16 % (1024 queries x 4096 keys, 4 heads, 64/128: dK/dV 35 -> 91 us, the chunked kernel).  FLASH_SLABS = 16 or
-// 24 costs less with few slabs, but 128 slabs then pay 27 or 15 %: at 32 the fewest passes are slower than on chunked kernels alone.
+// over 1364 shapes of 4 ... 128 slabs against a free choice (time of a pass, geometric mean): 32 slabs - 1 %, 16 + 1 %, 64 + 2 %, 8 + 7 %,
+// 128 + 10 %, 4 + 14 % (1024 keys x 4096 queries, 4 heads, 64/128: dK/dV 35 -> 91 us, the chunked kernel).  FLASH_SLABS = 16 or 24
+// costs less with few slabs, but 128 slabs then pay 27 or 15 %: at 32 the fewest passes are slower than on chunked kernels alone.
+// Forward passes at 64/128 and 128/128 that do not split the keys: slim workgroups below 3072 queries, where they take 0.70 of the
+// chunked time while they fit the chip at once and 0.75 ... 1.2 beyond; from there on chunked ones (4096 queries, 32 slabs: 1.1 ... 1.2).
 enum { FLASH_CHUNKED = 0, FLASH_SPLIT1 = 1, FLASH_SPLIT2 = 2, FLASH_SLIM = 3 };
-constexpr int FLASH_SLABS = 32;
+constexpr int FLASH_SLABS = 32, FLASH_SLIM_BELOW = 3072;
 constexpr unsigned FLASH_ALL = 15u;   // bit per kind
 struct FlashCost { int own; float start, chunk, slim_start, slim_chunk, fixed1, wg1, block1, fixed2, wg2, block2; };   // own: tokens of a chunked workgroup
 int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal, unsigned kinds) {
@@ -605,7 +607,8 @@ unsigned flash_same_bits(int pass, const DimClass& dc, int kind) {
   return 1u << FLASH_CHUNKED | 1u << FLASH_SLIM;
 }
 int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
-  const int order = flash_fastest(pass, dc, dims, FLASH_SLABS, own, other, causal, FLASH_ALL);
+  int order = flash_fastest(pass, dc, dims, FLASH_SLABS, own, other, causal, FLASH_ALL);
+  if (pass == 0 && (dc.id == 1 || dc.id == 2) && order != FLASH_SPLIT1 && order != FLASH_SPLIT2) order = own < FLASH_SLIM_BELOW ? FLASH_SLIM : FLASH_CHUNKED;
   return flash_fastest(pass, dc, dims, bh, own, other, causal, flash_same_bits(pass, dc, order));
 }
 
