@@ -352,11 +352,11 @@ int swa2_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream)
   a.p = p;
   // Two stacked patches per wave (4 waves per workgroup, two workgroups per CU) from more than one workgroup per CU on; below, a
   // CU has one workgroup either way and 8 waves of one patch each finish it sooner (64 workgroups 12.8 against 14.2 us, 224
-  // 11.2 / 12.2, 352 26.8 / 25.8).  Its copies need K and V at the same token stride.
+  // 11.2 / 12.2, 352 26.8 / 25.8).
   // DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the one-patch kernel for A/B timing and for its tests.
   static const bool single_patch = [] { const char* e = getenv("DLT_SWA2_SINGLE_PATCH"); return e != nullptr && e[0] == '1'; }();
   swa2_make_plan(p, a.plan);
-  a.plan.pairs = !single_patch && t.ks[2] == t.vs[2] && (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c > dlt_device_cus();
+  a.plan.pairs = !single_patch && (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c > dlt_device_cus();
   a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.out_o; a.lse = t.lse;
   for (int i = 0; i < 4; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; }
   for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];

@@ -14,7 +14,7 @@ template <typename TIO, int NCG>
 int swa2_launch_fwd_t(const Swa2FwdArgs& a, int grid, hipStream_t stream) {
   typedef Swa2Cfg<DLT_SWA2_D, NCG> C;
   const bool pairs = a.plan.pairs != 0;
-  auto kern = pairs ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG> : swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG>;
+  auto kern = !pairs ? swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG> : a.ks[2] == a.vs[2] ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, true> : swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, false>;
   const int lds = pairs ? C::BUF : C::LDS;
   int rc = swa2_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;

@@ -24,7 +24,7 @@ constexpr int SWA2S_THREADS = 256;
 // waves per SIMD the register budget is sized for (head dim 64 at 6 column groups spills at 3)
 constexpr int swa2s_occ(int D, int NCG) { return D == 64 && NCG == 4 ? 3 : 2; }
 
-template <typename TIO, int D, int NCG>
+template <typename TIO, int D, int NCG, bool SAME>
 __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_kernel(const Swa2FwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef Swa2Cfg<D, NCG> C;
@@ -46,13 +46,17 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   const int64_t os2 = a.os[2], ls2 = a.ls[2];
   const float scale = a.scale_log2;
 
-  // staging: wave w copies halo row w of every chunk, of K and of V
-  const int sn2 = (int)a.ks[2] * 2;
-  const uint32_t srow = (uint32_t)(G0.TC * sn2);
+  // staging: wave w copies halo row w of every chunk, of K and of V.  SAME: one set of lane offsets serves both tensors (equal token
+  // strides); V in another layout has offsets of its own (at head dim 128 and 6 column groups 6 more registers spill outside the
+  // loops; 128 x 128, 21 x 21, 16 slabs, V as [B, N, H, D]: 105 us, 119 on the one-patch kernel that took these calls before)
+  const int ksn2 = (int)a.ks[2] * 2, vsn2 = (int)a.vs[2] * 2;
+  const uint32_t krow = (uint32_t)(G0.TC * ksn2), vrow = (uint32_t)(G0.TC * vsn2);
   Swa2Geom G = G0;   // column pass 0
-  Swa2Stage<C> st;   // K and V have the same token stride (dispatch rule)
-  swa2_stage_init(st, G, wave, lane, sn2);
-  swa2_issue(st, G, G.ch_first, kb_, srow, smem, wave);
+  Swa2Stage<C> st, st_own;
+  swa2_stage_init(st, G, wave, lane, ksn2);
+  if constexpr (!SAME) swa2_stage_init(st_own, G, wave, lane, vsn2);
+  const Swa2Stage<C>& stv = SAME ? st : st_own;
+  swa2_issue(st, G, G.ch_first, kb_, krow, smem, wave);
 
   // own queries of both patches straight into B-operand fragments
   const int c_p = G.c0 + 4 * pc;
@@ -93,7 +97,7 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     constexpr bool P0 = (PM & 1) != 0, P1 = (PM & 2) != 0;
     Swa2Lds sK = (Swa2Lds)smem;
     Swa2Lds sV = sK + C::REGION;
-    const char* nrow = swa2_issue_row(G, ch, vb_, srow, wave);
+    const char* nrow = swa2_issue_row(G, ch, vb_, vrow, wave);
     char* ndst = swa2_issue_dst<C>(smem + C::REGION, wave);
     const int hrow = 4 * ch + g;
     // a lane's keys of a chunk are columns of ONE halo row; the column test is the same for both patches (the own token of patch 1
@@ -125,8 +129,8 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
       f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
       swa2_for<0, KC>([&](auto cc) {
         constexpr int c = decltype(cc)::value;
-        if constexpr (c == 0) swa2_issue_one<C, 2 * cg>(st, nrow, ndst);
-        if constexpr (c == KC / 2) swa2_issue_one<C, 2 * cg + 1>(st, nrow, ndst);
+        if constexpr (c == 0) swa2_issue_one<C, 2 * cg>(stv, nrow, ndst);
+        if constexpr (c == KC / 2) swa2_issue_one<C, 2 * cg + 1>(stv, nrow, ndst);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (P0) s0 = Mma<CT>::mfma(ka[c], qf[0][c], s0);
         if constexpr (P1) s1 = Mma<CT>::mfma(ka[c], qf[1][c], s1);
@@ -189,7 +193,7 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     for (int e = 0; e < 8; e++) prob(0, e);
     swa2_wait_copies();
     __syncthreads();   // V of the chunk has landed, every wave is done with its K
-    nrow = swa2_issue_row(G, ch + 1, kb_, srow, wave);
+    nrow = swa2_issue_row(G, ch + 1, kb_, krow, wave);
     ndst = swa2_issue_dst<C>(smem, wave);
 #pragma unroll
     for (int d = 0; d < 4; d++) read_v(std::integral_constant<int, 0>{}, d);
@@ -235,13 +239,13 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   const int both_lo = dlt_imax(a_lo, b_lo), both_hi = dlt_imin(a_hi, b_hi);
   // a wave without rows in a chunk copies its halo row of V, then of the next chunk's K, at the barriers of consume() and round()
   auto copy_v = [&](int ch) {
-    swa2_issue(st, G, ch, vb_, srow, smem + C::REGION, wave);
+    swa2_issue(stv, G, ch, vb_, vrow, smem + C::REGION, wave);
     swa2_wait_copies();
     __syncthreads();
   };
   auto copy_only = [&](int ch) {
     copy_v(ch);
-    swa2_issue(st, G, ch + 1, kb_, srow, smem, wave);
+    swa2_issue(st, G, ch + 1, kb_, krow, smem, wave);
     swa2_wait_copies();
     __syncthreads();
   };
@@ -273,8 +277,9 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     G = swa2_pass_geom(G0, NCG, pass);
     W[0] = swa2_pass_window(W0[0], NCG, pass);
     W[1] = swa2_pass_window(W0[1], NCG, pass);
-    swa2_stage_init(st, G, wave, lane, sn2);
-    swa2_issue(st, G, G.ch_first, kb_, srow, smem, wave);
+    swa2_stage_init(st, G, wave, lane, ksn2);
+    if constexpr (!SAME) swa2_stage_init(st_own, G, wave, lane, vsn2);
+    swa2_issue(st, G, G.ch_first, kb_, krow, smem, wave);
     swa2_wait_copies();
     __syncthreads();
   }

@@ -266,7 +266,7 @@ def test_marching_fp32(th, tw, WR, WC):
 
 
 # two stacked patches per wave (streaming kernels, more workgroups than CUs): bands without a lower patch, one band and a bit, ragged
-# columns, both window classes, windows in column passes, tiles of 4 tokens, and K / V strides that keep the one-patch kernel
+# columns, both window classes, windows in column passes, tiles of 4 tokens, K and V at one token stride and apart
 @pytest.mark.parametrize("B,H,S,th,tw,WR,WC,d", [(1, 300, 1, 3, 5, 7, 7, 128), (1, 300, 1, 4, 16, 2, 3, 128), (1, 150, 1, 9, 15, 10, 10, 128), (2, 40, 1, 17, 18, 3, 8, 128),
                                                  (1, 70, 1, 13, 33, 2, 12, 128), (1, 150, 1, 8, 17, 7, 9, 64), (1, 70, 1, 16, 31, 7, 2, 64), (1, 130, 4, 9, 7, 1, 1, 64),
                                                  (1, 130, 4, 8, 5, 2, 2, 128)])
@@ -356,3 +356,14 @@ def test_fp32_lse_keeps_its_bits(th, tw, WR, WC):
     products = (q.double().abs() @ k.double().abs().transpose(2, 3)).amax(-1)
     bound = 4 * 2.0 ** -18 * products * scale / math.log(2) + 1e-6 * (1 + want.abs())
     assert ((lse.cpu() - want).abs() <= bound).all(), ((lse.cpu() - want).abs() - bound).max()
+
+
+# K and V of different layouts run on the two-patch kernel as well: the bits of the same call with equal token strides
+@pytest.mark.parametrize("B,H,S,th,tw,WR,WC,d", [(1, 150, 1, 9, 15, 10, 10, 128), (2, 40, 1, 17, 18, 3, 8, 128), (1, 70, 1, 13, 60, 2, 12, 128), (1, 150, 1, 8, 17, 7, 9, 64),
+                                                 (1, 70, 1, 16, 31, 7, 2, 64), (1, 130, 4, 8, 5, 2, 2, 128)])
+def test_two_patches_with_keys_and_values_apart(B, H, S, th, tw, WR, WC, d):
+    sw, N = _swa(), S * th * tw
+    q, k, v, _ = (t.cuda() for t in orc.make_qkv(N + d + WC, B, H, N, N, d, d, torch.bfloat16))
+    apart = v.transpose(1, 2).contiguous().transpose(1, 2)
+    (o, lse), (o2, lse2) = (sw._forward(q, k, x, sw._shape(q, k, x, S, th, tw, WR, WC, 0.15), None) for x in (v, apart))
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
