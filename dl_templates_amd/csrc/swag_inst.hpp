@@ -11,7 +11,9 @@ constexpr int PC = SWAG_PC;
 template <typename TIO, int NCG, bool ROPE>
 int swag_fwd(const SwagArgs& a, int grid, hipStream_t stream) {
   typedef Swag<DLT_D, DLT_NCH, NCG, PC> C;
-  auto kern = swag_fwd_kernel<TIO, DLT_D, DLT_NCH, NCG, PC, ROPE>;
+  void (*kern)(SwagArgs);
+  if constexpr (ROPE) kern = swag_fwd_rope_kernel<TIO, DLT_D, DLT_NCH, NCG, PC>;
+  else kern = swag_fwd_kernel<TIO, DLT_D, DLT_NCH, NCG, PC>;
   constexpr int lds = C::RING + (ROPE ? SWAG_TAB_BYTES : 0);
   static_assert(lds <= 160 * 1024, "ring and tables exceed the LDS");
   const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), lds);

@@ -12,10 +12,11 @@
 // registers while the current one computes.  The whole window is resident: the softmax is one-shot.
 //
 // In the C layout of a block lane group g holds key row g and element i key column i, lane n is own token (n >> 2, n & 3): the
-// column tests are lane masks that stay in scalar registers for the whole march.  The row test of the forward kernels is a lane
-// mask too, joined to the column's on the scalar pipe: a score outside the window is replaced, whatever it is (an infinite or NaN
-// key row must not reach the queries that do not see it; as an addend of -inf it did).  In the backward kernels it enters as the
-// C operand of the score products (0 or -inf).
+// row test enters as the C operand of the score products (0 or -inf), the column tests are lane masks that stay in scalar
+// registers for the whole march.  -inf + inf and -inf + NaN are NaN: with an infinity or NaN in a key row, queries that do not see it
+// find their row sum NaN (one test per patch of the forward pass), and the patch is formed again by swag_fwd_exact.  (Replacing
+// masked scores always costs a scalar instruction in front of every select, and a second body inside the march registers: 89 x 98,
+// d = 32, 15 x 21 window, 32 slabs 49 -> 65 and 58 us.)
 //
 // LDS: token rows of 2 D bytes, 16-byte piece p of the token at halo row r, column c at p ^ swz(r, c), where the swizzle only
 // takes c & 3 and r & 1: operand reads and transposing reads are free of bank conflicts and their lane offsets are the same
@@ -353,10 +354,243 @@ DLT_DEV f32x4 swag_scores(swat_lds blk, const SwagLane<C>& L, const u32x4 (&own)
   return s;
 }
 
-// ROPE: K is turned in registers between HBM and LDS, the own queries in theirs
-template <typename TIO, int D, int NCH, int NCG, int PC, bool ROPE>
+// The forward pass of one patch where a key row holds an infinity or a NaN: block by block (`block(i, j)`: where it lies in LDS), every
+// score outside the window replaced, the softmax online.  Rare: rolled, so that it costs the common path few registers.
+template <typename C, typename CT, int NCG, typename Frame, typename Block>
+DLT_DEV void swag_fwd_exact(const Frame& F, const SwagLane<C>& L, int rp, const u32x4 (&q)[C::KC], float scale, f32x4 (&acc)[C::DB], float& l, float& m_use,
+                            Block block) {
+  float m = -INFINITY, sum = 0.f;
+#pragma unroll
+  for (int d = 0; d < C::DB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int k = 0; k < C::NB; k++) {
+    const int i = k / NCG, j = k - i * NCG;
+    swat_lds blk = block(i, j);
+    const bool row = F.sees_row(i, rp);
+    f32x4 t = swag_scores<C, CT>(blk, L, q, 0.f);
+#pragma unroll
+    for (int e = 0; e < 4; e++) t[e] = row && F.sees_col(4 * j + e) ? t[e] : -INFINITY;
+    const float m_new = fmaxf(m, wave_max4(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]))));
+    const float alpha = m_new == m ? 1.f : fast_exp2((m - m_new) * scale), neg_m2 = m_new == -INFINITY ? 0.f : -m_new * scale;
+    m = m_new;
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      p[e] = fast_exp2(fmaf(t[e], scale, neg_m2));
+      p[4 + e] = 0.f;
+    }
+    const u32x4 pb = pack8<CT>(p);
+    const unsigned one2 = pack2<CT>(1.f, 1.f);
+    sum = dot2_acc<CT>(pb.y, one2, dot2_acc<CT>(pb.x, one2, sum * alpha));
+#pragma unroll
+    for (int d = 0; d < C::DB; d++) {
+      const u32x2 v = swat_read_tr(blk + C::TB + L.tr[d]);
+      acc[d] = Mma<CT>::mfma(u32x4{v.x, v.y, v.x, v.y}, pb, acc[d] * alpha);
+    }
+  }
+  l = wave_sum4(sum);
+  m_use = m == -INFINITY ? 0.f : m;
+}
+
+// Forward pass without rotation.
+//
+// With one workgroup per CU (head dim 32, the largest windows: two waves per SIMD) the LDS reads are placed by hand, K one row of
+// blocks ahead of its products and V one pair of blocks: left to the compiler the read-ahead depends on the scalar registers that
+// happen to be free (89 x 98, 32 slabs: 19 x 21 window 66 -> 59 us; 15 x 21 49.5 and 58 us in two builds, 51.7 here).  Where two
+// workgroups share a CU the placed reads cost registers (64 x 64, 9 x 19 window 18.4 -> 25.7 us).
+template <typename TIO, int D, int NCH, int NCG, int PC>
 __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_kernel(const SwagArgs a) {
   typedef Swag<D, NCH, NCG, PC> C;
+  typedef typename ComputeOf<TIO>::type CT;
+  constexpr bool AHEAD = D == 32 && C::OCC == 2;
+  extern __shared__ __align__(16) char smem[];
+  swat_lds lds = (swat_lds)smem;
+  const int tid = threadIdx.x;
+  SwagFrame<C, PC> F;
+  F.init(a, tid);
+  const int b = F.w.b, h = F.w.h, n = F.n, g = F.g;
+  const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
+  const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
+  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
+  SwagRing<C> ring;
+  ring.init(lds, kb_, (int)a.ks[2], vb_, (int)a.vs[2], a, F.w.c0, tid, F.wave);
+  const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1]) + 16 * g;
+  char* ob = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.out_o) + b * a.os[0] + h * a.os[1]);
+  float* lseb = a.lse + b * a.ls[0] + h * a.ls[1];
+  const int qsn = (int)a.qs[2] * 2, osn = (int)a.os[2] * 2;
+  SwagLane<C> L;
+  L.init(n, g);
+  const float scale = a.scale_log2;
+  const unsigned one2 = pack2<CT>(1.f, 1.f);
+  const u32x4 ones = {one2, one2, one2, one2};
+
+  u32x4 qn[C::KC];
+  auto load_q = [&](int rp) {
+    const int tok = F.own_tok(rp);
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) qn[c] = *reinterpret_cast<const u32x4*>(qb + (uint32_t)(tok * qsn) + 64 * c);
+  };
+  load_q(F.w.r0 + 4 * F.rg);
+  ring.fill(F.w.r0 - F.WR);
+  __syncthreads();
+
+  int slot0 = 0;   // slot of the step's first chunk
+  uint64_t any_bad = 0;
+  for (int r = F.w.r0; r < F.w.r1; r += 4 * C::PR) {
+    const int rp = r + 4 * F.rg;
+    u32x4 q[C::KC];
+#pragma unroll
+    for (int c = 0; c < C::KC; c++) q[c] = qn[c];
+    pin_loaded(q);
+    const bool more = r + 4 * C::PR < F.w.r1;
+    u32x4 nx[C::PR][C::NIT];
+    const int next = r - F.WR + 4 * C::NRES;   // first halo row of the chunks to come
+    if (more) {
+#pragma unroll
+      for (int i = 0; i < C::PR; i++) ring.issue(nx[i], next + 4 * i);
+      load_q(rp + 4 * C::PR);
+    }
+    if (rp < F.TR && F.w.c0 + 4 * F.pc < F.TC) {
+      swat_lds rowp[NCH];
+#pragma unroll
+      for (int i = 0; i < NCH; i++) {
+        const int s = slot0 + F.rg + i;
+        rowp[i] = lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + 4 * F.pc * C::ROWB;
+      }
+      f32x4 s[C::NB + 1];
+      float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      u32x4 ka[2][NCG][C::KC];
+      auto read_row = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < NCG; j++)
+#pragma unroll
+          for (int c = 0; c < C::KC; c++) ka[i & 1][j][c] = swat_read16(rowp[i] + 4 * j * C::ROWB + L.row[c]);
+      };
+      if constexpr (AHEAD) read_row(0);
+#pragma unroll
+      for (int i = 0; i < NCH; i++) {
+        const float bias = F.row_bias(i, rp);
+        if constexpr (AHEAD) {
+          if (i + 1 < NCH) read_row(i + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int j = 0; j < NCG; j++) {
+          f32x4 t = {bias, bias, bias, bias};
+          if constexpr (AHEAD) {
+#pragma unroll
+            for (int c = 0; c < C::KC; c++) t = Mma<CT>::mfma(ka[i & 1][j][c], q[c], t);
+          } else {
+            t = swag_scores<C, CT>(rowp[i] + 4 * j * C::ROWB, L, q, bias);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; e++) t[e] = F.sees_col(4 * j + e) ? t[e] : -INFINITY;
+          s[i * NCG + j] = t;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < C::NB; k += 2)
+#pragma unroll
+        for (int e = 0; e < 4; e++) mx[e] = fmaxf(fmaxf(mx[e], s[k][e]), s[k + 1 < C::NB ? k + 1 : k][e]);
+      const float m = wave_max4(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
+      const float m_use = m == -INFINITY ? 0.f : m;   // own positions outside the grid see nothing
+      const float neg_m2 = -m_use * scale;
+      f32x4 acc[C::DB], acc_l = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < C::DB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+      u32x4 va[2][C::DB];
+      auto read_v = [&](int t) {
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        swat_lds v0 = rowp[b0 / NCG] + C::TB + 4 * (b0 % NCG) * C::ROWB, v1 = rowp[b1 / NCG] + C::TB + 4 * (b1 % NCG) * C::ROWB;
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(v0 + L.tr[d]), hi = swat_read_tr(v1 + L.tr[d]);
+          va[t & 1][d] = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
+      };
+      if constexpr (AHEAD) read_v(0);
+#pragma unroll
+      for (int t = 0; t < C::NP; t++) {
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        if constexpr (AHEAD) {
+          if (t + 1 < C::NP) read_v(t + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          p[e] = fast_exp2(fmaf(s[b0][e], scale, neg_m2));
+          p[4 + e] = 2 * t + 1 < C::NB ? fast_exp2(fmaf(s[b1][e], scale, neg_m2)) : 0.f;
+        }
+        const u32x4 pb = pack8<CT>(p);
+        if constexpr (AHEAD) {
+#pragma unroll
+          for (int d = 0; d < C::DB; d++) acc[d] = Mma<CT>::mfma(va[t & 1][d], pb, acc[d]);
+        } else {
+          swat_lds v0 = rowp[b0 / NCG] + C::TB + 4 * (b0 % NCG) * C::ROWB, v1 = rowp[b1 / NCG] + C::TB + 4 * (b1 % NCG) * C::ROWB;
+#pragma unroll
+          for (int d = 0; d < C::DB; d++) {
+            const u32x2 lo = swat_read_tr(v0 + L.tr[d]), hi = swat_read_tr(v1 + L.tr[d]);
+            acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc[d]);
+          }
+        }
+        acc_l = Mma<CT>::mfma(ones, pb, acc_l);
+      }
+      const float l = acc_l[0];
+      any_bad |= __builtin_amdgcn_ballot_w64(l != l);
+      if (F.own_ok(rp)) {
+        const int tok = F.own_tok(rp);
+        swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+        if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
+      }
+    }
+    if (more) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < C::PR; i++) ring.commit(nx[i], slot0 + i >= C::NRES ? slot0 + i - C::NRES : slot0 + i);
+      __syncthreads();
+      slot0 = slot0 + C::PR >= C::NRES ? slot0 + C::PR - C::NRES : slot0 + C::PR;
+    }
+  }
+  // Patches of a wave that met such a key are formed again behind the march, from memory: every block of the window passes through
+  // the wave's own 4 x 4 tokens of the ring.
+  __syncthreads();
+  if (any_bad) {
+    keep_branch();
+    constexpr int PER = D / 32;   // 16-byte pieces of a tensor's block per lane
+    int lane = F.lane;
+    asm volatile("" : "+v"(lane));   // keeps the addresses below out of the march
+    swat_lds own = lds + F.rg * C::SLOT + 4 * F.pc * C::ROWB;
+    for (int rp = F.w.r0 + 4 * F.rg; rp < dlt_imin(F.w.r1, F.TR); rp += 4 * C::PR) {
+      load_q(rp);
+      f32x4 acc[C::DB];
+      float l, m_use;
+      swag_fwd_exact<C, CT, NCG>(F, L, rp, qn, scale, acc, l, m_use, [&](int i, int j) {
+#pragma unroll
+        for (int x = 0; x < PER; x++) {
+          const int id = lane + 64 * x, t = id / C::PIECES, piece = id % C::PIECES, lr = t >> 2, lc = t & 3;
+          const int row = dlt_imax(0, dlt_imin(rp - F.WR + 4 * i + lr, F.TR - 1));
+          const int tok = row * F.TC + dlt_imax(0, dlt_imin(F.w.c0 + 4 * (F.pc + j) - F.WC + lc, F.TC - 1));
+          swat_lds p = own + (lr * C::HCW + lc) * C::ROWB + 16 * (piece ^ swag_swz<D>(lr, lc));
+          swat_write16(p, *reinterpret_cast<const u32x4*>(kb_ + (uint32_t)(tok * ksn) + 16 * piece));
+          swat_write16(p + C::TB, *reinterpret_cast<const u32x4*>(vb_ + (uint32_t)(tok * vsn) + 16 * piece));
+        }
+        return own;
+      });
+      if (F.own_ok(rp)) {
+        const int tok = F.own_tok(rp);
+        swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+        if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
+      }
+    }
+  }
+}
+
+// Forward pass with rotation: K is turned in registers between HBM and LDS, the own queries in theirs
+template <typename TIO, int D, int NCH, int NCG, int PC>
+__global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_rope_kernel(const SwagArgs a) {
+  typedef Swag<D, NCH, NCG, PC> C;
+  constexpr bool ROPE = true;
   typedef typename ComputeOf<TIO>::type CT;
   extern __shared__ __align__(16) char smem[];
   swat_lds lds = (swat_lds)smem;
