@@ -437,10 +437,14 @@ int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   a.nstrips = (p.g.TC + 4 * pc - 1) / (4 * pc);
   // Rows per workgroup: a band's prologue fills the ring; one or two workgroups per CU are on the chip at once.
   const int nres = nch + 8 / pc - 1, tok = 4 * (4 * pc + 4 * (ncg - 1)), lds = nres * tok * (p.dtype == DLT_FP32 ? 6 * p.dk : 4 * p.dk + 8);
-  const int64_t slots = (int64_t)dlt_device_cus() * (lds <= 80 * 1024 ? 2 : 1);
+  const bool two = lds <= 80 * 1024 && (bwd || !a.rope.enabled);   // the rotating forward kernel's registers leave room for one
+  const int64_t slots = (int64_t)dlt_device_cus() * (two ? 2 : 1);
   const int64_t cols = (int64_t)p.B * p.H * a.nstrips;
   dlt_band_plan((p.g.TR + step - 1) / step, cols, slots, a.band, a.nbands);
   a.band *= step;
+  dlt_fastdiv_make((uint32_t)a.nstrips, a.m_s, a.s_s);
+  dlt_fastdiv_make((uint32_t)a.nbands, a.m_b, a.s_b);
+  dlt_fastdiv_make((uint32_t)p.H, a.m_h, a.s_h);
   const int64_t grid = cols * a.nbands;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
   if (p.dtype == DLT_FP32) return dlt_swag_launch_f32(a, nch, ncg, (int)grid, stream);

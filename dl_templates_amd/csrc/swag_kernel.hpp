@@ -15,7 +15,7 @@
 // row test enters as the C operand of the score products (0 or -inf), the column tests are lane masks that stay in scalar
 // registers for the whole march.  -inf + inf and -inf + NaN are NaN: with an infinity or NaN in a key row, queries that do not see it
 // find their row sum NaN (one test per patch of the forward pass), and the patch is formed again by swag_fwd_exact.  (Replacing
-// masked scores always costs a scalar instruction in front of every select, and a second body inside the march registers: 89 x 98,
+// masked scores always costs a scalar instruction in front of every select, and a second body inside the march costs registers: 89 x 98,
 // d = 32, 15 x 21 window, 32 slabs 49 -> 65 and 58 us.)
 //
 // LDS: token rows of 2 D bytes, 16-byte piece p of the token at halo row r, column c at p ^ swz(r, c), where the swizzle only
@@ -33,6 +33,7 @@ struct SwagArgs {
   DltGeom g;
   int32_t B, H;
   int32_t nstrips, band, nbands;   // band: grid rows per workgroup, a multiple of 4 PR
+  uint32_t m_s, s_s, m_b, s_b, m_h, s_h;   // exact multiply-shift divisions by nstrips, nbands and H
   float scale_log2, sm_scale;
   RopeDev rope;              // ROPE kernels: 8 rotary pairs per axis
   void *q_rot, *k_rot;       // forward: where the rotated q and k go (NULL: nowhere)
@@ -140,12 +141,12 @@ template <int D> DLT_DEV int swag_swz(int row, int col) { return D == 32 ? (row 
 
 struct SwagWho { int b, h, r0, r1, c0; };
 DLT_DEV SwagWho swag_who(const SwagArgs& a, int strip) {
-  int lin = xcd_remap(blockIdx.x, gridDim.x);
+  const int lin = xcd_remap(blockIdx.x, gridDim.x);
   SwagWho w;
-  const int s = lin % a.nstrips; lin /= a.nstrips;
-  const int bd = lin % a.nbands; lin /= a.nbands;
-  w.h = lin % a.H;
-  w.b = lin / a.H;
+  const int row = (int)dlt_fastdiv(lin, a.m_s, a.s_s), s = lin - row * a.nstrips;
+  const int bh = (int)dlt_fastdiv(row, a.m_b, a.s_b), bd = row - bh * a.nbands;
+  w.b = (int)dlt_fastdiv(bh, a.m_h, a.s_h);
+  w.h = bh - w.b * a.H;
   w.c0 = s * strip;
   w.r0 = bd * a.band;
   w.r1 = dlt_imin(w.r0 + a.band, a.g.TR);
@@ -206,93 +207,95 @@ struct SwagRing {
   }
 };
 
-// The ring of the rotating forward kernel: G chunks at a time.  A K item is half of a token row, pieces (2 h, 2 h + 1) = the
-// rotary pair of axis h and (4 + 2 h, 5 + 2 h): a thread turns both partners of its pair with one read of the table row, and the
-// K items of the two chunks a step brings in fill 320 ... 448 of the 512 threads.
-template <typename C, int G>
+// Staging of the rotating forward kernel, two chunks at a time (what a step brings in).  A K item is half of a token row, pieces
+// (2 h, 2 h + 1) = the rotary pair of axis h and (4 + 2 h, 5 + 2 h): a thread turns both partners of its pair with one read of the
+// table row.  Waves 0 ... 3 take the K items of the first chunk (160 ... 224 of 256 threads), waves 4 ... 7 those of the second; the V
+// pieces of both chunks run through all threads.  A thread's items have the same place in every pair of chunks, so offsets inside a
+// grid row and inside a slot are formed once.
+template <typename C>
 struct SwagTurnStage {
-  static constexpr int NK = (G * C::TOK * 2 + 511) / 512, NVV = (G * C::TOK * 8 + 511) / 512;
-  u32x4 k[NK][4], v[NVV];
-  int32_t id[NK];
-  struct At { bool on; int chunk, hr, hc; };
-  static DLT_DEV At at(int i, int per_tok, int tid) {
-    const int x = tid + 512 * i;
-    At p;
-    p.on = x < G * C::TOK * per_tok;
-    p.chunk = x / (C::TOK * per_tok);
-    const int tok = (x - p.chunk * (C::TOK * per_tok)) / per_tok;
-    p.hr = tok / C::HCW;
-    p.hc = tok - p.hr * C::HCW;
-    return p;
-  }
-  // first: grid row of the first chunk's first halo row; chunk c starts 4 c rows further down
-  DLT_DEV void issue(const char* kb, int ksn, const char* vb, int vsn, const SwagArgs& a, int first, int c0, int tid) {
-    const int TC = a.g.TC;
-    auto tok_of = [&](const At& p) {
-      return dlt_imax(0, dlt_imin(first + 4 * p.chunk + p.hr, a.g.TR - 1)) * TC + dlt_imax(0, dlt_imin(c0 - a.g.WC + p.hc, TC - 1));
-    };
+  static constexpr int NV = (2 * C::TOK * 8 + 511) / 512;
+  static_assert(C::PR == 2 && 2 * C::TOK <= 256 && (C::TOK * 8) % 64 == 0, "two chunks per step, a K item per thread, waves of one chunk");
+  struct Data { u32x4 k[4], v[NV]; };
+  const char *kb, *vb;
+  uint32_t krs, vrs, koff, voff[NV];        // bytes between grid rows; offsets inside one
+  int kchunk, krow, kcol, kl, vchunk[NV], vrow[NV], vl[NV];   // chunk (wave-uniform), halo row of the pair, column; offset in a slot
+  bool kon, kown;
+  uint32_t kout;                            // offset of the own token's rotated row inside a grid row
+  int TR, TC, h;
+  DLT_DEV void init(const char* kb_, int ksn, const char* vb_, int vsn, int krsn, const SwagArgs& a, int c0, int tid, int wave) {
+    kb = kb_; vb = vb_; TR = a.g.TR; TC = a.g.TC;
+    krs = (uint32_t)(TC * ksn);
+    vrs = (uint32_t)(TC * vsn);
+    h = tid & 1;
+    const int x = tid & 255, kt = dlt_imin(x >> 1, C::TOK - 1), khr = kt / C::HCW, khc = kt - khr * C::HCW;
+    kon = x < 2 * C::TOK;
+    kchunk = wave >> 2;
+    krow = 4 * kchunk + khr;
+    const int col = c0 - a.g.WC + khc;
+    kcol = dlt_imax(0, dlt_imin(col, TC - 1));
+    koff = (uint32_t)(kcol * ksn) + 32 * h;
+    kl = (khr * C::HCW + khc) * C::ROWB + 16 * ((2 * h) ^ swag_swz<64>(khr, khc));
+    kown = col >= c0 && col < c0 + C::STRIP && col < TC;
+    kout = (uint32_t)(kcol * krsn) + 32 * h;
 #pragma unroll
-    for (int i = 0; i < NK; i++) {
-      const At p = at(i, 2, tid);
-      if (p.on) {
-        const int tok = tok_of(p);
-        id[i] = a.rope.idx[tok];
-        const char* q = kb + (uint32_t)(tok * ksn) + 32 * (tid & 1);
-        k[i][0] = *reinterpret_cast<const u32x4*>(q);
-        k[i][1] = *reinterpret_cast<const u32x4*>(q + 16);
-        k[i][2] = *reinterpret_cast<const u32x4*>(q + 64);
-        k[i][3] = *reinterpret_cast<const u32x4*>(q + 80);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NVV; i++) {
-      const At p = at(i, 8, tid);
-      if (p.on) v[i] = *reinterpret_cast<const u32x4*>(vb + (uint32_t)(tok_of(p) * vsn) + 16 * (tid & 7));
+    for (int i = 0; i < NV; i++) {
+      vchunk[i] = 64 * wave + 512 * i >= C::TOK * 8;
+      const int y = tid + 512 * i - (vchunk[i] ? C::TOK * 8 : 0), vt = dlt_imin(y >> 3, C::TOK - 1), hr = vt / C::HCW, hc = vt - hr * C::HCW;
+      vrow[i] = 4 * vchunk[i] + hr;
+      voff[i] = (uint32_t)(dlt_imax(0, dlt_imin(c0 - a.g.WC + hc, TC - 1)) * vsn) + 16 * (y & 7);
+      vl[i] = C::TB + (hr * C::HCW + hc) * C::ROWB + 16 * ((y & 7) ^ swag_swz<64>(hr, hc));
     }
   }
-  // the K pairs turned in registers; the workgroup's own tokens are also stored to `out` (NULL: nowhere)
+  DLT_DEV bool von(int i, int wave) const { return 512 * (i + 1) <= 2 * C::TOK * 8 || 64 * wave + 512 * i < 2 * C::TOK * 8; }
+  DLT_DEV uint32_t grid_row(int row) const { return (uint32_t)dlt_imax(0, dlt_imin(row, TR - 1)); }
+  // rotary index of the K item (first: see issue)
+  DLT_DEV int32_t index(const SwagArgs& a, int first) const { return a.rope.idx[grid_row(first + krow) * (uint32_t)TC + (uint32_t)kcol]; }
+  // first: grid row of the first chunk's first halo row, the second chunk starts four rows further down; n: chunks wanted
+  DLT_DEV void issue(Data& d, int first, int n, int wave) const {
+    if (kon && kchunk < n) {
+      const uint32_t r = grid_row(first + krow);
+      const char* p = kb + (r * krs + koff);
+      d.k[0] = *reinterpret_cast<const u32x4*>(p);
+      d.k[1] = *reinterpret_cast<const u32x4*>(p + 16);
+      d.k[2] = *reinterpret_cast<const u32x4*>(p + 64);
+      d.k[3] = *reinterpret_cast<const u32x4*>(p + 80);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+      if (von(i, wave) && vchunk[i] < n) d.v[i] = *reinterpret_cast<const u32x4*>(vb + (grid_row(first + vrow[i]) * vrs + voff[i]));
+  }
+  // the K pair turned in registers; the workgroup's own tokens are also stored to `out` (NULL: nowhere)
   template <typename CT>
-  DLT_DEV void turn(const SwagTab& tab, const SwagArgs& a, char* out, int sn2, int first, int r0, int r1, int c0, int tid) {
-#pragma unroll
-    for (int i = 0; i < NK; i++) {
-      const At p = at(i, 2, tid);
-      if (!p.on) continue;
-      f32x4 t[4];
-      if (tab.get(t, id[i], tid & 1, 0, a.rope)) {
-        const u32x4 x0 = k[i][0];
-        k[i][0] = swag_turn<CT>(x0, k[i][1], t, true);
-        k[i][1] = swag_turn<CT>(k[i][1], x0, t, false);
-      }
-      const int row = first + 4 * p.chunk + p.hr, col = c0 - a.g.WC + p.hc;
-      if (out != nullptr && row >= r0 && row < r1 && col >= c0 && col < c0 + C::STRIP && col < a.g.TC) {
-        char* q = out + (uint32_t)((row * a.g.TC + col) * sn2) + 32 * (tid & 1);
-        store_stream16(q, k[i][0]);
-        store_stream16(q + 16, k[i][1]);
-        store_stream16(q + 64, k[i][2]);
-        store_stream16(q + 80, k[i][3]);
-      }
+  DLT_DEV void turn(Data& d, const f32x4 (&t)[4], bool rot, char* out, uint32_t outrs, int first, int n, int r0, int r1) const {
+    if (!(kon && kchunk < n)) return;
+    if (rot) {
+      const u32x4 x0 = d.k[0];
+      d.k[0] = swag_turn<CT>(x0, d.k[1], t, true);
+      d.k[1] = swag_turn<CT>(d.k[1], x0, t, false);
+    }
+    const int row = first + krow;
+    if (out != nullptr && kown && row >= r0 && row < r1) {
+      char* q = out + ((uint32_t)row * outrs + kout);
+      store_stream16(q, d.k[0]);
+      store_stream16(q + 16, d.k[1]);
+      store_stream16(q + 64, d.k[2]);
+      store_stream16(q + 80, d.k[3]);
     }
   }
-  DLT_DEV void commit(swat_lds lds, int slot0, int tid) const {
+  static DLT_DEV int slot_of(int s) { return (s >= C::NRES ? s - C::NRES : s) * C::SLOT; }
+  DLT_DEV void commit_k(const Data& d, swat_lds lds, int slot0, int n) const {
+    if (!(kon && kchunk < n)) return;
+    swat_lds s = lds + slot_of(slot0 + kchunk);
+    swat_write16(s + kl, d.k[0]);
+    swat_write16(s + (kl ^ 16), d.k[1]);
+    swat_write16(s + (kl ^ 64), d.k[2]);
+    swat_write16(s + (kl ^ 80), d.k[3]);
+  }
+  DLT_DEV void commit_v(const Data& d, swat_lds lds, int slot0, int n, int wave) const {
 #pragma unroll
-    for (int i = 0; i < NK; i++) {
-      const At p = at(i, 2, tid);
-      if (!p.on) continue;
-      const int s = slot0 + p.chunk, h = tid & 1, z = swag_swz<64>(p.hr, p.hc);
-      swat_lds d = lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + (p.hr * C::HCW + p.hc) * C::ROWB;
-      swat_write16(d + 16 * ((2 * h) ^ z), k[i][0]);
-      swat_write16(d + 16 * ((2 * h + 1) ^ z), k[i][1]);
-      swat_write16(d + 16 * ((4 + 2 * h) ^ z), k[i][2]);
-      swat_write16(d + 16 * ((5 + 2 * h) ^ z), k[i][3]);
-    }
-#pragma unroll
-    for (int i = 0; i < NVV; i++) {
-      const At p = at(i, 8, tid);
-      if (!p.on) continue;
-      const int s = slot0 + p.chunk;
-      swat_write16(lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + C::TB + (p.hr * C::HCW + p.hc) * C::ROWB + 16 * ((tid & 7) ^ swag_swz<64>(p.hr, p.hc)),
-                   v[i]);
-    }
+    for (int i = 0; i < NV; i++)
+      if (von(i, wave) && vchunk[i] < n) swat_write16(lds + slot_of(slot0 + vchunk[i]) + vl[i], d.v[i]);
   }
 };
 
@@ -586,11 +589,17 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ke
   }
 }
 
-// Forward pass with rotation: K is turned in registers between HBM and LDS, the own queries in theirs
+// Forward pass with rotation: K is turned in registers between HBM and LDS, the own queries in theirs.
+//
+// At two steps per workgroup (2 x 8 slabs of 64 x 64, 13 x 13 window: one workgroup per CU) the time is the fill of the ring and
+// the turning between two steps.  The chunks of the prologue are turned and written pair by pair as their loads return; indices are
+// loaded a step ahead and table rows together with the data, so that nothing dependent is left behind the products; the last
+// step is peeled (a conditional prefetch leaves loads pending across the back edge and every later wait becomes a full one).  Two
+// waves per SIMD get the registers for that, also in the small window classes (5 x 5 spilled 70 registers at four).  Kernel trace,
+// against the version before: 64 x 64 19.3 -> 16.8 us, 128 x 128 64 -> 56, 5 x 5 window on 64 x 64 17.0 -> 10.8.
 template <typename TIO, int D, int NCH, int NCG, int PC>
-__global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_rope_kernel(const SwagArgs a) {
+__global__ __launch_bounds__(512, 2) void swag_fwd_rope_kernel(const SwagArgs a) {
   typedef Swag<D, NCH, NCG, PC> C;
-  constexpr bool ROPE = true;
   typedef typename ComputeOf<TIO>::type CT;
   extern __shared__ __align__(16) char smem[];
   swat_lds lds = (swat_lds)smem;
@@ -601,8 +610,6 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ro
   const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
   const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
   const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
-  SwagRing<C> ring;
-  if constexpr (!ROPE) ring.init(lds, kb_, (int)a.ks[2], vb_, (int)a.vs[2], a, F.w.c0, tid, F.wave);
   const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1]) + 16 * g;
   char* ob = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.out_o) + b * a.os[0] + h * a.os[1]);
   float* lseb = a.lse + b * a.ls[0] + h * a.ls[1];
@@ -615,65 +622,70 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ro
 
   SwagTab tab;
   char *krb = nullptr, *qrb = nullptr;
-  if constexpr (ROPE) {
-    tab.fetch(lds + C::RING, a.rope, tid);   // requested first: it does not depend on any index
-    if (a.k_rot != nullptr) {
-      krb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.k_rot) + b * a.krs[0] + h * a.krs[1]);
-      qrb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.q_rot) + b * a.qrs[0] + h * a.qrs[1]) + 16 * g;
-    }
+  tab.fetch(lds + C::RING, a.rope, tid);   // requested first: it does not depend on any index
+  if (a.k_rot != nullptr) {
+    krb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.k_rot) + b * a.krs[0] + h * a.krs[1]);
+    qrb = reinterpret_cast<char*>(reinterpret_cast<TIO*>(a.q_rot) + b * a.qrs[0] + h * a.qrs[1]) + 16 * g;
   }
-  const int krsn = ROPE ? (int)a.krs[2] * 2 : 0, qrsn = ROPE ? (int)a.qrs[2] * 2 : 0;
+  const int krsn = (int)a.krs[2] * 2, qrsn = (int)a.qrs[2] * 2;
   u32x4 qn[C::KC];
-  int32_t qid = -1;
   auto load_q = [&](int rp) {
     const int tok = F.own_tok(rp);
 #pragma unroll
     for (int c = 0; c < C::KC; c++) qn[c] = *reinterpret_cast<const u32x4*>(qb + (uint32_t)(tok * qsn) + 64 * c);
-    if constexpr (ROPE) qid = a.rope.idx[tok];
   };
+  // the own queries of patch rp turned in registers and stored
+  auto turn_q = [&](int rp, const f32x4 (&t)[4], bool rot) {
+    const u32x4 partner = {swag_lane_xor16(qn[0].x, g), swag_lane_xor16(qn[0].y, g), swag_lane_xor16(qn[0].z, g), swag_lane_xor16(qn[0].w, g)};
+    if (rot) qn[0] = swag_turn<CT>(qn[0], partner, t, (g & 1) == 0);
+    if (qrb != nullptr && F.own_ok(rp)) {
+#pragma unroll
+      for (int c = 0; c < C::KC; c++) store_stream16(qrb + (uint32_t)(F.own_tok(rp) * qrsn) + 64 * c, qn[c]);
+    }
+  };
+  typedef SwagTurnStage<C> Stage;
+  Stage stage;
+  const uint32_t outrs = (uint32_t)(F.TC * krsn);
+  stage.init(kb_, ksn, vb_, vsn, krsn, a, F.w.c0, tid, F.wave);
+  constexpr int NPAIR = (C::NRES + 1) / 2;
+  typename Stage::Data pre[NPAIR];
+  int32_t id[NPAIR];
+#pragma unroll
+  for (int j = 0; j < NPAIR; j++) id[j] = stage.index(a, F.w.r0 - F.WR + 8 * j);
+  const int32_t idq0 = a.rope.idx[F.own_tok(F.w.r0 + 4 * F.rg)];
+#pragma unroll
+  for (int j = 0; j < NPAIR; j++) stage.issue(pre[j], F.w.r0 - F.WR + 8 * j, C::NRES - 2 * j, F.wave);
   load_q(F.w.r0 + 4 * F.rg);
-  if constexpr (ROPE) {
-    SwagTurnStage<C, C::NRES> pre;
-    pre.issue(kb_, ksn, vb_, vsn, a, F.w.r0 - F.WR, F.w.c0, tid);
-    tab.store(tid);
-    __syncthreads();
-    pre.template turn<CT>(tab, a, krb, krsn, F.w.r0 - F.WR, F.w.r0, F.w.r1, F.w.c0, tid);
-    pre.commit(lds, 0, tid);
-  } else {
-    ring.fill(F.w.r0 - F.WR);
+  // rotary indices of the next step's K item and own queries: always loaded a step ahead
+  int32_t idk = stage.index(a, F.w.r0 - F.WR + 4 * C::NRES);
+  int32_t idq = a.rope.idx[F.own_tok(F.w.r0 + 4 * F.rg + 4 * C::PR)];
+  tab.store(tid);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NPAIR; j++) {
+    f32x4 t[4];
+    const bool rot = tab.get(t, id[j], stage.h, 0, a.rope);
+    stage.template turn<CT>(pre[j], t, rot, krb, outrs, F.w.r0 - F.WR + 8 * j, C::NRES - 2 * j, F.w.r0, F.w.r1);
+    stage.commit_k(pre[j], lds, 2 * j, C::NRES - 2 * j);
+    stage.commit_v(pre[j], lds, 2 * j, C::NRES - 2 * j, F.wave);
+  }
+  {
+    f32x4 t[4];
+    const bool rot = tab.get(t, idq0, g >> 1, 0, a.rope);
+    turn_q(F.w.r0 + 4 * F.rg, t, rot);
   }
   __syncthreads();
 
   int slot0 = 0;   // slot of the step's first chunk
-  for (int r = F.w.r0; r < F.w.r1; r += 4 * C::PR) {
-    const int rp = r + 4 * F.rg;
-    u32x4 q[C::KC];
-#pragma unroll
-    for (int c = 0; c < C::KC; c++) q[c] = qn[c];
-    pin_loaded(q);
-    if constexpr (ROPE) {
-      f32x4 t[4];
-      const bool rot = tab.get(t, qid, g >> 1, 0, a.rope);
-      const u32x4 partner = {swag_lane_xor16(q[0].x, g), swag_lane_xor16(q[0].y, g), swag_lane_xor16(q[0].z, g), swag_lane_xor16(q[0].w, g)};
-      if (rot) q[0] = swag_turn<CT>(q[0], partner, t, (g & 1) == 0);
-      if (qrb != nullptr && F.own_ok(rp)) {
-#pragma unroll
-        for (int c = 0; c < C::KC; c++) store_stream16(qrb + (uint32_t)(F.own_tok(rp) * qrsn) + 64 * c, q[c]);
-      }
+  auto store = [&](int rp, const f32x4 (&acc)[C::DB], float l, float m_use) {
+    if (F.own_ok(rp)) {
+      const int tok = F.own_tok(rp);
+      swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+      if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
     }
-    const bool more = r + 4 * C::PR < F.w.r1;
-    u32x4 nx[C::PR][C::NIT];
-    SwagTurnStage<C, C::PR> nt;
-    const int next = r - F.WR + 4 * C::NRES;   // first halo row of the chunks to come
-    if (more) {
-      if constexpr (ROPE) {
-        nt.issue(kb_, ksn, vb_, vsn, a, next, F.w.c0, tid);
-      } else {
-#pragma unroll
-        for (int i = 0; i < C::PR; i++) ring.issue(nx[i], next + 4 * i);
-      }
-      load_q(rp + 4 * C::PR);
-    }
+  };
+  // scores, softmax and output of the patch whose first own row is rp; q: its queries
+  auto attend = [&](int rp, const u32x4 (&q)[C::KC]) __attribute__((always_inline)) {
     if (rp < F.TR && F.w.c0 + 4 * F.pc < F.TC) {
       swat_lds rowp[NCH];
 #pragma unroll
@@ -685,12 +697,12 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ro
       float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
       for (int i = 0; i < NCH; i++) {
-        const bool row = F.sees_row(i, rp);
+        const float bias = F.row_bias(i, rp);
 #pragma unroll
         for (int j = 0; j < NCG; j++) {
-          f32x4 t = swag_scores<C, CT>(rowp[i] + 4 * j * C::ROWB, L, q, 0.f);
+          f32x4 t = swag_scores<C, CT>(rowp[i] + 4 * j * C::ROWB, L, q, bias);
 #pragma unroll
-          for (int e = 0; e < 4; e++) t[e] = (row & F.sees_col(4 * j + e)) ? t[e] : -INFINITY;
+          for (int e = 0; e < 4; e++) t[e] = F.sees_col(4 * j + e) ? t[e] : -INFINITY;
           s[i * NCG + j] = t;
         }
       }
@@ -699,7 +711,7 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ro
 #pragma unroll
         for (int e = 0; e < 4; e++) mx[e] = fmaxf(fmaxf(mx[e], s[k][e]), s[k + 1 < C::NB ? k + 1 : k][e]);
       const float m = wave_max4(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
-      const float m_use = m == -INFINITY ? 0.f : m;   // own positions outside the grid see nothing
+      float m_use = m == -INFINITY ? 0.f : m;   // own positions outside the grid see nothing
       const float neg_m2 = -m_use * scale;
       f32x4 acc[C::DB], acc_l = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -722,26 +734,41 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ro
         }
         acc_l = Mma<CT>::mfma(ones, pb, acc_l);
       }
-      const float l = acc_l[0];
-      if (F.own_ok(rp)) {
-        const int tok = F.own_tok(rp);
-        swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
-        if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
+      float l = acc_l[0];
+      if (__builtin_amdgcn_ballot_w64(l != l)) {   // an infinite or NaN key in or beside the window of some query
+        keep_branch();
+        swag_fwd_exact<C, CT, NCG>(F, L, rp, q, scale, acc, l, m_use, [&](int i, int j) {
+          const int s = slot0 + F.rg + i;
+          return lds + (s >= C::NRES ? s - C::NRES : s) * C::SLOT + 4 * (F.pc + j) * C::ROWB;
+        });
       }
+      store(rp, acc, l, m_use);
     }
-    if (more) {
-      if constexpr (ROPE) nt.template turn<CT>(tab, a, krb, krsn, next, F.w.r0, F.w.r1, F.w.c0, tid);
-      __syncthreads();
-      if constexpr (ROPE) {
-        nt.commit(lds, slot0, tid);
-      } else {
+  };
+  int r = F.w.r0;
+  for (; r + 4 * C::PR < F.w.r1; r += 4 * C::PR) {
+    const int rp = r + 4 * F.rg, next = r - F.WR + 4 * C::NRES;   // next: first halo row of the chunks to come
+    u32x4 q[C::KC];
 #pragma unroll
-        for (int i = 0; i < C::PR; i++) ring.commit(nx[i], slot0 + i >= C::NRES ? slot0 + i - C::NRES : slot0 + i);
-      }
-      __syncthreads();
-      slot0 = slot0 + C::PR >= C::NRES ? slot0 + C::PR - C::NRES : slot0 + C::PR;
-    }
+    for (int c = 0; c < C::KC; c++) q[c] = qn[c];
+    // the table rows are requested with the data and there when the products are done
+    f32x4 tk[4], tq[4];
+    const bool rk = tab.get(tk, idk, stage.h, 0, a.rope), rq = tab.get(tq, idq, g >> 1, 0, a.rope);
+    typename Stage::Data nt;
+    stage.issue(nt, next, 2, F.wave);
+    idk = stage.index(a, next + 4 * C::PR);
+    idq = a.rope.idx[F.own_tok(rp + 8 * C::PR)];
+    load_q(rp + 4 * C::PR);
+    attend(rp, q);
+    stage.template turn<CT>(nt, tk, rk, krb, outrs, next, 2, F.w.r0, F.w.r1);
+    turn_q(rp + 4 * C::PR, tq, rq);
+    __syncthreads();
+    stage.commit_k(nt, lds, slot0, 2);
+    stage.commit_v(nt, lds, slot0, 2, F.wave);
+    __syncthreads();
+    slot0 = slot0 + C::PR >= C::NRES ? slot0 + C::PR - C::NRES : slot0 + C::PR;
   }
+  attend(r + 4 * F.rg, qn);
 }
 
 // dQ: own = queries, K and V in the ring; delta = rowsum(o dO) of the own queries is formed and stored on the way.

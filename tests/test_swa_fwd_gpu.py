@@ -154,6 +154,31 @@ def test_fused_rope_forward_equals_composition():
     assert torch.equal(comp, got)
 
 
+# every window class of the rotating marching kernel, in bands of one step (few slabs) and of several (more strips than CUs), with rows
+# and columns that fill neither a step nor a strip, tables read from LDS (up to 128 positions) and from memory: rotated rows, outputs and
+# lse2 have the bits of the rotation followed by the plain kernel (each checked against the oracle on its own); the oracle on two slabs
+@pytest.mark.parametrize("WR,WC", [(2, 2), (1, 4), (2, 6), (4, 1), (4, 3), (3, 6), (6, 2), (5, 4), (6, 6), (0, 0)])
+@pytest.mark.parametrize("B,H,th,tw,table", [(1, 3, 5, 9, 32), (2, 2, 21, 33, 64), (4, 30, 42, 40, 65), (3, 90, 17, 15, 32)])
+def test_fused_rope_forward_in_steps_and_window_classes(B, H, th, tw, table, WR, WC):
+    from dl_templates_amd import fused_rope2d as fr
+    sw = _swa()
+    N, d, dtype = th * tw, 64, torch.float16 if WR == WC else torch.bfloat16
+    q, k, v, _ = orc.make_qkv(N + 7 * WR + WC, B, H, N, N, d, d, dtype)
+    idx, rcs, ccs = orc.make_rope_idx(N, th, tw, 0.1), orc.rope_tables(8, table), orc.rope_tables(8, table)
+    rope = (idx.cuda(), rcs.cuda(), ccs.cuda())
+    qg, kg, vg = q.cuda(), k.cuda(), v.cuda()
+    shape = sw._shape(qg, kg, vg, 1, th, tw, WR, WC, 0.125)
+    o, lse, q_rot, k_rot = sw._forward_rot(qg, kg, vg, shape, rope)
+    q2, k2 = fr.rope2d_qk_(qg.clone(), kg.clone(), *rope)
+    want, lse_w = sw._forward(q2, k2, vg, shape, None)
+    assert torch.equal(q_rot, q2) and torch.equal(k_rot, k2)
+    assert torch.equal(o, want) and torch.equal(lse, lse_w)
+    assert torch.equal(sw._forward(qg, kg, vg, shape, rope)[0], want)   # nothing kept of the rotation
+    few = (slice(B - 1, B), slice(H - 2, H))
+    ref = orc.rope_swa_ref(q[few].float(), k[few].float(), v[few].float(), idx, rcs, ccs, 1, th, tw, WR, WC, 0.125)
+    assert (o[few].float().cpu() - ref).abs().max().item() <= FWD_TOL
+
+
 @pytest.mark.parametrize("d,R", [(64, 8), (128, 32), (128, 16)])
 def test_fused_rope_forward_lse_and_head_dim_fully_rotated(d, R):
     """lse2 of the fused forward against the oracle's composition; (128, 32) rotates the whole head dim with
