@@ -26,9 +26,10 @@ def test_register_staged_kernels_behind_the_environment_switch():
 
 
 def test_one_patch_streaming_forward_kernel_behind_the_environment_switch():
-    """DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the forward kernel with one patch per wave at head dim 128 on
-    grids of more than 8 rows (without the switch it only runs on grids of up to 8 rows): the head-dim-128 token-grid
-    tests pass in a child process that sets it."""
+    """DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the streaming forward kernel with one patch per wave in launches of
+    more workgroups than CUs too (without the switch those run two patches per wave, at both head dims and any token
+    strides, and smaller launches one): the streaming kernels' forward tests, those of the large launches among them, pass in a
+    child process that sets it."""
     import os
     import subprocess
     import sys
@@ -37,7 +38,7 @@ def test_one_patch_streaming_forward_kernel_behind_the_environment_switch():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     env = dict(os.environ, DLT_SWA2_SINGLE_PATCH="1")
     r = subprocess.run([sys.executable, "-u", "-m", "pytest", "tests/test_swa_fwd_gpu.py", "tests/test_swa_tiles_gpu.py", "-m", "gpu", "-x", "-q",
-                        "-k", "head_dim_128 or wider or small_tiles or head_dims", "-p", "no:cacheprovider"],
+                        "-k", "head_dim_128 or wider or small_tiles or head_dims or two_patches", "-p", "no:cacheprovider"],
                        cwd=root, env=env, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-1000:]
     assert " passed" in r.stdout and "failed" not in r.stdout, r.stdout[-500:]
