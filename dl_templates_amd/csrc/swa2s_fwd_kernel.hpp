@@ -8,9 +8,10 @@
 // the output products, a barrier between the two.  A workgroup then fits into half the LDS of a CU (74 KB at head dim 128,
 // 6 column groups), and the two (head dim 64: up to four) workgroups of a CU are in different phases: one fills the waits of the
 // other.  An earlier version ran 8 waves over bands of 16 rows with both chunk buffers doubled, one workgroup per CU: the waves
-// stood together at every barrier, and half of them had no row of the first two and last two chunks.  Back-to-back calls, 16
-// slabs at d = 128, 21 x 21 window: 128 x 128 tokens 99.4 -> 95.6 us, 97 x 161 107.5 -> 98.0; 32 slabs of 103 x 36, 21 x 7: 54.6
-// -> 46.0; d = 64, 32 slabs of 89 x 98, 15 x 21: 73 -> 66.7 (there against one patch per wave).  Of 106 us in a short burst the
+// stood together at every barrier, and half of them had no row of the first two and last two chunks.  Back-to-back calls on one set
+// of inputs, 16 slabs at d = 128, 21 x 21 window: 128 x 128 tokens 99.7 -> 94.7 us, 97 x 161 105.7 -> 94 (over three sets of inputs in
+// turn 112.6 -> 104.5); 32 slabs of 103 x 36, 21 x 7: 54.2 -> 45.2; d = 64, 32 slabs of 89 x 98, 15 x 21: 74 -> 66.6 (there against one
+// patch per wave).  Of 106 us in a short burst the
 // matrix and vector instructions account for 71 (the issue port), LDS operand reads and the copies for the rest: without
 // either of the two it runs in 91 ... 94.  Leaving out the column test where a whole group is inside every window, a longer
 // read-ahead of K and copies issued earlier in their phase measured the same within 1 %.

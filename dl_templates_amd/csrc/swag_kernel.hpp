@@ -596,7 +596,7 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ke
 // loaded a step ahead and table rows together with the data, so that nothing dependent is left behind the products; the last
 // step is peeled (a conditional prefetch leaves loads pending across the back edge and every later wait becomes a full one).  Two
 // waves per SIMD get the registers for that, also in the small window classes (5 x 5 spilled 70 registers at four).  Kernel trace,
-// against the version before: 64 x 64 19.3 -> 16.8 us, 128 x 128 64 -> 56, 5 x 5 window on 64 x 64 17.0 -> 10.8.
+// against chunks staged with the plain kernel's frame: 64 x 64 19.3 -> 16.7 us, 128 x 128 63 -> 56, 5 x 5 window on 64 x 64 17.0 -> 10.7.
 template <typename TIO, int D, int NCH, int NCG, int PC>
 __global__ __launch_bounds__(512, 2) void swag_fwd_rope_kernel(const SwagArgs a) {
   typedef Swag<D, NCH, NCG, PC> C;
