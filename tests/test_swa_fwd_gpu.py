@@ -339,7 +339,11 @@ def test_two_patches_per_wave_column_passes(H, S, th, tw, WR, WC, d):
     (2, 1, 13, 21, 3, 2, 64, torch.bfloat16, True, "marching"), (2, 1, 25, 20, 7, 3, 64, torch.bfloat16, False, "streaming"),
     (50, 1, 25, 20, 7, 3, 64, torch.bfloat16, False, "streaming"), (2, 1, 25, 20, 2, 3, 128, torch.float16, False, "streaming"),
     (50, 1, 25, 20, 2, 3, 128, torch.float16, False, "streaming"), (50, 1, 26, 40, 9, 10, 128, torch.bfloat16, False, "streaming"),
-    (40, 1, 17, 60, 3, 12, 128, torch.bfloat16, False, "streaming"), (80, 4, 20, 9, 1, 1, 64, torch.bfloat16, False, "streaming")])
+    (40, 1, 17, 60, 3, 12, 128, torch.bfloat16, False, "streaming"), (80, 4, 20, 9, 1, 1, 64, torch.bfloat16, False, "streaming"),
+    # bands of several steps
+    (150, 1, 43, 37, 6, 6, 64, torch.float16, False, "marching"), (200, 1, 43, 37, 2, 1, 64, torch.bfloat16, False, "marching"),
+    (150, 1, 43, 37, 6, 5, 64, torch.bfloat16, True, "marching"), (200, 1, 43, 37, 1, 2, 64, torch.float16, True, "marching"),
+    (150, 1, 41, 40, 7, 10, 32, torch.bfloat16, False, "marching"), (150, 1, 43, 37, 4, 3, 32, torch.float32, False, "marching")])
 def test_infinite_and_nan_keys_stay_inside_their_window(H, S, th, tw, WR, WC, d, dtype, rope, family, bad):
     sw = _swa()
     from dl_templates_amd import _lib
