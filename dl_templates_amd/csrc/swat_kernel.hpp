@@ -23,6 +23,8 @@ struct SwatArgs {
   float* lse;
   float* delta;
   int64_t qs[5], ks[5], vs[5], os[5], dos[5], dqs[5], dks[5], dvs[5], ls[3];
+  const void* ring_p[4];   // swat_bwd_kernel: K, V, Q, dO as its ring holds them, picked by a wave-uniform index
+  int64_t ring_s[4][5];
   DltTokMap tm;
   DltGeom g;
   int32_t B, H;
@@ -72,7 +74,7 @@ template <typename T> DLT_DEV const char* swat_slab(const void* p, const int64_t
 // Who a workgroup is: heads innermost (image rows hold all heads of a pixel side by side: the workgroups that share its
 // 128-byte lines run at the same time on one XCD), then strips, bands and batches.
 struct SwatWho { int b, h, r0, r1, xs; };
-DLT_DEV SwatWho swat_who(const SwatArgs& a) {
+DLT_DEV SwatWho swat_who(const SwatArgs& a, int width = 128) {
   int lin = xcd_remap(blockIdx.x, gridDim.x);
   SwatWho w;
   if (a.tm.img) {
@@ -80,13 +82,13 @@ DLT_DEV SwatWho swat_who(const SwatArgs& a) {
     const int s = lin % a.nstrips; lin /= a.nstrips;
     const int bd = lin % a.nbands;
     w.b = lin / a.nbands;
-    w.xs = s * 128; w.r0 = bd * a.band;
+    w.xs = s * width; w.r0 = bd * a.band;
   } else {
     const int s = lin % a.nstrips; lin /= a.nstrips;
     const int bd = lin % a.nbands; lin /= a.nbands;
     w.h = lin % a.H;
     w.b = lin / a.H;
-    w.xs = s * 128; w.r0 = bd * a.band;
+    w.xs = s * width; w.r0 = bd * a.band;
   }
   w.r1 = dlt_imin(w.r0 + a.band, a.g.TR);
   return w;
@@ -170,17 +172,23 @@ struct SwatLane {
 };
 
 // Own rows leave straight from the accumulators: a lane of the C layout holds 4 dims of its token in each 16-dim block; the
-// lane swap of two blocks gives every lane 8 consecutive dims (16 bytes), four lanes a whole 64-byte piece.
+// lane swap of two blocks gives every lane 8 consecutive dims (16 bytes) of token n, and the permutation behind it brings the
+// four pieces of a 64-byte run to four consecutive lanes (lane l: token l / 4, piece l % 4).  Without it the 16 lanes that the
+// memory pipe takes at a time wrote 16 bytes each into 16 rows, and the streaming stores left in parts of a sector: 1.25 to 1.3
+// times the bytes (D = 64 forward, 210 MB of o: 268 MB written; 498 MB of gradients for 403 at D = 32).
+// p: row of token lane / 4 plus 16 (lane % 4) bytes.  Blocks of 16 tokens lie inside the grid or outside as a whole.
 template <typename CT, int DB>
-DLT_DEV void swat_store_row(char* p, const f32x4 (&acc)[DB], float mul, int g) {
+DLT_DEV void swat_store_row(char* p, const f32x4 (&acc)[DB], float mul, int lane) {
   typedef unsigned pair_t __attribute__((ext_vector_type(2)));
+  const int from = 4 * ((lane >> 2) + 16 * (((lane >> 1) & 1) | ((lane & 1) << 1)));
+  auto take = [&](unsigned v) { return (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)v); };
 #pragma unroll
   for (int d = 0; d < DB; d += 2) {
     const pair_t lo = __builtin_amdgcn_permlane16_swap(pack2<CT>(acc[d][0] * mul, acc[d][1] * mul), pack2<CT>(acc[d + 1][0] * mul, acc[d + 1][1] * mul),
                                                        false, false);
     const pair_t hi = __builtin_amdgcn_permlane16_swap(pack2<CT>(acc[d][2] * mul, acc[d][3] * mul), pack2<CT>(acc[d + 1][2] * mul, acc[d + 1][3] * mul),
                                                        false, false);
-    store_stream16(p + 2 * (16 * d + 16 * (g & 1) + 8 * (g >> 1)), u32x4{lo.x, hi.x, lo.y, hi.y});
+    store_stream16(p + 32 * d, u32x4{take(lo.x), take(hi.x), take(lo.y), take(hi.y)});
   }
 }
 
@@ -214,9 +222,9 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const bool own = w.xs + 16 * wave < XL;                     // wave-uniform: the wave has a block of the grid
   const int tile = (w.xs + 16 * wave) / (16 * NTB);
   const int blk = NTB == 1 ? wave : wave / NTB * NTB;         // first staged block of the wave's window
-  const int xc = dlt_imin(x, XL - 1);
+  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + (lane >> 2), XL - 1);   // token of the lane's loads, of its stores
   const char* qb = swat_slab<TIO>(a.q, a.qs, w.b, w.h) + swat_slot_off(a.tm, a.qs, xc) + 16 * g;
-  char* ob = const_cast<char*>(swat_slab<TIO>(a.out_o, a.os, w.b, w.h)) + swat_slot_off(a.tm, a.os, xc);
+  char* ob = const_cast<char*>(swat_slab<TIO>(a.out_o, a.os, w.b, w.h)) + swat_slot_off(a.tm, a.os, xw) + 16 * (lane & 3);
   float* lseb = a.lse + w.b * a.ls[0] + w.h * a.ls[1] + (int64_t)x * a.ls[2];
   const uint32_t qrs = swat_row_bytes(a.tm, a.qs, XL), ors = swat_row_bytes(a.tm, a.os, XL);
   SwatLane<C> L;
@@ -225,6 +233,9 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const unsigned one2 = pack2<CT>(1.f, 1.f);
   const u32x4 ones = {one2, one2, one2, one2};
 
+  // 18 blocks of scores at 128 registers a lane: requested in front of them the next q was spilled, i.e. waited for with
+  // every piece in flight; it is requested once half of the scores are gone
+  constexpr bool LATE_Q = C::OCC == 4 && C::NB > 15;
   u32x4 qn[C::KC];
   auto load_q = [&](int r) {
 #pragma unroll
@@ -243,7 +254,7 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
     const bool more = r + 1 < w.r1;
     if (more) {
       ring.issue(r + 1 + WR);
-      load_q(r + 1);
+      if constexpr (!LATE_Q) load_q(r + 1);
     }
     SwatSeen<C, NTB> seen;
     seen.init(a, r, tile, WC, WR);
@@ -290,6 +301,8 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
           p[4 + i] = 2 * t + 1 <= LAST ? fast_exp2(fmaf(s[b1][i], scale, neg_m2)) : 0.f;
         }
         const u32x4 pb = pack8<CT>(p);
+        if constexpr (LATE_Q)
+          if (t == C::NP / 2 && more) load_q(r + 1);
         swat_lds v0 = rowp[b0 / C::NWB] + C::TB + (b0 % C::NWB) * C::BLKB, v1 = rowp[b1 / C::NWB] + C::TB + (b1 % C::NWB) * C::BLKB;
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
@@ -299,10 +312,8 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
         acc_l = Mma<CT>::mfma(ones, pb, acc_l);
       }
       const float l = acc_l[0];
-      if (x < XL) {
-        swat_store_row<CT, C::DB>(ob + (uint32_t)r * ors, acc, fast_rcp(l), g);
-        if (g == 0) store_stream4(lseb + (int64_t)r * XL * a.ls[2], m * scale + fast_log2(l));
-      }
+      swat_store_row<CT, C::DB>(ob + (uint32_t)r * ors, acc, fast_rcp(l), lane);
+      if (g == 0) store_stream4(lseb + (int64_t)r * XL * a.ls[2], m * scale + fast_log2(l));
     };
     if (own) {
       if (seen.all()) step(std::false_type{});
@@ -335,11 +346,11 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const bool own = w.xs + 16 * wave < XL;
   const int tile = (w.xs + 16 * wave) / (16 * NTB);
   const int blk = NTB == 1 ? wave : wave / NTB * NTB;
-  const int xc = dlt_imin(x, XL - 1);
+  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + (lane >> 2), XL - 1);   // token of the lane's loads, of its stores
   const char* qb = swat_slab<TIO>(a.q, a.qs, w.b, w.h) + swat_slot_off(a.tm, a.qs, xc) + 16 * g;
   const char* dob = swat_slab<TIO>(a.d_o, a.dos, w.b, w.h) + swat_slot_off(a.tm, a.dos, xc) + 16 * g;
   const char* ob = swat_slab<TIO>(a.o, a.os, w.b, w.h) + swat_slot_off(a.tm, a.os, xc) + 16 * g;
-  char* dqb = const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xc);
+  char* dqb = const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xw) + 16 * (lane & 3);
   const float* lseb = a.lse + w.b * a.ls[0] + w.h * a.ls[1] + (int64_t)xc * a.ls[2];
   float* delb = a.delta + w.b * a.ls[0] + w.h * a.ls[1] + (int64_t)xc * a.ls[2];
   const uint32_t qrs = swat_row_bytes(a.tm, a.qs, XL), dors = swat_row_bytes(a.tm, a.dos, XL), ors = swat_row_bytes(a.tm, a.os, XL),
@@ -431,7 +442,7 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
           acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
         }
       }
-      if (x < XL) swat_store_row<CT, C::DB>(dqb + (uint32_t)r * dqrs, acc, a.sm_scale, g);
+      swat_store_row<CT, C::DB>(dqb + (uint32_t)r * dqrs, acc, a.sm_scale, lane);
     };
     if (own) {
       if (seen.all()) step(std::false_type{});
@@ -483,11 +494,11 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const bool own = w.xs + 16 * wave < XL;
   const int tile = (w.xs + 16 * wave) / (16 * NTB);
   const int blk = NTB == 1 ? wave : wave / NTB * NTB;
-  const int xc = dlt_imin(x, XL - 1);
+  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + (lane >> 2), XL - 1);   // token of the lane's loads, of its stores
   const char* kb = swat_slab<TIO>(a.k, a.ks, w.b, w.h) + swat_slot_off(a.tm, a.ks, xc) + 16 * g;
   const char* vb = swat_slab<TIO>(a.v, a.vs, w.b, w.h) + swat_slot_off(a.tm, a.vs, xc) + 16 * g;
-  char* dkb = const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xc);
-  char* dvb = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xc);
+  char* dkb = const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xw) + 16 * (lane & 3);
+  char* dvb = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xw) + 16 * (lane & 3);
   const uint32_t krs = swat_row_bytes(a.tm, a.ks, XL), vrs = swat_row_bytes(a.tm, a.vs, XL), dkrs = swat_row_bytes(a.tm, a.dks, XL),
                  dvrs = swat_row_bytes(a.tm, a.dvs, XL);
   SwatLane<C> L;
@@ -585,10 +596,8 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
           acc_k[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc_k[d]);
         }
       }
-      if (x < XL) {
-        swat_store_row<CT, C::DB>(dvb + (uint32_t)r * dvrs, acc_v, 1.f, g);
-        swat_store_row<CT, C::DB>(dkb + (uint32_t)r * dkrs, acc_k, a.sm_scale, g);
-      }
+      swat_store_row<CT, C::DB>(dvb + (uint32_t)r * dvrs, acc_v, 1.f, lane);
+      swat_store_row<CT, C::DB>(dkb + (uint32_t)r * dkrs, acc_k, a.sm_scale, lane);
     };
     if (own) {
       if (seen.all()) step(std::false_type{});
@@ -598,6 +607,276 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
       __syncthreads();
       ring.commit(slot0);
       commit_scal(slot0);
+      __syncthreads();
+      slot0 = slot0 + 1 == C::NR ? 0 : slot0 + 1;
+    }
+  }
+}
+
+// ---- dQ, dK and dV in one launch (16-token tiles, 3 x 3 window) ---------------------------------------------------
+// What bounded the two launches above: HBM.  Both read q, k, v and dO, dQ also o: with the gradients, delta and lse2 that is
+// 12 passes over a tensor of the operator where 8 are needed (B = 4, H = 8, 256 x 256 pixels in 4 x 4 tiles, d = 32, image
+// layout: 210 + 243 us at 4.3 TB/s).  With all four tensors of the window's rows in the ring (K, V, Q, dO: 120 KB at D = 32, 147 at
+// D = 64, one workgroup per CU) a strip's dQ, dK and dV leave in one march: the first half of the waves own query blocks, the
+// second half key blocks; both take their own fragments, lse2 and delta from the ring, and delta is formed by the threads
+// that stage dO (they fetch the pieces of o beside it), so nothing travels between launches.  Strips of 8 blocks and 16 waves
+// at D = 32; at D = 64 the ring holds strips of 4 (8 waves).  Measured: the backward pass above 453 -> 290 us (1.18 GB, 4.1
+// TB/s); d = 64, 16 slabs of 40 x 40 tiles x 4 batches 540 -> 433.  Larger windows and 32-token tiles stay on two launches: their
+// rows would fit at D = 32, but there the arithmetic is the bound and one workgroup per CU ties (5 columns: 164 against 166 us)
+// or loses (32-token tiles: 91 against 100).
+template <int D, int NTB, int WC, int WR>
+struct Swab : Swat<D, NTB, WC, WR> {
+  typedef Swat<D, NTB, WC, WR> Base;
+  static constexpr int SB = D == 32 ? 8 : 4;                        // 16-token blocks of a strip
+  static constexpr int NWAVE = 2 * SB, THREADS = 64 * NWAVE;
+  static constexpr int HB = SB + 2 * WC * NTB, TOK = 16 * HB;
+  static constexpr int TB = TOK * Base::ROWB, SLOT = 4 * TB;        // K, V, Q, dO of a grid row
+  static constexpr int WPT = TOK * Base::PIECES / 64;               // wave-wide vectors per tensor and row
+  static constexpr int NIT = (4 * WPT + NWAVE - 1) / NWAVE;
+  static constexpr int RING = Base::NR * SLOT, SCAL = Base::NR * 2 * TOK * 4, LDS = RING + SCAL;
+  static constexpr bool USED = NTB == 1 && WC == 1 && WR == 1;
+  static_assert(!USED || (TOK * Base::PIECES % 64 == 0 && TOK <= THREADS && LDS <= 160 * 1024), "staging map, LDS");
+};
+
+// sum over the lanes that hold the 16-byte pieces of one token (4 or 8 consecutive lanes)
+template <int PIECES>
+DLT_DEV float swat_sum_pieces(float v) {
+  static_assert(PIECES == 4 || PIECES == 8, "a quad or half a row of lanes");
+  auto dpp = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v += dpp(v, std::integral_constant<int, 0x4e>{});   // lane ^ 2
+  v += dpp(v, std::integral_constant<int, 0xb1>{});   // lane ^ 1
+  if constexpr (PIECES == 8) v += dpp(v, std::integral_constant<int, 0x141>{});   // the other quad of the eight
+  return v;
+}
+
+template <typename TIO, int D, int NTB, int WC, int WR>
+__global__ __launch_bounds__((Swab<D, NTB, WC, WR>::THREADS), (Swab<D, NTB, WC, WR>::NWAVE / 4)) void swat_bwd_kernel(const SwatArgs a) {
+  typedef Swab<D, NTB, WC, WR> C;
+  typedef typename ComputeOf<TIO>::type CT;
+  extern __shared__ __align__(16) char smem[];
+  swat_lds lds = (swat_lds)smem;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const SwatWho w = swat_who(a, 16 * C::SB);
+  const int XL = a.g.XLq, TR = a.g.TR;
+  DLT_LDS float* scal = reinterpret_cast<DLT_LDS float*>(lds + C::RING);   // [slot][-lse2 | delta][token]
+
+  // ---- staging: vector wave + NWAVE it of a grid row belongs to tensor (that) / WPT (K, V, Q, dO): wave-uniform
+  const int xh = w.xs - 16 * WC * NTB;   // first staged slot
+  const char* base[C::NIT];
+  uint32_t rs[C::NIT], goff[C::NIT], ooff[C::NIT];
+  int loff[C::NIT], tok_of[C::NIT];
+  const char* ob = swat_slab<TIO>(a.o, a.os, w.b, w.h);
+  const uint32_t ors = swat_row_bytes(a.tm, a.os, XL);
+  auto may_be_do = [](int it) { return C::NWAVE * (it + 1) > 3 * C::WPT; };
+#pragma unroll
+  for (int it = 0; it < C::NIT; it++) {
+    const int wv = wave + C::NWAVE * it, ten = dlt_imin(wv / C::WPT, 3);
+    const int v = (wv - ten * C::WPT) * 64 + lane, tok = v / C::PIECES, piece = v % C::PIECES;
+    // slots outside the grid row are clamped onto it: they belong to tiles that nobody sees
+    const int x = dlt_imax(0, dlt_imin(xh + tok, XL - 1));
+    base[it] = swat_slab<TIO>(a.ring_p[ten], a.ring_s[ten], w.b, w.h);
+    rs[it] = swat_row_bytes(a.tm, a.ring_s[ten], XL);
+    goff[it] = swat_slot_off(a.tm, a.ring_s[ten], x);
+    goff[it] += 16 * piece;
+    ooff[it] = may_be_do(it) ? swat_slot_off(a.tm, a.os, x) + 16 * piece : 0u;
+    loff[it] = ten * C::TB + tok * C::ROWB + 16 * (piece ^ swat_swz<D>(tok));
+    tok_of[it] = tok;
+  }
+  const int xsc = dlt_imax(0, dlt_imin(xh + tid, XL - 1));
+  const float* lseb = a.lse + w.b * a.ls[0] + w.h * a.ls[1];
+  struct Row { u32x4 r[C::NIT], o[C::NIT]; float lse; };
+  auto on = [&](int it) { return wave + C::NWAVE * it < 4 * C::WPT; };                                // wave-uniform
+  auto is_do = [&](int it) { return may_be_do(it) && wave + C::NWAVE * it >= 3 * C::WPT && on(it); };
+  auto issue = [&](int row, Row& R) __attribute__((always_inline)) {
+    const uint32_t rc = (uint32_t)dlt_imax(0, dlt_imin(row, TR - 1));   // rows outside the grid: clamped as well
+#pragma unroll
+    for (int it = 0; it < C::NIT; it++) {
+      if (on(it)) R.r[it] = *reinterpret_cast<const u32x4*>(base[it] + (goff[it] + rc * rs[it]));
+      if (may_be_do(it) && is_do(it)) R.o[it] = *reinterpret_cast<const u32x4*>(ob + (ooff[it] + rc * ors));
+    }
+    if (tid < C::TOK) R.lse = lseb[((int64_t)rc * XL + xsc) * a.ls[2]];
+  };
+  auto commit = [&](int slot, const Row& R) __attribute__((always_inline)) {
+#pragma unroll
+    for (int it = 0; it < C::NIT; it++) {
+      if (on(it)) swat_write16(lds + slot * C::SLOT + loff[it], R.r[it]);
+      if (may_be_do(it) && is_do(it)) {
+        float fo[8], fd[8], part = 0.f;
+        unpack8<CT>(R.o[it], fo);
+        unpack8<CT>(R.r[it], fd);
+#pragma unroll
+        for (int j = 0; j < 8; j++) part += fo[j] * fd[j];
+        const float del = swat_sum_pieces<C::PIECES>(part);
+        if (lane % C::PIECES == 0) scal[slot * 2 * C::TOK + C::TOK + tok_of[it]] = del;
+      }
+    }
+    if (tid < C::TOK) scal[slot * 2 * C::TOK + tid] = -R.lse;
+  };
+
+  const bool is_q = wave < C::SB;                            // this wave owns queries, else keys
+  const int blk_w = is_q ? wave : wave - C::SB;              // own block of the strip
+  const bool own = w.xs + 16 * blk_w < XL;
+  const int tile = (w.xs + 16 * blk_w) / (16 * NTB);
+  const int blk = NTB == 1 ? blk_w : blk_w / NTB * NTB;      // first staged block of the wave's window
+  const int own_blk = blk_w + WC * NTB;                      // own block among the staged ones
+  const int xw = dlt_imin(w.xs + 16 * blk_w + (lane >> 2), XL - 1);   // token of the lane's stores
+  char* out0 = is_q ? const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xw) + 16 * (lane & 3)
+                    : const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xw) + 16 * (lane & 3);
+  char* out1 = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xw) + 16 * (lane & 3);
+  const uint32_t out0rs = is_q ? swat_row_bytes(a.tm, a.dqs, XL) : swat_row_bytes(a.tm, a.dks, XL), out1rs = swat_row_bytes(a.tm, a.dvs, XL);
+  SwatLane<C> L;
+  L.init(n, g);
+  const float scale = a.scale_log2;
+
+  {
+    Row pre[C::NR];
+#pragma unroll
+    for (int i = 0; i < C::NR; i++) issue(w.r0 - WR + i, pre[i]);
+#pragma unroll
+    for (int i = 0; i < C::NR; i++) commit(i, pre[i]);
+  }
+  __syncthreads();
+
+  int slot0 = 0;   // slot of the window's first row
+  for (int r = w.r0; r < w.r1; r++) {
+    const bool more = r + 1 < w.r1;
+    Row next;
+    if (more) issue(r + 1 + WR, next);
+    SwatSeen<C, NTB> seen;
+    seen.init(a, r, tile, WC, WR);
+    swat_lds rowp[C::NR];
+    DLT_LDS float* scp[C::NR];
+#pragma unroll
+    for (int i = 0; i < C::NR; i++) {
+      const int s0 = slot0 + i, s = s0 >= C::NR ? s0 - C::NR : s0;
+      rowp[i] = lds + s * C::SLOT + blk * C::BLKB;
+      scp[i] = scal + s * 2 * C::TOK + blk * 16;
+    }
+    const int to_own = (own_blk - blk) * C::BLKB;
+    // queries: K and V stream past the own q, dO, lse2 and delta
+    auto step_q = [&](auto edge_tag) __attribute__((always_inline)) {
+      constexpr bool EDGE = decltype(edge_tag)::value;
+      u32x4 q[C::KC], d_o[C::KC];
+#pragma unroll
+      for (int c = 0; c < C::KC; c++) {
+        q[c] = swat_read16(rowp[WR] + 2 * C::TB + to_own + L.row[c]);
+        d_o[c] = swat_read16(rowp[WR] + 3 * C::TB + to_own + L.row[c]);
+      }
+      DLT_LDS float* sp = scp[WR] + (own_blk - blk) * 16 + n;
+      const float nlse = sp[0], del = sp[C::TOK];
+      f32x4 acc[C::DB];
+#pragma unroll
+      for (int d = 0; d < C::DB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < C::NP; t++) {
+        float ds[8];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const int b = 2 * t + u;
+          if (b >= C::NB) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) ds[4 * u + i] = 0.f;
+            continue;
+          }
+          swat_lds kp = rowp[b / C::NWB] + (b % C::NWB) * C::BLKB;
+          // the dP products start from -delta: the matrix pipe delivers dP - delta
+          f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {-del, -del, -del, -del};
+#pragma unroll
+          for (int c = 0; c < C::KC; c++) {
+            s = Mma<CT>::mfma(swat_read16(kp + L.row[c]), q[c], s);
+            dp = Mma<CT>::mfma(swat_read16(kp + C::TB + L.row[c]), d_o[c], dp);
+          }
+          if (EDGE && !seen.sees(b / C::NWB, b % C::NWB)) s = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+          for (int i = 0; i < 4; i++) ds[4 * u + i] = fast_exp2(fmaf(s[i], scale, nlse)) * dp[i];
+        }
+        const u32x4 dsb = pack8<CT>(ds);
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        swat_lds k0 = rowp[b0 / C::NWB] + (b0 % C::NWB) * C::BLKB, k1 = rowp[b1 / C::NWB] + (b1 % C::NWB) * C::BLKB;
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(k0 + L.tr[d]), hi = swat_read_tr(k1 + L.tr[d]);
+          acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
+        }
+      }
+      swat_store_row<CT, C::DB>(out0 + (uint32_t)r * out0rs, acc, a.sm_scale, lane);
+    };
+    // keys: Q, dO, lse2 and delta stream past the own k and v (the window is symmetric)
+    auto step_kv = [&](auto edge_tag) __attribute__((always_inline)) {
+      constexpr bool EDGE = decltype(edge_tag)::value;
+      // the own values are negated and the dP products start from delta: the matrix pipe delivers -(dP - delta)
+      u32x4 k[C::KC], v[C::KC];
+#pragma unroll
+      for (int c = 0; c < C::KC; c++) {
+        k[c] = swat_read16(rowp[WR] + to_own + L.row[c]);
+        v[c] = swat_read16(rowp[WR] + C::TB + to_own + L.row[c]);
+        v[c].x ^= 0x80008000u; v[c].y ^= 0x80008000u; v[c].z ^= 0x80008000u; v[c].w ^= 0x80008000u;
+      }
+      f32x4 acc_k[C::DB], acc_v[C::DB];
+#pragma unroll
+      for (int d = 0; d < C::DB; d++) acc_k[d] = acc_v[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < C::NP; t++) {
+        float p[8], ds[8];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const int b = 2 * t + u;
+          if (b >= C::NB) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[4 * u + i] = ds[4 * u + i] = 0.f;
+            continue;
+          }
+          swat_lds qp = rowp[b / C::NWB] + 2 * C::TB + (b % C::NWB) * C::BLKB;
+          DLT_LDS float* sp = scp[b / C::NWB] + (b % C::NWB) * 16 + 4 * g;
+          const f32x4 nl = *reinterpret_cast<DLT_LDS f32x4*>(sp);
+          f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = *reinterpret_cast<DLT_LDS f32x4*>(sp + C::TOK);
+#pragma unroll
+          for (int c = 0; c < C::KC; c++) {
+            s = Mma<CT>::mfma(swat_read16(qp + L.row[c]), k[c], s);
+            dp = Mma<CT>::mfma(swat_read16(qp + C::TB + L.row[c]), v[c], dp);
+          }
+          if (EDGE && !seen.sees(b / C::NWB, b % C::NWB)) s = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const float pv = fast_exp2(fmaf(s[i], scale, nl[i]));
+            p[4 * u + i] = pv;
+            ds[4 * u + i] = -pv * dp[i];
+          }
+        }
+        const u32x4 pb = pack8<CT>(p), dsb = pack8<CT>(ds);
+        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        swat_lds q0 = rowp[b0 / C::NWB] + 2 * C::TB + (b0 % C::NWB) * C::BLKB, q1 = rowp[b1 / C::NWB] + 2 * C::TB + (b1 % C::NWB) * C::BLKB;
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(q0 + C::TB + L.tr[d]), hi = swat_read_tr(q1 + C::TB + L.tr[d]);
+          acc_v[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc_v[d]);
+        }
+#pragma unroll
+        for (int d = 0; d < C::DB; d++) {
+          const u32x2 lo = swat_read_tr(q0 + L.tr[d]), hi = swat_read_tr(q1 + L.tr[d]);
+          acc_k[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc_k[d]);
+        }
+        // 128 registers a lane: reads hoisted across pairs of blocks spilled the pieces in flight, a wait for them at the step's start
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      swat_store_row<CT, C::DB>(out1 + (uint32_t)r * out1rs, acc_v, 1.f, lane);
+      swat_store_row<CT, C::DB>(out0 + (uint32_t)r * out0rs, acc_k, a.sm_scale, lane);
+    };
+    if (own) {
+      if (is_q) {
+        if (seen.all()) step_q(std::false_type{});
+        else step_q(std::true_type{});
+      } else {
+        if (seen.all()) step_kv(std::false_type{});
+        else step_kv(std::true_type{});
+      }
+    }
+    if (more) {
+      __syncthreads();
+      commit(slot0, next);   // the row that left the window
       __syncthreads();
       slot0 = slot0 + 1 == C::NR ? 0 : slot0 + 1;
     }

@@ -124,3 +124,24 @@ def test_marching_tile_windows(th, tw, B, S, WR, WC, d, image):
     assert (o.float().cpu() - lay(o_w)).abs().max().item() <= FWD_TOL
     errs = (_rel(qg.grad, lay(dq_w)), _rel(kg.grad, lay(dk_w)), _rel(vg.grad, lay(dv_w)))
     assert max(errs) <= GRAD_TOL, errs
+
+
+# the one-launch backward pass (16-token tiles, 3 x 3 window) stages K, V, Q and dO side by side and o behind them: strips of 128
+# (d = 32) and 64 (d = 64) tokens with one block left over, every tensor with strides of its own, same bits as contiguous tensors
+@pytest.mark.parametrize("th,tw,d", [(3, 9, 32), (2, 5, 64), (21, 8, 32)])
+def test_one_launch_backward_takes_each_tensors_own_strides(th, tw, d):
+    sw = _swa()
+    B, H, S = 2, 3, 16
+    N = th * tw * S
+    q, k, v, do = (t.cuda() for t in orc.make_qkv(N + d, B, H, N, N, d, d, torch.bfloat16))
+    as_bnhd = lambda t: t.transpose(1, 2).contiguous().transpose(1, 2)
+    padded = lambda t: torch.cat([t, t[..., :8]], dim=-1)[..., :d]
+    spaced = lambda t: torch.stack([t, t], dim=2)[:, :, 0]
+
+    def grads(q, k, v, do):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        return torch.autograd.grad(sw.TiledSwa.apply(*leaves, S, th, tw, 1, 1, 0.2), leaves, do)
+
+    want = grads(q, k, v, do)
+    got = grads(as_bnhd(q), padded(k), spaced(v), as_bnhd(padded(do)))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
