@@ -60,33 +60,49 @@ DLT_DEV u32x4 flashd_read_tr(Swa2Lds tile, const FlashDLane<D>& L, int d) {
 // Copy of one chunk of CK tokens of a [token][D] tensor by the NW waves of a workgroup: wave w copies tokens
 // w CK / NW .. + CK / NW - 1 in NI instructions; instruction i, lane l writes LDS slot l of its 1 KB = physical piece
 // l % PIECES of token w CK / NW + TPI i + l / PIECES, and therefore fetches the logical piece (l % PIECES) ^ (SWZ (token & 7)).
+// The lane's offsets inside a chunk are kept in registers and a chunk's place is a scalar base: formed per copy (clamp, multiply,
+// swizzle) the addresses were 20 to 40 vector instructions a chunk where the arithmetic takes 96 to 192, in kernels that are
+// bound by the issue port.
 template <int D, int CK, int NW = 4>
 struct FlashDStage {
   typedef FlashDRow<D> R;
   static constexpr int NI = CK / NW / R::TPI;
   static_assert(NI >= 1 && NI * R::TPI * NW == CK, "chunk must split evenly over the waves' copy instructions");
-  int tok0;      // token of the lane in instruction 0
-  int lp;        // physical piece the lane writes
-  int npieces;   // 16-byte pieces a row of the tensor really has (head dim / 8 <= PIECES)
+  static constexpr int NOFF = D == 64 || NI == 1 ? 1 : 2;   // instructions i and i + NOFF lie a multiple of 8 tokens apart: same swizzle
+  uint32_t off[NOFF]; // byte offset of the lane's piece inside a full chunk in instructions 0 .. NOFF - 1
+  int tok0;           // token of the lane in instruction 0
+  int lp;             // physical piece the lane writes
+  int npieces;        // 16-byte pieces a row of the tensor really has (head dim / 8 <= PIECES)
+  int sn2;            // bytes between tokens
 
-  DLT_DEV void init(int wave, int lane, int dact) {
+  DLT_DEV uint32_t piece(int i) const { return (uint32_t)(lp ^ (R::SWZ * ((tok0 + R::TPI * i) & 7))); }
+  DLT_DEV void init(int wave, int lane, int dact, int sn2_) {
     tok0 = wave * (CK / NW) + lane / R::PIECES;
     lp = lane % R::PIECES;
     npieces = dact >> 3;
+    sn2 = sn2_;
+#pragma unroll
+    for (int i = 0; i < NOFF; i++) off[i] = (uint32_t)(tok0 + R::TPI * i) * (uint32_t)sn2 + 16u * piece(i);   // used for full chunks only
   }
   // tokens past the end of the chunk are clamped onto its last token (the caller masks them).  With a head dim below
   // the padded one the lanes of the missing pieces copy nothing: their LDS slots were zeroed once (flashd_zero_pads) and
   // no copy ever writes them (PAD: a compile-time flag of the kernels, the test costs the exact-dim kernels 1.5 %).  Every
   // instruction still has active lanes, so the count of copies in flight is the same.
-  template <bool PAD, typename AD>
-  DLT_DEV void issue(const char* base, const AD& ad, const FlashChunk& c, char* region, int wave) const {
+  template <bool PAD>
+  DLT_DEV void issue(const char* base, const FlashChunk& c, char* region, int wave) const {
+    const char* cb = base + (uint32_t)(c.tok0 * sn2);             // wave-uniform
+    char* dst = region + wave * (CK / NW) * R::ROW;
+    if (c.nvalid >= CK) {
 #pragma unroll
-    for (int i = 0; i < NI; i++) {
-      const int t = tok0 + R::TPI * i;
-      const int lgp = lp ^ (R::SWZ * (t & 7));
-      const uint32_t off = ad(c, dlt_imin(t, c.nvalid - 1)) + 16u * (uint32_t)lgp;
-      char* dst = region + (wave * (CK / NW) + R::TPI * i) * R::ROW;   // wave-uniform
-      if (!PAD || lgp < npieces) dlt_copy16_to_lds(base, off, dst);
+      for (int i = 0; i < NI; i++)
+        if (!PAD || (int)piece(i) < npieces)
+          dlt_copy16_to_lds(cb + (uint32_t)(i / NOFF * NOFF * R::TPI * sn2), off[i % NOFF], dst + R::TPI * i * R::ROW);
+    } else {
+      keep_branch();
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+        if (!PAD || (int)piece(i) < npieces)
+          dlt_copy16_to_lds(cb, (uint32_t)(dlt_imin(tok0 + R::TPI * i, c.nvalid - 1) * sn2) + 16u * piece(i), dst + R::TPI * i * R::ROW);
     }
   }
 };
@@ -108,8 +124,8 @@ template <int CK>
 DLT_DEV void flashd_issue_scalars(const float* base, int stride, const FlashChunk& c, char* dst, int lane) {
 #pragma unroll
   for (int j = 0; j < CK / 64; j++) {
-    const uint32_t off = (uint32_t)((c.tok0 + dlt_imin(64 * j + lane, c.nvalid - 1)) * stride) * 4u;
-    dlt_copy4_to_lds(reinterpret_cast<const char*>(base), off, dst + 256 * j);
+    const uint32_t off = (uint32_t)(dlt_imin(64 * j + lane, c.nvalid - 1) * stride) * 4u;
+    dlt_copy4_to_lds(reinterpret_cast<const char*>(base) + (uint32_t)(c.tok0 * stride) * 4u, off, dst + 256 * j);
   }
 }
 
@@ -141,6 +157,11 @@ constexpr int flashd_bufs(int dk, int dv, int np, int nw) {
   return nw == 4 ? flashd_nbuf(dk, dv) : np == 2 || dk + dv > 192 ? 2 : dk + dv > 128 ? 3 : 4;
 }
 constexpr int flashd_occ(int nw) { return nw == 4 ? 2 : 1; }   // waves per SIMD the register allocation aims for
+
+// dQ at 64/128: with two buffers and 168 registers three workgroups share a CU (with three buffers two do; 16 + 16 slabs of 4096 x 8192:
+// 1441 -> 1433 us for the whole step); at 64/64 three do with three buffers
+constexpr int flashd_dq_occ(int dk, int dv, int nw) { return nw == 4 && dk + dv <= 192 ? 3 : flashd_occ(nw); }
+constexpr int flashd_dq_bufs(int dk, int dv, int np, int nw) { return nw == 4 && dk + dv > 128 ? 2 : flashd_bufs(dk, dv, np, nw); }
 
 template <int DK, int DV, int CK>
 struct FlashDBuf {
@@ -177,7 +198,6 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   const char* dob = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1]);
   const float* lseb = a.lse + b * a.ls[0] + h * a.ls[1];
   const float* delb = a.delta + b * a.ls[0] + h * a.ls[1];
-  const FlashAddr<false> aq = flash_addr<false>(a.qs, a.tm), ad = flash_addr<false>(a.dos, a.tm);
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
@@ -186,13 +206,13 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
 
   FlashDStage<DK, CK, NW> stq;
   FlashDStage<DV, CK, NW> std_;
-  stq.init(wave, lane, a.dk_);
-  std_.init(wave, lane, a.dv_);
+  stq.init(wave, lane, a.dk_, (int)a.qs[2] * 2);
+  std_.init(wave, lane, a.dv_, (int)a.dos[2] * 2);
   // waves 0 and 1 also copy the chunk's lse2 / delta
   const float* scal_base = wave == 0 ? lseb : delb;
   auto issue = [&](const FlashChunk& c, char* buf) {
-    stq.template issue<PAD>(qb, aq, c, buf, wave);
-    std_.template issue<PAD>(dob, ad, c, buf + B::REG_A, wave);
+    stq.template issue<PAD>(qb, c, buf, wave);
+    std_.template issue<PAD>(dob, c, buf + B::REG_A, wave);
     if (wave < 2) flashd_issue_scalars<CK>(scal_base, (int)a.ls[2], c, buf + B::REG_A + B::REG_B + wave * (CK * 4), lane);
   };
   constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
@@ -372,12 +392,26 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
       bi = bi + 1 == NBUF ? 0 : bi + 1;
     }
   }
-  for (; ci + AHEAD < W.nchunks; ci++) {
+  auto plain_round = [&]() __attribute__((always_inline)) {
     consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
     flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();   // chunk ci + 1 has landed: all copies but those of the AHEAD - 1 chunks behind it
     __syncthreads();
     bi = bi + 1 == NBUF ? 0 : bi + 1;
-  }
+    ci++;
+  };
+  // NBUF rounds at a time: the buffers' places are immediates of the LDS reads then (as run-time values they cost an addition per
+  // lane offset and chunk).  Two own blocks at 64/128 have no register left for it (20 would be spilled)
+  constexpr bool UNROLL = DK + DV <= 128 || NP == 1;
+  while (CAUSAL && UNROLL && ci + AHEAD < W.nchunks && bi != 0) plain_round();
+  while (UNROLL && ci + AHEAD + NBUF - 1 < W.nchunks)
+    swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
+      constexpr int BI = decltype(bc)::value;
+      consume_t(ci, (Swa2Lds)smem + BI * B::BUF_KV, smem + (BI + AHEAD) % NBUF * B::BUF_KV, std::false_type{}, std::true_type{});
+      flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
+      __syncthreads();
+      ci++;
+    });
+  while (ci + AHEAD < W.nchunks) plain_round();
   // without a mask a full last chunk runs here too (same test-free body): the code below, whose per-pair tests cost
   // registers the compiler finds by spilling, is then not executed at all
   const int n_plain = (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
@@ -431,7 +465,6 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
   const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
   TIO* ob = reinterpret_cast<TIO*>(a.o) + b * a.os[0] + h * a.os[1];
-  const FlashAddr<false> ak = flash_addr<false>(a.ks, a.tm), av = flash_addr<false>(a.vs, a.tm);
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
@@ -439,8 +472,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
 
   FlashDStage<DK, CK, NW> stk;
   FlashDStage<DV, CK, NW> stv;
-  stk.init(wave, lane, a.dk);
-  stv.init(wave, lane, a.dv);
+  stk.init(wave, lane, a.dk, (int)a.ks[2] * 2);
+  stv.init(wave, lane, a.dv, (int)a.vs[2] * 2);
   // head dims below the padded ones: the slots of the missing pieces are zeroed once, no copy writes them
 #pragma unroll
   for (int i = 0; PAD && i < NBUF; i++) {
@@ -448,8 +481,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     flashd_zero_pads<DV>(smem + i * B::BUF + B::REG_A, CK, a.dv >> 3, tid, 64 * NW);
   }
   auto issue = [&](const FlashChunk& c, char* buf) {
-    stk.template issue<PAD>(kb_, ak, c, buf, wave);
-    stv.template issue<PAD>(vb_, av, c, buf + B::REG_A, wave);
+    stk.template issue<PAD>(kb_, c, buf, wave);
+    stv.template issue<PAD>(vb_, c, buf + B::REG_A, wave);
   };
 #pragma unroll
   for (int i = 0; i < AHEAD; i++)
@@ -580,16 +613,31 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   };
   int ci = 0, bi = 0;
   auto buf_of = [&](int i) { return smem + (i >= NBUF ? i - NBUF : i) * B::BUF; };
+  // the first `n` chunks, as far as whole groups of NBUF rounds go: the buffers' places are immediates of the LDS reads (see
+  // flashd_bwd_kv_kernel).  64/64: -2.5 %, dense and causal; with 128-key chunks +1 % (64/128) and +3.5 % (128/128)
+  auto unrolled = [&](const int n) __attribute__((always_inline)) {
+    while (DK + DV <= 128 && ci + NBUF - 1 < n)
+      swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
+        constexpr int BI = decltype(bc)::value;
+        consume_t(ci, (Swa2Lds)smem + BI * B::BUF, smem + (BI + AHEAD) % NBUF * B::BUF, std::false_type{}, std::true_type{});
+        flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
+        __syncthreads();
+        ci++;
+      });
+  };
   if constexpr (CAUSAL) {
     // the chunks below the first query of the workgroup: every wave sees every pair, the body holds no test (as without
     // a mask); the chunks on the diagonal follow with the per-chunk and per-pair tests
     const int nfull = dlt_imin(x0, W.len) / CK;
+    unrolled(dlt_imin(W.nchunks - AHEAD, nfull));
     for (; ci + AHEAD < W.nchunks && ci < nfull; ci++) {
       consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
       flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
       __syncthreads();
       bi = bi + 1 == NBUF ? 0 : bi + 1;
     }
+  } else {
+    unrolled(W.nchunks - AHEAD);
   }
   for (; ci + AHEAD < W.nchunks; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::true_type{});
@@ -638,7 +686,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
 // delta pre-pass (:186-202).  Per 32-key block: per 16-key half KC pieces of K (S = K Q^T) and VC pieces of V
 // (dP = V dO^T), then KB transposed pieces of K (dQ^T += K^T dS).
 template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
-__global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
+__global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
@@ -646,7 +694,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(c
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
   constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16, NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
-  constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
+  constexpr int NBUF = flashd_dq_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;
 
   const int tid = threadIdx.x;
@@ -663,7 +711,6 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(c
   const TIO* dob = reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1];
   const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
   const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
-  const FlashAddr<false> ak = flash_addr<false>(a.ks, a.tm), av = flash_addr<false>(a.vs, a.tm);
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
@@ -671,8 +718,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(c
 
   FlashDStage<DK, CK, NW> stk;
   FlashDStage<DV, CK, NW> stv;
-  stk.init(wave, lane, a.dk_);
-  stv.init(wave, lane, a.dv_);
+  stk.init(wave, lane, a.dk_, (int)a.ks[2] * 2);
+  stv.init(wave, lane, a.dv_, (int)a.vs[2] * 2);
   // head dims below the padded ones: the slots of the missing pieces are zeroed once, no copy writes them
 #pragma unroll
   for (int i = 0; PAD && i < NBUF; i++) {
@@ -680,8 +727,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(c
     flashd_zero_pads<DV>(smem + i * B::BUF + B::REG_A, CK, a.dv_ >> 3, tid, 64 * NW);
   }
   auto issue = [&](const FlashChunk& c, char* buf) {
-    stk.template issue<PAD>(kb_, ak, c, buf, wave);
-    stv.template issue<PAD>(vb_, av, c, buf + B::REG_A, wave);
+    stk.template issue<PAD>(kb_, c, buf, wave);
+    stv.template issue<PAD>(vb_, c, buf + B::REG_A, wave);
   };
 #pragma unroll
   for (int i = 0; i < AHEAD; i++)
@@ -814,16 +861,31 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_q_kernel(c
   };
   int ci = 0, bi = 0;
   auto buf_of = [&](int i) { return smem + (i >= NBUF ? i - NBUF : i) * B::BUF; };
+  // the first `n` chunks, as far as whole groups of NBUF rounds go: the buffers' places are immediates of the LDS reads (see
+  // flashd_bwd_kv_kernel)
+  auto unrolled = [&](const int n) __attribute__((always_inline)) {
+    while (ci + NBUF - 1 < n)
+      swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
+        constexpr int BI = decltype(bc)::value;
+        consume_t(ci, (Swa2Lds)smem + BI * B::BUF, smem + (BI + AHEAD) % NBUF * B::BUF, std::false_type{}, std::true_type{});
+        flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
+        __syncthreads();
+        ci++;
+      });
+  };
   if constexpr (CAUSAL) {
     // the chunks below the first query of the workgroup: every wave sees every pair, the body holds no test (as without
     // a mask); the chunks on the diagonal follow with the per-chunk and per-pair tests
     const int nfull = dlt_imin(x0, W.len) / CK;
+    unrolled(dlt_imin(W.nchunks - AHEAD, nfull));
     for (; ci + AHEAD < W.nchunks && ci < nfull; ci++) {
       consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
       flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
       __syncthreads();
       bi = bi + 1 == NBUF ? 0 : bi + 1;
     }
+  } else {
+    unrolled(W.nchunks - AHEAD);
   }
   for (; ci + AHEAD < W.nchunks; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::true_type{});

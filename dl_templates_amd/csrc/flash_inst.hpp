@@ -93,7 +93,7 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
                                                    : flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DK * 2 + 16);
-  constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
+  constexpr int bufs = flashd_dq_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
   constexpr int lds = bufs > tile ? bufs : tile;
   const int rc = flash_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;
