@@ -531,7 +531,8 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
 
 // Which kernels a dense / causal pass runs on:
 //   CHUNKED: the streamed side passes through LDS chunk by chunk, 32 own tokens per wave (64 ... 256 per workgroup);
-//   SLIM:    the same with 8 waves of 16 own tokens: half the work per wave and chunk, twice the workgroups;
+//   SLIM:    the same with 16 own tokens per wave: half the work per wave and chunk.  Forward 8 waves (twice the workgroups of 64/128 and
+//            128/128), backward 4 (twice the workgroups);
 //   SPLIT1, SPLIT2: the streamed side is split over the waves of workgroups that own one or two blocks of 16 tokens
 //            (csrc/flash_split_kernel.hpp).
 // CHUNKED wins once its workgroups fill the chip.  Below that the time of a chunked pass is a start and the chunks of 64 streamed
@@ -573,7 +574,8 @@ int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, i
   const auto wgs = [&](int n) { return (float)(bh * ((own + n - 1) / n)); };
   const auto may = [&](int kind) { return (kinds >> kind & 1u) != 0; };
   const float chunks = (float)((other + 63) / 64);
-  const bool spills = pass == 2 && causal && dc.id == 2;   // two own blocks per wave: dK/dV at 64/128 under a mask
+  // two own blocks per wave: dK/dV at 64/128 under a mask (for passes 1 and 2 the choice here is between splitting and not: flash_pick)
+  const bool spills = pass == 2 && causal && dc.id == 2;
   int best = -1;
   float least = 0.f;
   const auto consider = [&](int kind, float t) {
@@ -613,6 +615,16 @@ unsigned flash_same_bits(int pass, const DimClass& dc, int kind) {
 int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
   int order = flash_fastest(pass, dc, dims, FLASH_SLABS, own, other, causal, FLASH_ALL);
   if (pass == 0 && (dc.id == 1 || dc.id == 2) && order != FLASH_SPLIT1 && order != FLASH_SPLIT2) order = own < FLASH_SLIM_BELOW ? FLASH_SLIM : FLASH_CHUNKED;
+  if (pass > 0 && order != FLASH_SPLIT1 && order != FLASH_SPLIT2) {
+    // Backward passes that do not split the other side: 64 own tokens per workgroup instead of 128 (one block per wave) while they all run at
+    // once, one per CU, or two under a mask, where the work is uneven.  8 slabs of 2048 x 2048, dQ and dK/dV: 64/64 32.3 -> 25.0 and 39.2 ->
+    // 30.0 us, 64/128 37.7 -> 28.5 and 50.5 -> 38.4, dQ at 128/128 52.0 -> 39.3; causal, 16 slabs: 35.4 -> 31.1 and 43.5 -> 39.3, 40.2 ->
+    // 35.3 and 67.0 -> 50.3, 53.0 -> 45.4.  12 slabs without a mask (384 workgroups): the same or slower.  The same bits.
+    // dK/dV at 64/128 under a mask below 3072 keys always: two blocks per wave spill there (64 slabs of 2048: 160 -> 138; 32 of 4096: 232 ->
+    // 249).
+    const bool fits = bh * ((own + 63) / 64) <= (causal ? 2 : 1) * (int64_t)dlt_device_cus();
+    return fits || (pass == 2 && causal && dc.id == 2 && own < FLASH_SLIM_BELOW) ? FLASH_SLIM : FLASH_CHUNKED;
+  }
   return flash_fastest(pass, dc, dims, bh, own, other, causal, flash_same_bits(pass, dc, order));
 }
 
@@ -713,6 +725,9 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
   const int np_q = seq ? flash_pick(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0) : 0;
   const int np_kv = seq ? flash_pick(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0) : 0;
   a.slim = np_kv == FLASH_SLIM;
+  // dQ with one workgroup of 128 queries per CU: 8 waves of one block (16 slabs of 2048 x 2048: 64/64 36.6 -> 34.6 us, 64/128 43.8 -> 41.0,
+  // 128/128 58.0 -> 54.2; from two workgroups per CU on slower, 32 slabs 54.8 -> 56.0, 70.4 -> 70.5, 94.9 -> 108.5)
+  a.slim_q = np_q == FLASH_SLIM ? 4 : seq && nbh * ((a.Lq + 127) / 128) <= dlt_device_cus() ? 8 : 0;
   int rc;
 #define DLT_FLASH_PASS(C)                                                                                                  \
   rc = np_q == FLASH_SPLIT1 || np_q == FLASH_SPLIT2 ? dlt_flashs_bwd_q_##C(a, p.dtype, np_q, stream) : dlt_flash_launch_bwd_q_##C(a, p.dtype, (int)grid_q, stream); \

@@ -128,6 +128,9 @@ template <typename TIO, int MODE>
 int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && flash_async_staging()) {
+      // few workgroups: one own block per wave, in 4 waves (twice the workgroups) or 8 (see flash_pick)
+      if (a.slim_q == 4) return flashd_launch_bwd_q<TIO, MODE, 1, 4>(a, stream);
+      if (a.slim_q == 8) return flashd_launch_bwd_q<TIO, MODE, 1, 8>(a, stream);
       return flashd_launch_bwd_q<TIO, MODE, FLASHD_DQ_NP(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }
@@ -148,9 +151,7 @@ int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream
     // where whole blocks are skipped, the register-staged kernel measured 1.5 % faster)
     const bool scalars_fit = a.ls[2] >= 0 && ((int64_t)a.Lq - 1) * a.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1);   // 32-bit offsets of the lse2 / delta copies
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && scalars_fit && flash_async_staging()) {
-      // under a causal mask two own blocks per wave spill at 64/128
-      if constexpr (MODE == 1 && DLT_DK == 64 && DLT_DV == 128)
-        if (a.slim) return flashd_launch_bwd_kv<TIO, MODE, 1, 8>(a, stream);
+      if (a.slim) return flashd_launch_bwd_kv<TIO, MODE, 1, 4>(a, stream);
       return flashd_launch_bwd_kv<TIO, MODE, flash_np_kv(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }

@@ -522,7 +522,8 @@ struct FlashBwdArgs {
   int32_t B, H, Lq, Lk, dk_, dv_;
   int32_t nblk_q, nblk_k;
   int32_t causal, causal_group;   // causal_group: see flash_block_causal
-  int32_t slim;                   // host only: dK/dV on 8 waves of one own block each
+  int32_t slim;                   // host only: dK/dV on 4 waves of one own block each
+  int32_t slim_q;                 // host only: dQ on this many waves of one own block each (0: two blocks on 4 waves)
   int32_t tile;
   DltGeom g;
   int32_t dq_vec, dk_vec, dv_vec;

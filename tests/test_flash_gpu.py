@@ -364,3 +364,19 @@ def test_a_slab_has_the_same_bits_in_any_call(causal, Lq, Lk, dk, dv, counts):
     for a, b in zip(runs[-2], runs[-1]):
         n = counts[-2]
         assert torch.equal(a[:, -n:], b[:, -n:])
+
+
+# backward passes with one own block per wave: 4 waves while their workgroups of 64 fit the chip, dQ on 8 waves while its workgroups of 128 do,
+# two blocks per wave beyond: a token past a workgroup's end, chunk remainders, every class and dims below it, counts on every side of the lines
+@pytest.mark.parametrize("causal,Lq,Lk,dk,dv,counts", [
+    (False, 1025, 1090, 64, 64, (1, 20, 40)), (False, 1090, 1025, 64, 128, (1, 20, 40)), (False, 1100, 1153, 128, 128, (1, 20, 40)),
+    (False, 1030, 1100, 80, 72, (1, 20, 40)), (True, 1090, 1090, 64, 64, (1, 35)), (True, 1090, 1090, 64, 128, (1, 40)),
+    (True, 1121, 1121, 128, 128, (1, 35)), (True, 3100, 3100, 64, 128, (1, 12))])
+def test_one_own_block_per_wave_backward(causal, Lq, Lk, dk, dv, counts):
+    scale = 1 / math.sqrt(dk)
+    q, k, v, do = orc.make_qkv(Lq + Lk + dk, 1, 1, Lq, Lk, dk, dv, torch.bfloat16)
+    want = orc.flash_grads(q.float(), k.float(), v.float(), do.float(), causal, scale)[1:]
+    qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    got = torch.autograd.grad(_fa().attention(qg, kg, vg, causal, scale), (qg, kg, vg), do.cuda())
+    assert max(_rel(g, w) for g, w in zip(got, want)) <= 5e-2
+    test_a_slab_has_the_same_bits_in_any_call(causal, Lq, Lk, dk, dv, counts)
