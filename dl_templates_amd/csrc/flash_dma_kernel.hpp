@@ -60,10 +60,13 @@ DLT_DEV u32x4 flashd_read_tr(Swa2Lds tile, const FlashDLane<D>& L, int d) {
 // Copy of one chunk of CK tokens of a [token][D] tensor by the NW waves of a workgroup: wave w copies tokens
 // w CK / NW .. + CK / NW - 1 in NI instructions; instruction i, lane l writes LDS slot l of its 1 KB = physical piece
 // l % PIECES of token w CK / NW + TPI i + l / PIECES, and therefore fetches the logical piece (l % PIECES) ^ (SWZ (token & 7)).
-// The lane's offsets inside a chunk are kept in registers and a chunk's place is a scalar base: formed per copy (clamp, multiply,
-// swizzle) the addresses were 20 to 40 vector instructions a chunk where the arithmetic takes 96 to 192, in kernels that are
-// bound by the issue port.
-template <int D, int CK, int NW = 4>
+// SB: a full chunk's place is a scalar base and the lane's offset inside it stays in registers.  Formed per copy (clamp, multiply,
+// swizzle) the addresses are 20 to 40 vector instructions a chunk where the arithmetic takes 96 to 192, in kernels bound by the
+// issue port.  Worth it in the forward (64/64 causal, 128 slabs of 4096: 355 -> 346 us) and in dQ at 64/128 and 128/128 (16 + 16
+// slabs of 4096 x 8192: 453 -> 447 us).  dQ at 64/64 and dK/dV hide the vector form behind their products and lose by the scalar
+// chain and the branch: 128 causal slabs of 1024, dQ 39.4 against 41.7 us, dK/dV 49.3 against 50.0; 8 of 2048, dK/dV 29.7 against
+// 30.8.  With 8 waves on 64-token chunks (one or two copies a wave) the branch costs what the addresses do.
+template <int D, int CK, int NW = 4, bool SB = true>
 struct FlashDStage {
   typedef FlashDRow<D> R;
   static constexpr int NI = CK / NW / R::TPI;
@@ -90,19 +93,24 @@ struct FlashDStage {
   // instruction still has active lanes, so the count of copies in flight is the same.
   template <bool PAD>
   DLT_DEV void issue(const char* base, const FlashChunk& c, char* region, int wave) const {
-    const char* cb = base + (uint32_t)(c.tok0 * sn2);             // wave-uniform
     char* dst = region + wave * (CK / NW) * R::ROW;
-    if (c.nvalid >= CK) {
+    auto clamped = [&](int i) __attribute__((always_inline)) {
+      if (!PAD || (int)piece(i) < npieces)
+        dlt_copy16_to_lds(base, (uint32_t)((c.tok0 + dlt_imin(tok0 + R::TPI * i, c.nvalid - 1)) * sn2) + 16u * piece(i), dst + R::TPI * i * R::ROW);
+    };
+    if constexpr (!SB || CK / NW < 16) {
+#pragma unroll
+      for (int i = 0; i < NI; i++) clamped(i);
+    } else if (c.nvalid >= CK) {
+      const char* cb = base + (uint32_t)(c.tok0 * sn2);   // wave-uniform
 #pragma unroll
       for (int i = 0; i < NI; i++)
         if (!PAD || (int)piece(i) < npieces)
           dlt_copy16_to_lds(cb + (uint32_t)(i / NOFF * NOFF * R::TPI * sn2), off[i % NOFF], dst + R::TPI * i * R::ROW);
     } else {
       keep_branch();
-#pragma unroll
-      for (int i = 0; i < NI; i++)
-        if (!PAD || (int)piece(i) < npieces)
-          dlt_copy16_to_lds(cb, (uint32_t)(dlt_imin(tok0 + R::TPI * i, c.nvalid - 1) * sn2) + 16u * piece(i), dst + R::TPI * i * R::ROW);
+#pragma unroll 1   // rare: kept small (cold code in front of the first products cost short calls 0.4 us)
+      for (int i = 0; i < NI; i++) clamped(i);
     }
   }
 };
@@ -204,8 +212,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   W.init_seq(CAUSAL ? (x0 / CK) * CK : 0, a.Lq);
   const int wk0 = x0 + wave * 16 * NP;  // first own key of this wave
 
-  FlashDStage<DK, CK, NW> stq;
-  FlashDStage<DV, CK, NW> std_;
+  FlashDStage<DK, CK, NW, false> stq;
+  FlashDStage<DV, CK, NW, false> std_;
   stq.init(wave, lane, a.dk_, (int)a.qs[2] * 2);
   std_.init(wave, lane, a.dv_, (int)a.dos[2] * 2);
   // waves 0 and 1 also copy the chunk's lse2 / delta
@@ -223,7 +231,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     flashd_zero_pads<DK>(smem + i * B::BUF_KV, CK, a.dk_ >> 3, tid, 64 * NW);
     flashd_zero_pads<DV>(smem + i * B::BUF_KV + B::REG_A, CK, a.dv_ >> 3, tid, 64 * NW);
   }
-#pragma unroll
+#pragma unroll 1
   for (int i = 0; i < AHEAD; i++)
     if (i < W.nchunks) issue(W.at(i), smem + i * B::BUF_KV);
 
@@ -484,7 +492,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     stk.template issue<PAD>(kb_, c, buf, wave);
     stv.template issue<PAD>(vb_, c, buf + B::REG_A, wave);
   };
-#pragma unroll
+#pragma unroll 1
   for (int i = 0; i < AHEAD; i++)
     if (i < W.nchunks) issue(W.at(i), smem + i * B::BUF);
 
@@ -614,9 +622,10 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   int ci = 0, bi = 0;
   auto buf_of = [&](int i) { return smem + (i >= NBUF ? i - NBUF : i) * B::BUF; };
   // the first `n` chunks, as far as whole groups of NBUF rounds go: the buffers' places are immediates of the LDS reads (see
-  // flashd_bwd_kv_kernel).  64/64: -2.5 %, dense and causal; with 128-key chunks +1 % (64/128) and +3.5 % (128/128)
+  // flashd_bwd_kv_kernel).  64/64: -2.5 %, dense and causal; with 128-key chunks +1 % (64/128) and +3.5 % (128/128); with one own
+  // block per wave the calls are too short for it (447 x 447 causal +4 %)
   auto unrolled = [&](const int n) __attribute__((always_inline)) {
-    while (DK + DV <= 128 && ci + NBUF - 1 < n)
+    while (DK + DV <= 128 && NP == 2 && ci + NBUF - 1 < n)
       swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
         constexpr int BI = decltype(bc)::value;
         consume_t(ci, (Swa2Lds)smem + BI * B::BUF, smem + (BI + AHEAD) % NBUF * B::BUF, std::false_type{}, std::true_type{});
@@ -716,8 +725,8 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   FlashWalk<MODE, CK> W;
   W.init_seq(0, CAUSAL ? dlt_imin(a.Lk, x0 + OWN) : a.Lk);
 
-  FlashDStage<DK, CK, NW> stk;
-  FlashDStage<DV, CK, NW> stv;
+  FlashDStage<DK, CK, NW, (DK + DV > 128)> stk;
+  FlashDStage<DV, CK, NW, (DK + DV > 128)> stv;
   stk.init(wave, lane, a.dk_, (int)a.ks[2] * 2);
   stv.init(wave, lane, a.dv_, (int)a.vs[2] * 2);
   // head dims below the padded ones: the slots of the missing pieces are zeroed once, no copy writes them
@@ -730,7 +739,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
     stk.template issue<PAD>(kb_, c, buf, wave);
     stv.template issue<PAD>(vb_, c, buf + B::REG_A, wave);
   };
-#pragma unroll
+#pragma unroll 1
   for (int i = 0; i < AHEAD; i++)
     if (i < W.nchunks) issue(W.at(i), smem + i * B::BUF);
 
