@@ -348,6 +348,21 @@ struct SwagFrame {
   DLT_DEV int own_tok(int rp) const { return dlt_imin(own_row(rp), TR - 1) * TC + dlt_imin(col, TC - 1); }
 };
 
+// Own rows leave straight from the accumulators: a lane of the C layout holds 4 dims of its token in each 16-dim block; the
+// lane swap of two blocks gives every lane 8 consecutive dims (16 bytes), four lanes a whole 64-byte piece.  p: row of the lane's token.
+template <typename CT, int DB>
+DLT_DEV void swag_store_row(char* p, const f32x4 (&acc)[DB], float mul, int g) {
+  typedef unsigned pair_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int d = 0; d < DB; d += 2) {
+    const pair_t lo = __builtin_amdgcn_permlane16_swap(pack2<CT>(acc[d][0] * mul, acc[d][1] * mul), pack2<CT>(acc[d + 1][0] * mul, acc[d + 1][1] * mul),
+                                                       false, false);
+    const pair_t hi = __builtin_amdgcn_permlane16_swap(pack2<CT>(acc[d][2] * mul, acc[d][3] * mul), pack2<CT>(acc[d + 1][2] * mul, acc[d + 1][3] * mul),
+                                                       false, false);
+    store_stream16(p + 2 * (16 * d + 16 * (g & 1) + 8 * (g >> 1)), u32x4{lo.x, hi.x, lo.y, hi.y});
+  }
+}
+
 // scores of block (i, j) on top of `bias`
 template <typename C, typename CT>
 DLT_DEV f32x4 swag_scores(swat_lds blk, const SwagLane<C>& L, const u32x4 (&own)[C::KC], float bias) {
@@ -543,7 +558,7 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ke
       any_bad |= __builtin_amdgcn_ballot_w64(l != l);
       if (F.own_ok(rp)) {
         const int tok = F.own_tok(rp);
-        swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+        swag_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
         if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
       }
     }
@@ -582,7 +597,7 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC)) void swag_fwd_ke
       });
       if (F.own_ok(rp)) {
         const int tok = F.own_tok(rp);
-        swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+        swag_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
         if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
       }
     }
@@ -680,7 +695,7 @@ __global__ __launch_bounds__(512, 2) void swag_fwd_rope_kernel(const SwagArgs a)
   auto store = [&](int rp, const f32x4 (&acc)[C::DB], float l, float m_use) {
     if (F.own_ok(rp)) {
       const int tok = F.own_tok(rp);
-      swat_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
+      swag_store_row<CT, C::DB>(ob + (uint32_t)(tok * osn), acc, fast_rcp(l), g);
       if (g == 0) store_stream4(lseb + tok * a.ls[2], m_use * scale + fast_log2(l));
     }
   };
@@ -893,7 +908,7 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC_BWD)) void swag_bw
         }
       }
       if constexpr (ROPE) swag_turn_back<CT>(acc, a.sm_scale, tr, rot, g);
-      if (ok) swat_store_row<CT, C::DB>(dqb + (uint32_t)(F.own_tok(rp) * dqsn), acc, ROPE ? 1.f : a.sm_scale, g);
+      if (ok) swag_store_row<CT, C::DB>(dqb + (uint32_t)(F.own_tok(rp) * dqsn), acc, ROPE ? 1.f : a.sm_scale, g);
     }
     if (more) {
       __syncthreads();
@@ -1053,8 +1068,8 @@ __global__ __launch_bounds__(512, (Swag<D, NCH, NCG, PC>::OCC_BWD)) void swag_bw
       if constexpr (ROPE) swag_turn_back<CT>(acc_k, a.sm_scale, tr, rot, g);
       if (F.own_ok(rp)) {
         const int tok = F.own_tok(rp);
-        swat_store_row<CT, C::DB>(dvb + (uint32_t)(tok * dvsn), acc_v, 1.f, g);
-        swat_store_row<CT, C::DB>(dkb + (uint32_t)(tok * dksn), acc_k, ROPE ? 1.f : a.sm_scale, g);
+        swag_store_row<CT, C::DB>(dvb + (uint32_t)(tok * dvsn), acc_v, 1.f, g);
+        swag_store_row<CT, C::DB>(dkb + (uint32_t)(tok * dksn), acc_k, ROPE ? 1.f : a.sm_scale, g);
       }
     }
     if (more) {
