@@ -9,10 +9,11 @@ template <typename TIO, int NTB, int WC, int WR>
 int swat_launch_fwd(const SwatArgs& a, int grid, hipStream_t stream) {
   typedef Swat<DLT_D, NTB, WC, WR> C;
   auto kern = swat_fwd_kernel<TIO, DLT_D, NTB, WC, WR>;
-  const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), C::RING);
+  const int lds = a.lone ? dlt_imax(C::RING, 81 * 1024) : C::RING;   // more than half of a CU's: a second workgroup does not fit
+  const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), lds);
   if (rc != DLT_OK) return rc;
   dlt_timing_before(DLT_K_FWD, stream);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(SWAT_THREADS), C::RING, stream, a);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(SWAT_THREADS), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("marching tile-window forward launch");
   return DLT_OK;

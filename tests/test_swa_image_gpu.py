@@ -149,3 +149,24 @@ def test_image_layout_with_fused_rotation():
     errs = (_rel(dq, to_img(dq_w)), _rel(dk, to_img(dk_w)), _rel(dv, to_img(dv_w)))
     assert max(errs) <= GRAD_TOL, errs
     del keep
+
+
+@pytest.mark.parametrize("B,th,tw", [
+    (32, 3, 8),     # 256 column strips: one workgroup per CU, one full round
+    (56, 2, 5),     # 448 strips: the second round just full enough, ragged strips
+    (55, 2, 5),     # 440: two workgroups per CU
+    (32, 9, 11),    # 512 strips, two per row, the second ragged
+])
+def test_image_forward_with_one_workgroup_per_cu(B, th, tw):
+    """A tile's output does not depend on how the strips are split into bands or placed on CUs: bit-equal to the token layout."""
+    sw = _swa()
+    H, d, S = 8, 32, 16
+    q, k, v, _ = orc.make_qkv(B + th, B, H, th * tw * S, th * tw * S, d, d, torch.float16)
+    scale = 1 / math.sqrt(d)
+    qi, ki, vi = (orc.tokens_to_image(t, th, tw, 4, 4).contiguous().cuda() for t in (q, k, v))
+    got = sw.TiledSwaImage.apply(qi, ki, vi, 4, 4, 1, 1, scale).cpu()
+    want = sw.TiledSwa.apply(q.cuda(), k.cuda(), v.cuda(), S, th, tw, 1, 1, scale).cpu()
+    assert torch.equal(got, orc.tokens_to_image(want, th, tw, 4, 4))
+    sub = slice(B - 1, B)
+    o_w, _, _, _ = orc.tiled_swa_grads(q[sub].float(), k[sub].float(), v[sub].float(), v[sub].float(), S, th, tw, 1, 1, scale)
+    assert (want[sub].float() - o_w).abs().max() <= FWD_TOL
