@@ -91,7 +91,7 @@ struct FlashDStage {
   // the padded one the lanes of the missing pieces copy nothing: their LDS slots were zeroed once (flashd_zero_pads) and
   // no copy ever writes them (PAD: a compile-time flag of the kernels, the test costs the exact-dim kernels 1.5 %).  Every
   // instruction still has active lanes, so the count of copies in flight is the same.
-  template <bool PAD>
+  template <int PAD>
   DLT_DEV void issue(const char* base, const FlashChunk& c, char* region, int wave) const {
     char* dst = region + wave * (CK / NW) * R::ROW;
     auto clamped = [&](int i) __attribute__((always_inline)) {
@@ -180,15 +180,24 @@ struct FlashDBuf {
   static constexpr int BUF_KV = REG_A + REG_B + SCAL;  // dK/dV
 };
 
+// Head dims the products run over.  PAD 0: the class's own; 1: any below them, the products run over the zeroed pieces too; 2: at
+// most 96 of 128, the last 32 dims are left out of every product, operand read and accumulator (their terms are zeros).  These
+// kernels are bound by the issue port and LDS reads, of which that is a quarter at 128/128 and a sixth to an eighth at 64/128.
+// Variant 1 -> 2, forward and backward: 32 slabs of 4096 at 80/80 231 -> 209 and 777 -> 675 us, causal 190 -> 168 and 508 -> 439;
+// 32 of 3000 at 96/96 157 -> 139 and 442 -> 383; 32 of 4096 at 64/96 202 -> 192 and 550 -> 514; 8 of 2048 at 80/80 38.1 -> 34.3 and
+// 81.4 -> 72.1; 64 causal of 700 at 80/80 23.0 -> 21.0 and 66.4 -> 59.6.  Variant 1 stays for 104 to 120 dims (and at 64/64).
+constexpr int flashd_dims(int d, int pad) { return pad == 2 && d == 128 ? 96 : d; }
+
 // ---- dK / dV: own = keys; Q, dO, lse2 and delta stream.  Replaces _attn_bwd_dkdv (src/flash_attn.py:204-307).
-template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
+template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
 __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
   constexpr bool CAUSAL = MODE == 1;
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
-  constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16, VB = DV / 16, NQB = CK / 32;
+  constexpr int AK = flashd_dims(DK, PAD), AV = flashd_dims(DV, PAD);
+  constexpr int KC = AK / 32, VC = AV / 32, KB = AK / 16, VB = AV / 16, NQB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
 
   const int tid = threadIdx.x;
@@ -242,8 +251,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     const int xk = wk0 + 16 * p + n;
     const int64_t tk = xk < a.Lk ? (int64_t)xk : (int64_t)-1;
     qmin[p] = CAUSAL ? xk : 0;
-    swa1_load_own<TIO, CT, DK>(kf[p], kb_, 1, a.dk_, flash_own_off<false>(a.ks, a.tm, tk), g, no_rope, false);
-    swa1_load_own<TIO, CT, DV>(vf[p], vb_, 1, a.dv_, flash_own_off<false>(a.vs, a.tm, tk), g, no_rope, false);
+    swa1_load_own<TIO, CT, AK>(kf[p], kb_, 1, a.dk_, flash_own_off<false>(a.ks, a.tm, tk), g, no_rope, false);
+    swa1_load_own<TIO, CT, AV>(vf[p], vb_, 1, a.dv_, flash_own_off<false>(a.vs, a.tm, tk), g, no_rope, false);
   }
   f32x4 dk_acc[NP][KB], dv_acc[NP][VB];
 #pragma unroll
@@ -445,7 +454,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
 // Per chunk: S^T = K Q^T for every 32-key block (a stream of NKB 2 KC operand reads, NP products each), one softmax
 // update per query block, then O^T += V^T P^T (NKB VB transposed operands) with the row sums from a ones-row product.
 // The reads of the second stream are already in flight while the softmax runs.
-template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
+template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
 __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(const FlashArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef typename TileOf<TIO>::type TL;
@@ -454,7 +463,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   constexpr bool CAUSAL = MODE == 1;
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
   constexpr int PO = DV * (int)sizeof(TL) + 16;
-  constexpr int KC = DK / 32, VB = DV / 16, NKB = CK / 32;
+  constexpr int AK = flashd_dims(DK, PAD);
+  constexpr int KC = AK / 32, VB = flashd_dims(DV, PAD) / 16, NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
   constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;
@@ -504,7 +514,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     const int xq = wq0 + 16 * p + n;
     tq[p] = xq < a.Lq ? (int64_t)xq : (int64_t)-1;
     klim[p] = CAUSAL ? dlt_imin(xq, a.Lk - 1) : a.Lk - 1;
-    swa1_load_own<TIO, CT, DK>(qf[p], qb, 1, a.dk, flash_own_off<false>(a.qs, a.tm, tq[p]), g, no_rope, false);
+    swa1_load_own<TIO, CT, AK>(qf[p], qb, 1, a.dk, flash_own_off<false>(a.qs, a.tm, tq[p]), g, no_rope, false);
   }
   float m_run[NP];
   f32x4 acc[NP][VB], acc_l[NP];
@@ -694,14 +704,15 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
 // ---- dQ: own = queries; K and V stream.  Replaces _attn_bwd_dq (src/flash_attn.py:310-449) and, with fuse_delta, the
 // delta pre-pass (:186-202).  Per 32-key block: per 16-key half KC pieces of K (S = K Q^T) and VC pieces of V
 // (dP = V dO^T), then KB transposed pieces of K (dQ^T += K^T dS).
-template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, bool PAD>
+template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
 __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
   constexpr bool CAUSAL = MODE == 1;
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
-  constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16, NKB = CK / 32;
+  constexpr int AK = flashd_dims(DK, PAD), AV = flashd_dims(DV, PAD);
+  constexpr int KC = AK / 32, VC = AV / 32, KB = AK / 16, NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
   constexpr int NBUF = flashd_dq_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;
@@ -751,14 +762,14 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
     const int xq = wq0 + 16 * p + n;
     const int64_t tq = xq < a.Lq ? (int64_t)xq : (int64_t)-1;
     klim[p] = CAUSAL ? dlt_imin(xq, a.Lk - 1) : a.Lk - 1;
-    swa1_load_own<TIO, CT, DK>(qf[p], qb, 1, a.dk_, flash_own_off<false>(a.qs, a.tm, tq), g, no_rope, false);
-    swa1_load_own<TIO, CT, DV>(dof[p], dob, 1, a.dv_, flash_own_off<false>(a.dos, a.tm, tq), g, no_rope, false);
+    swa1_load_own<TIO, CT, AK>(qf[p], qb, 1, a.dk_, flash_own_off<false>(a.qs, a.tm, tq), g, no_rope, false);
+    swa1_load_own<TIO, CT, AV>(dof[p], dob, 1, a.dv_, flash_own_off<false>(a.dos, a.tm, tq), g, no_rope, false);
     const int64_t off = b * a.ls[0] + h * a.ls[1] + (tq >= 0 ? tq : 0) * a.ls[2];
     nlse[p] = tq >= 0 ? -a.lse[off] : 0.f;
     if (a.fuse_delta != 0) {
       const TIO* ob = reinterpret_cast<const TIO*>(a.o) + b * a.os[0] + h * a.os[1];
       u32x4 of[VC];
-      swa1_load_own<TIO, CT, DV>(of, ob, 1, a.dv_, flash_own_off<false>(a.os, a.tm, tq), g, no_rope, false);
+      swa1_load_own<TIO, CT, AV>(of, ob, 1, a.dv_, flash_own_off<false>(a.os, a.tm, tq), g, no_rope, false);
       float part = 0.f;
 #pragma unroll
       for (int c_ = 0; c_ < VC; c_++) {

@@ -35,14 +35,24 @@ inline bool flash_async_staging() {
   return on;
 }
 
+// PAD of the asynchronously staged kernels for head dims dk, dv: 2 where the class's 128 dims hold 96 at most (both sides measured
+// at flashd_dims)
+inline int flashd_pad(int dk, int dv) {
+  if (dk == DLT_DK && dv == DLT_DV) return 0;
+  return DLT_DV == 128 && dv <= 96 && (DLT_DK == 64 || dk <= 96) ? 2 : 1;
+}
+
 template <typename KernT>
 int flash_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
 template <typename TIO, int MODE, int NP, int CK, int NW>
 int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
-  auto kern = (a.dk != DLT_DK || a.dv != DLT_DV) ? flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
-                                                 : flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
+  const int pad = flashd_pad(a.dk, a.dv);
+  auto kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
+  if (pad == 1) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+  if constexpr (DLT_DV == 128)
+    if (pad == 2) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DV * 2 + 16);
   constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
@@ -89,8 +99,11 @@ int flash_launch_fwd_t(const FlashArgs& a, int grid, hipStream_t stream) {
 template <typename TIO, int MODE, int NP, int NW>
 int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
-  auto kern = (a.dk_ != DLT_DK || a.dv_ != DLT_DV) ? flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
-                                                   : flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
+  const int pad = flashd_pad(a.dk_, a.dv_);
+  auto kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
+  if (pad == 1) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+  if constexpr (DLT_DV == 128)
+    if (pad == 2) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DK * 2 + 16);
   constexpr int bufs = flashd_dq_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
@@ -108,8 +121,11 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
 template <typename TIO, int MODE, int NP, int NW>
 int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
-  auto kern = (a.dk_ != DLT_DK || a.dv_ != DLT_DV) ? flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, true>
-                                                   : flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, false>;
+  const int pad = flashd_pad(a.dk_, a.dv_);
+  auto kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
+  if (pad == 1) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+  if constexpr (DLT_DV == 128)
+    if (pad == 2) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
   constexpr int own = 16 * NP * NW;
   constexpr int tile_k = own * (DLT_DK * 2 + 16), tile_v = own * (DLT_DV * 2 + 16);
   constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF_KV;

@@ -575,9 +575,9 @@ struct PairStage {
   }
 };
 
-// accumulators (C layout, [dim][own token]) of NP blocks -> LDS tile -> HBM rows
-template <typename TIO, int D, int NP, typename SN>
-DLT_DEV void flash_write_grad(char* sT, f32x4 (&acc)[NP][D / 16], float mul, TIO* base, const SN& sn, int64_t sd, int dact,
+// accumulators (C layout, [dim][own token]) of NP blocks -> LDS tile -> HBM rows (NA: 16-dim blocks held, dact <= 16 NA)
+template <typename TIO, int D, int NP, int NA, typename SN>
+DLT_DEV void flash_write_grad(char* sT, f32x4 (&acc)[NP][NA], float mul, TIO* base, const SN& sn, int64_t sd, int dact,
                               bool vec, int own_base, int x0, int len, int wave, int n, int g, int tid, int nrows = 64 * NP) {
   typedef typename TileOf<TIO>::type TL;
   constexpr int PT = D * (int)sizeof(TL) + 16;
@@ -586,7 +586,7 @@ DLT_DEV void flash_write_grad(char* sT, f32x4 (&acc)[NP][D / 16], float mul, TIO
   for (int p = 0; p < NP; p++) {
     TL* row = reinterpret_cast<TL*>(sT + (wave * 16 * NP + 16 * p + n) * PT);
 #pragma unroll
-    for (int d = 0; d < D / 16; d++)
+    for (int d = 0; d < NA; d++)
 #pragma unroll
       for (int i = 0; i < 4; i++) row[16 * d + 4 * g + i] = (TL)(acc[p][d][i] * mul);
   }
