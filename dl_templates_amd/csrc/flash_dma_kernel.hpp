@@ -181,12 +181,16 @@ struct FlashDBuf {
 };
 
 // Head dims the products run over.  PAD 0: the class's own; 1: any below them, the products run over the zeroed pieces too; 2: at
-// most 96 of 128, the last 32 dims are left out of every product, operand read and accumulator (their terms are zeros).  These
-// kernels are bound by the issue port and LDS reads, of which that is a quarter at 128/128 and a sixth to an eighth at 64/128.
-// Variant 1 -> 2, forward and backward: 32 slabs of 4096 at 80/80 231 -> 209 and 777 -> 675 us, causal 190 -> 168 and 508 -> 439;
-// 32 of 3000 at 96/96 157 -> 139 and 442 -> 383; 32 of 4096 at 64/96 202 -> 192 and 550 -> 514; 8 of 2048 at 80/80 38.1 -> 34.3 and
-// 81.4 -> 72.1; 64 causal of 700 at 80/80 23.0 -> 21.0 and 66.4 -> 59.6.  Variant 1 stays for 104 to 120 dims (and at 64/64).
-constexpr int flashd_dims(int d, int pad) { return pad == 2 && d == 128 ? 96 : d; }
+// most 96 of 128, the last 32 dims are left out of every product, operand read and accumulator (their terms are zeros); 3: at most 80,
+// the transposed products (O, dQ, dK, dV) leave out 48.  These kernels are bound by the issue port and LDS reads, of which that is a
+// quarter (2) or 5 / 16 (3) at 128/128, a sixth to a quarter at 64/128.  Variant 1 -> 2, forward and backward: 32 slabs of 3000 at 96/96
+// 157 -> 139 and 442 -> 383 us; 32 of 4096 at 64/96 202 -> 192 and 550 -> 514.  1 -> 2 -> 3: 32 of 4096 at 80/80 231 -> 208 -> 202 and
+// 777 -> 664 -> 644, causal 190 -> 170 -> 164 and 508 -> 432 -> 418; 8 of 2048 38.1 -> 34.3 -> 32.8 and 81.4 -> 71.9 -> 69.0; 64
+// causal of 700 23.0 -> 21.2 -> 20.8 and 66.4 -> 59.9 -> 57.5; 8 of 2048 at 64/80 33.7 -> 31.1 -> 30.5 and 65.6 -> 61.5 -> 60.9.
+// Variant 1 stays for 104 to 120 dims (and at 64/64).
+constexpr int flashd_dims(int d, int pad) { return pad >= 2 && d == 128 ? 96 : d; }
+// 16-dim blocks of the transposed products and of their accumulators
+constexpr int flashd_blocks(int d, int pad) { return pad == 3 && d == 128 ? 5 : flashd_dims(d, pad) / 16; }
 
 // ---- dK / dV: own = keys; Q, dO, lse2 and delta stream.  Replaces _attn_bwd_dkdv (src/flash_attn.py:204-307).
 template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   constexpr bool CAUSAL = MODE == 1;
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
   constexpr int AK = flashd_dims(DK, PAD), AV = flashd_dims(DV, PAD);
-  constexpr int KC = AK / 32, VC = AV / 32, KB = AK / 16, VB = AV / 16, NQB = CK / 32;
+  constexpr int KC = AK / 32, VC = AV / 32, KB = flashd_blocks(DK, PAD), VB = flashd_blocks(DV, PAD), NQB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
 
   const int tid = threadIdx.x;
@@ -464,7 +468,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
   constexpr int PO = DV * (int)sizeof(TL) + 16;
   constexpr int AK = flashd_dims(DK, PAD);
-  constexpr int KC = AK / 32, VB = flashd_dims(DV, PAD) / 16, NKB = CK / 32;
+  constexpr int KC = AK / 32, VB = flashd_blocks(DV, PAD), NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
   constexpr int NBUF = flashd_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;
@@ -712,7 +716,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   constexpr bool CAUSAL = MODE == 1;
   static_assert(MODE < 2, "asynchronous staging: dense and causal only");
   constexpr int AK = flashd_dims(DK, PAD), AV = flashd_dims(DV, PAD);
-  constexpr int KC = AK / 32, VC = AV / 32, KB = AK / 16, NKB = CK / 32;
+  constexpr int KC = AK / 32, VC = AV / 32, KB = flashd_blocks(DK, PAD), NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
   constexpr int NBUF = flashd_dq_bufs(DK, DV, NP, NW), AHEAD = NBUF - 1;
   constexpr int PER_CHUNK = FlashDStage<DK, CK, NW>::NI + FlashDStage<DV, CK, NW>::NI;

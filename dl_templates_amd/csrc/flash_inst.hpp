@@ -35,11 +35,12 @@ inline bool flash_async_staging() {
   return on;
 }
 
-// PAD of the asynchronously staged kernels for head dims dk, dv: 2 where the class's 128 dims hold 96 at most (both sides measured
-// at flashd_dims)
+// PAD of the asynchronously staged kernels for head dims dk, dv: 2 where the class's 128 dims hold 96 at most, 3 where they hold 80
+// (all sides measured at flashd_dims)
 inline int flashd_pad(int dk, int dv) {
   if (dk == DLT_DK && dv == DLT_DV) return 0;
-  return DLT_DV == 128 && dv <= 96 && (DLT_DK == 64 || dk <= 96) ? 2 : 1;
+  const int d = DLT_DV < 128 || dv > 96 || (DLT_DK > 64 && dk > 96) ? 128 : DLT_DK > 64 && dk > dv ? dk : dv;
+  return d > 96 ? 1 : d > 80 ? 2 : 3;
 }
 
 template <typename KernT>
@@ -51,8 +52,10 @@ int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   const int pad = flashd_pad(a.dk, a.dv);
   auto kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
   if (pad == 1) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
-  if constexpr (DLT_DV == 128)
+  if constexpr (DLT_DV == 128) {
     if (pad == 2) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
+    if (pad == 3) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
+  }
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DV * 2 + 16);
   constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
@@ -102,8 +105,10 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   const int pad = flashd_pad(a.dk_, a.dv_);
   auto kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
   if (pad == 1) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
-  if constexpr (DLT_DV == 128)
+  if constexpr (DLT_DV == 128) {
     if (pad == 2) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
+    if (pad == 3) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
+  }
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DK * 2 + 16);
   constexpr int bufs = flashd_dq_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF;
@@ -124,8 +129,10 @@ int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   const int pad = flashd_pad(a.dk_, a.dv_);
   auto kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
   if (pad == 1) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
-  if constexpr (DLT_DV == 128)
+  if constexpr (DLT_DV == 128) {
     if (pad == 2) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
+    if (pad == 3) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
+  }
   constexpr int own = 16 * NP * NW;
   constexpr int tile_k = own * (DLT_DK * 2 + 16), tile_v = own * (DLT_DV * 2 + 16);
   constexpr int bufs = flashd_bufs(DLT_DK, DLT_DV, NP, NW) * FlashDBuf<DLT_DK, DLT_DV, CK>::BUF_KV;

@@ -382,10 +382,11 @@ def test_one_own_block_per_wave_backward(causal, Lq, Lk, dk, dv, counts):
     test_a_slab_has_the_same_bits_in_any_call(causal, Lq, Lk, dk, dv, counts)
 
 
-# head dims of up to 96 in the classes of 128 run without the last 32 dims: on both sides of that line, in each tensor, with one and with
+# head dims of up to 96 and of up to 80 in the classes of 128 run without the dims beyond: on both sides of those lines, in each tensor, with one and with
 # several workgroups per CU, a token past a workgroup's and a chunk's end
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("dk,dv", [(96, 96), (72, 96), (96, 40), (104, 96), (96, 104), (64, 96), (40, 72), (64, 104)])
+@pytest.mark.parametrize("dk,dv", [(96, 96), (72, 96), (96, 40), (104, 96), (96, 104), (64, 96), (40, 72), (64, 104), (80, 80), (80, 40), (88, 80), (80, 88), (64, 80),
+                                   (64, 88)])
 def test_head_dims_of_up_to_96(dk, dv, causal):
     L, scale = 1025, 1 / math.sqrt(dk)
     q, k, v, do = orc.make_qkv(dk + dv, 1, 1, L, L, dk, dv, torch.float16)
