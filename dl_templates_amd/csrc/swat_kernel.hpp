@@ -44,6 +44,10 @@ struct Swat {
   static constexpr int RING = NR * SLOT, SCAL = NR * 2 * TOK * 4;
   // two workgroups per CU where two rings fit
   static constexpr int OCC = RING + SCAL <= 80 * 1024 ? 4 : 2;
+  // Forward rows leave in 64-byte runs (swat_store_row) where registers allow: at d = 32 five columns and 32-token tiles are held to 128 (with
+  // five rows, to arithmetic) and take 1 and 3.5 % less without.  With them: d = 64, 3 x 3, 64 slabs of 40 x 40 tiles 180 -> 174 us, five
+  // columns 214 -> 209, d = 32, five rows 138 -> 131.
+  static constexpr bool RUNS = !(D == 32 && (WC == 2 || NTB == 2));
   static_assert((TOK * PIECES) % 64 == 0, "a wave stages one tensor per vector");
   static_assert(RING + SCAL <= 160 * 1024, "the ring exceeds the LDS");
 };
@@ -172,24 +176,32 @@ struct SwatLane {
   }
 };
 
-// Own rows leave straight from the accumulators: a lane of the C layout holds 4 dims of its token in each 16-dim block; the
-// lane swap of two blocks gives every lane 8 consecutive dims (16 bytes) of token n, and the permutation behind it brings the
-// four pieces of a 64-byte run to four consecutive lanes (lane l: token l / 4, piece l % 4).  Without it the 16 lanes that the
-// memory pipe takes at a time wrote 16 bytes each into 16 rows, and the streaming stores left in parts of a sector: 1.25 to 1.3
-// times the bytes (D = 64 forward, 210 MB of o: 268 MB written; 498 MB of gradients for 403 at D = 32).
-// p: row of token lane / 4 plus 16 (lane % 4) bytes.  Blocks of 16 tokens lie inside the grid or outside as a whole.
-template <typename CT, int DB>
+// Own rows leave straight from the accumulators: a lane of the C layout holds 4 dims of its token in each 16-dim block, and the
+// lane swap of two blocks gives every lane 8 consecutive dims (16 bytes) of token n.  The 16 lanes that the memory pipe takes at a
+// time then write 16 bytes each into 16 rows, and streaming stores can leave in parts of a sector: 1.25 to 1.3 times the bytes
+// (D = 64 forward, 210 MB of o: 268 MB written; 498 MB of gradients for 403 at D = 32).  With RUNS a permutation brings the four
+// pieces of a 64-byte run to four consecutive lanes (lane l: token l / 4, piece l % 4).  That is 4 LDS permutes per 32 dims: it pays
+// where HBM is the bound (Swat::RUNS, swat_bwd_kernel) and not in the two backward launches of the larger windows and tiles, bound by
+// arithmetic: their passes take 1 to 3.5 % less without it (d = 64, 16-token tiles, five columns, 64 slabs of 40 x 40 tiles: 651 -> 629 us,
+// two registers spilled with it; d = 32, five rows, 128 slabs of 8 x 8: 35.1 -> 33.9).
+// p: row of token swat_store_tok plus swat_store_byte.  Blocks of 16 tokens lie inside the grid or outside as a whole.
+DLT_DEV int swat_store_tok(int lane, bool runs) { return runs ? lane >> 2 : lane & 15; }
+DLT_DEV int swat_store_byte(int lane, bool runs) { return runs ? 16 * (lane & 3) : 32 * ((lane >> 4) & 1) + 16 * (lane >> 5); }
+template <typename CT, int DB, bool RUNS>
 DLT_DEV void swat_store_row(char* p, const f32x4 (&acc)[DB], float mul, int lane) {
   typedef unsigned pair_t __attribute__((ext_vector_type(2)));
   const int from = 4 * ((lane >> 2) + 16 * (((lane >> 1) & 1) | ((lane & 1) << 1)));
-  auto take = [&](unsigned v) { return (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)v); };
 #pragma unroll
   for (int d = 0; d < DB; d += 2) {
     const pair_t lo = __builtin_amdgcn_permlane16_swap(pack2<CT>(acc[d][0] * mul, acc[d][1] * mul), pack2<CT>(acc[d + 1][0] * mul, acc[d + 1][1] * mul),
                                                        false, false);
     const pair_t hi = __builtin_amdgcn_permlane16_swap(pack2<CT>(acc[d][2] * mul, acc[d][3] * mul), pack2<CT>(acc[d + 1][2] * mul, acc[d + 1][3] * mul),
                                                        false, false);
-    store_stream16(p + 32 * d, u32x4{take(lo.x), take(hi.x), take(lo.y), take(hi.y)});
+    unsigned v[4] = {lo.x, hi.x, lo.y, hi.y};
+    if constexpr (RUNS)
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)v[i]);
+    store_stream16(p + 32 * d, u32x4{v[0], v[1], v[2], v[3]});
   }
 }
 
@@ -223,9 +235,9 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const bool own = w.xs + 16 * wave < XL;                     // wave-uniform: the wave has a block of the grid
   const int tile = (w.xs + 16 * wave) / (16 * NTB);
   const int blk = NTB == 1 ? wave : wave / NTB * NTB;         // first staged block of the wave's window
-  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + (lane >> 2), XL - 1);   // token of the lane's loads, of its stores
+  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + swat_store_tok(lane, C::RUNS), XL - 1);   // token of the lane's loads, of its stores
   const char* qb = swat_slab<TIO>(a.q, a.qs, w.b, w.h) + swat_slot_off(a.tm, a.qs, xc) + 16 * g;
-  char* ob = const_cast<char*>(swat_slab<TIO>(a.out_o, a.os, w.b, w.h)) + swat_slot_off(a.tm, a.os, xw) + 16 * (lane & 3);
+  char* ob = const_cast<char*>(swat_slab<TIO>(a.out_o, a.os, w.b, w.h)) + swat_slot_off(a.tm, a.os, xw) + swat_store_byte(lane, C::RUNS);
   float* lseb = a.lse + w.b * a.ls[0] + w.h * a.ls[1] + (int64_t)x * a.ls[2];
   const uint32_t qrs = swat_row_bytes(a.tm, a.qs, XL), ors = swat_row_bytes(a.tm, a.os, XL);
   SwatLane<C> L;
@@ -313,7 +325,7 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
         acc_l = Mma<CT>::mfma(ones, pb, acc_l);
       }
       const float l = acc_l[0];
-      swat_store_row<CT, C::DB>(ob + (uint32_t)r * ors, acc, fast_rcp(l), lane);
+      swat_store_row<CT, C::DB, C::RUNS>(ob + (uint32_t)r * ors, acc, fast_rcp(l), lane);
       if (g == 0) store_stream4(lseb + (int64_t)r * XL * a.ls[2], m * scale + fast_log2(l));
     };
     if (own) {
@@ -347,11 +359,11 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const bool own = w.xs + 16 * wave < XL;
   const int tile = (w.xs + 16 * wave) / (16 * NTB);
   const int blk = NTB == 1 ? wave : wave / NTB * NTB;
-  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + (lane >> 2), XL - 1);   // token of the lane's loads, of its stores
+  const int xc = dlt_imin(x, XL - 1);
   const char* qb = swat_slab<TIO>(a.q, a.qs, w.b, w.h) + swat_slot_off(a.tm, a.qs, xc) + 16 * g;
   const char* dob = swat_slab<TIO>(a.d_o, a.dos, w.b, w.h) + swat_slot_off(a.tm, a.dos, xc) + 16 * g;
   const char* ob = swat_slab<TIO>(a.o, a.os, w.b, w.h) + swat_slot_off(a.tm, a.os, xc) + 16 * g;
-  char* dqb = const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xw) + 16 * (lane & 3);
+  char* dqb = const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xc) + swat_store_byte(lane, false);
   const float* lseb = a.lse + w.b * a.ls[0] + w.h * a.ls[1] + (int64_t)xc * a.ls[2];
   float* delb = a.delta + w.b * a.ls[0] + w.h * a.ls[1] + (int64_t)xc * a.ls[2];
   const uint32_t qrs = swat_row_bytes(a.tm, a.qs, XL), dors = swat_row_bytes(a.tm, a.dos, XL), ors = swat_row_bytes(a.tm, a.os, XL),
@@ -443,7 +455,7 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
           acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
         }
       }
-      swat_store_row<CT, C::DB>(dqb + (uint32_t)r * dqrs, acc, a.sm_scale, lane);
+      if (x < XL) swat_store_row<CT, C::DB, false>(dqb + (uint32_t)r * dqrs, acc, a.sm_scale, lane);
     };
     if (own) {
       if (seen.all()) step(std::false_type{});
@@ -495,11 +507,11 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const bool own = w.xs + 16 * wave < XL;
   const int tile = (w.xs + 16 * wave) / (16 * NTB);
   const int blk = NTB == 1 ? wave : wave / NTB * NTB;
-  const int xc = dlt_imin(x, XL - 1), xw = dlt_imin(w.xs + 16 * wave + (lane >> 2), XL - 1);   // token of the lane's loads, of its stores
+  const int xc = dlt_imin(x, XL - 1);
   const char* kb = swat_slab<TIO>(a.k, a.ks, w.b, w.h) + swat_slot_off(a.tm, a.ks, xc) + 16 * g;
   const char* vb = swat_slab<TIO>(a.v, a.vs, w.b, w.h) + swat_slot_off(a.tm, a.vs, xc) + 16 * g;
-  char* dkb = const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xw) + 16 * (lane & 3);
-  char* dvb = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xw) + 16 * (lane & 3);
+  char* dkb = const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xc) + swat_store_byte(lane, false);
+  char* dvb = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xc) + swat_store_byte(lane, false);
   const uint32_t krs = swat_row_bytes(a.tm, a.ks, XL), vrs = swat_row_bytes(a.tm, a.vs, XL), dkrs = swat_row_bytes(a.tm, a.dks, XL),
                  dvrs = swat_row_bytes(a.tm, a.dvs, XL);
   SwatLane<C> L;
@@ -597,8 +609,10 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
           acc_k[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc_k[d]);
         }
       }
-      swat_store_row<CT, C::DB>(dvb + (uint32_t)r * dvrs, acc_v, 1.f, lane);
-      swat_store_row<CT, C::DB>(dkb + (uint32_t)r * dkrs, acc_k, a.sm_scale, lane);
+      if (x < XL) {
+        swat_store_row<CT, C::DB, false>(dvb + (uint32_t)r * dvrs, acc_v, 1.f, lane);
+        swat_store_row<CT, C::DB, false>(dkb + (uint32_t)r * dkrs, acc_k, a.sm_scale, lane);
+      }
     };
     if (own) {
       if (seen.all()) step(std::false_type{});
@@ -723,10 +737,10 @@ __global__ __launch_bounds__((Swab<D, NTB, WC, WR>::THREADS), (Swab<D, NTB, WC, 
   const int tile = (w.xs + 16 * blk_w) / (16 * NTB);
   const int blk = NTB == 1 ? blk_w : blk_w / NTB * NTB;      // first staged block of the wave's window
   const int own_blk = blk_w + WC * NTB;                      // own block among the staged ones
-  const int xw = dlt_imin(w.xs + 16 * blk_w + (lane >> 2), XL - 1);   // token of the lane's stores
-  char* out0 = is_q ? const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xw) + 16 * (lane & 3)
-                    : const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xw) + 16 * (lane & 3);
-  char* out1 = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xw) + 16 * (lane & 3);
+  const int xw = dlt_imin(w.xs + 16 * blk_w + swat_store_tok(lane, true), XL - 1);   // token of the lane's stores
+  char* out0 = is_q ? const_cast<char*>(swat_slab<TIO>(a.dq, a.dqs, w.b, w.h)) + swat_slot_off(a.tm, a.dqs, xw) + swat_store_byte(lane, true)
+                    : const_cast<char*>(swat_slab<TIO>(a.dk, a.dks, w.b, w.h)) + swat_slot_off(a.tm, a.dks, xw) + swat_store_byte(lane, true);
+  char* out1 = const_cast<char*>(swat_slab<TIO>(a.dv, a.dvs, w.b, w.h)) + swat_slot_off(a.tm, a.dvs, xw) + swat_store_byte(lane, true);
   const uint32_t out0rs = is_q ? swat_row_bytes(a.tm, a.dqs, XL) : swat_row_bytes(a.tm, a.dks, XL), out1rs = swat_row_bytes(a.tm, a.dvs, XL);
   SwatLane<C> L;
   L.init(n, g);
@@ -803,7 +817,7 @@ __global__ __launch_bounds__((Swab<D, NTB, WC, WR>::THREADS), (Swab<D, NTB, WC, 
           acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
         }
       }
-      swat_store_row<CT, C::DB>(out0 + (uint32_t)r * out0rs, acc, a.sm_scale, lane);
+      swat_store_row<CT, C::DB, true>(out0 + (uint32_t)r * out0rs, acc, a.sm_scale, lane);
     };
     // keys: Q, dO, lse2 and delta stream past the own k and v (the window is symmetric)
     auto step_kv = [&](auto edge_tag) __attribute__((always_inline)) {
@@ -863,8 +877,8 @@ __global__ __launch_bounds__((Swab<D, NTB, WC, WR>::THREADS), (Swab<D, NTB, WC, 
         // 128 registers a lane: reads hoisted across pairs of blocks spilled the pieces in flight, a wait for them at the step's start
         __builtin_amdgcn_sched_barrier(0);
       }
-      swat_store_row<CT, C::DB>(out1 + (uint32_t)r * out1rs, acc_v, 1.f, lane);
-      swat_store_row<CT, C::DB>(out0 + (uint32_t)r * out0rs, acc_k, a.sm_scale, lane);
+      swat_store_row<CT, C::DB, true>(out1 + (uint32_t)r * out1rs, acc_v, 1.f, lane);
+      swat_store_row<CT, C::DB, true>(out0 + (uint32_t)r * out0rs, acc_k, a.sm_scale, lane);
     };
     if (own) {
       if (is_q) {
