@@ -522,14 +522,7 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   // Rows per workgroup: a band's prologue fills the ring (the latency of its loads) and re-reads 2 WR rows.
   const int halo = 8 + 2 * p.g.WC * (p.g.S / 16), ring = (2 * p.g.WR + 1) * halo * 64 * p.dk;
   const int64_t cols = (int64_t)p.B * p.H * a.nstrips, cus = dlt_device_cus();
-  // Image layout, forward: a pixel's heads lie side by side, so the workgroups of 8 heads and more share every 128-byte line and
-  // must meet in the L2.  Two workgroups per CU drift apart and fetch 1.37 times the bytes; with one, whole strips and rounds
-  // over the CUs that are at least 7/8 full, the fetch is what has to move.  16-token tiles, d = 32, two per CU -> one: 4 x 8 slabs
-  // of 64 x 64 tiles 164 -> 142 us, of 100 x 64 247 -> 216, of 30 x 64 70 -> 68, 8 x 8 of 64 x 64 322 -> 284, 16 x 8 of 32 x 32 141 -> 139.
-  // Fewer heads share less (16 x 2 slabs of 64 x 64: 121 -> 122; 32 x 1: 109 -> 112), rounds that are not full cost more than the
-  // fetch (4 x 8 of 40 x 40: 67 -> 70; 6 x 8 of 64 x 64: 215 -> 223), 32-token tiles are bound by arithmetic (179 -> 208), as are windows
-  // of five columns (183 -> 184-188); at d = 64 and with five rows the ring leaves room for one anyway.
-  a.lone = !bwd && p.tm.img && p.dk == 32 && p.g.S == 16 && p.g.WR == 1 && p.g.WC == 1 && p.H >= 8 && cols >= cus && 8 * cols >= 7 * ((cols + cus - 1) / cus) * cus;
+  a.lone = !bwd && p.tm.img && dlt_image_fwd_alone(p.dk, p.g.S, p.g.WR, p.g.WC, p.g.TR, p.g.TC, p.H, cols, cus);
   const int64_t slots = cus * (!a.lone && ring + (2 * p.g.WR + 1) * halo * 128 <= 80 * 1024 ? 2 : 1);
   dlt_band_plan(p.g.TR, cols, slots, a.band, a.nbands);
   const int64_t grid = cols * a.nbands;

@@ -30,7 +30,7 @@ struct SwatArgs {
   int32_t B, H;
   int32_t nstrips, band, nbands;
   float scale_log2, sm_scale;
-  int32_t lone;   // forward: one workgroup per CU (see swat_run)
+  int32_t lone;   // forward: one workgroup per CU (dlt_image_fwd_alone)
 };
 
 template <int D, int NTB, int WC, int WR>

@@ -24,6 +24,9 @@ void shim_slot_pixel(unsigned bh, unsigned bw, unsigned TC, unsigned xs, unsigne
   dlt_slot_pixel(tm, xs, *i, *x);
 }
 int shim_band_plan(int units, long long cols, long long slots, int* per, int* nb) { return dlt_band_plan(units, cols, slots, *per, *nb); }
+int shim_image_fwd_alone(int d, int S, int WR, int WC, int TR, int TC, int H, long long cols, long long cus) {
+  return dlt_image_fwd_alone(d, S, WR, WC, TR, TC, H, cols, cus);
+}
 int shim_rope_row(int idx) { return dlt_rope_row(idx); }
 int shim_rope_col(int idx) { return dlt_rope_col(idx); }
 }

@@ -152,12 +152,12 @@ def test_image_layout_with_fused_rotation():
 
 
 @pytest.mark.parametrize("B,th,tw", [
-    (32, 3, 8),     # 256 column strips: one workgroup per CU, one full round
-    (56, 2, 5),     # 448 strips: the second round just full enough, ragged strips
-    (55, 2, 5),     # 440: two workgroups per CU
-    (32, 9, 11),    # 512 strips, two per row, the second ragged
+    (32, 3, 8),     # 256 column strips
+    (56, 2, 5),     # 448, ragged
+    (55, 2, 5),     # 440, ragged
+    (32, 9, 11),    # 512, two per row, the second ragged
 ])
-def test_image_forward_with_one_workgroup_per_cu(B, th, tw):
+def test_image_forward_with_many_strips(B, th, tw):
     """A tile's output does not depend on how the strips are split into bands or placed on CUs: bit-equal to the token layout."""
     sw = _swa()
     H, d, S = 8, 32, 16
@@ -170,3 +170,19 @@ def test_image_forward_with_one_workgroup_per_cu(B, th, tw):
     sub = slice(B - 1, B)
     o_w, _, _, _ = orc.tiled_swa_grads(q[sub].float(), k[sub].float(), v[sub].float(), v[sub].float(), S, th, tw, 1, 1, scale)
     assert (want[sub].float() - o_w).abs().max() <= FWD_TOL
+
+
+@pytest.mark.parametrize("B,H,th,tw", [
+    (32, 8, 64, 8),    # one workgroup per CU, one round of whole strips
+    (32, 8, 63, 8),    # a row less: two per CU
+    (60, 8, 48, 8),    # one per CU, two rounds, the second not full
+    (32, 8, 48, 9),    # ragged strips: two per CU
+])
+def test_image_forward_with_one_workgroup_per_cu(B, H, th, tw):
+    """Both sides of the lines of dlt_image_fwd_alone at 256 CUs: bit-equal to the token layout."""
+    sw = _swa()
+    gen = torch.Generator(device="cuda").manual_seed(B + tw)
+    q, k, v = (torch.randn((B, H, th * tw * 16, 32), generator=gen, device="cuda").half() for _ in range(3))
+    got = sw.TiledSwaImage.apply(*(orc.tokens_to_image(t, th, tw, 4, 4).contiguous() for t in (q, k, v)), 4, 4, 1, 1, 0.2)
+    want = sw.TiledSwa.apply(q, k, v, 16, th, tw, 1, 1, 0.2)
+    assert torch.equal(got, orc.tokens_to_image(want, th, tw, 4, 4))
