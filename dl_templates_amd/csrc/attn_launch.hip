@@ -518,13 +518,22 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   a.tm = p.tm; a.g = p.g; a.B = p.B; a.H = p.H;
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   a.sm_scale = p.sm_scale;
-  a.nstrips = (p.g.XLq + 127) / 128;
+  const int64_t cus = dlt_device_cus(), slabs = (int64_t)p.B * p.H;
+  a.one = bwd && dlt_tile_bwd_one_launch(p.dk, p.g.S, p.g.WR, p.g.WC, p.tm.img != 0, p.g.TC, slabs * p.g.TR, cus);
+  const void* const ring_p[4] = {t.k, t.v, t.q, t.d_o};
+  const int64_t* const ring_s[4] = {t.ks, t.vs, t.qs, t.dos};
+  for (int i = 0; i < 4; i++) {
+    a.ring_p[i] = ring_p[i];
+    for (int j = 0; j < 5; j++) a.ring_s[i][j] = ring_s[i][j];
+  }
+  const int strip = 16 * (!a.one ? 8 : p.dk == 32 ? Swab<32, 1, 1, 1>::SB : Swab<64, 1, 1, 1>::SB);
+  a.nstrips = (p.g.XLq + strip - 1) / strip;
+  const int64_t cols = slabs * a.nstrips;
+  a.lone = !bwd && p.tm.img && dlt_image_fwd_alone(p.dk, p.g.S, p.g.WR, p.g.WC, p.g.TR, p.g.TC, p.H, cols, cus);
   // Rows per workgroup: a band's prologue fills the ring (the latency of its loads) and re-reads 2 WR rows.
   const int halo = 8 + 2 * p.g.WC * (p.g.S / 16), ring = (2 * p.g.WR + 1) * halo * 64 * p.dk;
-  const int64_t cols = (int64_t)p.B * p.H * a.nstrips, cus = dlt_device_cus();
-  a.lone = !bwd && p.tm.img && dlt_image_fwd_alone(p.dk, p.g.S, p.g.WR, p.g.WC, p.g.TR, p.g.TC, p.H, cols, cus);
-  const int64_t slots = cus * (!a.lone && ring + (2 * p.g.WR + 1) * halo * 128 <= 80 * 1024 ? 2 : 1);
-  dlt_band_plan(p.g.TR, cols, slots, a.band, a.nbands);
+  const bool two = !a.one && !a.lone && ring + (2 * p.g.WR + 1) * halo * 128 <= 80 * 1024;   // workgroups per CU
+  dlt_band_plan(p.g.TR, cols, two ? 2 * cus : cus, a.band, a.nbands);
   const int64_t grid = cols * a.nbands;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
   return p.dk == 32 ? dlt_swat_launch_32(a, p.dtype, bwd, (int)grid, stream) : dlt_swat_launch_64(a, p.dtype, bwd, (int)grid, stream);

@@ -91,6 +91,18 @@ DLT_HD bool dlt_image_fwd_alone(int d, int S, int WR, int WC, int TR, int TC, in
   return rounds == 2 ? TR >= 48 : (rounds == 1 || rounds == 4) && TR >= 64;
 }
 
+// Backward over tiles at d = 32 / 64: whether dQ, dK and dV leave in one launch (16-token tiles, 3 x 3 window; TC tile columns, `rows` grid
+// rows of all (batch, head) slabs together).  At d = 32 a strip is 8 tiles wide and a CU holds one workgroup: on grids of a few tile
+// columns most of its 16 waves own nothing, and once a CU has some 12 rows to march the two launches, two workgroups per CU each,
+// are faster.  Token layout, 256 slabs of 24 rows, one launch -> two: 1 column 65 -> 56 us, 3 68 -> 63, 5 87 -> 78, 6 and more 87 -> 87, 9
+// 162 -> 162; 1024 slabs of 6 rows of 5 97 -> 84.  Images are bound by HBM sooner: 1 column 65 -> 57, 2 66 -> 64, 3 67 -> 66, 4 67 -> 72, 5 88 -> 91.
+// Fewer rows: 64 slabs of 6 rows, 1 ... 5 columns 10-12 against 13-15.  Where neither side wins clearly one launch stays: images of 3 columns
+// (+ 10 ... - 6 %), many slabs of 6 rows (512 of 9 columns, inputs in the caches 96 against 90, not 99 against 97).  At d = 64 strips are 4 tiles wide (256 slabs of 24 x 1: 81 against 120).
+DLT_HD bool dlt_tile_bwd_one_launch(int d, int S, int WR, int WC, bool img, int TC, int64_t rows, int64_t cus) {
+  if (S != 16 || WR != 1 || WC != 1) return false;
+  return d == 64 || TC > (img ? 2 : 5) || rows < 12 * cus;
+}
+
 // idx decode of the rotary op: row = int16(idx >> 16), col = int16(idx & 0xFFFF)
 // (src/fused_rope2d.py:41-42); an axis is rotated iff its value is >= 0 (:44-45).
 DLT_HD int dlt_rope_row(int32_t idx) { return (int)(int16_t)(idx >> 16); }

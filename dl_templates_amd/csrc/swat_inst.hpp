@@ -19,31 +19,23 @@ int swat_launch_fwd(const SwatArgs& a, int grid, hipStream_t stream) {
   return DLT_OK;
 }
 
+// dQ, dK and dV in one launch (booked as the dK/dV kernel by dlt_timing_collect)
 template <typename TIO, int NTB, int WC, int WR>
-int swat_launch_bwd(const SwatArgs& a, int grid, hipStream_t stream) {
+int swat_launch_bwd_one(const SwatArgs& a, int grid, hipStream_t stream) {
+  typedef Swab<DLT_D, NTB, WC, WR> C;
+  auto kern = swat_bwd_kernel<TIO, DLT_D, NTB, WC, WR>;
+  const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), C::LDS);
+  if (rc != DLT_OK) return rc;
+  dlt_timing_before(DLT_K_BWD_KV, stream);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(C::THREADS), C::LDS, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("marching tile-window backward launch");
+  return DLT_OK;
+}
+
+template <typename TIO, int NTB, int WC, int WR>
+int swat_launch_bwd_two(const SwatArgs& a, int grid, hipStream_t stream) {
   typedef Swat<DLT_D, NTB, WC, WR> C;
-  if constexpr (Swab<DLT_D, NTB, WC, WR>::USED) {   // one launch where HBM is the bound (figures at swat_bwd_kernel)
-    typedef Swab<DLT_D, NTB, WC, WR> CB;
-    auto kern = swat_bwd_kernel<TIO, DLT_D, NTB, WC, WR>;
-    const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), CB::LDS);
-    if (rc != DLT_OK) return rc;
-    SwatArgs b = a;
-    b.nstrips = (a.g.XLq + 16 * CB::SB - 1) / (16 * CB::SB);
-    const void* const ring_p[4] = {a.k, a.v, a.q, a.d_o};
-    const int64_t* const ring_s[4] = {a.ks, a.vs, a.qs, a.dos};
-    for (int t = 0; t < 4; t++) {
-      b.ring_p[t] = ring_p[t];
-      for (int i = 0; i < 5; i++) b.ring_s[t][i] = ring_s[t][i];
-    }
-    const int64_t cols = (int64_t)a.B * a.H * b.nstrips;
-    dlt_band_plan(a.g.TR, cols, dlt_device_cus(), b.band, b.nbands);
-    if (cols * b.nbands > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
-    dlt_timing_before(DLT_K_BWD_KV, stream);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(cols * b.nbands)), dim3(CB::THREADS), CB::LDS, stream, b);
-    dlt_timing_after(stream);
-    DLT_CHECK_LAUNCH("marching tile-window backward launch");
-    return DLT_OK;
-  } else {
   // dQ first: it produces the delta vector the dK/dV kernel consumes
   auto kq = swat_bwd_q_kernel<TIO, DLT_D, NTB, WC, WR>;
   auto kkv = swat_bwd_kv_kernel<TIO, DLT_D, NTB, WC, WR>;
@@ -59,7 +51,13 @@ int swat_launch_bwd(const SwatArgs& a, int grid, hipStream_t stream) {
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("marching tile-window dK/dV launch");
   return DLT_OK;
-  }
+}
+
+template <typename TIO, int NTB, int WC, int WR>
+int swat_launch_bwd(const SwatArgs& a, int grid, hipStream_t stream) {
+  if constexpr (!Swab<DLT_D, NTB, WC, WR>::USED) return swat_launch_bwd_two<TIO, NTB, WC, WR>(a, grid, stream);
+  else if constexpr (DLT_D == 64) return swat_launch_bwd_one<TIO, NTB, WC, WR>(a, grid, stream);   // see dlt_tile_bwd_one_launch
+  else return a.one ? swat_launch_bwd_one<TIO, NTB, WC, WR>(a, grid, stream) : swat_launch_bwd_two<TIO, NTB, WC, WR>(a, grid, stream);
 }
 
 template <typename TIO>

@@ -30,7 +30,8 @@ struct SwatArgs {
   int32_t B, H;
   int32_t nstrips, band, nbands;
   float scale_log2, sm_scale;
-  int32_t lone;   // forward: one workgroup per CU (dlt_image_fwd_alone)
+  int32_t lone;   // host only, forward: one workgroup per CU (dlt_image_fwd_alone)
+  int32_t one;    // host only, backward: swat_bwd_kernel (dlt_tile_bwd_one_launch)
 };
 
 template <int D, int NTB, int WC, int WR>
@@ -636,7 +637,8 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
 // second half key blocks; both take their own fragments, lse2 and delta from the ring, and delta is formed by the threads
 // that stage dO (they fetch the pieces of o beside it), so nothing travels between launches.  Strips of 8 blocks and 16 waves
 // at D = 32; at D = 64 the ring holds strips of 4 (8 waves).  Measured: the backward pass above 453 -> 290 us (1.18 GB, 4.1
-// TB/s); d = 64, 16 slabs of 40 x 40 tiles x 4 batches 540 -> 433.  Larger windows and 32-token tiles stay on two launches: their
+// TB/s); d = 64, 16 slabs of 40 x 40 tiles x 4 batches 540 -> 433.  Narrow grids at D = 32 (dlt_tile_bwd_one_launch), larger windows and
+// 32-token tiles stay on two launches: their
 // rows would fit at D = 32, but there the arithmetic is the bound and one workgroup per CU ties (5 columns: 164 against 166 us)
 // or loses (32-token tiles: 91 against 100).
 template <int D, int NTB, int WC, int WR>

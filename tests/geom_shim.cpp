@@ -27,6 +27,9 @@ int shim_band_plan(int units, long long cols, long long slots, int* per, int* nb
 int shim_image_fwd_alone(int d, int S, int WR, int WC, int TR, int TC, int H, long long cols, long long cus) {
   return dlt_image_fwd_alone(d, S, WR, WC, TR, TC, H, cols, cus);
 }
+int shim_tile_bwd_one_launch(int d, int S, int WR, int WC, int img, int TC, long long rows, long long cus) {
+  return dlt_tile_bwd_one_launch(d, S, WR, WC, img != 0, TC, rows, cus);
+}
 int shim_rope_row(int idx) { return dlt_rope_row(idx); }
 int shim_rope_col(int idx) { return dlt_rope_col(idx); }
 }

@@ -129,3 +129,15 @@ def test_image_forward_alone_only_where_it_is_faster(shim):
                   (16, 2, 64, 64), (8, 7, 64, 64), (3, 8, 64, 64)]:                                                        # heads, idle CUs
         assert not alone(*shape), shape
     assert not alone(4, 8, 64, 64, d=64) and not alone(4, 8, 64, 64, S=32) and not alone(4, 8, 64, 64, WC=2) and not alone(4, 8, 64, 64, WR=2)
+
+
+def test_narrow_tile_grids_take_two_backward_launches(shim):
+    """d = 32: grids of few tile columns with 12 rows and more per CU (256 CUs); everything else with a 3 x 3 window of 16-token tiles is one launch."""
+    one = lambda slabs, th, tw, img, d=32, S=16, WR=1, WC=1: bool(
+        shim.shim_tile_bwd_one_launch(d, S, WR, WC, img, tw, ctypes.c_longlong(slabs * th), ctypes.c_longlong(256)))
+    for slabs, th, tw in [(256, 24, 1), (512, 6, 3), (1024, 6, 5), (64, 64, 2)]:
+        assert not one(slabs, th, tw, 0) and one(slabs, th, tw, 1) == (tw > 2)
+        assert one(slabs, th, tw, 0, d=64)
+    for slabs, th, tw in [(64, 6, 1), (256, 11, 5), (1024, 64, 6), (4, 2000, 8)]:
+        assert one(slabs, th, tw, 0) and one(slabs, th, tw, 1)
+    assert not one(4, 16, 16, 0, S=32) and not one(4, 16, 16, 0, WC=2) and not one(4, 16, 16, 0, WR=2)

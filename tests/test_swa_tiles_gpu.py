@@ -145,3 +145,28 @@ def test_one_launch_backward_takes_each_tensors_own_strides(th, tw, d):
     want = grads(q, k, v, do)
     got = grads(as_bnhd(q), padded(k), spaced(v), as_bnhd(padded(do)))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+# narrow grids at d = 32: two backward launches from 12 rows per CU on (256 CUs), one below and from 6 tile columns on (images: 3); the same bits
+@pytest.mark.parametrize("image", [False, True])
+@pytest.mark.parametrize("tw", [1, 2, 3, 5, 6])
+def test_narrow_grids_backward(tw, image):
+    sw = _swa()
+    th, H, S, d = 13, 4, 16, 32
+    N = th * tw * S
+    q, k, v, do = orc.make_qkv(tw, 1, H, N, N, d, d, torch.float16)
+    want = orc.tiled_swa_grads(q.float(), k.float(), v.float(), do.float(), S, th, tw, 1, 1, 0.2)[1:]
+
+    def grads(B):
+        lay = (lambda t: orc.tokens_to_image(t, th, tw, 4, 4)) if image else (lambda t: t)
+        q_, k_, v_, do_ = (lay(t.cuda().repeat(B, 1, 1, 1)).contiguous() for t in (q, k, v, do))
+        leaves = [t.requires_grad_(True) for t in (q_, k_, v_)]
+        o = sw.TiledSwaImage.apply(*leaves, 4, 4, 1, 1, 0.2) if image else sw.TiledSwa.apply(*leaves, S, th, tw, 1, 1, 0.2)
+        got = torch.autograd.grad(o, leaves, do_)
+        assert all(torch.equal(g, g[:1].expand_as(g)) for g in got)
+        return [g[:1].clone() for g in got]
+
+    few, many = grads(2), grads(61)
+    assert all(torch.equal(a, b) for a, b in zip(few, many))
+    lay = (lambda t: orc.tokens_to_image(t, th, tw, 4, 4)) if image else (lambda t: t)
+    assert max(_rel(g, lay(w)) for g, w in zip(many, want)) <= GRAD_TOL
