@@ -141,3 +141,15 @@ def test_narrow_tile_grids_take_two_backward_launches(shim):
     for slabs, th, tw in [(64, 6, 1), (256, 11, 5), (1024, 64, 6), (4, 2000, 8)]:
         assert one(slabs, th, tw, 0) and one(slabs, th, tw, 1)
     assert not one(4, 16, 16, 0, S=32) and not one(4, 16, 16, 0, WC=2) and not one(4, 16, 16, 0, WR=2)
+
+
+def test_band_plan_of_the_long_band_cases(shim):
+    """tests/test_swa_tiles_gpu.py means its LONG_BANDS to march beyond the ring of 3 rows, over several strips, the last one ragged (256 CUs)."""
+    from tests.test_swa_tiles_gpu import LONG_BANDS
+    per, nb = ctypes.c_int(), ctypes.c_int()
+    for th, tw, slabs, d in LONG_BANDS:
+        strip = 8 if d == 32 else 4   # tiles
+        strips = -(-tw // strip)
+        assert shim.shim_tile_bwd_one_launch(d, 16, 1, 1, 0, tw, ctypes.c_longlong(slabs * th), ctypes.c_longlong(256)) and strips > 1 and tw % strip
+        shim.shim_band_plan(th, ctypes.c_longlong(slabs * strips), ctypes.c_longlong(256), ctypes.byref(per), ctypes.byref(nb))
+        assert per.value > 4, (th, tw, slabs, d, per.value)

@@ -170,3 +170,58 @@ def test_narrow_grids_backward(tw, image):
     assert all(torch.equal(a, b) for a, b in zip(few, many))
     lay = (lambda t: orc.tokens_to_image(t, th, tw, 4, 4)) if image else (lambda t: t)
     assert max(_rel(g, lay(w)) for g, w in zip(many, want)) <= GRAD_TOL
+
+
+# the one-launch backward pass over bands longer than its ring of 3 rows (tests/test_geom_cpu.py checks the plan of these shapes at 256 CUs): several
+# strips, the last one ragged.  th, tw, slabs, d
+LONG_BANDS = [(11, 9, 100, 64), (11, 9, 130, 32), (23, 17, 40, 64), (23, 12, 64, 32)]
+
+
+@pytest.mark.parametrize("th,tw,slabs,d", LONG_BANDS)
+@pytest.mark.parametrize("image", [False, True])
+def test_one_launch_backward_over_long_bands(th, tw, slabs, d, image):
+    sw = _swa()
+    S, H = 16, 2
+    gen = torch.Generator(device="cuda").manual_seed(th + tw + d)
+    q, k, v, do = (torch.randn((slabs // H, H, th * tw * S, d), generator=gen, device="cuda").bfloat16() for _ in range(4))
+    lay = (lambda t: orc.tokens_to_image(t, th, tw, 4, 4).contiguous()) if image else (lambda t: t)
+    leaves = [lay(t).requires_grad_(True) for t in (q, k, v)]
+    o = sw.TiledSwaImage.apply(*leaves, 4, 4, 1, 1, 0.2) if image else sw.TiledSwa.apply(*leaves, S, th, tw, 1, 1, 0.2)
+    got = (o,) + torch.autograd.grad(o, leaves, lay(do))
+    for b in (0, slabs // H - 1):
+        one = slice(b, b + 1)
+        want = orc.tiled_swa_grads(*(t[one, :1].float().cpu() for t in (q, k, v, do)), S, th, tw, 1, 1, 0.2)
+        mine = [g[one, ..., :1, :] if image else g[one, :1] for g in got]
+        assert (mine[0].float().cpu() - lay(want[0])).abs().max().item() <= FWD_TOL
+        errs = [_rel(g, lay(w)) for g, w in zip(mine[1:], want[1:])]
+        assert max(errs) <= GRAD_TOL, errs
+
+
+# infinite and NaN tiles reach the tiles that see them (and, through a query, that query's other keys) and no others, bit for bit: the
+# rows and columns outside the grid that the ring stages in their place are tiles of the window
+@pytest.mark.parametrize("d,th,tw,B", [(32, 7, 9, 1), (64, 7, 9, 1), (32, 13, 3, 122)])
+@pytest.mark.parametrize("which", ["q", "k", "v", "do"])
+def test_infinite_and_nan_tiles_stay_in_their_windows(d, th, tw, B, which):
+    sw = _swa()
+    S, H = 16, 2
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    base = dict(zip(("q", "k", "v", "do"), (torch.randn((B, H, th * tw * S, d), generator=gen, device="cuda").half() for _ in range(4))))
+
+    def grads(t):
+        leaves = [t[n].clone().requires_grad_(True) for n in ("q", "k", "v")]
+        return torch.autograd.grad(sw.TiledSwa.apply(*leaves, S, th, tw, 1, 1, 0.2), leaves, t["do"])
+
+    clean = grads(base)
+    assert all(torch.isfinite(g).all() for g in clean)
+    # how far a tile's values reach in dq, dk and dv (tiles; -1: not at all): dv holds probabilities and dO only
+    reach = {"q": (0, 1, 1), "k": (1, 2, 2), "v": (1, 2, -1), "do": (0, 1, 1)}[which]
+    for r, c in ((th // 2, tw // 2), (0, 0), (th - 1, tw - 1), (0, tw - 1)):
+        for value in (float("inf"), float("-inf"), float("nan")):
+            bad = dict(base, **{which: base[which].clone()})
+            at = ((r * tw + c) * S + 5, (r * tw + c) * S + 11)
+            bad[which][..., at[0], 3] = value
+            bad[which][..., at[1], d - 1] = value
+            rows, cols = torch.meshgrid(torch.arange(th), torch.arange(tw), indexing="ij")
+            far = torch.maximum((rows - r).abs(), (cols - c).abs()).reshape(-1).repeat_interleave(S).cuda()
+            for g, w, n in zip(grads(bad), clean, reach):
+                assert torch.equal(g[:, :, far > n], w[:, :, far > n]), (r, c, value)
