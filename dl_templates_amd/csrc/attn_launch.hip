@@ -625,16 +625,8 @@ unsigned flash_same_bits(int pass, const DimClass& dc, int kind) {
 int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal) {
   int order = flash_fastest(pass, dc, dims, FLASH_SLABS, own, other, causal, FLASH_ALL);
   if (pass == 0 && (dc.id == 1 || dc.id == 2) && order != FLASH_SPLIT1 && order != FLASH_SPLIT2) order = own < FLASH_SLIM_BELOW ? FLASH_SLIM : FLASH_CHUNKED;
-  if (pass > 0 && order != FLASH_SPLIT1 && order != FLASH_SPLIT2) {
-    // Backward passes that do not split the other side: 64 own tokens per workgroup instead of 128 (one block per wave) while they all run at
-    // once, one per CU, or two under a mask, where the work is uneven.  8 slabs of 2048 x 2048, dQ and dK/dV: 64/64 32.3 -> 25.0 and 39.2 ->
-    // 30.0 us, 64/128 37.7 -> 28.5 and 50.5 -> 38.4, dQ at 128/128 52.0 -> 39.3; causal, 16 slabs: 35.4 -> 31.1 and 43.5 -> 39.3, 40.2 ->
-    // 35.3 and 67.0 -> 50.3, 53.0 -> 45.4.  12 slabs without a mask (384 workgroups): the same or slower.  The same bits.
-    // dK/dV at 64/128 under a mask below 3072 keys always: two blocks per wave spill there (64 slabs of 2048: 160 -> 138; 32 of 4096: 232 ->
-    // 249).
-    const bool fits = bh * ((own + 63) / 64) <= (causal ? 2 : 1) * (int64_t)dlt_device_cus();
-    return fits || (pass == 2 && causal && dc.id == 2 && own < FLASH_SLIM_BELOW) ? FLASH_SLIM : FLASH_CHUNKED;
-  }
+  if (pass > 0 && order != FLASH_SPLIT1 && order != FLASH_SPLIT2)
+    return dlt_flash_bwd_64(causal, pass == 2 && dc.id == 2, own, bh * ((own + 63) / 64), dlt_device_cus()) ? FLASH_SLIM : FLASH_CHUNKED;
   return flash_fastest(pass, dc, dims, bh, own, other, causal, flash_same_bits(pass, dc, order));
 }
 

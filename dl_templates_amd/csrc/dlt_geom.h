@@ -103,6 +103,19 @@ DLT_HD bool dlt_tile_bwd_one_launch(int d, int S, int WR, int WC, bool img, int 
   return d == 64 || TC > (img ? 2 : 5) || rows < 12 * cus;
 }
 
+// Backward passes of dense / causal attention that do not split the other side: whether a workgroup owns 64 tokens (4 waves of one block)
+// instead of 128 (two blocks per wave).  `wgs`: workgroups of 64 tokens; `kv_64_128`: dK/dV at 64/128.  The same bits either way.
+// They do while they all run at once, one per CU, or two under a mask, where the work is uneven.  8 slabs of 2048 x 2048, dQ and dK/dV:
+// 64/64 32.3 -> 25.0 and 39.2 -> 30.0 us, 64/128 37.7 -> 28.5 and 50.5 -> 38.4, dQ at 128/128 52.0 -> 39.3; causal, 16 slabs: 35.4 -> 31.1 and
+// 43.5 -> 39.3, 40.2 -> 35.3 and 67.0 -> 50.3, 53.0 -> 45.4.  12 slabs without a mask (384 workgroups): the same or slower.
+// dK/dV at 64/128 under a mask, where two blocks per wave spill: always below 3072 keys (64 slabs of 2048: 160 -> 138; 32 of 4096: 232 ->
+// 249), up to four per CU below 8192 (whole backward pass, causal: 10 slabs of 4096 203 -> 186, 8 of 6000 253 -> 219, 6 of 8192 384 -> 360;
+// 10 of 6000 316 -> 327; beyond it loses: 4 of 12 000 510 -> 546).
+DLT_HD bool dlt_flash_bwd_64(bool causal, bool kv_64_128, int own, int64_t wgs, int64_t cus) {
+  if (causal && kv_64_128 && own < 3072) return true;
+  return wgs <= (!causal ? 1 : kv_64_128 && own <= 8192 ? 4 : 2) * cus;
+}
+
 // idx decode of the rotary op: row = int16(idx >> 16), col = int16(idx & 0xFFFF)
 // (src/fused_rope2d.py:41-42); an axis is rotated iff its value is >= 0 (:44-45).
 DLT_HD int dlt_rope_row(int32_t idx) { return (int)(int16_t)(idx >> 16); }

@@ -30,6 +30,7 @@ int shim_image_fwd_alone(int d, int S, int WR, int WC, int TR, int TC, int H, lo
 int shim_tile_bwd_one_launch(int d, int S, int WR, int WC, int img, int TC, long long rows, long long cus) {
   return dlt_tile_bwd_one_launch(d, S, WR, WC, img != 0, TC, rows, cus);
 }
+int shim_flash_bwd_64(int causal, int kv_64_128, int own, long long wgs, long long cus) { return dlt_flash_bwd_64(causal != 0, kv_64_128 != 0, own, wgs, cus); }
 int shim_rope_row(int idx) { return dlt_rope_row(idx); }
 int shim_rope_col(int idx) { return dlt_rope_col(idx); }
 }

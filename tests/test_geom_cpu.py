@@ -143,6 +143,20 @@ def test_narrow_tile_grids_take_two_backward_launches(shim):
     assert not one(4, 16, 16, 0, S=32) and not one(4, 16, 16, 0, WC=2) and not one(4, 16, 16, 0, WR=2)
 
 
+def test_flash_backward_workgroups_of_64_tokens(shim):
+    """One per CU, two under a mask; dK/dV at 64/128 under a mask always below 3072 keys and up to four per CU below 8192 (256 CUs)."""
+    def small(slabs, own, causal, kv_64_128):
+        return bool(shim.shim_flash_bwd_64(causal, kv_64_128, own, ctypes.c_longlong(slabs * -(-own // 64)), ctypes.c_longlong(256)))
+
+    for kv in (0, 1):
+        assert small(8, 2048, 0, kv) and not small(12, 2048, 0, kv) and small(1, 16384, 0, kv)
+        assert small(8, 4096, 1, kv) and small(2, 16384, 1, kv) and not small(4, 12000, 1, kv)
+    for slabs, own in [(10, 4096), (16, 4096), (8, 6000), (6, 8192), (8, 8192), (64, 2048), (256, 1024)]:
+        assert small(slabs, own, 1, 1) and not small(slabs, own, 1, 0), (slabs, own)
+    for slabs, own in [(17, 4096), (32, 4096), (9, 8192), (4, 8200)]:
+        assert not small(slabs, own, 1, 1), (slabs, own)
+
+
 def test_band_plan_of_the_long_band_cases(shim):
     """tests/test_swa_tiles_gpu.py means its LONG_BANDS to march beyond the ring of 3 rows, over several strips, the last one ragged (256 CUs)."""
     from tests.test_swa_tiles_gpu import LONG_BANDS
