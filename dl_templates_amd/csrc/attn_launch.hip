@@ -549,7 +549,11 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
 // tokens one after the other, however few the workgroups; the split ones take
 //     fixed + rounds over the CUs * (start and final sum of a workgroup + its 32-token blocks * time of a block on a CU).
 // The constants (us) are least-squares fits to launches of 32 ... 8192 tokens on either side and 4 ... 128 heads, dense and
-// causal; on those flash_fastest over all kinds picks the fastest kernel but for 2 % of the total time.
+// causal; on those flash_fastest over all kinds picked the fastest kernel but for 2 % of the total time.  Those of the backward passes
+// were fitted to chunked kernels of two blocks per wave and decide between splitting and not only; few workgroups have run up to a
+// quarter faster on one block per wave since (dlt_flash_bwd_64), so that short sides are split somewhat too often: of 263 shapes of 4 ... 64
+// slabs that are split in a pass 96 are faster by 3 % and more without (32 slabs of 300 x 300, 64/64, both passes 20.8 -> 15.4 us) and
+// 135 slower.
 //   77 queries x 1500 keys, 16 heads, 64/64: forward 22 -> 10 us, dQ 24 -> 11; 482 keys x 5450 queries, 4 heads: dK/dV 86 -> 26
 //   16 heads, 2048 x 2048: forward 64/128 46 -> 34 us, 128/128 55 -> 41 (SLIM)
 //
@@ -584,24 +588,26 @@ int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, i
   const auto wgs = [&](int n) { return (float)(bh * ((own + n - 1) / n)); };
   const auto may = [&](int kind) { return (kinds >> kind & 1u) != 0; };
   const float chunks = (float)((other + 63) / 64);
-  // two own blocks per wave: dK/dV at 64/128 under a mask (for passes 1 and 2 the choice here is between splitting and not: flash_pick)
-  const bool spills = pass == 2 && causal && dc.id == 2;
   int best = -1;
   float least = 0.f;
   const auto consider = [&](int kind, float t) {
     if (may(kind) && (best < 0 || t < least)) { least = t; best = kind; }
   };
-  consider(FLASH_CHUNKED, c.start + c.chunk * chunks);
-  if (wgs(128) > cus) {
+  // backward: split or not; which of the others runs is dlt_flash_bwd_64's choice (dK/dV at 64/128 under a mask: 0.65 on one block per wave)
+  const float whole = c.start + (pass == 2 && causal && dc.id == 2 ? 0.65f : 1.f) * c.chunk * chunks;
+  consider(FLASH_CHUNKED, whole);
+  if (pass > 0) {
+    if (wgs(128) > cus && may(FLASH_CHUNKED)) return FLASH_CHUNKED;
+  } else if (wgs(128) > cus) {
     // A CU has more than one slim workgroup.  Up to two of them run side by side, which still beats the chunked workgroups
     // at 64/64 and where a mask makes the work uneven (32 heads, 2048 x 2048, causal: 64/128 52 -> 46 us, 128/128 60 -> 49)
-    if ((pass == 0 && c.slim_chunk < NONE && (causal || dc.id == 0)) || spills) {
+    if (c.slim_chunk < NONE && (causal || dc.id == 0)) {
       const int kind = wgs(128) <= 2.f * cus ? FLASH_SLIM : FLASH_CHUNKED;
       if (may(kind)) return kind;
     }
     if (wgs(c.own) > cus && may(FLASH_CHUNKED)) return FLASH_CHUNKED;
   } else {
-    consider(FLASH_SLIM, spills ? c.start + 0.65f * c.chunk * chunks : c.slim_start + c.slim_chunk * chunks);
+    consider(FLASH_SLIM, c.slim_start + c.slim_chunk * chunks);
   }
   // the pieces of a row that a head dim below its class does not have are not read
   const float blocks = (float)((other + 31) / 32) * ((float)dims / (float)(dc.DK + dc.DV));
@@ -617,6 +623,7 @@ int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, i
 }
 // Kinds that give a slab the same bits as `kind`: one and two own blocks per split workgroup; slim and chunked workgroups where both
 // pass 64 tokens at a time (the chunked forward kernels at 64/128 and 128/128 pass 128: other reference maxima of the softmax).
+// Asked about backward passes only where they are split.
 unsigned flash_same_bits(int pass, const DimClass& dc, int kind) {
   if (kind == FLASH_SPLIT1 || kind == FLASH_SPLIT2) return 1u << FLASH_SPLIT1 | 1u << FLASH_SPLIT2;
   if (pass == 0 && (dc.id == 1 || dc.id == 2)) return 1u << kind;
@@ -729,7 +736,8 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
   a.slim = np_kv == FLASH_SLIM;
   // dQ with one workgroup of 128 queries per CU: 8 waves of one block (16 slabs of 2048 x 2048: 64/64 36.6 -> 34.6 us, 64/128 43.8 -> 41.0,
   // 128/128 58.0 -> 54.2; from two workgroups per CU on slower, 32 slabs 54.8 -> 56.0, 70.4 -> 70.5, 94.9 -> 108.5)
-  a.slim_q = np_q == FLASH_SLIM ? 4 : seq && nbh * ((a.Lq + 127) / 128) <= dlt_device_cus() ? 8 : 0;
+  // (under a mask 4 waves run up to there and beyond)
+  a.slim_q = np_q == FLASH_SLIM ? 4 : p.g.mode == DLT_GEOM_DENSE && nbh * ((a.Lq + 127) / 128) <= dlt_device_cus() ? 8 : 0;
   int rc;
 #define DLT_FLASH_PASS(C)                                                                                                  \
   rc = np_q == FLASH_SPLIT1 || np_q == FLASH_SPLIT2 ? dlt_flashs_bwd_q_##C(a, p.dtype, np_q, stream) : dlt_flash_launch_bwd_q_##C(a, p.dtype, (int)grid_q, stream); \

@@ -151,9 +151,10 @@ template <typename TIO, int MODE>
 int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && flash_async_staging()) {
-      // few workgroups: one own block per wave, in 4 waves (twice the workgroups) or 8 (see flash_pick)
+      // few workgroups: one own block per wave, in 4 waves (twice the workgroups) or, without a mask, 8 (see flash_backward)
       if (a.slim_q == 4) return flashd_launch_bwd_q<TIO, MODE, 1, 4>(a, stream);
-      if (a.slim_q == 8) return flashd_launch_bwd_q<TIO, MODE, 1, 8>(a, stream);
+      if constexpr (MODE == 0)
+        if (a.slim_q == 8) return flashd_launch_bwd_q<TIO, MODE, 1, 8>(a, stream);
       return flashd_launch_bwd_q<TIO, MODE, FLASHD_DQ_NP(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }

@@ -366,8 +366,8 @@ def test_a_slab_has_the_same_bits_in_any_call(causal, Lq, Lk, dk, dv, counts):
         assert torch.equal(a[:, -n:], b[:, -n:])
 
 
-# backward passes with one own block per wave: 4 waves while their workgroups of 64 fit the chip, dQ on 8 waves while its workgroups of 128 do,
-# two blocks per wave beyond: a token past a workgroup's end, chunk remainders, every class and dims below it, counts on every side of the lines
+# backward passes with one own block per wave: 4 waves while their workgroups of 64 fit the chip, without a mask dQ on 8 waves while its workgroups
+# of 128 do, two blocks per wave beyond: a token past a workgroup's end, chunk remainders, every class and dims below it, counts on every side of the lines
 @pytest.mark.parametrize("causal,Lq,Lk,dk,dv,counts", [
     (False, 1025, 1090, 64, 64, (1, 20, 40)), (False, 1090, 1025, 64, 128, (1, 20, 40)), (False, 1100, 1153, 128, 128, (1, 20, 40)),
     (False, 1030, 1100, 80, 72, (1, 20, 40)), (True, 1090, 1090, 64, 64, (1, 35)), (True, 1090, 1090, 64, 128, (1, 40)),

@@ -41,3 +41,9 @@ def test_tile_window_backward_kernels_spill_nothing(kernels):
     march = {n: k for n, k in kernels.items() if "swat_bwd_" in n}
     assert len(march) >= 20
     assert {n: k[".vgpr_spill_count"] for n, k in march.items() if k[".private_segment_fixed_size"]} == {}
+
+
+def test_dq_on_eight_waves_is_built_without_a_mask_only(kernels):
+    """flash_backward picks 8 waves of one block for dense calls; under a mask 4 waves run wherever they would."""
+    eight = [n for n in kernels if "flashd_bwd_q_kernel" in n and "ELi1ELi64ELi8E" in n]   # <.., NP 1, CK 64, NW 8, MODE, PAD>
+    assert eight and not [n for n in eight if "ELi1ELi64ELi8ELi1E" in n]
