@@ -106,7 +106,9 @@ int dlt_swa_fwd(const void* q, const int64_t q_strides[4], const void* k, const 
 
 /* Backward: replaces tiled_swa_bwd_preprocess_kernel (src/tiled_swa.py:253-282) and
  * tiled_swa_bwd_large_kernel_decoupled_q (:407-562) plus TiledSwa.backward (:649-689).
- * `delta` is caller-provided fp32 scratch with the strides of lse2.  dq/dk/dv are written
+ * `delta` is caller-provided fp32 scratch with the strides of lse2: a call overwrites it or leaves it
+ * as it is (kernels that form all three gradients in one launch need none), and nothing in it is a
+ * result.  dq/dk/dv are written
  * in the element type of q/k/v (the reference accumulates dq in an fp32 tensor, :656).
  * With `rope` the inputs q, k are the UN-rotated tensors and dq, dk are returned with
  * respect to them (transposed rotation applied on store). */
@@ -243,7 +245,9 @@ int dlt_flash_bwd(const void* q, const int64_t q_strides[4], const void* k, cons
  * Counterpart of the reference's triton.testing.do_bench calls (src/tiled_swa.py:765-774,
  * src/flash_attn.py:592,606), at kernel granularity.  While enabled for the calling thread,
  * every kernel the library launches is bracketed by a pair of hipEvents recorded on the
- * launch stream.  dlt_timing_collect waits for the recorded events, writes up to `max`
+ * launch stream.  A backward launch that forms dq, dk and dv together (tiles of 16 tokens with a 3 x 3
+ * window, head dim 32 / 64; narrow grids at 32 excepted) is recorded as DLT_K_BWD_KV, without a
+ * DLT_K_BWD_Q beside it.  dlt_timing_collect waits for the recorded events, writes up to `max`
  * records in launch order, stores the number available in *n and clears the list.
  * Enabling creates events lazily (host-side handles only, no device allocation). */
 enum { DLT_K_ROPE = 0, DLT_K_FWD = 1, DLT_K_DELTA = 2, DLT_K_BWD_KV = 3, DLT_K_BWD_Q = 4, DLT_K_COUNT = 5 };
