@@ -183,7 +183,7 @@ struct FlashDBuf {
 // Head dims the products run over.  PAD 0: the class's own; 1: any below them, the products run over the zeroed pieces too; 2: at
 // most 96 of 128, the last 32 dims are left out of every product, operand read and accumulator (their terms are zeros); 3: at most 80,
 // the transposed products (O, dQ, dK, dV) leave out 48.  These kernels are bound by the issue port and LDS reads, of which that is a
-// quarter (2) or 5 / 16 (3) at 128/128, a sixth to a quarter at 64/128.  Variant 1 -> 2, forward and backward: 32 slabs of 3000 at 96/96
+// quarter (2) or 5 / 16 (3) at 128/128, an eighth (dQ at 64/96) to a quarter (forward at 64/80) at 64/128.  Variant 1 -> 2, forward and backward: 32 slabs of 3000 at 96/96
 // 157 -> 139 and 442 -> 383 us; 32 of 4096 at 64/96 202 -> 192 and 550 -> 514.  1 -> 2 -> 3: 32 of 4096 at 80/80 231 -> 208 -> 202 and
 // 777 -> 664 -> 644, causal 190 -> 170 -> 164 and 508 -> 432 -> 418; 8 of 2048 38.1 -> 34.3 -> 32.8 and 81.4 -> 71.9 -> 69.0; 64
 // causal of 700 23.0 -> 21.2 -> 20.8 and 66.4 -> 59.9 -> 57.5; 8 of 2048 at 64/80 33.7 -> 31.1 -> 30.5 and 65.6 -> 61.5 -> 60.9.
