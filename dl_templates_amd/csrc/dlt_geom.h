@@ -76,19 +76,20 @@ DLT_HD int dlt_band_plan(int units, int64_t cols, int64_t slots, int& per, int& 
 
 // Image layout, forward over 16-token tiles at d = 32 with a 3 x 3 window: whether one workgroup per CU runs (`cols` strips of 8 tiles).
 // A pixel's heads lie side by side, so the workgroups of 8 heads and more share every 128-byte line and must meet in the L2.  Two
-// workgroups per CU march whole strips apart and fetch 1.37 times the bytes; one per CU gives up half of the waves that hide latency.
-// It wins where HBM is the bound and both launches would march whole strips: whole strips in 1, 2 or 4 rounds over the CUs that are at
-// least 7/8 full, and rows enough.  H = 8, us, two per CU -> one, inputs in the caches / not: one round, 64 rows of 64 tiles 153 -> 141 /
-// 160 -> 141, 48 rows 101 -> 103 / 119 -> 107, 16 rows 30 -> 31 / 42 -> 41; two rounds, 64 rows 316 -> 281, 48 of 16 tiles 196 -> 192, 24 of
-// 64 101 -> 106 / 118 -> 112, 8 rows 30 -> 34 / 43 -> 45; four, 64 rows 630 -> 553, 24 of 16 tiles 182 -> 195; 16 heads, two rounds of 48 rows
-// 257 -> 211.  It loses in three rounds (64 rows of 48 tiles 422 -> 436) and five (407 -> 433), on ragged strips (two rounds of 33 tiles,
-// 64 rows 262 -> 275; one tile 93 -> 149: half of a CU's waves own nothing) and with fewer heads (16 x 2 slabs of 64 x 64: 121 -> 122);
-// 32-token tiles (179 -> 208) and windows of five columns (183 -> 186) are bound by arithmetic, d = 64 and five rows leave LDS for one anyway.
+// workgroups per CU march strips apart and fetch 1.37 times the bytes; one per CU gives up half of the waves that hide latency.
+// It wins where HBM is the bound and both launches would march strips: strips and rounds over the CUs at least 15/16 full, 1, 2 or 4 rounds, and
+// rows enough, fewer with 16 heads.  Two per CU -> one, us, inputs in the caches / cycled through 800 MB: 8 heads, one round of 64 rows of
+// 64 tiles 153 -> 141 / 160 -> 141, of 16 or 32 tiles 132 -> 132 / 136 -> 131, 48 rows of 64 101 -> 103 / 119 -> 107; two rounds of 40 rows of 8 to
+// 64 tiles -11 ... +1 / -12 ... 0 %, 24 of 64 101 -> 106 / 118 -> 112, 8 rows 30 -> 34 / 43 -> 45; four of 48 rows -10 ... +3 %, of 24 -3 ... +8 %.
+// 16 heads: one round of 32 rows of 64 tiles 64 -> 59 / 92 -> 82, two of 24 114 -> 108 / 130 -> 111, four of 32 -9 ... +1 %.  It loses in three
+// rounds (64 rows of 48 tiles 422 -> 436) and five (407 -> 433), on ragged strips (two rounds of 33 tiles, 64 rows 262 -> 275; one
+// tile 93 -> 149: most of a CU's waves own nothing) and with fewer heads (16 x 2 slabs of 64 x 64: 121 -> 122); 32-token tiles (179 ->
+// 208) and windows of five columns (183 -> 186) are bound by arithmetic, d = 64 and five rows leave LDS for one anyway.
 DLT_HD bool dlt_image_fwd_alone(int d, int S, int WR, int WC, int TR, int TC, int H, int64_t cols, int64_t cus) {
-  if (d != 32 || S != 16 || WR != 1 || WC != 1 || H < 8 || TC % 8 != 0 || cols < cus) return false;
+  if (d != 32 || S != 16 || WR != 1 || WC != 1 || H < 8 || cols < cus || 16 * TC < 15 * 8 * ((TC + 7) / 8)) return false;
   const int64_t rounds = (cols + cus - 1) / cus;
-  if (8 * cols < 7 * rounds * cus) return false;
-  return rounds == 2 ? TR >= 48 : (rounds == 1 || rounds == 4) && TR >= 64;
+  if (16 * cols < 15 * rounds * cus) return false;
+  return rounds == 1 ? TR >= (H < 16 ? 64 : 32) : rounds == 2 ? TR >= (H < 16 ? 40 : 24) : rounds == 4 && TR >= (H < 16 ? 48 : 32);
 }
 
 // Backward over tiles at d = 32 / 64: whether dQ, dK and dV leave in one launch (16-token tiles, 3 x 3 window; TC tile columns, `rows` grid

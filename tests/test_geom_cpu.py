@@ -117,15 +117,16 @@ def test_band_plan_is_the_best_split_and_cheap_to_find(shim):
 
 
 def test_image_forward_alone_only_where_it_is_faster(shim):
-    """One workgroup per CU: whole strips of 8 tiles, 1, 2 or 4 rounds of them, many rows, 8 heads and more (256 CUs)."""
+    """One workgroup per CU: full strips of 8 tiles, 1, 2 or 4 full rounds of them, many rows, 8 heads and more (256 CUs)."""
     def alone(B, H, th, tw, d=32, S=16, WR=1, WC=1):
         return bool(shim.shim_image_fwd_alone(d, S, WR, WC, th, tw, H, ctypes.c_longlong(B * H * -(-tw * S // 128)), ctypes.c_longlong(256)))
 
-    for shape in [(4, 8, 64, 64), (32, 8, 64, 8), (8, 8, 48, 64), (16, 8, 64, 64), (4, 16, 100, 64), (7, 8, 60, 72), (3, 12, 64, 104)]:
+    for shape in [(4, 8, 64, 64), (32, 8, 64, 8), (8, 8, 40, 64), (16, 8, 48, 64), (4, 8, 100, 60), (8, 8, 64, 62),
+                  (2, 16, 32, 64), (4, 16, 24, 60), (8, 16, 32, 64), (3, 32, 24, 40)]:
         assert alone(*shape), shape
-    for shape in [(128, 8, 32, 1), (64, 8, 24, 5), (16, 8, 64, 9), (32, 8, 64, 9), (8, 8, 64, 33), (2, 8, 96, 61),     # ragged strips
-                  (4, 8, 48, 64), (32, 8, 16, 8), (8, 8, 47, 64), (8, 8, 1, 64), (16, 8, 63, 64), (64, 8, 30, 16),         # few rows
-                  (12, 8, 64, 64), (20, 8, 64, 64), (24, 8, 64, 64), (6, 8, 64, 64),                                       # other rounds
+    for shape in [(128, 8, 32, 1), (64, 8, 24, 5), (16, 8, 64, 9), (32, 8, 64, 7), (8, 8, 64, 33), (2, 8, 96, 61),     # ragged strips
+                  (4, 8, 63, 64), (32, 8, 16, 8), (8, 8, 39, 64), (8, 8, 1, 64), (16, 8, 47, 64), (2, 16, 31, 64), (4, 16, 23, 64),   # few rows
+                  (12, 8, 64, 64), (20, 8, 64, 64), (24, 8, 64, 64), (6, 8, 64, 64), (4, 32, 64, 56),                      # other rounds
                   (16, 2, 64, 64), (8, 7, 64, 64), (3, 8, 64, 64)]:                                                        # heads, idle CUs
         assert not alone(*shape), shape
     assert not alone(4, 8, 64, 64, d=64) and not alone(4, 8, 64, 64, S=32) and not alone(4, 8, 64, 64, WC=2) and not alone(4, 8, 64, 64, WR=2)

@@ -175,8 +175,10 @@ def test_image_forward_with_many_strips(B, th, tw):
 @pytest.mark.parametrize("B,H,th,tw", [
     (32, 8, 64, 8),    # one workgroup per CU, one round of whole strips
     (32, 8, 63, 8),    # a row less: two per CU
-    (60, 8, 48, 8),    # one per CU, two rounds, the second not full
-    (32, 8, 48, 9),    # ragged strips: two per CU
+    (16, 8, 40, 30),   # one per CU, two rounds, the last strip not full
+    (60, 8, 40, 8),    # the second round not full
+    (32, 8, 40, 9),    # ragged strips: two per CU
+    (4, 16, 24, 60),   # 16 heads: from 24 rows on
 ])
 def test_image_forward_with_one_workgroup_per_cu(B, H, th, tw):
     """Both sides of the lines of dlt_image_fwd_alone at 256 CUs: bit-equal to the token layout."""
