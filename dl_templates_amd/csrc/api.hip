@@ -387,17 +387,63 @@ extern "C" int dlt_swa_bwd_noalloc(const void* q, const int64_t q_strides[4], co
   return dlt_attn_backward(p, t, (hipStream_t)stream);
 }
 
-extern "C" int dlt_flash_fwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                             const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
-                             float* lse2, const int64_t lse_strides[3],
-                             const dlt_flash_shape_t* shape, void* stream) {
+extern "C" int dlt_flash_workspace(const dlt_flash_shape_t* shape, int backward, int64_t* bytes) {
+  DLT_REQUIRE(bytes != nullptr, "flash_workspace: bytes is NULL");
+  AttnProblem p;
+  const int rc = flash_problem("flash_workspace", shape, p);
+  if (rc != DLT_OK) return rc;
+  *bytes = 4 * dlt_attn_part_floats(p, backward != 0);
+  return DLT_OK;
+}
+
+// `ws` of at least dlt_flash_workspace bytes, or none: NULL comes back where the call needs none or has none
+static int flash_ws(const char* who, const AttnProblem& p, bool backward, void* ws, int64_t ws_bytes, float*& part) {
+  part = nullptr;
+  if (ws == nullptr) return DLT_OK;
+  const int64_t need = 4 * dlt_attn_part_floats(p, backward);
+  DLT_REQUIRE((uintptr_t)ws % 16 == 0, "%s: workspace is not 16-byte aligned", who);
+  DLT_REQUIRE(ws_bytes >= need, "%s: workspace of %lld bytes, %lld needed", who, (long long)ws_bytes, (long long)need);
+  if (need > 0) part = (float*)ws;
+  return DLT_OK;
+}
+
+extern "C" int dlt_flash_fwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                                const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
+                                float* lse2, const int64_t lse_strides[3],
+                                const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream) {
   AttnProblem p;
   int rc = flash_problem("flash_fwd", shape, p);
   if (rc != DLT_OK) return rc;
   AttnTensors t;
   rc = fill_fwd("flash_fwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides);
+  if (rc == DLT_OK) rc = flash_ws("flash_fwd", p, false, ws, ws_bytes, t.part);
   if (rc != DLT_OK) return rc;
   return dlt_attn_forward(p, t, (hipStream_t)stream);
+}
+
+extern "C" int dlt_flash_fwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                             const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
+                             float* lse2, const int64_t lse_strides[3],
+                             const dlt_flash_shape_t* shape, void* stream) {
+  return dlt_flash_fwd_ws(q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, nullptr, 0, stream);
+}
+
+extern "C" int dlt_flash_bwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                                const void* v, const int64_t v_strides[4], const void* o, const int64_t o_strides[4],
+                                const void* d_o, const int64_t do_strides[4],
+                                const float* lse2, float* delta, const int64_t lse_strides[3],
+                                void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
+                                void* dv, const int64_t dv_strides[4],
+                                const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream) {
+  AttnProblem p;
+  int rc = flash_problem("flash_bwd", shape, p);
+  if (rc != DLT_OK) return rc;
+  AttnTensors t;
+  rc = fill_bwd("flash_bwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta,
+                lse_strides, dq, dq_strides, dk, dk_strides, dv, dv_strides);
+  if (rc == DLT_OK) rc = flash_ws("flash_bwd", p, true, ws, ws_bytes, t.part);
+  if (rc != DLT_OK) return rc;
+  return dlt_attn_backward(p, t, (hipStream_t)stream);
 }
 
 extern "C" int dlt_flash_bwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
@@ -407,14 +453,8 @@ extern "C" int dlt_flash_bwd(const void* q, const int64_t q_strides[4], const vo
                              void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
                              void* dv, const int64_t dv_strides[4],
                              const dlt_flash_shape_t* shape, void* stream) {
-  AttnProblem p;
-  int rc = flash_problem("flash_bwd", shape, p);
-  if (rc != DLT_OK) return rc;
-  AttnTensors t;
-  rc = fill_bwd("flash_bwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta,
-                lse_strides, dq, dq_strides, dk, dk_strides, dv, dv_strides);
-  if (rc != DLT_OK) return rc;
-  return dlt_attn_backward(p, t, (hipStream_t)stream);
+  return dlt_flash_bwd_ws(q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq, dq_strides, dk,
+                          dk_strides, dv, dv_strides, shape, nullptr, 0, stream);
 }
 
 // ---- image-layout entry points ------------------------------------------------------------------

@@ -45,6 +45,9 @@ int dlt_flashs_bwd_kv_64_128(const FlashBwdArgs&, int dtype, int np, hipStream_t
 int dlt_flashs_fwd_128_128(const FlashArgs&, int dtype, int np, hipStream_t);
 int dlt_flashs_bwd_q_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
 int dlt_flashs_bwd_kv_128_128(const FlashBwdArgs&, int dtype, int np, hipStream_t);
+int dlt_flash_share_fwd(const FlashArgs&, int dtype, hipStream_t);
+int dlt_flash_share_bwd_q(const FlashBwdArgs&, int dtype, hipStream_t);
+int dlt_flash_share_bwd_kv(const FlashBwdArgs&, int dtype, hipStream_t);
 int dlt_swag_launch_f32(const SwagArgs&, int nch, int ncg, int grid, hipStream_t);
 int dlt_swag_launch_32_2(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swag_launch_32_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
@@ -69,6 +72,11 @@ int dlt_swa2_launch_fwd_64(const Swa2FwdArgs&, int, int, hipStream_t);
 int dlt_swa2_launch_bwd_64(const Swa2BwdArgs&, int, int, hipStream_t);
 int dlt_swa2_launch_fwd_128(const Swa2FwdArgs&, int, int, hipStream_t);
 int dlt_swa2_launch_bwd_128(const Swa2BwdArgs&, int, int, hipStream_t);
+
+bool dlt_flash_async() {
+  static const bool on = [] { const char* e = getenv("DLT_FLASH_SYNC_STAGING"); return !(e != nullptr && e[0] == '1'); }();
+  return on;
+}
 
 namespace {
 
@@ -637,6 +645,53 @@ int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int 
   return flash_fastest(pass, dc, dims, bh, own, other, causal, flash_same_bits(pass, dc, order));
 }
 
+// How a dense / causal pass runs: the kind, and over how many workgroups the other side of an own block is split (n; len: FlashShare).
+//
+// A dense pass with few own tokens and many others leaves most CUs idle, or has each of its small workgroups read all of the other side
+// (16 slabs, forward: 64 queries x 4000 keys at 64/64 ran on 64 CUs).  Its other side is cut into n shares of chunked workgroups instead; their
+// fp32 partial results are summed by a second launch, which costs some 3 us and 8 bytes per own element and share.  n follows from a
+// slab's shape alone (see above), as other / (a + b own) up to 8: the lines were fitted to 2100 shapes of 4 ... 128 slabs (n = 2, 3, 4, 6, 8), a loss
+// counted eightfold.  Inside them, not split -> split, geometric mean of the pass by slabs (4, 8, 16, 32, 64, 128): forward 1.7 ... 2.2,
+// 1.55 ... 2.0, 1.33 ... 1.8, 1.22 ... 1.6, 1.2, 1.15; both backward passes together 1.4 ... 1.8 down to 1.05 ... 1.3.  Shorter other sides and
+// longer own ones lose more to the sums than idle CUs cost (128 slabs of 734 x 3321, 64/64: 98 -> 144 us with n = 4).
+struct FlashPlan { int kind, n, len; };
+FlashPlan flash_plan(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal, bool may_split) {
+  if (may_split && !causal) {
+    // other side of at least `least` tokens and `times` the own one; a, 4 b
+    static const struct { int least, times, a, b4; } RULE[3][4] = {   // by pass; 64/64, 64/128, 128/128 with up to 192 dims in all, 128/128
+        {{2500, 3, 150, 4}, {2500, 3, 500, 3}, {2500, 3, 150, 4}, {1200, 3, 150, 6}},
+        {{1600, 1, 350, 4}, {600, 1, 150, 4}, {1600, 1, 150, 4}, {600, 4, 150, 6}},
+        {{2500, 1, 150, 6}, {1600, 4, 250, 4}, {2000, 1, 500, 4}, {1200, 4, 150, 8}}};
+    const auto& r = RULE[pass][dc.id == 0 ? 0 : dc.id == 2 ? 1 : dims <= 192 ? 2 : 3];
+    int n = other < r.least || other < (int64_t)r.times * own ? 1 : (int)(4 * (int64_t)other / (4 * r.a + (int64_t)r.b4 * own));
+    n = dlt_imin(n, 8);
+    if (n > 1) {
+      const int len = roundup((other + n - 1) / n, 128);
+      n = (other + len - 1) / len;
+      // one own block per wave or two (the same bits): one while its workgroups are few.  Forward at 64/64, 8 waves of one against 4 of two: 0.92 of the
+      // time below a workgroup of 128 queries per four CUs, 0.96 up to one per CU, 1.01 to two, 1.05 beyond; at 64/128 and 128/128 always
+      // 8 waves (their two-block kernel passes 128 keys at a time).  Backward, whole pass, one against two: 0.82 ... 0.89 below 64 workgroups of
+      // 64, 0.87 ... 0.96 to one per CU, 0.97 ... 1.0 to two, 0.95 ... 1.09 beyond
+      const int64_t cus = dlt_device_cus();
+      const bool slim = pass == 0 ? dc.id != 0 || bh * n * ((own + 127) / 128) <= cus : bh * n * ((own + 63) / 64) <= 2 * cus;
+      if (n > 1) return {slim ? FLASH_SLIM : FLASH_CHUNKED, n, len};
+    }
+  }
+  return {flash_pick(pass, dc, dims, bh, own, other, causal), 1, other};
+}
+// the asynchronously staged kernels know shares
+// (partial rows are counted in 32 bits: beyond that nothing is split)
+bool flash_may_split(const AttnProblem& p, const DimClass& dc) {
+  const int64_t rows = (int64_t)p.B * p.H * dlt_imax(p.g.XLq, p.g.XLk);
+  return p.g.mode == DLT_GEOM_DENSE && dc.id <= 2 && p.dtype != DLT_FP32 && p.dk % 8 == 0 && p.dv % 8 == 0 && rows <= 0x7fffffff / 16 && dlt_flash_async();
+}
+// floats of partial results a pass needs (0: not split)
+int64_t flash_part_fwd(const AttnProblem& p, const FlashPlan& f) {
+  return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLq * (p.dv + 2) : 0;
+}
+int64_t flash_part_q(const AttnProblem& p, const FlashPlan& f) { return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLq * p.dk : 0; }
+int64_t flash_part_kv(const AttnProblem& p, const FlashPlan& f) { return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLk * (p.dk + p.dv) : 0; }
+
 int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {
   if (dlt_route_note(DLT_FAMILY_FLASH)) return DLT_OK;
   FlashArgs a;
@@ -658,22 +713,25 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   const int64_t grid = (int64_t)p.B * p.H * p.g.TR * a.nblk;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "flash forward: grid too large");
+  a.share = {t.part, 1, a.Lk};
+  int np = FLASH_CHUNKED;
   if (p.g.mode != DLT_GEOM_SWA) {
-    const int np = flash_pick(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0);
+    const FlashPlan f = flash_plan(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0, t.part != nullptr && flash_may_split(p, dc));
+    np = f.kind;
     a.slim = np == FLASH_SLIM;
-    if (np == FLASH_SPLIT1 || np == FLASH_SPLIT2) switch (dc.id) {
-      case 0: return dlt_flashs_fwd_64_64(a, p.dtype, np, stream);
-      case 1: return dlt_flashs_fwd_128_128(a, p.dtype, np, stream);
-      case 3: return dlt_flashs_fwd_32_32(a, p.dtype, np, stream);
-      default: return dlt_flashs_fwd_64_128(a, p.dtype, np, stream);
-    }
+    a.share.n = f.n; a.share.len = f.len;
   }
+  const bool split = np == FLASH_SPLIT1 || np == FLASH_SPLIT2;
+  int rc;
+#define DLT_FLASH_FWD(C) rc = split ? dlt_flashs_fwd_##C(a, p.dtype, np, stream) : dlt_flash_launch_fwd_##C(a, p.dtype, (int)grid, stream); break
   switch (dc.id) {
-    case 0: return dlt_flash_launch_fwd_64_64(a, p.dtype, (int)grid, stream);
-    case 1: return dlt_flash_launch_fwd_128_128(a, p.dtype, (int)grid, stream);
-    case 3: return dlt_flash_launch_fwd_32_32(a, p.dtype, (int)grid, stream);
-    default: return dlt_flash_launch_fwd_64_128(a, p.dtype, (int)grid, stream);
+    case 0: DLT_FLASH_FWD(64_64);
+    case 1: DLT_FLASH_FWD(128_128);
+    case 3: DLT_FLASH_FWD(32_32);
+    default: DLT_FLASH_FWD(64_128);
   }
+#undef DLT_FLASH_FWD
+  return rc == DLT_OK && a.share.n > 1 ? dlt_flash_share_fwd(a, p.dtype, stream) : rc;
 }
 
 int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {
@@ -731,24 +789,36 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
   // each pass streams its other side through LDS or splits it over the waves, whichever suits its own shape
   const int64_t nbh = (int64_t)p.B * p.H;
   const bool seq = p.g.mode != DLT_GEOM_SWA;
-  const int np_q = seq ? flash_pick(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0) : 0;
-  const int np_kv = seq ? flash_pick(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0) : 0;
+  FlashPlan fq = {FLASH_CHUNKED, 1, a.Lk}, fkv = {FLASH_CHUNKED, 1, a.Lq};
+  if (seq) {
+    bool may_split = t.part != nullptr && flash_may_split(p, dc);
+    fq = flash_plan(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0, may_split);
+    may_split = may_split && dlt_flash_scalars_fit(a);   // else dK/dV stays on the register-staged kernel
+    fkv = flash_plan(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0, may_split);
+  }
+  const int np_q = fq.kind, np_kv = fkv.kind;
+  a.share_q = {t.part, fq.n, fq.len};
+  a.share_kv = {t.part + flash_part_q(p, fq), fkv.n, fkv.len};
   a.slim = np_kv == FLASH_SLIM;
   // dQ with one workgroup of 128 queries per CU: 8 waves of one block (16 slabs of 2048 x 2048: 64/64 36.6 -> 34.6 us, 64/128 43.8 -> 41.0,
   // 128/128 58.0 -> 54.2; from two workgroups per CU on slower, 32 slabs 54.8 -> 56.0, 70.4 -> 70.5, 94.9 -> 108.5)
   // (under a mask 4 waves run up to there and beyond)
-  a.slim_q = np_q == FLASH_SLIM ? 4 : p.g.mode == DLT_GEOM_DENSE && nbh * ((a.Lq + 127) / 128) <= dlt_device_cus() ? 8 : 0;
+  a.slim_q = np_q == FLASH_SLIM ? 4 : p.g.mode == DLT_GEOM_DENSE && fq.n == 1 && nbh * ((a.Lq + 127) / 128) <= dlt_device_cus() ? 8 : 0;
   int rc;
 #define DLT_FLASH_PASS(C)                                                                                                  \
   rc = np_q == FLASH_SPLIT1 || np_q == FLASH_SPLIT2 ? dlt_flashs_bwd_q_##C(a, p.dtype, np_q, stream) : dlt_flash_launch_bwd_q_##C(a, p.dtype, (int)grid_q, stream); \
   if (rc != DLT_OK) return rc;                                                                                             \
-  return np_kv == FLASH_SPLIT1 || np_kv == FLASH_SPLIT2 ? dlt_flashs_bwd_kv_##C(a, p.dtype, np_kv, stream) : dlt_flash_launch_bwd_kv_##C(a, p.dtype, (int)grid_kv, stream)
+  rc = np_kv == FLASH_SPLIT1 || np_kv == FLASH_SPLIT2 ? dlt_flashs_bwd_kv_##C(a, p.dtype, np_kv, stream) : dlt_flash_launch_bwd_kv_##C(a, p.dtype, (int)grid_kv, stream); \
+  break
   switch (dc.id) {
     case 0: DLT_FLASH_PASS(64_64);
     case 1: DLT_FLASH_PASS(128_128);
     case 3: DLT_FLASH_PASS(32_32);
     default: DLT_FLASH_PASS(64_128);
   }
+  if (rc == DLT_OK && fq.n > 1) rc = dlt_flash_share_bwd_q(a, p.dtype, stream);
+  if (rc == DLT_OK && fkv.n > 1) rc = dlt_flash_share_bwd_kv(a, p.dtype, stream);
+  return rc;
 #undef DLT_FLASH_PASS
 }
 
@@ -827,6 +897,15 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
     case 4: return dlt_launch_fwd_256_256(a, np, (int)grid, stream);
     default: return dlt_launch_fwd_64_128(a, np, (int)grid, stream);
   }
+}
+
+int64_t dlt_attn_part_floats(const AttnProblem& p, bool backward) {
+  DimClass dc;
+  if (p.g.mode != DLT_GEOM_DENSE || p.dk > 128 || p.dv > 128 || pick_dims(p, dc) != DLT_OK || !flash_may_split(p, dc)) return 0;
+  const int64_t bh = (int64_t)p.B * p.H;
+  if (!backward) return flash_part_fwd(p, flash_plan(0, dc, p.dk + p.dv, bh, p.g.XLq, p.g.XLk, false, true));
+  return flash_part_q(p, flash_plan(1, dc, p.dk + p.dv, bh, p.g.XLq, p.g.XLk, false, true)) +
+         flash_part_kv(p, flash_plan(2, dc, p.dk + p.dv, bh, p.g.XLk, p.g.XLq, false, true));
 }
 
 int dlt_attn_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream) {

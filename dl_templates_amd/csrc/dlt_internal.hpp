@@ -19,6 +19,8 @@ int dlt_ensure_lds(const void* kern, int bytes);
 bool dlt_route_note(int family);
 bool dlt_route_dry();
 void dlt_route_reset();
+// DLT_FLASH_SYNC_STAGING=1 in the environment keeps the register-staged flash kernels for every class (A/B timing)
+bool dlt_flash_async();
 // compute units of the current device (asked once per device; 256 when the query fails)
 int dlt_device_cus();
 
@@ -67,6 +69,7 @@ struct AttnTensors {
   void *q_rot, *k_rot;  // forward: optional outputs, the rotated q and k (NULL: not wanted)
   float* lse;        // written by forward, read by backward
   float* delta;      // scratch written by the backward pre-pass
+  float* part;       // flash: partial results of a split streamed side (dlt_flash_workspace), or NULL: not split
   // element strides [B, H, N, D]; entry 4 is only used with an image token map (AttnProblem::tm):
   // then [2] is the stride of a pixel column and [4] the stride of a pixel row
   int64_t qs[5], ks[5], vs[5], os[5], dos[5], dqs[5], dks[5], dvs[5], ls[3];
@@ -85,3 +88,5 @@ struct AttnProblem {
 
 int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream);
 int dlt_attn_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream);
+// floats of AttnTensors::part that a dense flash pass of this shape splits its work with (0: none)
+int64_t dlt_attn_part_floats(const AttnProblem& p, bool backward);

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_k, a.B * a.H, a.causal_group, OWN, false, bh, r_own, x0);
-  else flash_block(lin, a.nblk_k, 1, OWN, bh, r_own, x0);
+  else flash_block(lin, a.nblk_k, a.share_kv.n, OWN, bh, r_own, x0);   // r_own: the share
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* kb_ = reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1];
   const TIO* vb_ = reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1];
@@ -222,7 +222,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
-  W.init_seq(CAUSAL ? (x0 / CK) * CK : 0, a.Lq);
+  if constexpr (CAUSAL) W.init_seq((x0 / CK) * CK, a.Lq);
+  else W.init_seq(r_own * a.share_kv.len, r_own + 1 < a.share_kv.n ? (r_own + 1) * a.share_kv.len : a.Lq);
   const int wk0 = x0 + wave * 16 * NP;  // first own key of this wave
 
   FlashDStage<DK, CK, NW, false> stq;
@@ -447,6 +448,13 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
+  if (!CAUSAL && a.share_kv.n > 1) {
+    float* part = a.share_kv.part + flash_share_row(a.share_kv, bh, r_own, a.Lk) * a.dk_;
+    flash_share_put<NP>(part, dk_acc, a.dk_, wk0 + n, a.Lk, g);
+    part = a.share_kv.part + (int64_t)a.B * a.H * a.share_kv.n * a.Lk * a.dk_ + flash_share_row(a.share_kv, bh, r_own, a.Lk) * a.dv_;
+    flash_share_put<NP>(part, dv_acc, a.dv_, wk0 + n, a.Lk, g);
+    return;
+  }
   __syncthreads();
   TIO* dkb = reinterpret_cast<TIO*>(a.dk) + b * a.dks[0] + h * a.dks[1];
   TIO* dvb = reinterpret_cast<TIO*>(a.dv) + b * a.dvs[0] + h * a.dvs[1];
@@ -480,7 +488,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
-  else flash_block(lin, a.nblk, 1, OWN, bh, r_own, x0);
+  else flash_block(lin, a.nblk, a.share.n, OWN, bh, r_own, x0);   // r_own: the share
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
@@ -490,7 +498,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
-  W.init_seq(0, CAUSAL ? dlt_imin(a.Lk, x0 + OWN) : a.Lk);
+  if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
+  else W.init_seq(r_own * a.share.len, r_own + 1 < a.share.n ? (r_own + 1) * a.share.len : a.Lk);
 
   FlashDStage<DK, CK, NW> stk;
   FlashDStage<DV, CK, NW> stv;
@@ -683,6 +692,17 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
+  if (!CAUSAL && a.share.n > 1) {
+    const int64_t row0 = flash_share_row(a.share, bh, r_own, a.Lq);
+    float* ml = a.share.part + (int64_t)a.B * a.H * a.share.n * a.Lq * a.dv + 2 * row0;
+    flash_share_put<NP>(a.share.part + row0 * a.dv, acc, a.dv, wq0 + n, a.Lq, g);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const float lt = wave_sum4(acc_l[p][0]);
+      if (g == 0 && tq[p] >= 0) *reinterpret_cast<float2*>(ml + 2 * tq[p]) = float2{m_run[p], lt};
+    }
+    return;
+  }
   __syncthreads();
 
   // ---- epilogue: normalise, O^T fragments -> LDS tile -> coalesced rows
@@ -728,7 +748,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_q, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
-  else flash_block(lin, a.nblk_q, 1, OWN, bh, r_own, x0);
+  else flash_block(lin, a.nblk_q, a.share_q.n, OWN, bh, r_own, x0);   // r_own: the share
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
@@ -738,7 +758,8 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
-  W.init_seq(0, CAUSAL ? dlt_imin(a.Lk, x0 + OWN) : a.Lk);
+  if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
+  else W.init_seq(r_own * a.share_q.len, r_own + 1 < a.share_q.n ? (r_own + 1) * a.share_q.len : a.Lk);
 
   FlashDStage<DK, CK, NW, (DK + DV > 128)> stk;
   FlashDStage<DV, CK, NW, (DK + DV > 128)> stv;
@@ -784,7 +805,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
         for (int j = 0; j < 8; j++) part += fo[j] * fd[j];
       }
       del_n[p] = wave_sum4(part);
-      if (g == 0 && tq >= 0) store_stream4(a.delta_out + off, del_n[p]);
+      if (g == 0 && tq >= 0 && (CAUSAL || r_own == 0)) store_stream4(a.delta_out + off, del_n[p]);
     } else {
       del_n[p] = tq >= 0 ? a.delta[off] : 0.f;
     }
@@ -931,6 +952,10 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   if (ci < W.nchunks) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
+  }
+  if (!CAUSAL && a.share_q.n > 1) {
+    flash_share_put<NP>(a.share_q.part + flash_share_row(a.share_q, bh, r_own, a.Lq) * a.dk_, dq_acc, a.dk_, wq0 + n, a.Lq, g);
+    return;
   }
   __syncthreads();
   TIO* dqb = reinterpret_cast<TIO*>(a.dq) + b * a.dqs[0] + h * a.dqs[1];

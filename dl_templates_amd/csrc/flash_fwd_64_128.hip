@@ -1,3 +1,4 @@
 #define DLT_DK 64
 #define DLT_DV 128
+#define DLT_FLASH_PART 0
 #include "flash_inst.hpp"

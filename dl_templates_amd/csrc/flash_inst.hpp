@@ -1,6 +1,5 @@
-// Included by flash_inst_<DK>_<DV>.hip with DLT_DK / DLT_DV defined: dense flash kernels for
-// one pair of padded head dims.
-#include <cstdlib>
+// Included by flash_{fwd,dq,dkv}_<DK>_<DV>.hip with DLT_DK / DLT_DV defined: flash kernels for one pair of padded head dims;
+// DLT_FLASH_PART 0: forward, 1: dQ, 2: dK/dV (units of their own, since they take minutes to compile).
 #include "flash_dma_kernel.hpp"
 
 #define DLT_FCAT3_(a, b, c) a##b##_##c
@@ -29,12 +28,6 @@ namespace {
 #define FLASHD_BWD_NW 4
 #endif
 
-// DLT_FLASH_SYNC_STAGING=1 keeps the register-staged kernels for every class (A/B timing)
-inline bool flash_async_staging() {
-  static const bool on = [] { const char* e = std::getenv("DLT_FLASH_SYNC_STAGING"); return !(e != nullptr && e[0] == '1'); }();
-  return on;
-}
-
 // PAD of the asynchronously staged kernels for head dims dk, dv: 2 where the class's 128 dims hold 96 at most, 3 where they hold 80
 // (all sides measured at flashd_dims)
 inline int flashd_pad(int dk, int dv) {
@@ -46,6 +39,7 @@ inline int flashd_pad(int dk, int dv) {
 template <typename KernT>
 int flash_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
+#if DLT_FLASH_PART == 0
 template <typename TIO, int MODE, int NP, int CK, int NW>
 int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
@@ -64,7 +58,7 @@ int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk = (a.Lq + own - 1) / own;
   dlt_timing_before(DLT_K_FWD, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk * a.share.n), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash forward launch");
   return DLT_OK;
@@ -76,7 +70,7 @@ int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
     // dense / causal, head dims that are multiples of 8: chunks are copied HBM -> LDS asynchronously.  Measured per
     // class and mode against the register-staged kernel: dense -2 % (64/64), -4 % (64/128), -7 % (128/128); causal -4 %
     // (64/64), -18 % (128/128); head dims below the class (80/80, 96/96): -18 % on the step.
-    if (a.dk % 8 == 0 && a.dv % 8 == 0 && flash_async_staging()) {
+    if (a.dk % 8 == 0 && a.dv % 8 == 0 && dlt_flash_async()) {
       if (a.slim) return flashd_launch_fwd<TIO, MODE, 1, 64, 8>(a, stream);
       return flashd_launch_fwd<TIO, MODE, FLASHD_FWD_NP, FLASHD_FWD_CK(DLT_DK, DLT_DV), FLASHD_FWD_NW(DLT_DK, DLT_DV)>(a, stream);
     }
@@ -98,7 +92,13 @@ int flash_launch_fwd_t(const FlashArgs& a, int grid, hipStream_t stream) {
   if (a.tile) return a.tm.img ? flash_launch_fwd_c<TIO, 3>(a, grid, stream) : flash_launch_fwd_c<TIO, 2>(a, grid, stream);
   return a.causal ? flash_launch_fwd_c<TIO, 1>(a, grid, stream) : flash_launch_fwd_c<TIO, 0>(a, grid, stream);
 }
+}  // namespace
 
+int DLT_FCAT3(dlt_flash_launch_fwd_, DLT_DK, DLT_DV)(const FlashArgs& a, int dtype, int grid, hipStream_t stream) {
+  return dtype == DLT_BF16 ? flash_launch_fwd_t<bf16_t>(a, grid, stream) : flash_launch_fwd_t<f16_t>(a, grid, stream);
+}
+
+#elif DLT_FLASH_PART == 1
 template <typename TIO, int MODE, int NP, int NW>
 int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
@@ -117,12 +117,45 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk_q = (a.Lq + own - 1) / own;
   dlt_timing_before(DLT_K_BWD_Q, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q * a.share_q.n), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash dQ launch");
   return DLT_OK;
 }
 
+template <typename TIO, int MODE>
+int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
+  if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
+    if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && dlt_flash_async()) {
+      // few workgroups: one own block per wave, in 4 waves (twice the workgroups) or, without a mask, 8 (see flash_backward)
+      if (a.slim_q == 4) return flashd_launch_bwd_q<TIO, MODE, 1, 4>(a, stream);
+      if constexpr (MODE == 0)
+        if (a.slim_q == 8) return flashd_launch_bwd_q<TIO, MODE, 1, 8>(a, stream);
+      return flashd_launch_bwd_q<TIO, MODE, FLASHD_DQ_NP(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
+    }
+  }
+  auto kern = flash_bwd_q_kernel<TIO, DLT_DK, DLT_DV, flash_np_q(DLT_DK, DLT_DV), flash_ck_q(DLT_DK, DLT_DV), MODE>;
+  int rc = flash_set_lds(kern, a.lds_q);
+  if (rc != DLT_OK) return rc;
+  dlt_timing_before(DLT_K_BWD_Q, stream);
+  hipLaunchKernelGGL(kern, dim3(grid_q), dim3(256), a.lds_q, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("flash dQ launch");
+  return DLT_OK;
+}
+
+template <typename TIO>
+int flash_launch_bwd_q_t(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
+  if (a.tile) return a.tm.img ? flash_launch_bwd_q_c<TIO, 3>(a, grid_q, stream) : flash_launch_bwd_q_c<TIO, 2>(a, grid_q, stream);
+  return a.causal ? flash_launch_bwd_q_c<TIO, 1>(a, grid_q, stream) : flash_launch_bwd_q_c<TIO, 0>(a, grid_q, stream);
+}
+}  // namespace
+
+int DLT_FCAT3(dlt_flash_launch_bwd_q_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, int dtype, int grid_q, hipStream_t stream) {
+  return dtype == DLT_BF16 ? flash_launch_bwd_q_t<bf16_t>(a, grid_q, stream) : flash_launch_bwd_q_t<f16_t>(a, grid_q, stream);
+}
+
+#else
 template <typename TIO, int MODE, int NP, int NW>
 int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
@@ -141,30 +174,9 @@ int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk_k = (a.Lk + own - 1) / own;
   dlt_timing_before(DLT_K_BWD_KV, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k * a.share_kv.n), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash dK/dV launch");
-  return DLT_OK;
-}
-
-template <typename TIO, int MODE>
-int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
-  if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
-    if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && flash_async_staging()) {
-      // few workgroups: one own block per wave, in 4 waves (twice the workgroups) or, without a mask, 8 (see flash_backward)
-      if (a.slim_q == 4) return flashd_launch_bwd_q<TIO, MODE, 1, 4>(a, stream);
-      if constexpr (MODE == 0)
-        if (a.slim_q == 8) return flashd_launch_bwd_q<TIO, MODE, 1, 8>(a, stream);
-      return flashd_launch_bwd_q<TIO, MODE, FLASHD_DQ_NP(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
-    }
-  }
-  auto kern = flash_bwd_q_kernel<TIO, DLT_DK, DLT_DV, flash_np_q(DLT_DK, DLT_DV), flash_ck_q(DLT_DK, DLT_DV), MODE>;
-  int rc = flash_set_lds(kern, a.lds_q);
-  if (rc != DLT_OK) return rc;
-  dlt_timing_before(DLT_K_BWD_Q, stream);
-  hipLaunchKernelGGL(kern, dim3(grid_q), dim3(256), a.lds_q, stream, a);
-  dlt_timing_after(stream);
-  DLT_CHECK_LAUNCH("flash dQ launch");
   return DLT_OK;
 }
 
@@ -173,8 +185,7 @@ int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     // dense / causal, head dims that are multiples of 8: chunks are copied HBM -> LDS asynchronously (in tile mode,
     // where whole blocks are skipped, the register-staged kernel measured 1.5 % faster)
-    const bool scalars_fit = a.ls[2] >= 0 && ((int64_t)a.Lq - 1) * a.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1);   // 32-bit offsets of the lse2 / delta copies
-    if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && scalars_fit && flash_async_staging()) {
+    if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && dlt_flash_scalars_fit(a) && dlt_flash_async()) {
       if (a.slim) return flashd_launch_bwd_kv<TIO, MODE, 1, 4>(a, stream);
       return flashd_launch_bwd_kv<TIO, MODE, flash_np_kv(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
@@ -191,12 +202,6 @@ int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream
   return DLT_OK;
 }
 
-// dQ is launched first: with fuse_delta it produces the delta vector the dK/dV kernel consumes
-template <typename TIO>
-int flash_launch_bwd_q_t(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
-  if (a.tile) return a.tm.img ? flash_launch_bwd_q_c<TIO, 3>(a, grid_q, stream) : flash_launch_bwd_q_c<TIO, 2>(a, grid_q, stream);
-  return a.causal ? flash_launch_bwd_q_c<TIO, 1>(a, grid_q, stream) : flash_launch_bwd_q_c<TIO, 0>(a, grid_q, stream);
-}
 template <typename TIO>
 int flash_launch_bwd_kv_t(const FlashBwdArgs& a, int grid_kv, hipStream_t stream) {
   if (a.tile) return a.tm.img ? flash_launch_bwd_kv_c<TIO, 3>(a, grid_kv, stream) : flash_launch_bwd_kv_c<TIO, 2>(a, grid_kv, stream);
@@ -204,14 +209,7 @@ int flash_launch_bwd_kv_t(const FlashBwdArgs& a, int grid_kv, hipStream_t stream
 }
 }  // namespace
 
-int DLT_FCAT3(dlt_flash_launch_bwd_q_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, int dtype, int grid_q, hipStream_t stream) {
-  return dtype == DLT_BF16 ? flash_launch_bwd_q_t<bf16_t>(a, grid_q, stream) : flash_launch_bwd_q_t<f16_t>(a, grid_q, stream);
-}
-
 int DLT_FCAT3(dlt_flash_launch_bwd_kv_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, int dtype, int grid_kv, hipStream_t stream) {
   return dtype == DLT_BF16 ? flash_launch_bwd_kv_t<bf16_t>(a, grid_kv, stream) : flash_launch_bwd_kv_t<f16_t>(a, grid_kv, stream);
 }
-
-int DLT_FCAT3(dlt_flash_launch_fwd_, DLT_DK, DLT_DV)(const FlashArgs& a, int dtype, int grid, hipStream_t stream) {
-  return dtype == DLT_BF16 ? flash_launch_fwd_t<bf16_t>(a, grid, stream) : flash_launch_fwd_t<f16_t>(a, grid, stream);
-}
+#endif

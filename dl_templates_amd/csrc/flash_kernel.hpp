@@ -218,6 +218,14 @@ inline int flash_causal_group(int L, int dk, int dv) {
   return (int)(g < 1 ? 1 : (g > 16 ? 16 : g));
 }
 
+// The streamed side of an own block split over `n` workgroups (dense, asynchronously staged kernels): share i takes the tokens from i `len` on,
+// `len` of them (a multiple of the chunk), the last one the rest.  Results then go to `part`, fp32 rows [batch * head][share][own
+// token][head dim], and a second launch sums them (flash_share.hip).  n = 1: no split.
+struct FlashShare {
+  float* part;
+  int32_t n, len;
+};
+
 struct FlashArgs {
   const void *q, *k, *v;
   void* o;
@@ -233,7 +241,23 @@ struct FlashArgs {
   int32_t o_vec;
   int32_t lds_bytes;
   float scale_log2;
+  FlashShare share;   // part: behind its rows the {maximum, sum} of each
 };
+
+// first of the `rows` partial rows of one share
+DLT_DEV int64_t flash_share_row(const FlashShare& s, int bh, int share, int rows) { return ((int64_t)bh * s.n + share) * rows; }
+// accumulators in C layout (lane n = own token x, dims 16 d + 4 g ...) -> partial rows of `dact` dims (a multiple of 8)
+template <int NP, int NA>
+DLT_DEV void flash_share_put(float* rows, const f32x4 (&acc)[NP][NA], int dact, int x, int len, int g) {
+#pragma unroll
+  for (int p = 0; p < NP; p++)
+    if (x + 16 * p < len) {
+      float* r = rows + (int64_t)(x + 16 * p) * dact + 4 * g;
+#pragma unroll
+      for (int d = 0; d < NA; d++)
+        if (16 * d + 4 * g < dact) *reinterpret_cast<f32x4*>(r + 16 * d) = acc[p][d];
+    }
+}
 
 template <typename TIO, int DK, int DV, int NP, int CK, int MODE>
 __global__ __launch_bounds__(256, flash_occ_fwd(DK, DV)) void flash_fwd_kernel(const FlashArgs a) {
@@ -529,7 +553,11 @@ struct FlashBwdArgs {
   int32_t dq_vec, dk_vec, dv_vec;
   int32_t lds_q, lds_kv;
   float scale_log2, sm_scale;
+  FlashShare share_q, share_kv;   // dQ; dK/dV (rows of dK, then those of dV)
 };
+
+// lse2 / delta of a slab lie within 32-bit byte offsets: the asynchronously staged dK/dV kernel copies them
+inline bool dlt_flash_scalars_fit(const FlashBwdArgs& a) { return a.ls[2] >= 0 && ((int64_t)a.Lq - 1) * a.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1); }
 
 // Staging of one chunk of CK tokens of two [token][dim] tensors (dims DA and DB) through registers.
 template <int DA, int DB, int CK>

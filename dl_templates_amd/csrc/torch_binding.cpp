@@ -207,6 +207,22 @@ Spec flash_spec(const Tensor& q, const Tensor& k, const Tensor& v, bool causal, 
   return s;
 }
 
+// Partial results of a flash pass that splits its other side: from the caching allocator, on the call's stream, for the call alone.
+struct Workspace {
+  Tensor t;
+  void* ptr = nullptr;
+  int64_t bytes = 0;
+};
+Workspace flash_workspace(const dlt_flash_shape_t& shape, int backward, const Tensor& like) {
+  Workspace w;
+  check_rc(dlt_flash_workspace(&shape, backward, &w.bytes));
+  if (w.bytes > 0) {
+    w.t = empty({w.bytes / 4}, at::kFloat, like);
+    w.ptr = w.t.mutable_data_ptr();
+  }
+  return w;
+}
+
 struct Forward { Tensor o, lse, q_rot, k_rot; };
 
 // keep_rot: the rotated q and k are stored as well (for the backward pass)
@@ -219,8 +235,9 @@ Forward run_forward(const Spec& s, const Tensor& q, const Tensor& k, const Tenso
   if (s.op == Op::Flash) {
     f.o = empty({q.size(0), q.size(1), q.size(2), v.size(3)}, dt, q);
     f.lse = empty({q.size(0), q.size(1), q.size(2)}, at::kFloat, q);
-    check_rc(dlt_flash_fwd(q.const_data_ptr(), st(q), k.const_data_ptr(), st(k), v.const_data_ptr(), st(v), f.o.mutable_data_ptr(), st(f.o),
-                           (float*)f.lse.mutable_data_ptr(), st(f.lse), &s.flash, stream));
+    const Workspace ws = flash_workspace(s.flash, 0, q);
+    check_rc(dlt_flash_fwd_ws(q.const_data_ptr(), st(q), k.const_data_ptr(), st(k), v.const_data_ptr(), st(v), f.o.mutable_data_ptr(), st(f.o),
+                              (float*)f.lse.mutable_data_ptr(), st(f.lse), &s.flash, ws.ptr, ws.bytes, stream));
     return f;
   }
   if (s.op == Op::Image) {
@@ -258,7 +275,10 @@ std::array<Tensor, 3> run_backward(const Spec& s, const Tensor& q, const Tensor&
                 dk.mutable_data_ptr(), st(dk), dv.mutable_data_ptr(), st(dv), shape..., stream));
   };
   const dlt_rope_t* none = nullptr;
-  if (s.op == Op::Flash) call(dlt_flash_bwd, &s.flash);
+  if (s.op == Op::Flash) {
+    const Workspace ws = flash_workspace(s.flash, 1, q);
+    call(dlt_flash_bwd_ws, &s.flash, ws.ptr, ws.bytes);
+  }
   else if (s.op == Op::Image) call(dlt_swa_bwd_image, &s.swa, &s.tile, none);
   else if (rotated) call(dlt_swa_bwd_rot, &s.swa, (const dlt_rope_t*)&rope->d);
   else call(dlt_swa_bwd, &s.swa, rope ? (const dlt_rope_t*)&rope->d : none);

@@ -241,13 +241,32 @@ int dlt_flash_bwd(const void* q, const int64_t q_strides[4], const void* k, cons
                   void* dv, const int64_t dv_strides[4],
                   const dlt_flash_shape_t* shape, void* stream);
 
+/* The same calls with a workspace.  Dense passes whose own side (queries in the forward pass and for dQ, keys for dK / dV) is too
+ * short to fill the chip split their other side over workgroups; each leaves fp32 partial results in `ws`, which a second
+ * launch sums in a fixed order.  dlt_flash_workspace() says how many bytes a shape's pass needs (0: it is not split); the
+ * split follows from Lq, Lk, dk and dv alone.  `ws` is 16-byte aligned device memory whose contents need not be set and are
+ * of no use afterwards; it belongs to the call until its kernels have run.  With ws == NULL nothing is split, as in
+ * dlt_flash_fwd / dlt_flash_bwd; results of the two ways differ by the rounding of another order of summation. */
+int dlt_flash_workspace(const dlt_flash_shape_t* shape, int backward, int64_t* bytes);
+int dlt_flash_fwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                     const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
+                     float* lse2, const int64_t lse_strides[3],
+                     const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream);
+int dlt_flash_bwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                     const void* v, const int64_t v_strides[4], const void* o, const int64_t o_strides[4],
+                     const void* d_o, const int64_t do_strides[4],
+                     const float* lse2, float* delta, const int64_t lse_strides[3],
+                     void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
+                     void* dv, const int64_t dv_strides[4],
+                     const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream);
+
 /* ---- per-kernel timing (measurement aid) ---------------------------------------------------
  * Counterpart of the reference's triton.testing.do_bench calls (src/tiled_swa.py:765-774,
  * src/flash_attn.py:592,606), at kernel granularity.  While enabled for the calling thread,
  * every kernel the library launches is bracketed by a pair of hipEvents recorded on the
  * launch stream.  A backward launch that forms dq, dk and dv together (tiles of 16 tokens with a 3 x 3
  * window, head dim 32 / 64; narrow grids at 32 excepted) is recorded as DLT_K_BWD_KV, without a
- * DLT_K_BWD_Q beside it.  dlt_timing_collect waits for the recorded events, writes up to `max`
+ * DLT_K_BWD_Q beside it.  A flash pass split with a workspace gives a second record of its kind for the sum.  dlt_timing_collect waits for the recorded events, writes up to `max`
  * records in launch order, stores the number available in *n and clears the list.
  * Enabling creates events lazily (host-side handles only, no device allocation). */
 enum { DLT_K_ROPE = 0, DLT_K_FWD = 1, DLT_K_DELTA = 2, DLT_K_BWD_KV = 3, DLT_K_BWD_Q = 4, DLT_K_COUNT = 5 };

@@ -114,3 +114,28 @@ def test_operators_are_autograd_functions():
     for op in (TiledSwa, TiledSwaRope, TiledSwaImage, RotaryPE2D, _attention):
         assert issubclass(op, torch.autograd.Function)
         assert "forward" in vars(op) and "backward" in vars(op)
+
+
+def test_flash_workspace_of_a_shape():
+    L = _lib()
+    lib = L.load()
+
+    def need(backward, *shape):
+        n = ctypes.c_int64(-1)
+        assert lib.dlt_flash_workspace(L.FlashShape(*shape), backward, ctypes.byref(n)) == 0, lib.dlt_last_error()
+        return n.value
+    # 64 queries x 4000 keys: 8 shares of a forward pass (64 output dims, maximum and sum), of dQ 7 (512 keys each but the last)
+    assert need(0, 1, 2, 64, 4000, 64, 64, 0.1, 0, 0) == 4 * 2 * 8 * 64 * (64 + 2)
+    assert need(1, 1, 2, 64, 4000, 64, 64, 0.1, 0, 0) == 4 * 2 * 8 * 64 * 64
+    assert need(1, 1, 1, 4000, 64, 64, 64, 0.1, 0, 0) % (4 * 64 * 128) == 0
+    # nothing is split under a mask, for balanced sides, in fp32, at odd head dims and outside the classes of 64 and 128
+    for shape in ((1, 1, 4000, 4000, 64, 64, 0.1, 1, 0), (1, 1, 2048, 2048, 64, 64, 0.1, 0, 0), (1, 1, 64, 4000, 64, 64, 0.1, 0, 2),
+                  (1, 1, 64, 4000, 60, 64, 0.1, 0, 0), (1, 1, 64, 4000, 32, 32, 0.1, 0, 0), (1, 1, 64, 4000, 136, 136, 0.1, 0, 0)):
+        assert need(0, *shape) == 0 and need(1, *shape) == 0
+    n = ctypes.c_int64()
+    assert lib.dlt_flash_workspace(L.FlashShape(1, 1, 8, 16, 64, 64, 1.0, 1, 0), 0, ctypes.byref(n)) == 1   # causal, Lq != Lk
+    assert lib.dlt_flash_workspace(L.FlashShape(1, 1, 8, 16, 64, 64, 1.0, 0, 0), 0, None) == 1
+    one, st4, st3 = ctypes.c_void_p(16), (ctypes.c_int64 * 4)(4096, 4096, 64, 1), (ctypes.c_int64 * 3)(64, 64, 1)
+    for ws, size, word in ((16, 100, b"needed"), (20, 1 << 30, b"aligned")):
+        rc = lib.dlt_flash_fwd_ws(one, st4, one, st4, one, st4, one, st4, one, st3, L.FlashShape(1, 1, 64, 4000, 64, 64, 0.1, 0, 0), ctypes.c_void_p(ws), size, None)
+        assert rc == 1 and word in lib.dlt_last_error()

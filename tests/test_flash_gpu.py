@@ -398,3 +398,37 @@ def test_head_dims_of_up_to_96(dk, dv, causal):
         for g, w in zip(got, want):
             assert torch.equal(g, g[:, :1].expand_as(g))
             assert _rel(g[:, :1], w) <= 1e-2
+
+
+# other sides cut into shares over several workgroups: a token past a share's end and one before it, a last share of a few tokens, own sides that
+# end inside a workgroup, every class, 2 ... 8 shares, one own block per wave and two
+@pytest.mark.parametrize("Lq,Lk,dk,dv,counts", [
+    (33, 2560, 64, 64, (1, 20)), (129, 2689, 64, 128, (1, 40)), (128, 1281, 128, 128, (1, 90)), (300, 2500, 80, 72, (1, 60)), (700, 4097, 64, 64, (1, 30)),
+    (2600, 90, 64, 64, (1, 40)), (1700, 65, 64, 128, (1, 90)), (1281, 130, 128, 128, (1, 40)), (2100, 200, 96, 40, (1, 60)), (64, 2000, 104, 128, (1, 16))])
+def test_other_side_in_shares(Lq, Lk, dk, dv, counts):
+    scale = 1 / math.sqrt(dk)
+    q, k, v, do = orc.make_qkv(Lq + Lk + dk, 1, 1, Lq, Lk, dk, dv, torch.float16)
+    want = orc.flash_grads(q.float(), k.float(), v.float(), do.float(), False, scale)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    o = _fa().attention(*leaves, False, scale)
+    # fp16 probabilities and results: 1e-2 of the largest value, as for the other kernels
+    for g, w in zip((o,) + torch.autograd.grad(o, leaves, do.cuda()), want):
+        assert _rel(g, w) <= 1e-2
+    _, M = _fa()._forward(q.cuda(), k.cuda(), v.cuda(), False, scale)
+    assert (M.cpu() - orc.flash_lse2(q, k, scale, False)).abs().max().item() <= 2e-2
+    test_a_slab_has_the_same_bits_in_any_call(False, Lq, Lk, dk, dv, counts)
+
+
+# a share whose scores are all -inf or hold NaN / inf, and an infinite key in one share: what the whole row gives
+def test_shares_with_infinite_and_nan_scores():
+    Lq, Lk, d = 40, 3000, 64
+    q, k, v, _ = (t.cuda() for t in orc.make_qkv(3, 1, 4, Lq, Lk, d, d, torch.float16))
+    q[:, :, :, 0] = 1.0
+    k[:, 1, :1500, 0] = -float("inf")     # the first shares of head 1 score -inf
+    k[:, 2, 7, 0] = float("nan")
+    v[:, 3, 2990, 5] = float("inf")
+    o, M = _fa()._forward(q, k, v, False, 0.125)
+    kf, vf = k[:, 1, 1500:].float(), v[:, 1, 1500:].float()
+    want = torch.softmax(torch.matmul(q[:, 1].float(), kf.transpose(-1, -2).contiguous()) * 0.125, -1) @ vf
+    assert torch.isfinite(M[:, :2]).all() and _rel(o[:, 1], want.cpu()) <= 1e-2
+    assert torch.isnan(o[:, 2]).all() and torch.isinf(o[:, 3, :, 5]).all() and torch.isfinite(o[:, 3, :, :5]).all() and torch.isfinite(o[:, 0]).all()
