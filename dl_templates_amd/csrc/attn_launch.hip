@@ -22,9 +22,13 @@ int dlt_launch_bwd_64_128(const BwdArgs&, int, const BwdArgs&, int, int, hipStre
 int dlt_launch_bwd_256_256(const BwdArgs&, int, const BwdArgs&, int, int, hipStream_t);
 
 int dlt_flash_launch_fwd_32_32(const FlashArgs&, int, int, hipStream_t);
+int dlt_flash_launch_fwdc_32_32(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_fwd_64_64(const FlashArgs&, int, int, hipStream_t);
+int dlt_flash_launch_fwdc_64_64(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_fwd_128_128(const FlashArgs&, int, int, hipStream_t);
+int dlt_flash_launch_fwdc_128_128(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_fwd_64_128(const FlashArgs&, int, int, hipStream_t);
+int dlt_flash_launch_fwdc_64_128(const FlashArgs&, int, int, hipStream_t);
 int dlt_flash_launch_bwd_q_32_32(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
 int dlt_flash_launch_bwd_kv_32_32(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
 int dlt_flash_launch_bwd_q_64_64(const FlashBwdArgs&, int dtype, int grid, hipStream_t);
@@ -550,7 +554,7 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
 // Which kernels a dense / causal pass runs on:
 //   CHUNKED: the streamed side passes through LDS chunk by chunk, 32 own tokens per wave (64 ... 256 per workgroup);
 //   SLIM:    the same with 16 own tokens per wave: half the work per wave and chunk.  Forward 8 waves (twice the workgroups of 64/128 and
-//            128/128), backward 4 (twice the workgroups);
+//            128/128) or 4 (flash_forward), backward 4 (twice the workgroups);
 //   SPLIT1, SPLIT2: the streamed side is split over the waves of workgroups that own one or two blocks of 16 tokens
 //            (csrc/flash_split_kernel.hpp).
 // CHUNKED wins once its workgroups fill the chip.  Below that the time of a chunked pass is a start and the chunks of 64 streamed
@@ -659,7 +663,7 @@ FlashPlan flash_plan(int pass, const DimClass& dc, int dims, int64_t bh, int own
   if (may_split && !causal) {
     // other side of at least `least` tokens and `times` the own one; a, 4 b
     static const struct { int least, times, a, b4; } RULE[3][4] = {   // by pass; 64/64, 64/128, 128/128 with up to 192 dims in all, 128/128
-        {{2500, 3, 150, 4}, {2500, 3, 500, 3}, {2500, 3, 150, 4}, {1200, 3, 150, 6}},
+        {{2500, 3, 150, 5}, {2500, 3, 500, 5}, {2500, 3, 150, 5}, {1200, 3, 150, 6}},
         {{1600, 1, 350, 4}, {600, 1, 150, 4}, {1600, 1, 150, 4}, {600, 4, 150, 6}},
         {{2500, 1, 150, 6}, {1600, 4, 250, 4}, {2000, 1, 500, 4}, {1200, 4, 150, 8}}};
     const auto& r = RULE[pass][dc.id == 0 ? 0 : dc.id == 2 ? 1 : dims <= 192 ? 2 : 3];
@@ -704,7 +708,7 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   a.nblk = (a.Lq + own - 1) / own;
   a.causal = p.g.mode == DLT_GEOM_CAUSAL;
   a.causal_group = flash_causal_group(a.Lk, p.dk, p.dv);
-  a.slim = 0;
+  a.slim = 0; a.chunk = 64;
   a.tile = p.g.mode == DLT_GEOM_SWA;
   a.g = p.g;
   a.o_vec = tvec_ok(t.out_o, t.os, p.dv, 2);
@@ -718,12 +722,24 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   if (p.g.mode != DLT_GEOM_SWA) {
     const FlashPlan f = flash_plan(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0, t.part != nullptr && flash_may_split(p, dc));
     np = f.kind;
-    a.slim = np == FLASH_SLIM;
+    // One own block per wave, with the bits of the kernel it stands for: 8 waves (workgroups of 128 queries) or, while workgroups of 64 all
+    // run at once, one per CU (two under a mask, where the work is uneven), 4 waves.  Slim workgroups, 8 waves -> 4: 0.83 ... 0.89 of
+    // the time up to one per CU (head dims of 80: 0.92 ... 0.96), under a mask 0.80 ... 0.88 and 0.83 ... 0.96 up to two; beyond 1.0 and
+    // more.  Chunked ones of 64/128 and 128/128 (from 3072 queries on; two blocks on 8 waves): 4 waves 0.53 ... 0.64 up to one workgroup of 64 per
+    // CU, then 8 waves 0.65 ... 0.76 up to one of 128, under a mask 0.62 ... 0.70 and 0.66 ... 0.85 up to two (4 slabs of 7232, causal,
+    // 64/128: 151 -> 78 us)
+    const int64_t cus = dlt_device_cus(), nbh = (int64_t)p.B * p.H * f.n, most = a.causal ? 2 * cus : cus;
+    const bool long_chunks = np == FLASH_CHUNKED && dc.DV == 128;
+    const bool four = nbh * ((a.Lq + 63) / 64) <= (long_chunks ? cus : most);
+    a.chunk = long_chunks ? 128 : 64;
+    a.slim = np == FLASH_SLIM ? (four ? 4 : 8) : long_chunks ? (four ? 4 : nbh * ((a.Lq + 127) / 128) <= most ? 8 : 0) : 0;
     a.share.n = f.n; a.share.len = f.len;
   }
   const bool split = np == FLASH_SPLIT1 || np == FLASH_SPLIT2;
   int rc;
-#define DLT_FLASH_FWD(C) rc = split ? dlt_flashs_fwd_##C(a, p.dtype, np, stream) : dlt_flash_launch_fwd_##C(a, p.dtype, (int)grid, stream); break
+#define DLT_FLASH_FWD(C) \
+  rc = split ? dlt_flashs_fwd_##C(a, p.dtype, np, stream) : a.causal ? dlt_flash_launch_fwdc_##C(a, p.dtype, (int)grid, stream) : dlt_flash_launch_fwd_##C(a, p.dtype, (int)grid, stream); \
+  break
   switch (dc.id) {
     case 0: DLT_FLASH_FWD(64_64);
     case 1: DLT_FLASH_FWD(128_128);

@@ -1,0 +1,4 @@
+#define DLT_DK 128
+#define DLT_DV 128
+#define DLT_FLASH_PART 3
+#include "flash_inst.hpp"

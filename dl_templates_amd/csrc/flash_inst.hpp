@@ -1,5 +1,5 @@
-// Included by flash_{fwd,dq,dkv}_<DK>_<DV>.hip with DLT_DK / DLT_DV defined: flash kernels for one pair of padded head dims;
-// DLT_FLASH_PART 0: forward, 1: dQ, 2: dK/dV (units of their own, since they take minutes to compile).
+// Included by flash_{fwd,fwdc,dq,dkv}_<DK>_<DV>.hip with DLT_DK / DLT_DV defined: flash kernels for one pair of padded head dims;
+// DLT_FLASH_PART 0: forward, 3: forward under a mask, 1: dQ, 2: dK/dV (units of their own, since they take minutes to compile).
 #include "flash_dma_kernel.hpp"
 
 #define DLT_FCAT3_(a, b, c) a##b##_##c
@@ -39,7 +39,7 @@ inline int flashd_pad(int dk, int dv) {
 template <typename KernT>
 int flash_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
-#if DLT_FLASH_PART == 0
+#if DLT_FLASH_PART == 0 || DLT_FLASH_PART == 3
 template <typename TIO, int MODE, int NP, int CK, int NW>
 int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
@@ -71,7 +71,11 @@ int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
     // class and mode against the register-staged kernel: dense -2 % (64/64), -4 % (64/128), -7 % (128/128); causal -4 %
     // (64/64), -18 % (128/128); head dims below the class (80/80, 96/96): -18 % on the step.
     if (a.dk % 8 == 0 && a.dv % 8 == 0 && dlt_flash_async()) {
-      if (a.slim) return flashd_launch_fwd<TIO, MODE, 1, 64, 8>(a, stream);
+      // few workgroups: one own block per wave (see flash_forward)
+      if constexpr (DLT_DV == 128)
+        if (a.slim != 0 && a.chunk == 128)
+          return a.slim == 4 ? flashd_launch_fwd<TIO, MODE, 1, 128, 4>(a, stream) : flashd_launch_fwd<TIO, MODE, 1, 128, 8>(a, stream);
+      if (a.slim != 0) return a.slim == 4 ? flashd_launch_fwd<TIO, MODE, 1, 64, 4>(a, stream) : flashd_launch_fwd<TIO, MODE, 1, 64, 8>(a, stream);
       return flashd_launch_fwd<TIO, MODE, FLASHD_FWD_NP, FLASHD_FWD_CK(DLT_DK, DLT_DV), FLASHD_FWD_NW(DLT_DK, DLT_DV)>(a, stream);
     }
   }
@@ -87,16 +91,24 @@ int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
   return DLT_OK;
 }
 
+#if DLT_FLASH_PART == 0
 template <typename TIO>
 int flash_launch_fwd_t(const FlashArgs& a, int grid, hipStream_t stream) {
   if (a.tile) return a.tm.img ? flash_launch_fwd_c<TIO, 3>(a, grid, stream) : flash_launch_fwd_c<TIO, 2>(a, grid, stream);
-  return a.causal ? flash_launch_fwd_c<TIO, 1>(a, grid, stream) : flash_launch_fwd_c<TIO, 0>(a, grid, stream);
+  return flash_launch_fwd_c<TIO, 0>(a, grid, stream);
 }
 }  // namespace
 
 int DLT_FCAT3(dlt_flash_launch_fwd_, DLT_DK, DLT_DV)(const FlashArgs& a, int dtype, int grid, hipStream_t stream) {
   return dtype == DLT_BF16 ? flash_launch_fwd_t<bf16_t>(a, grid, stream) : flash_launch_fwd_t<f16_t>(a, grid, stream);
 }
+#else
+}  // namespace
+
+int DLT_FCAT3(dlt_flash_launch_fwdc_, DLT_DK, DLT_DV)(const FlashArgs& a, int dtype, int grid, hipStream_t stream) {
+  return dtype == DLT_BF16 ? flash_launch_fwd_c<bf16_t, 1>(a, grid, stream) : flash_launch_fwd_c<f16_t, 1>(a, grid, stream);
+}
+#endif
 
 #elif DLT_FLASH_PART == 1
 template <typename TIO, int MODE, int NP, int NW>

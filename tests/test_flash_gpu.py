@@ -432,3 +432,23 @@ def test_shares_with_infinite_and_nan_scores():
     want = torch.softmax(torch.matmul(q[:, 1].float(), kf.transpose(-1, -2).contiguous()) * 0.125, -1) @ vf
     assert torch.isfinite(M[:, :2]).all() and _rel(o[:, 1], want.cpu()) <= 1e-2
     assert torch.isnan(o[:, 2]).all() and torch.isinf(o[:, 3, :, 5]).all() and torch.isfinite(o[:, 3, :, :5]).all() and torch.isfinite(o[:, 0]).all()
+
+
+# forward passes with one own block per wave, 4 waves or 8, 64-key chunks and (from 3072 queries on, 64/128 and 128/128) 128-key ones: counts on every side
+# of the lines, chunk remainders, a token past a workgroup's end, every class and dims below it
+@pytest.mark.parametrize("causal,Lq,Lk,dk,dv,counts", [
+    (False, 1030, 705, 64, 64, (1, 15, 16)), (False, 705, 1090, 128, 128, (1, 21, 22)), (False, 3100, 193, 64, 128, (1, 6, 12)), (False, 3073, 260, 96, 104, (1, 6, 12)),
+    (False, 3137, 129, 80, 80, (1, 5, 12)), (True, 1030, 1030, 64, 64, (1, 30, 31)), (True, 800, 800, 48, 128, (1, 39, 40)), (True, 3100, 3100, 64, 128, (1, 6, 21)),
+    (True, 3073, 3073, 128, 128, (1, 6, 21)), (True, 3201, 3201, 80, 72, (1, 5, 21))])
+def test_one_own_block_per_wave_forward(causal, Lq, Lk, dk, dv, counts):
+    scale = 1 / math.sqrt(dk)
+    q, k, v, _ = (t.cuda() for t in orc.make_qkv(Lq + Lk + dk, 1, max(counts), Lq, Lk, dk, dv, torch.float16))
+    o, M = _fa()._forward(q, k, v, causal, scale)
+    s = torch.matmul(q[:, -1].float(), k[:, -1].float().transpose(-1, -2).contiguous()) * scale
+    if causal:
+        s = s.masked_fill(torch.ones(Lq, Lk, dtype=torch.bool, device="cuda").triu(1), -math.inf)
+    assert _rel(o[:, -1], (torch.softmax(s, -1) @ v[:, -1].float()).cpu()) <= 1e-2
+    assert (M[:, -1] - torch.logsumexp(s, -1) / math.log(2)).abs().max().item() <= 2e-2
+    for n in counts[:-1]:
+        got = _fa()._forward(q[:, -n:].contiguous(), k[:, -n:].contiguous(), v[:, -n:].contiguous(), causal, scale)
+        assert torch.equal(got[0], o[:, -n:]) and torch.equal(got[1], M[:, -n:])
