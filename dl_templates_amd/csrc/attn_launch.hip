@@ -657,14 +657,15 @@ int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int 
 // slab's shape alone (see above), as other / (a + b own) up to 8: the lines were fitted to 2100 shapes of 4 ... 128 slabs (n = 2, 3, 4, 6, 8), a loss
 // counted eightfold.  Inside them, not split -> split, geometric mean of the pass by slabs (4, 8, 16, 32, 64, 128): forward 1.7 ... 2.2,
 // 1.55 ... 2.0, 1.33 ... 1.8, 1.22 ... 1.6, 1.2, 1.15; both backward passes together 1.4 ... 1.8 down to 1.05 ... 1.3.  Shorter other sides and
-// longer own ones lose more to the sums than idle CUs cost (128 slabs of 734 x 3321, 64/64: 98 -> 144 us with n = 4).
+// longer own ones lose more to the sums than idle CUs cost (128 slabs of 734 x 3321, 64/64: 98 -> 144 us with n = 4).  Over 1500 drawn
+// calls of 4 ... 128 slabs the slowest lose 10 % (128 of 802 x 4159, 80/80: 221 -> 242; 64 of 2011 x 400, 128/128, both directions: 170 -> 190).
 struct FlashPlan { int kind, n, len; };
 FlashPlan flash_plan(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal, bool may_split) {
   if (may_split && !causal) {
     // other side of at least `least` tokens and `times` the own one; a, 4 b
     static const struct { int least, times, a, b4; } RULE[3][4] = {   // by pass; 64/64, 64/128, 128/128 with up to 192 dims in all, 128/128
-        {{2500, 3, 150, 5}, {2500, 3, 500, 5}, {2500, 3, 150, 5}, {1200, 3, 150, 6}},
-        {{1600, 1, 350, 4}, {600, 1, 150, 4}, {1600, 1, 150, 4}, {600, 4, 150, 6}},
+        {{3000, 3, 150, 6}, {3000, 3, 500, 5}, {2500, 3, 150, 6}, {1200, 3, 150, 9}},
+        {{1600, 1, 350, 4}, {600, 1, 150, 4}, {1600, 1, 150, 4}, {600, 4, 150, 8}},
         {{2500, 1, 150, 6}, {1600, 4, 250, 4}, {2000, 1, 500, 4}, {1200, 4, 150, 8}}};
     const auto& r = RULE[pass][dc.id == 0 ? 0 : dc.id == 2 ? 1 : dims <= 192 ? 2 : 3];
     int n = other < r.least || other < (int64_t)r.times * own ? 1 : (int)(4 * (int64_t)other / (4 * r.a + (int64_t)r.b4 * own));

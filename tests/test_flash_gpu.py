@@ -403,7 +403,7 @@ def test_head_dims_of_up_to_96(dk, dv, causal):
 # other sides cut into shares over several workgroups: a token past a share's end and one before it, a last share of a few tokens, own sides that
 # end inside a workgroup, every class, 2 ... 8 shares, one own block per wave and two
 @pytest.mark.parametrize("Lq,Lk,dk,dv,counts", [
-    (33, 2560, 64, 64, (1, 20)), (129, 2689, 64, 128, (1, 40)), (128, 1281, 128, 128, (1, 90)), (300, 2500, 80, 72, (1, 60)), (700, 4097, 64, 64, (1, 30)),
+    (33, 3073, 64, 64, (1, 20)), (129, 3201, 64, 128, (1, 40)), (128, 1281, 128, 128, (1, 90)), (300, 2500, 80, 72, (1, 60)), (700, 4097, 64, 64, (1, 30)),
     (2600, 90, 64, 64, (1, 40)), (1700, 65, 64, 128, (1, 90)), (1281, 130, 128, 128, (1, 40)), (2100, 200, 96, 40, (1, 60)), (64, 2000, 104, 128, (1, 16))])
 def test_other_side_in_shares(Lq, Lk, dk, dv, counts):
     scale = 1 / math.sqrt(dk)
@@ -421,7 +421,7 @@ def test_other_side_in_shares(Lq, Lk, dk, dv, counts):
 
 # a share whose scores are all -inf or hold NaN / inf, and an infinite key in one share: what the whole row gives
 def test_shares_with_infinite_and_nan_scores():
-    Lq, Lk, d = 40, 3000, 64
+    Lq, Lk, d = 40, 3001, 64
     q, k, v, _ = (t.cuda() for t in orc.make_qkv(3, 1, 4, Lq, Lk, d, d, torch.float16))
     q[:, :, :, 0] = 1.0
     k[:, 1, :1500, 0] = -float("inf")     # the first shares of head 1 score -inf
