@@ -1,4 +1,4 @@
-// Flash kernels with asynchronous staging: the variants of flash_kernel.hpp for the classes of head dim 64 and 128
+// Flash kernels with asynchronous staging: the variants of flash_kernel.hpp for the classes of head dim 64 and 128 (tiles: 32 too)
 // (head dims below the class in multiples of 8: template flag PAD, the copies skip the missing 16-byte pieces, whose
 // LDS slots are zeroed once).  Streamed chunks travel HBM -> LDS by the DMA path of the vector
 // memory unit (16 bytes per lane, no staging registers, no LDS write instructions) into a ring of two or three chunk
@@ -6,6 +6,14 @@
 // padding; the 16-byte piece c of token t is stored at piece c ^ (m (t & 7)), m = D / 64, which keeps the operand
 // reads (16 lanes x 16 bytes), the transposing reads (32 lanes x 8 bytes) and the 64 x 16 bytes a copy instruction
 // writes on distinct banks.  The arithmetic, the masks and the chunk walk are those of flash_kernel.hpp.
+//
+// MODE 2 and 3 (images): windows over tiles of 64 k tokens, also at head dim 32.  A chunk of 64 tokens and the own tokens of a wave lie inside
+// one tile each, so a wave takes a chunk as a whole or leaves it out: no mask, no tail, and chunk offsets that are lane constants.  The
+// register-staged kernels had two barriers a chunk and tested every half block.  3 x 3 tiles of 64, forward and backward, us: d = 64, 32 slabs of 17 x
+// 30 tiles 306 -> 246 and 745 -> 620, 4 of 15 x 4 21.7 -> 11.1 and 49 -> 26; d = 32 217 -> 174 and 407 -> 335, 18 -> 9.6 and 36 -> 19;
+// d = 128 532 -> 421 and 1440 -> 1208, 32 -> 17 and 45 -> 38; images of 8 x 8-pixel tiles, 16 slabs of 40 x 41, d = 64 520 -> 408 and
+// 1360 -> 1100, 8 of 11 x 5 28 -> 14 and 65 -> 31.  Bound by the issue port and LDS reads as the dense kernels, and by the share of chunks
+// that a wave leaves out (a quarter with 3 tile columns).
 #pragma once
 #include "flash_kernel.hpp"
 #include "swa2_common.hpp"
@@ -14,9 +22,10 @@ template <int D>
 struct FlashDRow {
   static constexpr int ROW = 2 * D;          // bytes of a token row
   static constexpr int PIECES = D / 8;       // 16-byte pieces of a row
-  static constexpr int SWZ = PIECES / 8;     // swizzle multiplier
   static constexpr int TPI = 64 / PIECES;    // tokens per copy instruction
-  static_assert(D == 64 || D == 128, "asynchronous staging: head dim 64 or 128");
+  static_assert(D == 32 || D == 64 || D == 128, "asynchronous staging: head dim 32 (tiles), 64 or 128");
+  // piece c of token t lies at c ^ swz(t); at D = 32 four rows fill the banks and the lanes served together hold two pieces of eight rows
+  static DLT_DEV int swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : (PIECES / 8) * (t & 7); }
 };
 
 // Lane constants for the operand reads of a swizzled [token][D] tile.
@@ -34,10 +43,10 @@ template <int D>
 DLT_DEV void flashd_lane_init(FlashDLane<D>& L, int n, int g) {
   typedef FlashDRow<D> R;
 #pragma unroll
-  for (int c = 0; c < D / 32; c++) L.a[c] = n * R::ROW + 16 * ((4 * c + g) ^ (R::SWZ * (n & 7)));
+  for (int c = 0; c < D / 32; c++) L.a[c] = n * R::ROW + 16 * ((4 * c + g) ^ R::swz(n));
   const int t2 = 4 * g + (n >> 2);
 #pragma unroll
-  for (int d = 0; d < D / 16; d++) L.tr[d] = t2 * R::ROW + 16 * ((2 * d + ((n & 3) >> 1)) ^ (R::SWZ * (t2 & 7))) + 8 * (n & 1);
+  for (int d = 0; d < D / 16; d++) L.tr[d] = t2 * R::ROW + 16 * ((2 * d + ((n & 3) >> 1)) ^ R::swz(t2)) + 8 * (n & 1);
 }
 
 // A-operand pieces of the 16 tokens that start at row T0 (a multiple of 16) of a tile
@@ -71,14 +80,14 @@ struct FlashDStage {
   typedef FlashDRow<D> R;
   static constexpr int NI = CK / NW / R::TPI;
   static_assert(NI >= 1 && NI * R::TPI * NW == CK, "chunk must split evenly over the waves' copy instructions");
-  static constexpr int NOFF = D == 64 || NI == 1 ? 1 : 2;   // instructions i and i + NOFF lie a multiple of 8 tokens apart: same swizzle
+  static constexpr int NOFF = D <= 64 || NI == 1 ? 1 : 2;   // instructions i and i + NOFF lie a multiple of 8 tokens apart: same swizzle
   uint32_t off[NOFF]; // byte offset of the lane's piece inside a full chunk in instructions 0 .. NOFF - 1
   int tok0;           // token of the lane in instruction 0
   int lp;             // physical piece the lane writes
   int npieces;        // 16-byte pieces a row of the tensor really has (head dim / 8 <= PIECES)
   int sn2;            // bytes between tokens
 
-  DLT_DEV uint32_t piece(int i) const { return (uint32_t)(lp ^ (R::SWZ * ((tok0 + R::TPI * i) & 7))); }
+  DLT_DEV uint32_t piece(int i) const { return (uint32_t)(lp ^ R::swz(tok0 + R::TPI * i)); }
   DLT_DEV void init(int wave, int lane, int dact, int sn2_) {
     tok0 = wave * (CK / NW) + lane / R::PIECES;
     lp = lane % R::PIECES;
@@ -115,6 +124,44 @@ struct FlashDStage {
   }
 };
 
+// The same for chunks that lie inside one tile of a tiled window (tiles of 64 k tokens, MODE 2 and 3): always full, so a lane's offsets inside a
+// chunk are constants and its place is a scalar.  IMG: pixel rows of bw pixels, 64 a multiple of bw, so that a chunk is whole pixel rows.
+template <int D, int CK, int NW, bool IMG>
+struct FlashDStageTile {
+  typedef FlashDRow<D> R;
+  static constexpr int NI = CK / NW / R::TPI;
+  static_assert(NI >= 1 && NI * R::TPI * NW == CK, "chunk must split evenly over the waves' copy instructions");
+  uint32_t off[NI];
+  int sn2, sy2;   // bytes between tokens (IMG: pixel columns) and between pixel rows
+  const DltTokMap* tm;
+  DLT_DEV void init(int wave, int lane, const int64_t (&st)[5], const DltTokMap& tm_) {
+    sn2 = (int)st[2] * 2; sy2 = (int)st[4] * 2; tm = &tm_;
+    const int lp = lane % R::PIECES;
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const uint32_t t = (uint32_t)(wave * (CK / NW) + lane / R::PIECES + R::TPI * i);
+      off[i] = 16u * (uint32_t)(lp ^ R::swz((int)t));
+      if constexpr (IMG) {
+        const uint32_t y = dlt_fastdiv(t, tm_.mbw, tm_.sbw);
+        off[i] += y * (uint32_t)sy2 + (t - y * tm_.bw) * (uint32_t)sn2;
+      } else off[i] += t * (uint32_t)sn2;
+    }
+  }
+  template <int PAD>
+  DLT_DEV void issue(const char* base, const FlashChunk& c, char* region, int wave) const {
+    uint32_t at = (uint32_t)(c.tok0 * sn2);
+    if constexpr (IMG) {
+      uint32_t y, x;
+      dlt_slot_pixel(*tm, (uint32_t)c.x, y, x);
+      at = ((uint32_t)c.row * tm->bh + y) * (uint32_t)sy2 + x * (uint32_t)sn2;
+    }
+    const char* cb = base + at;   // wave-uniform
+    char* dst = region + wave * (CK / NW) * R::ROW;
+#pragma unroll
+    for (int i = 0; i < NI; i++) dlt_copy16_to_lds(cb, off[i], dst + R::TPI * i * R::ROW);
+  }
+};
+
 // zeroes the 16-byte slots of a swizzled [ntok][D] region that hold head dims at or beyond 8 * npieces
 template <int D>
 DLT_DEV void flashd_zero_pads(char* region, int ntok, int npieces, int tid, int nthreads) {
@@ -122,7 +169,7 @@ DLT_DEV void flashd_zero_pads(char* region, int ntok, int npieces, int tid, int 
   if (npieces == R::PIECES) return;
   for (int s = tid; s < ntok * R::PIECES; s += nthreads) {
     const int t = s / R::PIECES, pp = s % R::PIECES;
-    if ((pp ^ (R::SWZ * (t & 7))) >= npieces) *reinterpret_cast<u32x4*>(region + s * 16) = u32x4{0u, 0u, 0u, 0u};
+    if ((pp ^ R::swz((int)t)) >= npieces) *reinterpret_cast<u32x4*>(region + s * 16) = u32x4{0u, 0u, 0u, 0u};
   }
 }
 
@@ -180,6 +227,40 @@ struct FlashDBuf {
   static constexpr int BUF_KV = REG_A + REG_B + SCAL;  // dK/dV
 };
 
+// The chunks in their order, once as they are copied and once as they are used.  Tile mode walks rows of a window: the next chunk follows from
+// the last one without a division.
+template <int MODE, int CK>
+struct FlashOrder {
+  const FlashWalk<MODE, CK>& W;
+  FlashChunk c, u;
+  DLT_DEV explicit FlashOrder(const FlashWalk<MODE, CK>& W_) : W(W_) {
+    if constexpr (MODE >= 2) c = u = W.at(0);
+  }
+  DLT_DEV static FlashChunk turn(const FlashWalk<MODE, CK>& W, FlashChunk& x) {
+    const FlashChunk now = x;
+    x = W.next(x);
+    return now;
+  }
+  DLT_DEV FlashChunk copied(int i) {
+    if constexpr (MODE >= 2) return turn(W, c);
+    else return W.at(i);
+  }
+  DLT_DEV FlashChunk used(int i) {
+    if constexpr (MODE >= 2) return turn(W, u);
+    else return W.at(i);
+  }
+};
+// Tile mode: whether the wave's own tokens (in one tile, from x on) see the chunk that starts at the given x (wave-uniform)
+template <int MODE>
+struct FlashSeen {
+  int lo = 0, hi = 0;
+  DLT_DEV void init(const DltGeom& g, int r, int x, int len) {
+    int rl, rh;
+    if (x < len) dlt_key_range(g, r, x, rl, rh, lo, hi);   // the window is symmetric: also the queries that see a key
+  }
+  DLT_DEV bool operator()(int x) const { return MODE < 2 || (x >= lo && x < hi); }
+};
+
 // Head dims the products run over.  PAD 0: the class's own; 1: any below them, the products run over the zeroed pieces too; 2: at
 // most 96 of 128, the last 32 dims are left out of every product, operand read and accumulator (their terms are zeros); 3: at most 80,
 // the transposed products (O, dQ, dK, dV) leave out 48.  These kernels are bound by the issue port and LDS reads, of which that is a
@@ -199,7 +280,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
   constexpr bool CAUSAL = MODE == 1;
-  static_assert(MODE < 2, "asynchronous staging: dense and causal only");
+  constexpr bool TILE = MODE >= 2, IMG = MODE == 3;
+  static_assert(!TILE || (PAD == 0 && CK == 64 && 16 * NP <= 64), "tiles of 64 k tokens: a chunk and a wave's own tokens lie inside one tile each");
   constexpr int AK = flashd_dims(DK, PAD), AV = flashd_dims(DV, PAD);
   constexpr int KC = AK / 32, VC = AV / 32, KB = flashd_blocks(DK, PAD), VB = flashd_blocks(DV, PAD), NQB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
@@ -211,7 +293,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_k, a.B * a.H, a.causal_group, OWN, false, bh, r_own, x0);
-  else flash_block(lin, a.nblk_k, a.share_kv.n, OWN, bh, r_own, x0);   // r_own: the share
+  else if constexpr (IMG) flash_block_image(lin, a.nblk_k, a.g.TR, a.H, OWN, bh, r_own, x0);
+  else flash_block(lin, a.nblk_k, TILE ? a.g.TR : a.share_kv.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* kb_ = reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1];
   const TIO* vb_ = reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1];
@@ -222,14 +305,19 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
-  if constexpr (CAUSAL) W.init_seq((x0 / CK) * CK, a.Lq);
+  if constexpr (TILE) W.init_tile(a.g, r_own, x0, OWN, true);
+  else if constexpr (CAUSAL) W.init_seq((x0 / CK) * CK, a.Lq);
   else W.init_seq(r_own * a.share_kv.len, r_own + 1 < a.share_kv.n ? (r_own + 1) * a.share_kv.len : a.Lq);
   const int wk0 = x0 + wave * 16 * NP;  // first own key of this wave
+  const int own_base = TILE ? r_own * a.Lk : 0;   // token index of own x = 0
+  FlashSeen<MODE> seen;
+  if constexpr (TILE) seen.init(a.g, r_own, wk0, a.Lk);
+  FlashOrder<MODE, CK> order(W);
 
-  FlashDStage<DK, CK, NW, false> stq;
-  FlashDStage<DV, CK, NW, false> std_;
-  stq.init(wave, lane, a.dk_, (int)a.qs[2] * 2);
-  std_.init(wave, lane, a.dv_, (int)a.dos[2] * 2);
+  typename std::conditional<TILE, FlashDStageTile<DK, CK, NW, IMG>, FlashDStage<DK, CK, NW, false>>::type stq;
+  typename std::conditional<TILE, FlashDStageTile<DV, CK, NW, IMG>, FlashDStage<DV, CK, NW, false>>::type std_;
+  if constexpr (TILE) { stq.init(wave, lane, a.qs, a.tm); std_.init(wave, lane, a.dos, a.tm); }
+  else { stq.init(wave, lane, a.dk_, (int)a.qs[2] * 2); std_.init(wave, lane, a.dv_, (int)a.dos[2] * 2); }
   // waves 0 and 1 also copy the chunk's lse2 / delta
   const float* scal_base = wave == 0 ? lseb : delb;
   auto issue = [&](const FlashChunk& c, char* buf) {
@@ -247,17 +335,17 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   }
 #pragma unroll 1
   for (int i = 0; i < AHEAD; i++)
-    if (i < W.nchunks) issue(W.at(i), smem + i * B::BUF_KV);
+    if (i < W.nchunks) issue(order.copied(i), smem + i * B::BUF_KV);
 
   u32x4 kf[NP][KC], vf[NP][VC];
   int qmin[NP];           // causal: first query that sees this lane's key
 #pragma unroll
   for (int p = 0; p < NP; p++) {
     const int xk = wk0 + 16 * p + n;
-    const int64_t tk = xk < a.Lk ? (int64_t)xk : (int64_t)-1;
+    const int64_t tk = xk < a.Lk ? (int64_t)(own_base + xk) : (int64_t)-1;
     qmin[p] = CAUSAL ? xk : 0;
-    swa1_load_own<TIO, CT, AK>(kf[p], kb_, 1, a.dk_, flash_own_off<false>(a.ks, a.tm, tk), g, no_rope, false);
-    swa1_load_own<TIO, CT, AV>(vf[p], vb_, 1, a.dv_, flash_own_off<false>(a.vs, a.tm, tk), g, no_rope, false);
+    swa1_load_own<TIO, CT, AK>(kf[p], kb_, 1, a.dk_, flash_own_off<IMG>(a.ks, a.tm, tk), g, no_rope, false);
+    swa1_load_own<TIO, CT, AV>(vf[p], vb_, 1, a.dv_, flash_own_off<IMG>(a.vs, a.tm, tk), g, no_rope, false);
   }
   f32x4 dk_acc[NP][KB], dv_acc[NP][VB];
 #pragma unroll
@@ -303,11 +391,12 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     bool tail;
     if constexpr (std::is_same<decltype(tail_tag), FlashTailDyn>::value) tail = chunk_tail(ci);
     else tail = decltype(tail_tag)::value;
-    if constexpr (decltype(more_tag)::value) issue(W.at(ci + AHEAD), nxt);
+    if constexpr (decltype(more_tag)::value) issue(order.copied(ci + AHEAD), nxt);
     Swa2Lds sQ = cur, sDO = cur + B::REG_A;
     Swa2Lds sLse = cur + B::REG_A + B::REG_B + 16 * g, sDel = sLse + CK * 4;
-    const FlashChunk c = W.at(ci);
+    const FlashChunk c = order.used(ci);
     const int q0 = c.x;
+    if (!seen(q0)) return;
     // causal: every query of the chunk lies below every own key of this wave
     if (CAUSAL && !std::is_same<decltype(tail_tag), std::false_type>::value && q0 + CK - 1 < wk0) return;
     // Order of a chunk's operands: the first products (S, dP) of every 16-query half of every block, then the second
@@ -317,7 +406,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     // and vector ALU take turns instead of running side by side.
     constexpr int N1H = KC + VC, NH = 2 * NQB, N1 = NH * N1H, NP2 = VB + KB, NT = N1 + NQB * NP2;
     constexpr int NU = 2 * NP;   // element-wise pieces of a half: (own block p, pair of queries)
-    static_assert(N1H >= NU && NP2 >= NU, "a segment must have room for the element-wise pieces of a half");
+    constexpr int NUR = (NU + N1H - 1) / N1H;   // pieces behind an operand of a first product: one but at 32/32
+    static_assert(NP2 >= NU, "a segment must have room for the element-wise pieces of a half");
     constexpr int RD = FLASHD_RD;
     u32x4 ring[RD + 1];
     auto rd = [&](auto kc) __attribute__((always_inline)) {
@@ -381,8 +471,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
           if constexpr (r < KC) sv[hh & 1][p] = Mma<CT>::mfma(x, kf[p][r], r == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sv[hh & 1][p]);
           else dp[hh & 1][p] = Mma<CT>::mfma(x, vf[p][r - KC], r == KC ? dl[hh & 1] : dp[hh & 1][p]);
         }
-        if constexpr (hh >= 1 && r < NU) {
-          ew(std::integral_constant<int, hh - 1>{}, std::integral_constant<int, r>{});
+        if constexpr (hh >= 1 && r * NUR < NU) {
+          swa2_for<r * NUR, (r + 1) * NUR < NU ? (r + 1) * NUR : NU>([&](auto uc) __attribute__((always_inline)) { ew(std::integral_constant<int, hh - 1>{}, uc); });
           FLASHD_EW_MIX
         }
       } else {
@@ -436,7 +526,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   while (ci + AHEAD < W.nchunks) plain_round();
   // without a mask a full last chunk runs here too (same test-free body): the code below, whose per-pair tests cost
   // registers the compiler finds by spilling, is then not executed at all
-  const int n_plain = (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
+  const int n_plain = TILE || (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
   for (; ci < n_plain; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::false_type{});
@@ -444,11 +534,11 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     __syncthreads();
     bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
-  if (ci < W.nchunks) {
+  if (!TILE && ci < W.nchunks) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
-  if (!CAUSAL && a.share_kv.n > 1) {
+  if (MODE == 0 && a.share_kv.n > 1) {
     float* part = a.share_kv.part + flash_share_row(a.share_kv, bh, r_own, a.Lk) * a.dk_;
     flash_share_put<NP>(part, dk_acc, a.dk_, wk0 + n, a.Lk, g);
     part = a.share_kv.part + (int64_t)a.B * a.H * a.share_kv.n * a.Lk * a.dk_ + flash_share_row(a.share_kv, bh, r_own, a.Lk) * a.dv_;
@@ -458,8 +548,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   __syncthreads();
   TIO* dkb = reinterpret_cast<TIO*>(a.dk) + b * a.dks[0] + h * a.dks[1];
   TIO* dvb = reinterpret_cast<TIO*>(a.dv) + b * a.dvs[0] + h * a.dvs[1];
-  flash_write_grad<TIO, DK, NP>(smem, dk_acc, a.sm_scale, dkb, flash_tok<false>(a.dks, a.tm), a.dks[3], a.dk_, a.dk_vec != 0, 0, x0, a.Lk, wave, n, g, tid, OWN);
-  flash_write_grad<TIO, DV, NP>(smem, dv_acc, 1.0f, dvb, flash_tok<false>(a.dvs, a.tm), a.dvs[3], a.dv_, a.dv_vec != 0, 0, x0, a.Lk, wave, n, g, tid, OWN);
+  flash_write_grad<TIO, DK, NP>(smem, dk_acc, a.sm_scale, dkb, flash_tok<IMG>(a.dks, a.tm), a.dks[3], a.dk_, a.dk_vec != 0, own_base, x0, a.Lk, wave, n, g, tid, OWN);
+  flash_write_grad<TIO, DV, NP>(smem, dv_acc, 1.0f, dvb, flash_tok<IMG>(a.dvs, a.tm), a.dvs[3], a.dv_, a.dv_vec != 0, own_base, x0, a.Lk, wave, n, g, tid, OWN);
 }
 
 // ---- forward: own = queries; K and V stream.  Replaces _attn_fwd (src/flash_attn.py:81-172).
@@ -473,7 +563,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
   constexpr bool CAUSAL = MODE == 1;
-  static_assert(MODE < 2, "asynchronous staging: dense and causal only");
+  constexpr bool TILE = MODE >= 2, IMG = MODE == 3;
+  static_assert(!TILE || (PAD == 0 && CK == 64 && 16 * NP <= 64), "tiles of 64 k tokens: a chunk and a wave's own tokens lie inside one tile each");
   constexpr int PO = DV * (int)sizeof(TL) + 16;
   constexpr int AK = flashd_dims(DK, PAD);
   constexpr int KC = AK / 32, VB = flashd_blocks(DV, PAD), NKB = CK / 32;
@@ -488,7 +579,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
-  else flash_block(lin, a.nblk, a.share.n, OWN, bh, r_own, x0);   // r_own: the share
+  else if constexpr (IMG) flash_block_image(lin, a.nblk, a.g.TR, a.H, OWN, bh, r_own, x0);
+  else flash_block(lin, a.nblk, TILE ? a.g.TR : a.share.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
@@ -498,13 +590,18 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
-  if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
+  if constexpr (TILE) W.init_tile(a.g, r_own, x0, OWN, false);
+  else if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
   else W.init_seq(r_own * a.share.len, r_own + 1 < a.share.n ? (r_own + 1) * a.share.len : a.Lk);
 
-  FlashDStage<DK, CK, NW> stk;
-  FlashDStage<DV, CK, NW> stv;
-  stk.init(wave, lane, a.dk, (int)a.ks[2] * 2);
-  stv.init(wave, lane, a.dv, (int)a.vs[2] * 2);
+  const int own_base = TILE ? r_own * a.Lq : 0;   // token index of own x = 0
+  FlashSeen<MODE> seen;
+  if constexpr (TILE) seen.init(a.g, r_own, wq0, a.Lq);
+  FlashOrder<MODE, CK> order(W);
+  typename std::conditional<TILE, FlashDStageTile<DK, CK, NW, IMG>, FlashDStage<DK, CK, NW>>::type stk;
+  typename std::conditional<TILE, FlashDStageTile<DV, CK, NW, IMG>, FlashDStage<DV, CK, NW>>::type stv;
+  if constexpr (TILE) { stk.init(wave, lane, a.ks, a.tm); stv.init(wave, lane, a.vs, a.tm); }
+  else { stk.init(wave, lane, a.dk, (int)a.ks[2] * 2); stv.init(wave, lane, a.dv, (int)a.vs[2] * 2); }
   // head dims below the padded ones: the slots of the missing pieces are zeroed once, no copy writes them
 #pragma unroll
   for (int i = 0; PAD && i < NBUF; i++) {
@@ -517,7 +614,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   };
 #pragma unroll 1
   for (int i = 0; i < AHEAD; i++)
-    if (i < W.nchunks) issue(W.at(i), smem + i * B::BUF);
+    if (i < W.nchunks) issue(order.copied(i), smem + i * B::BUF);
 
   u32x4 qf[NP][KC];
   int64_t tq[NP];
@@ -525,9 +622,9 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
 #pragma unroll
   for (int p = 0; p < NP; p++) {
     const int xq = wq0 + 16 * p + n;
-    tq[p] = xq < a.Lq ? (int64_t)xq : (int64_t)-1;
+    tq[p] = xq < a.Lq ? (int64_t)(own_base + xq) : (int64_t)-1;
     klim[p] = CAUSAL ? dlt_imin(xq, a.Lk - 1) : a.Lk - 1;
-    swa1_load_own<TIO, CT, AK>(qf[p], qb, 1, a.dk, flash_own_off<false>(a.qs, a.tm, tq[p]), g, no_rope, false);
+    swa1_load_own<TIO, CT, AK>(qf[p], qb, 1, a.dk, flash_own_off<IMG>(a.qs, a.tm, tq[p]), g, no_rope, false);
   }
   float m_run[NP];
   f32x4 acc[NP][VB], acc_l[NP];
@@ -560,10 +657,11 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     bool tail;
     if constexpr (std::is_same<decltype(tail_tag), FlashTailDyn>::value) tail = chunk_tail(ci);
     else tail = decltype(tail_tag)::value;
-    if constexpr (decltype(more_tag)::value) issue(W.at(ci + AHEAD), nxt);
+    if constexpr (decltype(more_tag)::value) issue(order.copied(ci + AHEAD), nxt);
     Swa2Lds sK = cur, sV = cur + B::REG_A;
-    const FlashChunk c = W.at(ci);
+    const FlashChunk c = order.used(ci);
     const int k0 = c.x;
+    if (!seen(k0)) return;
     // causal: every key of the chunk lies above every query of this wave
     if (CAUSAL && !std::is_same<decltype(tail_tag), std::false_type>::value && k0 > wq0 + 16 * NP - 1) return;
     constexpr int N1 = NKB * 2 * KC, NT = N1 + NKB * VB;
@@ -680,7 +778,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   }
   // without a mask a full last chunk runs here too (same test-free body): the code below, whose per-pair tests cost
   // registers the compiler finds by spilling, is then not executed at all
-  const int n_plain = (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
+  const int n_plain = TILE || (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
   for (; ci < n_plain; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::false_type{});
@@ -688,11 +786,11 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     __syncthreads();
     bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
-  if (ci < W.nchunks) {
+  if (!TILE && ci < W.nchunks) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
-  if (!CAUSAL && a.share.n > 1) {
+  if (MODE == 0 && a.share.n > 1) {
     const int64_t row0 = flash_share_row(a.share, bh, r_own, a.Lq);
     float* ml = a.share.part + (int64_t)a.B * a.H * a.share.n * a.Lq * a.dv + 2 * row0;
     flash_share_put<NP>(a.share.part + row0 * a.dv, acc, a.dv, wq0 + n, a.Lq, g);
@@ -721,8 +819,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   int tw = tid;   // opaque copy: keeps the tile writer's addresses out of the registers that live across the chunk loop
   asm volatile("" : "+v"(tw));
   if (tw < 256)   // the tile writer walks the rows with 256 threads
-    store_tile<TIO, TL, DV>(smem, PO, ob, flash_tok<false>(a.os, a.tm), a.os[3], a.dv, a.o_vec != 0, OWN,
-                            [&](int row) { return x0 + row < a.Lq ? (int64_t)(x0 + row) : (int64_t)-1; }, no_rope, tw);
+    store_tile<TIO, TL, DV>(smem, PO, ob, flash_tok<IMG>(a.os, a.tm), a.os[3], a.dv, a.o_vec != 0, OWN,
+                            [&](int row) { return x0 + row < a.Lq ? (int64_t)(own_base + x0 + row) : (int64_t)-1; }, no_rope, tw);
 }
 
 // ---- dQ: own = queries; K and V stream.  Replaces _attn_bwd_dq (src/flash_attn.py:310-449) and, with fuse_delta, the
@@ -734,7 +832,8 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
   constexpr bool CAUSAL = MODE == 1;
-  static_assert(MODE < 2, "asynchronous staging: dense and causal only");
+  constexpr bool TILE = MODE >= 2, IMG = MODE == 3;
+  static_assert(!TILE || (PAD == 0 && CK == 64 && 16 * NP <= 64), "tiles of 64 k tokens: a chunk and a wave's own tokens lie inside one tile each");
   constexpr int AK = flashd_dims(DK, PAD), AV = flashd_dims(DV, PAD);
   constexpr int KC = AK / 32, VC = AV / 32, KB = flashd_blocks(DK, PAD), NKB = CK / 32;
   constexpr int OWN = 16 * NP * NW;
@@ -748,7 +847,8 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_q, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
-  else flash_block(lin, a.nblk_q, a.share_q.n, OWN, bh, r_own, x0);   // r_own: the share
+  else if constexpr (IMG) flash_block_image(lin, a.nblk_q, a.g.TR, a.H, OWN, bh, r_own, x0);
+  else flash_block(lin, a.nblk_q, TILE ? a.g.TR : a.share_q.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
@@ -758,13 +858,18 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   RopeDev no_rope = RopeDev{};
 
   FlashWalk<MODE, CK> W;
-  if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
+  if constexpr (TILE) W.init_tile(a.g, r_own, x0, OWN, false);
+  else if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
   else W.init_seq(r_own * a.share_q.len, r_own + 1 < a.share_q.n ? (r_own + 1) * a.share_q.len : a.Lk);
 
-  FlashDStage<DK, CK, NW, (DK + DV > 128)> stk;
-  FlashDStage<DV, CK, NW, (DK + DV > 128)> stv;
-  stk.init(wave, lane, a.dk_, (int)a.ks[2] * 2);
-  stv.init(wave, lane, a.dv_, (int)a.vs[2] * 2);
+  const int own_base = TILE ? r_own * a.Lq : 0;   // token index of own x = 0
+  FlashSeen<MODE> seen;
+  if constexpr (TILE) seen.init(a.g, r_own, wq0, a.Lq);
+  FlashOrder<MODE, CK> order(W);
+  typename std::conditional<TILE, FlashDStageTile<DK, CK, NW, IMG>, FlashDStage<DK, CK, NW, (DK + DV > 128)>>::type stk;
+  typename std::conditional<TILE, FlashDStageTile<DV, CK, NW, IMG>, FlashDStage<DV, CK, NW, (DK + DV > 128)>>::type stv;
+  if constexpr (TILE) { stk.init(wave, lane, a.ks, a.tm); stv.init(wave, lane, a.vs, a.tm); }
+  else { stk.init(wave, lane, a.dk_, (int)a.ks[2] * 2); stv.init(wave, lane, a.dv_, (int)a.vs[2] * 2); }
   // head dims below the padded ones: the slots of the missing pieces are zeroed once, no copy writes them
 #pragma unroll
   for (int i = 0; PAD && i < NBUF; i++) {
@@ -777,7 +882,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   };
 #pragma unroll 1
   for (int i = 0; i < AHEAD; i++)
-    if (i < W.nchunks) issue(W.at(i), smem + i * B::BUF);
+    if (i < W.nchunks) issue(order.copied(i), smem + i * B::BUF);
 
   u32x4 qf[NP][KC], dof[NP][VC];
   float nlse[NP], del_n[NP];
@@ -785,16 +890,16 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
 #pragma unroll
   for (int p = 0; p < NP; p++) {
     const int xq = wq0 + 16 * p + n;
-    const int64_t tq = xq < a.Lq ? (int64_t)xq : (int64_t)-1;
+    const int64_t tq = xq < a.Lq ? (int64_t)(own_base + xq) : (int64_t)-1;
     klim[p] = CAUSAL ? dlt_imin(xq, a.Lk - 1) : a.Lk - 1;
-    swa1_load_own<TIO, CT, AK>(qf[p], qb, 1, a.dk_, flash_own_off<false>(a.qs, a.tm, tq), g, no_rope, false);
-    swa1_load_own<TIO, CT, AV>(dof[p], dob, 1, a.dv_, flash_own_off<false>(a.dos, a.tm, tq), g, no_rope, false);
+    swa1_load_own<TIO, CT, AK>(qf[p], qb, 1, a.dk_, flash_own_off<IMG>(a.qs, a.tm, tq), g, no_rope, false);
+    swa1_load_own<TIO, CT, AV>(dof[p], dob, 1, a.dv_, flash_own_off<IMG>(a.dos, a.tm, tq), g, no_rope, false);
     const int64_t off = b * a.ls[0] + h * a.ls[1] + (tq >= 0 ? tq : 0) * a.ls[2];
     nlse[p] = tq >= 0 ? -a.lse[off] : 0.f;
     if (a.fuse_delta != 0) {
       const TIO* ob = reinterpret_cast<const TIO*>(a.o) + b * a.os[0] + h * a.os[1];
       u32x4 of[VC];
-      swa1_load_own<TIO, CT, AV>(of, ob, 1, a.dv_, flash_own_off<false>(a.os, a.tm, tq), g, no_rope, false);
+      swa1_load_own<TIO, CT, AV>(of, ob, 1, a.dv_, flash_own_off<IMG>(a.os, a.tm, tq), g, no_rope, false);
       float part = 0.f;
 #pragma unroll
       for (int c_ = 0; c_ < VC; c_++) {
@@ -805,7 +910,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
         for (int j = 0; j < 8; j++) part += fo[j] * fd[j];
       }
       del_n[p] = wave_sum4(part);
-      if (g == 0 && tq >= 0 && (CAUSAL || r_own == 0)) store_stream4(a.delta_out + off, del_n[p]);
+      if (g == 0 && tq >= 0 && (MODE != 0 || r_own == 0)) store_stream4(a.delta_out + off, del_n[p]);
     } else {
       del_n[p] = tq >= 0 ? a.delta[off] : 0.f;
     }
@@ -845,10 +950,11 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
     bool tail;
     if constexpr (std::is_same<decltype(tail_tag), FlashTailDyn>::value) tail = chunk_tail(ci);
     else tail = decltype(tail_tag)::value;
-    if constexpr (decltype(more_tag)::value) issue(W.at(ci + AHEAD), nxt);
+    if constexpr (decltype(more_tag)::value) issue(order.copied(ci + AHEAD), nxt);
     Swa2Lds sK = cur, sV = cur + B::REG_A;
-    const FlashChunk c = W.at(ci);
+    const FlashChunk c = order.used(ci);
     const int k0 = c.x;
+    if (!seen(k0)) return;
     if (CAUSAL && !std::is_same<decltype(tail_tag), std::false_type>::value && k0 > wq0 + 16 * NP - 1) return;
     constexpr int N1H = KC + VC, N1 = 2 * N1H, NB = N1 + KB, NT = NKB * NB;
     constexpr int RD = FLASHD_RD;
@@ -941,7 +1047,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   }
   // without a mask a full last chunk runs here too (same test-free body): the code below, whose per-pair tests cost
   // registers the compiler finds by spilling, is then not executed at all
-  const int n_plain = (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
+  const int n_plain = TILE || (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
   for (; ci < n_plain; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::false_type{});
@@ -949,15 +1055,15 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
     __syncthreads();
     bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
-  if (ci < W.nchunks) {
+  if (!TILE && ci < W.nchunks) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
-  if (!CAUSAL && a.share_q.n > 1) {
+  if (MODE == 0 && a.share_q.n > 1) {
     flash_share_put<NP>(a.share_q.part + flash_share_row(a.share_q, bh, r_own, a.Lq) * a.dk_, dq_acc, a.dk_, wq0 + n, a.Lq, g);
     return;
   }
   __syncthreads();
   TIO* dqb = reinterpret_cast<TIO*>(a.dq) + b * a.dqs[0] + h * a.dqs[1];
-  flash_write_grad<TIO, DK, NP>(smem, dq_acc, a.sm_scale, dqb, flash_tok<false>(a.dqs, a.tm), a.dqs[3], a.dk_, a.dq_vec != 0, 0, x0, a.Lq, wave, n, g, tid, OWN);
+  flash_write_grad<TIO, DK, NP>(smem, dq_acc, a.sm_scale, dqb, flash_tok<IMG>(a.dqs, a.tm), a.dqs[3], a.dk_, a.dq_vec != 0, own_base, x0, a.Lq, wave, n, g, tid, OWN);
 }

@@ -36,6 +36,19 @@ inline int flashd_pad(int dk, int dv) {
   return d > 96 ? 1 : d > 80 ? 2 : 3;
 }
 
+// Windows over tiles of 64 k tokens run on the asynchronously staged kernels: exact head dims, chunks of whole pixel rows in the image layout.
+inline bool flashd_tiles(int dk, int dv, const DltGeom& g, const DltTokMap& tm) {
+  return dk == DLT_DK && dv == DLT_DV && g.S % 64 == 0 && (!tm.img || 64 % tm.bw == 0) && dlt_flash_async();
+}
+// ... in workgroups of 64 own tokens (one block per wave) while they are few, and where workgroups of 128 would be a sixth empty.  Two blocks
+// per wave -> one, 3 x 3 tiles of 64 unless said, us, forward and backward: 4 slabs of 15 x 4, d = 64 14.9 -> 11.1 and 34.5 -> 26.0; images, 8 of 11 x 5
+// 21 -> 14.5 and 46 -> 31; 64 of 11 x 5 60 -> 56 and 155 -> 145; 32 of 17 x 30 249 -> 278 and 611 -> 639; d = 128, 4 of 15 x 4 21 -> 16 and 46 -> 39, but 64 of
+// 11 x 5 (8 waves of one block in the forward pass there) 92 -> 105 and 261 -> 261.
+inline bool flashd_tiles_one(int slabs, int xl, const DltGeom& g) {
+  const int64_t n = (xl + 63) / 64;
+  return slabs * (int64_t)g.TR * n <= 3 * (int64_t)dlt_device_cus() || (DLT_DK + DLT_DV <= 192 && 6 * n <= 5 * ((n + 1) / 2 * 2));
+}
+
 template <typename KernT>
 int flash_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
@@ -45,8 +58,9 @@ int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
   const int pad = flashd_pad(a.dk, a.dv);
   auto kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
-  if (pad == 1) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
-  if constexpr (DLT_DV == 128) {
+  if constexpr (MODE < 2)
+    if (pad == 1) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+  if constexpr (MODE < 2 && DLT_DV == 128) {
     if (pad == 2) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
     if (pad == 3) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
   }
@@ -57,8 +71,9 @@ int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   const int rc = flash_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;
   a.nblk = (a.Lq + own - 1) / own;
+  const int rows = MODE >= 2 ? a.g.TR : a.share.n;
   dlt_timing_before(DLT_K_FWD, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk * a.share.n), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk * rows), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash forward launch");
   return DLT_OK;
@@ -79,6 +94,11 @@ int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
       return flashd_launch_fwd<TIO, MODE, FLASHD_FWD_NP, FLASHD_FWD_CK(DLT_DK, DLT_DV), FLASHD_FWD_NW(DLT_DK, DLT_DV)>(a, stream);
     }
   }
+  if constexpr (MODE >= 2)
+    if (flashd_tiles(a.dk, a.dv, a.g, a.tm)) {
+      if (flashd_tiles_one(a.B * a.H, a.Lq, a.g)) return flashd_launch_fwd<TIO, MODE, 1, 64, 4>(a, stream);
+      return flashd_launch_fwd<TIO, MODE, (DLT_DK + DLT_DV > 192 ? 1 : 2), 64, (DLT_DK + DLT_DV > 192 ? 8 : 4)>(a, stream);
+    }
   auto kern = flash_fwd_kernel<TIO, DLT_DK, DLT_DV, FLASH_NP, flash_ck_fwd(DLT_DK, DLT_DV), MODE>;
   {
     const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), a.lds_bytes);
@@ -116,8 +136,9 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
   const int pad = flashd_pad(a.dk_, a.dv_);
   auto kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
-  if (pad == 1) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
-  if constexpr (DLT_DV == 128) {
+  if constexpr (MODE < 2)
+    if (pad == 1) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+  if constexpr (MODE < 2 && DLT_DV == 128) {
     if (pad == 2) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
     if (pad == 3) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
   }
@@ -129,7 +150,7 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk_q = (a.Lq + own - 1) / own;
   dlt_timing_before(DLT_K_BWD_Q, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q * a.share_q.n), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q * (MODE >= 2 ? a.g.TR : a.share_q.n)), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash dQ launch");
   return DLT_OK;
@@ -146,6 +167,9 @@ int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) 
       return flashd_launch_bwd_q<TIO, MODE, FLASHD_DQ_NP(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }
+  if constexpr (MODE >= 2)
+    if (flashd_tiles(a.dk_, a.dv_, a.g, a.tm))
+      return flashd_tiles_one(a.B * a.H, a.Lq, a.g) ? flashd_launch_bwd_q<TIO, MODE, 1, 4>(a, stream) : flashd_launch_bwd_q<TIO, MODE, 2, 4>(a, stream);
   auto kern = flash_bwd_q_kernel<TIO, DLT_DK, DLT_DV, flash_np_q(DLT_DK, DLT_DV), flash_ck_q(DLT_DK, DLT_DV), MODE>;
   int rc = flash_set_lds(kern, a.lds_q);
   if (rc != DLT_OK) return rc;
@@ -173,8 +197,9 @@ int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
   const int pad = flashd_pad(a.dk_, a.dv_);
   auto kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
-  if (pad == 1) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
-  if constexpr (DLT_DV == 128) {
+  if constexpr (MODE < 2)
+    if (pad == 1) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+  if constexpr (MODE < 2 && DLT_DV == 128) {
     if (pad == 2) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
     if (pad == 3) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
   }
@@ -186,7 +211,7 @@ int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk_k = (a.Lk + own - 1) / own;
   dlt_timing_before(DLT_K_BWD_KV, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k * a.share_kv.n), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k * (MODE >= 2 ? a.g.TR : a.share_kv.n)), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash dK/dV launch");
   return DLT_OK;
@@ -195,13 +220,16 @@ int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
 template <typename TIO, int MODE>
 int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
-    // dense / causal, head dims that are multiples of 8: chunks are copied HBM -> LDS asynchronously (in tile mode,
-    // where whole blocks are skipped, the register-staged kernel measured 1.5 % faster)
+    // dense / causal, head dims that are multiples of 8: chunks are copied HBM -> LDS asynchronously (tiles that are no multiple of 64
+    // tokens: parts of a chunk are skipped, the register-staged kernel measured 1.5 % faster)
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && dlt_flash_scalars_fit(a) && dlt_flash_async()) {
       if (a.slim) return flashd_launch_bwd_kv<TIO, MODE, 1, 4>(a, stream);
       return flashd_launch_bwd_kv<TIO, MODE, flash_np_kv(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }
   }
+  if constexpr (MODE >= 2)
+    if (flashd_tiles(a.dk_, a.dv_, a.g, a.tm) && dlt_flash_scalars_fit(a))
+      return flashd_tiles_one(a.B * a.H, a.Lk, a.g) ? flashd_launch_bwd_kv<TIO, MODE, 1, 4>(a, stream) : flashd_launch_bwd_kv<TIO, MODE, flash_np_kv(DLT_DK, DLT_DV), 4>(a, stream);
   {
     auto kern = flash_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, flash_np_kv(DLT_DK, DLT_DV), flash_ck_kv(DLT_DK, DLT_DV), MODE>;
     int rc = flash_set_lds(kern, a.lds_kv);

@@ -557,7 +557,10 @@ struct FlashBwdArgs {
 };
 
 // lse2 / delta of a slab lie within 32-bit byte offsets: the asynchronously staged dK/dV kernel copies them
-inline bool dlt_flash_scalars_fit(const FlashBwdArgs& a) { return a.ls[2] >= 0 && ((int64_t)a.Lq - 1) * a.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1); }
+inline bool dlt_flash_scalars_fit(const FlashBwdArgs& a) {
+  const int64_t n = (int64_t)a.Lq * (a.tile ? a.g.TR : 1);
+  return a.ls[2] >= 0 && (n - 1) * a.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1);
+}
 
 // Staging of one chunk of CK tokens of two [token][dim] tensors (dims DA and DB) through registers.
 template <int DA, int DB, int CK>

@@ -225,3 +225,30 @@ def test_infinite_and_nan_tiles_stay_in_their_windows(d, th, tw, B, which):
             far = torch.maximum((rows - r).abs(), (cols - c).abs()).reshape(-1).repeat_interleave(S).cuda()
             for g, w, n in zip(grads(bad), clean, reach):
                 assert torch.equal(g[:, :, far > n], w[:, :, far > n]), (r, c, value)
+
+
+# tiles of 64 k tokens on the asynchronously staged kernels: workgroups of 64 own tokens (few, or rows that leave 128 a sixth empty) and of 128, tiles of
+# two and three chunks, rows of odd and even tile counts, windows beyond the grid, every class; image tiles of whole pixel rows per chunk and others
+@pytest.mark.parametrize("th,tw,tile,WR,WC,dk,dv,many", [
+    (3, 6, 64, 1, 1, 32, 32, 60), (2, 9, 64, 1, 2, 64, 64, 60), (4, 1, 128, 1, 1, 64, 64, 110), (2, 4, 192, 2, 0, 32, 32, 50), (3, 5, 64, 0, 1, 128, 128, 60),
+    (1, 8, 64, 3, 1, 64, 128, 110), (3, 4, (8, 8), 1, 1, 32, 32, 80), (2, 6, (4, 16), 1, 1, 64, 64, 80), (2, 3, (64, 2), 1, 1, 128, 128, 80),
+    (2, 4, (2, 64), 1, 2, 64, 128, 50), (2, 4, (4, 48), 1, 1, 64, 64, 50)])
+def test_tiles_of_64_tokens(th, tw, tile, WR, WC, dk, dv, many):
+    sw = _swa()
+    img = isinstance(tile, tuple)
+    S = tile[0] * tile[1] if img else tile
+    N, scale = th * tw * S, 1 / math.sqrt(dk)
+    ops = orc.make_qkv(N + dk + th, 1, 1, N, N, dk, dv, torch.float16)
+    want = orc.tiled_swa_grads(*(t.float() for t in ops), S, th, tw, WR, WC, scale)
+    lay = (lambda t: orc.tokens_to_image(t, th, tw, *tile).contiguous()) if img else (lambda t: t)
+    runs = []
+    for slabs in (1, many):
+        q, k, v, do = (lay(t).cuda().repeat(slabs, *[1] * (4 if img else 3)) for t in ops)
+        leaves = [t.requires_grad_(True) for t in (q, k, v)]
+        o = sw.TiledSwaImage.apply(*leaves, *tile, WR, WC, scale) if img else sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
+        runs.append((o.detach(),) + torch.autograd.grad(o, leaves, do))
+    assert (runs[0][0].float().cpu() - lay(want[0])).abs().max().item() <= FWD_TOL
+    errs = [_rel(g, lay(w)) for g, w in zip(runs[0][1:], want[1:])]
+    assert max(errs) <= 1e-2, errs   # fp16
+    for one, all_ in zip(*runs):
+        assert torch.equal(all_, one.expand_as(all_))   # the same bits in both workgroup sizes
