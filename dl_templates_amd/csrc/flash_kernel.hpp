@@ -236,6 +236,7 @@ struct FlashArgs {
   int32_t nblk;       // workgroups per (batch, head) and grid row
   int32_t causal, causal_group;   // causal_group: see flash_block_causal
   int32_t slim, chunk;   // host only: this many waves of one own block each (0: two), keys a chunk then (flash_launch_fwd_c)
+  int32_t parts, part_dv;   // kernels of flash_split_kernel.hpp: workgroups that share the output dims of an own block; host only: dims of each
   int32_t tile;       // MODE 2: Lq = Lk = tokens per grid row, geometry in g
   DltGeom g;
   int32_t o_vec;

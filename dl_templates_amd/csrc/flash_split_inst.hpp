@@ -21,11 +21,20 @@ int flashs_run(KernT kern, const Args& a, int lds, int grid, int id, hipStream_t
   return DLT_OK;
 }
 
+template <typename TIO, int NP, int DV>
+int flashs_fwd_dv(FlashArgs a, hipStream_t stream) {
+  a.parts = (a.dv + DV - 1) / DV;
+  return flashs_run(a.causal ? flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, true> : flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, false>, a,
+                    flashs_lds_fwd<DLT_DK, DV, NP, NW>(), a.B * a.H * a.nblk * a.parts, DLT_K_FWD, stream);
+}
 template <typename TIO, int NP>
 int flashs_fwd(FlashArgs a, hipStream_t stream) {
   a.nblk = (a.Lq + 16 * NP - 1) / (16 * NP);
-  return flashs_run(a.causal ? flashs_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, NW, true> : flashs_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, NW, false>, a,
-                    flashs_lds_fwd<DLT_DK, DLT_DV, NP, NW>(), a.B * a.H * a.nblk, DLT_K_FWD, stream);
+  if constexpr (NP == 1 && DLT_DV == 128)
+    if (a.part_dv == DLT_DV / 4) return flashs_fwd_dv<TIO, NP, DLT_DV / 4>(a, stream);
+  if constexpr (NP == 1 && DLT_DV >= 64)
+    if (a.part_dv == DLT_DV / 2) return flashs_fwd_dv<TIO, NP, DLT_DV / 2>(a, stream);
+  return flashs_fwd_dv<TIO, NP, DLT_DV>(a, stream);
 }
 template <typename TIO, int NP>
 int flashs_bwd_q(FlashBwdArgs a, hipStream_t stream) {

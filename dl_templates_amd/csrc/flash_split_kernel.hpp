@@ -101,6 +101,9 @@ constexpr int flashs_lds_fwd() {
   return tiles > sum ? tiles : sum;
 }
 
+// a.parts workgroups take DV of an own block's output dims each: scores and softmax are formed in every one of them, K is read by all and V by
+// one.  A CU reads the other side at 55 B/ns whatever the others do, so narrower parts take less time while CUs are idle (flash_forward has the
+// line and figures), with the same bits.
 template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
 __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const FlashArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
@@ -110,12 +113,13 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
   typedef FlashsSum<DV, NP, NW> Sum;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int bh, x0;
-  flashs_block(a.nblk, 16 * NP, bh, x0);
+  int bh, part, x0;
+  flash_block(xcd_remap(blockIdx.x, gridDim.x), a.nblk, a.parts, 16 * NP, bh, part, x0);
+  const int v0 = part * DV, dv = dlt_imin(a.dv - v0, DV);   // first output dim, their number
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
-  const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
+  const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1] + v0);
   const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
   const int len = CAUSAL ? dlt_imin(a.Lk, x0 + 16 * NP) : a.Lk;   // causal: keys up to the last own query
   const int nkb = (len + 31) / 32;
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
   u32x4 kf[2][KC], vr[VT::NV];
   if (wave < nkb) {
     flashs_load_rows<DK>(kf, kb_, ksn, wave, a.Lk, a.dk, n, g);
-    VT::load(vr, vb_, vsn, wave, a.Lk, a.dv, lane);
+    VT::load(vr, vb_, vsn, wave, a.Lk, dv, lane);
   }
   RopeDev no_rope = RopeDev{};
   u32x4 qf[NP][KC];
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
       for (int c = 0; c < KC; c++) ka[mb][c] = kf[mb][c];
     if (kb + NW < nkb) {
       flashs_load_rows<DK>(kf, kb_, ksn, kb + NW, a.Lk, a.dk, n, g);
-      VT::load(vr, vb_, vsn, kb + NW, a.Lk, a.dv, lane);
+      VT::load(vr, vb_, vsn, kb + NW, a.Lk, dv, lane);
     }
     const bool tail = 32 * kb + 32 > a.Lk || (CAUSAL && 32 * kb + 31 > x0);
     u32x4 pb[NP];
@@ -232,14 +236,14 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
   };
   TIO* ob = reinterpret_cast<TIO*>(a.o) + b * a.os[0] + h * a.os[1];
   Sum::reduce(sums, tid, [&](int row, int d0, float* v) {
-    if (x0 + row >= a.Lq || d0 >= a.dv) return;
+    if (x0 + row >= a.Lq || d0 >= dv) return;
     float m, l;
     total(row, m, l);
     const float inv = l > 0.f ? fast_rcp(l) : 0.f;
 #pragma unroll
     for (int j = 0; j < 8; j++) v[j] *= inv;
-    Io<TIO, CT>::store8(ob + (x0 + row) * a.os[2] + d0 * a.os[3], v, a.o_vec != 0, a.os[3], dlt_imin(8, a.dv - d0));
-    if (d0 == 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + (x0 + row) * a.ls[2]), m * scale + fast_log2(l));
+    Io<TIO, CT>::store8(ob + (x0 + row) * a.os[2] + (v0 + d0) * a.os[3], v, a.o_vec != 0, a.os[3], dlt_imin(8, dv - d0));
+    if (d0 == 0 && part == 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + (x0 + row) * a.ls[2]), m * scale + fast_log2(l));
   });
 }
 

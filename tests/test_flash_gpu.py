@@ -452,3 +452,20 @@ def test_one_own_block_per_wave_forward(causal, Lq, Lk, dk, dv, counts):
     for n in counts[:-1]:
         got = _fa()._forward(q[:, -n:].contiguous(), k[:, -n:].contiguous(), v[:, -n:].contiguous(), causal, scale)
         assert torch.equal(got[0], o[:, -n:]) and torch.equal(got[1], M[:, -n:])
+
+
+# dense split forward passes whose workgroups take a half or a quarter of the output dims: counts on both sides of the lines (256 CUs; 5 blocks of 16
+# queries to a slab), dims that fill the last part or not, a last part of one vector, the remainders of 32-key blocks
+@pytest.mark.parametrize("Lk", [1500, 2017])
+@pytest.mark.parametrize("dk,dv,counts", [(64, 64, (1, 25, 26)), (40, 40, (1, 25, 26)), (64, 128, (1, 12, 13, 25, 26)), (64, 72, (1, 17, 18, 25, 26)),
+                                          (128, 128, (1, 12, 13, 25, 26)), (80, 80, (1, 17, 18, 25, 26)), (128, 104, (1, 12, 25, 26)), (128, 24, (1, 26))])
+def test_output_dims_over_workgroups(dk, dv, counts, Lk):
+    Lq, scale = 77, 1 / math.sqrt(dk)
+    q, k, v, _ = (t.cuda() for t in orc.make_qkv(Lk + dk + dv, 1, max(counts), Lq, Lk, dk, dv, torch.bfloat16))
+    o, M = _fa()._forward(q, k, v, False, scale)
+    s = torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * scale
+    assert _rel(o, (torch.softmax(s, -1) @ v.float()).cpu()) <= 2e-2
+    assert (M - torch.logsumexp(s, -1) / math.log(2)).abs().max().item() <= 4e-2
+    for n in counts[:-1]:
+        got = _fa()._forward(q[:, :n].contiguous(), k[:, :n].contiguous(), v[:, :n].contiguous(), False, scale)
+        assert torch.equal(got[0], o[:, :n]) and torch.equal(got[1], M[:, :n])
