@@ -2,6 +2,7 @@
 // for one pair of (padded) head dims and exports their launchers.
 #include "attn_fwd_kernel.hpp"
 #include "attn_bwd_kernel.hpp"
+#include "attn_win_kernel.hpp"
 
 #define DLT_CAT3_(a, b, c) a##b##_##c
 #define DLT_CAT3(a, b, c) DLT_CAT3_(a, b, c)
@@ -68,6 +69,21 @@ int DLT_CAT3(dlt_launch_delta_, DLT_DK, DLT_DV)(const BwdArgs& a, hipStream_t st
     default: return launch_delta_t<float>(a, stream);
   }
 }
+
+#ifndef DLT_ONE_PATCH
+// fp32 windows (win_forward); `lds` holds a chunk's rows
+int DLT_CAT3(dlt_launch_win_, DLT_DK, DLT_DV)(const WinArgs& a, int bh, int lds, hipStream_t stream) {
+  auto kern = attn_win_fwd_kernel<DLT_DK, DLT_DV>;
+  int rc = set_lds_limit(kern, lds);
+  if (rc != DLT_OK) return rc;
+  const int rows = 4 >> a.wave_shift, cols = 16 << a.patch_shift;
+  dlt_timing_before(DLT_K_FWD, stream);
+  hipLaunchKernelGGL(kern, dim3(bh, (a.TR + rows - 1) / rows, (a.XL + cols - 1) / cols), dim3(256), lds, stream, a);
+  dlt_timing_after(stream);
+  DLT_CHECK_LAUNCH("windowed fp32 forward launch");
+  return DLT_OK;
+}
+#endif
 
 #ifdef DLT_ONE_PATCH
 // head-dim classes whose accumulators leave no room for two query blocks per wave: np must be 1

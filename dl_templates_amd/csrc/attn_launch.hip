@@ -1,6 +1,7 @@
 // Host side of the attention core: validation that depends on the kernels' limits, the
 // per-launch LDS / chunking plan, and dispatch to the instantiation for the padded head dims.
 #include "attn_fwd_kernel.hpp"
+#include "attn_win_kernel.hpp"
 #include "attn_bwd_kernel.hpp"
 #include "swa1_fwd_kernel.hpp"
 #include "swa1_bwd_kernel.hpp"
@@ -11,6 +12,10 @@
 
 int dlt_launch_fwd_32_32(const FwdArgs&, int, int, hipStream_t);
 int dlt_launch_fwd_64_64(const FwdArgs&, int, int, hipStream_t);
+int dlt_launch_win_32_32(const WinArgs&, int, int, hipStream_t);
+int dlt_launch_win_64_64(const WinArgs&, int, int, hipStream_t);
+int dlt_launch_win_64_128(const WinArgs&, int, int, hipStream_t);
+int dlt_launch_win_128_128(const WinArgs&, int, int, hipStream_t);
 int dlt_launch_fwd_128_128(const FwdArgs&, int, int, hipStream_t);
 int dlt_launch_fwd_64_128(const FwdArgs&, int, int, hipStream_t);
 int dlt_launch_fwd_256_256(const FwdArgs&, int, int, hipStream_t);
@@ -425,6 +430,56 @@ bool swag_f32_eligible(const AttnProblem& p, const AttnTensors& t) {
   for (int i = 0; i < 4; i++)
     if (!tvec_ok(ptrs[i], st[i], p.dk, 4) || st[i][2] < 0 || ((int64_t)p.g.TR * p.g.TC - 1) * st[i][2] * 4 + 4 * p.dk > ((int64_t)1 << 31) - 1) return false;
   return true;
+}
+
+// fp32 windows on the kernel of attn_win_kernel.hpp: rows readable in 16-byte pieces, slabs of less than 2^31 bytes, no rotation, and one halo row
+// at least fits the LDS; false: the generic kernel.  Generic -> this, us, over 150 shapes (1 ... 128 slabs, maps of 3 x 3 to 160 x 160, every head
+// dim class) 0.44 of the time in the mean and nowhere more: head dim 64, 9 x 7 columns: 2 slabs of 22 x 15 23.0 -> 7.7, 32 of 25 x 11 39.8 -> 8.5, 16 of
+// 30 x 30 30.0 -> 14.7, 64 slabs of 27 x 127 (11 x 19 columns, 64/128) 897 -> 315; 2 slabs of 3 x 128 at head dim 96 24 -> 14.
+bool win_plan(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, WinArgs& a, int& lds) {
+  if (p.g.mode != DLT_GEOM_SWA || p.tm.img || p.dtype != DLT_FP32 || dc.id == 4 || t.q_rot != nullptr || (p.rope.enabled && p.rope.R > 0)) return false;
+  const void* const ptrs[4] = {t.q, t.k, t.v, t.out_o};
+  const int64_t* const st[4] = {t.qs, t.ks, t.vs, t.os};
+  const int dims[4] = {p.dk, p.dk, p.dv, p.dv};
+  const int64_t ntok = (int64_t)p.g.TR * p.g.XLq, lim = ((int64_t)1 << 31) - 1, bh = (int64_t)p.B * p.H;
+  for (int i = 0; i < 4; i++)
+    if (!tvec_ok(ptrs[i], st[i], dims[i], 4) || st[i][2] < 0 || (ntok - 1) * st[i][2] * 4 + 4 * dims[i] > lim) return false;
+  if (t.ls[2] < 0 || (ntok - 1) * t.ls[2] > lim || bh > 1 << 23) return false;
+  a.patch_shift = p.g.XLq <= 16 ? 0 : p.g.XLq <= 32 ? 1 : 2;
+  const int cols = 16 << a.patch_shift;
+  const int64_t nx = (p.g.XLq + cols - 1) / cols, cus = dlt_device_cus();
+  auto grid = [&](int ws) { return bh * ((p.g.TR + (4 >> ws) - 1) / (4 >> ws)) * nx; };
+  // A row's halo is dealt over as many waves as keeps one and a half workgroups per CU: 64 slabs of 11 x 15 (1, 2, 4 waves to a row) 9.1, 8.2 and 11.0 us,
+  // 2 of 22 x 15 9.2, 8.1, 7.8, 64 of 19 x 16 11.1, 13.2, 18.2
+  a.wave_shift = 2;
+  while (a.wave_shift > a.patch_shift && 2 * grid(a.wave_shift) > 3 * cus) a.wave_shift--;
+  if (((int64_t)p.g.TR + 3) / (4 >> a.wave_shift) > 65535 || nx > 65535) return false;
+  const int per_tok = win_per_token(dc.DK, dc.DV), nrows = dlt_imin(2 * p.g.WR + (4 >> a.wave_shift), p.g.TR);
+  a.pair = p.g.XLq <= 16;
+  a.cx = a.pair ? 16 : p.g.XLq <= 32 ? 32 : roundup(dlt_imin(p.g.XLk, cols + (2 * p.g.WC + 2) * p.g.S) + 32, 8);
+  const int64_t row = (int64_t)a.cx * per_tok;
+  // chunks leave room for two workgroups per CU where so many run: one takes 1.1 times the time of two in the mean of those shapes, three 1.06 times
+  int budget = grid(a.wave_shift) <= cus ? LDS_TOTAL : LDS_TOTAL / 2;
+  if (row > budget) budget = LDS_TOTAL;
+  if (row > budget) return false;
+  a.chunk_rows = dlt_imin((int)(budget / row), nrows);
+  if (a.pair) a.chunk_rows = a.chunk_rows < nrows ? dlt_imax(2, a.chunk_rows & ~1) : a.chunk_rows + (a.chunk_rows & 1);
+  lds = dlt_imax((int)(a.chunk_rows * row), win_sum_bytes(dc.DV));
+  return lds <= LDS_TOTAL;
+}
+
+int win_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, WinArgs& a, int lds, hipStream_t stream) {
+  a.q = (const float*)t.q; a.k = (const float*)t.k; a.v = (const float*)t.v; a.o = (float*)t.out_o; a.lse = t.lse;
+  for (int i = 0; i < 2; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; a.ls[i] = t.ls[i]; }
+  a.qn = (int32_t)t.qs[2]; a.kn = (int32_t)t.ks[2]; a.vn = (int32_t)t.vs[2]; a.on = (int32_t)t.os[2]; a.ln = (int32_t)t.ls[2];
+  a.H = p.H; a.TR = p.g.TR; a.XL = p.g.XLq; a.S = p.g.S; a.TC = p.g.TC; a.WR = p.g.WR; a.WC = p.g.WC; a.dk = p.dk; a.dv = p.dv;
+  a.scale_log2 = p.sm_scale * 1.4426950408889634f;
+  switch (dc.id) {
+    case 0: return dlt_launch_win_64_64(a, p.B * p.H, lds, stream);
+    case 1: return dlt_launch_win_128_128(a, p.B * p.H, lds, stream);
+    case 3: return dlt_launch_win_32_32(a, p.B * p.H, lds, stream);
+    default: return dlt_launch_win_64_128(a, p.B * p.H, lds, stream);
+  }
 }
 
 int swag_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t stream) {
@@ -899,6 +954,9 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
   if (flash_eligible(p, t, false)) return flash_forward(p, t, dc, stream);
   if (swa2_tiles_eligible(p, t, false)) return swa2_forward(p, t, stream);
   if (dlt_route_note(DLT_FAMILY_GENERIC)) return DLT_OK;
+  WinArgs win;
+  int win_lds;
+  if (win_plan(p, t, dc, win, win_lds)) return win_forward(p, t, dc, win, win_lds, stream);
   const int np = (p.g.mode == DLT_GEOM_SWA || dc.id == 4) ? 1 : 2;
   const int own = 64 * np;
   // fp32 tensors: q and k rows are staged as hi + lo bf16 pairs (must match SPLIT in attn_fwd_kernel.hpp)

@@ -290,6 +290,37 @@ def test_marching_fp32(th, tw, WR, WC):
         assert (lse.cpu() - lse_w).abs().max().item() <= LSE_TOL
 
 
+# fp32 windows off the marching kernel: rows of one, two and more 16-token blocks, halo rows dealt over four waves, two and one (slab counts on both
+# sides of the lines), pairs of rows with an odd one left, several chunks (last case of each kind), tiles, every head dim class and dims below it;
+# a key row of infinities or NaN changes no query that does not see it
+@pytest.mark.parametrize("BH,S,th,tw,WR,WC,dk,dv", [
+    (1, 1, 1, 1, 0, 0, 64, 64), (2, 1, 9, 15, 4, 3, 64, 64), (40, 1, 17, 16, 2, 2, 64, 64), (150, 1, 9, 11, 3, 1, 64, 64), (3, 1, 70, 13, 40, 5, 64, 64),
+    (2, 1, 10, 17, 1, 4, 64, 64), (60, 1, 13, 31, 4, 2, 40, 64), (2, 1, 40, 32, 18, 9, 128, 128), (70, 1, 9, 24, 2, 2, 96, 80),
+    (2, 1, 7, 33, 2, 12, 64, 128), (3, 1, 5, 81, 9, 3, 64, 64), (60, 1, 6, 130, 3, 10, 64, 64), (2, 1, 25, 12, 8, 8, 32, 32), (2, 1, 25, 40, 7, 2, 24, 32),
+    (2, 4, 9, 4, 1, 2, 64, 64), (30, 4, 6, 7, 2, 1, 64, 128), (2, 16, 5, 6, 1, 1, 128, 128), (90, 16, 3, 1, 1, 1, 64, 64)])
+def test_windows_fp32(BH, S, th, tw, WR, WC, dk, dv):
+    sw = _swa()
+    from dl_templates_amd import _lib
+    N, scale, bad = th * tw * S, 0.15, (th * tw // 2) * S
+    q, k, v, _ = orc.make_qkv(N + WR + dk, 1, BH, N, N, dk, dv, torch.float32)
+    want, lse_w = orc.tiled_swa_explicit(q[:, -2:], k[:, -2:], v[:, -2:], S, th, tw, WR, WC, scale, return_lse2=True)
+    q, k, v = (t.cuda() for t in (q, k, v))
+    flat = [t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for t in (q, k, v)]   # heads inside the token rows
+    slow = [torch.stack([t, t], -1)[..., 0] for t in (q, k, v)]                          # last-dim stride 2: the generic kernel
+    for args in ((q, k, v), flat, slow):
+        o, lse = sw._forward(*args, sw._shape(*args, S, th, tw, WR, WC, scale), None)
+        assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "generic"
+        assert (o[:, -2:].cpu() - want).abs().max().item() <= FWD_TOL
+        assert (lse[:, -2:].cpu() - lse_w).abs().max().item() <= LSE_TOL
+    o = sw.tiled_swa_fwd(q, k, v, S, th, tw, WR, WC, scale)
+    cell = torch.arange(N, device="cuda") // S
+    blind = ((cell // tw - bad // S // tw).abs() > WR) | ((cell % tw - bad // S % tw).abs() > WC)
+    for value in (float("inf"), float("nan")):
+        k2 = k.clone()
+        k2[:, :, bad] = value
+        assert (sw.tiled_swa_fwd(q, k2, v, S, th, tw, WR, WC, scale)[:, :, blind] - o[:, :, blind]).abs().sum().item() <= FWD_TOL * BH * N
+
+
 # two stacked patches per wave (streaming kernels, more workgroups than CUs): bands without a lower patch, one band and a bit, ragged
 # columns, both window classes, windows in column passes, tiles of 4 tokens, K and V at one token stride and apart
 @pytest.mark.parametrize("B,H,S,th,tw,WR,WC,d", [(1, 300, 1, 3, 5, 7, 7, 128), (1, 300, 1, 4, 16, 2, 3, 128), (1, 150, 1, 9, 15, 10, 10, 128), (2, 40, 1, 17, 18, 3, 8, 128),
