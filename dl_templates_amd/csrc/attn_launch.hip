@@ -432,12 +432,13 @@ bool swag_f32_eligible(const AttnProblem& p, const AttnTensors& t) {
   return true;
 }
 
-// fp32 windows on the kernel of attn_win_kernel.hpp: rows readable in 16-byte pieces, slabs of less than 2^31 bytes, no rotation, and one halo row
-// at least fits the LDS; false: the generic kernel.  Generic -> this, us, over 150 shapes (1 ... 128 slabs, maps of 3 x 3 to 160 x 160, every head
-// dim class) 0.44 of the time in the mean and nowhere more: head dim 64, 9 x 7 columns: 2 slabs of 22 x 15 23.0 -> 7.7, 32 of 25 x 11 39.8 -> 8.5, 16 of
+// fp32 windows on the kernel of attn_win_kernel.hpp: one token to a tile (larger ones keep the bits of the image layout, which the generic kernel
+// serves), rows readable in 16-byte pieces, slabs of less than 2^31 bytes, no rotation, and one halo row
+// at least fits the LDS; false: the generic kernel.  Generic -> this, us, over 97 shapes (1 ... 128 slabs, maps of 3 x 3 to 160 x 160, every head
+// dim class) 0.39 of the time in the mean, 0.72 at most: head dim 64, 9 x 7 columns: 2 slabs of 22 x 15 23.0 -> 7.7, 32 of 25 x 11 39.8 -> 8.5, 16 of
 // 30 x 30 30.0 -> 14.7, 64 slabs of 27 x 127 (11 x 19 columns, 64/128) 897 -> 315; 2 slabs of 3 x 128 at head dim 96 24 -> 14.
 bool win_plan(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, WinArgs& a, int& lds) {
-  if (p.g.mode != DLT_GEOM_SWA || p.tm.img || p.dtype != DLT_FP32 || dc.id == 4 || t.q_rot != nullptr || (p.rope.enabled && p.rope.R > 0)) return false;
+  if (p.g.mode != DLT_GEOM_SWA || p.g.S != 1 || p.tm.img || p.dtype != DLT_FP32 || dc.id == 4 || t.q_rot != nullptr || (p.rope.enabled && p.rope.R > 0)) return false;
   const void* const ptrs[4] = {t.q, t.k, t.v, t.out_o};
   const int64_t* const st[4] = {t.qs, t.ks, t.vs, t.os};
   const int dims[4] = {p.dk, p.dk, p.dv, p.dv};
@@ -456,7 +457,7 @@ bool win_plan(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, Wi
   if (((int64_t)p.g.TR + 3) / (4 >> a.wave_shift) > 65535 || nx > 65535) return false;
   const int per_tok = win_per_token(dc.DK, dc.DV), nrows = dlt_imin(2 * p.g.WR + (4 >> a.wave_shift), p.g.TR);
   a.pair = p.g.XLq <= 16;
-  a.cx = a.pair ? 16 : p.g.XLq <= 32 ? 32 : roundup(dlt_imin(p.g.XLk, cols + (2 * p.g.WC + 2) * p.g.S) + 32, 8);
+  a.cx = a.pair ? 16 : p.g.XLq <= 32 ? 32 : roundup(dlt_imin(p.g.XLk, cols + 2 * p.g.WC + 2) + 32, 8);
   const int64_t row = (int64_t)a.cx * per_tok;
   // chunks leave room for two workgroups per CU where so many run: one takes 1.1 times the time of two in the mean of those shapes, three 1.06 times
   int budget = grid(a.wave_shift) <= cus ? LDS_TOTAL : LDS_TOTAL / 2;
@@ -472,7 +473,7 @@ int win_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, 
   a.q = (const float*)t.q; a.k = (const float*)t.k; a.v = (const float*)t.v; a.o = (float*)t.out_o; a.lse = t.lse;
   for (int i = 0; i < 2; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; a.ls[i] = t.ls[i]; }
   a.qn = (int32_t)t.qs[2]; a.kn = (int32_t)t.ks[2]; a.vn = (int32_t)t.vs[2]; a.on = (int32_t)t.os[2]; a.ln = (int32_t)t.ls[2];
-  a.H = p.H; a.TR = p.g.TR; a.XL = p.g.XLq; a.S = p.g.S; a.TC = p.g.TC; a.WR = p.g.WR; a.WC = p.g.WC; a.dk = p.dk; a.dv = p.dv;
+  a.H = p.H; a.TR = p.g.TR; a.XL = p.g.XLq; a.WR = p.g.WR; a.WC = p.g.WC; a.dk = p.dk; a.dv = p.dv;
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   switch (dc.id) {
     case 0: return dlt_launch_win_64_64(a, p.B * p.H, lds, stream);

@@ -16,7 +16,7 @@ struct WinArgs {
   float *o, *lse;
   int64_t qs[2], ks[2], vs[2], os[2], ls[2];    // batch, head strides (elements)
   int32_t qn, kn, vn, on, ln;                   // token strides (elements; a slab spans less than 2^31 bytes)
-  int32_t H, TR, XL, S, TC, WR, WC;
+  int32_t H, TR, XL, WR, WC;
   int32_t dk, dv;
   int32_t patch_shift;   // 1 << patch_shift blocks of 16 queries lie side by side
   int32_t wave_shift;    // 1 << wave_shift waves share a grid row: the blocks, times the parts its halo rows are dealt in
@@ -84,8 +84,8 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
   const bool live = r <= rlast && xw <= xlast;
 
   // columns [lo, hi) that queries x1 ... x2 see
-  auto first = [&](int x) { return dlt_imax((a.S == 1 ? x : x / a.S) - a.WC, 0) * a.S; };
-  auto past = [&](int x) { return dlt_imin((a.S == 1 ? x : x / a.S) + a.WC + 1, a.TC) * a.S; };
+  auto first = [&](int x) { return dlt_imax(x - a.WC, 0); };
+  auto past = [&](int x) { return dlt_imin(x + a.WC + 1, a.XL); };
   const int rlo = dlt_imax(r0 - a.WR, 0), rhi = dlt_imin(rlast + a.WR, a.TR - 1);
   const int wrlo = dlt_imax(r - a.WR, 0), wrhi = live ? dlt_imin(r + a.WR, a.TR - 1) : -1;
   const int X0 = first(x0), w = past(xlast) - X0;
