@@ -757,6 +757,30 @@ int64_t flash_part_fwd(const AttnProblem& p, const FlashPlan& f) {
 int64_t flash_part_q(const AttnProblem& p, const FlashPlan& f) { return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLq * p.dk : 0; }
 int64_t flash_part_kv(const AttnProblem& p, const FlashPlan& f) { return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLk * (p.dk + p.dv) : 0; }
 
+// Windows over tiles of 16 k tokens off the marching kernels: whether the kernels of flash_split_kernel.hpp run, which take 16 own tokens to a
+// workgroup and deal the window's keys over its waves, so that a call of few tiles is not a handful of workgroups with 64 keys after the other.
+// Tiles of 64 k tokens stay on the asynchronously staged kernels (0.67 ... 1.1 of whose time it takes up to 256 blocks), where a slab's bits do not
+// depend on the call.  A workgroup's time is a0 + a1 + a2 per key, one per CU and a3 of them at once, that of the chunked kernels
+// b0 + b1 + b2 per 64 keys, b3 workgroups per CU at once; fitted to 1717 shapes (us), rms 7 and 13 %, so 15 % are asked for.  Chosen that way a forward pass takes
+// 0.59 (d = 32), 0.73 and 0.80 (128) of the chunked time in the mean of shapes of 9 ... 60000 tiles, a backward pass 0.63, 0.74, 0.94, none over 1.10:
+// windows of 5 x 3 tiles of 16, d = 64, 8 slabs of 7 x 6 forward 17.5 -> 7.6 us and backward 32.7 -> 17.1, 2 slabs of 6 x 11 forward 22.9 -> 6.2.
+bool flash_tiles_split(const AttnProblem& p, const DimClass& dc, bool backward) {
+  const DltGeom& g = p.g;
+  if (g.mode != DLT_GEOM_SWA || g.S % 64 == 0) return false;
+  const int64_t cus = dlt_device_cus(), bh = (int64_t)p.B * p.H, blocks = bh * g.TR * (g.XLk / 16);
+  if (blocks > 0x7fffffff || (int64_t)g.TR * g.XLk > 0x7fffffff) return false;
+  static const struct { float a0, a1, a2, a3, b0, b1, b2, b3; } COST[3][2] = {   // d = 32, 64, 128; forward, backward
+    {{4.9f, .52f, .00068f, .54f, 4.8f, .52f, 1.1f, 2.2f}, {7.9f, 1.4f, .0019f, .60f, 7.9f, 2.8f, 1.9f, 2.2f}},
+    {{4.7f, 1.2f, .0027f, .79f, 3.5f, 1.8f, 1.3f, 1.8f}, {7.4f, 3.3f, .0051f, .65f, 4.0f, 6.5f, 2.7f, 1.6f}},
+    {{4.0f, 2.9f, .0056f, .69f, 2.8f, 3.9f, 1.8f, 1.4f}, {7.5f, 8.4f, .0100f, .66f, 6.5f, 7.0f, 2.1f, 1.3f}}};
+  const auto& c = COST[dc.id == 3 ? 0 : dc.id == 0 ? 1 : 2][backward];
+  const int rows = dlt_imin(g.TR, 2 * g.WR + 1), own = 64 * (backward ? flash_np_q(dc.DK, dc.DV) : FLASH_NP);
+  const int64_t cols = own + 2 * (int64_t)g.WC * g.S + (own % g.S ? g.S : 0), wgs = bh * g.TR * ((g.XLk + own - 1) / own);
+  const float keys = (float)rows * dlt_imin(g.TC, 2 * g.WC + 1) * g.S, chunks = (float)rows * (((cols < g.XLk ? cols : g.XLk) + 63) / 64);
+  const float split = c.a0 + fmaxf(1.f, blocks / (c.a3 * cus)) * (c.a1 + c.a2 * keys), chunked = c.b0 + fmaxf(1.f, wgs / (c.b3 * cus)) * (c.b1 + c.b2 * chunks);
+  return split < .85f * chunked;
+}
+
 int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {
   if (dlt_route_note(DLT_FAMILY_FLASH)) return DLT_OK;
   FlashArgs a;
@@ -796,13 +820,17 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
     a.slim = np == FLASH_SLIM ? (four ? 4 : 8) : long_chunks ? (four ? 4 : nbh * ((a.Lq + 127) / 128) <= most ? 8 : 0) : 0;
     a.share.n = f.n; a.share.len = f.len;
   }
+  if (flash_tiles_split(p, dc, false)) {
+    np = FLASH_SPLIT1;
+    a.Lq = a.Lk = p.g.TR * p.g.XLq;
+  }
   const bool split = np == FLASH_SPLIT1 || np == FLASH_SPLIT2;
   // Dense split calls with one block of 16: as many workgroups to a block as leave one per CU (bits are equal, so the line may look at the real
   // count).  Over 18096 shapes of 1 ... 16 slabs two take 0.94 ... 0.96 of one's time at 64/64, 0.89 ... 0.92 at 64/128 and 0.94 ... 0.97 at
   // 128/128, four another 0.94 ... 0.98 of two's there (77 x 1500, 16 slabs, 64/64: 11.5 -> 10.8 us); with more workgroups than CUs either takes
   // 1.17 ... 1.3, and under a mask, where the longest row decides, 0.99 ... 1.01.
   a.part_dv = dc.DV;
-  if (np == FLASH_SPLIT1 && !a.causal)
+  if (np == FLASH_SPLIT1 && !a.causal && !a.tile)
     for (int w = dc.DV / 2; w >= 32 && 4 * w >= dc.DV; w /= 2)
       if ((int64_t)p.B * p.H * ((a.Lq + 15) / 16) * ((a.dv + w - 1) / w) <= dlt_device_cus()) a.part_dv = w;
   int rc;
@@ -880,6 +908,10 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
     fq = flash_plan(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0, may_split);
     may_split = may_split && dlt_flash_scalars_fit(a);   // else dK/dV stays on the register-staged kernel
     fkv = flash_plan(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0, may_split);
+  }
+  if (flash_tiles_split(p, dc, true)) {
+    fq.kind = fkv.kind = FLASH_SPLIT1;
+    a.Lq = a.Lk = p.g.TR * p.g.XLq;
   }
   const int np_q = fq.kind, np_kv = fkv.kind;
   a.share_q = {t.part, fq.n, fq.len};

@@ -21,10 +21,15 @@ int flashs_run(KernT kern, const Args& a, int lds, int grid, int id, hipStream_t
   return DLT_OK;
 }
 
+// (tiles: one own block, all output dims)
+template <typename Args, typename KernT>
+KernT flashs_mode(const Args& a, KernT dense, KernT causal, KernT tiles, KernT image) { return a.tile ? (a.tm.img ? image : tiles) : a.causal ? causal : dense; }
+
 template <typename TIO, int NP, int DV>
 int flashs_fwd_dv(FlashArgs a, hipStream_t stream) {
   a.parts = (a.dv + DV - 1) / DV;
-  return flashs_run(a.causal ? flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, true> : flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, false>, a,
+  return flashs_run(flashs_mode(a, flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, 0>, flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, 1>, 
+                                flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, NP == 1 && DV == DLT_DV ? 2 : 0>, flashs_fwd_kernel<TIO, DLT_DK, DV, NP, NW, NP == 1 && DV == DLT_DV ? 3 : 0>), a,
                     flashs_lds_fwd<DLT_DK, DV, NP, NW>(), a.B * a.H * a.nblk * a.parts, DLT_K_FWD, stream);
 }
 template <typename TIO, int NP>
@@ -39,13 +44,15 @@ int flashs_fwd(FlashArgs a, hipStream_t stream) {
 template <typename TIO, int NP>
 int flashs_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   a.nblk_q = (a.Lq + 16 * NP - 1) / (16 * NP);
-  return flashs_run(a.causal ? flashs_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, NW, true> : flashs_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, NW, false>, a,
+  return flashs_run(flashs_mode(a, flashs_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, NW, 0>, flashs_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, NW, 1>, 
+                                flashs_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, NW, NP == 1 ? 2 : 0>, flashs_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, NW, NP == 1 ? 3 : 0>), a,
                     flashs_lds_q<DLT_DK, DLT_DV, NP, NW>(), a.B * a.H * a.nblk_q, DLT_K_BWD_Q, stream);
 }
 template <typename TIO, int NP>
 int flashs_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   a.nblk_k = (a.Lk + 16 * NP - 1) / (16 * NP);
-  return flashs_run(a.causal ? flashs_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, NW, true> : flashs_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, NW, false>, a,
+  return flashs_run(flashs_mode(a, flashs_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, NW, 0>, flashs_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, NW, 1>, 
+                                flashs_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, NW, NP == 1 ? 2 : 0>, flashs_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, NW, NP == 1 ? 3 : 0>), a,
                     flashs_lds_kv<DLT_DK, DLT_DV, NP, NW>(), a.B * a.H * a.nblk_k, DLT_K_BWD_KV, stream);
 }
 }  // namespace

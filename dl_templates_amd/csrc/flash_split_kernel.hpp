@@ -13,17 +13,77 @@
 
 template <int D> DLT_DEV int flashs_swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : (t & 7) * (D / 64); }
 
+// The other side's tokens as a list, in blocks of 32.  MODE 0 dense, 1 causal: tokens 0 ... len - 1, reads clamped to the last one.
+template <int MODE>
+struct FlashsList {
+  int len;
+  DLT_DEV int token(int b, int half, int i) const { return dlt_imin(32 * b + 16 * half + i, len - 1); }
+};
+// 2 (3: tensors in the image layout): the window of own token x0 over tiles of S = 16 k tokens, which its whole block shares: runs of `pieces` x 16 tokens, one per grid row, and no
+// pair of tokens in it is masked.  The window is symmetric: queries that see a key are listed the same way.
+template <>
+struct FlashsList<2> {
+  int len, first, row, pieces;
+  unsigned magic;       // ceil(2^32 / pieces)
+  DLT_DEV FlashsList(const DltGeom& g, int x0) {
+    const int r = x0 / g.XLk, c = (x0 - r * g.XLk) / g.S;
+    const int rlo = dlt_imax(r - g.WR, 0), rhi = dlt_imin(r + g.WR, g.TR - 1), clo = dlt_imax(c - g.WC, 0), chi = dlt_imin(c + g.WC, g.TC - 1);
+    row = g.XLk;
+    first = rlo * row + clo * g.S;
+    pieces = (chi - clo + 1) * (g.S / 16);
+    len = 16 * pieces * (rhi - rlo + 1);
+    magic = 0xffffffffu / (unsigned)pieces + 1;
+  }
+  DLT_DEV int token(int b, int half, int i) const {
+    const int p = dlt_imin(2 * b + half, len / 16 - 1), r = pieces == 1 ? p : (int)__umulhi((unsigned)p, magic);
+    return first + r * row + 16 * (p - r * pieces) + i;
+  }
+};
+
+template <> struct FlashsList<3> : FlashsList<2> { using FlashsList<2>::FlashsList; };
+template <int MODE>
+DLT_DEV FlashsList<MODE> flashs_list(const DltGeom& g, int len, int x0) {
+  if constexpr (MODE >= 2) return FlashsList<MODE>(g, x0);
+  else return FlashsList<MODE>{len};
+}
+// elements between a slab's start and token x; Rows: the same in 32 bits and bytes for the other side's tokens
+template <int MODE>
+DLT_DEV int64_t flashs_at(const DltTokMap& tm, const int64_t (&s)[5], int x) {
+  if constexpr (MODE == 3) return tok_addr(s, tm)(x);
+  else return x * s[2];
+}
+template <int MODE>
+struct FlashsRows {
+  int sn2;
+  DLT_DEV FlashsRows(const DltTokMap&, const int64_t (&s)[5]) : sn2((int)s[2] * 2) {}
+  DLT_DEV int operator()(int token) const { return token * sn2; }
+};
+template <>
+struct FlashsRows<3> {
+  int sn2, sy2;
+  const DltTokMap& tm;
+  DLT_DEV FlashsRows(const DltTokMap& m, const int64_t (&s)[5]) : sn2((int)s[2] * 2), sy2((int)s[4] * 2), tm(m) {}
+  DLT_DEV int operator()(int token) const {
+    uint32_t y, x;
+    dlt_token_pixel(tm, (uint32_t)token, y, x);
+    return (int)y * sy2 + (int)x * sn2;
+  }
+};
+
 // wave-private [32 tokens][D] tile, rows of 2 D bytes, 16-byte piece p of token t at p ^ swz(t)
 template <int D>
 struct FlashsTile {
   static constexpr int BYTES = 64 * D, NV = D / 16;   // 16-byte vectors per lane of one block
-  // rows of block `b` (tokens clamped to the last one), pieces past `dact` are zero
-  static DLT_DEV void load(u32x4 (&r)[NV], const char* base, int sn2, int b, int len, int dact, int lane) {
+  // rows of block `b`; pieces past `dact` are left as they are (zero, from the caller).  A lane has one piece of every row: one branch, inside which the
+  // loads follow each other
+  template <typename Rows, typename List>
+  static DLT_DEV void load(u32x4 (&r)[NV], const char* base, const Rows& at, int b, const List& list, int dact, int lane) {
+    const int p = lane % (D / 8);
+    if (8 * p >= dact) return;
 #pragma unroll
     for (int it = 0; it < NV; it++) {
-      const int v = lane + 64 * it, t = v / (D / 8), p = v % (D / 8);
-      r[it] = u32x4{0u, 0u, 0u, 0u};
-      if (8 * p < dact) r[it] = *reinterpret_cast<const u32x4*>(base + (uint32_t)(dlt_imin(32 * b + t, len - 1) * sn2 + 16 * p));
+      const int t = (lane + 64 * it) / (D / 8), half = 64 * it / (D / 8) / 16;
+      r[it] = *reinterpret_cast<const u32x4*>(base + (uint32_t)(at(list.token(b, half, t - 16 * half)) + 16 * p));
     }
   }
   static DLT_DEV void write(char* s, const u32x4 (&r)[NV], int lane) {
@@ -46,17 +106,26 @@ struct FlashsTile {
   }
 };
 
-// A operand rows straight from HBM: 32 tokens of block b
-template <int D>
-DLT_DEV void flashs_load_rows(u32x4 (&f)[2][D / 32], const char* base, int sn2, int b, int len, int dact, int n, int g) {
+// A operand rows straight from HBM: 32 tokens of block b (pieces past `dact`: as above)
+template <int D, typename Rows, typename List>
+DLT_DEV void flashs_load_rows(u32x4 (&f)[2][D / 32], const char* base, const Rows& at, int b, const List& list, int dact, int n, int g) {
 #pragma unroll
-  for (int mb = 0; mb < 2; mb++)
+  for (int c = 0; c < D / 32; c++)
+    if (8 * (4 * c + g) < dact) {
 #pragma unroll
-    for (int c = 0; c < D / 32; c++) {
-      f[mb][c] = u32x4{0u, 0u, 0u, 0u};
-      if (8 * (4 * c + g) < dact)
-        f[mb][c] = *reinterpret_cast<const u32x4*>(base + (uint32_t)(dlt_imin(32 * b + 16 * mb + n, len - 1) * sn2 + 64 * c + 16 * g));
+      for (int mb = 0; mb < 2; mb++) f[mb][c] = *reinterpret_cast<const u32x4*>(base + (uint32_t)(at(list.token(b, mb, n)) + 64 * c + 16 * g));
     }
+}
+// an own row's operands, one lane's 8 dims of every 32
+template <int N, typename T>
+DLT_DEV void flashs_own(u32x4 (&f)[N], const T* row, int dact, int g) {
+#pragma unroll
+  for (int c = 0; c < N; c++) f[c] = *reinterpret_cast<const u32x4*>(row + (8 * (4 * c + g) < dact ? 32 * c + 8 * g : 0));
+}
+template <int N>
+DLT_DEV void flashs_own_zero(u32x4 (&f)[N], int dact, int g) {
+#pragma unroll
+  for (int c = 0; c < N; c++) f[c] = 8 * (4 * c + g) < dact ? f[c] : u32x4{0u, 0u, 0u, 0u};
 }
 
 // Partial [16 NP][D] results of NW waves (C layout: lane n = own token, dims 16 d + 4 g + i) -> their sum, 8 dims per thread and
@@ -104,9 +173,10 @@ constexpr int flashs_lds_fwd() {
 // a.parts workgroups take DV of an own block's output dims each: scores and softmax are formed in every one of them, K is read by all and V by
 // one.  A CU reads the other side at 55 B/ns whatever the others do, so narrower parts take less time while CUs are idle (flash_forward has the
 // line and figures), with the same bits.
-template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
+template <typename TIO, int DK, int DV, int NP, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const FlashArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
+  constexpr bool CAUSAL = MODE == 1;
   extern __shared__ __align__(16) char smem[];
   constexpr int KC = DK / 32, VB = DV / 16;
   typedef FlashsTile<DV> VT;
@@ -120,27 +190,27 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
   const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1] + v0);
-  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
-  const int len = CAUSAL ? dlt_imin(a.Lk, x0 + 16 * NP) : a.Lk;   // causal: keys up to the last own query
-  const int nkb = (len + 31) / 32;
+  const FlashsRows<MODE> ksn(a.tm, a.ks), vsn(a.tm, a.vs);
+  const FlashsList<MODE> keys = flashs_list<MODE>(a.g, a.Lk, x0);
+  const int nkb = ((CAUSAL ? dlt_imin(keys.len, x0 + 16 * NP) : keys.len) + 31) / 32;   // causal: keys up to the last own query
   char* sV = smem + wave * VT::BYTES;
 
-  u32x4 kf[2][KC], vr[VT::NV];
+  u32x4 kf[2][KC] = {}, vr[VT::NV] = {};
   if (wave < nkb) {
-    flashs_load_rows<DK>(kf, kb_, ksn, wave, a.Lk, a.dk, n, g);
-    VT::load(vr, vb_, vsn, wave, a.Lk, dv, lane);
+    flashs_load_rows<DK>(kf, kb_, ksn, wave, keys, a.dk, n, g);
+    VT::load(vr, vb_, vsn, wave, keys, dv, lane);
   }
-  RopeDev no_rope = RopeDev{};
   u32x4 qf[NP][KC];
 #pragma unroll
   for (int p = 0; p < NP; p++) {
     const int x = x0 + 16 * p + n;
-    swa1_load_own<TIO, CT, DK>(qf[p], qb, 1, a.dk, x < a.Lq ? x * a.qs[2] : (int64_t)-1, g, no_rope, false);
+    flashs_own(qf[p], qb + flashs_at<MODE>(a.tm, a.qs, dlt_imin(x, a.Lq - 1)), a.dk, g);
   }
   float m_run[NP], l_run[NP];
   f32x4 acc[NP][VB];
 #pragma unroll
   for (int p = 0; p < NP; p++) {
+    flashs_own_zero(qf[p], x0 + 16 * p + n < a.Lq ? a.dk : 0, g);
     m_run[p] = -INFINITY;
     l_run[p] = 0.f;
 #pragma unroll
@@ -155,10 +225,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
 #pragma unroll
       for (int c = 0; c < KC; c++) ka[mb][c] = kf[mb][c];
     if (kb + NW < nkb) {
-      flashs_load_rows<DK>(kf, kb_, ksn, kb + NW, a.Lk, a.dk, n, g);
-      VT::load(vr, vb_, vsn, kb + NW, a.Lk, dv, lane);
+      flashs_load_rows<DK>(kf, kb_, ksn, kb + NW, keys, a.dk, n, g);
+      VT::load(vr, vb_, vsn, kb + NW, keys, dv, lane);
     }
-    const bool tail = 32 * kb + 32 > a.Lk || (CAUSAL && 32 * kb + 31 > x0);
+    const bool tail = 32 * kb + 32 > keys.len || (CAUSAL && 32 * kb + 31 > x0);
     u32x4 pb[NP];
 #pragma unroll
     for (int p = 0; p < NP; p++) {
@@ -170,7 +240,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
       }
       float t[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
       if (tail) {
-        const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, a.Lk - 1) : a.Lk - 1;
+        const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, keys.len - 1) : keys.len - 1;
 #pragma unroll
         for (int i = 0; i < 8; i++) t[i] = 32 * kb + 16 * (i >> 2) + 4 * g + (i & 3) <= klim ? t[i] : -INFINITY;
       }
@@ -242,7 +312,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
     const float inv = l > 0.f ? fast_rcp(l) : 0.f;
 #pragma unroll
     for (int j = 0; j < 8; j++) v[j] *= inv;
-    Io<TIO, CT>::store8(ob + (x0 + row) * a.os[2] + (v0 + d0) * a.os[3], v, a.o_vec != 0, a.os[3], dlt_imin(8, dv - d0));
+    Io<TIO, CT>::store8(ob + flashs_at<MODE>(a.tm, a.os, x0 + row) + (v0 + d0) * a.os[3], v, a.o_vec != 0, a.os[3], dlt_imin(8, dv - d0));
     if (d0 == 0 && part == 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + (x0 + row) * a.ls[2]), m * scale + fast_log2(l));
   });
 }
@@ -254,9 +324,10 @@ constexpr int flashs_lds_q() {
 }
 
 // dQ: own = queries, the waves split the keys; delta of the own queries is formed (fuse_delta) and stored on the way
-template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
+template <typename TIO, int DK, int DV, int NP, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
+  constexpr bool CAUSAL = MODE == 1;
   extern __shared__ __align__(16) char smem[];
   constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16;
   typedef FlashsTile<DK> KT;
@@ -271,17 +342,16 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
   const TIO* ob = reinterpret_cast<const TIO*>(a.o) + b * a.os[0] + h * a.os[1];
   const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1]);
   const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1]);
-  const int ksn = (int)a.ks[2] * 2, vsn = (int)a.vs[2] * 2;
-  const int len = CAUSAL ? dlt_imin(a.Lk, x0 + 16 * NP) : a.Lk;
-  const int nkb = (len + 31) / 32;
+  const FlashsRows<MODE> ksn(a.tm, a.ks), vsn(a.tm, a.vs);
+  const FlashsList<MODE> keys = flashs_list<MODE>(a.g, a.Lk, x0);
+  const int nkb = ((CAUSAL ? dlt_imin(keys.len, x0 + 16 * NP) : keys.len) + 31) / 32;
   char* sK = smem + wave * KT::BYTES;
 
-  u32x4 kr[KT::NV], vf[2][VC];
+  u32x4 kr[KT::NV] = {}, vf[2][VC] = {};
   if (wave < nkb) {
-    KT::load(kr, kb_, ksn, wave, a.Lk, a.dk_, lane);
-    flashs_load_rows<DV>(vf, vb_, vsn, wave, a.Lk, a.dv_, n, g);
+    KT::load(kr, kb_, ksn, wave, keys, a.dk_, lane);
+    flashs_load_rows<DV>(vf, vb_, vsn, wave, keys, a.dv_, n, g);
   }
-  RopeDev no_rope = RopeDev{};
   u32x4 qf[NP][KC], dof[NP][VC];
   float nlse[NP];
   f32x4 dinit[NP], acc[NP][KB];
@@ -289,14 +359,17 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
   for (int p = 0; p < NP; p++) {
     const int x = x0 + 16 * p + n;
     const bool in = x < a.Lq;
-    swa1_load_own<TIO, CT, DK>(qf[p], qb, 1, a.dk_, in ? x * a.qs[2] : (int64_t)-1, g, no_rope, false);
-    swa1_load_own<TIO, CT, DV>(dof[p], dob, 1, a.dv_, in ? x * a.dos[2] : (int64_t)-1, g, no_rope, false);
-    const int64_t off = b * a.ls[0] + h * a.ls[1] + (in ? x : 0) * a.ls[2];
-    nlse[p] = in ? -a.lse[off] : 0.f;
+    const int xc = dlt_imin(x, a.Lq - 1);
+    flashs_own(qf[p], qb + flashs_at<MODE>(a.tm, a.qs, xc), a.dk_, g);
+    flashs_own(dof[p], dob + flashs_at<MODE>(a.tm, a.dos, xc), a.dv_, g);
+    const int64_t off = b * a.ls[0] + h * a.ls[1] + xc * a.ls[2];
+    nlse[p] = a.lse[off];
     float del;
     if (a.fuse_delta != 0) {
       u32x4 of[VC];
-      swa1_load_own<TIO, CT, DV>(of, ob, 1, a.dv_, in ? x * a.os[2] : (int64_t)-1, g, no_rope, false);
+      flashs_own(of, ob + flashs_at<MODE>(a.tm, a.os, xc), a.dv_, g);
+      flashs_own_zero(of, in ? a.dv_ : 0, g);
+      flashs_own_zero(dof[p], in ? a.dv_ : 0, g);
       float part = 0.f;
 #pragma unroll
       for (int c = 0; c < VC; c++) {
@@ -309,8 +382,11 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
       del = wave_sum4(part);
       if (wave == 0 && g == 0 && in) store_stream4(a.delta_out + off, del);
     } else {
+      flashs_own_zero(dof[p], in ? a.dv_ : 0, g);
       del = in ? a.delta[off] : 0.f;
     }
+    flashs_own_zero(qf[p], in ? a.dk_ : 0, g);
+    nlse[p] = in ? -nlse[p] : 0.f;
     dinit[p] = f32x4{-del, -del, -del, -del};
 #pragma unroll
     for (int d = 0; d < KB; d++) acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -324,10 +400,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
 #pragma unroll
       for (int c = 0; c < VC; c++) va[mb][c] = vf[mb][c];
     if (kb + NW < nkb) {
-      KT::load(kr, kb_, ksn, kb + NW, a.Lk, a.dk_, lane);
-      flashs_load_rows<DV>(vf, vb_, vsn, kb + NW, a.Lk, a.dv_, n, g);
+      KT::load(kr, kb_, ksn, kb + NW, keys, a.dk_, lane);
+      flashs_load_rows<DV>(vf, vb_, vsn, kb + NW, keys, a.dv_, n, g);
     }
-    const bool tail = 32 * kb + 32 > a.Lk || (CAUSAL && 32 * kb + 31 > x0);
+    const bool tail = 32 * kb + 32 > keys.len || (CAUSAL && 32 * kb + 31 > x0);
     u32x4 dsb[NP];
     float ds[NP][8];
 #pragma unroll
@@ -342,7 +418,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
         for (int c = 0; c < KC; c++) s = Mma<CT>::mfma(ka[c], qf[p][c], s);
 #pragma unroll
         for (int c = 0; c < VC; c++) dp = Mma<CT>::mfma(va[mb][c], dof[p][c], dp);
-        const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, a.Lk - 1) : a.Lk - 1;
+        const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, keys.len - 1) : keys.len - 1;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           float pv = fast_exp2(fmaf(s[i], scale, nlse[p]));
@@ -369,7 +445,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
     if (x0 + row >= a.Lq || d0 >= a.dk_) return;
 #pragma unroll
     for (int j = 0; j < 8; j++) v[j] *= a.sm_scale;
-    Io<TIO, CT>::store8(dqb + (x0 + row) * a.dqs[2] + d0 * a.dqs[3], v, a.dq_vec != 0, a.dqs[3], dlt_imin(8, a.dk_ - d0));
+    Io<TIO, CT>::store8(dqb + flashs_at<MODE>(a.tm, a.dqs, x0 + row) + d0 * a.dqs[3], v, a.dq_vec != 0, a.dqs[3], dlt_imin(8, a.dk_ - d0));
   });
 }
 
@@ -381,9 +457,10 @@ constexpr int flashs_lds_kv() {
 }
 
 // dK / dV: own = keys, the waves split the queries
-template <typename TIO, int DK, int DV, int NP, int NW, bool CAUSAL>
+template <typename TIO, int DK, int DV, int NP, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
+  constexpr bool CAUSAL = MODE == 1;
   extern __shared__ __align__(16) char smem[];
   constexpr int KC = DK / 32, VC = DV / 32, KB = DK / 16, VB = DV / 16;
   typedef FlashsTile<DK> QT;
@@ -399,29 +476,32 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
   const char* dob = reinterpret_cast<const char*>(reinterpret_cast<const TIO*>(a.d_o) + b * a.dos[0] + h * a.dos[1]);
   // lanes 0 ... 31 fetch lse2, lanes 32 ... 63 delta of a block's queries
   const float* scb = (lane < 32 ? a.lse : a.delta) + b * a.ls[0] + h * a.ls[1];
-  const int qsn = (int)a.qs[2] * 2, dosn = (int)a.dos[2] * 2;
-  const int nqb = (a.Lq + 31) / 32;
+  const FlashsRows<MODE> qsn(a.tm, a.qs), dosn(a.tm, a.dos);
+  const FlashsList<MODE> queries = flashs_list<MODE>(a.g, a.Lq, x0);
+  const int nqb = (queries.len + 31) / 32;
   char* sQ = smem + wave * (QT::BYTES + DT::BYTES + 256);
   char* sD = sQ + QT::BYTES;
   float* sc = reinterpret_cast<float*>(sD + DT::BYTES);
 
-  u32x4 qr[QT::NV], dr[DT::NV];
+  u32x4 qr[QT::NV] = {}, dr[DT::NV] = {};
   float scr = 0.f;
   const int first = (CAUSAL ? x0 / 32 : 0) + wave;   // causal: queries below the first own key see none of the own keys
   auto fetch = [&](int blk) {
-    QT::load(qr, qb, qsn, blk, a.Lq, a.dk_, lane);
-    DT::load(dr, dob, dosn, blk, a.Lq, a.dv_, lane);
-    scr = scb[dlt_imin(32 * blk + (lane & 31), a.Lq - 1) * a.ls[2]];
+    QT::load(qr, qb, qsn, blk, queries, a.dk_, lane);
+    DT::load(dr, dob, dosn, blk, queries, a.dv_, lane);
+    if constexpr (MODE >= 2) scr = scb[((lane & 16) ? queries.token(blk, 1, lane & 15) : queries.token(blk, 0, lane & 15)) * a.ls[2]];
+    else scr = scb[dlt_imin(32 * blk + (lane & 31), queries.len - 1) * a.ls[2]];
   };
   if (first < nqb) fetch(first);
-  RopeDev no_rope = RopeDev{};
   u32x4 kf[NP][KC], vf[NP][VC];
   f32x4 acc_k[NP][KB], acc_v[NP][VB];
 #pragma unroll
   for (int p = 0; p < NP; p++) {
     const int x = x0 + 16 * p + n;
-    swa1_load_own<TIO, CT, DK>(kf[p], kb_, 1, a.dk_, x < a.Lk ? x * a.ks[2] : (int64_t)-1, g, no_rope, false);
-    swa1_load_own<TIO, CT, DV>(vf[p], vb_, 1, a.dv_, x < a.Lk ? x * a.vs[2] : (int64_t)-1, g, no_rope, false);
+    flashs_own(kf[p], kb_ + flashs_at<MODE>(a.tm, a.ks, dlt_imin(x, a.Lk - 1)), a.dk_, g);
+    flashs_own(vf[p], vb_ + flashs_at<MODE>(a.tm, a.vs, dlt_imin(x, a.Lk - 1)), a.dv_, g);
+    flashs_own_zero(kf[p], x < a.Lk ? a.dk_ : 0, g);
+    flashs_own_zero(vf[p], x < a.Lk ? a.dv_ : 0, g);
     // negated: with the products started from delta the matrix pipe delivers -(dP - delta)
 #pragma unroll
     for (int c = 0; c < VC; c++) {
@@ -438,7 +518,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
     DT::write(sD, dr, lane);
     sc[lane] = scr;
     if (qbk + NW < nqb) fetch(qbk + NW);
-    const bool tail = 32 * qbk + 32 > a.Lq || (CAUSAL && 32 * qbk < x0 + 16 * NP - 1);
+    const bool tail = 32 * qbk + 32 > queries.len || (CAUSAL && 32 * qbk < x0 + 16 * NP - 1);
     float pr[NP][8], ds[NP][8];
 #pragma unroll
     for (int mb = 0; mb < 2; mb++) {
@@ -461,7 +541,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
           float pv = fast_exp2(fmaf(s[i], scale, -lq[i]));
           if (tail) {
             const int qi = 32 * qbk + 16 * mb + 4 * g + i;
-            pv = (qi >= qmin && qi < a.Lq) ? pv : 0.f;
+            pv = (qi >= qmin && qi < queries.len) ? pv : 0.f;
           }
           pr[p][4 * mb + i] = pv;
           ds[p][4 * mb + i] = -pv * dp[i];
@@ -496,7 +576,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
     if (x0 + row >= a.Lk || d0 >= a.dk_) return;
 #pragma unroll
     for (int j = 0; j < 8; j++) v[j] *= a.sm_scale;
-    Io<TIO, CT>::store8(dkb + (x0 + row) * a.dks[2] + d0 * a.dks[3], v, a.dk_vec != 0, a.dks[3], dlt_imin(8, a.dk_ - d0));
+    Io<TIO, CT>::store8(dkb + flashs_at<MODE>(a.tm, a.dks, x0 + row) + d0 * a.dks[3], v, a.dk_vec != 0, a.dks[3], dlt_imin(8, a.dk_ - d0));
   });
   __syncthreads();
   FlashsSum<DV, NP, NW>::put(sums, acc_v, wave, n, g);
@@ -504,6 +584,6 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
   TIO* dvb = reinterpret_cast<TIO*>(a.dv) + b * a.dvs[0] + h * a.dvs[1];
   FlashsSum<DV, NP, NW>::reduce(sums, tid, [&](int row, int d0, float* v) {
     if (x0 + row >= a.Lk || d0 >= a.dv_) return;
-    Io<TIO, CT>::store8(dvb + (x0 + row) * a.dvs[2] + d0 * a.dvs[3], v, a.dv_vec != 0, a.dvs[3], dlt_imin(8, a.dv_ - d0));
+    Io<TIO, CT>::store8(dvb + flashs_at<MODE>(a.tm, a.dvs, x0 + row) + d0 * a.dvs[3], v, a.dv_vec != 0, a.dvs[3], dlt_imin(8, a.dv_ - d0));
   });
 }

@@ -227,6 +227,42 @@ def test_infinite_and_nan_tiles_stay_in_their_windows(d, th, tw, B, which):
                 assert torch.equal(g[:, :, far > n], w[:, :, far > n]), (r, c, value)
 
 
+# few tiles of 16 k tokens: 16 own tokens to a workgroup, the window's keys dealt over its waves; one slab, and as many as leave that rule.  Odd and even
+# numbers of 16-token runs, runs of one, windows of one tile and beyond the grid, every class and dims below it.  The image layout has the same bits.
+# A tile of infinities and NaN is not read for the tiles that do not see it
+@pytest.mark.parametrize("th,tw,S,WR,WC,dk,dv,many", [
+    (7, 5, 16, 2, 2, 64, 64, 40), (4, 10, 16, 2, 1, 64, 64, 60), (5, 9, 16, 0, 0, 64, 64, 90), (3, 7, 16, 1, 1, 128, 128, 40), (1, 9, 16, 4, 3, 64, 128, 60),
+    (9, 1, 16, 3, 2, 32, 32, 90), (3, 4, 48, 1, 1, 64, 64, 40), (2, 5, 80, 1, 0, 32, 32, 40), (4, 3, 16, 2, 2, 40, 64, 90), (3, 5, 32, 2, 1, 80, 80, 40)])
+def test_few_tiles_over_waves(th, tw, S, WR, WC, dk, dv, many):
+    sw = _swa()
+    N, scale = th * tw * S, 1 / math.sqrt(dk)
+    ops = orc.make_qkv(N + dk + th, 1, 1, N, N, dk, dv, torch.float16)
+    want = orc.tiled_swa_grads(*(t.float() for t in ops), S, th, tw, WR, WC, scale)
+    def run(q, k, v, do):
+        leaves = [t.requires_grad_(True) for t in (q, k, v)]
+        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
+        return (o.detach(),) + torch.autograd.grad(o, leaves, do)
+    one = run(*(t.cuda() for t in ops))
+    apart = run(*(t.cuda().permute(0, 2, 1, 3).repeat(1, 1, 3, 1)[:, :, 1:2].permute(0, 2, 1, 3) for t in ops))   # token rows of three heads
+    all_ = run(*(t.cuda().repeat(many, 1, 1, 1) for t in ops))
+    for got in (one, apart, all_):
+        assert (got[0][-1:].float().cpu() - want[0]).abs().max().item() <= FWD_TOL
+        errs = [_rel(g[-1:], w) for g, w in zip(got[1:], want[1:])]
+        assert max(errs) <= 1e-2, errs   # fp16
+    assert all(torch.equal(x, y) for x, y in zip(one, apart))
+    bh, lay = 4 if S == 16 else 2, lambda t: orc.tokens_to_image(t.cpu(), th, tw, bh, S // bh).contiguous().cuda()
+    leaves = [lay(t).requires_grad_(True) for t in ops[:3]]
+    o = sw.TiledSwaImage.apply(*leaves, bh, S // bh, WR, WC, scale)
+    assert all(torch.equal(x, lay(y)) for x, y in zip((o,) + torch.autograd.grad(o, leaves, lay(ops[3])), one))
+    q, k, v, do = (t.cuda() for t in ops)
+    cell = torch.arange(N, device="cuda") // S
+    far = ((cell // tw - th // 2).abs() > WR) | ((cell % tw - tw // 2).abs() > WC)
+    k[:, :, cell == th // 2 * tw + tw // 2] = float("inf")
+    v[:, :, cell == th // 2 * tw + tw // 2] = float("nan")
+    o, dq, _, _ = run(q, k, v, do)
+    assert torch.equal(o[:, :, far], one[0][:, :, far]) and torch.equal(dq[:, :, far], one[1][:, :, far])
+
+
 # tiles of 64 k tokens on the asynchronously staged kernels: workgroups of 64 own tokens (few, or rows that leave 128 a sixth empty) and of 128, tiles of
 # two and three chunks, rows of odd and even tile counts, windows beyond the grid, every class; image tiles of whole pixel rows per chunk and others
 @pytest.mark.parametrize("th,tw,tile,WR,WC,dk,dv,many", [
