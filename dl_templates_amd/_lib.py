@@ -25,7 +25,7 @@ _DTYPES = {torch.bfloat16: DLT_BF16, torch.float16: DLT_FP16, torch.float32: DLT
 
 EXPORTS = (
     "dlt_last_error", "dlt_version", "dlt_rope2d", "dlt_rope2d_copy", "dlt_rope2d_pair", "dlt_rope_pe_mask",
-    "dlt_swa_fwd", "dlt_swa_bwd", "dlt_swa_neighbors", "dlt_flash_fwd", "dlt_flash_bwd", "dlt_flash_workspace", "dlt_flash_fwd_ws", "dlt_flash_bwd_ws",
+    "dlt_swa_fwd", "dlt_swa_bwd", "dlt_swa_fwd_narrow", "dlt_swa_bwd_narrow", "dlt_swa_neighbors", "dlt_flash_fwd", "dlt_flash_bwd", "dlt_flash_workspace", "dlt_flash_fwd_ws", "dlt_flash_bwd_ws",
     "dlt_timing_enable", "dlt_timing_collect", "dlt_debug_copy",
     "dlt_swa_fwd_image", "dlt_swa_bwd_image", "dlt_swa_image_offsets", "dlt_swa_fwd_rot", "dlt_swa_bwd_rot",
     "dlt_swa_bwd_noalloc", "dlt_dry_run", "dlt_last_kernel_family",
@@ -112,6 +112,10 @@ def _declare(lib) -> None:
     lib.dlt_swa_fwd.argtypes = fwd + [POINTER(SwaShape), POINTER(RopeDesc), c_void_p]
     lib.dlt_swa_bwd.restype = c_int
     lib.dlt_swa_bwd.argtypes = bwd + [POINTER(SwaShape), POINTER(RopeDesc), c_void_p]
+    lib.dlt_swa_fwd_narrow.restype = c_int
+    lib.dlt_swa_fwd_narrow.argtypes = fwd + [POINTER(SwaShape), c_void_p]
+    lib.dlt_swa_bwd_narrow.restype = c_int
+    lib.dlt_swa_bwd_narrow.argtypes = bwd + [POINTER(SwaShape), c_void_p]
     lib.dlt_swa_bwd_noalloc.restype = c_int
     lib.dlt_swa_bwd_noalloc.argtypes = [c_void_p, P64] * 5 + [c_void_p, P64] + [c_void_p, P64] * 3 + [
         POINTER(SwaShape), POINTER(RopeDesc), c_void_p]

@@ -137,6 +137,7 @@ int swa_problem(const char* who, const dlt_swa_shape_t* s, const dlt_rope_t* rop
   }
   p.rope = dlt_make_rope_dev(rope, 0);
   p.rope_prerot = 0;
+  p.narrow = 0;
   p.tm = dlt_tokmap_none();
   return DLT_OK;
 }
@@ -154,6 +155,7 @@ int flash_problem(const char* who, const dlt_flash_shape_t* s, AttnProblem& p) {
   p.B = s->B; p.H = s->H; p.dk = s->dk; p.dv = s->dv; p.sm_scale = s->sm_scale; p.dtype = s->dtype;
   p.rope = dlt_make_rope_dev(nullptr, 0);
   p.rope_prerot = 0;
+  p.narrow = 0;
   p.tm = dlt_tokmap_none();
   return DLT_OK;
 }
@@ -256,34 +258,58 @@ extern "C" int dlt_swa_neighbors(int32_t t_height, int32_t t_width, int32_t row_
   return DLT_OK;
 }
 
-extern "C" int dlt_swa_fwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                           const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
-                           float* lse2, const int64_t lse_strides[3],
-                           const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
+namespace {
+int swa_fwd(const char* who, bool narrow, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+            const void* v, const int64_t* v_strides, void* o, const int64_t* o_strides, float* lse2, const int64_t* lse_strides,
+            const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
   AttnProblem p;
-  int rc = swa_problem("swa_fwd", shape, rope, p);
+  int rc = swa_problem(who, shape, rope, p);
   if (rc != DLT_OK) return rc;
+  p.narrow = narrow;
   AttnTensors t;
-  rc = fill_fwd("swa_fwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides);
+  rc = fill_fwd(who, t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides);
   if (rc != DLT_OK) return rc;
   return dlt_attn_forward(p, t, (hipStream_t)stream);
 }
 
-extern "C" int dlt_swa_bwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                           const void* v, const int64_t v_strides[4], const void* o, const int64_t o_strides[4],
-                           const void* d_o, const int64_t do_strides[4],
-                           const float* lse2, float* delta, const int64_t lse_strides[3],
-                           void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
-                           void* dv, const int64_t dv_strides[4],
-                           const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
+int swa_bwd(const char* who, bool narrow, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+            const void* v, const int64_t* v_strides, const void* o, const int64_t* o_strides, const void* d_o, const int64_t* do_strides,
+            const float* lse2, float* delta, const int64_t* lse_strides, void* dq, const int64_t* dq_strides, void* dk,
+            const int64_t* dk_strides, void* dv, const int64_t* dv_strides, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
   AttnProblem p;
-  int rc = swa_problem("swa_bwd", shape, rope, p);
+  int rc = swa_problem(who, shape, rope, p);
   if (rc != DLT_OK) return rc;
+  p.narrow = narrow;
   AttnTensors t;
-  rc = fill_bwd("swa_bwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta,
+  rc = fill_bwd(who, t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta,
                 lse_strides, dq, dq_strides, dk, dk_strides, dv, dv_strides);
   if (rc != DLT_OK) return rc;
   return dlt_attn_backward(p, t, (hipStream_t)stream);
+}
+}  // namespace
+
+#define DLT_SWA_FWD_ARGS                                                                                    \
+  const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4], const void *v,      \
+      const int64_t v_strides[4], void *o, const int64_t o_strides[4], float *lse2, const int64_t lse_strides[3]
+#define DLT_SWA_BWD_ARGS                                                                                    \
+  const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4], const void *v,      \
+      const int64_t v_strides[4], const void *o, const int64_t o_strides[4], const void *d_o,               \
+      const int64_t do_strides[4], const float *lse2, float *delta, const int64_t lse_strides[3], void *dq, \
+      const int64_t dq_strides[4], void *dk, const int64_t dk_strides[4], void *dv, const int64_t dv_strides[4]
+
+extern "C" int dlt_swa_fwd(DLT_SWA_FWD_ARGS, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
+  return swa_fwd("swa_fwd", false, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, rope, stream);
+}
+extern "C" int dlt_swa_fwd_narrow(DLT_SWA_FWD_ARGS, const dlt_swa_shape_t* shape, void* stream) {
+  return swa_fwd("swa_fwd_narrow", true, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, nullptr, stream);
+}
+extern "C" int dlt_swa_bwd(DLT_SWA_BWD_ARGS, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
+  return swa_bwd("swa_bwd", false, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq, dq_strides,
+                 dk, dk_strides, dv, dv_strides, shape, rope, stream);
+}
+extern "C" int dlt_swa_bwd_narrow(DLT_SWA_BWD_ARGS, const dlt_swa_shape_t* shape, void* stream) {
+  return swa_bwd("swa_bwd_narrow", true, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq,
+                 dq_strides, dk, dk_strides, dv, dv_strides, shape, nullptr, stream);
 }
 
 // ---- backward without a caller-provided scratch buffer ------------------------------------------

@@ -340,7 +340,7 @@ void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan) {
 }
 
 bool swa2_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
-  return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && ((int64_t)p.g.TR * swa2_slots(p) - 1) * st[2] * 2 + 2 * p.dk <= (((int64_t)1 << 31) - 1);
+  return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && ((int64_t)p.g.TR * swa2_slots(p) - 1) * st[2] * 2 + 2 * dlt_imax(p.dk, p.dv) <= (((int64_t)1 << 31) - 1);
 }
 bool swa2_scalars_ok(const AttnProblem& p, const AttnTensors& t) {
   return t.ls[2] >= 0 && ((int64_t)p.g.TR * swa2_slots(p) - 1) * t.ls[2] * 4 + 4 <= (((int64_t)1 << 31) - 1);
@@ -348,12 +348,12 @@ bool swa2_scalars_ok(const AttnProblem& p, const AttnTensors& t) {
 
 // Tiles of 2 ... 15 tokens (the regime of the reference's small-tile kernel, src/tiled_swa.py:15-133, b_size < 16 at
 // :611): the streaming kernels on the grid of token slots, with the window of a token given by its tile
-// (csrc/swa2_index.h).  Head dim 64 or 128 exactly, 2-byte types, no rotation, plain token layout.
+// (csrc/swa2_index.h).  Head dim 64 or 128 exactly (calls that ask for it: multiples of 8 below 64), 2-byte types, no rotation, plain token layout.
 bool swa2_tiles_eligible(const AttnProblem& p, const AttnTensors& t, bool backward) {
   if (p.g.mode != DLT_GEOM_SWA || p.g.S < 2 || p.g.S > 15 || p.tm.img) return false;
   if (p.dtype != DLT_BF16 && p.dtype != DLT_FP16) return false;
   if (!(p.sm_scale > 0.f)) return false;
-  if (!((p.dk == 64 || p.dk == 128) && p.dv == p.dk)) return false;
+  if (!((p.dk == 64 || p.dk == 128) && p.dv == p.dk) && !(p.narrow && p.dk <= 64 && p.dv <= 64 && p.dv % 8 == 0)) return false;
   if (p.rope.enabled && p.rope.R > 0) return false;
   if ((4 + 2 * swa2_extent(p) + 3) / 4 > SWA2_MAX_PASSES * 6) return false;
   if ((int64_t)p.g.TR * swa2_slots(p) >= ((int64_t)1 << 31) / 1024) return false;
@@ -380,7 +380,7 @@ int swa2_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream)
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   const int64_t grid = (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention forward: grid too large");
-  return p.dk == 64 ? dlt_swa2_launch_fwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_fwd_128(a, swa2_ncg(p), (int)grid, stream);
+  return p.dk <= 64 ? dlt_swa2_launch_fwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_fwd_128(a, swa2_ncg(p), (int)grid, stream);
 }
 
 int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream) {
@@ -398,7 +398,7 @@ int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   const int64_t grid = (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention backward: grid too large");
-  return p.dk == 64 ? dlt_swa2_launch_bwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_bwd_128(a, swa2_ncg(p), (int)grid, stream);
+  return p.dk <= 64 ? dlt_swa2_launch_bwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_bwd_128(a, swa2_ncg(p), (int)grid, stream);
 }
 
 // ---- marching token-grid kernels: head dim 32 (windows up to 21 x 21) or 64 (13 x 13) exactly, by window class ----------------------

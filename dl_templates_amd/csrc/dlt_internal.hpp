@@ -83,6 +83,7 @@ struct AttnProblem {
   int32_t dtype;
   RopeDev rope;
   int32_t rope_prerot;  // backward: q and k arrive rotated; only dq and dk are rotated (back) on store
+  int32_t narrow;       // tiles of 2 ... 15 tokens: head dims in multiples of 8 below 64 may run on the streaming kernels
   DltTokMap tm;  // token -> element offset map of q, k, v, o and the gradients (lse2 / delta stay [B, H, N])
 };
 

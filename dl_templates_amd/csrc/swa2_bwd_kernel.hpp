@@ -27,10 +27,10 @@ constexpr int swa2_occ_bwd_q(int D) { return D == 64 ? 4 : 2; }
 constexpr int swa2_occ_bwd_kv(int D) { return 2; }
 
 // =============================================================================================== dQ
-template <typename TIO, int D, int NCG>
+template <typename TIO, int D, int NCG, bool PAD>
 __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_kernel(const Swa2BwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
-  typedef Swa2Cfg<D, NCG> C;
+  typedef Swa2Cfg<D, NCG, PAD> C;
   constexpr int KC = C::KC, VB = C::VB, NKB = C::NKB;
   constexpr int NG = VB / 4;   // groups of four 16-dim blocks of dQ
   extern __shared__ __align__(16) char smem[];
@@ -54,10 +54,12 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_ke
   const bool stage_k = wave < 4;
   const char* sbase = stage_k ? kb_ : vb_;
   const int ssn2 = (int)(stage_k ? a.ks[2] : a.vs[2]) * 2;
+  const int sdims = stage_k ? a.p.dk : a.p.dv;
   const uint32_t srow = (uint32_t)(G0.TC * ssn2);
+  swa2_clear<C, SWA2_THREADS>(smem, C::LDS, tid);
   Swa2Geom G = G0;   // column pass 0 (see the forward kernel)
   Swa2Stage<C> st;
-  swa2_stage_init(st, G, wave, lane, ssn2);
+  swa2_stage_init(st, G, wave, lane, ssn2, sdims);
   swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
 
   const int r_p = G.r0 + 4 * rg, c_p = G.c0 + 4 * pc;
@@ -66,9 +68,9 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_ke
   float neg_lse, del_n;
   {
     u32x4 of[KC];
-    swa2_own_frags<KC>(qf, qb, (int)a.qs[2] * 2, tq, g);
-    swa2_own_frags<KC>(dof, dob, (int)a.dos[2] * 2, tq, g);
-    swa2_own_frags<KC>(of, ob, (int)a.os[2] * 2, tq, g);
+    swa2_own_frags<KC, PAD>(qf, qb, (int)a.qs[2] * 2, tq, g, a.p.dk);
+    swa2_own_frags<KC, PAD>(dof, dob, (int)a.dos[2] * 2, tq, g, a.p.dv);
+    swa2_own_frags<KC, PAD>(of, ob, (int)a.os[2] * 2, tq, g, a.p.dv);
     neg_lse = tq >= 0 ? -lseb[(int64_t)tq * a.ls[2]] : -INFINITY;
     // delta = rowsum(o * dO) of the own token: D / 4 head dims per lane, summed over the four lanes of the token
     float part = 0.f;
@@ -203,21 +205,21 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_ke
     G = swa2_pass_geom(G0, NCG, pass);
     W = swa2_pass_window(W0, NCG, pass);
     ncg = swa2_pass_ncg(G0.WC, NCG, pass);
-    swa2_stage_init(st, G, wave, lane, ssn2);
+    swa2_stage_init(st, G, wave, lane, ssn2, sdims);
     swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
     swa2_wait_copies();
     __syncthreads();
   }
 
-  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acc, a.p.sm_scale, dqb, a.dqs[2], G, r_p, c_p, lane);
+  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acc, a.p.sm_scale, dqb, a.dqs[2], G, r_p, c_p, lane, a.p.dk);
 }
 
 // =============================================================================================== dK / dV
 // A chunk buffer holds Q, dO and a table of per-token scalars: lse2 then delta, [4 halo rows][HCW halo columns] each.
-template <typename TIO, int D, int NCG>
+template <typename TIO, int D, int NCG, bool PAD>
 __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_kernel(const Swa2BwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
-  typedef Swa2Cfg<D, NCG> C;
+  typedef Swa2Cfg<D, NCG, PAD> C;
   constexpr int KC = C::KC, VB = C::VB, NKB = C::NKB;
   constexpr int NP2 = VB / 2;   // pairs of 16-dim blocks per gradient
   extern __shared__ __align__(16) char smem[];
@@ -241,10 +243,12 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_
   const bool stage_q = wave < 4;
   const char* sbase = stage_q ? qb : dob;
   const int ssn2 = (int)(stage_q ? a.qs[2] : a.dos[2]) * 2;
+  const int sdims = stage_q ? a.p.dk : a.p.dv;
   const uint32_t srow = (uint32_t)(G0.TC * ssn2);
+  swa2_clear<C, SWA2_THREADS>(smem, C::LDS_KV, tid);
   Swa2Geom G = G0;   // column pass 0 (see the forward kernel)
   Swa2Stage<C> st;
-  swa2_stage_init(st, G, wave, lane, ssn2);
+  swa2_stage_init(st, G, wave, lane, ssn2, sdims);
   const float* scal_base = stage_q ? lseb : delb;
   const int ls2 = (int)a.ls[2];
   // lane l < HCW copies the scalar of halo column l (clamped like the rows: positions outside the grid are masked)
@@ -262,8 +266,8 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_
   const int r_p = G.r0 + 4 * rg, c_p = G.c0 + 4 * pc;
   const int tk = (r_p + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
   u32x4 kf[KC], vf[KC];
-  swa2_own_frags<KC>(kf, kb_, (int)a.ks[2] * 2, tk, g);
-  swa2_own_frags<KC>(vf, vb_, (int)a.vs[2] * 2, tk, g);
+  swa2_own_frags<KC, PAD>(kf, kb_, (int)a.ks[2] * 2, tk, g, a.p.dk);
+  swa2_own_frags<KC, PAD>(vf, vb_, (int)a.vs[2] * 2, tk, g, a.p.dv);
   const Swa2Win W0 = swa2_window(G0, rg, pc, n);
   Swa2Win W = W0;
   Swa2Lane<C> L;
@@ -424,7 +428,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_
     G = swa2_pass_geom(G0, NCG, pass);
     W = swa2_pass_window(W0, NCG, pass);
     ncg = swa2_pass_ncg(G0.WC, NCG, pass);
-    swa2_stage_init(st, G, wave, lane, ssn2);
+    swa2_stage_init(st, G, wave, lane, ssn2, sdims);
     scal_off = (uint32_t)(swa2_scal_col(G, lane) * ls2) * 4u;
     swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF_KV, wave);
     issue_scalars(G.ch_first, smem + (G.ch_first & 1) * C::BUF_KV);
@@ -432,6 +436,6 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_
     __syncthreads();
   }
 
-  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, accv, 1.f, dvb, a.dvs[2], G, r_p, c_p, lane);
-  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acck, a.p.sm_scale, dkb, a.dks[2], G, r_p, c_p, lane);
+  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, accv, 1.f, dvb, a.dvs[2], G, r_p, c_p, lane, a.p.dv);
+  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acck, a.p.sm_scale, dkb, a.dks[2], G, r_p, c_p, lane, a.p.dk);
 }

@@ -65,13 +65,16 @@ template <typename C>
 struct Swa2Stage {
   uint32_t off[C::NI];   // byte offset of the lane's piece inside a grid row of the tensor, per instruction
   bool last_on;          // the lane takes part in the last instruction
+  bool on;               // PAD: the lane's piece exists (it has the same one in every instruction: 64 / PIECES tokens each, swizzled mod 8)
 };
 
 template <typename C>
-DLT_DEV void swa2_stage_init(Swa2Stage<C>& st, const Swa2Geom& G, int wave, int lane, int sn2) {
+DLT_DEV void swa2_stage_init(Swa2Stage<C>& st, const Swa2Geom& G, int wave, int lane, int sn2, int dims) {
 #pragma unroll
   for (int i = 0; i < C::NI; i++) st.off[i] = swa2_stage_off<C>(G, wave, lane, sn2, i);
   st.last_on = swa2_stage_last_on<C>(lane);
+  static_assert(!C::PAD || C::TPI == 8, "a lane copies the same piece of every token");
+  if constexpr (C::PAD) st.on = 8 * swa2_stage_piece<C>(wave, lane) < dims;
 }
 
 // one of the NI copy instructions of a halo row (to be spread between the products of a chunk: issued together they
@@ -79,7 +82,7 @@ DLT_DEV void swa2_stage_init(Swa2Stage<C>& st, const Swa2Geom& G, int wave, int 
 template <typename C, int I>
 DLT_DEV void swa2_issue_one(const Swa2Stage<C>& st, const char* row, char* dst) {
   if constexpr (I < C::NI) {
-    if (I + 1 < C::NI || C::HCW % C::TPI == 0 || st.last_on)
+    if ((!C::PAD || st.on) && (I + 1 < C::NI || C::HCW % C::TPI == 0 || st.last_on))
       dlt_copy16_to_lds(row, st.off[I], dst + 1024 * I);
   }
 }
@@ -95,6 +98,15 @@ DLT_DEV void swa2_issue(const Swa2Stage<C>& st, const Swa2Geom& G, int ch, const
   const char* row = swa2_issue_row(G, ch, base, rowstride, wave);
   char* dst = swa2_issue_dst<C>(buf, wave);
   swa2_for<0, C::NI>([&](auto ic) { swa2_issue_one<C, decltype(ic)::value>(st, row, dst); });
+}
+
+// PAD: no copy writes the pieces that do not exist; they are cleared before the first one
+template <typename C, int THREADS>
+DLT_DEV void swa2_clear(char* smem, int bytes, int tid) {
+  if constexpr (C::PAD) {
+    for (int i = tid; i < bytes / 16; i += THREADS) lds_write16(smem + 16 * i, u32x4{0u, 0u, 0u, 0u});
+    __syncthreads();
+  }
 }
 
 // every copy this wave issued has landed in LDS (the workgroup barrier that follows makes all of them visible)
@@ -132,18 +144,21 @@ DLT_DEV void swa2_read_tr(Swa2Lds region, const Swa2Lane<C>& L, u32x4 (&v)[ND]) 
 }
 
 // own-token fragments in B-operand layout: lane (n, g) holds head dims 32 c + 8 g .. + 7 of token n
-template <int KC>
-DLT_DEV void swa2_own_frags(u32x4 (&f)[KC], const char* base, int sn2, int tok, int g) {
+template <int KC, bool PAD = false>
+DLT_DEV void swa2_own_frags(u32x4 (&f)[KC], const char* base, int sn2, int tok, int g, int dims) {
   const char* p = base + ((uint32_t)((tok >= 0 ? tok : 0) * sn2) + 16 * g);
 #pragma unroll
-  for (int c = 0; c < KC; c++) f[c] = *reinterpret_cast<const u32x4*>(p + 64 * c);
+  for (int c = 0; c < KC; c++) {
+    if constexpr (PAD) f[c] = u32x4{0u, 0u, 0u, 0u};
+    if (!PAD || 8 * (4 * c + g) < dims) f[c] = *reinterpret_cast<const u32x4*>(p + 64 * c);
+  }
 }
 
 // ---- store epilogue: accumulators in C layout (lane (n, g): dims 16 d + 4 g .. + 3 of own token n, times `mul`) -> a
 // wave-private LDS tile [16 tokens][2 D bytes] (pieces swizzled with the token index) -> 16-byte pieces -> HBM rows
 template <typename C, typename TIO, typename CT>
 DLT_DEV void swa2_store_own(char* sW, const f32x4 (&acc)[C::VB], float mul, TIO* base, int64_t sn, const Swa2Geom& G, int r_p, int c_p,
-                            int lane) {
+                            int lane, int dims) {
   const int n = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int d = 0; d < C::VB; d++) {
@@ -162,7 +177,7 @@ DLT_DEV void swa2_store_own(char* sW, const f32x4 (&acc)[C::VB], float mul, TIO*
     const int row = lane / C::PIECES + RPI * it;
     const u32x4 v = lds_read16(sW + swa2_tile_read_off<C>(row, c));
     const int r = r_p + (row >> 2), col = c_p + (row & 3);
-    if (r < G.TR && col < G.TC) store_stream16(base + (int64_t)(r * G.TC + col) * sn + 8 * c, v);
+    if (r < G.TR && col < G.TC && (!C::PAD || 8 * c < dims)) store_stream16(base + (int64_t)(r * G.TC + col) * sn + 8 * c, v);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -19,10 +19,10 @@ struct Swa2FwdArgs {
 // waves per SIMD the register budget is sized for: at head dim 64 two workgroups share a CU
 constexpr int swa2_occ_fwd(int D) { return D == 64 ? 4 : 2; }
 
-template <typename TIO, int D, int NCG>
+template <typename TIO, int D, int NCG, bool PAD>
 __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_fwd(D)) void swa2_fwd_kernel(const Swa2FwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
-  typedef Swa2Cfg<D, NCG> C;
+  typedef Swa2Cfg<D, NCG, PAD> C;
   constexpr int KC = C::KC, VB = C::VB, NKB = C::NKB;
   constexpr int NG = VB / 4;   // groups of four 16-dim blocks of the output
   extern __shared__ __align__(16) char smem[];
@@ -44,18 +44,20 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_fwd(D)) void swa2_fwd_kernel
   const bool stage_k = wave < 4;
   const char* sbase = stage_k ? kb_ : vb_;
   const int ssn2 = (int)(stage_k ? a.ks[2] : a.vs[2]) * 2;
+  const int sdims = stage_k ? a.p.dk : a.p.dv;
   const uint32_t srow = (uint32_t)(G0.TC * ssn2);
+  swa2_clear<C, SWA2_THREADS>(smem, C::LDS, tid);
   // column pass 0 (the only one unless the window is wider than the class: swa2_pass_geom)
   Swa2Geom G = G0;
   Swa2Stage<C> st;
-  swa2_stage_init(st, G, wave, lane, ssn2);
+  swa2_stage_init(st, G, wave, lane, ssn2, sdims);
   swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
 
   // own queries straight into B-operand fragments: lane (n, g) holds head dims 32 c + 8 g .. + 7 of query n
   const int r_p = G.r0 + 4 * rg, c_p = G.c0 + 4 * pc;
   const int tq = (r_p + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
   u32x4 qf[KC];
-  swa2_own_frags<KC>(qf, qb, (int)a.qs[2] * 2, tq, g);
+  swa2_own_frags<KC, PAD>(qf, qb, (int)a.qs[2] * 2, tq, g, a.p.dk);
   const Swa2Win W0 = swa2_window(G0, rg, pc, n);
   Swa2Win W = W0;
   Swa2Lane<C> L;
@@ -190,7 +192,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_fwd(D)) void swa2_fwd_kernel
     G = swa2_pass_geom(G0, NCG, pass);
     W = swa2_pass_window(W0, NCG, pass);
     ncg = swa2_pass_ncg(G0.WC, NCG, pass);
-    swa2_stage_init(st, G, wave, lane, ssn2);
+    swa2_stage_init(st, G, wave, lane, ssn2, sdims);
     swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
     swa2_wait_copies();
     __syncthreads();
@@ -200,5 +202,5 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_fwd(D)) void swa2_fwd_kernel
   const float lt = wave_sum4(acc_l[0]);   // only row 0 of the ones operand is set: the other lane groups hold zeros
   const float inv = lt > 0.f ? fast_rcp(lt) : 0.f;
   if (g == 0 && tq >= 0) store_stream4(lseb + (int64_t)tq * ls2, m_run * scale + fast_log2(lt));
-  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acc, inv, ob, os2, G, r_p, c_p, lane);
+  swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acc, inv, ob, os2, G, r_p, c_p, lane, a.p.dv);
 }

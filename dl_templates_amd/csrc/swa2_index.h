@@ -16,9 +16,11 @@
 
 constexpr int SWA2_THREADS = 512;
 
-template <int D_, int NCG_>
+// PAD: head dims below D in multiples of 8
+template <int D_, int NCG_, bool PAD_ = false>
 struct Swa2Cfg {
   static constexpr int D = D_, NCG = NCG_;
+  static constexpr bool PAD = PAD_;
   static constexpr int NKB = NCG / 2;            // blocks of 32 streamed tokens (two column groups) per chunk
   static constexpr int KC = D / 32;              // 32-dim steps of a product that contracts over the head dim
   static constexpr int VB = D / 16;              // 16-dim blocks of an accumulator
@@ -157,6 +159,9 @@ DLT_HD uint32_t swa2_stage_off(const Swa2Geom& G, int wave, int lane, int sn2, i
   const int cc = dlt_imax(0, dlt_imin(G.c0 - G.WC + hc, G.TC - 1));   // clamped: positions outside the grid are masked
   return (uint32_t)(cc * sn2 + 16 * ((lane % C::PIECES) ^ (C::SWZ * (tok & 7))));
 }
+// that piece, where every instruction copies 8 tokens (64-dim rows)
+template <typename C>
+DLT_HD int swa2_stage_piece(int wave, int lane) { return (lane % C::PIECES) ^ (C::SWZ * (((wave & 3) * C::HCW + lane / C::PIECES) & 7)); }
 // the lane takes part in the last instruction of a halo row
 template <typename C>
 DLT_HD bool swa2_stage_last_on(int lane) { return C::TPI * (C::NI - 1) + lane / C::PIECES < C::HCW; }

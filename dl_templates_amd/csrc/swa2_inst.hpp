@@ -10,11 +10,12 @@ namespace {
 template <typename KernT>
 int swa2_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
-template <typename TIO, int NCG>
+template <typename TIO, int NCG, bool PAD>
 int swa2_launch_fwd_t(const Swa2FwdArgs& a, int grid, hipStream_t stream) {
-  typedef Swa2Cfg<DLT_SWA2_D, NCG> C;
+  typedef Swa2Cfg<DLT_SWA2_D, NCG, PAD> C;
   const bool pairs = a.plan.pairs != 0;
-  auto kern = !pairs ? swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG> : a.ks[2] == a.vs[2] ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, true> : swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, false>;
+  auto kern = !pairs ? swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG, PAD>
+                    : a.ks[2] == a.vs[2] && a.p.dk == a.p.dv ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, true, PAD> : swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, false, PAD>;
   const int lds = pairs ? C::BUF : C::LDS;
   int rc = swa2_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;
@@ -25,11 +26,11 @@ int swa2_launch_fwd_t(const Swa2FwdArgs& a, int grid, hipStream_t stream) {
   return DLT_OK;
 }
 
-template <typename TIO, int NCG>
+template <typename TIO, int NCG, bool PAD>
 int swa2_launch_bwd_t(const Swa2BwdArgs& a, int grid, hipStream_t stream) {
-  typedef Swa2Cfg<DLT_SWA2_D, NCG> C;
-  auto kq = swa2_bwd_q_kernel<TIO, DLT_SWA2_D, NCG>;
-  auto kkv = swa2_bwd_kv_kernel<TIO, DLT_SWA2_D, NCG>;
+  typedef Swa2Cfg<DLT_SWA2_D, NCG, PAD> C;
+  auto kq = swa2_bwd_q_kernel<TIO, DLT_SWA2_D, NCG, PAD>;
+  auto kkv = swa2_bwd_kv_kernel<TIO, DLT_SWA2_D, NCG, PAD>;
   int rc = swa2_set_lds(kq, C::LDS);
   if (rc != DLT_OK) return rc;
   rc = swa2_set_lds(kkv, C::LDS_KV);
@@ -49,17 +50,23 @@ int swa2_launch_bwd_t(const Swa2BwdArgs& a, int grid, hipStream_t stream) {
 // instantiation and is rejected
 template <typename TIO>
 int swa2_pick_fwd(const Swa2FwdArgs& a, int ncg, int grid, hipStream_t stream) {
+  if constexpr (DLT_SWA2_D == 64) {   // tiles of 2 ... 15 tokens at smaller head dims
+    if (a.p.dk != 64 || a.p.dv != 64) return ncg == 4 ? swa2_launch_fwd_t<TIO, 4, true>(a, grid, stream) : swa2_launch_fwd_t<TIO, 6, true>(a, grid, stream);
+  }
   switch (ncg) {
-    case 4: return swa2_launch_fwd_t<TIO, 4>(a, grid, stream);
-    case 6: return swa2_launch_fwd_t<TIO, 6>(a, grid, stream);
+    case 4: return swa2_launch_fwd_t<TIO, 4, false>(a, grid, stream);
+    case 6: return swa2_launch_fwd_t<TIO, 6, false>(a, grid, stream);
     default: return dlt_set_error(DLT_ERR_UNSUPPORTED, "streaming token-grid kernels: no instantiation for %d column groups", ncg);
   }
 }
 template <typename TIO>
 int swa2_pick_bwd(const Swa2BwdArgs& a, int ncg, int grid, hipStream_t stream) {
+  if constexpr (DLT_SWA2_D == 64) {   // tiles of 2 ... 15 tokens at smaller head dims
+    if (a.p.dk != 64 || a.p.dv != 64) return ncg == 4 ? swa2_launch_bwd_t<TIO, 4, true>(a, grid, stream) : swa2_launch_bwd_t<TIO, 6, true>(a, grid, stream);
+  }
   switch (ncg) {
-    case 4: return swa2_launch_bwd_t<TIO, 4>(a, grid, stream);
-    case 6: return swa2_launch_bwd_t<TIO, 6>(a, grid, stream);
+    case 4: return swa2_launch_bwd_t<TIO, 4, false>(a, grid, stream);
+    case 6: return swa2_launch_bwd_t<TIO, 6, false>(a, grid, stream);
     default: return dlt_set_error(DLT_ERR_UNSUPPORTED, "streaming token-grid kernels: no instantiation for %d column groups", ncg);
   }
 }

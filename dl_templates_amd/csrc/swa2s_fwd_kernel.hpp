@@ -25,10 +25,10 @@ constexpr int SWA2S_THREADS = 256;
 // waves per SIMD the register budget is sized for (head dim 64 at 6 column groups spills at 3)
 constexpr int swa2s_occ(int D, int NCG) { return D == 64 && NCG == 4 ? 3 : 2; }
 
-template <typename TIO, int D, int NCG, bool SAME>
+template <typename TIO, int D, int NCG, bool SAME, bool PAD>
 __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_kernel(const Swa2FwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
-  typedef Swa2Cfg<D, NCG> C;
+  typedef Swa2Cfg<D, NCG, PAD> C;
   constexpr int KC = C::KC, VB = C::VB, NKB = C::NKB;
   constexpr int NG = VB / 4;   // groups of four 16-dim blocks of the output
   static_assert(C::NI <= 2 * NCG && C::NI <= 2 * NKB * NG && 4 * C::TILE <= C::BUF, "copy slots of a phase; the store epilogue");
@@ -54,8 +54,9 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   const uint32_t krow = (uint32_t)(G0.TC * ksn2), vrow = (uint32_t)(G0.TC * vsn2);
   Swa2Geom G = G0;   // column pass 0
   Swa2Stage<C> st, st_own;
-  swa2_stage_init(st, G, wave, lane, ksn2);
-  if constexpr (!SAME) swa2_stage_init(st_own, G, wave, lane, vsn2);
+  swa2_clear<C, SWA2S_THREADS>(smem, C::BUF, tid);
+  swa2_stage_init(st, G, wave, lane, ksn2, a.p.dk);
+  if constexpr (!SAME) swa2_stage_init(st_own, G, wave, lane, vsn2, a.p.dv);
   const Swa2Stage<C>& stv = SAME ? st : st_own;
   swa2_issue(st, G, G.ch_first, kb_, krow, smem, wave);
 
@@ -68,7 +69,7 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   for (int p = 0; p < 2; p++) {
     r_p[p] = G.r0 + 4 * p;
     tq[p] = (r_p[p] + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p[p] + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
-    swa2_own_frags<KC>(qf[p], qb, (int)a.qs[2] * 2, tq[p], g);
+    swa2_own_frags<KC, PAD>(qf[p], qb, (int)a.qs[2] * 2, tq[p], g, a.p.dk);
     W0[p] = swa2_window(G0, p, pc, n);
     W[p] = W0[p];
   }
@@ -278,8 +279,8 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     G = swa2_pass_geom(G0, NCG, pass);
     W[0] = swa2_pass_window(W0[0], NCG, pass);
     W[1] = swa2_pass_window(W0[1], NCG, pass);
-    swa2_stage_init(st, G, wave, lane, ksn2);
-    if constexpr (!SAME) swa2_stage_init(st_own, G, wave, lane, vsn2);
+    swa2_stage_init(st, G, wave, lane, ksn2, a.p.dk);
+    if constexpr (!SAME) swa2_stage_init(st_own, G, wave, lane, vsn2, a.p.dv);
     swa2_issue(st, G, G.ch_first, kb_, krow, smem, wave);
     swa2_wait_copies();
     __syncthreads();
@@ -291,6 +292,6 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
     const float lt = wave_sum4(lsum[p]);
     const float inv = lt > 0.f ? fast_rcp(lt) : 0.f;
     if (g == 0 && tq[p] >= 0) store_stream4(lseb + (int64_t)tq[p] * ls2, m_run[p] * scale + fast_log2(lt));
-    swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acc[p], inv, ob, os2, G, r_p[p], c_p, lane);
+    swa2_store_own<C, TIO, CT>(smem + wave * C::TILE, acc[p], inv, ob, os2, G, r_p[p], c_p, lane, a.p.dv);
   }
 }

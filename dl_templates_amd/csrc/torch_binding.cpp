@@ -164,6 +164,7 @@ struct Spec {
   dlt_swa_shape_t swa{};
   dlt_swa_tile_t tile{};
   dlt_flash_shape_t flash{};
+  bool narrow = false;   // Swa: see small_tiles
 };
 
 Spec swa_spec(const Tensor& q, const Tensor& k, const Tensor& v, const int64_t* dims /* b_size, th, tw, row, col */, double scale) {
@@ -256,8 +257,12 @@ Forward run_forward(const Spec& s, const Tensor& q, const Tensor& k, const Tenso
                              (float*)f.lse.mutable_data_ptr(), st(f.lse), f.q_rot.mutable_data_ptr(), st(f.q_rot), f.k_rot.mutable_data_ptr(),
                              st(f.k_rot), &s.swa, &rope->d, stream));
   } else {
-    check_rc(dlt_swa_fwd(q.const_data_ptr(), st(q), k.const_data_ptr(), st(k), v.const_data_ptr(), st(v), f.o.mutable_data_ptr(), st(f.o),
-                         (float*)f.lse.mutable_data_ptr(), st(f.lse), &s.swa, rope ? &rope->d : nullptr, stream));
+    if (s.narrow)
+      check_rc(dlt_swa_fwd_narrow(q.const_data_ptr(), st(q), k.const_data_ptr(), st(k), v.const_data_ptr(), st(v), f.o.mutable_data_ptr(), st(f.o),
+                                  (float*)f.lse.mutable_data_ptr(), st(f.lse), &s.swa, stream));
+    else
+      check_rc(dlt_swa_fwd(q.const_data_ptr(), st(q), k.const_data_ptr(), st(k), v.const_data_ptr(), st(v), f.o.mutable_data_ptr(), st(f.o),
+                           (float*)f.lse.mutable_data_ptr(), st(f.lse), &s.swa, rope ? &rope->d : nullptr, stream));
   }
   return f;
 }
@@ -281,6 +286,7 @@ std::array<Tensor, 3> run_backward(const Spec& s, const Tensor& q, const Tensor&
   }
   else if (s.op == Op::Image) call(dlt_swa_bwd_image, &s.swa, &s.tile, none);
   else if (rotated) call(dlt_swa_bwd_rot, &s.swa, (const dlt_rope_t*)&rope->d);
+  else if (s.narrow) call(dlt_swa_bwd_narrow, &s.swa);
   else call(dlt_swa_bwd, &s.swa, rope ? (const dlt_rope_t*)&rope->d : none);
   return {dq, dk, dv};
 }
@@ -300,6 +306,18 @@ Pad swa_pad(int64_t dk, int64_t dv, at::ScalarType dt, int64_t b_size) {
   if (b_size != 1) return {dk, dv};
   auto up = [](int64_t d) { return (d + 31) / 32 * 32; };
   return big <= 64 ? Pad{up(dk), up(dv)} : Pad{std::max<int64_t>(96, up(dk)), std::max<int64_t>(96, up(dv))};
+}
+
+// Tiles of 2 ... 15 tokens at smaller head dims whose rows can be read in 16-byte pieces as they lie run there without padding (d = 32, 16 heads of 20 x 6
+// tiles of 4: the copies around the kernels were 22 of 35 us of host time in the forward pass).
+bool rows_of_pieces(const Tensor& x) {
+  return x.dim() == 4 && x.size(3) % 8 == 0 && x.stride(3) == 1 && (uintptr_t)x.const_data_ptr() % 16 == 0 && x.stride(0) % 8 == 0 && x.stride(1) % 8 == 0 &&
+         x.stride(2) % 8 == 0 && x.stride(2) >= 0 && (x.size(2) + 64) * std::max<int64_t>(x.stride(2), 64) < ((int64_t)1 << 30);
+}
+bool small_tiles(const Tensor& q, const Tensor& k, const Tensor& v, int64_t b_size, double scale) {
+  const at::ScalarType dt = q.scalar_type();
+  return 2 <= b_size && b_size <= 15 && (dt == at::kBFloat16 || dt == at::kHalf) && scale > 0 && q.size(-1) <= 64 && v.size(-1) <= 64 &&
+         rows_of_pieces(q) && rows_of_pieces(k) && rows_of_pieces(v);
 }
 
 // The flash kernels read 16-byte row pieces: head dims that are not multiples of 8 run 3 to 6 times slower on the generic ones.
@@ -338,7 +356,9 @@ struct AttnBackward : public Node {
     at::AutoDispatchBelowADInplaceOrView below;
     Rope rope;
     if (has_rope) rope = make_rope_for(idx_, row_, col_, q_, q_.size(2));
-    auto g = run_backward(spec, q_, k_, v_, o_, lse_, pad_last(grads[0], v_.size(-1)), has_rope ? &rope : nullptr, rotated);
+    Tensor d_o = pad_last(grads[0], v_.size(-1));
+    if (spec.narrow && !rows_of_pieces(d_o)) d_o = d_o.contiguous();
+    auto g = run_backward(spec, q_, k_, v_, o_, lse_, d_o, has_rope ? &rope : nullptr, rotated);
     return {cut_last(g[0], dk), cut_last(g[1], dk), cut_last(g[2], dv)};
   }
 };
@@ -375,13 +395,15 @@ Tensor attention(Op op, const Tensor& q, const Tensor& k, const Tensor& v, const
   const int64_t dk = q.size(-1), dv = v.size(-1);
   {
     at::AutoDispatchBelowADInplaceOrView below;
-    const Pad pad = op == Op::Flash ? flash_pad(dk, dv, q.scalar_type()) : op == Op::Swa ? swa_pad(dk, dv, q.scalar_type(), dims[0]) : Pad{dk, dv};
+    const bool narrow = op == Op::Swa && rope_t == nullptr && small_tiles(q, k, v, dims[0], scale);
+    const Pad pad = narrow ? Pad{dk, dv} : op == Op::Flash ? flash_pad(dk, dv, q.scalar_type()) : op == Op::Swa ? swa_pad(dk, dv, q.scalar_type(), dims[0]) : Pad{dk, dv};
     if (C10_UNLIKELY(pad.dk != dk || pad.dv != dv)) {
       pq = pad_last(q, pad.dk);
       pk = pad_last(k, pad.dk);
       pv = pad_last(v, pad.dv);
     }
     spec = op == Op::Flash ? flash_spec(pq, pk, pv, causal, scale) : op == Op::Image ? image_spec(pq, pk, pv, dims, scale) : swa_spec(pq, pk, pv, dims, scale);
+    spec.narrow = narrow;
     Rope rope;
     if (rope_t != nullptr) {
       check_assert(rope_t[1].dim() == 3 && rope_t[2].dim() == 3 && rope_t[1].size(1) == rope_t[2].size(1), "row and column table must have one R");

@@ -120,6 +120,19 @@ int dlt_swa_bwd(const void* q, const int64_t q_strides[4], const void* k, const 
                 void* dv, const int64_t dv_strides[4],
                 const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream);
 
+/* The same calls, without rotation, that also take tiles of 2 ... 15 tokens at head dims in multiples of 8 below 64 (2-byte
+ * types, 16-byte aligned rows) to the streaming kernels, where dlt_swa_fwd / dlt_swa_bwd keep them on the generic ones, two to
+ * four times slower: the tile copies skip the dims that are not there.  Every other call is routed as there. */
+int dlt_swa_fwd_narrow(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                       const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
+                       float* lse2, const int64_t lse_strides[3], const dlt_swa_shape_t* shape, void* stream);
+int dlt_swa_bwd_narrow(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
+                       const void* v, const int64_t v_strides[4], const void* o, const int64_t o_strides[4],
+                       const void* d_o, const int64_t do_strides[4],
+                       const float* lse2, float* delta, const int64_t lse_strides[3],
+                       void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
+                       void* dv, const int64_t dv_strides[4], const dlt_swa_shape_t* shape, void* stream);
+
 /* dlt_swa_bwd without the `delta` argument: the fp32 scratch lives in a buffer inside the library
  * (one static device array per GPU, DLT_NOALLOC_MAX_DELTA floats = 4 MiB, held until the process
  * ends) and the call allocates nothing: no hipMalloc / hipFree, no allocating library routine.

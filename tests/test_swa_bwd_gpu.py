@@ -352,3 +352,37 @@ def test_marching_large_windows(B, H, th, tw, WR, WC):
     assert (o.float().cpu() - want[0]).abs().max().item() <= 2e-2
     errs = (_rel(qg.grad, want[1]), _rel(kg.grad, want[2]), _rel(vg.grad, want[3]))
     assert max(errs) <= GRAD_TOL, errs
+
+
+# tiles of 2 ... 15 tokens at head dims below 64: the bits of tensors padded by hand, one workgroup per CU and (many slabs, forward) two patches per wave,
+# both window classes and column passes; tensors cut out of wider ones whose other columns are NaN, K and V at other strides, a gradient that
+# cannot be read in 16-byte pieces; rows that cannot either are padded as before
+@pytest.mark.parametrize("H,S,th,tw,WR,WC,dk,dv,dtype", [
+    (2, 4, 9, 7, 1, 1, 32, 32, torch.bfloat16), (130, 4, 9, 7, 1, 2, 32, 32, torch.float16), (2, 2, 5, 33, 3, 2, 8, 8, torch.float16), (3, 9, 4, 5, 2, 1, 40, 40, torch.bfloat16),
+    (110, 15, 3, 4, 1, 0, 56, 24, torch.bfloat16), (2, 8, 3, 9, 0, 2, 16, 64, torch.float16), (140, 4, 8, 5, 2, 4, 24, 48, torch.float16)])
+def test_small_tiles_of_few_head_dims(H, S, th, tw, WR, WC, dk, dv, dtype):
+    from dl_templates_amd import _lib, tiled_swa as sw
+    N, scale = th * tw * S, 0.2
+    q, k, v, do = (t.cuda() for t in orc.make_qkv(N + dk, 1, H, N, N, dk, dv, dtype))
+
+    def run(*ts, d_o=do):
+        leaves = [t.detach().requires_grad_(True) for t in ts]
+        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
+        assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
+        return [o.detach()] + list(torch.autograd.grad(o, leaves, d_o))
+
+    def wide(t, w):   # the same rows inside rows of w, NaN behind them
+        return torch.cat([t, torch.full((*t.shape[:3], w - t.shape[3]), float("nan"), dtype=dtype, device="cuda")], -1)[..., :t.shape[3]]
+
+    pad = lambda t: torch.nn.functional.pad(t, (0, 64 - t.shape[-1]))
+    got, want = run(q, k, v), run(pad(q), pad(k), pad(v), d_o=pad(do))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b[..., :a.shape[-1]])
+    for a, b in zip(got, run(wide(q, 72), wide(k, 128), wide(v, 80), d_o=do.transpose(2, 3).contiguous().transpose(2, 3))):
+        assert torch.equal(a, b)
+    for a, b in zip(got, run(wide(q, 65), wide(k, 67), wide(v, 66 if dv < 64 else 72))):   # rows off the 16-byte grid
+        assert torch.equal(a, b)
+    ref = orc.tiled_swa_grads(*(t[:, -1:].float().cpu() for t in (q, k, v, do)), S, th, tw, WR, WC, scale)
+    assert (got[0][:, -1:].float().cpu() - ref[0]).abs().max().item() <= 2e-2
+    for a, b in zip(got[1:], ref[1:]):
+        assert ((a[:, -1:].float().cpu() - b).abs().max() / b.abs().max()).item() <= 5e-2
