@@ -557,7 +557,7 @@ bool flash_eligible(const AttnProblem& p, const AttnTensors& t, bool with_do) {
 // ---- marching tile-window kernels: tiles of 16 or 32 tokens, head dim 32 or 64 exactly ------------------------------
 // What they take beyond flash_eligible: windows whose rows fit the LDS ring (3 x 3 tiles; with 16-token tiles also 5 tile
 // columns, and 5 tile rows at head dim 32), and 16-byte rows with 32-bit offsets for every tensor.  Larger tiles stay on the
-// chunked kernels: a window row of 64-token tiles gives a 64-token chunk work for every wave, and its rows do not fit the ring.
+// flash kernels: a window row of 64-token tiles gives a 64-token chunk work for every wave, and its rows do not fit the ring.
 bool swat_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
   return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && st[4] >= 0 && slab_span(p, st, (int64_t)p.g.TR * p.g.XLq) * 2 <= ((int64_t)1 << 31) - 1;
 }

@@ -303,7 +303,8 @@ int dlt_debug_copy(void* dst, const void* src, int64_t bytes, void* stream);
  *             the backward pass rotated q / k kept), also the forward pass of fp32 tensors at head dim 32; tiles of 16 or 32
  *             tokens at those head dims report FLASH
  *   STREAMING token grids, head dim 64 / 128, windows up to 93 columns (beyond 21 columns in column passes), no rotation;
- *             tiles of 2 ... 15 tokens at head dim 64 / 128 (the grid of token slots, up to 24 column groups of 4 slots)
+ *             tiles of 2 ... 15 tokens at head dim 64 / 128 (the grid of token slots, up to 24 column groups of 4 slots), through
+ *             dlt_swa_*_narrow also at multiples of 8 below 64
  *   TILE      token grids, head dims in multiples of 32 up to 128, windows up to 21 columns (rotation in the tile loads)
  *   FLASH     dense / causal / tiles of 16 k tokens, 2-byte element types, head dims up to 128 (multiples of 8)
  *   GENERIC   everything else */
