@@ -618,9 +618,10 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
 //     fixed + rounds over the CUs * (start and final sum of a workgroup + its 32-token blocks * time of a block on a CU).
 // The constants of the split kernels (us) are least-squares fits to launches of 32 ... 8192 tokens on either side and 4 ... 128 heads, dense
 // and causal.  Those of the chunked kernels were fitted the same way to two blocks per wave; in the backward passes they were then scaled, by
-// class, to what decides best now that few workgroups run one block per wave (dlt_flash_bwd_64; 7900 shapes of up to 4000 tokens).  Gained by
-// it, on the whole backward pass: by dQ at 128/128 1.077 under a mask and 1.027 without, at 64/128 1.028 and 1.019, at 64/64 1.028 and
-// 1.019, by dK/dV 1.00 ... 1.02 (32 slabs of 300 x 300, 64/64, both 20.8 -> 15.4 us).  In the forward pass the same scaling gained 1 % in the mean
+// class, to what decides best now that few workgroups run one block per wave (dlt_flash_bwd_64; 7900 shapes of up to 4000 tokens); of the
+// scales of start and chunk within 0.3 % of the best, those with the fewest passes over 5 % slower than before (some 140 against 329 with one scale
+// for both).  Gained by it, on the whole backward pass: by dQ at 128/128 1.046, at 64/128 1.022, at 64/64 1.020, by dK/dV 1.00 ... 1.02 (32 slabs of
+// 300 x 300, 64/64, both 20.8 -> 15.4 us).  In the forward pass the same scaling gained 1 % in the mean
 // and lost up to 40 % with few slabs (8 of 480 x 2581, 64/64, 16 -> 27 us): left.
 //   77 queries x 1500 keys, 16 heads, 64/64: forward 22 -> 10 us, dQ 24 -> 11; 482 keys x 5450 queries, 4 heads: dK/dV 86 -> 26
 //   16 heads, 2048 x 2048: forward 64/128 46 -> 34 us, 128/128 55 -> 41 (SLIM)
@@ -643,18 +644,18 @@ int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, i
        {256, 6.78f, 1.493f, 2.40f, 1.125f, .59f, 3.70f, .272f, 0.f, 5.81f, .322f},     // 128/128
        {256, 6.06f, 1.272f, 2.40f, .960f, 1.53f, 2.57f, .174f, 0.f, 5.73f, .185f},     // 64/128
        {128, 2.94f, .698f, NONE, NONE, 2.84f, .52f, .055f, 2.41f, 1.13f, .094f}},      // 32/32
-      {{128, 3.15f, .553f, NONE, NONE, 2.07f, 2.19f, .138f, .43f, 5.72f, .144f},
-       {128, 3.29f, .702f, NONE, NONE, .67f, 4.25f, .289f, NONE, NONE, NONE},
-       {128, 2.99f, .590f, NONE, NONE, .99f, 4.27f, .244f, NONE, NONE, NONE},
+      {{128, 3.48f, .748f, NONE, NONE, 2.07f, 2.19f, .138f, .43f, 5.72f, .144f},
+       {128, 2.63f, 1.236f, NONE, NONE, .67f, 4.25f, .289f, NONE, NONE, NONE},
+       {128, 3.04f, .773f, NONE, NONE, .99f, 4.27f, .244f, NONE, NONE, NONE},
        {128, 4.44f, .825f, NONE, NONE, 2.73f, .68f, .057f, 2.36f, 1.44f, .090f}},
-      {{128, 4.05f, .888f, NONE, NONE, 1.85f, 2.73f, .134f, 1.36f, 4.59f, .171f},
-       {64, 4.78f, 1.042f, NONE, NONE, 1.31f, 4.42f, .283f, NONE, NONE, NONE},
-       {128, 5.38f, 1.513f, NONE, NONE, 1.32f, 4.15f, .185f, NONE, NONE, NONE},
+      {{128, 4.35f, .953f, NONE, NONE, 1.85f, 2.73f, .134f, 1.36f, 4.59f, .171f},
+       {64, 4.95f, 1.275f, NONE, NONE, 1.31f, 4.42f, .283f, NONE, NONE, NONE},
+       {128, 5.79f, 1.627f, NONE, NONE, 1.32f, 4.15f, .185f, NONE, NONE, NONE},
        {128, 4.28f, 1.038f, NONE, NONE, 2.51f, 1.14f, .072f, 2.79f, 1.38f, .114f}}};
   FlashCost c = COST[pass][dc.id];
   if (pass > 0 && dc.id == 1 && dims <= 192) {   // the split kernels leave out missing pieces of a row, of the chunked ones' work more stays (flashd_dims)
-    const float more = pass == 1 ? 1.6f : 1.3f;
-    c.start *= more; c.chunk *= more;
+    c.start = pass == 1 ? 7.58f : 5.26f;
+    c.chunk = pass == 1 ? 1.26f : 1.40f;
   }
   const float cus = (float)dlt_device_cus();
   const auto wgs = [&](int n) { return (float)(bh * ((own + n - 1) / n)); };
