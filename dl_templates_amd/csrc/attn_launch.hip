@@ -326,7 +326,10 @@ bool swa2_compose_ok(const AttnProblem& p, const Swa1Class& c) {
 }
 
 void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan) {
-  constexpr int band = 8;
+  // Bands of four rows (the waves of the lower four only copy; the same bits) while those too have a CU each: a band's time is its halo's copies and
+  // chunks, 4 + 2 WR rows instead of 8 + 2 WR.  Over 3508 shapes of up to 128 workgroups forward 0.81 ... 0.87 of the time, backward 0.76 ... 0.82
+  // (d = 128, 4 slabs of 47 x 25, 15 x 5 window, forward 10.3 -> 8.5 us); from 129 on, where workgroups of 4 rows would queue, 0.9 ... 1.1 and 1.1 ... 1.3.
+  const int band = 2 * (int64_t)p.B * p.H * ((p.g.TR + 7) / 8) * ((swa2_slots(p) + 15) / 16) <= dlt_device_cus() ? 4 : 8;
   plan.pairs = 0;
   { int c; swa2_split(p, c, plan.npass); }
   plan.S = p.g.S; plan.WCt = p.g.WC;

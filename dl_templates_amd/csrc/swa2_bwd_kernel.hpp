@@ -63,7 +63,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_ke
   swa2_issue(st, G, G.ch_first, sbase, srow, smem + (G.ch_first & 1) * C::BUF, wave);
 
   const int r_p = G.r0 + 4 * rg, c_p = G.c0 + 4 * pc;
-  const int tq = (r_p + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
+  const int tq = (r_p + (n >> 2) < G.r_end && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
   u32x4 qf[KC], dof[KC];
   float neg_lse, del_n;
   {
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_
   issue_scalars(G.ch_first, smem + (G.ch_first & 1) * C::BUF_KV);
 
   const int r_p = G.r0 + 4 * rg, c_p = G.c0 + 4 * pc;
-  const int tk = (r_p + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
+  const int tk = (r_p + (n >> 2) < G.r_end && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
   u32x4 kf[KC], vf[KC];
   swa2_own_frags<KC, PAD>(kf, kb_, (int)a.ks[2] * 2, tk, g, a.p.dk);
   swa2_own_frags<KC, PAD>(vf, vb_, (int)a.vs[2] * 2, tk, g, a.p.dv);

@@ -1,7 +1,7 @@
 // Streaming token-grid kernels (b_size == 1, head dim 64 or 128, windows up to 21 columns, any number of rows):
 // shared geometry, asynchronous staging and swizzled operand reads.
 //
-// A workgroup of 8 waves owns a band of 8 grid rows x 16 grid columns; wave w owns the 4x4 patch at rows
+// A workgroup of 8 waves owns a band of 8 grid rows x 16 grid columns (small grids: 4 rows, Swa2Plan::band); wave w owns the 4x4 patch at rows
 // 4 (w >> 2), columns 4 (w & 3).  The tokens of the other side that any own token can see (8 + 2 WR halo rows x HCW
 // halo columns) stream through LDS in chunks of 4 halo rows.  A chunk is copied HBM -> LDS by the DMA path of the
 // vector memory unit (16 bytes per lane, no staging registers: at head dim 128 those were a third of the register
@@ -177,7 +177,7 @@ DLT_DEV void swa2_store_own(char* sW, const f32x4 (&acc)[C::VB], float mul, TIO*
     const int row = lane / C::PIECES + RPI * it;
     const u32x4 v = lds_read16(sW + swa2_tile_read_off<C>(row, c));
     const int r = r_p + (row >> 2), col = c_p + (row & 3);
-    if (r < G.TR && col < G.TC && (!C::PAD || 8 * c < dims)) store_stream16(base + (int64_t)(r * G.TC + col) * sn + 8 * c, v);
+    if (r < G.r_end && col < G.TC && (!C::PAD || 8 * c < dims)) store_stream16(base + (int64_t)(r * G.TC + col) * sn + 8 * c, v);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

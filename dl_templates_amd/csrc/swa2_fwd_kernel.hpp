@@ -55,7 +55,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_fwd(D)) void swa2_fwd_kernel
 
   // own queries straight into B-operand fragments: lane (n, g) holds head dims 32 c + 8 g .. + 7 of query n
   const int r_p = G.r0 + 4 * rg, c_p = G.c0 + 4 * pc;
-  const int tq = (r_p + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
+  const int tq = (r_p + (n >> 2) < G.r_end && c_p + (n & 3) < G.TC) ? (r_p + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
   u32x4 qf[KC];
   swa2_own_frags<KC, PAD>(qf, qb, (int)a.qs[2] * 2, tq, g, a.p.dk);
   const Swa2Win W0 = swa2_window(G0, rg, pc, n);

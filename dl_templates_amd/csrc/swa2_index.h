@@ -55,13 +55,14 @@ struct Swa2Plan {
   int32_t npass;   // column passes: a window of more than NCG column groups is walked in npass slices of NCG groups
   int32_t S, WCt;  // tokens per tile, window half-width in tiles
   uint32_t m_S, s_S;   // division by S
-  int32_t band;    // grid rows of a workgroup's band: 8
+  int32_t band;    // grid rows of a workgroup's band: 8, or 4 (the lower four waves only copy)
   int32_t pairs;   // forward pass: 4 waves of two stacked patches instead of 8 waves of one
 };
 
 struct Swa2Geom {
   int TR, TC, WR, WC;   // grid rows, token slots per row, window half-height in rows, largest column extent in slots
   int r0, c0;   // first grid row / column of the band
+  int r_end;    // one past its last grid row
   int b, h;
   int ch_first, ch_last;   // chunks of the band's halo that hold grid rows
   int S, WCt;
@@ -86,6 +87,7 @@ DLT_HD Swa2Geom swa2_geom_at(int TR, int TC, int WR, int WC, int H, const Swa2Pl
   G.h = bh - G.b * H;
   G.TR = TR; G.TC = TC; G.WR = WR; G.WC = WC;
   G.r0 = P.band * br;
+  G.r_end = dlt_imin(TR, G.r0 + P.band);
   G.c0 = 16 * (rem - br * P.nblk_c);
   const int lo = dlt_imax(0, G.WR - G.r0), hi = dlt_imin(P.band - 1 + 2 * G.WR, G.TR - 1 - G.r0 + G.WR);
   G.ch_first = lo >> 2;
@@ -104,7 +106,7 @@ DLT_HD Swa2Win swa2_window(const Swa2Geom& G, int rg, int pc, int n) {
   Swa2Win w;
   const int qr = 4 * rg + (n >> 2), qc = n & 3;
   const int c_p = G.c0 + 4 * pc;
-  const bool ok = (G.r0 + qr < G.TR) && (c_p + qc < G.TC);
+  const bool ok = (G.r0 + qr < G.r_end) && (c_p + qc < G.TC);
   w.rlo = dlt_imax(qr, G.WR - G.r0);
   w.rhi = dlt_imin(qr + 2 * G.WR, G.TR - 1 - G.r0 + G.WR);
   // window columns: the wave window starts at slot c_p - WC, the own token sits at window column WC + qc
@@ -116,7 +118,7 @@ DLT_HD Swa2Win swa2_window(const Swa2Geom& G, int rg, int pc, int n) {
   w.cspan = ok ? chi - w.clo : -1;
   // halo rows of the patch that hold grid rows
   const int plo = dlt_imax(4 * rg, G.WR - G.r0), phi = dlt_imin(4 * rg + 3 + 2 * G.WR, G.TR - 1 - G.r0 + G.WR);
-  const bool patch_ok = (G.r0 + 4 * rg < G.TR) && (c_p < G.TC) && plo <= phi;
+  const bool patch_ok = (G.r0 + 4 * rg < G.r_end) && (c_p < G.TC) && plo <= phi;
   w.ch_lo = patch_ok ? plo >> 2 : 1;
   w.ch_hi = patch_ok ? phi >> 2 : 0;
   return w;

@@ -386,3 +386,29 @@ def test_small_tiles_of_few_head_dims(H, S, th, tw, WR, WC, dk, dv, dtype):
     assert (got[0][:, -1:].float().cpu() - ref[0]).abs().max().item() <= 2e-2
     for a, b in zip(got[1:], ref[1:]):
         assert ((a[:, -1:].float().cpu() - b).abs().max() / b.abs().max()).item() <= 5e-2
+
+
+# bands of four rows and of eight (up to and beyond 128 workgroups of eight rows on 256 CUs): a slab's bits are the same; grids below a band, of whole
+# bands and a row more, both window classes, a window in column passes, tiles of 4 tokens at 64 and 32 dims
+@pytest.mark.parametrize("few,many,S,th,tw,WR,WC,d", [
+    (2, 200, 1, 3, 12, 2, 3, 128), (8, 64, 1, 4, 33, 1, 2, 128), (4, 22, 1, 41, 31, 7, 8, 64), (64, 65, 1, 12, 16, 10, 10, 128), (3, 30, 1, 13, 60, 3, 12, 128),
+    (5, 40, 4, 17, 5, 1, 2, 64), (5, 40, 4, 21, 5, 2, 1, 32)])
+def test_bands_of_four_rows(few, many, S, th, tw, WR, WC, d):
+    from dl_templates_amd import _lib, tiled_swa as sw
+    N, scale = th * tw * S, 0.15
+    ts = [t.cuda() for t in orc.make_qkv(N + d, 1, many, N, N, d, d, torch.bfloat16)]
+
+    def run(n):
+        q, k, v, do = (t[:, -n:].contiguous() for t in ts)
+        leaves = [t.requires_grad_(True) for t in (q, k, v)]
+        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
+        assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
+        return [o.detach()] + list(torch.autograd.grad(o, leaves, do))
+
+    got, all_ = run(few), run(many)
+    if many * -(-th // 8) * -(-tw * S // 16) <= 256:   # beyond, the forward pass takes two patches per wave (other reference maxima)
+        assert all(torch.equal(a, b[:, -few:]) for a, b in zip(got, all_))
+    ref = orc.tiled_swa_grads(*(t[:, -1:].float().cpu() for t in ts), S, th, tw, WR, WC, scale)
+    for run_ in (got, all_):
+        assert (run_[0][:, -1:].float().cpu() - ref[0]).abs().max().item() <= FWD_TOL
+        assert max(_rel(a[:, -1:], b) for a, b in zip(run_[1:], ref[1:])) <= GRAD_TOL
