@@ -325,11 +325,35 @@ bool swa2_compose_ok(const AttnProblem& p, const Swa1Class& c) {
   return (c.D == 64 || c.D == 128) && p.dk == c.D && p.dv == c.D && (p.g.WC > 3 || (int64_t)p.B * p.H * p.g.TR * p.g.TC >= 131072);
 }
 
-void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan) {
+// Time of a launch in rounds of one chunk, the last columns on 2^lpc patch columns (2: workgroups of 8 rows as everywhere): a workgroup takes its chunks
+// and three more for its start and end, a CU one at a time in the backward pass and two in the forward pass; behind the mean load of the CUs, the longest one stands
+// alone for part of its time (fitted to the shapes below).
+float swa2_estimate(const AttnProblem& p, int lpc, bool backward) {
+  const int64_t bh = (int64_t)p.B * p.H, blocks = (swa2_slots(p) + 15) / 16, full = bh * (lpc == 2 ? blocks : blocks - 1) * ((p.g.TR + 7) / 8);
+  auto len = [&](int band) { return (float)((dlt_imin(p.g.TR, band + 2 * p.g.WR) + 3) / 4 + 3); };
+  const int band = 32 >> lpc;
+  const int64_t tall = lpc == 2 ? 0 : bh * ((p.g.TR + band - 1) / band), n = full + tall, cap = (backward ? 1 : 2) * (int64_t)dlt_device_cus();
+  const float longest = tall ? len(band) : len(8), mean = ((float)full * len(8) + (float)tall * len(band)) / (float)cap;
+  return n > cap ? mean + 0.35f * longest : fmaxf(mean, longest) + (backward ? 0.f : 0.14f * longest);
+}
+// log2 of the patch columns for the last `rest` slots of a row: 1, 0 (up to 4 slots), or 2, plain workgroups, unless the estimate falls by 7 % (less is lost as often as won)
+int swa2_pick_tall(const AttnProblem& p, int rest, bool backward) {
+  float best = 0.93f * swa2_estimate(p, 2, backward);
+  int pick = 2;
+  for (int lpc = rest <= 4 ? 0 : 1; lpc < 2; lpc++) {
+    const float e = swa2_estimate(p, lpc, backward);
+    if (e < best) { best = e; pick = lpc; }
+  }
+  return pick;
+}
+
+// returns the workgroups of 8 rows x 16 columns that the grids of all slabs take
+int64_t swa2_make_plan(const AttnProblem& p, bool backward, Swa2Plan& plan) {
   // Bands of four rows (the waves of the lower four only copy; the same bits) while those too have a CU each: a band's time is its halo's copies and
   // chunks, 4 + 2 WR rows instead of 8 + 2 WR.  Over 3508 shapes of up to 128 workgroups forward 0.81 ... 0.87 of the time, backward 0.76 ... 0.82
   // (d = 128, 4 slabs of 47 x 25, 15 x 5 window, forward 10.3 -> 8.5 us); from 129 on, where workgroups of 4 rows would queue, 0.9 ... 1.1 and 1.1 ... 1.3.
-  const int band = 2 * (int64_t)p.B * p.H * ((p.g.TR + 7) / 8) * ((swa2_slots(p) + 15) / 16) <= dlt_device_cus() ? 4 : 8;
+  const int64_t bands = (int64_t)p.B * p.H * ((p.g.TR + 7) / 8) * ((swa2_slots(p) + 15) / 16);
+  const int band = 2 * bands <= dlt_device_cus() ? 4 : 8;
   plan.pairs = 0;
   { int c; swa2_split(p, c, plan.npass); }
   plan.S = p.g.S; plan.WCt = p.g.WC;
@@ -337,9 +361,20 @@ void swa2_make_plan(const AttnProblem& p, Swa2Plan& plan) {
   plan.band = band;
   plan.nblk_r = (p.g.TR + band - 1) / band;
   plan.nblk_c = (swa2_slots(p) + 15) / 16;
-  dlt_fastdiv_make((uint32_t)(plan.nblk_r * plan.nblk_c), plan.m_bh, plan.s_bh);
-  dlt_fastdiv_make((uint32_t)plan.nblk_c, plan.m_c, plan.s_c);
+  plan.ntall = 0; plan.lpc = 2;
+  const int rest = swa2_slots(p) & 15;
+  if (rest >= 1 && rest <= 8 && bands > dlt_device_cus() && (backward || p.dk == 128)) {
+    // The last columns fill half a workgroup or less: 2 or 1 patch columns and bands of 16 or 32 rows (the same bits), where the estimate says that
+    // it pays.  90 shapes of 257 ... 2300 bands, backward 0.945 of the time in the mean of all, 0.61 ... 1.016, taken for 34 of them (d = 128, 16
+    // slabs of 71 x 17, 17 x 7 window 0.64; 64 of 99 x 18, 15 x 9 184 -> 139 us); forward at d = 128, taken for 10, 0.98 in the mean, 56 -> 49 there; at
+    // d = 64, where more workgroups share a CU, under 0.01.  Up to one band per CU the longer workgroups take 1.1 to 1.6 times as long.
+    const int pick = swa2_pick_tall(p, rest, backward);
+    if (pick < 2) swa2_plan_tall(plan, p.g.TR, swa2_slots(p), pick);
+  }
+  dlt_fastdiv_make((uint32_t)swa2_groups(plan), plan.m_bh, plan.s_bh);
+  dlt_fastdiv_make((uint32_t)dlt_imax(1, plan.nblk_c), plan.m_c, plan.s_c);
   dlt_fastdiv_make((uint32_t)p.H, plan.m_h, plan.s_h);
+  return bands;
 }
 
 bool swa2_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
@@ -375,13 +410,13 @@ int swa2_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream)
   // 11.2 / 12.2, 352 26.8 / 25.8).
   // DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the one-patch kernel for A/B timing and for its tests.
   static const bool single_patch = [] { const char* e = getenv("DLT_SWA2_SINGLE_PATCH"); return e != nullptr && e[0] == '1'; }();
-  swa2_make_plan(p, a.plan);
-  a.plan.pairs = !single_patch && (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c > dlt_device_cus();
+  const int64_t bands = swa2_make_plan(p, false, a.plan);
+  a.plan.pairs = !single_patch && bands > dlt_device_cus();
   a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.out_o; a.lse = t.lse;
   for (int i = 0; i < 4; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; }
   for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
-  const int64_t grid = (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c;
+  const int64_t grid = (int64_t)p.B * p.H * swa2_groups(a.plan);
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention forward: grid too large");
   return p.dk <= 64 ? dlt_swa2_launch_fwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_fwd_128(a, swa2_ncg(p), (int)grid, stream);
 }
@@ -390,7 +425,7 @@ int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream
   if (dlt_route_note(DLT_FAMILY_STREAMING)) return DLT_OK;
   Swa2BwdArgs a;
   a.p = p;
-  swa2_make_plan(p, a.plan);
+  swa2_make_plan(p, true, a.plan);
   a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.o; a.d_o = t.d_o; a.lse = t.lse; a.delta = t.delta;
   a.dq = t.dq; a.dk = t.dk; a.dv = t.dv;
   for (int i = 0; i < 4; i++) {
@@ -399,7 +434,7 @@ int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream
   }
   for (int i = 0; i < 3; i++) a.ls[i] = t.ls[i];
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
-  const int64_t grid = (int64_t)p.B * p.H * a.plan.nblk_r * a.plan.nblk_c;
+  const int64_t grid = (int64_t)p.B * p.H * swa2_groups(a.plan);
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention backward: grid too large");
   return p.dk <= 64 ? dlt_swa2_launch_bwd_64(a, swa2_ncg(p), (int)grid, stream) : dlt_swa2_launch_bwd_128(a, swa2_ncg(p), (int)grid, stream);
 }

@@ -1,8 +1,9 @@
 // Streaming token-grid kernels (b_size == 1, head dim 64 or 128, windows up to 21 columns, any number of rows):
 // shared geometry, asynchronous staging and swizzled operand reads.
 //
-// A workgroup of 8 waves owns a band of 8 grid rows x 16 grid columns (small grids: 4 rows, Swa2Plan::band); wave w owns the 4x4 patch at rows
-// 4 (w >> 2), columns 4 (w & 3).  The tokens of the other side that any own token can see (8 + 2 WR halo rows x HCW
+// A workgroup of 8 waves owns a band of 8 grid rows x 16 grid columns (small grids: 4 rows, Swa2Plan::band); wave w owns the 4x4 patch at
+// rows 4 (w >> 2), columns 4 (w & 3).  Last columns of up to 8 slots, where half of the waves or more would only copy, are 16 or 32 rows x 8 or 4
+// columns to a workgroup where that is faster (Swa2Plan::ntall).  The tokens of the other side that any own token can see (8 + 2 WR halo rows x HCW
 // halo columns) stream through LDS in chunks of 4 halo rows.  A chunk is copied HBM -> LDS by the DMA path of the
 // vector memory unit (16 bytes per lane, no staging registers: at head dim 128 those were a third of the register
 // file) into one of two buffers while the other one is consumed, so a chunk costs one workgroup barrier, every

@@ -57,12 +57,16 @@ struct Swa2Plan {
   uint32_t m_S, s_S;   // division by S
   int32_t band;    // grid rows of a workgroup's band: 8, or 4 (the lower four waves only copy)
   int32_t pairs;   // forward pass: 4 waves of two stacked patches instead of 8 waves of one
+  int32_t ntall;   // workgroups of a slab on its last columns where those fill half a workgroup or less (nblk_c then counts the blocks before): their
+                   // waves stand on 2 or 1 patch columns (lpc: log2) and 4 or 8 patch rows, a band of 16 or 32 rows; 0: none
+  int32_t lpc;
 };
 
 struct Swa2Geom {
   int TR, TC, WR, WC;   // grid rows, token slots per row, window half-height in rows, largest column extent in slots
   int r0, c0;   // first grid row / column of the band
   int r_end;    // one past its last grid row
+  int lpc;      // log2 of the patch columns its waves stand on: wave w on patch column w & (2^lpc - 1), patch row w >> lpc
   int b, h;
   int ch_first, ch_last;   // chunks of the band's halo that hold grid rows
   int S, WCt;
@@ -75,21 +79,34 @@ DLT_HD void swa2_plan_tokens(Swa2Plan& P, int WC) {
   dlt_fastdiv_make(1u, P.m_S, P.s_S);
 }
 
+// Tall workgroups of a slab (Swa2Plan::ntall): the last columns fill half a workgroup or less, and a band of 8 rows is not all there is.
+DLT_HD void swa2_plan_tall(Swa2Plan& P, int TR, int slots, int lpc) {
+  P.lpc = lpc;
+  P.nblk_c = slots >> 4;
+  P.ntall = (TR + (32 >> P.lpc) - 1) / (32 >> P.lpc);
+}
+
+// workgroups of a slab
+DLT_HD int swa2_groups(const Swa2Plan& P) { return P.nblk_r * P.nblk_c + P.ntall; }
+
 // geometry of workgroup `lin` (its index after the XCD remap); TC: token slots per grid row, WC: S WCt + S - 1
 DLT_HD Swa2Geom swa2_geom_at(int TR, int TC, int WR, int WC, int H, const Swa2Plan& P, int lin) {
   Swa2Geom G;
   G.S = P.S; G.WCt = P.WCt; G.m_S = P.m_S; G.s_S = P.s_S;
-  const int per_bh = P.nblk_r * P.nblk_c;
+  const int per_bh = swa2_groups(P);
   const int bh = (int)dlt_fastdiv((uint32_t)lin, P.m_bh, P.s_bh);
-  const int rem = lin - bh * per_bh;
-  const int br = (int)dlt_fastdiv((uint32_t)rem, P.m_c, P.s_c);
+  const int rem = lin - bh * per_bh - P.ntall;   // the tall workgroups, which take longer, come first
+  const bool tall = rem < 0;
+  const int full = dlt_imax(0, rem), br = tall ? rem + P.ntall : (int)dlt_fastdiv((uint32_t)full, P.m_c, P.s_c);
+  G.lpc = tall ? P.lpc : 2;
+  const int band = tall ? 32 >> P.lpc : P.band;
   G.b = (int)dlt_fastdiv((uint32_t)bh, P.m_h, P.s_h);
   G.h = bh - G.b * H;
   G.TR = TR; G.TC = TC; G.WR = WR; G.WC = WC;
-  G.r0 = P.band * br;
-  G.r_end = dlt_imin(TR, G.r0 + P.band);
-  G.c0 = 16 * (rem - br * P.nblk_c);
-  const int lo = dlt_imax(0, G.WR - G.r0), hi = dlt_imin(P.band - 1 + 2 * G.WR, G.TR - 1 - G.r0 + G.WR);
+  G.r0 = band * br;
+  G.r_end = dlt_imin(TR, G.r0 + band);
+  G.c0 = 16 * (tall ? P.nblk_c : full - br * P.nblk_c);
+  const int lo = dlt_imax(0, G.WR - G.r0), hi = dlt_imin(band - 1 + 2 * G.WR, G.TR - 1 - G.r0 + G.WR);
   G.ch_first = lo >> 2;
   G.ch_last = hi >> 2;
   return G;

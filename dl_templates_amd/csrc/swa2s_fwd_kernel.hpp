@@ -36,8 +36,8 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   const int tid = threadIdx.x;
   const int lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pc = wave;
   const Swa2Geom G0 = swa2_geom(a.p, a.plan);
+  const int pc = wave & ((1 << G0.lpc) - 1), rg = 2 * (wave >> G0.lpc);
 
   const char* qb = reinterpret_cast<const char*>(a.q) + 2 * (G0.b * a.qs[0] + G0.h * a.qs[1]);
   const char* kb_ = reinterpret_cast<const char*>(a.k) + 2 * (G0.b * a.ks[0] + G0.h * a.ks[1]);
@@ -67,10 +67,10 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   Swa2Win W0[2], W[2];
 #pragma unroll
   for (int p = 0; p < 2; p++) {
-    r_p[p] = G.r0 + 4 * p;
+    r_p[p] = G.r0 + 4 * (rg + p);
     tq[p] = (r_p[p] + (n >> 2) < G.TR && c_p + (n & 3) < G.TC) ? (r_p[p] + (n >> 2)) * G.TC + c_p + (n & 3) : -1;
     swa2_own_frags<KC, PAD>(qf[p], qb, (int)a.qs[2] * 2, tq[p], g, a.p.dk);
-    W0[p] = swa2_window(G0, p, pc, n);
+    W0[p] = swa2_window(G0, rg + p, pc, n);
     W[p] = W0[p];
   }
   Swa2Lane<C> L;

@@ -25,7 +25,7 @@ int fail(const char* fmt, int a = 0, int b = 0, int c = 0, int d = 0, int e = 0,
 struct Slot { int tensor, r, c, piece; };   // tensor -1: never written
 
 template <typename C>
-int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band, int sn2, int ls2, long long slab_bytes, long long scal_elems, int lds_bytes, int lds_kv_bytes) {
+int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band_arg, int sn2, int ls2, long long slab_bytes, long long scal_elems, int lds_bytes, int lds_kv_bytes) {
   if (lds_bytes != C::LDS) return fail("launcher asks for %d bytes of LDS, the class needs %d", lds_bytes, C::LDS);
   if (lds_kv_bytes != C::LDS_KV) return fail("launcher asks for %d bytes of LDS (dK/dV), the class needs %d", lds_kv_bytes, C::LDS_KV);
   // token slots per grid row and the largest column extent of a window in slots (tiles of S tokens)
@@ -33,20 +33,25 @@ int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band, int sn2,
   const int ncg_total = (4 + 2 * WC + 3) >> 2;
   if (ncg_total > C::NCG * npass) return fail("window of %d column groups on a class with %d in %d column passes", ncg_total, C::NCG, npass);
   Swa2Plan P;
-  if (band != 8 && band != 16) return fail("bands of %d rows", band);
-  P.band = band;   // 16: two stacked patches per wave (row groups 0 .. 3)
-  P.nblk_r = (TR + band - 1) / band;
+  // 0, 1: bands of 8 rows, and tall workgroups on 1 or 2 patch columns for the last columns, where those fill half a workgroup or less
+  const bool tall = band_arg == 0 || band_arg == 1;
+  if (!tall && band_arg != 4 && band_arg != 8 && band_arg != 16) return fail("bands of %d rows", band_arg);
+  P.band = tall ? 8 : band_arg;   // 16: two stacked patches per wave (row groups 0 .. 3)
+  P.nblk_r = (TR + P.band - 1) / P.band;
   P.nblk_c = (TC + 15) / 16;
+  P.ntall = 0; P.lpc = 2;
+  if (tall) swa2_plan_tall(P, TR, TC, band_arg);
   const int H = 1;
   P.npass = npass; P.S = S; P.WCt = WCt;
   dlt_fastdiv_make((uint32_t)S, P.m_S, P.s_S);
-  dlt_fastdiv_make((uint32_t)(P.nblk_r * P.nblk_c), P.m_bh, P.s_bh);
-  dlt_fastdiv_make((uint32_t)P.nblk_c, P.m_c, P.s_c);
+  dlt_fastdiv_make((uint32_t)swa2_groups(P), P.m_bh, P.s_bh);
+  dlt_fastdiv_make((uint32_t)dlt_imax(1, P.nblk_c), P.m_c, P.s_c);
   dlt_fastdiv_make((uint32_t)H, P.m_h, P.s_h);
   DltGeom dg;
   dg.mode = DLT_GEOM_SWA; dg.TR = TR; dg.XLq = dg.XLk = TC; dg.S = S; dg.TC = TCt; dg.WR = WR; dg.WC = WCt;
   std::vector<Slot> lds(C::LDS_KV / 4);
-  const int nwg = P.nblk_r * P.nblk_c;
+  std::vector<int> owners(TR * TC, 0);
+  const int nwg = swa2_groups(P);
   for (int lin = 0; lin < nwg; lin++) {
     const Swa2Geom G0 = swa2_geom_at(TR, TC, WR, WC, H, P, lin);
     const Swa2Geom& G = G0;
@@ -54,12 +59,15 @@ int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band, int sn2,
     if (G.r0 >= TR || G.c0 >= TC) return fail("workgroup %d starts outside the grid (%d, %d)", lin, G.r0, G.c0);
     if (G.ch_first > G.ch_last) return fail("workgroup %d: empty chunk range", lin);
     // ---- windows against the shared geometry routine
-    for (int patch = 0; patch < band / 4 * 4; patch++) {
-      const int pc = patch & 3, rg = patch >> 2;
+    const int band = G.lpc == 2 ? P.band : 32 >> G.lpc, cols = 1 << G.lpc;
+    for (int patch = 0; patch < dlt_imax(8, band / 4 * cols); patch++) {
+      const int pc = patch & (cols - 1), rg = patch >> G.lpc;
       for (int n = 0; n < 16; n++) {
         const Swa2Win W0 = swa2_window(G, rg, pc, n);
         const int r = G.r0 + 4 * rg + (n >> 2), c = G.c0 + 4 * pc + (n & 3);
-        const bool own = r < TR && c < TC;
+        const bool own = r < G.r_end && c < TC;
+        if (own) owners[r * TC + c]++;
+        if (!own && W0.cspan >= 0) return fail("position (%d, %d) outside the workgroup sees keys", r, c);
         int rlo = 0, rhi = -1, xlo = 0, xhi = 0;
         if (own) dlt_key_range(dg, r, c, rlo, rhi, xlo, xhi);
         int hits = 0;
@@ -136,7 +144,7 @@ int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band, int sn2,
         }
         // reads
         for (int wave = 0; wave < 8; wave++) {
-          const int pc = wave & 3;
+          const int pc = wave & ((1 << G.lpc) - 1);
           for (int lane = 0; lane < 64; lane++) {
             const int n = lane & 15, g = lane >> 4;
             Swa2Lane<C> L;
@@ -219,6 +227,8 @@ int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band, int sn2,
       }
     }
   }
+  for (int i = 0; i < TR * TC; i++)
+    if (owners[i] != 1) return fail("token (%d, %d) has %d owners", i / TC, i % TC, owners[i]);
   // ---- store epilogue: wave-private tiles
   {
     std::vector<int> tile(C::TILE / 4, -1);

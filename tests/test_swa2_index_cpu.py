@@ -41,7 +41,7 @@ def _classes(WC):
 
 
 def _run(shim, D, NCG, npass, TR, TC, WR, WC, pad=0, ls2=1, S=1, band=8):
-    """TC, WC in tiles of S tokens; band: grid rows per workgroup (16: two stacked patches per wave)."""
+    """TC, WC in tiles of S tokens; band: grid rows per workgroup (16: two stacked patches per wave; 0, 1: 8, tall workgroups on the last columns)."""
     sn2 = 2 * D + pad
     slab = (TR * TC * S - 1) * sn2 + 2 * D
     scal = (TR * TC * S - 1) * ls2 + 1
@@ -62,6 +62,19 @@ def test_every_class_on_small_and_ragged_grids(shim, TR, TC):
             _run(shim, D, NCG, npass, TR, TC, WR, WC)
             if D == 128:   # the forward kernel with two stacked patches per wave: bands of 16 rows
                 _run(shim, D, NCG, npass, TR, TC, WR, WC, band=16)
+
+
+@pytest.mark.parametrize("TR", [1, 9, 17, 33, 70])
+def test_tall_workgroups_on_the_last_columns(shim, TR):
+    """Last columns that fill 1 ... 8 slots of a workgroup, alone and behind whole blocks: bands of 32 and 16 rows (band 0 and 1)."""
+    for TC in (1, 4, 5, 8, 20, 21):
+        for WR, WC in [(0, 0), (7, 3), (10, 10), (3, 14)]:
+            for D, NCG, npass in _classes(WC):
+                if NCG <= 6:
+                    for band in (0, 1) if TC % 16 <= 4 else (1,):
+                        _run(shim, D, NCG, npass, TR, TC, WR, WC, band=band)
+    for S, TC, WR, WC in [(3, 7, 1, 1), (4, 5, 2, 1), (5, 1, 3, 1)]:
+        _run(shim, 64, 6, 2, TR, TC, WR, WC, S=S, band=0 if S * TC % 16 <= 4 else 1)
 
 
 def test_more_passes_than_needed_change_nothing(shim):

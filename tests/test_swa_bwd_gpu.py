@@ -412,3 +412,22 @@ def test_bands_of_four_rows(few, many, S, th, tw, WR, WC, d):
     for run_ in (got, all_):
         assert (run_[0][:, -1:].float().cpu() - ref[0]).abs().max().item() <= FWD_TOL
         assert max(_rel(a[:, -1:], b) for a, b in zip(run_[1:], ref[1:])) <= GRAD_TOL
+
+
+# last columns of up to 8 slots on workgroups of 32 or 16 rows, first and last slab: one and two patch columns, ragged in both directions and filled,
+# alone and behind whole blocks, a window in column passes, tiles of 4 and 3 tokens at 64 and 32 dims
+@pytest.mark.parametrize("H,S,th,tw,WR,WC,d", [
+    (64, 1, 99, 18, 7, 4, 128), (32, 1, 71, 24, 8, 3, 128), (128, 1, 77, 7, 3, 9, 128), (64, 1, 85, 20, 4, 12, 128), (64, 1, 64, 21, 6, 10, 64),
+    (128, 4, 66, 5, 1, 1, 64), (128, 3, 70, 2, 2, 1, 32)])
+def test_last_columns_on_tall_workgroups(H, S, th, tw, WR, WC, d):
+    from dl_templates_amd import _lib, tiled_swa as sw
+    N, scale = th * tw * S, 0.15
+    q, k, v, do = (t.cuda() for t in orc.make_qkv(N + d, 1, H, N, N, d, d, torch.bfloat16))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
+    assert _lib.KERNEL_FAMILIES[_lib.load().dlt_last_kernel_family()] == "streaming"
+    got = [o.detach()] + list(torch.autograd.grad(o, leaves, do))
+    for h in (0, H - 1):
+        ref = orc.tiled_swa_grads(*(t.detach()[:, h:h + 1].float().cpu() for t in (q, k, v, do)), S, th, tw, WR, WC, scale)
+        assert (got[0][:, h:h + 1].float().cpu() - ref[0]).abs().max().item() <= FWD_TOL
+        assert max(_rel(a[:, h:h + 1], b) for a, b in zip(got[1:], ref[1:])) <= GRAD_TOL
