@@ -604,7 +604,14 @@ bool swat_eligible(const AttnProblem& p, const AttnTensors& t, bool bwd) {
   if (p.dk != p.dv || (p.dk != 32 && p.dk != 64)) return false;
   if (p.g.WR < 1 || p.g.WC < 1 || p.g.WR > 2 || p.g.WC > 2) return false;
   if (p.g.S == 32 && (p.g.WR != 1 || p.g.WC != 1)) return false;
-  if (p.g.WR == 2 && p.dk != 32) return false;
+  // d = 64, five rows of three columns: strips of four tiles (a ring of eight does not fit the LDS).  Against the register-staged flash kernels, 60 shapes from 80
+  // strips and rows on, forward 0.36 ... 0.9 of the time, backward 0.5 ... 1.0 (three shapes of 5 and 6 columns, whose last strip is nearly empty,
+  // 1.04 ... 1.15, no longer with their forward pass): 2 slabs of 30 x 30 tiles 25.3 -> 9.6 and 52.4 -> 29.5 us, 64 of 21 x 33 206 -> 133 and 537 -> 440.  Up to 56 the
+  // window's keys over a workgroup's waves (flash_tiles_split) are faster: 2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2.
+  if (p.g.WR == 2 && p.dk == 64) {
+    if (p.g.WC != 1 || p.g.TC < 4) return false;
+    if (4 * (int64_t)p.B * p.H * ((p.g.TC + Swat<64, 1, 1, 2>::SB - 1) / Swat<64, 1, 1, 2>::SB) * p.g.TR < dlt_device_cus()) return false;
+  }
   if (!swat_rows_ok(p, t.q, t.qs) || !swat_rows_ok(p, t.k, t.ks) || !swat_rows_ok(p, t.v, t.vs)) return false;
   if (!bwd) return swat_rows_ok(p, t.out_o, t.os);
   return swat_rows_ok(p, t.o, t.os) && swat_rows_ok(p, t.d_o, t.dos) && swat_rows_ok(p, t.dq, t.dqs) && swat_rows_ok(p, t.dk, t.dks) &&
@@ -632,12 +639,12 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
     a.ring_p[i] = ring_p[i];
     for (int j = 0; j < 5; j++) a.ring_s[i][j] = ring_s[i][j];
   }
-  const int strip = 16 * (!a.one ? 8 : p.dk == 32 ? Swab<32, 1, 1, 1>::SB : Swab<64, 1, 1, 1>::SB);
+  const int sb = a.one ? (p.dk == 32 ? Swab<32, 1, 1, 1>::SB : Swab<64, 1, 1, 1>::SB) : p.dk == 64 && p.g.WR == 2 ? Swat<64, 1, 1, 2>::SB : 8, strip = 16 * sb;
   a.nstrips = (p.g.XLq + strip - 1) / strip;
   const int64_t cols = slabs * a.nstrips;
   a.lone = !bwd && p.tm.img && dlt_image_fwd_alone(p.dk, p.g.S, p.g.WR, p.g.WC, p.g.TR, p.g.TC, p.H, cols, cus);
   // Rows per workgroup: a band's prologue fills the ring (the latency of its loads) and re-reads 2 WR rows.
-  const int halo = 8 + 2 * p.g.WC * (p.g.S / 16), ring = (2 * p.g.WR + 1) * halo * 64 * p.dk;
+  const int halo = sb + 2 * p.g.WC * (p.g.S / 16), ring = (2 * p.g.WR + 1) * halo * 64 * p.dk;
   const bool two = !a.one && !a.lone && ring + (2 * p.g.WR + 1) * halo * 128 <= 80 * 1024;   // workgroups per CU
   dlt_band_plan(p.g.TR, cols, two ? 2 * cus : cus, a.band, a.nbands);
   const int64_t grid = cols * a.nbands;

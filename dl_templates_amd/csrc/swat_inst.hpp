@@ -13,7 +13,7 @@ int swat_launch_fwd(const SwatArgs& a, int grid, hipStream_t stream) {
   const int rc = dlt_ensure_lds(reinterpret_cast<const void*>(kern), lds);
   if (rc != DLT_OK) return rc;
   dlt_timing_before(DLT_K_FWD, stream);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(SWAT_THREADS), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(C::THREADS), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("marching tile-window forward launch");
   return DLT_OK;
@@ -43,11 +43,11 @@ int swat_launch_bwd_two(const SwatArgs& a, int grid, hipStream_t stream) {
   if (rc == DLT_OK) rc = dlt_ensure_lds(reinterpret_cast<const void*>(kkv), C::RING + C::SCAL);
   if (rc != DLT_OK) return rc;
   dlt_timing_before(DLT_K_BWD_Q, stream);
-  hipLaunchKernelGGL(kq, dim3(grid), dim3(SWAT_THREADS), C::RING, stream, a);
+  hipLaunchKernelGGL(kq, dim3(grid), dim3(C::THREADS), C::RING, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("marching tile-window dQ launch");
   dlt_timing_before(DLT_K_BWD_KV, stream);
-  hipLaunchKernelGGL(kkv, dim3(grid), dim3(SWAT_THREADS), C::RING + C::SCAL, stream, a);
+  hipLaunchKernelGGL(kkv, dim3(grid), dim3(C::THREADS), C::RING + C::SCAL, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("marching tile-window dK/dV launch");
   return DLT_OK;
@@ -69,8 +69,8 @@ int swat_pick(const SwatArgs& a, bool bwd, int grid, hipStream_t stream) {
     if (a.g.WC == 1) DLT_SWAT(1, 1, 1);
     DLT_SWAT(1, 2, 1);
   }
-#if DLT_D == 32
   if (a.g.WC == 1) DLT_SWAT(1, 1, 2);
+#if DLT_D == 32
   DLT_SWAT(1, 2, 2);
 #endif
   return dlt_set_error(DLT_ERR_UNSUPPORTED, "marching tile-window kernels: no instantiation for this window");

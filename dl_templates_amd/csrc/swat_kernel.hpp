@@ -4,7 +4,7 @@
 // What bounded the chunked kernels here: a query tile sees only 9 ... 25 tiles, so a workgroup of 128 queries walked nine
 // 64-token chunks, each a load, two barriers and work for one or two of its four waves (image layout, B = 4, H = 8,
 // 256 x 256 pixels, 4 x 4-pixel tiles, d = 32: forward 301 us for 537 MB, latency of 9 rounds, 1.8 TB/s).
-// Here a workgroup owns a strip of 8 blocks of 16 tokens (one per wave) and marches down the grid rows.  The rows its
+// Here a workgroup owns a strip of 8 blocks of 16 tokens (one per wave; 4 at head dim 64 with five window rows) and marches down the grid rows.  The rows its
 // window covers (2 WR + 1 grid rows of both streamed tensors) live in an LDS ring; a step needs one new row, which travels
 // HBM -> registers while the step computes, so every row is fetched once per strip and the loads of a step have a whole
 // step to arrive.  All tiles of the window are resident: the softmax is one-shot, there is no mask inside a tile (a block of
@@ -38,13 +38,15 @@ template <int D, int NTB, int WC, int WR>
 struct Swat {
   static constexpr int NWB = (2 * WC + 1) * NTB, NR = 2 * WR + 1;   // 16-token blocks per window row, window rows
   static constexpr int NB = NR * NWB, NP = (NB + 1) / 2;            // blocks of a window, pairs of them (32 tokens of a product)
-  static constexpr int HB = 8 + 2 * WC * NTB, TOK = 16 * HB;        // staged blocks / tokens per grid row
+  // strips of four blocks where a ring of eight exceeds the LDS; one wave per SIMD then, with all of its registers
+  static constexpr int SB = D == 64 && WR == 2 ? 4 : 8, THREADS = 64 * SB;   // 16-token blocks of a strip, one per wave
+  static constexpr int HB = SB + 2 * WC * NTB, TOK = 16 * HB;       // staged blocks / tokens per grid row
   static constexpr int ROWB = 2 * D, BLKB = 16 * ROWB, TB = TOK * ROWB, SLOT = 2 * TB;
-  static constexpr int PIECES = D / 8, NV = 2 * TOK * PIECES, NIT = (NV + 511) / 512;
+  static constexpr int PIECES = D / 8, NV = 2 * TOK * PIECES, NIT = (NV + THREADS - 1) / THREADS;
   static constexpr int KC = D / 32, DB = D / 16;
   static constexpr int RING = NR * SLOT, SCAL = NR * 2 * TOK * 4;
-  // two workgroups per CU where two rings fit
-  static constexpr int OCC = RING + SCAL <= 80 * 1024 ? 4 : 2;
+  // waves per SIMD: two workgroups per CU where two rings fit
+  static constexpr int OCC = (RING + SCAL <= 80 * 1024 ? 2 : 1) * SB / 4;
   // Forward rows leave in 64-byte runs (swat_store_row) where registers allow: at d = 32 five columns and 32-token tiles are held to 128 (with
   // five rows, to arithmetic) and take 1 and 3.5 % less without.  With them: d = 64, 3 x 3, 64 slabs of 40 x 40 tiles 180 -> 174 us, five
   // columns 214 -> 209, d = 32, five rows 138 -> 131.
@@ -52,7 +54,6 @@ struct Swat {
   static_assert((TOK * PIECES) % 64 == 0, "a wave stages one tensor per vector");
   static_assert(RING + SCAL <= 160 * 1024, "the ring exceeds the LDS");
 };
-constexpr int SWAT_THREADS = 512;
 
 template <int D> DLT_DEV int swat_swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : t & 7; }
 
@@ -80,7 +81,7 @@ template <typename T> DLT_DEV const char* swat_slab(const void* p, const int64_t
 // Who a workgroup is: heads innermost (image rows hold all heads of a pixel side by side: the workgroups that share its
 // 128-byte lines run at the same time on one XCD), then strips, bands and batches.
 struct SwatWho { int b, h, r0, r1, xs; };
-DLT_DEV SwatWho swat_who(const SwatArgs& a, int width = 128) {
+DLT_DEV SwatWho swat_who(const SwatArgs& a, int width) {
   int lin = xcd_remap(blockIdx.x, gridDim.x);
   SwatWho w;
   if (a.tm.img) {
@@ -118,11 +119,11 @@ struct SwatRing {
     const int XL = a.g.XLq;
     rs0 = swat_row_bytes(a.tm, s0, XL);
     rs1 = swat_row_bytes(a.tm, s1, XL);
-    const int xh = xs - (C::HB - 8) * 8;   // first staged slot: half of the extra blocks lie to the left
+    const int xh = xs - (C::HB - C::SB) * 8;   // first staged slot: half of the extra blocks lie to the left
 #pragma unroll
     for (int it = 0; it < C::NIT; it++) {
-      const int id = tid + SWAT_THREADS * it;
-      second[it] = 64 * wave + SWAT_THREADS * it >= C::NV / 2;
+      const int id = tid + C::THREADS * it;
+      second[it] = 64 * wave + C::THREADS * it >= C::NV / 2;
       const int v = second[it] ? id - C::NV / 2 : id;
       const int tok = v / C::PIECES, piece = v % C::PIECES;
       // slots outside the grid row are clamped onto it: they belong to tiles that nobody sees
@@ -137,13 +138,13 @@ struct SwatRing {
     const uint32_t o0 = rc * rs0, o1 = rc * rs1;
 #pragma unroll
     for (int it = 0; it < C::NIT; it++)
-      if (C::NV % SWAT_THREADS == 0 || it + 1 < C::NIT || tid + SWAT_THREADS * it < C::NV)
+      if (C::NV % C::THREADS == 0 || it + 1 < C::NIT || tid + C::THREADS * it < C::NV)
         r[it] = *reinterpret_cast<const u32x4*>((second[it] ? base1 : base0) + (goff[it] + (second[it] ? o1 : o0)));
   }
   DLT_DEV void commit(int slot) {
 #pragma unroll
     for (int it = 0; it < C::NIT; it++)
-      if (C::NV % SWAT_THREADS == 0 || it + 1 < C::NIT || tid + SWAT_THREADS * it < C::NV) swat_write16(lds + slot * C::SLOT + loff[it], r[it]);
+      if (C::NV % C::THREADS == 0 || it + 1 < C::NIT || tid + C::THREADS * it < C::NV) swat_write16(lds + slot * C::SLOT + loff[it], r[it]);
   }
   // window rows of the first step: all requested before the first is written
   DLT_DEV void fill(int first) {
@@ -219,14 +220,14 @@ struct SwatSeen {
 };
 
 template <typename TIO, int D, int NTB, int WC, int WR>
-__global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swat_fwd_kernel(const SwatArgs a) {
+__global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, WR>::OCC)) void swat_fwd_kernel(const SwatArgs a) {
   typedef Swat<D, NTB, WC, WR> C;
   typedef typename ComputeOf<TIO>::type CT;
   extern __shared__ __align__(16) char smem[];
   swat_lds lds = (swat_lds)smem;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const SwatWho w = swat_who(a);
+  const SwatWho w = swat_who(a, 16 * C::SB);
   const int XL = a.g.XLq;
 
   SwatRing<TIO, C> ring;
@@ -344,14 +345,14 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
 
 // dQ: own = queries, K and V in the ring; delta = rowsum(o dO) of the own queries is formed and stored on the way.
 template <typename TIO, int D, int NTB, int WC, int WR>
-__global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swat_bwd_q_kernel(const SwatArgs a) {
+__global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, WR>::OCC)) void swat_bwd_q_kernel(const SwatArgs a) {
   typedef Swat<D, NTB, WC, WR> C;
   typedef typename ComputeOf<TIO>::type CT;
   extern __shared__ __align__(16) char smem[];
   swat_lds lds = (swat_lds)smem;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const SwatWho w = swat_who(a);
+  const SwatWho w = swat_who(a, 16 * C::SB);
   const int XL = a.g.XLq;
 
   SwatRing<TIO, C> ring;
@@ -473,14 +474,14 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
 
 // dK / dV: own = keys, Q and dO in the ring with -lse2 and delta of their tokens behind it (the window is symmetric).
 template <typename TIO, int D, int NTB, int WC, int WR>
-__global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swat_bwd_kv_kernel(const SwatArgs a) {
+__global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, WR>::OCC)) void swat_bwd_kv_kernel(const SwatArgs a) {
   typedef Swat<D, NTB, WC, WR> C;
   typedef typename ComputeOf<TIO>::type CT;
   extern __shared__ __align__(16) char smem[];
   swat_lds lds = (swat_lds)smem;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const SwatWho w = swat_who(a);
+  const SwatWho w = swat_who(a, 16 * C::SB);
   const int XL = a.g.XLq;
 
   SwatRing<TIO, C> ring;
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(SWAT_THREADS, (Swat<D, NTB, WC, WR>::OCC)) void swa
   const float* lseb = a.lse + w.b * a.ls[0] + w.h * a.ls[1];
   const float* delb = a.delta + w.b * a.ls[0] + w.h * a.ls[1];
   DLT_LDS float* scal = reinterpret_cast<DLT_LDS float*>(lds + C::RING);   // [slot][-lse2 | delta][token]
-  const int xsc = dlt_imax(0, dlt_imin(w.xs - (C::HB - 8) * 8 + tid, XL - 1));
+  const int xsc = dlt_imax(0, dlt_imin(w.xs - (C::HB - C::SB) * 8 + tid, XL - 1));
   float r_lse = 0.f, r_del = 0.f;
   auto issue_scal = [&](int row) {
     const int rc = dlt_imax(0, dlt_imin(row, a.g.TR - 1));
