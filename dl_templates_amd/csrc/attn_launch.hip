@@ -68,6 +68,7 @@ int dlt_swag_launch_64_3(const SwagArgs&, int dtype, int ncg, bool bwd, int grid
 int dlt_swag_launch_64_4(const SwagArgs&, int dtype, int ncg, bool bwd, int grid, hipStream_t);
 int dlt_swat_launch_32(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_swat_launch_64(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
+int dlt_swat_launch_128(const SwatArgs&, int dtype, bool bwd, int grid, hipStream_t);
 int dlt_launch_delta_32_32(const BwdArgs&, hipStream_t);
 int dlt_launch_delta_64_64(const BwdArgs&, hipStream_t);
 int dlt_launch_delta_128_128(const BwdArgs&, hipStream_t);
@@ -592,25 +593,30 @@ bool flash_eligible(const AttnProblem& p, const AttnTensors& t, bool with_do) {
   return true;
 }
 
-// ---- marching tile-window kernels: tiles of 16 or 32 tokens, head dim 32 or 64 exactly ------------------------------
+// ---- marching tile-window kernels: tiles of 16 or 32 tokens, head dim 32 or 64 exactly, forward also 128 -----------------
 // What they take beyond flash_eligible: windows whose rows fit the LDS ring (3 x 3 tiles; with 16-token tiles also 5 tile
-// columns, and 5 tile rows at head dim 32), and 16-byte rows with 32-bit offsets for every tensor.  Larger tiles stay on the
+// columns, 5 tile rows at head dim 32, and 5 x 3 tiles at 64), and 16-byte rows with 32-bit offsets for every tensor.  Larger tiles stay on the
 // flash kernels: a window row of 64-token tiles gives a 64-token chunk work for every wave, and its rows do not fit the ring.
 bool swat_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
   return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && st[4] >= 0 && slab_span(p, st, (int64_t)p.g.TR * p.g.XLq) * 2 <= ((int64_t)1 << 31) - 1;
 }
 bool swat_eligible(const AttnProblem& p, const AttnTensors& t, bool bwd) {
   if (p.g.mode != DLT_GEOM_SWA || (p.g.S != 16 && p.g.S != 32)) return false;
-  if (p.dk != p.dv || (p.dk != 32 && p.dk != 64)) return false;
+  if (p.dk != p.dv || (p.dk != 32 && p.dk != 64 && (p.dk != 128 || bwd))) return false;
   if (p.g.WR < 1 || p.g.WC < 1 || p.g.WR > 2 || p.g.WC > 2) return false;
   if (p.g.S == 32 && (p.g.WR != 1 || p.g.WC != 1)) return false;
-  // d = 64, five rows of three columns: strips of four tiles (a ring of eight does not fit the LDS).  Against the register-staged flash kernels, 60 shapes from 80
-  // strips and rows on, forward 0.36 ... 0.9 of the time, backward 0.5 ... 1.0 (three shapes of 5 and 6 columns, whose last strip is nearly empty,
-  // 1.04 ... 1.15, no longer with their forward pass): 2 slabs of 30 x 30 tiles 25.3 -> 9.6 and 52.4 -> 29.5 us, 64 of 21 x 33 206 -> 133 and 537 -> 440.  Up to 56 the
-  // window's keys over a workgroup's waves (flash_tiles_split) are faster: 2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2.
-  if (p.g.WR == 2 && p.dk == 64) {
-    if (p.g.WC != 1 || p.g.TC < 4) return false;
-    if (4 * (int64_t)p.B * p.H * ((p.g.TC + Swat<64, 1, 1, 2>::SB - 1) / Swat<64, 1, 1, 2>::SB) * p.g.TR < dlt_device_cus()) return false;
+  // Strips of four tiles, of which a ring of eight does not fit the LDS, against the flash kernels:
+  // d = 64, five rows of three columns, 60 shapes from 80 strips and rows on: forward 0.36 ... 0.9 of the time, backward 0.5 ... 1.0 (three shapes of 5 and 6
+  // columns, whose last strip is nearly empty, 1.04 ... 1.15, no longer with their forward pass): 2 slabs of 30 x 30 tiles 25.3 -> 9.6 and
+  // 52.4 -> 29.5 us, 64 of 21 x 33 206 -> 133 and 537 -> 440.  Up to 56 the window's keys over a workgroup's waves (flash_tiles_split) are
+  // faster: 2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2.
+  // d = 128, 3 x 3 tiles, forward: 0.40 ... 0.98 where strips are three quarters full (2 slabs of 30 x 30 23.8 -> 13.4, 64 of 30 x 10 174 -> 106), five columns
+  // up to 1.10; the backward kernels take 0.95 ... 1.5 of the time and stay there.
+  if (p.dk == 128 && (p.g.S != 16 || p.g.WR != 1)) return false;
+  if (p.dk == 128 || (p.g.WR == 2 && p.dk == 64)) {
+    const int64_t sb = Swat<64, 1, 1, 2>::SB, strips = (p.g.TC + sb - 1) / sb;
+    if (p.g.WC != 1 || p.g.TC < sb || (p.dk == 128 && 4 * p.g.TC < 3 * sb * strips)) return false;
+    if (4 * (int64_t)p.B * p.H * strips * p.g.TR < dlt_device_cus()) return false;
   }
   if (!swat_rows_ok(p, t.q, t.qs) || !swat_rows_ok(p, t.k, t.ks) || !swat_rows_ok(p, t.v, t.vs)) return false;
   if (!bwd) return swat_rows_ok(p, t.out_o, t.os);
@@ -639,7 +645,7 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
     a.ring_p[i] = ring_p[i];
     for (int j = 0; j < 5; j++) a.ring_s[i][j] = ring_s[i][j];
   }
-  const int sb = a.one ? (p.dk == 32 ? Swab<32, 1, 1, 1>::SB : Swab<64, 1, 1, 1>::SB) : p.dk == 64 && p.g.WR == 2 ? Swat<64, 1, 1, 2>::SB : 8, strip = 16 * sb;
+  const int sb = a.one ? (p.dk == 32 ? Swab<32, 1, 1, 1>::SB : Swab<64, 1, 1, 1>::SB) : p.dk == 128 || (p.dk == 64 && p.g.WR == 2) ? Swat<64, 1, 1, 2>::SB : 8, strip = 16 * sb;
   a.nstrips = (p.g.XLq + strip - 1) / strip;
   const int64_t cols = slabs * a.nstrips;
   a.lone = !bwd && p.tm.img && dlt_image_fwd_alone(p.dk, p.g.S, p.g.WR, p.g.WC, p.g.TR, p.g.TC, p.H, cols, cus);
@@ -649,6 +655,7 @@ int swat_run(const AttnProblem& p, const AttnTensors& t, bool bwd, hipStream_t s
   dlt_band_plan(p.g.TR, cols, two ? 2 * cus : cus, a.band, a.nbands);
   const int64_t grid = cols * a.nbands;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "attention: grid too large");
+  if (p.dk == 128) return dlt_swat_launch_128(a, p.dtype, bwd, (int)grid, stream);
   return p.dk == 32 ? dlt_swat_launch_32(a, p.dtype, bwd, (int)grid, stream) : dlt_swat_launch_64(a, p.dtype, bwd, (int)grid, stream);
 }
 

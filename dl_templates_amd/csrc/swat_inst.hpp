@@ -64,6 +64,9 @@ template <typename TIO>
 int swat_pick(const SwatArgs& a, bool bwd, int grid, hipStream_t stream) {
 #define DLT_SWAT(NTB, WC, WR) return bwd ? swat_launch_bwd<TIO, NTB, WC, WR>(a, grid, stream) : swat_launch_fwd<TIO, NTB, WC, WR>(a, grid, stream)
   const int ntb = a.g.S / 16;
+#if DLT_D == 128   // forward only (swat_eligible)
+  if (!bwd && ntb == 1 && a.g.WR == 1 && a.g.WC == 1) return swat_launch_fwd<TIO, 1, 1, 1>(a, grid, stream);
+#else
   if (ntb == 2) DLT_SWAT(2, 1, 1);
   if (a.g.WR == 1) {
     if (a.g.WC == 1) DLT_SWAT(1, 1, 1);
@@ -72,6 +75,7 @@ int swat_pick(const SwatArgs& a, bool bwd, int grid, hipStream_t stream) {
   if (a.g.WC == 1) DLT_SWAT(1, 1, 2);
 #if DLT_D == 32
   DLT_SWAT(1, 2, 2);
+#endif
 #endif
   return dlt_set_error(DLT_ERR_UNSUPPORTED, "marching tile-window kernels: no instantiation for this window");
 #undef DLT_SWAT

@@ -1,10 +1,10 @@
-// Marching kernels for windows over tiles of 16 or 32 tokens at head dim 32 / 64 (the reference's demo regime,
+// Marching kernels for windows over tiles of 16 or 32 tokens at head dim 32 / 64, forward also at 128 (the reference's demo regime,
 // src/tiled_swa.py:142-244 and :741-750), in the token layout and in the image layout.
 //
 // What bounded the chunked kernels here: a query tile sees only 9 ... 25 tiles, so a workgroup of 128 queries walked nine
 // 64-token chunks, each a load, two barriers and work for one or two of its four waves (image layout, B = 4, H = 8,
 // 256 x 256 pixels, 4 x 4-pixel tiles, d = 32: forward 301 us for 537 MB, latency of 9 rounds, 1.8 TB/s).
-// Here a workgroup owns a strip of 8 blocks of 16 tokens (one per wave; 4 at head dim 64 with five window rows) and marches down the grid rows.  The rows its
+// Here a workgroup owns a strip of 8 blocks of 16 tokens (one per wave; 4 at head dim 64 with five window rows and at 128) and marches down the grid rows.  The rows its
 // window covers (2 WR + 1 grid rows of both streamed tensors) live in an LDS ring; a step needs one new row, which travels
 // HBM -> registers while the step computes, so every row is fetched once per strip and the loads of a step have a whole
 // step to arrive.  All tiles of the window are resident: the softmax is one-shot, there is no mask inside a tile (a block of
@@ -39,7 +39,7 @@ struct Swat {
   static constexpr int NWB = (2 * WC + 1) * NTB, NR = 2 * WR + 1;   // 16-token blocks per window row, window rows
   static constexpr int NB = NR * NWB, NP = (NB + 1) / 2;            // blocks of a window, pairs of them (32 tokens of a product)
   // strips of four blocks where a ring of eight exceeds the LDS; one wave per SIMD then, with all of its registers
-  static constexpr int SB = D == 64 && WR == 2 ? 4 : 8, THREADS = 64 * SB;   // 16-token blocks of a strip, one per wave
+  static constexpr int SB = D == 128 || (D == 64 && WR == 2) ? 4 : 8, THREADS = 64 * SB;   // 16-token blocks of a strip, one per wave
   static constexpr int HB = SB + 2 * WC * NTB, TOK = 16 * HB;       // staged blocks / tokens per grid row
   static constexpr int ROWB = 2 * D, BLKB = 16 * ROWB, TB = TOK * ROWB, SLOT = 2 * TB;
   static constexpr int PIECES = D / 8, NV = 2 * TOK * PIECES, NIT = (NV + THREADS - 1) / THREADS;
@@ -55,7 +55,7 @@ struct Swat {
   static_assert(RING + SCAL <= 160 * 1024, "the ring exceeds the LDS");
 };
 
-template <int D> DLT_DEV int swat_swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : t & 7; }
+template <int D> DLT_DEV int swat_swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : D / 64 * (t & 7); }
 
 typedef DLT_LDS char* swat_lds;
 DLT_DEV u32x4 swat_read16(swat_lds p) { return *reinterpret_cast<DLT_LDS u32x4*>(p); }

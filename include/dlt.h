@@ -301,7 +301,7 @@ int dlt_debug_copy(void* dst, const void* src, int64_t bytes, void* stream);
  * of the real ones, so the query also works in a process without a GPU.
  *   MARCHING  token grids (b_size 1), head dim 32, windows up to 21 x 21, and 64, up to 13 x 13 (rotation: head dim 64, 8 rotary pairs, in
  *             the backward pass rotated q / k kept), also the forward pass of fp32 tensors at head dim 32; tiles of 16 or 32
- *             tokens at those head dims report FLASH
+ *             tokens report FLASH on every kernel
  *   STREAMING token grids, head dim 64 / 128, windows up to 93 columns (beyond 21 columns in column passes), no rotation;
  *             tiles of 2 ... 15 tokens at head dim 64 / 128 (the grid of token slots, up to 24 column groups of 4 slots), through
  *             dlt_swa_*_narrow also at multiples of 8 below 64
