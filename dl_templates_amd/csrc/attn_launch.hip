@@ -595,7 +595,7 @@ bool flash_eligible(const AttnProblem& p, const AttnTensors& t, bool with_do) {
 
 // ---- marching tile-window kernels: tiles of 16 or 32 tokens, head dim 32 or 64 exactly, forward also 128 -----------------
 // What they take beyond flash_eligible: windows whose rows fit the LDS ring (3 x 3 tiles; with 16-token tiles also 5 tile
-// columns, 5 tile rows at head dim 32, and 5 x 3 tiles at 64), and 16-byte rows with 32-bit offsets for every tensor.  Larger tiles stay on the
+// columns, 5 tile rows at head dim 32, 5 x 3 tiles at 64 and 5 x 5 there in the forward pass), and 16-byte rows with 32-bit offsets for every tensor.  Larger tiles stay on the
 // flash kernels: a window row of 64-token tiles gives a 64-token chunk work for every wave, and its rows do not fit the ring.
 bool swat_rows_ok(const AttnProblem& p, const void* ptr, const int64_t* st) {
   return tvec_ok(ptr, st, p.dk, 2) && st[2] >= 0 && st[4] >= 0 && slab_span(p, st, (int64_t)p.g.TR * p.g.XLq) * 2 <= ((int64_t)1 << 31) - 1;
@@ -610,12 +610,15 @@ bool swat_eligible(const AttnProblem& p, const AttnTensors& t, bool bwd) {
   // columns, whose last strip is nearly empty, 1.04 ... 1.15, no longer with their forward pass): 2 slabs of 30 x 30 tiles 25.3 -> 9.6 and
   // 52.4 -> 29.5 us, 64 of 21 x 33 206 -> 133 and 537 -> 440.  Up to 56 the window's keys over a workgroup's waves (flash_tiles_split) are
   // faster: 2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2.
+  // The same with five columns, forward (the scalars of the backward pass do not fit beside the ring): 0.41 ... 0.98, 64 slabs of 21 x 33 225 -> 174, 4 of 40 x 12
+  // 28.9 -> 11.9.
   // d = 128, 3 x 3 tiles, forward: 0.40 ... 0.98 where strips are three quarters full (2 slabs of 30 x 30 23.8 -> 13.4, 64 of 30 x 10 174 -> 106), five columns
   // up to 1.10; the backward kernels take 0.95 ... 1.5 of the time and stay there.
   if (p.dk == 128 && (p.g.S != 16 || p.g.WR != 1)) return false;
   if (p.dk == 128 || (p.g.WR == 2 && p.dk == 64)) {
     const int64_t sb = Swat<64, 1, 1, 2>::SB, strips = (p.g.TC + sb - 1) / sb;
-    if (p.g.WC != 1 || p.g.TC < sb || (p.dk == 128 && 4 * p.g.TC < 3 * sb * strips)) return false;
+    if (p.g.WC == 2 && (p.dk == 128 || bwd)) return false;
+    if (p.g.TC < sb || (p.dk == 128 && 4 * p.g.TC < 3 * sb * strips)) return false;
     if (4 * (int64_t)p.B * p.H * strips * p.g.TR < dlt_device_cus()) return false;
   }
   if (!swat_rows_ok(p, t.q, t.qs) || !swat_rows_ok(p, t.k, t.ks) || !swat_rows_ok(p, t.v, t.vs)) return false;

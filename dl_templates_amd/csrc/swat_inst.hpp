@@ -36,6 +36,7 @@ int swat_launch_bwd_one(const SwatArgs& a, int grid, hipStream_t stream) {
 template <typename TIO, int NTB, int WC, int WR>
 int swat_launch_bwd_two(const SwatArgs& a, int grid, hipStream_t stream) {
   typedef Swat<DLT_D, NTB, WC, WR> C;
+  static_assert(C::BWD, "ring and scalars exceed the LDS");
   // dQ first: it produces the delta vector the dK/dV kernel consumes
   auto kq = swat_bwd_q_kernel<TIO, DLT_D, NTB, WC, WR>;
   auto kkv = swat_bwd_kv_kernel<TIO, DLT_D, NTB, WC, WR>;
@@ -75,6 +76,8 @@ int swat_pick(const SwatArgs& a, bool bwd, int grid, hipStream_t stream) {
   if (a.g.WC == 1) DLT_SWAT(1, 1, 2);
 #if DLT_D == 32
   DLT_SWAT(1, 2, 2);
+#else
+  if (!bwd) return swat_launch_fwd<TIO, 1, 2, 2>(a, grid, stream);   // swat_eligible
 #endif
 #endif
   return dlt_set_error(DLT_ERR_UNSUPPORTED, "marching tile-window kernels: no instantiation for this window");

@@ -52,7 +52,8 @@ struct Swat {
   // columns 214 -> 209, d = 32, five rows 138 -> 131.
   static constexpr bool RUNS = !(D == 32 && (WC == 2 || NTB == 2));
   static_assert((TOK * PIECES) % 64 == 0, "a wave stages one tensor per vector");
-  static_assert(RING + SCAL <= 160 * 1024, "the ring exceeds the LDS");
+  static constexpr bool BWD = RING + SCAL <= 160 * 1024;   // else forward only
+  static_assert(RING <= 160 * 1024, "the ring exceeds the LDS");
 };
 
 template <int D> DLT_DEV int swat_swz(int t) { return D == 32 ? ((t >> 2) & 1) << 1 : D / 64 * (t & 7); }

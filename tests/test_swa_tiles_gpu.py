@@ -290,12 +290,12 @@ def test_tiles_of_64_tokens(th, tw, tile, WR, WC, dk, dv, many):
         assert torch.equal(all_, one.expand_as(all_))   # the same bits in both workgroup sizes
 
 
-# windows of 5 x 3 tiles at d = 64 and, forward, 3 x 3 at d = 128, on strips of four tiles: grids below the window, rows below a band's ring, strips whole,
+# windows of 5 x 3 tiles at d = 64 and, forward, 3 x 3 at d = 128 and 5 x 5 at d = 64, on strips of four tiles: grids below the window, rows below a band's ring, strips whole,
 # ragged and with one tile, the fewest strips of the rule; image layout with the same bits; infinite and NaN tiles stay with the queries that see them
-@pytest.mark.parametrize("WR,d", [(2, 64), (1, 128)])
+@pytest.mark.parametrize("WR,WC,d", [(2, 1, 64), (1, 1, 128), (2, 2, 64)])
 @pytest.mark.parametrize("th,tw,B,dtype", [(1, 4, 80, torch.float16), (2, 5, 20, torch.bfloat16), (4, 8, 8, torch.float16), (11, 9, 2, torch.bfloat16), (7, 13, 9, torch.float16),
                                           (5, 4, 200, torch.bfloat16)])
-def test_strips_of_four_tiles(th, tw, B, dtype, WR, d):
+def test_strips_of_four_tiles(th, tw, B, dtype, WR, WC, d):
     sw = _swa()
     S, H, scale = 16, 2, 0.125
     N = th * tw * S
@@ -304,26 +304,26 @@ def test_strips_of_four_tiles(th, tw, B, dtype, WR, d):
 
     def run(q, k, v, do):
         leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
-        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, 1, scale)
+        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
         return (o.detach(),) + torch.autograd.grad(o, leaves, do)
 
     got = run(*dev)
     for b in (0, B - 1):
-        want = orc.tiled_swa_grads(*(t[b:b + 1].float() for t in ops), S, th, tw, WR, 1, scale)
+        want = orc.tiled_swa_grads(*(t[b:b + 1].float() for t in ops), S, th, tw, WR, WC, scale)
         assert (got[0][b:b + 1].float().cpu() - want[0]).abs().max().item() <= FWD_TOL
         assert max(_rel(g[b:b + 1], w) for g, w in zip(got[1:], want[1:])) <= GRAD_TOL
     lay = lambda t: orc.tokens_to_image(t.cpu(), th, tw, 4, 4).contiguous().cuda()
     leaves = [lay(t).requires_grad_(True) for t in ops[:3]]
-    o = sw.TiledSwaImage.apply(*leaves, 4, 4, WR, 1, scale)
+    o = sw.TiledSwaImage.apply(*leaves, 4, 4, WR, WC, scale)
     assert all(torch.equal(x, lay(y)) for x, y in zip((o,) + torch.autograd.grad(o, leaves, lay(ops[3])), got))
     cell = torch.arange(N, device="cuda") // S
     at = cell == th // 2 * tw + tw // 2
-    far = ((cell // tw - th // 2).abs() > WR) | ((cell % tw - tw // 2).abs() > 1)
+    far = ((cell // tw - th // 2).abs() > WR) | ((cell % tw - tw // 2).abs() > WC)
     q, k, v, do = (t.clone() for t in dev)
     k[:, :, at], v[:, :, at] = float("inf"), float("nan")
     o, dq, _, _ = run(q, k, v, do)
     assert torch.equal(o[:, :, far], got[0][:, :, far])
-    if d == 128:   # the gradients come from the chunked flash kernels, whose masked products of a whole chunk meet NaN
+    if d == 128 or WC == 2:   # the gradients come from the chunked flash kernels, whose masked products of a whole chunk meet NaN
         return
     assert torch.equal(dq[:, :, far], got[1][:, :, far])
     q, k, v, do = (t.clone() for t in dev)
