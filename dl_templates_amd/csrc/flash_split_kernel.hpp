@@ -93,6 +93,13 @@ struct FlashsTile {
       lds_write16(s + t * 2 * D + 16 * (p ^ flashs_swz<D>(t)), r[it]);
     }
   }
+  // A block's tokens from `left` on repeat the list's last one: their probabilities are 0, which times an infinite value is not, so that they are cleared
+  static DLT_DEV void clear_past(u32x4 (&r)[NV], int left, int lane) {
+    if (left >= 32) return;   // wave-uniform
+#pragma unroll
+    for (int it = 0; it < NV; it++)
+      if ((lane + 64 * it) / (D / 8) >= left) r[it] = u32x4{0u, 0u, 0u, 0u};
+  }
   // A operand, 16 tokens (half mb) x dims 32 c ..
   static DLT_DEV u32x4 rows(const char* s, int mb, int c, int n, int g) {
     return lds_read16(s + (16 * mb + n) * 2 * D + 16 * ((4 * c + g) ^ flashs_swz<D>(n)));
@@ -218,6 +225,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
   }
   const float scale = a.scale_log2;
   for (int kb = wave; kb < nkb; kb += NW) {
+    VT::clear_past(vr, keys.len - 32 * kb, lane);
     VT::write(sV, vr, lane);
     u32x4 ka[2][KC];
 #pragma unroll
@@ -393,6 +401,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
   }
   const float scale = a.scale_log2;
   for (int kb = wave; kb < nkb; kb += NW) {
+    KT::clear_past(kr, keys.len - 32 * kb, lane);
     KT::write(sK, kr, lane);
     u32x4 va[2][VC];
 #pragma unroll
@@ -421,9 +430,9 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
         const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, keys.len - 1) : keys.len - 1;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float pv = fast_exp2(fmaf(s[i], scale, nlse[p]));
-          if (tail) pv = 32 * kb + 16 * mb + 4 * g + i <= klim ? pv : 0.f;
-          ds[p][4 * mb + i] = pv * dp[i];
+          float dsv = fast_exp2(fmaf(s[i], scale, nlse[p])) * dp[i];
+          if (tail) dsv = 32 * kb + 16 * mb + 4 * g + i <= klim ? dsv : 0.f;
+          ds[p][4 * mb + i] = dsv;
         }
       }
     }
@@ -514,6 +523,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
   }
   const float scale = a.scale_log2;
   for (int qbk = first; qbk < nqb; qbk += NW) {
+    QT::clear_past(qr, queries.len - 32 * qbk, lane);
+    DT::clear_past(dr, queries.len - 32 * qbk, lane);
     QT::write(sQ, qr, lane);
     DT::write(sD, dr, lane);
     sc[lane] = scr;
@@ -538,13 +549,15 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
         const int qmin = CAUSAL ? x0 + 16 * p + n : 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float pv = fast_exp2(fmaf(s[i], scale, -lq[i]));
+          float pv = fast_exp2(fmaf(s[i], scale, -lq[i])), dsv = -pv * dp[i];
           if (tail) {
             const int qi = 32 * qbk + 16 * mb + 4 * g + i;
-            pv = (qi >= qmin && qi < queries.len) ? pv : 0.f;
+            const bool in = qi >= qmin && qi < queries.len;
+            pv = in ? pv : 0.f;
+            dsv = in ? dsv : 0.f;
           }
           pr[p][4 * mb + i] = pv;
-          ds[p][4 * mb + i] = -pv * dp[i];
+          ds[p][4 * mb + i] = dsv;
         }
       }
     }

@@ -40,6 +40,12 @@ struct Swat {
   static constexpr int NB = NR * NWB, NP = (NB + 1) / 2;            // blocks of a window, pairs of them (32 tokens of a product)
   // strips of four blocks where a ring of eight exceeds the LDS; one wave per SIMD then, with all of its registers
   static constexpr int SB = D == 128 || (D == 64 && WR == 2) ? 4 : 8, THREADS = 64 * SB;   // 16-token blocks of a strip, one per wave
+  // Strips of four write slots outside the grid as zeros: their probabilities are 0, and 0 times an infinite value is not.  A workgroup there fills a
+  // ring of up to 147 KB, beside which the ANDs are 0 ... 3 %; strips of eight, which it would cost 1 ... 4 % (32 slabs of 16 x 16 tiles, d = 32: 10.7 -> 11.1 us), hold copies of the edge
+  static constexpr bool CLEAR = SB == 4;
+  // The last of an odd number of blocks has zeros beside it instead of its values again, for the same reason: no time or less but at five columns and strips of
+  // eight (d = 64, 16 slabs of 40 x 40 tiles: forward 52.4 -> 53.4 us, backward 151 -> 162)
+  static constexpr bool ALONE = CLEAR || WC == 1;
   static constexpr int HB = SB + 2 * WC * NTB, TOK = 16 * HB;       // staged blocks / tokens per grid row
   static constexpr int ROWB = 2 * D, BLKB = 16 * ROWB, TB = TOK * ROWB, SLOT = 2 * TB;
   static constexpr int PIECES = D / 8, NV = 2 * TOK * PIECES, NIT = (NV + THREADS - 1) / THREADS;
@@ -111,6 +117,8 @@ struct SwatRing {
   uint32_t goff[C::NIT];           // this thread's pieces: offset inside a grid row, LDS offset inside a slot
   int loff[C::NIT];
   bool second[C::NIT];             // wave-uniform
+  unsigned outside;                // wave-uniform, bit `it`: the slots of that vector lie outside the grid row
+  bool row_in;                     // the row in flight lies inside the grid
   u32x4 r[C::NIT];
   int tid, TR;
 
@@ -121,20 +129,24 @@ struct SwatRing {
     rs0 = swat_row_bytes(a.tm, s0, XL);
     rs1 = swat_row_bytes(a.tm, s1, XL);
     const int xh = xs - (C::HB - C::SB) * 8;   // first staged slot: half of the extra blocks lie to the left
+    outside = 0;
 #pragma unroll
     for (int it = 0; it < C::NIT; it++) {
       const int id = tid + C::THREADS * it;
       second[it] = 64 * wave + C::THREADS * it >= C::NV / 2;
       const int v = second[it] ? id - C::NV / 2 : id;
       const int tok = v / C::PIECES, piece = v % C::PIECES;
-      // slots outside the grid row are clamped onto it: they belong to tiles that nobody sees
+      // slots outside the grid row are clamped onto it: they belong to tiles that nobody sees (CLEAR)
       const int x = dlt_imax(0, dlt_imin(xh + tok, XL - 1));
+      const int x0 = xh + (64 * wave + C::THREADS * it - (second[it] ? C::NV / 2 : 0)) / C::PIECES;   // a vector's slots lie in one block of 16
+      outside |= (unsigned)(x0 < 0 || x0 >= XL) << it;
       goff[it] = (second[it] ? swat_slot_off(a.tm, s1, x) : swat_slot_off(a.tm, s0, x)) + 16 * piece;
       loff[it] = (second[it] ? C::TB : 0) + tok * C::ROWB + 16 * (piece ^ swat_swz<C::ROWB / 2>(tok));
     }
   }
-  // rows outside the grid are clamped onto it as well
+  // rows outside the grid likewise
   DLT_DEV void issue(int row) {
+    row_in = row >= 0 && row < TR;
     const uint32_t rc = (uint32_t)dlt_imax(0, dlt_imin(row, TR - 1));
     const uint32_t o0 = rc * rs0, o1 = rc * rs1;
 #pragma unroll
@@ -143,9 +155,11 @@ struct SwatRing {
         r[it] = *reinterpret_cast<const u32x4*>((second[it] ? base1 : base0) + (goff[it] + (second[it] ? o1 : o0)));
   }
   DLT_DEV void commit(int slot) {
+    const unsigned zero = row_in ? outside : ~0u;
 #pragma unroll
     for (int it = 0; it < C::NIT; it++)
-      if (C::NV % C::THREADS == 0 || it + 1 < C::NIT || tid + C::THREADS * it < C::NV) swat_write16(lds + slot * C::SLOT + loff[it], r[it]);
+      if (C::NV % C::THREADS == 0 || it + 1 < C::NIT || tid + C::THREADS * it < C::NV)
+        swat_write16(lds + slot * C::SLOT + loff[it], C::CLEAR ? r[it] & ((zero >> it & 1u) - 1u) : r[it]);
   }
   // window rows of the first step: all requested before the first is written
   DLT_DEV void fill(int first) {
@@ -160,6 +174,7 @@ struct SwatRing {
     for (int i = 0; i < C::NR; i++) {
 #pragma unroll
       for (int it = 0; it < C::NIT; it++) r[it] = pre[i][it];
+      row_in = first + i >= 0 && first + i < TR;
       commit(i);
     }
   }
@@ -309,12 +324,13 @@ __global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, 
 #pragma unroll
       for (int t = 0; t < C::NP; t++) {
         constexpr int LAST = C::NB - 1;
-        const int b0 = 2 * t, b1 = 2 * t + 1 <= LAST ? 2 * t + 1 : 2 * t;
+        const bool pair = 2 * t < LAST;
+        const int b0 = 2 * t, b1 = pair ? 2 * t + 1 : 2 * t;
         float p[8];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           p[i] = fast_exp2(fmaf(s[b0][i], scale, neg_m2));
-          p[4 + i] = 2 * t + 1 <= LAST ? fast_exp2(fmaf(s[b1][i], scale, neg_m2)) : 0.f;
+          p[4 + i] = pair ? fast_exp2(fmaf(s[b1][i], scale, neg_m2)) : 0.f;
         }
         const u32x4 pb = pack8<CT>(p);
         if constexpr (LATE_Q)
@@ -322,7 +338,7 @@ __global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, 
         swat_lds v0 = rowp[b0 / C::NWB] + C::TB + (b0 % C::NWB) * C::BLKB, v1 = rowp[b1 / C::NWB] + C::TB + (b1 % C::NWB) * C::BLKB;
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(v0 + L.tr[d]), hi = swat_read_tr(v1 + L.tr[d]);
+          const u32x2 lo = swat_read_tr(v0 + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(v1 + L.tr[d]) : u32x2{0u, 0u};
           acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc[d]);
         }
         acc_l = Mma<CT>::mfma(ones, pb, acc_l);
@@ -450,11 +466,12 @@ __global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, 
           for (int i = 0; i < 4; i++) ds[4 * u + i] = fast_exp2(fmaf(s[i], scale, nlse)) * dp[i];
         }
         const u32x4 dsb = pack8<CT>(ds);
-        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        const bool pair = 2 * t + 1 < C::NB;
+        const int b0 = 2 * t, b1 = pair ? 2 * t + 1 : 2 * t;
         swat_lds k0 = rowp[b0 / C::NWB] + (b0 % C::NWB) * C::BLKB, k1 = rowp[b1 / C::NWB] + (b1 % C::NWB) * C::BLKB;
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(k0 + L.tr[d]), hi = swat_read_tr(k1 + L.tr[d]);
+          const u32x2 lo = swat_read_tr(k0 + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(k1 + L.tr[d]) : u32x2{0u, 0u};
           acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
         }
       }
@@ -599,16 +616,17 @@ __global__ __launch_bounds__((Swat<D, NTB, WC, WR>::THREADS), (Swat<D, NTB, WC, 
           }
         }
         const u32x4 pb = pack8<CT>(p), dsb = pack8<CT>(ds);
-        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        const bool pair = 2 * t + 1 < C::NB;
+        const int b0 = 2 * t, b1 = pair ? 2 * t + 1 : 2 * t;
         swat_lds q0 = rowp[b0 / C::NWB] + (b0 % C::NWB) * C::BLKB, q1 = rowp[b1 / C::NWB] + (b1 % C::NWB) * C::BLKB;
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(q0 + C::TB + L.tr[d]), hi = swat_read_tr(q1 + C::TB + L.tr[d]);
+          const u32x2 lo = swat_read_tr(q0 + C::TB + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(q1 + C::TB + L.tr[d]) : u32x2{0u, 0u};
           acc_v[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc_v[d]);
         }
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(q0 + L.tr[d]), hi = swat_read_tr(q1 + L.tr[d]);
+          const u32x2 lo = swat_read_tr(q0 + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(q1 + L.tr[d]) : u32x2{0u, 0u};
           acc_k[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc_k[d]);
         }
       }
@@ -813,11 +831,12 @@ __global__ __launch_bounds__((Swab<D, NTB, WC, WR>::THREADS), (Swab<D, NTB, WC, 
           for (int i = 0; i < 4; i++) ds[4 * u + i] = fast_exp2(fmaf(s[i], scale, nlse)) * dp[i];
         }
         const u32x4 dsb = pack8<CT>(ds);
-        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        const bool pair = 2 * t + 1 < C::NB;
+        const int b0 = 2 * t, b1 = pair ? 2 * t + 1 : 2 * t;
         swat_lds k0 = rowp[b0 / C::NWB] + (b0 % C::NWB) * C::BLKB, k1 = rowp[b1 / C::NWB] + (b1 % C::NWB) * C::BLKB;
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(k0 + L.tr[d]), hi = swat_read_tr(k1 + L.tr[d]);
+          const u32x2 lo = swat_read_tr(k0 + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(k1 + L.tr[d]) : u32x2{0u, 0u};
           acc[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc[d]);
         }
       }
@@ -866,16 +885,17 @@ __global__ __launch_bounds__((Swab<D, NTB, WC, WR>::THREADS), (Swab<D, NTB, WC, 
           }
         }
         const u32x4 pb = pack8<CT>(p), dsb = pack8<CT>(ds);
-        const int b0 = 2 * t, b1 = 2 * t + 1 < C::NB ? 2 * t + 1 : 2 * t;
+        const bool pair = 2 * t + 1 < C::NB;
+        const int b0 = 2 * t, b1 = pair ? 2 * t + 1 : 2 * t;
         swat_lds q0 = rowp[b0 / C::NWB] + 2 * C::TB + (b0 % C::NWB) * C::BLKB, q1 = rowp[b1 / C::NWB] + 2 * C::TB + (b1 % C::NWB) * C::BLKB;
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(q0 + C::TB + L.tr[d]), hi = swat_read_tr(q1 + C::TB + L.tr[d]);
+          const u32x2 lo = swat_read_tr(q0 + C::TB + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(q1 + C::TB + L.tr[d]) : u32x2{0u, 0u};
           acc_v[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, acc_v[d]);
         }
 #pragma unroll
         for (int d = 0; d < C::DB; d++) {
-          const u32x2 lo = swat_read_tr(q0 + L.tr[d]), hi = swat_read_tr(q1 + L.tr[d]);
+          const u32x2 lo = swat_read_tr(q0 + L.tr[d]), hi = pair || !C::ALONE ? swat_read_tr(q1 + L.tr[d]) : u32x2{0u, 0u};
           acc_k[d] = Mma<CT>::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, dsb, acc_k[d]);
         }
         // 128 registers a lane: reads hoisted across pairs of blocks spilled the pieces in flight, a wait for them at the step's start

@@ -330,3 +330,35 @@ def test_strips_of_four_tiles(th, tw, B, dtype, WR, WC, d):
     q[:, :, at], do[:, :, at] = float("nan"), float("inf")
     _, _, dk, dv = run(q, k, v, do)
     assert torch.equal(dk[:, :, far], got[2][:, :, far]) and torch.equal(dv[:, :, far], got[3][:, :, far])
+
+
+# A value row with infinities: queries that see it get them in those dims and their plain results in the others, also where the window has an odd number of
+# 16-token runs (the last pair of runs holds nothing beside the last one) and where it hangs over the grid's edge (strips of eight tiles: rows
+# away from it, `edge`); the same for dV under a dO row with them.  Windows' keys over waves (runs of 16, 48 and 80 tokens), strips of four tiles and of eight
+@pytest.mark.parametrize("th,tw,S,WR,WC,d,slabs,bwd,edge", [
+    (5, 6, 16, 1, 3, 64, 1, True, True), (4, 5, 16, 1, 1, 128, 1, True, True), (3, 5, 48, 1, 1, 64, 1, True, True), (3, 4, 80, 1, 1, 32, 1, True, True),
+    (9, 8, 16, 1, 1, 128, 8, False, True), (9, 8, 16, 2, 1, 64, 8, True, True), (6, 9, 16, 2, 2, 64, 16, False, True), (7, 9, 16, 1, 1, 32, 4, True, False)])
+def test_infinite_values_reach_the_queries_that_see_them(th, tw, S, WR, WC, d, slabs, bwd, edge):
+    sw, N, scale, inf = _swa(), th * tw * S, 1 / math.sqrt(d), float("inf")
+    q, k, v, do = (t.cuda() for t in orc.make_qkv(N + d, 1, slabs, N, N, d, d, torch.bfloat16))
+
+    def run(v, do):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, scale)
+        return (o.detach(),) + torch.autograd.grad(o, leaves, do)
+
+    o, _, dk, dv = run(v, do)
+    cell = torch.arange(N, device="cuda") // S
+    for r, c in ((th // 2, tw // 2),) + (((0, 0), (th - 1, tw - 1), (0, tw - 1), (th - 1, 0)) if edge else ()):
+        at = (r * tw + c) * S + (S - 1 if r else 0)
+        sees = ((cell // tw - r).abs() <= WR) & ((cell % tw - c).abs() <= WC)
+        bad, want = v.clone(), o.clone()
+        for t, rows in ((bad, at), (want, sees)):
+            t[:, :, rows, 3], t[:, :, rows, d - 1] = inf, -inf
+        assert torch.equal(run(bad, do)[0], want), (r, c)
+        if bwd:
+            bad, want = do.clone(), dv.clone()
+            for t, rows in ((bad, at), (want, sees)):
+                t[:, :, rows, 3], t[:, :, rows, d - 1] = inf, -inf
+            _, _, dk2, dv2 = run(v, bad)
+            assert torch.equal(dv2, want) and torch.equal(dk2[:, :, ~sees], dk[:, :, ~sees]), (r, c)
