@@ -114,17 +114,18 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
   }
   u32x4 qf[KC], qlo[KC];
 
-  // a probability of 0 times an infinite value is not 0: columns that no query of the wave sees are cleared
-  u32x4 vmask = {~0u, ~0u, ~0u, ~0u};
-  if (whole) {
+  // a probability of 0 times an infinite value is not 0: the columns of a block from kx on that no query of the wave sees are cleared
+  auto seen_values = [&](int kx) {
     unsigned m[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const int x = (i < 4 || a.pair ? 4 * g : 16 + 4 * g) + (i & 3);
+      const int x = kx + (i < 4 || a.pair ? 4 * g : 16 + 4 * g) + (i & 3);
       m[i] = x >= wlo && x < whi ? 0xffffu : 0u;
     }
-    vmask = u32x4{m[0] | m[1] << 16, m[2] | m[3] << 16, m[4] | m[5] << 16, m[6] | m[7] << 16};
-  }
+    return u32x4{m[0] | m[1] << 16, m[2] | m[3] << 16, m[4] | m[5] << 16, m[6] | m[7] << 16};
+  };
+  // (the blocks of longer rows start at the first such column: it is their last one that holds others)
+  const u32x4 vmask = seen_values(whole ? 0 : wlo + (whi - 1 - wlo) / 32 * 32), all = {~0u, ~0u, ~0u, ~0u};
   // slots past the halo's columns hold no value
   for (int i = tid; i < a.chunk_rows * (cx - w) * (DV / 8); i += 256) {
     const int t = i / (DV / 8), ri = t / (cx - w);
@@ -211,10 +212,10 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
 #pragma unroll
           for (int d = 0; d < VB; d++) acc[d] *= alpha;
         }
-        const u32x4 pb = pack8<CT>(t);
+        const u32x4 pb = pack8<CT>(t), seen = whole || kx + 32 > whi ? vmask : all;
 #pragma unroll
         for (int d = 0; d < VB; d++) {
-          vt[d] &= vmask;
+          vt[d] &= seen;
           if (lone) vt[d].z = vt[d].w = 0u;
           acc[d] = Mma<CT>::mfma(vt[d], pb, acc[d]);
         }

@@ -292,7 +292,7 @@ def test_marching_fp32(th, tw, WR, WC):
 
 # fp32 windows off the marching kernel: rows of one, two and more 16-token blocks, halo rows dealt over four waves, two and one (slab counts on both
 # sides of the lines), pairs of rows with an odd one left, several chunks (last case of each kind), every head dim class and dims below it;
-# a key row of infinities or NaN changes no query that does not see it
+# a key row of infinities or NaN changes no query that does not see it, a value row none whose block of 16 columns does not
 @pytest.mark.parametrize("BH,S,th,tw,WR,WC,dk,dv", [
     (1, 1, 1, 1, 0, 0, 64, 64), (2, 1, 9, 15, 4, 3, 64, 64), (40, 1, 17, 16, 2, 2, 64, 64), (150, 1, 9, 11, 3, 1, 64, 64), (3, 1, 70, 13, 40, 5, 64, 64),
     (2, 1, 10, 17, 1, 4, 64, 64), (60, 1, 13, 31, 4, 2, 40, 64), (2, 1, 40, 32, 18, 9, 128, 128), (70, 1, 9, 24, 2, 2, 96, 80),
@@ -317,7 +317,14 @@ def test_windows_fp32(BH, S, th, tw, WR, WC, dk, dv):
     for value in (float("inf"), float("nan")):
         k2 = k.clone()
         k2[:, :, bad] = value
-        assert (sw.tiled_swa_fwd(q, k2, v, S, th, tw, WR, WC, scale)[:, :, blind] - o[:, :, blind]).abs().sum().item() <= FWD_TOL * BH * N
+        assert torch.equal(sw.tiled_swa_fwd(q, k2, v, S, th, tw, WR, WC, scale)[:, :, blind], o[:, :, blind])
+    for at in sorted({bad, 0, tw - 1, tw // 2, (th // 2) * tw, (th // 2) * tw + tw - 1, min(tw - 1, 16 + WC), N - 1}):
+        first = cell % tw // 16 * 16
+        apart = ((cell // tw - at // tw).abs() > WR) | (at % tw < first - WC) | (at % tw > first + 15 + WC)
+        for value in (float("inf"), float("nan")):
+            v2 = v.clone()
+            v2[:, :, at] = value
+            assert torch.equal(sw.tiled_swa_fwd(q, k, v2, S, th, tw, WR, WC, scale)[:, :, apart], o[:, :, apart])
 
 
 # two stacked patches per wave (streaming kernels, more workgroups than CUs): bands without a lower patch, one band and a bit, ragged
