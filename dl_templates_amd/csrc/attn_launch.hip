@@ -474,8 +474,9 @@ bool swag_f32_eligible(const AttnProblem& p, const AttnTensors& t) {
 // fp32 windows on the kernel of attn_win_kernel.hpp: one token to a tile (larger ones keep the bits of the image layout, which the generic kernel
 // serves), rows readable in 16-byte pieces, slabs of less than 2^31 bytes, no rotation, and one halo row
 // at least fits the LDS; false: the generic kernel.  Generic -> this, us, over 97 shapes (1 ... 128 slabs, maps of 3 x 3 to 160 x 160, every head
-// dim class) 0.39 of the time in the mean, 0.72 at most: head dim 64, 9 x 7 columns: 2 slabs of 22 x 15 23.0 -> 7.7, 32 of 25 x 11 39.8 -> 8.5, 16 of
-// 30 x 30 30.0 -> 14.7, 64 slabs of 27 x 127 (11 x 19 columns, 64/128) 897 -> 315; 2 slabs of 3 x 128 at head dim 96 24 -> 14.
+// dim class) some 0.4 of the time in the mean: head dim 64, 9 x 7 columns: 2 slabs of 22 x 15 23.0 -> 7.5, 32 of 25 x 11 39.8 -> 9.9, 16 of
+// 30 x 30 30.0 -> 14.6; 2 slabs of 3 x 128 at head dim 96 24 -> 14.  166 registers at 64/64 where one wave takes one part (176 with the sums of all
+// cases in one kernel) let a third workgroup onto a CU where chunks are one wide row: 64 slabs of 27 x 127, 11 x 19 columns 212 -> 168, 16 of 96 x 96, 13 x 13 177 -> 138.
 bool win_plan(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, WinArgs& a, int& lds) {
   if (p.g.mode != DLT_GEOM_SWA || p.g.S != 1 || p.tm.img || p.dtype != DLT_FP32 || dc.id == 4 || t.q_rot != nullptr || (p.rope.enabled && p.rope.R > 0)) return false;
   const void* const ptrs[4] = {t.q, t.k, t.v, t.out_o};
@@ -489,23 +490,24 @@ bool win_plan(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, Wi
   const int cols = 16 << a.patch_shift;
   const int64_t nx = (p.g.XLq + cols - 1) / cols, cus = dlt_device_cus();
   auto grid = [&](int ws) { return bh * ((p.g.TR + (4 >> ws) - 1) / (4 >> ws)) * nx; };
-  // A row's halo is dealt over as many waves as keeps one and a half workgroups per CU: 64 slabs of 11 x 15 (1, 2, 4 waves to a row) 9.1, 8.2 and 11.0 us,
-  // 2 of 22 x 15 9.2, 8.1, 7.8, 64 of 19 x 16 11.1, 13.2, 18.2
+  // The parts of a row's window are dealt over as many waves as keeps one and a half workgroups per CU: against lines at two and three, 60 shapes of 8 ... 128 slabs
+  // take 1.007 and 1.034 of the time.  Taking several parts costs the merges of their sums: 64 slabs of 25 x 11 10.5 -> 12.3 us, of 19 x 16 7.8 -> 8.3
   a.wave_shift = 2;
   while (a.wave_shift > a.patch_shift && 2 * grid(a.wave_shift) > 3 * cus) a.wave_shift--;
   if (((int64_t)p.g.TR + 3) / (4 >> a.wave_shift) > 65535 || nx > 65535) return false;
-  const int per_tok = win_per_token(dc.DK, dc.DV), nrows = dlt_imin(2 * p.g.WR + (4 >> a.wave_shift), p.g.TR);
+  const int nrows = dlt_imin(2 * p.g.WR + (4 >> a.wave_shift), p.g.TR);
   a.pair = p.g.XLq <= 16;
   a.cx = a.pair ? 16 : p.g.XLq <= 32 ? 32 : roundup(dlt_imin(p.g.XLk, cols + 2 * p.g.WC + 2) + 32, 8);
-  const int64_t row = (int64_t)a.cx * per_tok;
+  auto bytes = [&](int rows) { return win_lds_bytes(dc.DK, dc.DV, rows, a.cx, a.pair != 0); };
+  const int least = 1 + a.pair;   // rows of a chunk
   // chunks leave room for two workgroups per CU where so many run: one takes 1.1 times the time of two in the mean of those shapes, three 1.06 times
   int budget = grid(a.wave_shift) <= cus ? LDS_TOTAL : LDS_TOTAL / 2;
-  if (row > budget) budget = LDS_TOTAL;
-  if (row > budget) return false;
-  a.chunk_rows = dlt_imin((int)(budget / row), nrows);
-  if (a.pair) a.chunk_rows = a.chunk_rows < nrows ? dlt_imax(2, a.chunk_rows & ~1) : a.chunk_rows + (a.chunk_rows & 1);
-  lds = dlt_imax((int)(a.chunk_rows * row), win_sum_bytes(dc.DV));
-  return lds <= LDS_TOTAL;
+  if (bytes(least) > budget) budget = LDS_TOTAL;
+  if (bytes(least) > budget) return false;
+  a.chunk_rows = dlt_imax(least, nrows);
+  while (bytes(a.chunk_rows) > budget) a.chunk_rows--;
+  lds = bytes(a.chunk_rows);
+  return true;
 }
 
 int win_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, WinArgs& a, int lds, hipStream_t stream) {

@@ -5,8 +5,11 @@
 // fetches its arguments as it needs them.  Here
 //   - the halo rows of a chunk are one list of tokens, 4 x 32 rows of K and as many of V in flight at once, and a small map is one chunk;
 //   - a workgroup of 4 waves owns 16, 32 or 64 columns of 4, 2 or 1 grid rows (every halo row is staged once for all of them), or, while CUs would
-//     be idle, of fewer rows with the halo rows dealt over the waves that are left (WinArgs::wave_shift; their sums meet in LDS);
+//     be idle, of fewer rows with the parts of a row's window dealt over the waves that are left (WinArgs::wave_shift; their sums meet in LDS);
 //   - a block of 32 keys is two halo rows where a row has at most 16 tokens, one whole row up to 32, else it starts at the wave's first column.
+// A slab's bits do not depend on how many a call holds: a window's rows are summed in WinArgs::parts parts, each from nothing, which are added in order
+// whether one wave takes them one after the other or several side by side, and the blocks start at the window's first row whatever the
+// rows of a workgroup and of a chunk (in pairs of rows chunks overlap by one).
 // (figures at win_plan)
 #pragma once
 #include "attn_common.hpp"
@@ -19,7 +22,7 @@ struct WinArgs {
   int32_t H, TR, XL, WR, WC;
   int32_t dk, dv;
   int32_t patch_shift;   // 1 << patch_shift blocks of 16 queries lie side by side
-  int32_t wave_shift;    // 1 << wave_shift waves share a grid row: the blocks, times the parts its halo rows are dealt in
+  int32_t wave_shift;    // 1 << wave_shift waves share a grid row: the blocks, times the waves that its parts are dealt over
   int32_t chunk_rows, cx, pair;   // halo rows staged at once, LDS slots of a row, two rows to a block of keys
   float scale_log2;
 };
@@ -27,7 +30,34 @@ struct WinArgs {
 constexpr int win_pitch_k(int DK) { return DK * 4 + 16; }
 constexpr int win_pitch_v(int DV) { return DV * 2 + 16; }
 constexpr int win_per_token(int DK, int DV) { return win_pitch_k(DK) + win_pitch_v(DV); }
-constexpr int win_sum_bytes(int DV) { return 3 * 64 * (DV + 8); }   // DV / 16 fragments of 16 bytes, maximum and sum: per lane of up to three waves
+constexpr int win_parts(int patch_shift) { return 4 >> patch_shift; }
+constexpr int win_sum_bytes(int DV) { return 4 * 64 * (DV + 8); }   // DV / 16 fragments of 16 bytes, maximum and sum: per lane of up to four parts
+// (in pairs of rows the half block beside a lone one may lie behind the chunk)
+constexpr int win_lds_bytes(int DK, int DV, int rows, int cx, bool pair) {
+  const int chunk = rows * cx * win_per_token(DK, DV) + (pair ? 16 * win_pitch_v(DV) : 0);
+  return chunk > win_sum_bytes(DV) ? chunk : win_sum_bytes(DV);
+}
+
+// running maximum, row sum and output rows of a part
+template <int VB>
+struct WinSum {
+  float m, l;
+  f32x4 acc[VB];
+  DLT_DEV void clear() {
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int d = 0; d < VB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  template <typename F>
+  DLT_DEV void add(float m2, float l2, const F& acc2) {
+    const float m_new = fmaxf(m, m2), m_use = m_new == -INFINITY ? 0.f : m_new, f1 = fast_exp2(m - m_use), f2 = fast_exp2(m2 - m_use);
+    m = m_new;
+    l = l * f1 + l2 * f2;
+#pragma unroll
+    for (int d = 0; d < VB; d++) acc[d] = acc[d] * f1 + acc2(d) * f2;
+  }
+};
 
 // U rows per thread of one operand: loads, then conversion and LDS writes.  Reads are clamped into the chunk and the head dims, not predicated.
 template <int D, int U>
@@ -66,8 +96,9 @@ struct WinTile {
   }
 };
 
-template <int DK, int DV>
-__global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
+// MULTI: a wave takes several parts
+template <int DK, int DV, bool MULTI>
+__global__ __launch_bounds__(256, 2) void attn_win_fwd_kernel(const WinArgs a) {
   typedef bf16_t CT;
   extern __shared__ __align__(16) char smem[];
   constexpr int PK = win_pitch_k(DK), PV = win_pitch_v(DV), KC = DK / 32, VB = DV / 16;
@@ -79,7 +110,7 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
   const int r0 = blockIdx.y * rows, rlast = dlt_imin(r0 + rows, a.TR) - 1;
   const int x0 = (int)blockIdx.z * (16 << a.patch_shift), xlast = dlt_imin(x0 + (16 << a.patch_shift), a.XL) - 1;
   const int r = r0 + (wave >> a.wave_shift);
-  const int in_row = wave & ((1 << a.wave_shift) - 1), part = in_row >> a.patch_shift, parts = 1 << (a.wave_shift - a.patch_shift);
+  const int in_row = wave & ((1 << a.wave_shift) - 1), turn = in_row >> a.patch_shift;
   const int xw = x0 + 16 * (in_row & ((1 << a.patch_shift) - 1));   // first column of the wave's queries
   const bool live = r <= rlast && xw <= xlast;
 
@@ -132,15 +163,27 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
     lds_write16(sV + (ri * cx + w + t - ri * (cx - w)) * PV + i % (DV / 8) * 16, u32x4{0u, 0u, 0u, 0u});
   }
 
-  float m_run = -INFINITY, l_run = 0.f;
-  f32x4 acc[VB];
-#pragma unroll
-  for (int d = 0; d < VB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the wave's parts of the window: rows next ... stop in steps of part_rows; the first wave of a row adds them up, others keep theirs (two at most) apart
+  const int parts = win_parts(a.patch_shift), own_parts = MULTI ? parts >> (a.wave_shift - a.patch_shift) : 1, nwin = wrhi - wrlo + 1;
+  const int part_rows = a.pair ? ((nwin + 2 * parts - 1) / (2 * parts)) * 2 : (nwin + parts - 1) / parts;
+  int next = wrlo + turn * own_parts * part_rows, part_end = next + part_rows;
+  const int stop = dlt_imin(wrhi, next + own_parts * part_rows - 1);
+  WinSum<VB> cur, sum;   // of the current part; of those before it
+  cur.clear();
+  if constexpr (MULTI) sum.clear();
+  auto close = [&]() {
+    cur.l = wave_sum4(cur.l);
+    if constexpr (MULTI) {
+      if (turn == 0) sum.add(cur.m, cur.l, [&](int d) { return cur.acc[d]; });
+      else sum = cur;
+    }
+  };
   const float scale = a.scale_log2;
   const unsigned magic = (0x100000u + w - 1) / (unsigned)w;   // i / w while i * w < 2^20: a chunk holds some 1000 tokens at most
 
-  for (int kr0 = rlo; kr0 <= rhi; kr0 += a.chunk_rows) {
+  for (int kr0 = rlo, last = 0; !last; kr0 += a.chunk_rows - a.pair) {
     const int nr = dlt_imin(a.chunk_rows, rhi - kr0 + 1), total = nr * w;
+    last = kr0 + nr > rhi;
     if (kr0 != rlo) __syncthreads();
     for (int j = 0; j * U * (2048 / DK) < total; j++) {
       WinTile<DK, U> K;
@@ -164,9 +207,16 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
     }
     __syncthreads();
 
-    const int step = a.pair ? 2 : 1, ri1 = dlt_imin(nr, wrhi + 1 - kr0);
-    for (int ri = dlt_imax(0, wrlo - kr0) + part * step; ri < ri1; ri += parts * step) {
-      const bool lone = a.pair && ri + 1 == ri1;   // the block's second half is no row of this wave
+    for (; next <= stop && next < kr0 + nr; next += 1 + a.pair) {
+      const bool lone = a.pair && next == wrhi;   // the block's second half is no row of this wave
+      if (a.pair && !lone && next + 1 == kr0 + nr) break;   // the pair lies in the next chunk
+      const int ri = next - kr0;
+      if constexpr (MULTI)
+        if (next == part_end) {
+          close();
+          cur.clear();
+          part_end += part_rows;
+        }
       for (int kx = whole ? 0 : wlo; kx < whi; kx += 32) {
         const int kb = ri * cx + kx;
         u32x4 ka[2][KC], kl[2][KC], vt[VB];
@@ -200,60 +250,60 @@ __global__ __launch_bounds__(256) void attn_win_fwd_kernel(const WinArgs a) {
         }
         float mloc = fmaxf(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])), fmaxf(fmaxf(t[4], t[5]), fmaxf(t[6], t[7])));
         mloc = wave_max4(mloc);
-        const float m_new = fmaxf(m_run, mloc);
+        const float m_new = fmaxf(cur.m, mloc);
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = fast_exp2(m_run - m_use);
-        m_run = m_new;
+        const float alpha = fast_exp2(cur.m - m_use);
+        cur.m = m_new;
         float psum = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) { t[i] = fast_exp2(t[i] - m_use); psum += t[i]; }
-        l_run = l_run * alpha + psum;
+        cur.l = cur.l * alpha + psum;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
-          for (int d = 0; d < VB; d++) acc[d] *= alpha;
+          for (int d = 0; d < VB; d++) cur.acc[d] *= alpha;
         }
         const u32x4 pb = pack8<CT>(t), seen = whole || kx + 32 > whi ? vmask : all;
 #pragma unroll
         for (int d = 0; d < VB; d++) {
           vt[d] &= seen;
           if (lone) vt[d].z = vt[d].w = 0u;
-          acc[d] = Mma<CT>::mfma(vt[d], pb, acc[d]);
+          cur.acc[d] = Mma<CT>::mfma(vt[d], pb, cur.acc[d]);
         }
       }
     }
   }
-  l_run = wave_sum4(l_run);
 
-  if (parts > 1) {   // parts 1 ... of a row leave theirs in LDS, part 0 adds them in order
+  WinSum<VB>& total = MULTI ? sum : cur;
+  if (own_parts < parts) {   // the other waves' parts reach the first one through LDS
     __syncthreads();
     const int patches = 1 << a.patch_shift;
-    // slot of (part, block) of a row: the parts from 1 on, row by row
-    auto slot = [&](int pt) { return smem + (((wave >> a.wave_shift) * (parts - 1) + pt - 1) * patches + (in_row & (patches - 1))) * 64 * (DV + 8); };
-    if (part > 0) {
+    auto slot = [&](int part) { return smem + (((wave >> a.wave_shift) * (parts - own_parts) + part - own_parts) * patches + (in_row & (patches - 1))) * 64 * (DV + 8); };
+    auto put = [&](int part, const WinSum<VB>& p) {
       char* s = slot(part);
 #pragma unroll
-      for (int d = 0; d < VB; d++) lds_write16(s + (d * 64 + lane) * 16, __builtin_bit_cast(u32x4, acc[d]));
+      for (int d = 0; d < VB; d++) lds_write16(s + (d * 64 + lane) * 16, __builtin_bit_cast(u32x4, p.acc[d]));
       float* ml = reinterpret_cast<float*>(s + 64 * DV);
-      ml[lane] = m_run; ml[64 + lane] = l_run;
+      ml[lane] = p.m; ml[64 + lane] = p.l;
+    };
+    if (turn > 0) {
+      cur.l = wave_sum4(cur.l);
+      if (own_parts > 1) put(turn * own_parts, sum);
+      put((turn + 1) * own_parts - 1, cur);
     }
     __syncthreads();
-    if (part > 0) return;
-    for (int pt = 1; pt < parts; pt++) {
-      const char* s = slot(pt);
+    if (turn > 0) return;
+    close();
+    for (int part = own_parts; part < parts; part++) {
+      const char* s = slot(part);
       const float* ml = reinterpret_cast<const float*>(s + 64 * DV);
-      const float m2 = ml[lane], l2 = ml[64 + lane], m_new = fmaxf(m_run, m2), m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float f1 = fast_exp2(m_run - m_use), f2 = fast_exp2(m2 - m_use);
-      m_run = m_new;
-      l_run = l_run * f1 + l2 * f2;
-#pragma unroll
-      for (int d = 0; d < VB; d++) acc[d] = acc[d] * f1 + __builtin_bit_cast(f32x4, lds_read16(s + (d * 64 + lane) * 16)) * f2;
+      total.add(ml[lane], ml[64 + lane], [&](int d) { return __builtin_bit_cast(f32x4, lds_read16(s + (d * 64 + lane) * 16)); });
     }
-  }
+  } else close();
   if (!live || xw + n > xlast) return;
-  const float inv = l_run > 0.f ? fast_rcp(l_run) : 0.f;
+  const float inv = total.l > 0.f ? fast_rcp(total.l) : 0.f;
   float* o = reinterpret_cast<float*>(reinterpret_cast<char*>(a.o + b * a.os[0] + h * a.os[1]) + (uint32_t)((r * a.XL + xq) * (a.on * 4)));
 #pragma unroll
   for (int d = 0; d < VB; d++)
-    if (16 * d + 4 * g < a.dv) store_stream16f(o + 16 * d + 4 * g, acc[d][0] * inv, acc[d][1] * inv, acc[d][2] * inv, acc[d][3] * inv);
-  if (g == 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + (int64_t)(r * a.XL + xq) * a.ln), m_run + fast_log2(l_run));
+    if (16 * d + 4 * g < a.dv) store_stream16f(o + 16 * d + 4 * g, total.acc[d][0] * inv, total.acc[d][1] * inv, total.acc[d][2] * inv, total.acc[d][3] * inv);
+  if (g == 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + (int64_t)(r * a.XL + xq) * a.ln), total.m + fast_log2(total.l));
 }

@@ -290,7 +290,7 @@ def test_marching_fp32(th, tw, WR, WC):
         assert (lse.cpu() - lse_w).abs().max().item() <= LSE_TOL
 
 
-# fp32 windows off the marching kernel: rows of one, two and more 16-token blocks, halo rows dealt over four waves, two and one (slab counts on both
+# fp32 windows off the marching kernel: rows of one, two and more 16-token blocks, a row's parts dealt over four waves, two and one (slab counts on both
 # sides of the lines), pairs of rows with an odd one left, several chunks (last case of each kind), every head dim class and dims below it;
 # a key row of infinities or NaN changes no query that does not see it, a value row none whose block of 16 columns does not
 @pytest.mark.parametrize("BH,S,th,tw,WR,WC,dk,dv", [
@@ -325,6 +325,29 @@ def test_windows_fp32(BH, S, th, tw, WR, WC, dk, dv):
             v2 = v.clone()
             v2[:, :, at] = value
             assert torch.equal(sw.tiled_swa_fwd(q, k, v2, S, th, tw, WR, WC, scale)[:, :, apart], o[:, :, apart])
+
+
+# fp32 windows: a slab has the same bits beside any number of others, although their number decides how many waves share a grid row, how many of its parts
+# a wave takes and how many halo rows a chunk holds.  Pairs of rows, single ones and wide rows; windows of fewer rows than parts; several chunks
+@pytest.mark.parametrize("th,tw,WR,WC,dk,dv", [
+    (1, 7, 0, 3, 64, 64), (3, 5, 1, 2, 32, 32), (9, 15, 4, 3, 64, 64), (17, 16, 2, 2, 64, 128), (70, 13, 40, 5, 64, 64), (33, 9, 9, 4, 128, 128), (25, 12, 8, 8, 32, 32),
+    (10, 17, 1, 4, 64, 64), (40, 32, 18, 9, 128, 128), (13, 31, 4, 2, 40, 64), (7, 33, 2, 12, 64, 128), (5, 81, 9, 3, 64, 64)])
+def test_windows_fp32_bits_of_a_slab(th, tw, WR, WC, dk, dv):
+    sw, N = _swa(), th * tw
+    q, k, v, _ = (t.cuda() for t in orc.make_qkv(N + WR + dk, 1, 3, N, N, dk, dv, torch.float32))
+
+    def run(slabs):   # the first of them 1, 5, 60 ... times
+        args = [t[:, :1].repeat(slabs, 1, 1, 1) if slabs > 3 else t[:, :slabs] for t in (q, k, v)]
+        o, lse = sw._forward(*args, sw._shape(*args, 1, th, tw, WR, WC, 0.15), None)
+        return o, lse
+
+    o, lse = run(1)
+    for slabs in (3, 5, 30, 60, 130, 400):
+        o2, lse2 = run(slabs)
+        if slabs == 3:
+            assert torch.equal(o2[:, :1], o) and torch.equal(lse2[:, :1], lse)
+        else:
+            assert torch.equal(o2, o.expand_as(o2)) and torch.equal(lse2, lse.expand_as(lse2)), slabs
 
 
 # two stacked patches per wave (streaming kernels, more workgroups than CUs): bands without a lower patch, one band and a bit, ragged
