@@ -607,21 +607,22 @@ bool swat_eligible(const AttnProblem& p, const AttnTensors& t, bool bwd) {
   if (p.dk != p.dv || (p.dk != 32 && p.dk != 64 && (p.dk != 128 || bwd))) return false;
   if (p.g.WR < 1 || p.g.WC < 1 || p.g.WR > 2 || p.g.WC > 2) return false;
   if (p.g.S == 32 && (p.g.WR != 1 || p.g.WC != 1)) return false;
-  // Strips of four tiles, of which a ring of eight does not fit the LDS, against the flash kernels:
-  // d = 64, five rows of three columns, 60 shapes from 80 strips and rows on: forward 0.36 ... 0.9 of the time, backward 0.5 ... 1.0 (three shapes of 5 and 6
-  // columns, whose last strip is nearly empty, 1.04 ... 1.15, no longer with their forward pass): 2 slabs of 30 x 30 tiles 25.3 -> 9.6 and
-  // 52.4 -> 29.5 us, 64 of 21 x 33 206 -> 133 and 537 -> 440.  Up to 56 the window's keys over a workgroup's waves (flash_tiles_split) are
-  // faster: 2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2.
-  // The same with five columns, forward (the scalars of the backward pass do not fit beside the ring): 0.41 ... 0.98, 64 slabs of 21 x 33 225 -> 174, 4 of 40 x 12
-  // 28.9 -> 11.9.
+  // Strips of four tiles, of which a ring of eight does not fit the LDS, against the flash kernels.  The lines follow from a slab's shape alone, so that its
+  // bits do not depend on how many a call holds.
+  // d = 64, five rows of three columns, 190 shapes of 1 ... 256 slabs: forward 0.28 ... 0.90 of the time of the chunked kernels, backward 0.38 ... 1.04 where two
+  // strips hold seven columns or more (5 and 6 columns, whose second strip is mostly empty, up to 1.24 there and left to the others): 2 slabs of 30 x 30 tiles
+  // 25.3 -> 10 and 52.4 -> 31 us, 64 of 21 x 33 206 -> 136 and 537 -> 445.  On up to 20 tiles or so the window's keys over a workgroup's waves
+  // (flash_tiles_split) take 0.9 of the forward and 0.65 of the backward time (2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2).
+  // The same with five columns, forward (the scalars of the backward pass do not fit beside the ring): 0.41 ... 0.98, 64 slabs of 21 x 33 225 -> 177, 4 of 40 x 12
+  // 28.9 -> 12.
   // d = 128, 3 x 3 tiles, forward: 0.40 ... 0.98 where strips are three quarters full (2 slabs of 30 x 30 23.8 -> 13.4, 64 of 30 x 10 174 -> 106), five columns
   // up to 1.10; the backward kernels take 0.95 ... 1.5 of the time and stay there.
   if (p.dk == 128 && (p.g.S != 16 || p.g.WR != 1)) return false;
   if (p.dk == 128 || (p.g.WR == 2 && p.dk == 64)) {
-    const int64_t sb = Swat<64, 1, 1, 2>::SB, strips = (p.g.TC + sb - 1) / sb;
+    const int sb = Swat<64, 1, 1, 2>::SB, strips = (p.g.TC + sb - 1) / sb;
     if (p.g.WC == 2 && (p.dk == 128 || bwd)) return false;
     if (p.g.TC < sb || (p.dk == 128 && 4 * p.g.TC < 3 * sb * strips)) return false;
-    if (4 * (int64_t)p.B * p.H * strips * p.g.TR < dlt_device_cus()) return false;
+    if (bwd && strips == 2 && p.g.TC <= 6) return false;
   }
   if (!swat_rows_ok(p, t.q, t.qs) || !swat_rows_ok(p, t.k, t.ks) || !swat_rows_ok(p, t.v, t.vs)) return false;
   if (!bwd) return swat_rows_ok(p, t.out_o, t.os);
@@ -817,6 +818,8 @@ int64_t flash_part_kv(const AttnProblem& p, const FlashPlan& f) { return f.n > 1
 
 // Windows over tiles of 16 k tokens off the marching kernels: whether the kernels of flash_split_kernel.hpp run, which take 16 own tokens to a
 // workgroup and deal the window's keys over its waves, so that a call of few tiles is not a handful of workgroups with 64 keys after the other.
+// This is the one choice for tiles that looks at the number of slabs, and with it their bits depend on it: by the shape alone it would cost calls of
+// one to eight slabs up to 4 times, or calls of 64 and more up to 3 times the time (130 shapes; the split kernels take 0.45 of the chunked time on one slab, 1.8 on 32).
 // Tiles of 64 k tokens stay on the asynchronously staged kernels (0.67 ... 1.1 of whose time it takes up to 256 blocks), where a slab's bits do not
 // depend on the call.  A workgroup's time is a0 + a1 + a2 per key, one per CU and a3 of them at once, that of the chunked kernels
 // b0 + b1 + b2 per 64 keys, b3 workgroups per CU at once; fitted to 1717 shapes (us), rms 7 and 13 %, so 15 % are asked for.  Chosen that way a forward pass takes

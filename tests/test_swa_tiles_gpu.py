@@ -227,12 +227,13 @@ def test_infinite_and_nan_tiles_stay_in_their_windows(d, th, tw, B, which):
                 assert torch.equal(g[:, :, far > n], w[:, :, far > n]), (r, c, value)
 
 
-# few tiles of 16 k tokens: 16 own tokens to a workgroup, the window's keys dealt over its waves; one slab, and as many as leave that rule.  Odd and even
+# few tiles of 16 k tokens: 16 own tokens to a workgroup, the window's keys dealt over its waves; one slab, and as many as leave that rule (whose bits are
+# others, but at five tile rows or columns where strips of four take the pass).  Odd and even
 # numbers of 16-token runs, runs of one, windows of one tile and beyond the grid, every class and dims below it.  The image layout has the same bits.
 # A tile of infinities and NaN is not read for the tiles that do not see it
 @pytest.mark.parametrize("th,tw,S,WR,WC,dk,dv,many", [
     (7, 5, 16, 2, 2, 64, 64, 40), (4, 10, 16, 2, 1, 64, 64, 60), (5, 9, 16, 0, 0, 64, 64, 90), (3, 7, 16, 1, 1, 128, 128, 40), (1, 9, 16, 4, 3, 64, 128, 60),
-    (9, 1, 16, 3, 2, 32, 32, 90), (3, 4, 48, 1, 1, 64, 64, 40), (2, 5, 80, 1, 0, 32, 32, 40), (4, 3, 16, 2, 2, 40, 64, 90), (3, 5, 32, 2, 1, 80, 80, 40)])
+    (9, 1, 16, 3, 2, 32, 32, 90), (7, 5, 16, 3, 2, 64, 64, 40), (4, 10, 16, 2, 3, 64, 64, 60), (3, 4, 48, 1, 1, 64, 64, 40), (2, 5, 80, 1, 0, 32, 32, 40), (4, 3, 16, 2, 2, 40, 64, 90), (3, 5, 32, 2, 1, 80, 80, 40)])
 def test_few_tiles_over_waves(th, tw, S, WR, WC, dk, dv, many):
     sw = _swa()
     N, scale = th * tw * S, 1 / math.sqrt(dk)
@@ -291,7 +292,7 @@ def test_tiles_of_64_tokens(th, tw, tile, WR, WC, dk, dv, many):
 
 
 # windows of 5 x 3 tiles at d = 64 and, forward, 3 x 3 at d = 128 and 5 x 5 at d = 64, on strips of four tiles: grids below the window, rows below a band's ring, strips whole,
-# ragged and with one tile, the fewest strips of the rule; image layout with the same bits; infinite and NaN tiles stay with the queries that see them
+# ragged and with one tile; image layout with the same bits; infinite and NaN tiles stay with the queries that see them
 @pytest.mark.parametrize("WR,WC,d", [(2, 1, 64), (1, 1, 128), (2, 2, 64)])
 @pytest.mark.parametrize("th,tw,B,dtype", [(1, 4, 80, torch.float16), (2, 5, 20, torch.bfloat16), (4, 8, 8, torch.float16), (11, 9, 2, torch.bfloat16), (7, 13, 9, torch.float16),
                                           (5, 4, 200, torch.bfloat16)])
@@ -362,3 +363,22 @@ def test_infinite_values_reach_the_queries_that_see_them(th, tw, S, WR, WC, d, s
                 t[:, :, rows, 3], t[:, :, rows, d - 1] = inf, -inf
             _, _, dk2, dv2 = run(v, bad)
             assert torch.equal(dv2, want) and torch.equal(dk2[:, :, ~sees], dk[:, :, ~sees]), (r, c)
+
+
+# ... where a slab has the same bits alone and beside any number of others (backward: not two strips of which the second is mostly empty)
+@pytest.mark.parametrize("th,tw,WR,WC,d,bwd", [
+    (3, 4, 2, 1, 64, True), (1, 7, 2, 1, 64, True), (14, 9, 2, 1, 64, True), (5, 6, 2, 1, 64, False), (7, 5, 2, 2, 64, False), (2, 4, 2, 2, 64, False), (6, 4, 1, 1, 128, False),
+    (5, 7, 1, 1, 128, False), (1, 12, 1, 1, 128, False)])
+def test_strips_of_four_tiles_bits_of_a_slab(th, tw, WR, WC, d, bwd):
+    sw, S = _swa(), 16
+    N = th * tw * S
+    ops = [t.cuda() for t in orc.make_qkv(N + d, 1, 1, N, N, d, d, torch.bfloat16)]
+
+    def run(slabs):
+        leaves = [t.repeat(slabs, 1, 1, 1).requires_grad_(True) for t in ops[:3]]
+        o = sw.TiledSwa.apply(*leaves, S, th, tw, WR, WC, 0.125)
+        return (o.detach(),) + (torch.autograd.grad(o, leaves, ops[3].repeat(slabs, 1, 1, 1)) if bwd else ())
+
+    one = run(1)
+    for slabs in (2, 7, 40, 300):
+        assert all(torch.equal(a, b.expand_as(a)) for a, b in zip(run(slabs), one)), slabs
