@@ -288,26 +288,26 @@ int swa_bwd(const char* who, bool narrow, const void* q, const int64_t* q_stride
 }
 }  // namespace
 
-#define DLT_SWA_FWD_ARGS                                                                                    \
+#define DLT_FWD_ARGS                                                                                    \
   const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4], const void *v,      \
       const int64_t v_strides[4], void *o, const int64_t o_strides[4], float *lse2, const int64_t lse_strides[3]
-#define DLT_SWA_BWD_ARGS                                                                                    \
+#define DLT_BWD_ARGS                                                                                    \
   const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4], const void *v,      \
       const int64_t v_strides[4], const void *o, const int64_t o_strides[4], const void *d_o,               \
       const int64_t do_strides[4], const float *lse2, float *delta, const int64_t lse_strides[3], void *dq, \
       const int64_t dq_strides[4], void *dk, const int64_t dk_strides[4], void *dv, const int64_t dv_strides[4]
 
-extern "C" int dlt_swa_fwd(DLT_SWA_FWD_ARGS, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
+extern "C" int dlt_swa_fwd(DLT_FWD_ARGS, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
   return swa_fwd("swa_fwd", false, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, rope, stream);
 }
-extern "C" int dlt_swa_fwd_narrow(DLT_SWA_FWD_ARGS, const dlt_swa_shape_t* shape, void* stream) {
+extern "C" int dlt_swa_fwd_narrow(DLT_FWD_ARGS, const dlt_swa_shape_t* shape, void* stream) {
   return swa_fwd("swa_fwd_narrow", true, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, nullptr, stream);
 }
-extern "C" int dlt_swa_bwd(DLT_SWA_BWD_ARGS, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
+extern "C" int dlt_swa_bwd(DLT_BWD_ARGS, const dlt_swa_shape_t* shape, const dlt_rope_t* rope, void* stream) {
   return swa_bwd("swa_bwd", false, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq, dq_strides,
                  dk, dk_strides, dv, dv_strides, shape, rope, stream);
 }
-extern "C" int dlt_swa_bwd_narrow(DLT_SWA_BWD_ARGS, const dlt_swa_shape_t* shape, void* stream) {
+extern "C" int dlt_swa_bwd_narrow(DLT_BWD_ARGS, const dlt_swa_shape_t* shape, void* stream) {
   return swa_bwd("swa_bwd_narrow", true, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq,
                  dq_strides, dk, dk_strides, dv, dv_strides, shape, nullptr, stream);
 }
@@ -422,65 +422,54 @@ extern "C" int dlt_flash_workspace(const dlt_flash_shape_t* shape, int backward,
   return DLT_OK;
 }
 
-// `ws` of at least dlt_flash_workspace bytes, or none: NULL comes back where the call needs none or has none
-static int flash_ws(const char* who, const AttnProblem& p, bool backward, void* ws, int64_t ws_bytes, float*& part) {
-  part = nullptr;
-  if (ws == nullptr) return DLT_OK;
+// `ws` of at least dlt_flash_workspace bytes, or none.  Shares (AttnTensors::shares) are taken where the call has what it needs for them
+static int flash_ws(const char* who, const AttnProblem& p, bool backward, void* ws, int64_t ws_bytes, AttnTensors& t) {
+  t.part = nullptr;
   const int64_t need = 4 * dlt_attn_part_floats(p, backward);
+  t.shares = ws != nullptr || need == 0;
+  if (ws == nullptr) return DLT_OK;
   DLT_REQUIRE((uintptr_t)ws % 16 == 0, "%s: workspace is not 16-byte aligned", who);
   DLT_REQUIRE(ws_bytes >= need, "%s: workspace of %lld bytes, %lld needed", who, (long long)ws_bytes, (long long)need);
-  if (need > 0) part = (float*)ws;
+  if (need > 0) t.part = (float*)ws;
   return DLT_OK;
 }
 
-extern "C" int dlt_flash_fwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                                const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
-                                float* lse2, const int64_t lse_strides[3],
-                                const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream) {
+// `with_ws`: the entry points that take a workspace
+static int flash_fwd(DLT_FWD_ARGS, const dlt_flash_shape_t* shape, bool with_ws, void* ws, int64_t ws_bytes, void* stream) {
   AttnProblem p;
   int rc = flash_problem("flash_fwd", shape, p);
   if (rc != DLT_OK) return rc;
   AttnTensors t;
   rc = fill_fwd("flash_fwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides);
-  if (rc == DLT_OK) rc = flash_ws("flash_fwd", p, false, ws, ws_bytes, t.part);
+  if (rc == DLT_OK && with_ws) rc = flash_ws("flash_fwd", p, false, ws, ws_bytes, t);
   if (rc != DLT_OK) return rc;
   return dlt_attn_forward(p, t, (hipStream_t)stream);
 }
-
-extern "C" int dlt_flash_fwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                             const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],
-                             float* lse2, const int64_t lse_strides[3],
-                             const dlt_flash_shape_t* shape, void* stream) {
-  return dlt_flash_fwd_ws(q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, nullptr, 0, stream);
-}
-
-extern "C" int dlt_flash_bwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                                const void* v, const int64_t v_strides[4], const void* o, const int64_t o_strides[4],
-                                const void* d_o, const int64_t do_strides[4],
-                                const float* lse2, float* delta, const int64_t lse_strides[3],
-                                void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
-                                void* dv, const int64_t dv_strides[4],
-                                const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream) {
+static int flash_bwd(DLT_BWD_ARGS, const dlt_flash_shape_t* shape, bool with_ws, void* ws, int64_t ws_bytes, void* stream) {
   AttnProblem p;
   int rc = flash_problem("flash_bwd", shape, p);
   if (rc != DLT_OK) return rc;
   AttnTensors t;
   rc = fill_bwd("flash_bwd", t, q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta,
                 lse_strides, dq, dq_strides, dk, dk_strides, dv, dv_strides);
-  if (rc == DLT_OK) rc = flash_ws("flash_bwd", p, true, ws, ws_bytes, t.part);
+  if (rc == DLT_OK && with_ws) rc = flash_ws("flash_bwd", p, true, ws, ws_bytes, t);
   if (rc != DLT_OK) return rc;
   return dlt_attn_backward(p, t, (hipStream_t)stream);
 }
 
-extern "C" int dlt_flash_bwd(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
-                             const void* v, const int64_t v_strides[4], const void* o, const int64_t o_strides[4],
-                             const void* d_o, const int64_t do_strides[4],
-                             const float* lse2, float* delta, const int64_t lse_strides[3],
-                             void* dq, const int64_t dq_strides[4], void* dk, const int64_t dk_strides[4],
-                             void* dv, const int64_t dv_strides[4],
-                             const dlt_flash_shape_t* shape, void* stream) {
-  return dlt_flash_bwd_ws(q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq, dq_strides, dk,
-                          dk_strides, dv, dv_strides, shape, nullptr, 0, stream);
+extern "C" int dlt_flash_fwd_ws(DLT_FWD_ARGS, const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream) {
+  return flash_fwd(q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, true, ws, ws_bytes, stream);
+}
+extern "C" int dlt_flash_fwd(DLT_FWD_ARGS, const dlt_flash_shape_t* shape, void* stream) {
+  return flash_fwd(q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse2, lse_strides, shape, false, nullptr, 0, stream);
+}
+extern "C" int dlt_flash_bwd_ws(DLT_BWD_ARGS, const dlt_flash_shape_t* shape, void* ws, int64_t ws_bytes, void* stream) {
+  return flash_bwd(q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq, dq_strides, dk, dk_strides,
+                   dv, dv_strides, shape, true, ws, ws_bytes, stream);
+}
+extern "C" int dlt_flash_bwd(DLT_BWD_ARGS, const dlt_flash_shape_t* shape, void* stream) {
+  return flash_bwd(q, q_strides, k, k_strides, v, v_strides, o, o_strides, d_o, do_strides, lse2, delta, lse_strides, dq, dq_strides, dk, dk_strides,
+                   dv, dv_strides, shape, false, nullptr, 0, stream);
 }
 
 // ---- image-layout entry points ------------------------------------------------------------------

@@ -776,32 +776,51 @@ int flash_pick(int pass, const DimClass& dc, int dims, int64_t bh, int own, int 
 // slab's shape alone (see above), as other / (a + b own) up to 8: the lines were fitted to 2100 shapes of 4 ... 128 slabs (n = 2, 3, 4, 6, 8), a loss
 // counted eightfold.  Inside them, not split -> split, geometric mean of the pass by slabs (4, 8, 16, 32, 64, 128): forward 1.7 ... 2.2,
 // 1.55 ... 2.0, 1.33 ... 1.8, 1.22 ... 1.6, 1.2, 1.15; both backward passes together 1.4 ... 1.8 down to 1.05 ... 1.3.  Shorter other sides and
-// longer own ones lose more to the sums than idle CUs cost (128 slabs of 734 x 3321, 64/64: 98 -> 144 us with n = 4).  Over 1500 drawn
-// calls of 4 ... 128 slabs the slowest lose 10 % (128 of 802 x 4159, 80/80: 221 -> 242; 64 of 2011 x 400, 128/128, both directions: 170 -> 190).
-struct FlashPlan { int kind, n, len; };
-FlashPlan flash_plan(int pass, const DimClass& dc, int dims, int64_t bh, int own, int other, bool causal, bool may_split) {
+// longer own ones lose more to the sums than idle CUs cost (128 slabs of 734 x 3321, 64/64: 98 -> 144 us with n = 4).  The slowest against no
+// shares: forward 1.26 on 128 slabs (53 x 3868, 64/128: 33 -> 42 us; one share of a handful of tokens is half a workgroup), backward 1.14 (30 x 1149, 128/128).
+//
+// Once workgroups fill the chip without it, partial results only cost: one workgroup then takes all shares of its own block (FlashShare::walk, the same
+// bits), from 1.5 workgroups of 64 own tokens per CU on, 0.75 where they are all there are.  Over 110 shapes of 4 ... 256 slabs, walked against split
+// in the mean below and above that line: up to 64 own tokens forward 1.27 and 0.9, dQ 1.04 and 0.89, dK/dV 1.08 and 0.87; more own tokens 1.03 and 0.93,
+// 0.99 and 0.95, 0.95 and 0.9.  Long own sides of forward and dQ stay split (128/128 forward beyond 512 queries 1.03, dQ 1.04): their shares are few and
+// long.  All of those shapes against no shares, forward and backward, split alone -> so: 128 slabs 1.01 and 1.00 -> 0.99 and 0.96, 256 slabs 1.01 and 1.01 -> 0.96
+// and 0.93; the slowest of 256 slabs 1.30 -> 1.14 (995 x 5280, 128/128).  A pass whose partial results would take more than half of
+// DLT_FLASH_WORKSPACE_MAX is walked as well, whatever its sides (128 MiB; at 64 MiB 32 slabs of 8943 x 294, 128/128, were, backward 211 -> 252 us).
+constexpr int64_t FLASH_PART_MAX = (int64_t)DLT_FLASH_WORKSPACE_MAX / 4;   // floats
+struct FlashShares { int n, len; bool walk; };
+FlashShares flash_shares(int pass, const DimClass& dc, int dk, int dv, int64_t bh, int own, int other) {
+  // other side of at least `least` tokens and `times` the own one; a, 4 b
+  static const struct { int least, times, a, b4; } RULE[3][4] = {   // by pass; 64/64, 64/128, 128/128 with up to 192 dims in all, 128/128
+      {{3000, 3, 150, 6}, {3000, 3, 500, 5}, {2500, 3, 150, 6}, {1200, 3, 150, 9}},
+      {{1600, 1, 350, 4}, {600, 1, 150, 4}, {1600, 1, 150, 4}, {600, 4, 150, 8}},
+      {{2500, 1, 150, 6}, {1600, 4, 250, 4}, {2000, 1, 500, 4}, {1200, 4, 150, 8}}};
+  const auto& r = RULE[pass][dc.id == 0 ? 0 : dc.id == 2 ? 1 : dk + dv <= 192 ? 2 : 3];
+  if (other < r.least || other < (int64_t)r.times * own) return {1, other, false};
+  int n = dlt_imin((int)(4 * (int64_t)other / (4 * r.a + (int64_t)r.b4 * own)), FLASH_SHARES_MAX);
+  if (n <= 1) return {1, other, false};
+  const int len = roundup((other + n - 1) / n, 128);
+  n = (other + len - 1) / len;
+  const int64_t row = pass == 0 ? dv + 2 : pass == 1 ? dk : dk + dv;
+  const int most = pass == 2 ? 1 << 30 : (pass == 0 ? dk + dv <= 192 : dc.id != 1) ? 1024 : 512;
+  const bool full = own <= most && 4 * bh * ((own + 63) / 64) >= (own <= 64 ? 3 : 6) * (int64_t)dlt_device_cus();
+  const bool walk = full || bh * n * own * row > FLASH_PART_MAX / 2;
+  return {n, len, walk};
+}
+
+struct FlashPlan { int kind, n, len; bool walk; };
+FlashPlan flash_plan(int pass, const DimClass& dc, int dk, int dv, int64_t bh, int own, int other, bool causal, bool may_split) {
   if (may_split && !causal) {
-    // other side of at least `least` tokens and `times` the own one; a, 4 b
-    static const struct { int least, times, a, b4; } RULE[3][4] = {   // by pass; 64/64, 64/128, 128/128 with up to 192 dims in all, 128/128
-        {{3000, 3, 150, 6}, {3000, 3, 500, 5}, {2500, 3, 150, 6}, {1200, 3, 150, 9}},
-        {{1600, 1, 350, 4}, {600, 1, 150, 4}, {1600, 1, 150, 4}, {600, 4, 150, 8}},
-        {{2500, 1, 150, 6}, {1600, 4, 250, 4}, {2000, 1, 500, 4}, {1200, 4, 150, 8}}};
-    const auto& r = RULE[pass][dc.id == 0 ? 0 : dc.id == 2 ? 1 : dims <= 192 ? 2 : 3];
-    int n = other < r.least || other < (int64_t)r.times * own ? 1 : (int)(4 * (int64_t)other / (4 * r.a + (int64_t)r.b4 * own));
-    n = dlt_imin(n, 8);
-    if (n > 1) {
-      const int len = roundup((other + n - 1) / n, 128);
-      n = (other + len - 1) / len;
-      // one own block per wave or two (the same bits): one while its workgroups are few.  Forward at 64/64, 8 waves of one against 4 of two: 0.92 of the
-      // time below a workgroup of 128 queries per four CUs, 0.96 up to one per CU, 1.01 to two, 1.05 beyond; at 64/128 and 128/128 always
-      // 8 waves (their two-block kernel passes 128 keys at a time).  Backward, whole pass, one against two: 0.82 ... 0.89 below 64 workgroups of
-      // 64, 0.87 ... 0.96 to one per CU, 0.97 ... 1.0 to two, 0.95 ... 1.09 beyond
-      const int64_t cus = dlt_device_cus();
-      const bool slim = pass == 0 ? dc.id != 0 || bh * n * ((own + 127) / 128) <= cus : bh * n * ((own + 63) / 64) <= 2 * cus;
-      if (n > 1) return {slim ? FLASH_SLIM : FLASH_CHUNKED, n, len};
-    }
+    const FlashShares s = flash_shares(pass, dc, dk, dv, bh, own, other);
+    // one own block per wave or two (the same bits): one while its workgroups are few.  Forward at 64/64, 8 waves of one against 4 of two: 0.92 of the
+    // time below a workgroup of 128 queries per four CUs, 0.96 up to one per CU, 1.01 to two, 1.05 beyond; at 64/128 and 128/128 always
+    // 8 waves (their two-block kernel passes 128 keys at a time).  Backward, whole pass, one against two: 0.82 ... 0.89 below 64 workgroups of
+    // 64, 0.87 ... 0.96 to one per CU, 0.97 ... 1.0 to two, 0.95 ... 1.09 beyond; up to 64 own tokens always, which the others' waves would idle beside
+    // (and forward on 4 waves: 47 shapes of 128 and 256 slabs forward 0.98 of the time, backward 0.97)
+    const int64_t cus = dlt_device_cus();
+    const bool slim = own <= 64 || (pass == 0 ? dc.id != 0 || bh * s.n * ((own + 127) / 128) <= cus : bh * s.n * ((own + 63) / 64) <= 2 * cus);
+    if (s.n > 1) return {slim ? FLASH_SLIM : FLASH_CHUNKED, s.n, s.len, s.walk};
   }
-  return {flash_pick(pass, dc, dims, bh, own, other, causal), 1, other};
+  return {flash_pick(pass, dc, dk + dv, bh, own, other, causal), 1, other, false};
 }
 // the asynchronously staged kernels know shares
 // (partial rows are counted in 32 bits: beyond that nothing is split)
@@ -809,12 +828,10 @@ bool flash_may_split(const AttnProblem& p, const DimClass& dc) {
   const int64_t rows = (int64_t)p.B * p.H * dlt_imax(p.g.XLq, p.g.XLk);
   return p.g.mode == DLT_GEOM_DENSE && dc.id <= 2 && p.dtype != DLT_FP32 && p.dk % 8 == 0 && p.dv % 8 == 0 && rows <= 0x7fffffff / 16 && dlt_flash_async();
 }
-// floats of partial results a pass needs (0: not split)
-int64_t flash_part_fwd(const AttnProblem& p, const FlashPlan& f) {
-  return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLq * (p.dv + 2) : 0;
-}
-int64_t flash_part_q(const AttnProblem& p, const FlashPlan& f) { return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLq * p.dk : 0; }
-int64_t flash_part_kv(const AttnProblem& p, const FlashPlan& f) { return f.n > 1 ? (int64_t)p.B * p.H * f.n * p.g.XLk * (p.dk + p.dv) : 0; }
+// floats of partial results that a pass leaves for a second launch
+int64_t flash_part_fwd(const AttnProblem& p, int n, bool walk) { return n > 1 && !walk ? (int64_t)p.B * p.H * n * p.g.XLq * (p.dv + 2) : 0; }
+int64_t flash_part_q(const AttnProblem& p, int n, bool walk) { return n > 1 && !walk ? (int64_t)p.B * p.H * n * p.g.XLq * p.dk : 0; }
+int64_t flash_part_kv(const AttnProblem& p, int n, bool walk) { return n > 1 && !walk ? (int64_t)p.B * p.H * n * p.g.XLk * (p.dk + p.dv) : 0; }
 
 // Windows over tiles of 16 k tokens off the marching kernels: whether the kernels of flash_split_kernel.hpp run, which take 16 own tokens to a
 // workgroup and deal the window's keys over its waves, so that a call of few tiles is not a handful of workgroups with 64 keys after the other.
@@ -863,10 +880,10 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
   a.scale_log2 = p.sm_scale * 1.4426950408889634f;
   const int64_t grid = (int64_t)p.B * p.H * p.g.TR * a.nblk;
   if (grid > 0x7fffffff) return dlt_set_error(DLT_ERR_UNSUPPORTED, "flash forward: grid too large");
-  a.share = {t.part, 1, a.Lk};
+  a.share = {t.part, 1, a.Lk, 0};
   int np = FLASH_CHUNKED;
   if (p.g.mode != DLT_GEOM_SWA) {
-    const FlashPlan f = flash_plan(0, dc, p.dk + p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0, t.part != nullptr && flash_may_split(p, dc));
+    const FlashPlan f = flash_plan(0, dc, p.dk, p.dv, (int64_t)p.B * p.H, a.Lq, a.Lk, a.causal != 0, t.shares && flash_may_split(p, dc));
     np = f.kind;
     // One own block per wave, with the bits of the kernel it stands for: 8 waves (workgroups of 128 queries) or, while workgroups of 64 all
     // run at once, one per CU (two under a mask, where the work is uneven), 4 waves.  Slim workgroups, 8 waves -> 4: 0.83 ... 0.89 of
@@ -876,10 +893,10 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
     // 64/128: 151 -> 78 us)
     const int64_t cus = dlt_device_cus(), nbh = (int64_t)p.B * p.H * f.n, most = a.causal ? 2 * cus : cus;
     const bool long_chunks = np == FLASH_CHUNKED && dc.DV == 128;
-    const bool four = nbh * ((a.Lq + 63) / 64) <= (long_chunks ? cus : most);
+    const bool four = (f.n > 1 && a.Lq <= 64) || nbh * ((a.Lq + 63) / 64) <= (long_chunks ? cus : most);
     a.chunk = long_chunks ? 128 : 64;
     a.slim = np == FLASH_SLIM ? (four ? 4 : 8) : long_chunks ? (four ? 4 : nbh * ((a.Lq + 127) / 128) <= most ? 8 : 0) : 0;
-    a.share.n = f.n; a.share.len = f.len;
+    a.share.n = f.n; a.share.len = f.len; a.share.walk = f.walk;
   }
   if (flash_tiles_split(p, dc, false)) {
     np = FLASH_SPLIT1;
@@ -905,7 +922,7 @@ int flash_forward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc
     default: DLT_FLASH_FWD(64_128);
   }
 #undef DLT_FLASH_FWD
-  return rc == DLT_OK && a.share.n > 1 ? dlt_flash_share_fwd(a, p.dtype, stream) : rc;
+  return rc == DLT_OK && a.share.n > 1 && !a.share.walk ? dlt_flash_share_fwd(a, p.dtype, stream) : rc;
 }
 
 int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, hipStream_t stream) {
@@ -963,20 +980,20 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
   // each pass streams its other side through LDS or splits it over the waves, whichever suits its own shape
   const int64_t nbh = (int64_t)p.B * p.H;
   const bool seq = p.g.mode != DLT_GEOM_SWA;
-  FlashPlan fq = {FLASH_CHUNKED, 1, a.Lk}, fkv = {FLASH_CHUNKED, 1, a.Lq};
+  FlashPlan fq = {FLASH_CHUNKED, 1, a.Lk, false}, fkv = {FLASH_CHUNKED, 1, a.Lq, false};
   if (seq) {
-    bool may_split = t.part != nullptr && flash_may_split(p, dc);
-    fq = flash_plan(1, dc, p.dk + p.dv, nbh, a.Lq, a.Lk, a.causal != 0, may_split);
+    bool may_split = t.shares && flash_may_split(p, dc);
+    fq = flash_plan(1, dc, p.dk, p.dv, nbh, a.Lq, a.Lk, a.causal != 0, may_split);
     may_split = may_split && dlt_flash_scalars_fit(a);   // else dK/dV stays on the register-staged kernel
-    fkv = flash_plan(2, dc, p.dk + p.dv, nbh, a.Lk, a.Lq, a.causal != 0, may_split);
+    fkv = flash_plan(2, dc, p.dk, p.dv, nbh, a.Lk, a.Lq, a.causal != 0, may_split);
   }
   if (flash_tiles_split(p, dc, true)) {
     fq.kind = fkv.kind = FLASH_SPLIT1;
     a.Lq = a.Lk = p.g.TR * p.g.XLq;
   }
   const int np_q = fq.kind, np_kv = fkv.kind;
-  a.share_q = {t.part, fq.n, fq.len};
-  a.share_kv = {t.part + flash_part_q(p, fq), fkv.n, fkv.len};
+  a.share_q = {t.part, fq.n, fq.len, fq.walk};
+  a.share_kv = {t.part + flash_part_q(p, fq.n, fq.walk), fkv.n, fkv.len, fkv.walk};
   a.slim = np_kv == FLASH_SLIM;
   // dQ with one workgroup of 128 queries per CU: 8 waves of one block (16 slabs of 2048 x 2048: 64/64 36.6 -> 34.6 us, 64/128 43.8 -> 41.0,
   // 128/128 58.0 -> 54.2; from two workgroups per CU on slower, 32 slabs 54.8 -> 56.0, 70.4 -> 70.5, 94.9 -> 108.5)
@@ -994,8 +1011,8 @@ int flash_backward(const AttnProblem& p, const AttnTensors& t, const DimClass& d
     case 3: DLT_FLASH_PASS(32_32);
     default: DLT_FLASH_PASS(64_128);
   }
-  if (rc == DLT_OK && fq.n > 1) rc = dlt_flash_share_bwd_q(a, p.dtype, stream);
-  if (rc == DLT_OK && fkv.n > 1) rc = dlt_flash_share_bwd_kv(a, p.dtype, stream);
+  if (rc == DLT_OK && fq.n > 1 && !fq.walk) rc = dlt_flash_share_bwd_q(a, p.dtype, stream);
+  if (rc == DLT_OK && fkv.n > 1 && !fkv.walk) rc = dlt_flash_share_bwd_kv(a, p.dtype, stream);
   return rc;
 #undef DLT_FLASH_PASS
 }
@@ -1082,11 +1099,13 @@ int dlt_attn_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t str
 
 int64_t dlt_attn_part_floats(const AttnProblem& p, bool backward) {
   DimClass dc;
-  if (p.g.mode != DLT_GEOM_DENSE || p.dk > 128 || p.dv > 128 || pick_dims(p, dc) != DLT_OK || !flash_may_split(p, dc)) return 0;
+  if (p.g.mode != DLT_GEOM_DENSE || p.dk > 128 || p.dv > 128 || pick_dims(p, dc) != DLT_OK) return 0;
+  if (!flash_may_split(p, dc)) return 0;
   const int64_t bh = (int64_t)p.B * p.H;
-  if (!backward) return flash_part_fwd(p, flash_plan(0, dc, p.dk + p.dv, bh, p.g.XLq, p.g.XLk, false, true));
-  return flash_part_q(p, flash_plan(1, dc, p.dk + p.dv, bh, p.g.XLq, p.g.XLk, false, true)) +
-         flash_part_kv(p, flash_plan(2, dc, p.dk + p.dv, bh, p.g.XLk, p.g.XLq, false, true));
+  const FlashShares f = flash_shares(backward ? 1 : 0, dc, p.dk, p.dv, bh, p.g.XLq, p.g.XLk);
+  if (!backward) return flash_part_fwd(p, f.n, f.walk);
+  const FlashShares kv = flash_shares(2, dc, p.dk, p.dv, bh, p.g.XLk, p.g.XLq);
+  return flash_part_q(p, f.n, f.walk) + flash_part_kv(p, kv.n, kv.walk);
 }
 
 int dlt_attn_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream) {

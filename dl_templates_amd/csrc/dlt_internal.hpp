@@ -69,7 +69,8 @@ struct AttnTensors {
   void *q_rot, *k_rot;  // forward: optional outputs, the rotated q and k (NULL: not wanted)
   float* lse;        // written by forward, read by backward
   float* delta;      // scratch written by the backward pre-pass
-  float* part;       // flash: partial results of a split streamed side (dlt_flash_workspace), or NULL: not split
+  float* part;       // flash: partial results of a split streamed side (dlt_flash_workspace); NULL where none are needed
+  bool shares;       // flash: the streamed side may be taken in shares
   // element strides [B, H, N, D]; entry 4 is only used with an image token map (AttnProblem::tm):
   // then [2] is the stride of a pixel column and [4] the stride of a pixel row
   int64_t qs[5], ks[5], vs[5], os[5], dos[5], dqs[5], dks[5], dvs[5], ls[3];

@@ -216,6 +216,9 @@ constexpr int flashd_occ(int nw) { return nw == 4 ? 2 : 1; }   // waves per SIMD
 // dQ at 64/128: with two buffers and 168 registers three workgroups share a CU (with three buffers two do; 16 + 16 slabs of 4096 x 8192:
 // 1441 -> 1433 us for the whole step); at 64/64 three do with three buffers
 constexpr int flashd_dq_occ(int dk, int dv, int nw) { return nw == 4 && dk + dv <= 192 ? 3 : flashd_occ(nw); }
+// Sums of shares beside the current ones (WALK) take 8 waves of one block past 128 registers, which would leave one workgroup on a CU: at 64/128 20 of them are
+// spilled, between shares only (821 x 3276 on 256 slabs 1.16 -> 1.05 of the time without shares); at 128/128 72 would be (512 slabs of 128 x 4096 219 -> 262 us)
+constexpr int flashd_fwd_occ(int dk, int dv, int nw, bool walk) { return walk && nw == 8 && dk + dv <= 192 ? 4 : flashd_occ(nw); }
 constexpr int flashd_dq_bufs(int dk, int dv, int np, int nw) { return nw == 4 && dk + dv > 128 ? 2 : flashd_bufs(dk, dv, np, nw); }
 
 template <int DK, int DV, int CK>
@@ -274,7 +277,7 @@ constexpr int flashd_dims(int d, int pad) { return pad >= 2 && d == 128 ? 96 : d
 constexpr int flashd_blocks(int d, int pad) { return pad == 3 && d == 128 ? 5 : flashd_dims(d, pad) / 16; }
 
 // ---- dK / dV: own = keys; Q, dO, lse2 and delta stream.  Replaces _attn_bwd_dkdv (src/flash_attn.py:204-307).
-template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
+template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD, bool WALK = false>
 __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_k, a.B * a.H, a.causal_group, OWN, false, bh, r_own, x0);
   else if constexpr (IMG) flash_block_image(lin, a.nblk_k, a.g.TR, a.H, OWN, bh, r_own, x0);
-  else flash_block(lin, a.nblk_k, TILE ? a.g.TR : a.share_kv.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
+  else flash_block(lin, a.nblk_k, TILE ? a.g.TR : WALK ? 1 : a.share_kv.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* kb_ = reinterpret_cast<const TIO*>(a.k) + b * a.ks[0] + h * a.ks[1];
   const TIO* vb_ = reinterpret_cast<const TIO*>(a.v) + b * a.vs[0] + h * a.vs[1];
@@ -307,6 +310,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   FlashWalk<MODE, CK> W;
   if constexpr (TILE) W.init_tile(a.g, r_own, x0, OWN, true);
   else if constexpr (CAUSAL) W.init_seq((x0 / CK) * CK, a.Lq);
+  else if constexpr (WALK) W.init_seq(0, a.Lq);
   else W.init_seq(r_own * a.share_kv.len, r_own + 1 < a.share_kv.n ? (r_own + 1) * a.share_kv.len : a.Lq);
   const int wk0 = x0 + wave * 16 * NP;  // first own key of this wave
   const int own_base = TILE ? r_own * a.Lk : 0;   // token index of own x = 0
@@ -492,6 +496,28 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   // Chunk ci lives in buffer ci % NBUF; its copy is started AHEAD chunks before it is consumed (the latency of a copy
   // is longer than the products of one chunk take).  Without a causal mask only the last chunk can be short: the loop
   // bodies then hold no per-pair test.
+  // WALK: a share's sums are done (`edge`: the first chunk of the next one): they join those of the shares before it
+  int edge = WALK ? a.share_kv.len / CK : 0;
+  f32x4 dk_tot[WALK ? NP : 1][KB], dv_tot[WALK ? NP : 1][VB];
+  auto close = [&]() __attribute__((always_inline)) {
+    edge += a.share_kv.len / CK;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+#pragma unroll
+      for (int d = 0; d < KB; d++) { dk_tot[p][d] += dk_acc[p][d]; dk_acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+#pragma unroll
+      for (int d = 0; d < VB; d++) { dv_tot[p][d] += dv_acc[p][d]; dv_acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    }
+  };
+  if constexpr (WALK) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+#pragma unroll
+      for (int d = 0; d < KB; d++) dk_tot[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < VB; d++) dv_tot[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
   int ci = 0, bi = 0;   // bi = ci % NBUF
   auto buf_of = [&](int i) { return smem + (i >= NBUF ? i - NBUF : i) * B::BUF_KV; };
   if constexpr (CAUSAL) {
@@ -513,7 +539,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
   };
   // NBUF rounds at a time: the buffers' places are immediates of the LDS reads then (as run-time values they cost an addition per
   // lane offset and chunk).  Two own blocks at 64/128 have no register left for it (20 would be spilled)
-  constexpr bool UNROLL = DK + DV <= 128 || NP == 1;
+  constexpr bool UNROLL = !WALK && (DK + DV <= 128 || NP == 1);
   while (CAUSAL && UNROLL && ci + AHEAD < W.nchunks && bi != 0) plain_round();
   while (UNROLL && ci + AHEAD + NBUF - 1 < W.nchunks)
     swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
@@ -523,11 +549,17 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
       __syncthreads();
       ci++;
     });
+  if constexpr (WALK)
+    while (ci + AHEAD < W.nchunks) {
+      for (const int stop = dlt_imin(edge, W.nchunks - AHEAD); ci < stop;) plain_round();
+      if (ci == edge) close();
+    }
   while (ci + AHEAD < W.nchunks) plain_round();
   // without a mask a full last chunk runs here too (same test-free body): the code below, whose per-pair tests cost
   // registers the compiler finds by spilling, is then not executed at all
   const int n_plain = TILE || (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
   for (; ci < n_plain; ci++) {
+    if (WALK && ci == edge) close();
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::false_type{});
     swa2_wait_copies();
@@ -535,10 +567,21 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
     bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
   if (!TILE && ci < W.nchunks) {
+    if (WALK && ci == edge) close();
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
-  if (MODE == 0 && a.share_kv.n > 1) {
+  if constexpr (WALK) {
+    close();
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+#pragma unroll
+      for (int d = 0; d < KB; d++) dk_acc[p][d] = dk_tot[p][d];
+#pragma unroll
+      for (int d = 0; d < VB; d++) dv_acc[p][d] = dv_tot[p][d];
+    }
+  }
+  if (MODE == 0 && !WALK && a.share_kv.n > 1) {
     float* part = a.share_kv.part + flash_share_row(a.share_kv, bh, r_own, a.Lk) * a.dk_;
     flash_share_put<NP>(part, dk_acc, a.dk_, wk0 + n, a.Lk, g);
     part = a.share_kv.part + (int64_t)a.B * a.H * a.share_kv.n * a.Lk * a.dk_ + flash_share_row(a.share_kv, bh, r_own, a.Lk) * a.dv_;
@@ -556,8 +599,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_bwd_kv_kernel(
 // Per chunk: S^T = K Q^T for every 32-key block (a stream of NKB 2 KC operand reads, NP products each), one softmax
 // update per query block, then O^T += V^T P^T (NKB VB transposed operands) with the row sums from a ones-row product.
 // The reads of the second stream are already in flight while the softmax runs.
-template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
-__global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(const FlashArgs a) {
+template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD, bool WALK = false>
+__global__ __launch_bounds__(64 * NW, flashd_fwd_occ(DK, DV, NW, WALK)) void flashd_fwd_kernel(const FlashArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef typename TileOf<TIO>::type TL;
   typedef FlashDBuf<DK, DV, CK> B;
@@ -580,7 +623,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
   else if constexpr (IMG) flash_block_image(lin, a.nblk, a.g.TR, a.H, OWN, bh, r_own, x0);
-  else flash_block(lin, a.nblk, TILE ? a.g.TR : a.share.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
+  else flash_block(lin, a.nblk, TILE ? a.g.TR : WALK ? 1 : a.share.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
@@ -592,6 +635,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   FlashWalk<MODE, CK> W;
   if constexpr (TILE) W.init_tile(a.g, r_own, x0, OWN, false);
   else if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
+  else if constexpr (WALK) W.init_seq(0, a.Lk);
   else W.init_seq(r_own * a.share.len, r_own + 1 < a.share.n ? (r_own + 1) * a.share.len : a.Lk);
 
   const int own_base = TILE ? r_own * a.Lq : 0;   // token index of own x = 0
@@ -740,13 +784,43 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
       }
     });
   };
+  // WALK: as in the dK / dV kernel
+  int edge = WALK ? a.share.len / CK : 0;
+  f32x4 tot[WALK ? NP : 1][VB];
+  float tot_m[WALK ? NP : 1], tot_l[WALK ? NP : 1];
+  auto close = [&]() __attribute__((always_inline)) {
+    edge += a.share.len / CK;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      float f1, f2;
+      flash_merge(tot_m[p], m_run[p], scale, f1, f2);
+      tot_l[p] = flash_add(tot_l[p], f1, wave_sum4(acc_l[p][0]), f2);
+      m_run[p] = -INFINITY;
+      acc_l[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < VB; d++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) tot[p][d][i] = flash_add(tot[p][d][i], f1, acc[p][d][i], f2);
+        acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  if constexpr (WALK) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      tot_m[p] = -INFINITY;
+      tot_l[p] = 0.f;
+#pragma unroll
+      for (int d = 0; d < VB; d++) tot[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
   int ci = 0, bi = 0;
   auto buf_of = [&](int i) { return smem + (i >= NBUF ? i - NBUF : i) * B::BUF; };
   // the first `n` chunks, as far as whole groups of NBUF rounds go: the buffers' places are immediates of the LDS reads (see
   // flashd_bwd_kv_kernel).  64/64: -2.5 %, dense and causal; with 128-key chunks +1 % (64/128) and +3.5 % (128/128); with one own
   // block per wave the calls are too short for it (447 x 447 causal +4 %)
   auto unrolled = [&](const int n) __attribute__((always_inline)) {
-    while (DK + DV <= 128 && NP == 2 && ci + NBUF - 1 < n)
+    while (!WALK && DK + DV <= 128 && NP == 2 && ci + NBUF - 1 < n)
       swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
         constexpr int BI = decltype(bc)::value;
         consume_t(ci, (Swa2Lds)smem + BI * B::BUF, smem + (BI + AHEAD) % NBUF * B::BUF, std::false_type{}, std::true_type{});
@@ -769,6 +843,16 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   } else {
     unrolled(W.nchunks - AHEAD);
   }
+  if constexpr (WALK)
+    while (ci + AHEAD < W.nchunks) {
+      for (const int stop = dlt_imin(edge, W.nchunks - AHEAD); ci < stop; ci++) {
+        consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
+        flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
+        __syncthreads();
+        bi = bi + 1 == NBUF ? 0 : bi + 1;
+      }
+      if (ci == edge) close();
+    }
   for (; ci + AHEAD < W.nchunks; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::true_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
@@ -780,6 +864,7 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   // registers the compiler finds by spilling, is then not executed at all
   const int n_plain = TILE || (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
   for (; ci < n_plain; ci++) {
+    if (WALK && ci == edge) close();
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::false_type{});
     swa2_wait_copies();
@@ -787,10 +872,20 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
     bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
   if (!TILE && ci < W.nchunks) {
+    if (WALK && ci == edge) close();
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
-  if (MODE == 0 && a.share.n > 1) {
+  if constexpr (WALK) {
+    close();
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      m_run[p] = tot_m[p];
+#pragma unroll
+      for (int d = 0; d < VB; d++) acc[p][d] = tot[p][d];
+    }
+  }
+  if (MODE == 0 && !WALK && a.share.n > 1) {
     const int64_t row0 = flash_share_row(a.share, bh, r_own, a.Lq);
     float* ml = a.share.part + (int64_t)a.B * a.H * a.share.n * a.Lq * a.dv + 2 * row0;
     flash_share_put<NP>(a.share.part + row0 * a.dv, acc, a.dv, wq0 + n, a.Lq, g);
@@ -806,14 +901,14 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
   // ---- epilogue: normalise, O^T fragments -> LDS tile -> coalesced rows
 #pragma unroll
   for (int p = 0; p < NP; p++) {
-    const float lt = wave_sum4(acc_l[p][0]);
+    const float lt = WALK ? tot_l[WALK ? p : 0] : wave_sum4(acc_l[p][0]);
     const float inv = lt > 0.f ? fast_rcp(lt) : 0.f;
     TL* orow = reinterpret_cast<TL*>(smem + (wave * 16 * NP + 16 * p + n) * PO);
 #pragma unroll
     for (int d = 0; d < VB; d++)
 #pragma unroll
       for (int i = 0; i < 4; i++) orow[16 * d + 4 * g + i] = (TL)(acc[p][d][i] * inv);
-    if (g == 0 && tq[p] >= 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + tq[p] * a.ls[2]), m_run[p] * scale + fast_log2(lt));
+    if (g == 0 && tq[p] >= 0) store_stream4(a.lse + (b * a.ls[0] + h * a.ls[1] + tq[p] * a.ls[2]), WALK ? flash_lse2(m_run[p], scale, lt) : m_run[p] * scale + fast_log2(lt));
   }
   __syncthreads();
   int tw = tid;   // opaque copy: keeps the tile writer's addresses out of the registers that live across the chunk loop
@@ -826,8 +921,8 @@ __global__ __launch_bounds__(64 * NW, flashd_occ(NW)) void flashd_fwd_kernel(con
 // ---- dQ: own = queries; K and V stream.  Replaces _attn_bwd_dq (src/flash_attn.py:310-449) and, with fuse_delta, the
 // delta pre-pass (:186-202).  Per 32-key block: per 16-key half KC pieces of K (S = K Q^T) and VC pieces of V
 // (dP = V dO^T), then KB transposed pieces of K (dQ^T += K^T dS).
-template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD>
-__global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
+template <typename TIO, int DK, int DV, int NP, int CK, int NW, int MODE, int PAD, bool WALK = false>
+__global__ __launch_bounds__(64 * NW, WALK ? flashd_occ(NW) : flashd_dq_occ(DK, DV, NW)) void flashd_bwd_q_kernel(const FlashBwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef FlashDBuf<DK, DV, CK> B;
   extern __shared__ __align__(16) char smem[];
@@ -848,7 +943,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   int bh, r_own, x0;
   if constexpr (CAUSAL) flash_block_causal(lin, a.nblk_q, a.B * a.H, a.causal_group, OWN, true, bh, r_own, x0);
   else if constexpr (IMG) flash_block_image(lin, a.nblk_q, a.g.TR, a.H, OWN, bh, r_own, x0);
-  else flash_block(lin, a.nblk_q, TILE ? a.g.TR : a.share_q.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
+  else flash_block(lin, a.nblk_q, TILE ? a.g.TR : WALK ? 1 : a.share_q.n, OWN, bh, r_own, x0);   // r_own: the grid row, or the share
   const int wq0 = x0 + wave * 16 * NP;
   const int b = bh / a.H, h = bh - b * a.H;
   const TIO* qb = reinterpret_cast<const TIO*>(a.q) + b * a.qs[0] + h * a.qs[1];
@@ -860,6 +955,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   FlashWalk<MODE, CK> W;
   if constexpr (TILE) W.init_tile(a.g, r_own, x0, OWN, false);
   else if constexpr (CAUSAL) W.init_seq(0, dlt_imin(a.Lk, x0 + OWN));
+  else if constexpr (WALK) W.init_seq(0, a.Lk);
   else W.init_seq(r_own * a.share_q.len, r_own + 1 < a.share_q.n ? (r_own + 1) * a.share_q.len : a.Lk);
 
   const int own_base = TILE ? r_own * a.Lq : 0;   // token index of own x = 0
@@ -1010,12 +1106,28 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
       });
     });
   };
+  // WALK: as in the dK / dV kernel
+  int edge = WALK ? a.share_q.len / CK : 0;
+  f32x4 dq_tot[WALK ? NP : 1][KB];
+  auto close = [&]() __attribute__((always_inline)) {
+    edge += a.share_q.len / CK;
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int d = 0; d < KB; d++) { dq_tot[p][d] += dq_acc[p][d]; dq_acc[p][d] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+  };
+  if constexpr (WALK) {
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int d = 0; d < KB; d++) dq_tot[p][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   int ci = 0, bi = 0;
   auto buf_of = [&](int i) { return smem + (i >= NBUF ? i - NBUF : i) * B::BUF; };
   // the first `n` chunks, as far as whole groups of NBUF rounds go: the buffers' places are immediates of the LDS reads (see
   // flashd_bwd_kv_kernel)
   auto unrolled = [&](const int n) __attribute__((always_inline)) {
-    while (ci + NBUF - 1 < n)
+    while (!WALK && ci + NBUF - 1 < n)
       swa2_for<0, NBUF>([&](auto bc) __attribute__((always_inline)) {
         constexpr int BI = decltype(bc)::value;
         consume_t(ci, (Swa2Lds)smem + BI * B::BUF, smem + (BI + AHEAD) % NBUF * B::BUF, std::false_type{}, std::true_type{});
@@ -1038,6 +1150,16 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   } else {
     unrolled(W.nchunks - AHEAD);
   }
+  if constexpr (WALK)
+    while (ci + AHEAD < W.nchunks) {
+      for (const int stop = dlt_imin(edge, W.nchunks - AHEAD); ci < stop; ci++) {
+        consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
+        flashd_wait_copies<(AHEAD - 1) * PER_CHUNK>();
+        __syncthreads();
+        bi = bi + 1 == NBUF ? 0 : bi + 1;
+      }
+      if (ci == edge) close();
+    }
   for (; ci + AHEAD < W.nchunks; ci++) {
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::true_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::true_type{});
@@ -1049,6 +1171,7 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
   // registers the compiler finds by spilling, is then not executed at all
   const int n_plain = TILE || (!CAUSAL && W.nchunks > 0 && !chunk_tail(W.nchunks - 1)) ? W.nchunks : W.nchunks - 1;
   for (; ci < n_plain; ci++) {
+    if (WALK && ci == edge) close();
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::false_type{}, std::false_type{});
     swa2_wait_copies();
@@ -1056,10 +1179,18 @@ __global__ __launch_bounds__(64 * NW, flashd_dq_occ(DK, DV, NW)) void flashd_bwd
     bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
   if (!TILE && ci < W.nchunks) {
+    if (WALK && ci == edge) close();
     if (CAUSAL) consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), FlashTailDyn{}, std::false_type{});
     else consume_t(ci, (Swa2Lds)buf_of(bi), buf_of(bi + AHEAD), std::true_type{}, std::false_type{});
   }
-  if (MODE == 0 && a.share_q.n > 1) {
+  if constexpr (WALK) {
+    close();
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int d = 0; d < KB; d++) dq_acc[p][d] = dq_tot[p][d];
+  }
+  if (MODE == 0 && !WALK && a.share_q.n > 1) {
     flash_share_put<NP>(a.share_q.part + flash_share_row(a.share_q, bh, r_own, a.Lq) * a.dk_, dq_acc, a.dk_, wq0 + n, a.Lq, g);
     return;
   }

@@ -53,16 +53,16 @@ template <typename KernT>
 int flash_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast<const void*>(kern), bytes); }
 
 #if DLT_FLASH_PART == 0 || DLT_FLASH_PART == 3
-template <typename TIO, int MODE, int NP, int CK, int NW>
+template <typename TIO, int MODE, int NP, int CK, int NW, bool WALK = false>
 int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   // head dims below the padded ones (multiples of 8): the kernel variant whose copies skip the missing pieces
   const int pad = flashd_pad(a.dk, a.dv);
-  auto kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
+  auto kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0, WALK>;
   if constexpr (MODE < 2)
-    if (pad == 1) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+    if (pad == 1) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1, WALK>;
   if constexpr (MODE < 2 && DLT_DV == 128) {
-    if (pad == 2) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
-    if (pad == 3) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
+    if (pad == 2) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2, WALK>;
+    if (pad == 3) kern = flashd_fwd_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3, WALK>;
   }
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DV * 2 + 16);
@@ -71,7 +71,7 @@ int flashd_launch_fwd(FlashArgs a, hipStream_t stream) {
   const int rc = flash_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;
   a.nblk = (a.Lq + own - 1) / own;
-  const int rows = MODE >= 2 ? a.g.TR : a.share.n;
+  const int rows = MODE >= 2 ? a.g.TR : WALK ? 1 : a.share.n;
   dlt_timing_before(DLT_K_FWD, stream);
   hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk * rows), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
@@ -86,6 +86,9 @@ int flash_launch_fwd_c(const FlashArgs& a, int grid, hipStream_t stream) {
     // class and mode against the register-staged kernel: dense -2 % (64/64), -4 % (64/128), -7 % (128/128); causal -4 %
     // (64/64), -18 % (128/128); head dims below the class (80/80, 96/96): -18 % on the step.
     if (a.dk % 8 == 0 && a.dv % 8 == 0 && dlt_flash_async()) {
+      if constexpr (MODE == 0)
+        if (a.share.walk)   // workgroups of 64 queries or 128
+          return a.Lq <= 64 ? flashd_launch_fwd<TIO, 0, 1, 64, 4, true>(a, stream) : flashd_launch_fwd<TIO, 0, (DLT_DV == 128 ? 1 : 2), 64, (DLT_DV == 128 ? 8 : 4), true>(a, stream);
       // few workgroups: one own block per wave (see flash_forward)
       if constexpr (DLT_DV == 128)
         if (a.slim != 0 && a.chunk == 128)
@@ -131,16 +134,16 @@ int DLT_FCAT3(dlt_flash_launch_fwdc_, DLT_DK, DLT_DV)(const FlashArgs& a, int dt
 #endif
 
 #elif DLT_FLASH_PART == 1
-template <typename TIO, int MODE, int NP, int NW>
+template <typename TIO, int MODE, int NP, int NW, bool WALK = false>
 int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
   const int pad = flashd_pad(a.dk_, a.dv_);
-  auto kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
+  auto kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0, WALK>;
   if constexpr (MODE < 2)
-    if (pad == 1) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+    if (pad == 1) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1, WALK>;
   if constexpr (MODE < 2 && DLT_DV == 128) {
-    if (pad == 2) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
-    if (pad == 3) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
+    if (pad == 2) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2, WALK>;
+    if (pad == 3) kern = flashd_bwd_q_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3, WALK>;
   }
   constexpr int own = 16 * NP * NW;
   constexpr int tile = own * (DLT_DK * 2 + 16);
@@ -150,7 +153,7 @@ int flashd_launch_bwd_q(FlashBwdArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk_q = (a.Lq + own - 1) / own;
   dlt_timing_before(DLT_K_BWD_Q, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q * (MODE >= 2 ? a.g.TR : a.share_q.n)), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_q * (MODE >= 2 ? a.g.TR : WALK ? 1 : a.share_q.n)), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash dQ launch");
   return DLT_OK;
@@ -160,6 +163,12 @@ template <typename TIO, int MODE>
 int flash_launch_bwd_q_c(const FlashBwdArgs& a, int grid_q, hipStream_t stream) {
   if constexpr (DLT_DK >= 64 && DLT_DV >= 64 && MODE < 2) {
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && dlt_flash_async()) {
+      if constexpr (MODE == 0)
+        if (a.share_q.walk) {   // (two blocks' sums of 128 dims do not fit the registers)
+          if constexpr (DLT_DK == 64)
+            if (a.Lq > 256) return flashd_launch_bwd_q<TIO, 0, 2, 4, true>(a, stream);
+          return flashd_launch_bwd_q<TIO, 0, 1, 4, true>(a, stream);
+        }
       // few workgroups: one own block per wave, in 4 waves (twice the workgroups) or, without a mask, 8 (see flash_backward)
       if (a.slim_q == 4) return flashd_launch_bwd_q<TIO, MODE, 1, 4>(a, stream);
       if constexpr (MODE == 0)
@@ -192,16 +201,16 @@ int DLT_FCAT3(dlt_flash_launch_bwd_q_, DLT_DK, DLT_DV)(const FlashBwdArgs& a, in
 }
 
 #else
-template <typename TIO, int MODE, int NP, int NW>
+template <typename TIO, int MODE, int NP, int NW, bool WALK = false>
 int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   constexpr int CK = 64;
   const int pad = flashd_pad(a.dk_, a.dv_);
-  auto kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0>;
+  auto kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 0, WALK>;
   if constexpr (MODE < 2)
-    if (pad == 1) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1>;
+    if (pad == 1) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 1, WALK>;
   if constexpr (MODE < 2 && DLT_DV == 128) {
-    if (pad == 2) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2>;
-    if (pad == 3) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3>;
+    if (pad == 2) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 2, WALK>;
+    if (pad == 3) kern = flashd_bwd_kv_kernel<TIO, DLT_DK, DLT_DV, NP, CK, NW, MODE, 3, WALK>;
   }
   constexpr int own = 16 * NP * NW;
   constexpr int tile_k = own * (DLT_DK * 2 + 16), tile_v = own * (DLT_DV * 2 + 16);
@@ -211,7 +220,7 @@ int flashd_launch_bwd_kv(FlashBwdArgs a, hipStream_t stream) {
   if (rc != DLT_OK) return rc;
   a.nblk_k = (a.Lk + own - 1) / own;
   dlt_timing_before(DLT_K_BWD_KV, stream);
-  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k * (MODE >= 2 ? a.g.TR : a.share_kv.n)), dim3(64 * NW), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3(a.B * a.H * a.nblk_k * (MODE >= 2 ? a.g.TR : WALK ? 1 : a.share_kv.n)), dim3(64 * NW), lds, stream, a);
   dlt_timing_after(stream);
   DLT_CHECK_LAUNCH("flash dK/dV launch");
   return DLT_OK;
@@ -223,6 +232,12 @@ int flash_launch_bwd_kv_c(const FlashBwdArgs& a, int grid_kv, hipStream_t stream
     // dense / causal, head dims that are multiples of 8: chunks are copied HBM -> LDS asynchronously (tiles that are no multiple of 64
     // tokens: parts of a chunk are skipped, the register-staged kernel measured 1.5 % faster)
     if (a.dk_ % 8 == 0 && a.dv_ % 8 == 0 && dlt_flash_scalars_fit(a) && dlt_flash_async()) {
+      if constexpr (MODE == 0)
+        if (a.share_kv.walk) {
+          if constexpr (DLT_DV == 64)
+            if (a.Lk > 64) return flashd_launch_bwd_kv<TIO, 0, 2, 4, true>(a, stream);
+          return flashd_launch_bwd_kv<TIO, 0, 1, 4, true>(a, stream);
+        }
       if (a.slim) return flashd_launch_bwd_kv<TIO, MODE, 1, 4>(a, stream);
       return flashd_launch_bwd_kv<TIO, MODE, flash_np_kv(DLT_DK, DLT_DV), FLASHD_BWD_NW>(a, stream);
     }

@@ -220,11 +220,23 @@ inline int flash_causal_group(int L, int dk, int dv) {
 
 // The streamed side of an own block split over `n` workgroups (dense, asynchronously staged kernels): share i takes the tokens from i `len` on,
 // `len` of them (a multiple of the chunk), the last one the rest.  Results then go to `part`, fp32 rows [batch * head][share][own
-// token][head dim], and a second launch sums them (flash_share.hip).  n = 1: no split.
+// token][head dim], and a second launch sums them (flash_share.hip).  n = 1: no split.  `walk`: one workgroup takes the shares of its own block one after the
+// other, each from nothing, and adds them up itself in the same order with the same operations (flash_merge): the same bits without `part`.
+constexpr int FLASH_SHARES_MAX = 8;
 struct FlashShare {
   float* part;
   int32_t n, len;
+  bool walk;   // host only
 };
+// weights of two partial results of a softmax with reference maxima m and m2 (raw scores); m becomes that of their sum
+DLT_DEV void flash_merge(float& m, float m2, float scale, float& f1, float& f2) {
+  const float m_new = fmaxf(m, m2);
+  f1 = m == -INFINITY ? 0.f : fast_exp2((m - m_new) * scale);
+  f2 = m2 == -INFINITY ? 0.f : fast_exp2((m2 - m_new) * scale);
+  m = m_new;
+}
+DLT_DEV float flash_add(float x, float f1, float x2, float f2) { return fmaf(x2, f2, x * f1); }
+DLT_DEV float flash_lse2(float m, float scale, float l) { return fmaf(m, scale, fast_log2(l)); }
 
 struct FlashArgs {
   const void *q, *k, *v;

@@ -49,24 +49,23 @@ __global__ __launch_bounds__(256) void flash_share_fwd_kernel(const ShareOut o, 
   for (int s = 0; s < S; s++) w[s] = *reinterpret_cast<const float2*>(ml + 2 * (row0 + (int64_t)s * o.L));
   share_load<S>(o.part + row0 * o.d + it.d0, (int64_t)o.L * o.d, lo, hi);
   float m = -INFINITY, l = 0.f;
-#pragma unroll
-  for (int s = 0; s < S; s++) m = fmaxf(m, w[s].x);
   f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
 #pragma unroll
   for (int s = 0; s < S; s++) {
-    const float f = w[s].x == -INFINITY ? 0.f : fast_exp2((w[s].x - m) * scale);
-    l = fmaf(w[s].y, f, l);
+    float f1, f2;
+    flash_merge(m, w[s].x, scale, f1, f2);
+    l = flash_add(l, f1, w[s].y, f2);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      a[j] = fmaf(lo[s][j], f, a[j]);
-      b[j] = fmaf(hi[s][j], f, b[j]);
+      a[j] = flash_add(a[j], f1, lo[s][j], f2);
+      b[j] = flash_add(b[j], f1, hi[s][j], f2);
     }
   }
   const float inv = l > 0.f ? fast_rcp(l) : 0.f;
   const float v[8] = {a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv, b[0] * inv, b[1] * inv, b[2] * inv, b[3] * inv};
   const int bb = it.bh / H, h = it.bh - bb * H;
   Io<TIO, TIO>::store8(reinterpret_cast<TIO*>(o.out) + bb * o.st[0] + h * o.st[1] + it.row * o.st[2] + it.d0 * o.st[3], v, o.vec != 0, o.st[3], 8);
-  if (it.d0 == 0) store_stream4(lse + bb * ls0 + h * ls1 + it.row * ls2, m * scale + fast_log2(l));
+  if (it.d0 == 0) store_stream4(lse + bb * ls0 + h * ls1 + it.row * ls2, flash_lse2(m, scale, l));
 }
 
 // workgroups [0, split) sum `x`, the others `y`
@@ -82,9 +81,9 @@ __global__ __launch_bounds__(256) void flash_share_grad_kernel(const ShareOut x,
   float v[8];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    float a = lo[0][j], b = hi[0][j];
+    float a = 0.f, b = 0.f;
 #pragma unroll
-    for (int s = 1; s < S; s++) { a += lo[s][j]; b += hi[s][j]; }
+    for (int s = 0; s < S; s++) { a += lo[s][j]; b += hi[s][j]; }
     v[j] = a * o.mul;
     v[4 + j] = b * o.mul;
   }
@@ -101,6 +100,7 @@ ShareOut share_out(const float* part, void* out, const int64_t (&st)[5], float m
 }
 uint32_t share_blocks(const ShareOut& o) { return (uint32_t)((o.items + 255) / 256); }
 
+static_assert(FLASH_SHARES_MAX == 8, "share_switch");
 template <typename F>
 int share_switch(int n, F&& f) {
   switch (n) {
@@ -111,14 +111,6 @@ int share_switch(int n, F&& f) {
     case 6: return f(std::integral_constant<int, 6>{});
     case 7: return f(std::integral_constant<int, 7>{});
     case 8: return f(std::integral_constant<int, 8>{});
-    case 9: return f(std::integral_constant<int, 9>{});
-    case 10: return f(std::integral_constant<int, 10>{});
-    case 11: return f(std::integral_constant<int, 11>{});
-    case 12: return f(std::integral_constant<int, 12>{});
-    case 13: return f(std::integral_constant<int, 13>{});
-    case 14: return f(std::integral_constant<int, 14>{});
-    case 15: return f(std::integral_constant<int, 15>{});
-    case 16: return f(std::integral_constant<int, 16>{});
     default: return dlt_set_error(DLT_ERR_UNSUPPORTED, "flash: %d shares of a streamed side", n);
   }
 }

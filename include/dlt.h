@@ -255,11 +255,15 @@ int dlt_flash_bwd(const void* q, const int64_t q_strides[4], const void* k, cons
                   const dlt_flash_shape_t* shape, void* stream);
 
 /* The same calls with a workspace.  Dense passes whose own side (queries in the forward pass and for dQ, keys for dK / dV) is too
- * short to fill the chip split their other side over workgroups; each leaves fp32 partial results in `ws`, which a second
- * launch sums in a fixed order.  dlt_flash_workspace() says how many bytes a shape's pass needs (0: it is not split); the
- * split follows from Lq, Lk, dk and dv alone.  `ws` is 16-byte aligned device memory whose contents need not be set and are
- * of no use afterwards; it belongs to the call until its kernels have run.  With ws == NULL nothing is split, as in
+ * short to fill the chip split their other side into shares over workgroups; each leaves fp32 partial results in `ws`, which a
+ * second launch sums in a fixed order.  Where the slabs of a call fill the chip one workgroup takes all shares, with the same bits
+ * and without `ws`.  dlt_flash_workspace() says how many bytes a call's pass needs (0: none), at most DLT_FLASH_WORKSPACE_MAX.  The shares follow
+ * from Lq, Lk, dk and dv, so that a slab's bits do not depend on how many a call holds; calls of fp32 tensors, of head dims that are no multiples of 8,
+ * beyond 128 or both up to 32, of B H max(Lq, Lk) >= 2^27, with rows that cannot be read in 16-byte pieces or with DLT_FLASH_SYNC_STAGING
+ * set have none, nor has dK / dV where one slab's lse2 spans 2 GiB.  `ws` is 16-byte aligned device memory whose contents need not be set and are
+ * of no use afterwards; it belongs to the call until its kernels have run.  With ws == NULL where bytes are needed there are no shares, as in
  * dlt_flash_fwd / dlt_flash_bwd; results of the two ways differ by the rounding of another order of summation. */
+#define DLT_FLASH_WORKSPACE_MAX (256 << 20)
 int dlt_flash_workspace(const dlt_flash_shape_t* shape, int backward, int64_t* bytes);
 int dlt_flash_fwd_ws(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
                      const void* v, const int64_t v_strides[4], void* o, const int64_t o_strides[4],

@@ -124,10 +124,15 @@ def test_flash_workspace_of_a_shape():
         n = ctypes.c_int64(-1)
         assert lib.dlt_flash_workspace(L.FlashShape(*shape), backward, ctypes.byref(n)) == 0, lib.dlt_last_error()
         return n.value
-    # 64 queries x 4000 keys: 8 shares of a forward pass (64 output dims, maximum and sum), of dQ 7 (512 keys each but the last)
+    # 64 queries x 4000 keys: 8 shares of a forward pass (64 output dims, maximum and sum) and of dQ (512 keys each but the last); dK and dV of 64 keys the same way
     assert need(0, 1, 2, 64, 4000, 64, 64, 0.1, 0, 0) == 4 * 2 * 8 * 64 * (64 + 2)
     assert need(1, 1, 2, 64, 4000, 64, 64, 0.1, 0, 0) == 4 * 2 * 8 * 64 * 64
-    assert need(1, 1, 1, 4000, 64, 64, 64, 0.1, 0, 0) % (4 * 64 * 128) == 0
+    assert need(1, 1, 1, 4000, 64, 64, 64, 0.1, 0, 0) == 4 * 8 * 64 * 128
+    # on a full chip one workgroup takes all shares of its own block and needs nothing; partial results never exceed the stated maximum
+    assert need(0, 2, 95, 64, 4000, 64, 64, 0.1, 0, 0) == 4 * 190 * 8 * 64 * (64 + 2) and need(0, 2, 96, 64, 4000, 64, 64, 0.1, 0, 0) == 0
+    for shape in ((64, 32, 512, 8192, 128, 128), (128, 32, 8192, 1024, 64, 64), (1, 1, 40000, 1000000, 128, 128), (1, 1, 1000000, 40000, 64, 128), (1, 90, 128, 8192, 128, 128),
+                  (1, 1, 24000, 400000, 128, 128), (1, 1, 24000, 400000, 64, 128), (1, 180, 64, 8192, 64, 128), (1, 1, 400000, 24000, 128, 128)):
+        assert need(0, *shape, 0.1, 0, 0) <= 256 << 20 and need(1, *shape, 0.1, 0, 0) <= 256 << 20
     # nothing is split under a mask, for balanced sides, in fp32, at odd head dims and outside the classes of 64 and 128
     for shape in ((1, 1, 4000, 4000, 64, 64, 0.1, 1, 0), (1, 1, 2048, 2048, 64, 64, 0.1, 0, 0), (1, 1, 64, 4000, 64, 64, 0.1, 0, 2),
                   (1, 1, 64, 4000, 60, 64, 0.1, 0, 0), (1, 1, 64, 4000, 32, 32, 0.1, 0, 0), (1, 1, 64, 4000, 136, 136, 0.1, 0, 0)):

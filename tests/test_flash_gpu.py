@@ -469,3 +469,33 @@ def test_output_dims_over_workgroups(dk, dv, counts, Lk):
     for n in counts[:-1]:
         got = _fa()._forward(q[:, :n].contiguous(), k[:, :n].contiguous(), v[:, :n].contiguous(), False, scale)
         assert torch.equal(got[0], o[:, :n]) and torch.equal(got[1], M[:, :n])
+
+
+# dense passes in shares: split over workgroups on few slabs, walked by one workgroup once the chip is full (192 workgroups of up to 64 own tokens, 384 of more), with the
+# same bits as a slab alone; forward, dQ and dK/dV in shares, every class and dims below it, own tokens of one wave and past a workgroup's end, last shares of one token and of one
+# chunk, one full and one short; an infinite score, an infinite value and NaN in one slab
+@pytest.mark.parametrize("Lq,Lk,dk,dv,counts", [
+    (64, 3073, 64, 64, (2, 191, 192)), (19, 3300, 64, 128, (2, 191, 192)), (37, 2600, 80, 80, (2, 200)), (64, 1281, 128, 128, (2, 200)), (130, 3200, 64, 64, (2, 127, 128)),
+    (70, 3585, 48, 40, (2, 200)), (100, 3137, 64, 128, (2, 191, 192)), (129, 2700, 96, 88, (2, 130)), (90, 1300, 128, 104, (2, 200)), (1700, 70, 64, 64, (2, 191, 192)),
+    (2600, 19, 64, 64, (2, 200)), (1665, 40, 64, 128, (2, 200)), (2100, 90, 80, 72, (2, 200)), (1300, 33, 128, 128, (2, 200)), (2561, 200, 48, 64, (2, 100))])
+def test_shares_walked_by_one_workgroup(Lq, Lk, dk, dv, counts):
+    scale = 1 / math.sqrt(dk)
+    q, k, v, do = (t.cuda() for t in orc.make_qkv(Lq + Lk + dk, 1, 3, Lq, Lk, dk, dv, torch.bfloat16))
+    want = orc.flash_grads(*(t[:, :1].float().cpu() for t in (q, k, v, do)), False, scale)
+    k[:, 2, Lk // 2, 0], v[:, 2, Lk - 1, 3], q[:, 2, 0, 1] = float("inf"), float("inf"), float("nan")
+
+    def run(slabs):   # the first, as often as asked, and the two others
+        args = [torch.cat([t[:, :1].expand(-1, slabs - 2, -1, -1), t[:, 1:]], 1) if slabs > 2 else t[:, :2] for t in (q, k, v, do)]
+        leaves = [t.detach().contiguous().requires_grad_(True) for t in args[:3]]
+        o = _fa().attention(*leaves, False, scale)
+        _, M = _fa()._forward(*(t.detach() for t in leaves), False, scale)
+        return (o.detach(), M) + torch.autograd.grad(o, leaves, args[3].contiguous())
+
+    few, runs = run(3), [run(n) for n in counts]
+    assert (few[0][:, :1].float().cpu() - want[0]).abs().max().item() <= 2e-2 and max(_rel(g[:, :1], w) for g, w in zip(few[2:], want[1:])) <= 5e-2
+    for n, got in zip(counts, runs):
+        for a, b in zip(got, few):
+            assert torch.equal(a[:, :1], b[:, :1])
+            if n > 2:
+                assert torch.equal(a[:, :-2], b[:, :1].expand_as(a[:, :-2])) and torch.equal(a[:, -2], b[:, 1]) and torch.equal(a[:, -1].isfinite(), b[:, 2].isfinite())
+                assert torch.equal(a[:, -1].nan_to_num(), b[:, 2].nan_to_num())
