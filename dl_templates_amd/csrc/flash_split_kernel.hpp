@@ -93,7 +93,8 @@ struct FlashsTile {
       lds_write16(s + t * 2 * D + 16 * (p ^ flashs_swz<D>(t)), r[it]);
     }
   }
-  // A block's tokens from `left` on repeat the list's last one: their probabilities are 0, which times an infinite value is not, so that they are cleared
+  // Tiles: a block's tokens from `left` on repeat the list's last one: their probabilities are 0, which times an infinite value is not, so that they are cleared
+  // (dense calls, where that token is the sequence's last one, go without: it costs short backward passes 3 to 5 %)
   static DLT_DEV void clear_past(u32x4 (&r)[NV], int left, int lane) {
     if (left >= 32) return;   // wave-uniform
 #pragma unroll
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_fwd_kernel(const Flash
   }
   const float scale = a.scale_log2;
   for (int kb = wave; kb < nkb; kb += NW) {
-    VT::clear_past(vr, keys.len - 32 * kb, lane);
+    if constexpr (MODE >= 2) VT::clear_past(vr, keys.len - 32 * kb, lane);
     VT::write(sV, vr, lane);
     u32x4 ka[2][KC];
 #pragma unroll
@@ -401,7 +402,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
   }
   const float scale = a.scale_log2;
   for (int kb = wave; kb < nkb; kb += NW) {
-    KT::clear_past(kr, keys.len - 32 * kb, lane);
+    if constexpr (MODE >= 2) KT::clear_past(kr, keys.len - 32 * kb, lane);
     KT::write(sK, kr, lane);
     u32x4 va[2][VC];
 #pragma unroll
@@ -430,9 +431,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_q_kernel(const Fla
         const int klim = CAUSAL ? dlt_imin(x0 + 16 * p + n, keys.len - 1) : keys.len - 1;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float dsv = fast_exp2(fmaf(s[i], scale, nlse[p])) * dp[i];
-          if (tail) dsv = 32 * kb + 16 * mb + 4 * g + i <= klim ? dsv : 0.f;
-          ds[p][4 * mb + i] = dsv;
+          float pv = fast_exp2(fmaf(s[i], scale, nlse[p]));
+          if (tail) pv = 32 * kb + 16 * mb + 4 * g + i <= klim ? pv : 0.f;
+          ds[p][4 * mb + i] = pv * dp[i];
+          if (MODE >= 2 && tail) ds[p][4 * mb + i] = 32 * kb + 16 * mb + 4 * g + i <= klim ? ds[p][4 * mb + i] : 0.f;
         }
       }
     }
@@ -523,8 +525,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
   }
   const float scale = a.scale_log2;
   for (int qbk = first; qbk < nqb; qbk += NW) {
-    QT::clear_past(qr, queries.len - 32 * qbk, lane);
-    DT::clear_past(dr, queries.len - 32 * qbk, lane);
+    if constexpr (MODE >= 2) {
+      QT::clear_past(qr, queries.len - 32 * qbk, lane);
+      DT::clear_past(dr, queries.len - 32 * qbk, lane);
+    }
     QT::write(sQ, qr, lane);
     DT::write(sD, dr, lane);
     sc[lane] = scr;
@@ -549,15 +553,12 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void flashs_bwd_kv_kernel(const Fl
         const int qmin = CAUSAL ? x0 + 16 * p + n : 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float pv = fast_exp2(fmaf(s[i], scale, -lq[i])), dsv = -pv * dp[i];
-          if (tail) {
-            const int qi = 32 * qbk + 16 * mb + 4 * g + i;
-            const bool in = qi >= qmin && qi < queries.len;
-            pv = in ? pv : 0.f;
-            dsv = in ? dsv : 0.f;
-          }
+          float pv = fast_exp2(fmaf(s[i], scale, -lq[i]));
+          const int qi = 32 * qbk + 16 * mb + 4 * g + i;
+          if (tail) pv = (qi >= qmin && qi < queries.len) ? pv : 0.f;
           pr[p][4 * mb + i] = pv;
-          ds[p][4 * mb + i] = dsv;
+          ds[p][4 * mb + i] = -pv * dp[i];
+          if (MODE >= 2 && tail) ds[p][4 * mb + i] = qi < queries.len ? ds[p][4 * mb + i] : 0.f;
         }
       }
     }
