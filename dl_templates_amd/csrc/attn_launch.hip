@@ -349,7 +349,7 @@ int swa2_pick_tall(const AttnProblem& p, int rest, bool backward) {
 }
 
 // returns the workgroups of 8 rows x 16 columns that the grids of all slabs take
-int64_t swa2_make_plan(const AttnProblem& p, bool backward, Swa2Plan& plan) {
+int64_t swa2_make_plan(const AttnProblem& p, bool backward, bool may_tall, Swa2Plan& plan) {
   // Bands of four rows (the waves of the lower four only copy; the same bits) while those too have a CU each: a band's time is its halo's copies and
   // chunks, 4 + 2 WR rows instead of 8 + 2 WR.  Over 3508 shapes of up to 128 workgroups forward 0.81 ... 0.87 of the time, backward 0.76 ... 0.82
   // (d = 128, 4 slabs of 47 x 25, 15 x 5 window, forward 10.3 -> 8.5 us); from 129 on, where workgroups of 4 rows would queue, 0.9 ... 1.1 and 1.1 ... 1.3.
@@ -364,7 +364,7 @@ int64_t swa2_make_plan(const AttnProblem& p, bool backward, Swa2Plan& plan) {
   plan.nblk_c = (swa2_slots(p) + 15) / 16;
   plan.ntall = 0; plan.lpc = 2;
   const int rest = swa2_slots(p) & 15;
-  if (rest >= 1 && rest <= 8 && bands > dlt_device_cus() && (backward || p.dk == 128)) {
+  if (may_tall && rest >= 1 && rest <= 8 && bands > dlt_device_cus()) {
     // The last columns fill half a workgroup or less: 2 or 1 patch columns and bands of 16 or 32 rows (the same bits), where the estimate says that
     // it pays.  90 shapes of 257 ... 2300 bands, backward 0.945 of the time in the mean of all, 0.61 ... 1.016, taken for 34 of them (d = 128, 16
     // slabs of 71 x 17, 17 x 7 window 0.64; 64 of 99 x 18, 15 x 9 184 -> 139 us); forward at d = 128, taken for 10, 0.98 in the mean, 56 -> 49 there; at
@@ -411,7 +411,7 @@ int swa2_forward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream)
   // 11.2 / 12.2, 352 26.8 / 25.8).
   // DLT_SWA2_SINGLE_PATCH=1 (read once per process) keeps the one-patch kernel for A/B timing and for its tests.
   static const bool single_patch = [] { const char* e = getenv("DLT_SWA2_SINGLE_PATCH"); return e != nullptr && e[0] == '1'; }();
-  const int64_t bands = swa2_make_plan(p, false, a.plan);
+  const int64_t bands = swa2_make_plan(p, false, p.dk == 128 && !single_patch, a.plan);   // tall workgroups: two patches per wave only
   a.plan.pairs = !single_patch && bands > dlt_device_cus();
   a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.out_o; a.lse = t.lse;
   for (int i = 0; i < 4; i++) { a.qs[i] = t.qs[i]; a.ks[i] = t.ks[i]; a.vs[i] = t.vs[i]; a.os[i] = t.os[i]; }
@@ -426,7 +426,7 @@ int swa2_backward(const AttnProblem& p, const AttnTensors& t, hipStream_t stream
   if (dlt_route_note(DLT_FAMILY_STREAMING)) return DLT_OK;
   Swa2BwdArgs a;
   a.p = p;
-  swa2_make_plan(p, true, a.plan);
+  swa2_make_plan(p, true, true, a.plan);
   a.q = t.q; a.k = t.k; a.v = t.v; a.o = t.o; a.d_o = t.d_o; a.lse = t.lse; a.delta = t.delta;
   a.dq = t.dq; a.dk = t.dk; a.dv = t.dv;
   for (int i = 0; i < 4; i++) {

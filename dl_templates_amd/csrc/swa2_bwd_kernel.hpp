@@ -27,7 +27,7 @@ constexpr int swa2_occ_bwd_q(int D) { return D == 64 ? 4 : 2; }
 constexpr int swa2_occ_bwd_kv(int D) { return 2; }
 
 // =============================================================================================== dQ
-template <typename TIO, int D, int NCG, bool PAD>
+template <typename TIO, int D, int NCG, bool PAD, bool TALL>
 __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_kernel(const Swa2BwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef Swa2Cfg<D, NCG, PAD> C;
@@ -37,7 +37,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_ke
   const int tid = threadIdx.x;
   const int lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Swa2Geom G0 = swa2_geom(a.p, a.plan);
+  const Swa2Geom G0 = swa2_geom<TALL>(a.p, a.plan);
   const int pc = wave & ((1 << G0.lpc) - 1), rg = wave >> G0.lpc;
 
   const char* qb = reinterpret_cast<const char*>(a.q) + 2 * (G0.b * a.qs[0] + G0.h * a.qs[1]);
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_q(D)) void swa2_bwd_q_ke
 
 // =============================================================================================== dK / dV
 // A chunk buffer holds Q, dO and a table of per-token scalars: lse2 then delta, [4 halo rows][HCW halo columns] each.
-template <typename TIO, int D, int NCG, bool PAD>
+template <typename TIO, int D, int NCG, bool PAD, bool TALL>
 __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_kernel(const Swa2BwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef Swa2Cfg<D, NCG, PAD> C;
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_bwd_kv(D)) void swa2_bwd_kv_
   const int tid = threadIdx.x;
   const int lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Swa2Geom G0 = swa2_geom(a.p, a.plan);
+  const Swa2Geom G0 = swa2_geom<TALL>(a.p, a.plan);
   const int pc = wave & ((1 << G0.lpc) - 1), rg = wave >> G0.lpc;
 
   const char* qb = reinterpret_cast<const char*>(a.q) + 2 * (G0.b * a.qs[0] + G0.h * a.qs[1]);

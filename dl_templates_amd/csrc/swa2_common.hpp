@@ -34,9 +34,12 @@ DLT_DEV u32x2 swa2_lds_tr(Swa2Lds p) {
   return __builtin_bit_cast(u32x2, v);
 }
 
+// TALL: kernels of their own for plans with tall workgroups, whose decoding the others start without (1 to 3 % of kernels of 10 to 30 us: 2 slabs of 81 x 114,
+// 11 x 11, d = 128, backward 28.7 -> 27.7)
+template <bool TALL>
 DLT_DEV Swa2Geom swa2_geom(const AttnProblem& p, const Swa2Plan& P) {
   // token slots per grid row and the largest column extent of a window in slots (tiles of P.S tokens)
-  return swa2_geom_at(p.g.TR, p.g.TC * P.S, p.g.WR, P.S * P.WCt + P.S - 1, p.H, P, xcd_remap(blockIdx.x, gridDim.x));
+  return swa2_geom_at<TALL>(p.g.TR, p.g.TC * P.S, p.g.WR, P.S * P.WCt + P.S - 1, p.H, P, xcd_remap(blockIdx.x, gridDim.x));
 }
 
 // One copy instruction as the hardware sees it: 64 lanes x 16 (or 4) bytes from `base + voff` (base wave-uniform)

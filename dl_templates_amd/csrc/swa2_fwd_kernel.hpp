@@ -29,8 +29,8 @@ __global__ __launch_bounds__(SWA2_THREADS, swa2_occ_fwd(D)) void swa2_fwd_kernel
   const int tid = threadIdx.x;
   const int lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Swa2Geom G0 = swa2_geom(a.p, a.plan);
-  const int pc = wave & ((1 << G0.lpc) - 1), rg = wave >> G0.lpc;
+  const Swa2Geom G0 = swa2_geom<false>(a.p, a.plan);
+  const int pc = wave & 3, rg = wave >> 2;
 
   const char* qb = reinterpret_cast<const char*>(a.q) + 2 * (G0.b * a.qs[0] + G0.h * a.qs[1]);
   const char* kb_ = reinterpret_cast<const char*>(a.k) + 2 * (G0.b * a.ks[0] + G0.h * a.ks[1]);

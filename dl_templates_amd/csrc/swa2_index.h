@@ -89,15 +89,16 @@ DLT_HD void swa2_plan_tall(Swa2Plan& P, int TR, int slots, int lpc) {
 // workgroups of a slab
 DLT_HD int swa2_groups(const Swa2Plan& P) { return P.nblk_r * P.nblk_c + P.ntall; }
 
-// geometry of workgroup `lin` (its index after the XCD remap); TC: token slots per grid row, WC: S WCt + S - 1
+// geometry of workgroup `lin` (its index after the XCD remap); TC: token slots per grid row, WC: S WCt + S - 1.  TALL: the plan may have tall workgroups
+template <bool TALL = true>
 DLT_HD Swa2Geom swa2_geom_at(int TR, int TC, int WR, int WC, int H, const Swa2Plan& P, int lin) {
   Swa2Geom G;
   G.S = P.S; G.WCt = P.WCt; G.m_S = P.m_S; G.s_S = P.s_S;
-  const int per_bh = swa2_groups(P);
+  const int per_bh = TALL ? swa2_groups(P) : P.nblk_r * P.nblk_c;
   const int bh = (int)dlt_fastdiv((uint32_t)lin, P.m_bh, P.s_bh);
-  const int rem = lin - bh * per_bh - P.ntall;   // the tall workgroups, which take longer, come first
-  const bool tall = rem < 0;
-  const int full = dlt_imax(0, rem), br = tall ? rem + P.ntall : (int)dlt_fastdiv((uint32_t)full, P.m_c, P.s_c);
+  const int rem = lin - bh * per_bh - (TALL ? P.ntall : 0);   // the tall workgroups, which take longer, come first
+  const bool tall = TALL && rem < 0;
+  const int full = TALL ? dlt_imax(0, rem) : rem, br = tall ? rem + P.ntall : (int)dlt_fastdiv((uint32_t)full, P.m_c, P.s_c);
   G.lpc = tall ? P.lpc : 2;
   const int band = tall ? 32 >> P.lpc : P.band;
   G.b = (int)dlt_fastdiv((uint32_t)bh, P.m_h, P.s_h);

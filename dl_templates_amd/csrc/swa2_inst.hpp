@@ -13,9 +13,11 @@ int swa2_set_lds(KernT kern, int bytes) { return dlt_ensure_lds(reinterpret_cast
 template <typename TIO, int NCG, bool PAD>
 int swa2_launch_fwd_t(const Swa2FwdArgs& a, int grid, hipStream_t stream) {
   typedef Swa2Cfg<DLT_SWA2_D, NCG, PAD> C;
-  const bool pairs = a.plan.pairs != 0;
+  const bool pairs = a.plan.pairs != 0, same = a.ks[2] == a.vs[2] && a.p.dk == a.p.dv;
   auto kern = !pairs ? swa2_fwd_kernel<TIO, DLT_SWA2_D, NCG, PAD>
-                    : a.ks[2] == a.vs[2] && a.p.dk == a.p.dv ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, true, PAD> : swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, false, PAD>;
+                    : same ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, true, PAD, false> : swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, false, PAD, false>;
+  if constexpr (DLT_SWA2_D == 128)   // (swa2_make_plan)
+    if (a.plan.ntall > 0) kern = same ? swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, true, PAD, true> : swa2s_fwd_kernel<TIO, DLT_SWA2_D, NCG, false, PAD, true>;
   const int lds = pairs ? C::BUF : C::LDS;
   int rc = swa2_set_lds(kern, lds);
   if (rc != DLT_OK) return rc;
@@ -29,8 +31,8 @@ int swa2_launch_fwd_t(const Swa2FwdArgs& a, int grid, hipStream_t stream) {
 template <typename TIO, int NCG, bool PAD>
 int swa2_launch_bwd_t(const Swa2BwdArgs& a, int grid, hipStream_t stream) {
   typedef Swa2Cfg<DLT_SWA2_D, NCG, PAD> C;
-  auto kq = swa2_bwd_q_kernel<TIO, DLT_SWA2_D, NCG, PAD>;
-  auto kkv = swa2_bwd_kv_kernel<TIO, DLT_SWA2_D, NCG, PAD>;
+  auto kq = a.plan.ntall > 0 ? swa2_bwd_q_kernel<TIO, DLT_SWA2_D, NCG, PAD, true> : swa2_bwd_q_kernel<TIO, DLT_SWA2_D, NCG, PAD, false>;
+  auto kkv = a.plan.ntall > 0 ? swa2_bwd_kv_kernel<TIO, DLT_SWA2_D, NCG, PAD, true> : swa2_bwd_kv_kernel<TIO, DLT_SWA2_D, NCG, PAD, false>;
   int rc = swa2_set_lds(kq, C::LDS);
   if (rc != DLT_OK) return rc;
   rc = swa2_set_lds(kkv, C::LDS_KV);

@@ -25,7 +25,7 @@ constexpr int SWA2S_THREADS = 256;
 // waves per SIMD the register budget is sized for (head dim 64 at 6 column groups spills at 3)
 constexpr int swa2s_occ(int D, int NCG) { return D == 64 && NCG == 4 ? 3 : 2; }
 
-template <typename TIO, int D, int NCG, bool SAME, bool PAD>
+template <typename TIO, int D, int NCG, bool SAME, bool PAD, bool TALL>
 __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_kernel(const Swa2FwdArgs a) {
   typedef typename ComputeOf<TIO>::type CT;
   typedef Swa2Cfg<D, NCG, PAD> C;
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(SWA2S_THREADS, swa2s_occ(D, NCG)) void swa2s_fwd_ke
   const int tid = threadIdx.x;
   const int lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Swa2Geom G0 = swa2_geom(a.p, a.plan);
+  const Swa2Geom G0 = swa2_geom<TALL>(a.p, a.plan);
   const int pc = wave & ((1 << G0.lpc) - 1), rg = 2 * (wave >> G0.lpc);
 
   const char* qb = reinterpret_cast<const char*>(a.q) + 2 * (G0.b * a.qs[0] + G0.h * a.qs[1]);

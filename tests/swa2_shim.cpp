@@ -54,6 +54,11 @@ int model(int TR, int TCt, int WR, int WCt, int S, int npass, int band_arg, int 
   const int nwg = swa2_groups(P);
   for (int lin = 0; lin < nwg; lin++) {
     const Swa2Geom G0 = swa2_geom_at(TR, TC, WR, WC, H, P, lin);
+    if (!tall) {   // the kernels for plans without tall workgroups
+      const Swa2Geom g = swa2_geom_at<false>(TR, TC, WR, WC, H, P, lin);
+      if (g.b != G0.b || g.h != G0.h || g.r0 != G0.r0 || g.c0 != G0.c0 || g.r_end != G0.r_end || g.lpc != G0.lpc || g.ch_first != G0.ch_first || g.ch_last != G0.ch_last)
+        return fail("workgroup %d without tall ones", lin);
+    }
     const Swa2Geom& G = G0;
     if (G.b != 0 || G.h != 0) return fail("workgroup %d decoded to batch %d head %d", lin, G.b, G.h);
     if (G.r0 >= TR || G.c0 >= TC) return fail("workgroup %d starts outside the grid (%d, %d)", lin, G.r0, G.c0);
