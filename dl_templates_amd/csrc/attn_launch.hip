@@ -712,8 +712,11 @@ int flash_fastest(int pass, const DimClass& dc, int dims, int64_t bh, int own, i
        {128, 4.28f, 1.038f, NONE, NONE, 2.51f, 1.14f, .072f, 2.79f, 1.38f, .114f}}};
   FlashCost c = COST[pass][dc.id];
   if (pass > 0 && dc.id == 1 && dims <= 192) {   // the split kernels leave out missing pieces of a row, of the chunked ones' work more stays (flashd_dims)
-    c.start = pass == 1 ? 7.58f : 5.26f;
-    c.chunk = pass == 1 ? 1.26f : 1.40f;
+    // dQ: scaled for other sides of more than seven chunks only, dK/dV not at all: scaled, 80/80 was split where chunked workgroups take 0.64 of the time on 64
+    // slabs and more and as long on fewer (272 x 272 causal, 324 keys of 1710 queries)
+    const bool scaled = pass == 1 && other > 448;
+    c.start = pass == 2 ? 5.62f : scaled ? 7.58f : 6.58f;
+    c.chunk = pass == 2 ? 1.226f : scaled ? 1.26f : 1.404f;
   }
   const float cus = (float)dlt_device_cus();
   const auto wgs = [&](int n) { return (float)(bh * ((own + n - 1) / n)); };
