@@ -73,7 +73,7 @@ int DLT_CAT3(dlt_launch_delta_, DLT_DK, DLT_DV)(const BwdArgs& a, hipStream_t st
 #ifndef DLT_ONE_PATCH
 // fp32 windows (win_forward); `lds` holds a chunk's rows
 int DLT_CAT3(dlt_launch_win_, DLT_DK, DLT_DV)(const WinArgs& a, int bh, int lds, hipStream_t stream) {
-  auto kern = win_parts(a.patch_shift) >> (a.wave_shift - a.patch_shift) > 1 ? attn_win_fwd_kernel<DLT_DK, DLT_DV, true> : attn_win_fwd_kernel<DLT_DK, DLT_DV, false>;
+  auto kern = a.parts >> (a.wave_shift - a.patch_shift) > 1 ? attn_win_fwd_kernel<DLT_DK, DLT_DV, true> : attn_win_fwd_kernel<DLT_DK, DLT_DV, false>;
   int rc = set_lds_limit(kern, lds);
   if (rc != DLT_OK) return rc;
   const int rows = 4 >> a.wave_shift, cols = 16 << a.patch_shift;

@@ -490,9 +490,12 @@ bool win_plan(const AttnProblem& p, const AttnTensors& t, const DimClass& dc, Wi
   const int cols = 16 << a.patch_shift;
   const int64_t nx = (p.g.XLq + cols - 1) / cols, cus = dlt_device_cus();
   auto grid = [&](int ws) { return bh * ((p.g.TR + (4 >> ws) - 1) / (4 >> ws)) * nx; };
-  // The parts of a row's window are dealt over as many waves as keeps one and a half workgroups per CU: against lines at two and three, 60 shapes of 8 ... 128 slabs
-  // take 1.007 and 1.034 of the time.  Taking several parts costs the merges of their sums: 64 slabs of 25 x 11 10.5 -> 12.3 us, of 19 x 16 7.8 -> 8.3
-  a.wave_shift = 2;
+  // Parts of a window where a row has at most 32 columns and wave slots are left: two, and four in 9 rows and more of up to 16 columns.  Against four for all of
+  // those, 140 shapes of 2 ... 128 slabs take 0.98 of the time, with three rows up to 0.82 (16 slabs of 29 x 16, 3 x 9, 6.8 -> 5.8 us); few slabs with five rows and seven 1.03
+  a.parts = a.patch_shift == 2 ? 1 : a.patch_shift == 0 && p.g.WR >= 4 ? 4 : 2;
+  // They are dealt over as many waves as keeps one and a half workgroups per CU: against lines at two and three, 60 shapes of 8 ... 128 slabs
+  // take 1.007 and 1.034 of the time.  Taking several parts costs the merges of their sums: 64 slabs of 25 x 11, 9 x 7, 10.6 -> 12.3 us
+  a.wave_shift = a.patch_shift + (a.parts >> 1);
   while (a.wave_shift > a.patch_shift && 2 * grid(a.wave_shift) > 3 * cus) a.wave_shift--;
   if (((int64_t)p.g.TR + 3) / (4 >> a.wave_shift) > 65535 || nx > 65535) return false;
   const int nrows = dlt_imin(2 * p.g.WR + (4 >> a.wave_shift), p.g.TR);

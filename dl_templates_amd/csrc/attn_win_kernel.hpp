@@ -7,7 +7,7 @@
 //   - a workgroup of 4 waves owns 16, 32 or 64 columns of 4, 2 or 1 grid rows (every halo row is staged once for all of them), or, while CUs would
 //     be idle, of fewer rows with the parts of a row's window dealt over the waves that are left (WinArgs::wave_shift; their sums meet in LDS);
 //   - a block of 32 keys is two halo rows where a row has at most 16 tokens, one whole row up to 32, else it starts at the wave's first column.
-// A slab's bits do not depend on how many a call holds: a window's rows are summed in WinArgs::parts parts, each from nothing, which are added in order
+// A slab's bits do not depend on how many a call holds: a window's rows are summed in parts (WinArgs::parts), each from nothing, which are added in order
 // whether one wave takes them one after the other or several side by side, and the blocks start at the window's first row whatever the
 // rows of a workgroup and of a chunk (in pairs of rows chunks overlap by one).
 // (figures at win_plan)
@@ -22,6 +22,7 @@ struct WinArgs {
   int32_t H, TR, XL, WR, WC;
   int32_t dk, dv;
   int32_t patch_shift;   // 1 << patch_shift blocks of 16 queries lie side by side
+  int32_t parts;         // a window's rows are summed in 4, 2 or 1 parts (by the map's width and the window alone: win_plan)
   int32_t wave_shift;    // 1 << wave_shift waves share a grid row: the blocks, times the waves that its parts are dealt over
   int32_t chunk_rows, cx, pair;   // halo rows staged at once, LDS slots of a row, two rows to a block of keys
   float scale_log2;
@@ -30,7 +31,6 @@ struct WinArgs {
 constexpr int win_pitch_k(int DK) { return DK * 4 + 16; }
 constexpr int win_pitch_v(int DV) { return DV * 2 + 16; }
 constexpr int win_per_token(int DK, int DV) { return win_pitch_k(DK) + win_pitch_v(DV); }
-constexpr int win_parts(int patch_shift) { return 4 >> patch_shift; }
 constexpr int win_sum_bytes(int DV) { return 4 * 64 * (DV + 8); }   // DV / 16 fragments of 16 bytes, maximum and sum: per lane of up to four parts
 // (in pairs of rows the half block beside a lone one may lie behind the chunk)
 constexpr int win_lds_bytes(int DK, int DV, int rows, int cx, bool pair) {
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void attn_win_fwd_kernel(const WinArgs a) {
   }
 
   // the wave's parts of the window: rows next ... stop in steps of part_rows; the first wave of a row adds them up, others keep theirs (two at most) apart
-  const int parts = win_parts(a.patch_shift), own_parts = MULTI ? parts >> (a.wave_shift - a.patch_shift) : 1, nwin = wrhi - wrlo + 1;
+  const int parts = a.parts, own_parts = MULTI ? parts >> (a.wave_shift - a.patch_shift) : 1, nwin = wrhi - wrlo + 1;
   const int part_rows = a.pair ? ((nwin + 2 * parts - 1) / (2 * parts)) * 2 : (nwin + parts - 1) / parts;
   int next = wrlo + turn * own_parts * part_rows, part_end = next + part_rows;
   const int stop = dlt_imin(wrhi, next + own_parts * part_rows - 1);
