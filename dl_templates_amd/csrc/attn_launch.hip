@@ -615,9 +615,9 @@ bool swat_eligible(const AttnProblem& p, const AttnTensors& t, bool bwd) {
   // d = 64, five rows of three columns, 190 shapes of 1 ... 256 slabs: forward 0.28 ... 0.90 of the time of the chunked kernels, backward 0.38 ... 1.04 where two
   // strips hold seven columns or more (5 and 6 columns, whose second strip is mostly empty, up to 1.24 there and left to the others): 2 slabs of 30 x 30 tiles
   // 25.3 -> 10 and 52.4 -> 31 us, 64 of 21 x 33 206 -> 136 and 537 -> 445.  On up to 20 tiles or so the window's keys over a workgroup's waves
-  // (flash_tiles_split) take 0.9 of the forward and 0.65 of the backward time (2 of 14 x 6 6.1 against 6.8, 12.6 against 18.2).
+  // (flash_tiles_split) take 0.9 of the forward and 0.65 of the backward time (2 of 14 x 6, forward, 5.8 against 6.3).
   // The same with five columns, forward (the scalars of the backward pass do not fit beside the ring): 0.41 ... 0.98, 64 slabs of 21 x 33 225 -> 177, 4 of 40 x 12
-  // 28.9 -> 12.
+  // 28.9 -> 11.2.
   // d = 128, 3 x 3 tiles, forward: 0.40 ... 0.98 where strips are three quarters full (2 slabs of 30 x 30 23.8 -> 13.4, 64 of 30 x 10 174 -> 106), five columns
   // up to 1.10; the backward kernels take 0.95 ... 1.5 of the time and stay there.
   if (p.dk == 128 && (p.g.S != 16 || p.g.WR != 1)) return false;

@@ -201,13 +201,14 @@ template <int N>
 DLT_DEV void flashd_wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 // chunk buffers per workgroup: a copy is started NBUF - 1 chunks ahead of its use; three where two workgroups
-// still fit a CU
+// still fit a CU with chunks of 64 tokens
 #ifndef FLASHD_NBUF
 #define FLASHD_NBUF(dk, dv) ((dk) + (dv) > 192 ? 2 : 3)
 #endif
 constexpr int flashd_nbuf(int dk, int dv) { return FLASHD_NBUF(dk, dv); }
-// the same for 8-wave workgroups: two in the forward kernel with two query blocks per wave (128-key chunks); with one own
-// block per wave (64-token chunks) as many as leave room for two workgroups per CU
+// the same for 8-wave workgroups: two in the forward kernel with two query blocks per wave (128-key chunks); with one own block per wave as many
+// as leave room for two workgroups per CU with 64-token chunks.  (One block per wave on 128-key chunks runs while workgroups are few, flash_forward: one to a
+// CU, with three buffers of 48 KB at 64/128 and two of 64 at 128/128.)
 constexpr int flashd_bufs(int dk, int dv, int np, int nw) {
   return nw == 4 ? flashd_nbuf(dk, dv) : np == 2 || dk + dv > 192 ? 2 : dk + dv > 128 ? 3 : 4;
 }
